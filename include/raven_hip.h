@@ -99,7 +99,9 @@ const char* raven_last_error(void);
  * more, that the tiled MFMA kernel takes), gemm_tiled_variant (0 = tile size by shape, 1 = 256 x 256, 2 = 128 x 128 and
  * no tile-count rule, 3 = 256 x 256 by the eight-wave kernel instead of the four-wave ring kernel), gemm_tiled_split_tail
  * (1 = the tile columns of a last round that fills at most half the chip go to
- * 128 x 128 tiles, 0 = never), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
+ * 128 x 128 tiles, 0 = never), gemm_mid (1 = products over 33 and more bf16 rows that do not fill the chip with 256 x 256 tiles may run as
+ * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (its tile
+ * shape and slice count, 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
  * gemm_ragged (1 = a 5..32-row product whose output columns divide into about two workgroups per compute unit runs as one
@@ -151,7 +153,8 @@ int raven_gemm_swiglu(const void* x, const void* fc, void* out,
  *     z = concat(x0, x1) W^T,  y = swiglu ? T(T(silu(T(z[:, :N]))) * T(z[:, N:])) : T(z) [+ residual] [as float]
  * With a workspace (raven_linear_workspace_bytes(M, widest output: 2N for SwiGLU)) and 5 or more bf16 rows,
  * K is split across workgroups and the X tile of a K step is shared by the workgroup's waves, which is
- * what batches of 8..32 rows need to approach HBM bandwidth; partial sums are added in a fixed order.
+ * what batches of 8..32 rows need to approach HBM bandwidth; partial sums are added in a fixed order.  The same holds from 33
+ * rows on for matrices with too few rows to give every compute unit a tile.
  * Without one (or for 1..4 rows, fp32) the call is forwarded to raven_gemm / _adapter_gemm_concat / _gemm_swiglu. */
 size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max);
 int    raven_linear(const void* x0, const void* x1, const void* w, const void* residual, void* y,

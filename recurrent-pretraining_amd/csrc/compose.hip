@@ -27,7 +27,7 @@ int gemv1_column_block(const void* x, const void* norm_a, const void* w_block, i
 int linear_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K,
                         void* workspace, size_t workspace_bytes, hipStream_t s);
 
-int linear_leave_sums(const void* x0, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
+int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
                       int N, int K0, int K1, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 
 int splitk_sums_then_norm(const float* partial, int ks, const float* extra, const void* residual, void* sum_out, const void* weight,
@@ -36,23 +36,24 @@ const void* packed_weight_of(const void* w, int rows, int K, int* ld);
 
 int qkv_linear_rope_append(const void* x, int ldx, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out,
                            const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, int n_heads,
-                           int head_dim, int dtype, hipStream_t s, int* done);
+                           int head_dim, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* done);
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype);
-int tiled_gemm_pitched(const void* x, int ldx, const void* w, const void* residual, void* y, int M, int N, int K, int swiglu, hipStream_t s);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes);
+int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
+               int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int rmsnorm_pitched(const void* x, const void* residual, const void* weight, void* y, int ldy, void* sum_out, const void* weight2,
                     void* y2, int ldy2, int64_t rows, int32_t dim, float eps, int32_t dtype, void* stream);
 int prefill_attention_pitched(const void* q, void* y, int ldy, const raven_kv_cache* cache, int32_t slot, int32_t B, int32_t S,
                               int32_t pos0, const int32_t* pos_dev, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
 
 // y = round(round(x W^T) + residual), then RMSNorm(weight) -> out1 and RMSNorm(weight2) of that -> out2 (either may be
-// null): two launches where the product is K-split (the norm launch adds the slices), three otherwise
-static int linear_then_norm(const void* x, const void* w, const void* residual, void* y, const void* weight, void* out1,
+// null): one launch fewer where the product is K-split (the norm launch adds the slices).  ldx: elements between two rows of x (chunks)
+static int linear_then_norm(const void* x, int ldx, const void* w, const void* residual, void* y, const void* weight, void* out1,
                             const void* weight2, void* out2, int M, int N, int K, float eps, int dtype, void* ws, size_t ws_bytes,
                             hipStream_t s, int ld_out2 = 0) {
     int ks = 0;
-    if (int rc = linear_leave_sums(x, nullptr, w, 0, nullptr, residual, y, M, N, K, 0, dtype, ws, ws_bytes, s, &ks)) return rc;
+    if (int rc = linear_leave_sums(x, ldx, nullptr, w, 0, nullptr, residual, y, M, N, K, 0, dtype, ws, ws_bytes, s, &ks)) return rc;
     // ld_out2: the row pitch of the LAST output (out2, or out1 when there is no second norm)
     const int ld1 = (weight2 == nullptr && ld_out2) ? ld_out2 : N, ld2 = ld_out2 ? ld_out2 : N;
     if (ks) return splitk_sums_then_norm(static_cast<const float*>(ws), ks, nullptr, residual, nullptr, weight, out1, weight2, out2, M, N, eps, s, ld1, ld2);
@@ -145,6 +146,24 @@ static int decode_row_pitch(const raven_dims* d, const BlockScratch& s, const ra
     return s.ld_pad;
 }
 
+// chunks of 16 or more rows per sequence: 64 or 128 query rows of a head per workgroup on the matrix cores; a few
+// rows per sequence (or a partially filled cache, which only that kernel looks up): one row at a time
+static bool chunk_on_matrix_cores(const raven_dims* d, const raven_kv_cache* cache, int S, bool paged) {
+    return !paged && d->dtype == RAVEN_BF16 && S >= 16 && (d->head_dim == 64 || d->head_dim == 96 || d->head_dim == 128) &&
+           (cache->steps_present == nullptr || cache->lookup_mode == RAVEN_LOOKUP_NONE);
+}
+
+// Rows of n_embd bf16 values that are not whole cache lines (5280: 82.5 lines): norm_1's and norm_3's output and the
+// attention output, which the products over many rows read, are laid out with rows padded to whole lines (the pad
+// is never read: the products' K stays n_embd).  The row pitch of these; every block of a call decides this the same way.
+static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const raven_kv_cache* cache, int M, int S, bool paged) {
+    const int h = d->n_embd, dt = d->dtype;
+    const bool pad = g_pad_chunk_rows && chunk_on_matrix_cores(d, cache, S, paged) && s.ld_pad != h && M >= g_tiled_min_rows &&
+                     tiled_gemm_fits(M, 3 * h, h, 0, dt, 0, s.lin_ws_bytes) && tiled_gemm_fits(M, h, h, 0, dt, 0, s.lin_ws_bytes) &&
+                     tiled_gemm_fits(M, d->intermediate, h, 0, dt, 1, s.lin_ws_bytes);
+    return pad ? s.ld_pad : h;
+}
+
 // Several rows.  n1_ready: scratch.n1 already holds norm_1(x_in).  tail_w / tail_out: a second norm
 // applied to the block output (next block's norm_1, or ln_f); y_out may be null when only the tail
 // result is wanted.
@@ -155,16 +174,8 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
     const int M = B * S, h = d->n_embd, I = d->intermediate, dt = d->dtype;
     hipStream_t hs = static_cast<hipStream_t>(stream);
     int rc;
-    // chunks of 16 or more rows per sequence: 64 or 128 query rows of a head per workgroup on the matrix cores; a few
-    // rows per sequence (or a partially filled cache, which only that kernel looks up): one row at a time
-    const bool chunk = !paged && S > 1;
-    const bool mfma = chunk && dt == RAVEN_BF16 && S >= 16 && (d->head_dim == 64 || d->head_dim == 96 || d->head_dim == 128) &&
-                      (cache->steps_present == nullptr || cache->lookup_mode == RAVEN_LOOKUP_NONE);
-    // Rows of n_embd bf16 values that are not whole cache lines (5280: 82.5 lines): norm_1's and norm_3's output and the
-    // attention output, which the tiled GEMM reads as its token rows, are laid out with rows padded to whole lines (the pad
-    // is never read: the products' K stays n_embd).  Every block of a call decides this the same way.
-    const bool pad = g_pad_chunk_rows && mfma && s.ld_pad != h && M >= g_tiled_min_rows && tiled_gemm_fits(M, 3 * h, h, 0, dt) &&
-                     tiled_gemm_fits(M, h, h, 0, dt) && tiled_gemm_fits(M, I, h, 0, dt);
+    const bool chunk = !paged && S > 1, mfma = chunk_on_matrix_cores(d, cache, S, paged != nullptr);
+    const bool pad = chunk_row_pitch(d, s, cache, M, S, paged != nullptr) != h;
     // Decode steps of 17..32 rows: the MFMA kernels of Wqkv and mlp.fc stream 5 % faster over operands with rows of whole
     // lines (fc 67.9 -> 64.5 us, Wqkv 33.1 -> 31.6 at 32 rows; no gain at 8).  Where the caller has registered line-aligned
     // copies of both matrices, the two products run over the padded length: the copies' pad columns are zeros, and so are
@@ -185,9 +196,9 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
     int qkv_done = 0;
     if (chunk)
         if ((rc = qkv_linear_rope_append(s.n1, ld, w->wqkv, w->qk_bias, freqs, s.q, cache, slot, B, S, pos0, pos_dev, d->n_heads, d->head_dim,
-                                         dt, hs, &qkv_done))) return rc;
+                                         dt, s.lin_ws, s.lin_ws_bytes, hs, &qkv_done))) return rc;
     if (!qkv_done) {
-        if (pad) rc = tiled_gemm_pitched(s.n1, ld, w->wqkv, nullptr, s.qkv, M, 3 * h, h, 0, hs);
+        if (pad) rc = tiled_gemm(s.n1, ld, nullptr, w->wqkv, nullptr, s.qkv, M, 3 * h, h, 0, 0, 0, s.lin_ws, s.lin_ws_bytes, hs, nullptr);
         else if (padk) rc = raven_linear(s.n1, nullptr, wqkv_p, nullptr, s.qkv, M, 3 * h, ld, 0, 0, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
         else rc = raven_linear(s.n1, nullptr, w->wqkv, nullptr, s.qkv, M, 3 * h, h, 0, 0, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
         if (rc) return rc;
@@ -207,19 +218,17 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
         else rc = raven_decode_attention(s.q, s.ya, cache, slot, B, S, pos0, pos_dev, d->n_heads, d->head_dim, dt, s.attn_ws, s.attn_ws_bytes, stream);
         if (rc) return rc;
     }
+    if ((rc = linear_then_norm(s.ya, pad ? ld : 0, w->proj, x_in, s.x1, w->norm_2, s.x2, w->norm_3, s.n3, M, h, h, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, ld))) return rc;
     if (pad) {
-        if ((rc = tiled_gemm_pitched(s.ya, ld, w->proj, x_in, s.x1, M, h, h, 0, hs))) return rc;
-        if ((rc = rmsnorm_pitched(s.x1, nullptr, w->norm_2, s.x2, h, nullptr, w->norm_3, s.n3, ld, M, h, d->eps, dt, stream))) return rc;
-        if ((rc = tiled_gemm_pitched(s.n3, ld, w->fc, nullptr, s.g, M, I, h, 1, hs))) return rc;
+        if ((rc = tiled_gemm(s.n3, ld, nullptr, w->fc, nullptr, s.g, M, I, h, 0, 1, 0, s.lin_ws, s.lin_ws_bytes, hs, nullptr))) return rc;
     } else {
-        if ((rc = linear_then_norm(s.ya, w->proj, x_in, s.x1, w->norm_2, s.x2, w->norm_3, s.n3, M, h, h, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, ld))) return rc;
         if (padk) rc = raven_linear(s.n3, nullptr, fc_p, nullptr, s.g, M, I, ld, 0, 1, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
         else rc = raven_linear(s.n3, nullptr, w->fc, nullptr, s.g, M, I, h, 0, 1, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
         if (rc) return rc;
     }
     // the tail norm's output is the next block's norm_1 input when it goes to scratch.n1: rows as that block will read them
     const int tail_ld = tail_out == static_cast<void*>(s.n1) ? ld : h;
-    return linear_then_norm(s.g, w->mlp_proj, s.x2, s.x3, w->norm_4, y_out, tail_w, tail_out, M, h, I, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, tail_ld);
+    return linear_then_norm(s.g, 0, w->mlp_proj, s.x2, s.x3, w->norm_4, y_out, tail_w, tail_out, M, h, I, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, tail_ld);
 }
 
 // One row.  x_raw is the block input before `pre_norm` (the previous block's norm_4, or null when x_raw is
@@ -353,6 +362,7 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
         if ((rc = linear_column_block(embeds, static_cast<const char*>(adapter_w) + (size_t)h * 2, 2 * h, nullptr, s.e_sums, 1, M, h, h,
                                       s.lin_ws, s.lin_ws_bytes, hs))) return rc;
     const int ld_decode = decode_row_pitch(dims, s, blocks, n_blocks, M, S, paged != nullptr);
+    const int ld_n1 = ld_decode ? ld_decode : chunk_row_pitch(dims, s, cache, M, S, paged != nullptr);  // rows of norm_1's output as run_block reads them
     for (int it = 0; it < n_iterations; ++it) {
         const int32_t* sl = slots ? slots + (size_t)it * n_blocks : nullptr;
         const bool last_it = it == n_iterations - 1;
@@ -362,12 +372,12 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
         if (adapter_w) {
             // where the product is K-split, the launch that adds its slices also applies the first block's norm_1
             int ks = 0;
-            if (split) rc = linear_leave_sums(st, nullptr, adapter_w, 2 * h, s.e_sums, nullptr, s.xa, M, h, h, 0, dims->dtype, s.lin_ws, s.lin_ws_bytes, hs, &ks);
-            else rc = linear_leave_sums(st, embeds, adapter_w, 0, nullptr, nullptr, s.xa, M, h, h, h, dims->dtype, s.lin_ws, s.lin_ws_bytes, hs, &ks);
+            if (split) rc = linear_leave_sums(st, 0, nullptr, adapter_w, 2 * h, s.e_sums, nullptr, s.xa, M, h, h, 0, dims->dtype, s.lin_ws, s.lin_ws_bytes, hs, &ks);
+            else rc = linear_leave_sums(st, 0, embeds, adapter_w, 0, nullptr, nullptr, s.xa, M, h, h, h, dims->dtype, s.lin_ws, s.lin_ws_bytes, hs, &ks);
             if (rc) return rc;
             if (ks) {
                 if ((rc = splitk_sums_then_norm(static_cast<const float*>(s.lin_ws), ks, split ? s.e_sums : nullptr, nullptr, s.xa, blocks[0].norm_1,
-                                                s.n1, nullptr, nullptr, M, h, dims->eps, hs, ld_decode, 0))) return rc;
+                                                s.n1, nullptr, nullptr, M, h, dims->eps, hs, ld_n1, 0))) return rc;
                 n1_ready = true;
             }
         }

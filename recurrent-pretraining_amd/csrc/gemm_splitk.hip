@@ -27,11 +27,11 @@ extern "C" int raven_gemm_swiglu(const void* x, const void* fc, void* out, int32
 namespace raven {
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype);
-int tiled_gemm(const void* x0, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
-               int out_f32, hipStream_t s);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes);
+int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
+               int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
-                    hipStream_t s);
+                    void* workspace, size_t workspace_bytes, hipStream_t s);
 int gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
               hipStream_t s);
 
@@ -352,14 +352,21 @@ int linear_column_block(const void* x, const void* w_block, int ldw, const float
 
 int g_fuse_sums_norm = 1;  // raven_set_tuning("fuse_sums_norm"): 0 = a K-split product always adds its slices in a launch of its own
 
-// A product whose result goes straight into an RMSNorm launch: y = round(round(x W^T [+ extra]) + residual) for at most 32
-// bf16 rows, W either a whole [N, K0 + K1] matrix (ldw = 0) or a column block with row pitch ldw (K1 = 0).  When the product
+// The workspace a caller offers, as the kernels may use it
+static size_t usable(const void* workspace, size_t bytes) { return workspace && ((uintptr_t)workspace & 255) == 0 ? bytes : 0; }
+
+// A product whose result goes straight into an RMSNorm launch: y = round(round(x W^T [+ extra]) + residual), W either a whole [N, K0 + K1] matrix (ldw = 0) or a column block with row pitch ldw (K1 = 0).  When the product
 // takes the K-split kernel, its slices are left in the workspace un-added (*ks_left slices, to be handed to
 // splitk_sums_then_norm before anything else uses the workspace) and y is not written; otherwise the product is finished
 // into y and *ks_left is 0.
-int linear_leave_sums(const void* x0, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
+// From 33 rows on the slices are those of gemm_mid.hip; ldx: elements between two rows of x0 there (0: K0).
+int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
                       int N, int K0, int K1, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
     *ks_left = 0;
+    const size_t room = usable(workspace, workspace_bytes);
+    if (!ldw && M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room))
+        return tiled_gemm(x0, ldx, x1, w, residual, y, M, N, K0, K1, 0, 0, workspace, room, s, g_fuse_sums_norm && N <= 8192 ? ks_left : nullptr);
+    RAVEN_REQUIRE(ldx == 0 || ldx == K0, "linear: rows of x0 %d elements apart", ldx);
     bool split = g_fuse_sums_norm && dtype == RAVEN_BF16 && M >= 2 && M <= 32 && N % 16 == 0 && N <= 8192 && K0 % 32 == 0 && K1 % 32 == 0 &&
                  workspace != nullptr && ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 8 && M > g_linear_min_rows;
     if (split && !ldw && g_linear_ks == 0) split = N / 16 < 2 * ns_cus() && (M >= 5 || K0 + K1 >= 8192);  // from 5 rows on, from 2 for long K: the product's second launch is saved, and the norm launch requests all slices of a row at once (5 / 8 / 12 rows: 228.7 / 350.7 / 501.5 tokens/s against 228.3 / 348.5 / 495.0 with the K split only from 13 rows or K >= 8192)
@@ -382,7 +389,12 @@ int linear_leave_sums(const void* x0, const void* x1, const void* w, int ldw, co
 extern "C" size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max) {
     if (M <= 0 || n_out_max <= 0) return 0;
     const int rows = M < 32 ? M : 32;
-    return raven_host::align_up((size_t)8 * rows * n_out_max * sizeof(float));
+    size_t bytes = (size_t)8 * rows * n_out_max * sizeof(float);
+    if (M > 32) {  // gemm_mid.hip: at most 8 slices, and at most one unit of 192 x 256 sums per CU (and a few more)
+        const size_t all = (size_t)8 * M * n_out_max * sizeof(float), most = (size_t)264 * 192 * 256 * sizeof(float);
+        bytes = bytes > (all < most ? all : most) ? bytes : (all < most ? all : most);
+    }
+    return raven_host::align_up(bytes);
 }
 
 extern "C" int raven_linear(const void* x0, const void* x1, const void* w, const void* residual, void* y, int32_t M, int32_t N,
@@ -396,8 +408,8 @@ extern "C" int raven_linear(const void* x0, const void* x1, const void* w, const
     RAVEN_REQUIRE((K1 == 0) == (x1 == nullptr), "linear: x1 and K1 must be given together");
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32 || K1)), "linear: the SwiGLU epilogue takes one operand, no residual, and stores T");
     RAVEN_REQUIRE(!(K1 && (residual || out_f32)), "linear: the two-operand form has a plain epilogue");
-    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype))  // many rows: tiles of the whole product on the matrix cores
-        return tiled_gemm(x0, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, static_cast<hipStream_t>(stream));
+    if (const size_t room = usable(workspace, workspace_bytes); M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, swiglu, room))  // many rows
+        return tiled_gemm(x0, 0, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, workspace, room, static_cast<hipStream_t>(stream), nullptr);
     bool fits = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                 ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1;
     // Matrices with many rows give the kernel without a workspace enough workgroups and it is then the faster one
@@ -453,7 +465,8 @@ extern "C" int raven_linear_epilogue(const void* x0, const void* x1, const void*
     RAVEN_REQUIRE(!epi->residual || epi->out_f32, "linear_epilogue: a residual needs a float output");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (K1 == 0 && gemm_narrow_fits(M, N, K0, dtype)) return gemm_narrow_free(x0, w, y, N, M, N, K0, *epi, s);
-    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype)) return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, s);
+    if (const size_t room = usable(workspace, workspace_bytes); M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room))
+        return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, workspace, room, s);
     // the same choice between the kernels with and without a K split as raven_linear
     const bool split = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                        ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1 &&

@@ -40,13 +40,10 @@
 // M, N and the last tile: rows past the end are clamped on the load side and not stored.  K0 and K1 are multiples of 8
 // (pieces past K come from a zero page); two segments share one row pitch (K1 == K0).
 
-#include <type_traits>
-#include <utility>
-
 #include <mutex>
 #include <unordered_map>
 
-#include "raven_common.h"
+#include "gemm_common.h"
 
 namespace raven {
 
@@ -75,34 +72,8 @@ struct TiledArgs {
         int64_t w_stride;        // elements between two groups' matrices
     } groups;
     int rope_on;           // the epilogue below instead of y
-    // The product is a chunk's fused q | k | v rows (3 * nh * hd columns): instead of y, the epilogue adds the q / k bias,
-    // rotates q and k (RoPE on adjacent pairs) and writes q to q_out and k, v to their cache rows -- what
-    // qkv_rope_append_tiled_kernel (attention.hip) does to a stored product, with the same functions in the same order.
-    struct RopeAppend {
-        const float* freqs;
-        const bf16* qk_bias;   // [2, nh * hd] or null
-        bf16* q_out;           // [M, nh * hd]
-        bf16 *k, *v;           // cache tensors, [.., batch, nh, t_max, hd] from slot_off on
-        int64_t slot_off;
-        const int* pos_dev;    // position of a sequence's first row, on the device (or null: pos0)
-        int nh, hd, t_max, S, pos0;
-        int col0;              // column of the whole product that this launch's column 0 is
-    } rope;
+    RopeAppend rope;       // (gemm_common.h)
 };
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-
-template <int... I, typename F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
-}
 
 // Epilogue of both kernels.  Accumulator tile [ta][tb] (16 weight rows x 16 token rows) leaves a lane with token row
 // 16 tb + l16 and output columns 16 ta + 4 q4 + (0 .. 3); under SwiGLU tile 2 t holds gate columns and 2 t + 1 the
@@ -277,8 +248,8 @@ __device__ __forceinline__ void store_tiles_rope(const TiledArgs& a, const f32x4
     // arguments the fields are fetched at the top and held in scalar registers through the K loop
     const char __attribute__((address_space(4)))* ka = (const char __attribute__((address_space(4)))*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(ka));
-    TiledArgs::RopeAppend r;
-#define RAVEN_ROPE_FIELD(F_) r.F_ = *reinterpret_cast<const decltype(r.F_) __attribute__((address_space(4)))*>(ka + offsetof(TiledArgs, rope) + offsetof(TiledArgs::RopeAppend, F_))
+    RopeAppend r;
+#define RAVEN_ROPE_FIELD(F_) r.F_ = *reinterpret_cast<const decltype(r.F_) __attribute__((address_space(4)))*>(ka + offsetof(TiledArgs, rope) + offsetof(RopeAppend, F_))
     RAVEN_ROPE_FIELD(freqs); RAVEN_ROPE_FIELD(qk_bias); RAVEN_ROPE_FIELD(q_out); RAVEN_ROPE_FIELD(k); RAVEN_ROPE_FIELD(v);
     RAVEN_ROPE_FIELD(slot_off); RAVEN_ROPE_FIELD(pos_dev); RAVEN_ROPE_FIELD(nh); RAVEN_ROPE_FIELD(hd); RAVEN_ROPE_FIELD(t_max);
     RAVEN_ROPE_FIELD(S); RAVEN_ROPE_FIELD(pos0); RAVEN_ROPE_FIELD(col0);
@@ -869,17 +840,30 @@ static int launch_tiled(TiledArgs a, hipStream_t s) {
     return raven_host::check_launch("gemm (tiled MFMA)");
 }
 
-// Host entry for the other translation units: true when the shape is one the tiled kernel takes and is the better choice
-// for.  Few token rows against a matrix with few rows give too few tiles to fill the chip (there is no K split here):
-// those go to the skinny kernels, 32 rows per pass over the weights -- up to two passes at K = 5280, four at 10560 and
-// five (160 rows) at 17920, where the passes' split over K still beats one round of 128 x 128 tiles walking the whole of K
-// (measured at 33 .. 160 rows: Wqkv 98 / 130 us in three / four passes against 75 / 81 tiled, mlp.proj 172 against 199).
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype) {
+// The plan of gemm_mid.hip for a product, or one without tiles where the kernels of this file are the better choice: once 256 x 256 tiles
+// fill the chip (256 of them), and where the K slices of the plan would not fit the caller's workspace.
+static MidPlan mid_choice(int M, int N, int K0, int K1, int swiglu, size_t workspace_bytes) {
+    MidPlan none{};
+    const int bn_out = swiglu ? 128 : 256;
+    if (g_tiled_variant != 0 || M < g_tiled_min_rows || (int64_t)((M + 255) / 256) * ((N + bn_out - 1) / bn_out) >= 256) return none;
+    const MidPlan p = mid_plan(M, N, K0, K1, swiglu);
+    return mid_workspace_bytes(M, N, p, swiglu) <= workspace_bytes ? p : none;
+}
+
+// Host entry for the other translation units: true when the shape is one the kernels over many rows take and they are the better
+// choice for.  Few token rows against a matrix with few rows give too few tiles to fill the chip: gemm_mid.hip then cuts K
+// into slices, which needs a workspace (workspace_bytes of raven_linear_workspace_bytes); without one those products go to the skinny
+// kernels, 32 rows per pass over the weights -- up to two passes at K = 5280, four at 10560 and five (160 rows) at 17920, where
+// the passes' split over K still beats one round of 128 x 128 tiles walking the whole of K (measured at 33 .. 160 rows: Wqkv
+// 98 / 130 us in three / four passes against 75 / 81 tiled, mlp.proj 172 against 199).
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes) {
+    const bool ok = dtype == RAVEN_BF16 && M >= 1 && N % 8 == 0 && K0 % 8 == 0 && K0 > 0 && (K1 == 0 || K1 == K0) &&
+                    (int64_t)M * (K0 > K1 ? K0 : K1) < (1ll << 31) && (int64_t)N * 2 * (K0 + K1) < (1ll << 31);
+    if (!ok) return false;
     const int64_t small_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int passes = (K0 + K1 + 3499) / 3500;
-    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) return false;
-    return dtype == RAVEN_BF16 && M >= 1 && N % 8 == 0 && K0 % 8 == 0 && K0 > 0 && (K1 == 0 || K1 == K0) && (int64_t)M * (K0 > K1 ? K0 : K1) < (1ll << 31) &&
-           (int64_t)N * 2 * (K0 + K1) < (1ll << 31);
+    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) return mid_choice(M, N, K0, K1, swiglu, workspace_bytes).nt != 0;
+    return true;
 }
 
 // Copies of weight matrices with their rows padded to whole 128-byte lines (raven_register_packed_weight): at K = 5280 every
@@ -911,8 +895,10 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const bf16* __restrict__
 }
 
 static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0,
-                           int K1, int swiglu, int out_f32, const TiledArgs::RopeAppend* rope, hipStream_t s, const raven_epilogue* epi = nullptr) {
-    RAVEN_REQUIRE(tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
+                           int K1, int swiglu, int out_f32, const RopeAppend* rope, void* workspace, size_t workspace_bytes, hipStream_t s,
+                           const raven_epilogue* epi = nullptr, int* ks_left = nullptr) {
+    if (ks_left) *ks_left = 0;
+    RAVEN_REQUIRE(tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32)), "gemm (tiled): the SwiGLU epilogue has no residual and stores bf16");
     RAVEN_REQUIRE(((uintptr_t)x0 & 15) == 0 && ((uintptr_t)x1 & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
                       ((uintptr_t)residual & 15) == 0, "gemm (tiled): operands must be 16-byte aligned");
@@ -935,6 +921,11 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
             a.w = it->second.packed;
             a.ldw = it->second.ld;
         }
+    }
+    const MidPlan mid = mid_choice(M, N, K0, a.K1, swiglu, workspace_bytes);
+    if (mid.nt) {
+        const ProductArgs q{a.w, a.x0, a.x1, a.residual, y, M, N, K0, a.K1, a.ldw, a.ldx, swiglu, out_f32, epi, rope};
+        return mid_gemm(q, mid, workspace, s, ks_left);
     }
     if (epi) a.epi = *epi;
     if (rope) {
@@ -981,15 +972,17 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     return launch(a, big);
 }
 
-int tiled_gemm(const void* x0, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
-               int out_f32, hipStream_t s) {
-    return tiled_gemm_impl(x0, 0, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, nullptr, s);
+// ldx: elements between two rows of x0 (0: K0; activations may have their rows padded to whole cache lines, one segment only).  The
+// workspace takes the K slices of gemm_mid.hip; ks_left (may be null): as in mid_gemm.
+int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
+               int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
+    return tiled_gemm_impl(x0, ldx, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, nullptr, workspace, workspace_bytes, s, nullptr, ks_left);
 }
 
 // The product with the free epilogue: y = act(scale * z + bias) + residual, float or bf16
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
-                    hipStream_t s) {
-    return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, s, &epi);
+                    void* workspace, size_t workspace_bytes, hipStream_t s) {
+    return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, workspace, workspace_bytes, s, &epi);
 }
 
 // Products of row groups (tile_rows = 128 or 256 rows to a tile row): y[r] = x[x_row[r]] W_g^T, W_g = w + g * w_stride [N or 2N, K] of the group that row r of the
@@ -1013,19 +1006,14 @@ int grouped_gemm(const void* x, int x_rows, const void* w, int64_t w_stride, voi
     return swiglu ? launch_tiled<EPI_SWIGLU, 2, 1, 2, 4, true>(a, s) : launch_tiled<EPI_FREE, 2, 1, 2, 4, true>(a, s);
 }
 
-// The same with the rows of x `ldx` elements apart (>= K, one segment): activations whose rows are padded to whole cache lines
-int tiled_gemm_pitched(const void* x, int ldx, const void* w, const void* residual, void* y, int M, int N, int K, int swiglu, hipStream_t s) {
-    return tiled_gemm_impl(x, ldx, nullptr, w, residual, y, M, N, K, 0, swiglu, 0, nullptr, s);
-}
-
 // A chunk's q | k | v product (wqkv: [3 * nh * hd, K]) whose epilogue adds the q / k bias, applies RoPE and writes q to
 // q_out [M, nh * hd] and k, v to the cache rows of positions pos0 (or *pos_dev) + 0 .. S - 1 of each of the M / S sequences:
 // the product itself is never stored.  k_cache / v_cache: the cache tensors, slot_off the slot's element offset.
 int tiled_gemm_qkv_rope(const void* x, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out, void* k_cache,
                         void* v_cache, int64_t slot_off, int nh, int hd, int t_max, int M, int S, int K, int ldx, int pos0,
-                        const int* pos_dev, hipStream_t s) {
+                        const int* pos_dev, void* workspace, size_t workspace_bytes, hipStream_t s) {
     RAVEN_REQUIRE(freqs && q_out && k_cache && v_cache && hd % 8 == 0 && S > 0 && M % S == 0, "gemm (tiled, q/k/v epilogue): bad arguments");
-    TiledArgs::RopeAppend r{};
+    RopeAppend r{};
     r.freqs = freqs;
     r.qk_bias = static_cast<const bf16*>(qk_bias);
     r.q_out = static_cast<bf16*>(q_out);
@@ -1034,7 +1022,7 @@ int tiled_gemm_qkv_rope(const void* x, const void* wqkv, const void* qk_bias, co
     r.slot_off = slot_off;
     r.pos_dev = pos_dev;
     r.nh = nh; r.hd = hd; r.t_max = t_max; r.S = S; r.pos0 = pos0; r.col0 = 0;
-    return tiled_gemm_impl(x, ldx, nullptr, wqkv, nullptr, nullptr, M, 3 * nh * hd, K, 0, 0, 0, &r, s);
+    return tiled_gemm_impl(x, ldx, nullptr, wqkv, nullptr, nullptr, M, 3 * nh * hd, K, 0, 0, 0, &r, workspace, workspace_bytes, s);
 }
 
 }  // namespace raven

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
 int g_norm_early = -1;  // raven_set_tuning("norm_early"): -1 = by row count, 0 / 1 = weights fetched late / early
 
 // The second launch of a K-split product (its slices added in order, rounded, plus the residual) and the RMSNorm(s) that
-// consume the result, as one launch: bf16, up to 32 rows of at most 8192 columns.  sum_out (may be null) receives the
+// consume the result, as one launch: bf16 rows of at most 8192 columns.  sum_out (may be null) receives the
 // product's value, y (may be null) the first norm's, y2 the second's when weight2 is given.
 int splitk_sums_then_norm(const float* partial, int ks, const float* extra, const void* residual, void* sum_out, const void* weight,
                           void* y, const void* weight2, void* y2, int rows, int dim, float eps, hipStream_t s, int ldy, int ldy2) {

@@ -85,7 +85,7 @@ class GitipelLayer:
 
 class GitipelForCausalLM(StreamDecoderForCausalLM):
     config_class = GitipelConfig
-    KERNEL_SOURCES = ("gemm_skinny.hip", "gemm_splitk.hip", "gemm_tiled.hip", "gemv_decode.hip", "norm_conv.hip", "attention_capped.hip",
+    KERNEL_SOURCES = ("gemm_skinny.hip", "gemm_splitk.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemv_decode.hip", "norm_conv.hip", "attention_capped.hip",
                       "delta_rule.hip", "compose_mixer.hip", "misc.hip")
 
     def build(self, w: Weights) -> None:

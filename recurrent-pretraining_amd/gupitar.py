@@ -154,7 +154,7 @@ class GupitarLayer:
 
 class GupitarForCausalLM(StreamDecoderForCausalLM):
     config_class = GupitarConfig
-    KERNEL_SOURCES = ("gemm_skinny.hip", "gemm_splitk.hip", "gemm_tiled.hip", "gemv_decode.hip", "norm_conv.hip", "latent_attention.hip", "rglru.hip",
+    KERNEL_SOURCES = ("gemm_skinny.hip", "gemm_splitk.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemv_decode.hip", "norm_conv.hip", "latent_attention.hip", "rglru.hip",
                       "moe.hip", "compose_mixer.hip", "misc.hip")
 
     def build(self, w: Weights) -> None:

@@ -94,19 +94,19 @@ class PagedDecoder:
 
     # ------------------------------------------------------------------ rows of any sequences (prompt chunks, decode rows)
 
-    def _token_block(self, blk, f: int, x: torch.Tensor, meta) -> torch.Tensor:
+    def _token_block(self, blk, f: int, x: torch.Tensor, meta, ws: torch.Tensor) -> torch.Tensor:
         """One SandwichBlock (vllm/raven_vllm.py:289-294 around its attention layer, :184-203) on flat rows, flat layer f."""
         eps = self.cfg.norm_eps
         positions, slots, table, lens, q_start, max_q = meta
         n1 = hip.rmsnorm_residual(x, blk.norm_1.weight, eps)[0]
-        qkv = hip.linear(n1, blk.attn.Wqkv.weight)
+        qkv = hip.linear(n1, blk.attn.Wqkv.weight, workspace=ws)
         bias = blk.attn.qk_bias if hasattr(blk.attn, "qk_bias") else None
         q = hip.paged_qkv_rope_append(qkv, bias, self.model._natives()["freqs"], positions, slots, self.k[f], self.v[f], layout=self.layout)
         ya = hip.paged_prefill_attention(q, self.k[f], self.v[f], table, lens, q_start, max_q, layout=self.layout)
         # the residual adds (RMM:534-535) and the SwiGLU (RMM:507-508) ride in the epilogues of the products
-        x1 = hip.linear(ya, blk.attn.proj.weight, residual=x)
+        x1 = hip.linear(ya, blk.attn.proj.weight, residual=x, workspace=ws)
         x2, _, n3 = hip.rmsnorm_residual(x1, blk.norm_2.weight, eps, weight2=blk.norm_3.weight)
-        x3 = hip.linear(hip.linear(n3, blk.mlp.fc.weight, swiglu=True), blk.mlp.proj.weight, residual=x2)
+        x3 = hip.linear(hip.linear(n3, blk.mlp.fc.weight, swiglu=True, workspace=ws), blk.mlp.proj.weight, residual=x2, workspace=ws)
         return hip.rmsnorm_residual(x3, blk.norm_4.weight, eps)[0]
 
     @torch.no_grad()
@@ -131,22 +131,23 @@ class PagedDecoder:
         meta = (positions.to(dev, torch.int64), slot_mapping.to(dev, torch.int64), block_table.to(dev, torch.int32).contiguous(),
                 seq_lens.to(dev, torch.int32), query_start_loc.to(dev, torch.int32), int(max_query_len))
         n_pre, n_core = cfg.n_layers_in_prelude, cfg.n_layers_in_recurrent_block
+        ws = hip.linear_workspace(T, max(3 * cfg.n_embd, 2 * cfg.intermediate_size), dev)  # K slices of the products
         x = hip.embed(t.wte.weight, input_ids.reshape(-1).to(dev, torch.int64).contiguous(), m.emb_scale)
         for i in range(n_pre):
-            x = self._token_block(t.prelude[i], i, x, meta)
+            x = self._token_block(t.prelude[i], i, x, meta, ws)
         embeds = x
         if input_states is None:
             state = m.initialize_state(embeds, init_scale) if init_scale > 0 else torch.zeros_like(embeds)
         else:
             state = input_states.reshape(T, -1).to(dev, m.dtype)
         for _ in range(self.r):
-            state = hip.linear(state, t.adapter.weight, x1=embeds)  # the concat of RMM:776 as two K segments
+            state = hip.linear(state, t.adapter.weight, x1=embeds, workspace=ws)  # the concat of RMM:776 as two K segments
             for j in range(n_core):
-                state = self._token_block(t.core_block[j], n_pre + j, state, meta)
+                state = self._token_block(t.core_block[j], n_pre + j, state, meta, ws)
         latents = hip.rmsnorm_residual(state, t.ln_f.weight, cfg.norm_eps)[0]
         x = latents
         for i in range(cfg.n_layers_in_coda):
-            x = self._token_block(t.coda[i], n_pre + n_core + i, x, meta)
+            x = self._token_block(t.coda[i], n_pre + n_core + i, x, meta, ws)
         x = hip.rmsnorm_residual(x, t.ln_f.weight, cfg.norm_eps)[0]
         logits = hip.gemm(x, m.lm_head.weight, out_f32=True)
         return logits, latents

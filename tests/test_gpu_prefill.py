@@ -144,6 +144,65 @@ def test_tiled_gemm_edges_against_oracle(pkg, tuned, variant, M, N, K):
         assert torch.equal(a, pkg.hip.linear(dev(x), dev(w))), (variant, other)
 
 
+@pytest.mark.parametrize("ks", [1, 3])
+@pytest.mark.parametrize("mt", [1, 2, 4])
+@pytest.mark.parametrize("nt", [2, 4, 6])
+def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, ks):
+    """gemm_mid.hip: every tile shape, whole and in K slices, at sizes where units, steps and tiles end early: columns that leave the last
+    unit and its last tile partly filled, rows past the last tile, fewer K steps than the ring has stages, a K that is no
+    multiple of 64, a boundary between two segments inside a step; every epilogue, with rows of x padded or not."""
+    dt = torch.bfloat16
+    for M, N, K in ((33, 72, 72), (130, 328, 200), (259, 1048, 456), (70, 200, 1096)):
+        tuned(gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
+        ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+        x, w, res = _gpu_randn((M, K), 700 + M), _gpu_randn((N, K), 701 + N, 0.05), _gpu_randn((M, N), 702)
+        z = x.float() @ w.float().T
+        what = f"{M} x {N} x {K}"
+        check(pkg.hip.linear(x, w, workspace=ws), z.to(dt), dt, what)
+        check(pkg.hip.linear(x, w, residual=res, workspace=ws), (z.to(dt).float() + res.float()).to(dt), dt, what + " + residual", mag=z, ulps=ULPS_RESIDUAL)
+        check(pkg.hip.linear(x, w, out_f32=True, workspace=ws), z.to(dt).float(), dt, what + ", float")
+        fc = _gpu_randn((2 * N, K), 703, 0.05)
+        u = (x.float() @ fc.float().T).to(dt).float()
+        check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :N]).to(dt).float() * u[:, N:]).to(dt), dt, what + ", SwiGLU", ulps=ULPS_SWIGLU)
+        x1, w2 = _gpu_randn((M, K), 704), _gpu_randn((N, 2 * K), 705, 0.05)
+        check(pkg.hip.linear(x, w2, x1=x1, workspace=ws), (torch.cat([x, x1], -1).float() @ w2.float().T).to(dt), dt, what + ", two operands")
+        bias, resf = torch.randn(N, device="cuda"), torch.randn(M, N, device="cuda")
+        got = pkg.hip.linear_epilogue(x, w, bias=bias, residual=resf, scale=0.5, workspace=ws)
+        assert close(got, z * 0.5 + bias + resf)[1] < 3e-6, what + ", unrounded"   # fp32 sums of at most 1096 products in another order
+        check(pkg.hip.linear_epilogue(x, w, bias=bias, act=pkg.hip.ACT_GELU, out_f32=False, workspace=ws), F.gelu(z + bias).to(dt), dt, what + ", gelu")
+        check(pkg.hip.linear_epilogue(x, w, act=pkg.hip.ACT_TANH, out_f32=False, workspace=ws), torch.tanh(z).to(dt), dt, what + ", tanh")
+        # the slices' sums do not depend on who adds them, and the same call gives the same bits
+        assert torch.equal(pkg.hip.linear(x, w, workspace=ws), pkg.hip.linear(x, w, workspace=ws))
+
+
+@pytest.mark.parametrize("M", [40, 100])
+def test_slices_of_many_rows_folded_into_the_norm_change_no_bit(pkg, tuned, M):
+    """A block over 33 and more rows at widths whose attn.proj and mlp.proj are cut into K slices: the norm launch adds them
+    (fuse_sums_norm = 1) or a launch of their own does, with activation rows padded or not; same bits.  A workspace too small for the
+    slices is no error: the product then takes another kernel."""
+    h, nh, inter, dt = 480, 5, 2816, torch.bfloat16
+    g = torch.Generator().manual_seed(3)
+    mk = lambda *s: (torch.randn(*s, generator=g) * 0.03).to(dt).cuda()
+    norms = [1 + mk(h) for _ in range(4)]
+    blk = pkg.hip.make_block_weights(*norms, *(keep := [mk(3 * h, h), mk(2, 1, nh, 96), mk(h, h), mk(2 * inter, h), mk(h, inter)]))
+    dims = pkg.hip.make_dims(h, nh, inter, 1e-6, dt)
+    freqs = O.rope_table(96, M, 50000).to(dt).float().reshape(M, 48, 2).contiguous().cuda()
+    x, ws = _gpu_randn((M, h), 9), pkg.hip.block_workspace(dims, M, "cuda")
+    outs = []
+    for fuse, pad, ks in ((1, 1, 0), (0, 1, 0), (1, 0, 0), (1, 1, 3), (0, 0, 3)):
+        tuned(fuse_sums_norm=fuse, pad_chunk_rows=pad, gemm_mid_ks=ks)
+        k, v = (torch.zeros(1, 1, nh, M, 96, dtype=dt, device="cuda") for _ in range(2))
+        out = pkg.hip.sandwich_block(dims, blk, x, torch.empty_like(x), freqs, pkg.hip.make_cache(k, v), 0, 1, M, 0, ws)
+        outs.append((out.clone(), k, v))
+    for o in outs[1:3]:
+        assert all(torch.equal(a, b) for a, b in zip(o, outs[0]))
+    assert all(torch.equal(a, b) for a, b in zip(outs[3], outs[4]))
+    check(outs[3][0], outs[0][0].float(), dt, "three slices against the default", ulps=ULPS_COMPOSED)
+    a, w = _gpu_randn((M, inter), 10), keep[4]
+    tiny = torch.empty(256, dtype=torch.uint8, device="cuda")
+    check(pkg.hip.linear(a, w, workspace=tiny), (a.float() @ w.float().T).to(dt), dt, "without room for slices")
+
+
 @pytest.mark.parametrize("N", [16640, 16544])
 def test_tiled_gemm_last_round_as_small_tiles_changes_no_bit(pkg, tuned, N):
     """4 x 65 tiles of 256 x 256 (4 x 130 under SwiGLU): the tiles of the last, nearly empty round (the last tile
