@@ -49,6 +49,19 @@ struct ProductArgs {
     const RopeAppend* rope;      // or null
 };
 
+// Products of row groups with a weight matrix each: tile row t multiplies rows group_row[t] .. group_end[t] - 1 (at most tile_rows of them)
+// with the matrix of group group_of[t].  The first *used entries are tiles; a launch is sized for n_tiles, and its workgroups share the used
+// ones out over the XCDs (shared out by n_tiles, a fifth of the chip idled behind the unused ones of a 4096-token chunk)
+struct RowGroups {
+    const int *group_of, *group_row, *group_end, *used;
+    int n_tiles, tile_rows;
+    const int* x_row;        // row of x behind a row of the product, or null: the same
+    const float* x_scale;    // SwiGLU: factor of a row of x, applied to its sums
+    int64_t w_stride;        // elements between two groups' matrices
+    const bf16* w_extra;     // matrix of group extra_group (-1: none), which lies elsewhere
+    int extra_group;
+};
+
 // gemm_mid.hip: how a product over a middling number of rows is cut (0 units: not one for that kernel)
 struct MidPlan {
     int nt, mt;            // 16-row tiles of a wave along the weight rows / the token rows
@@ -62,5 +75,8 @@ size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu);  // 0 wh
 // ks_left (may be null): the K slices stay in the workspace ([slices, M, N] float) for the caller to add; receives their number, 0
 // when the product was finished
 int mid_gemm(const ProductArgs& a, const MidPlan& p, void* workspace, hipStream_t s, int* ks_left);
+// y[r] = x[x_row[r]] W_g^T, W_g [N or 2N, K] the matrix of row r's group.  swiglu: y = T(silu(s gate) * (s up)) with s = x_scale[r]; else
+// y = the sums, as T or (out_f32) as they are.  tile_rows 16, 32 or 64; rows: rows of the product, x_rows: rows of x.
+int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, int out_f32, const RowGroups& g, hipStream_t s);
 
 }  // namespace raven

@@ -35,18 +35,23 @@ struct MidArgs {
     raven_epilogue epi;    // EPI_FREE only
     int rope_on;           // EPI_PLAIN: the rope epilogue instead of y
     RopeAppend rope;
+    RowGroups groups;      // GROUPED only
 };
 
 __device__ __align__(16) unsigned int g_mid_zero[4];  // what a 16-byte piece past the end of K is loaded from
 
-// Four neighbouring output columns n .. n + 3 of token row m
-template <int EPI>
-__device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 v, f32x4 up) {
+// Four neighbouring output columns n .. n + 3 of token row m; xs: the factor of a grouped SwiGLU row
+template <int EPI, bool GROUPED = false>
+__device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 v, f32x4 up, float xs = 1.f) {
     const int64_t at = (int64_t)m * a.N + n;
     if constexpr (EPI == EPI_SWIGLU) {
         bf16 o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            if (GROUPED) {
+                o[i] = from_f32<bf16>(silu_f32(v[i] * xs) * (up[i] * xs));
+                continue;
+            }
             const float g = round_to<bf16>(v[i]), u = round_to<bf16>(up[i]);
             o[i] = from_f32<bf16>(round_to<bf16>(silu_f32(g)) * u);
         }
@@ -107,14 +112,18 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 
     }
 }
 
-template <int EPI, int NT, int MT, int NS>
-__global__ __launch_bounds__(512) void gemm_mid_kernel(MidArgs a) {
+// GROUPED: row groups with a weight matrix each; a unit works on a copy of the arguments cut to its group's rows
+template <int EPI, int WN, int WM, int NT, int MT, int NS, bool GROUPED = false>
+__global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
-    constexpr int LPW = NT / 2 + MT;  // kilobyte pieces (8 rows x 128 bytes) a wave requests per step: NT / 2 of W, MT of X
-    static_assert(NT % 2 == 0 && (NS - 1) * LPW < 64, "the wait counter holds 63 requests");
+    constexpr int NW = WN * WM, XROWS = 16 * WM * MT, XP = XROWS / 8;
+    // kilobyte pieces (8 rows x 128 bytes) a wave requests per step; with fewer token pieces than waves some are requested twice
+    constexpr int WPW = 2 * NT / WM, XPW = XP >= NW ? XP / NW : 1, LPW = WPW + XPW;
+    static_assert(NT % 2 == 0 && (2 * NT) % WM == 0 && (XP % NW == 0 || NW % XP == 0) && (NS - 1) * LPW < 64, "whole pieces; the wait counter holds 63 requests");
     extern __shared__ __align__(1024) unsigned char smem[];
 
     // which unit: K slices outermost, then bands of eight token tiles, so that the units of an XCD (ids congruent modulo 8) are neighbours
+    if (GROUPED) a.tiles_m = *a.groups.used;
     const int mn = a.tiles_m * a.tiles_n, n_units = mn * a.ks;
     const int per_xcd = (n_units + 7) >> 3;
     const int logical = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
@@ -122,26 +131,38 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(MidArgs a) {
     const int slice = logical / mn, in_slice = logical - slice * mn;
     constexpr int GROUP = 8;
     const int band = in_slice / (GROUP * a.tiles_n), first_m = band * GROUP, gsz = min(a.tiles_m - first_m, GROUP);
-    const int in_band = in_slice - band * GROUP * a.tiles_n, tile_n = in_band / gsz, tile_m = first_m + (in_band - tile_n * gsz);
+    const int in_band = in_slice - band * GROUP * a.tiles_n, tile_n = in_band / gsz;
+    int tile_m = first_m + (in_band - tile_n * gsz);
+    const int* x_row = nullptr;
+    if constexpr (GROUPED) {
+        const int g = a.groups.group_of[tile_m], row = a.groups.group_row[tile_m];
+        a.M = a.groups.group_end[tile_m] - row;
+        a.w = g == a.groups.extra_group ? a.groups.w_extra : a.w + g * a.groups.w_stride;
+        a.y = static_cast<char*>(a.y) + (int64_t)row * a.N * (a.out_f32 ? 4 : 2);
+        if (a.groups.x_scale) a.groups.x_scale += row;
+        if (a.groups.x_row) x_row = a.groups.x_row + row;
+        else a.x0 += (int64_t)row * a.ldx;
+        tile_m = 0;
+    }
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wn = wave & 1, wm = wave >> 1;
+    const int wn = wave % WN, wm = wave / WN;
     const int K = a.K0 + a.K1, nk = (K + 63) >> 6;
     const int k0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * slice / a.ks));
     const int n_steps = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * (slice + 1) / a.ks)) - k0;
     const int n0 = tile_n * a.cols, ncols = min(a.cols, a.N - n0), m0 = tile_m * a.bm;
-    const int wbytes = a.wrows * 128, stage = wbytes + MT * 8192;
+    const int wbytes = a.wrows * 128, stage = wbytes + XROWS * 128;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_byte*)smem;
 
-    // ---- global side: request i of a wave is piece 8 i + wave, rows 8 (8 i + wave) ..+7 of the weight tile (i < NT / 2) or of the token
+    // ---- global side: request i of a wave is piece NW i + wave, rows 8 (NW i + wave) ..+7 of the weight tile (i < WPW) or of the token
     // rows; the lane that fills position s of row r fetches piece s ^ ((r >> 1) & 7) of the row's 128-byte step
     const int colp = ((lane & 7) ^ ((lane >> 4) | (4 * (wave & 1)))) * 8;
     unsigned goff[LPW];
     unsigned dst[LPW];  // offset inside a stage; weight pieces past the tile land behind the ring
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
-        const bool is_w = i < NT / 2;
-        const int piece = 8 * (is_w ? i : i - NT / 2) + wave, r = piece * 8 + (lane >> 3);
+        const bool is_w = i < WPW;
+        const int piece = is_w ? NW * i + wave : (NW * (i - WPW) + wave) % XP, r = piece * 8 + (lane >> 3);
         if (is_w) {
             int row;
             if (SWIGLU) row = n0 + min((r >> 5) * 16 + (r & 15), ncols - 1) + ((r & 16) ? a.N : 0);
@@ -149,7 +170,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(MidArgs a) {
             goff[i] = (unsigned)row * (2u * a.ldw) + 2u * colp;
             dst[i] = piece * 1024;
         } else {
-            goff[i] = (unsigned)min(m0 + r, a.M - 1) * (2u * a.ldx) + 2u * colp;
+            int row = min(m0 + r, a.M - 1);
+            if (GROUPED && x_row) row = x_row[row];
+            goff[i] = (unsigned)row * (2u * a.ldx) + 2u * colp;
             dst[i] = wbytes + piece * 1024;
         }
     }
@@ -163,8 +186,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(MidArgs a) {
         const bool whole = c0 + 64 <= a.K0 || (c0 >= a.K0 && c0 + 64 <= K);  // the 64 columns lie in one segment and below K
 #pragma unroll
         for (int i = decltype(first_tag)::value; i < decltype(last_tag)::value; ++i) {
-            const bool is_w = i < NT / 2;
-            const bool spare = is_w && (8 * i + wave) * 8 >= a.wrows;
+            const bool is_w = i < WPW;
+            const bool spare = is_w && (NW * i + wave) * 8 >= a.wrows;
             const unsigned to = __builtin_amdgcn_readfirstlane(lds_base + (spare ? NS * stage : o + (int)dst[i]));
             if (whole) {
                 const char* base = (is_w ? w0 : (c0 < a.K0 ? x0 : x1)) + 2 * c0;
@@ -305,7 +328,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(MidArgs a) {
                 *reinterpret_cast<f32x4*>(p) = v;
                 if (SWIGLU) *reinterpret_cast<f32x4*>(p + a.N) = up;
             } else {
-                mid_store<EPI>(a, m, n0 + col, v, up);
+                const float xs = GROUPED && SWIGLU ? a.groups.x_scale[m] : 1.f;
+                mid_store<EPI, GROUPED>(a, m, n0 + col, v, up, xs);
             }
         }
         wave_sync();
@@ -443,7 +467,7 @@ static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
     constexpr int NS = mid_stages(NT, MT);
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, NT, MT, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, 2, 4, NT, MT, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) {
             raven_host::set_error("gemm (mid): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
@@ -453,7 +477,7 @@ static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
     const size_t lds = (size_t)NS * (a.wrows * 128 + MT * 8192) + (a.wrows < 32 * NT ? 1024 : 0);
     RAVEN_REQUIRE(lds <= (size_t)kLds && a.wrows <= 32 * NT && a.bm <= 64 * MT, "gemm (mid): a unit of %d x %d does not fit", a.cols, a.bm);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n * a.ks;
-    gemm_mid_kernel<EPI, NT, MT, NS><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
+    gemm_mid_kernel<EPI, 2, 4, NT, MT, NS><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
     return raven_host::check_launch("gemm (mid)");
 }
 
@@ -502,6 +526,59 @@ int mid_gemm(const ProductArgs& q, const MidPlan& p, void* workspace, hipStream_
     if (q.epi) return launch_mid<EPI_FREE>(a, p, s, finish);
     if (q.swiglu) return launch_mid<EPI_SWIGLU>(a, p, s, finish);
     return launch_mid<EPI_PLAIN>(a, p, s, finish);
+}
+
+template <int EPI, int WN, int WM, int NT, int MT, int NS>
+static int launch_grouped(const MidArgs& a, hipStream_t s) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, WN, WM, NT, MT, NS, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        if (e != hipSuccess) {
+            raven_host::set_error("gemm (grouped): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+            return (int)e;
+        }
+        attr_set = true;
+    }
+    const size_t lds = (size_t)NS * (a.wrows + 16 * WM * MT) * 128 + (a.wrows < 16 * WN * NT ? 1024 : 0);
+    RAVEN_REQUIRE(lds <= (size_t)kLds && a.wrows <= 16 * WN * NT, "gemm (grouped): a unit of %d columns does not fit", a.cols);
+    const int64_t units = (int64_t)a.tiles_m * a.tiles_n;
+    RAVEN_REQUIRE(units < (1 << 28), "gemm (grouped): too many units");
+    gemm_mid_kernel<EPI, WN, WM, NT, MT, NS, true><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(64 * WN * WM), lds, s>>>(a);
+    return raven_host::check_launch("gemm (grouped)");
+}
+
+// Tiles of 16 and 32 rows: four waves side by side along the weight rows -- with few token rows the eight waves of the larger tiles would
+// read mostly rows that do not exist out of LDS --, four stages of 18 or 20 KB, two workgroups per CU, so that one streams while the
+// other fills its ring or stores (a unit of an expert of 768 channels has 12 to 32 K steps).
+template <int EPI>
+static int launch_grouped_rows(const MidArgs& a, hipStream_t s) {
+    switch (a.bm) {
+        case 16: return launch_grouped<EPI, 4, 1, 2, 1, 4>(a, s);
+        case 32: return launch_grouped<EPI, 4, 1, 2, 2, 4>(a, s);
+        case 64: return launch_grouped<EPI, 2, 4, 4, 1, 3>(a, s);
+        default: RAVEN_REQUIRE(false, "gemm (grouped): tiles of %d rows", a.bm);
+    }
+}
+
+int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, int out_f32, const RowGroups& g, hipStream_t s) {
+    RAVEN_REQUIRE(x && w && y && g.group_of && g.group_row && g.group_end && g.used && g.n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 &&
+                      (!swiglu || (g.x_scale && !out_f32)) && (g.extra_group < 0 || g.w_extra), "gemm (grouped): bad arguments");
+    RAVEN_REQUIRE((int64_t)x_rows * K < (1ll << 31) && (int64_t)N * 2 * K < (1ll << 31) && (int64_t)rows * N < (1ll << 40), "gemm (grouped): too large");
+    MidArgs a{};
+    a.w = static_cast<const bf16*>(w);
+    a.x0 = static_cast<const bf16*>(x);
+    a.y = y;
+    a.M = rows; a.N = N; a.K0 = K; a.ldw = K; a.ldx = K; a.out_f32 = out_f32;
+    const int side = swiglu ? 2 : 1, cap = 128 / side;
+    const int tiles_n = (N + cap - 1) / cap;
+    a.cols = ((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
+    if (a.cols < cap / 2) a.cols = cap / 2;
+    a.wrows = (a.cols + 15) / 16 * 16 * side;
+    a.tiles_n = (N + a.cols - 1) / a.cols;
+    a.bm = g.tile_rows; a.tiles_m = g.n_tiles; a.ks = 1;
+    a.epi.scale = 1.f;
+    a.groups = g;
+    return swiglu ? launch_grouped_rows<EPI_SWIGLU>(a, s) : launch_grouped_rows<EPI_FREE>(a, s);
 }
 
 }  // namespace raven

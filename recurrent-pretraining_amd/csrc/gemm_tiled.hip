@@ -63,14 +63,7 @@ struct TiledArgs {
     int out_f32;
     int tiles_m, tiles_n;
     raven_epilogue epi;    // EPI_FREE only (y and residual [M, ldy])
-    // Products of row groups with a weight matrix each (grouped_gemm): tile row t multiplies rows group_row[t] .. group_row[t] + BM - 1
-    // (below group_end[t]) with the matrix of group group_of[t]; group_of < 0: no such tile
-    struct Groups {
-        const int *group_of, *group_row, *group_end;
-        const int* x_row;        // row of x0 behind a row of the product, or null: the same
-        const float* x_scale;    // SwiGLU: factor of a row of x0, applied to its sums
-        int64_t w_stride;        // elements between two groups' matrices
-    } groups;
+    RowGroups groups;      // GROUPED only (grouped_gemm)
     int rope_on;           // the epilogue below instead of y
     RopeAppend rope;       // (gemm_common.h)
 };
@@ -321,10 +314,9 @@ __device__ __forceinline__ void store_tiles_rope(const TiledArgs& a, const f32x4
 
 __device__ __align__(16) unsigned int g_zero_piece[4];  // what a 16-byte piece past the end of K is loaded from
 
-// Cuts the arguments to the rows and the matrix of tile row tile_m's group; false: no such tile
-__device__ __forceinline__ bool enter_group(TiledArgs& a, int tile_m, const int*& x_row) {
+// Cuts the arguments to the rows and the matrix of tile row tile_m's group
+__device__ __forceinline__ void enter_group(TiledArgs& a, int tile_m, const int*& x_row) {
     const int g = a.groups.group_of[tile_m];
-    if (g < 0) return false;
     const int row = a.groups.group_row[tile_m];
     a.M = a.groups.group_end[tile_m] - row;
     a.w += g * a.groups.w_stride;
@@ -332,11 +324,9 @@ __device__ __forceinline__ bool enter_group(TiledArgs& a, int tile_m, const int*
     if (a.groups.x_scale) a.groups.x_scale += row;
     if (a.groups.x_row) x_row = a.groups.x_row + row;
     else a.x0 += (int64_t)row * a.ldx;
-    return true;
 }
 
-// GROUPED: row groups with a weight matrix each (TiledArgs::groups); a tile works on a copy of the arguments cut to its group's rows
-template <int EPI, int TM, int TN, int WM = 2, int WN = 4, bool GROUPED = false>
+template <int EPI, int TM, int TN, int WM = 2, int WN = 4>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
@@ -357,19 +347,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
     const int n_tiles = a.tiles_m * a.tiles_n;
     const int per_xcd = (n_tiles + 7) >> 3;
     const int logical = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-    if (logical >= n_tiles) return;
+    if (((int)blockIdx.x >> 3) >= per_xcd || logical >= n_tiles) return;
     constexpr int GROUP = 8;
     const int band = logical / (GROUP * a.tiles_n);
     const int first_m = band * GROUP;
     const int gsz = min(a.tiles_m - first_m, GROUP);
     const int in_band = logical - band * GROUP * a.tiles_n;
     const int tile_n = in_band / gsz;
-    int tile_m = first_m + (in_band - tile_n * gsz);
-    const int* x_row = nullptr;
-    if constexpr (GROUPED) {
-        if (!enter_group(a, tile_m, x_row)) return;
-        tile_m = 0;
-    }
+    const int tile_m = first_m + (in_band - tile_n * gsz);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -393,7 +378,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
             else row = min(tile_n * BN + r, a.N - 1);
         } else {
             row = min(tile_m * BM + (r - BN), a.M - 1);
-            if (GROUPED && x_row) row = x_row[row];
         }
         goff[p] = (unsigned)row * ld2 + 2u * col8;
     }
@@ -573,7 +557,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
         }
     }
     if (a.out_f32) store_tiles<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wm, wn, l16, q4);
-    else store_tiles_lds<EPI, TM, TN, WM, WN, GROUPED>(a, acc, tile_m, tile_n, wave, lane, lds_base);
+    else store_tiles_lds<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wave, lane, lds_base);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -592,6 +576,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
 //     of step k + 1 have landed, and its slice 0 is read under the last products.  A request has between 1.4 and 2.4
 //     steps to land.
 // Same products in the same order per accumulator as the eight-wave kernel: bit-identical results.
+// GROUPED: row groups with a weight matrix each (TiledArgs::groups); a tile works on a copy of the arguments cut to its group's rows
 template <int EPI, bool GROUPED = false>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(TiledArgs a) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
@@ -602,10 +587,11 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(TiledArgs a) {
     constexpr int PPW = 8;                        // pieces (8 rows x 128 bytes) a wave requests per operand and step
     extern __shared__ __align__(1024) unsigned char smem[];
 
+    if (GROUPED) a.tiles_m = *a.groups.used;
     const int n_tiles = a.tiles_m * a.tiles_n;
     const int per_xcd = (n_tiles + 7) >> 3;
     const int logical = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-    if (logical >= n_tiles) return;
+    if (((int)blockIdx.x >> 3) >= per_xcd || logical >= n_tiles) return;
     constexpr int GROUP = 8;
     const int band = logical / (GROUP * a.tiles_n);
     const int first_m = band * GROUP;
@@ -615,7 +601,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(TiledArgs a) {
     int tile_m = first_m + (in_band - tile_n * gsz);
     const int* x_row = nullptr;
     if constexpr (GROUPED) {
-        if (!enter_group(a, tile_m, x_row)) return;
+        enter_group(a, tile_m, x_row);
         tile_m = 0;
     }
 
@@ -817,26 +803,26 @@ int g_tiled_min_rows = 33;  // raven_set_tuning("gemm_tiled_min_rows"): fewest r
 int g_tiled_variant = 0;    // raven_set_tuning("gemm_tiled_variant"): 0 = by shape, 1 = 256 x 256 tiles, 2 = 128 x 128 tiles, 3 = 256 x 256 tiles by the eight-wave kernel
 int g_tiled_split_tail = 1; // raven_set_tuning("gemm_tiled_split_tail"): 0 = never hand the last round's tile columns to 128 x 128 tiles
 
-template <int EPI, int TM, int TN, int WM = 2, int WN = 4, bool GROUPED = false>
+template <int EPI, int TM, int TN, int WM = 2, int WN = 4>
 static int launch_tiled(TiledArgs a, hipStream_t s) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BN_OUT = SWIGLU ? BN / 2 : BN;
     constexpr size_t lds = (size_t)2 * (BM + BN) * 128;
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<EPI, TM, TN, WM, WN, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<EPI, TM, TN, WM, WN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             raven_host::set_error("gemm (tiled): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
         }
         attr_set = true;
     }
-    if (!GROUPED) a.tiles_m = (a.M + BM - 1) / BM;
+    a.tiles_m = (a.M + BM - 1) / BM;
     a.tiles_n = (a.N + BN_OUT - 1) / BN_OUT;
     const int64_t n_tiles = (int64_t)a.tiles_m * a.tiles_n;
     RAVEN_REQUIRE(n_tiles < (1 << 28), "gemm (tiled): too many tiles (M=%d N=%d)", a.M, a.N);
     const unsigned grid = (unsigned)((n_tiles + 7) / 8 * 8);
-    gemm_tiled_kernel<EPI, TM, TN, WM, WN, GROUPED><<<dim3(grid), dim3(64 * WM * WN), lds, s>>>(a);
+    gemm_tiled_kernel<EPI, TM, TN, WM, WN><<<dim3(grid), dim3(64 * WM * WN), lds, s>>>(a);
     return raven_host::check_launch("gemm (tiled MFMA)");
 }
 
@@ -985,25 +971,21 @@ int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int 
     return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, workspace, workspace_bytes, s, &epi);
 }
 
-// Products of row groups (tile_rows = 128 or 256 rows to a tile row): y[r] = x[x_row[r]] W_g^T, W_g = w + g * w_stride [N or 2N, K] of the group that row r of the
-// product belongs to.  swiglu: y = T(silu(s gate) * (s up)) with s = x_scale[r]; else y = T(sums).  n_tiles: entries of the three tile
-// tables (unused ones have group_of < 0); rows: rows of the product, x_rows: rows of x.
-int grouped_gemm(const void* x, int x_rows, const void* w, int64_t w_stride, void* y, int rows, int N, int K, int swiglu, const int* group_of,
-                 const int* group_row, const int* group_end, int n_tiles, int tile_rows, const int* x_row, const float* x_scale, hipStream_t s) {
-    RAVEN_REQUIRE(x && w && y && group_of && group_row && group_end && n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (!swiglu || x_scale),
-                  "gemm (grouped): bad arguments");
+// mid_grouped (gemm_common.h) in tiles of 256 rows by the ring kernel
+int ring_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, const RowGroups& g, hipStream_t s) {
+    RAVEN_REQUIRE(x && w && y && g.group_of && g.group_row && g.group_end && g.used && g.n_tiles > 0 && g.tile_rows == 256 && g.extra_group < 0 && N > 0 &&
+                      N % 8 == 0 && K > 0 && K % 8 == 0 && (!swiglu || g.x_scale), "gemm (grouped): bad arguments");
     RAVEN_REQUIRE((int64_t)x_rows * K < (1ll << 31) && (int64_t)N * 2 * K < (1ll << 31) && (int64_t)rows * N < (1ll << 40), "gemm (grouped): too large");
     TiledArgs a{};
     a.w = static_cast<const bf16*>(w);
     a.x0 = static_cast<const bf16*>(x);
     a.y = y;
-    a.M = rows; a.N = N; a.K0 = K; a.out_f32 = 0;
+    a.M = rows; a.N = N; a.K0 = K;
     a.ldy = N; a.up_off = N; a.ldw = K; a.ldx = K;
-    a.tiles_m = n_tiles;
+    a.tiles_m = g.n_tiles;
     a.epi.scale = 1.f;
-    a.groups = TiledArgs::Groups{group_of, group_row, group_end, x_row, x_scale, w_stride};
-    if (tile_rows == 256) return swiglu ? launch_ring<EPI_SWIGLU, true>(a, s) : launch_ring<EPI_FREE, true>(a, s);
-    return swiglu ? launch_tiled<EPI_SWIGLU, 2, 1, 2, 4, true>(a, s) : launch_tiled<EPI_FREE, 2, 1, 2, 4, true>(a, s);
+    a.groups = g;
+    return swiglu ? launch_ring<EPI_SWIGLU, true>(a, s) : launch_ring<EPI_FREE, true>(a, s);
 }
 
 // A chunk's q | k | v product (wqkv: [3 * nh * hd, K]) whose epilogue adds the q / k bias, applies RoPE and writes q to

@@ -2,23 +2,27 @@
 //     x += sum over the chosen experts of W_down ( silu(s W_gate h) * (s W_up h) )  +  sigmoid(g) W_down' ( silu(W_gate' h) * (W_up' h) )
 // s = sigmoid(router logit): the factor of an expert's input is applied to the sums of its first two products, which is the same.
 //
-// Few rows (and fp32): moe_up_kernel forms the gated activations of a row's experts and of the shared one side by side, moe_down_kernel
+// One to a handful of rows (and fp32): moe_up_kernel forms the gated activations of a row's experts and of the shared one side by side, moe_down_kernel
 // multiplies them by the down matrices and adds to the stream.  The first picks the row's experts itself from its logits -- a handful
 // of wave reductions -- so no routing launch stands in between; for a single row it also takes the norm of the stream as a prologue.
-// bf16 chunks: the rows are sorted by expert (moe_pick_kernel, moe_sort_kernel) and the experts run as one grouped product on the
-// matrix cores (gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of its own, and
-// moe_combine_kernel adds a token's slots and its shared expert to the stream in a fixed order.
+// More bf16 rows: the rows are sorted by expert (moe_route_kernel, or moe_pick_kernel and moe_sort_kernel) and the experts run as one
+// grouped product on the matrix cores (gemm_mid.hip, gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of
+// its own, and moe_combine_kernel adds a token's slots and its shared expert to the stream in a fixed order.  So an expert's weights
+// are read once and not once per row that picked it: 20 rows over 64 experts of 768 channels at width 2048, 6 each, read
+// 55 experts instead of 120 (246 us before, 124 now).
 
+#include "gemm_common.h"
 #include "row_helpers.h"
 
 namespace raven {
 
-int grouped_gemm(const void* x, int x_rows, const void* w, int64_t w_stride, void* y, int rows, int N, int K, int swiglu, const int* group_of,
-                 const int* group_row, const int* group_end, int n_tiles, int tile_rows, const int* x_row, const float* x_scale, hipStream_t s);
+int ring_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, const RowGroups& g, hipStream_t s);
 
 constexpr int kMaxExperts = 1024, kMaxTop = 32;
-constexpr int kBigTileRows = 320;  // rows per expert from which the grouped products take 256-row tiles
+constexpr int kBigTileRows = 110;  // rows per expert from which the grouped products take 256-row tiles
 constexpr int kPickRows = 32;  // tokens a workgroup of the two sorting kernels owns
+constexpr double kMoeBytesAgain = 25e6;
+constexpr int kRouteRows = 64, kRoutePairs = 2048;  // tokens and (token, expert) pairs up to which one workgroup picks and sorts
 
 struct MoeArgs {
     const void *h, *up, *down, *shared_up, *shared_down;
@@ -35,10 +39,11 @@ struct MoeArgs {
     int *slot_of;           // [M, top]: row of the grouped product
     int *slot_row;          // [M * top]: token of a slot
     float* slot_scale;      // [M * top]
-    int *group_of, *group_row, *group_end;
-    int n_tiles, tile_rows;
+    int *group_of, *group_row, *group_end, *used;
+    int tile_rows;
     int* block_count;       // [ceil(M / kPickRows), experts]: pairs of a workgroup's tokens
-    const bf16* y;          // [M * top, ld]
+    int fold;               // the shared expert is one more group (rows M * top ..+M - 1 of the product): extra group `experts`
+    const void* y;          // [M * top, ld] of T, or float when fold
     const float* ys;        // [M, ld] or null
 };
 
@@ -258,7 +263,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeArgs a) {
         }
         int used = 0;
         for (int w = 0; w < 16; ++w) used += wave_sums[1][w];
-        for (int i = used + tid; i < a.n_tiles; i += 1024) a.group_of[i] = -1;
+        if (tid == 0) *a.used = used;
     }
     __syncthreads();
     const int lo = me * kPickRows * a.top, hi = min(a.M, (me + 1) * kPickRows) * a.top;
@@ -270,32 +275,116 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeArgs a) {
     }
 }
 
+// Both of the above in one workgroup, for few rows; with fold the shared expert's rows follow as one more group of factor one
+__global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
+    __shared__ int count[kMaxExperts], start[kMaxExperts], pick[kRoutePairs], wave_sums[2][16];
+    __shared__ float scale[kRoutePairs];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, pairs = a.M * a.top;
+    count[tid] = 0;
+    __syncthreads();
+    for (int m = wave; m < a.M; m += 16) {
+        int e;
+        float s;
+        pick_experts(a.logits + (int64_t)m * a.ldl, a.experts, a.top, e, s);
+        if (lane < a.top) {
+            pick[m * a.top + lane] = e;
+            scale[m * a.top + lane] = s;
+            atomicAdd(&count[e], 1);
+        }
+    }
+    __syncthreads();
+    const int rows = count[tid], tiles = (rows + a.tile_rows - 1) / a.tile_rows;
+    int r = rows, t = tiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int pr = __shfl_up(r, d, 64), pt = __shfl_up(t, d, 64);
+        if (lane >= d) {
+            r += pr;
+            t += pt;
+        }
+    }
+    if (lane == 63) {
+        wave_sums[0][wave] = r;
+        wave_sums[1][wave] = t;
+    }
+    __syncthreads();
+    int used = 0;
+    for (int w = 0; w < 16; ++w) {
+        if (w < wave) {
+            r += wave_sums[0][w];
+            t += wave_sums[1][w];
+        }
+        used += wave_sums[1][w];
+    }
+    const int first = r - rows, first_tile = t - tiles;
+    start[tid] = first;
+    for (int i = 0; i < tiles; ++i) {
+        a.group_of[first_tile + i] = tid;
+        a.group_row[first_tile + i] = first + i * a.tile_rows;
+        a.group_end[first_tile + i] = min(first + (i + 1) * a.tile_rows, first + rows);
+    }
+    const int shared_tiles = a.fold ? (a.M + a.tile_rows - 1) / a.tile_rows : 0;
+    for (int i = tid; i < shared_tiles; i += 1024) {
+        a.group_of[used + i] = a.experts;
+        a.group_row[used + i] = pairs + i * a.tile_rows;
+        a.group_end[used + i] = pairs + min((i + 1) * a.tile_rows, a.M);
+    }
+    if (tid == 0) *a.used = used + shared_tiles;
+    __syncthreads();
+    for (int i = tid; i < pairs; i += 1024) {
+        const int slot = atomicAdd(&start[pick[i]], 1);
+        a.slot_of[i] = slot;
+        a.slot_row[slot] = i / a.top;
+        a.slot_scale[slot] = scale[i];
+    }
+    if (a.fold)
+        for (int m = tid; m < a.M; m += 1024) {
+            a.slot_row[pairs + m] = m;
+            a.slot_scale[pairs + m] = 1.f;
+        }
+}
+
+template <typename Y>
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int per = a.ld / 4;
     if (i >= (int64_t)a.M * per) return;
     const int m = (int)(i / per), c = 4 * (int)(i % per);
-    f32x4 x = load4(a.x + (int64_t)m * a.ld + c);
-    for (int k0 = 0; k0 < a.top; k0 += 4) {
-        f32x4 v[4];
+    const Y* y = static_cast<const Y*>(a.y);
+    f32x4 x = load4(a.x + (int64_t)m * a.ld + c), shared = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float gate = a.ys ? sigmoid_f32(a.logits[(int64_t)m * a.ldl + a.experts]) : 0.f;
+    if (a.ys) shared = load4(a.ys + (int64_t)m * a.ld + c);
+    for (int k0 = 0; k0 < a.top; k0 += 8) {
+        f32x4 v[8];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = load4(a.y + (int64_t)a.slot_of[m * a.top + min(k0 + k, a.top - 1)] * a.ld + c);
+        for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)a.slot_of[m * a.top + min(k0 + k, a.top - 1)] * a.ld + c);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < 8; ++k)
             if (k0 + k < a.top) x += v[k];
     }
-    if (a.ys) x += load4(a.ys + (int64_t)m * a.ld + c) * sigmoid_f32(a.logits[(int64_t)m * a.ldl + a.experts]);
+    if (a.ys) x += shared * gate;
     store4(a.x + (int64_t)m * a.ld + c, x);
 }
 
-// rows from which a chunk's experts run as a grouped product: once they share weights (or there are enough rows anyway)
-static bool moe_grouped(const raven_moe* m, int M, int dtype) {
-    return dtype == RAVEN_BF16 && M > 8 && ((int64_t)M * m->top >= 2 * m->experts || M > 128);
+// What runs the experts of M rows.  A chunk -- once its rows share weights (two per expert), or there are enough rows anyway -- keeps its slots in T
+// and runs the shared expert as a product of its own.  Fewer rows keep slots and sums in float, as the row kernels do, and take the
+// grouped product once reading each expert once saves more than its two further launches cost.  us at width 2048 (64 experts of 768
+// channels, 6 per row and a shared one), row kernels / grouped: 2 rows 31 / 34, 3: 45 / 42, 4: 59 / 55, 8: 105 / 78, 20: 246 / 124;
+// width 1024: 4 rows 22 / 26, 6: 29 / 27, 8: 38 / 31, 20: 80 / 40 -- the lines cross where rows would read 25 MB again.
+enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
+static MoePath moe_path(const raven_moe* m, int M, int ld, int dtype) {
+    if (dtype != RAVEN_BF16) return kMoeRows;
+    const double pairs = (double)M * m->top;
+    if (M > 8 && (pairs >= 2.0 * m->experts || M > 128)) return kMoeChunk;
+    const bool fold = !m->shared_up || m->shared_ff == m->ff;
+    if (!fold || M < 2 || M > kRouteRows || pairs > kRoutePairs) return kMoeRows;
+    const double touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), again = pairs - touched + (m->shared_up ? M - 1 : 0);
+    return again * 6.0 * ld * m->ff > kMoeBytesAgain ? kMoeFew : kMoeRows;
 }
 
 struct MoeChunk {
-    int *pick, *slot_of, *slot_row, *group_of, *group_row, *group_end, *block_count;
-    bf16* y;
+    int *pick, *slot_of, *slot_row, *group_of, *group_row, *group_end, *used, *block_count;
+    void* y;
     float *pick_scale, *slot_scale, *ys;
     char *act, *sact, *lin;
     size_t lin_bytes;
@@ -310,25 +399,35 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, char* base
         return p;
     };
     MoeChunk c{};
-    if (!moe_grouped(m, M, dtype)) {
+    const MoePath path = moe_path(m, M, ld, dtype);
+    if (path == kMoeRows) {
         c.act = take((size_t)M * (m->top * (size_t)m->ff + m->shared_ff) * es);
         c.pick = (int*)take(pairs * 4);
     } else {
-        // 256-row tiles (twice the speed per row) once an expert fills most of two of them on average
-        c.tile_rows = pairs >= (size_t)kBigTileRows * m->experts ? 256 : 128;
-        c.n_tiles = (int)(pairs / c.tile_rows) + m->experts;
+        const bool fold = path == kMoeFew && m->shared_up;
+        const size_t rows = pairs + (fold ? M : 0);
+        // The smallest tile that most experts' rows fit into; 256 (by the ring kernel, twice the speed per row) from an average of 110 on.
+        // us for all launches of a mixture, width 2048, tiles of 16 / 32 / 64 / 256 rows: 100 tokens 169 / 163 / 167 / 218, 500:
+        // 232 / 196 / 181 / 232, 1000: 344 / 255 / 218 / 249, 1500: 474 / 340 / 282 / 272, 4096: - / 695 / 518 / 394; width 1024, 500
+        // tokens: 80 / 70 / 63 / 83, 1500: 144 / 109 / 94 / 96.  (128-row tiles of eight waves, as before: 230 at 500, 327 at 1500.)
+        const size_t mean = pairs / m->experts;
+        c.tile_rows = path == kMoeFew || mean <= 6 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows ? 64 : 256;
+        c.n_tiles = (int)(pairs / c.tile_rows) + m->experts + (fold ? (M + c.tile_rows - 1) / c.tile_rows : 0);
         c.pick = (int*)take(pairs * 4);
         c.pick_scale = (float*)take(pairs * 4);
         c.slot_of = (int*)take(pairs * 4);
-        c.slot_row = (int*)take(pairs * 4);
-        c.slot_scale = (float*)take(pairs * 4);
+        c.slot_row = (int*)take(rows * 4);
+        c.slot_scale = (float*)take(rows * 4);
         c.group_of = (int*)take((size_t)c.n_tiles * 4);
         c.group_row = (int*)take((size_t)c.n_tiles * 4);
         c.group_end = (int*)take((size_t)c.n_tiles * 4);
+        c.used = (int*)take(4);
         c.block_count = (int*)take((size_t)((M + kPickRows - 1) / kPickRows) * m->experts * 4);
-        c.act = take(pairs * m->ff * es);
-        c.y = (bf16*)take(pairs * ld * sizeof(bf16));
-        if (m->shared_up) {
+        c.act = take(rows * m->ff * es);
+        c.y = take(rows * ld * (path == kMoeFew ? sizeof(float) : sizeof(bf16)));
+        if (fold) {
+            c.ys = static_cast<float*>(c.y) + pairs * ld;
+        } else if (m->shared_up) {
             c.sact = take((size_t)M * m->shared_ff * es);
             c.ys = (float*)take((size_t)M * ld * sizeof(float));
             c.lin_bytes = raven_linear_workspace_bytes(M, ld > 2 * m->shared_ff ? ld : 2 * m->shared_ff);
@@ -380,28 +479,43 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
     a.h = h; a.up = m->up; a.down = m->down; a.shared_up = m->shared_up; a.shared_down = m->shared_down;
     a.logits = logits; a.x = x; a.act = c.act; a.norm = norm; a.dim = dim; a.eps = eps; a.pick = c.pick;
     a.M = M; a.ld = ld; a.ldl = m->logit_ld; a.experts = m->experts; a.top = m->top; a.ff = m->ff; a.sff = m->shared_ff;
-    if (!moe_grouped(m, M, dtype)) {
+    const MoePath path = moe_path(m, M, ld, dtype);
+    if (path == kMoeRows) {
         RAVEN_REQUIRE(M <= 65535, "moe: %d rows in one call", M);
         return dtype == RAVEN_BF16 ? run_moe_rows<bf16>(a, s) : run_moe_rows<float>(a, s);
     }
     const int pairs = M * m->top, blocks = (M + kPickRows - 1) / kPickRows;
+    const bool fold = path == kMoeFew && m->shared_up, few = path == kMoeFew;
+    const int rows = pairs + (fold ? M : 0);
     a.pick_scale = c.pick_scale; a.slot_of = c.slot_of; a.slot_row = c.slot_row; a.slot_scale = c.slot_scale;
-    a.group_of = c.group_of; a.group_row = c.group_row; a.group_end = c.group_end; a.n_tiles = c.n_tiles; a.tile_rows = c.tile_rows; a.block_count = c.block_count;
-    a.y = c.y; a.ys = c.ys;
-    moe_pick_kernel<<<dim3(blocks), dim3(1024), 0, s>>>(a);
-    moe_sort_kernel<<<dim3(blocks), dim3(1024), 0, s>>>(a);
+    a.group_of = c.group_of; a.group_row = c.group_row; a.group_end = c.group_end; a.used = c.used; a.tile_rows = c.tile_rows; a.block_count = c.block_count;
+    a.y = c.y; a.ys = c.ys; a.fold = fold;
+    if (few || (M <= kRouteRows && pairs <= kRoutePairs)) {
+        moe_route_kernel<<<dim3(1), dim3(1024), 0, s>>>(a);
+    } else {
+        moe_pick_kernel<<<dim3(blocks), dim3(1024), 0, s>>>(a);
+        moe_sort_kernel<<<dim3(blocks), dim3(1024), 0, s>>>(a);
+    }
     if (const int rc = raven_host::check_launch("moe (sort)")) return rc;
-    if (const int rc = grouped_gemm(h, M, m->up, (int64_t)2 * m->ff * ld, c.act, pairs, m->ff, ld, 1, c.group_of, c.group_row, c.group_end, c.n_tiles, c.tile_rows, c.slot_row,
-                                    c.slot_scale, s)) return rc;
-    if (const int rc = grouped_gemm(c.act, pairs, m->down, (int64_t)ld * m->ff, c.y, pairs, ld, m->ff, 0, c.group_of, c.group_row, c.group_end, c.n_tiles, c.tile_rows, nullptr,
-                                    nullptr, s)) return rc;
-    if (m->shared_up) {
+    const int64_t up_stride = (int64_t)2 * m->ff * ld, down_stride = (int64_t)ld * m->ff;
+    RowGroups g{c.group_of, c.group_row, c.group_end, c.used, c.n_tiles, c.tile_rows, c.slot_row, c.slot_scale, up_stride,
+                fold ? static_cast<const bf16*>(m->shared_up) : nullptr, fold ? m->experts : -1};
+    const bool ring = c.tile_rows == 256;
+    int rc = ring ? ring_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, g, s) : mid_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, 0, g, s);
+    if (rc) return rc;
+    g.x_row = nullptr; g.x_scale = nullptr; g.w_stride = down_stride;
+    g.w_extra = fold ? static_cast<const bf16*>(m->shared_down) : nullptr;
+    rc = ring ? ring_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, g, s) : mid_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, few, g, s);
+    if (rc) return rc;
+    if (m->shared_up && !fold) {
         raven_epilogue e{};
         e.scale = 1.f; e.out_f32 = 1;
         if (const int rc = raven_linear(h, nullptr, m->shared_up, nullptr, c.sact, M, m->shared_ff, ld, 0, 1, 0, dtype, c.lin, c.lin_bytes, s)) return rc;
         if (const int rc = raven_linear_epilogue(c.sact, nullptr, m->shared_down, c.ys, M, ld, m->shared_ff, 0, &e, dtype, c.lin, c.lin_bytes, s)) return rc;
     }
-    moe_combine_kernel<<<dim3((unsigned)(((int64_t)M * (ld / 4) + 255) / 256)), dim3(256), 0, s>>>(a);
+    const dim3 grid((unsigned)(((int64_t)M * (ld / 4) + 255) / 256));
+    if (few) moe_combine_kernel<float><<<grid, dim3(256), 0, s>>>(a);
+    else moe_combine_kernel<bf16><<<grid, dim3(256), 0, s>>>(a);
     return raven_host::check_launch("moe (combine)");
 }
 }  // namespace raven

@@ -342,6 +342,39 @@ def test_mixture_in_large_tiles(pkg, M, D, E, top, ff):
     assert (stream.cpu().double() - x - want).abs().max() < 2e-2 * max(1.0, want.abs().max().item())
 
 
+@pytest.mark.parametrize("same", [False, True])
+@pytest.mark.parametrize("M,D,E,top,ff,shared", [(5, 1032, 64, 6, 392, True), (20, 1032, 64, 6, 392, True), (21, 1032, 64, 6, 392, False), (64, 520, 300, 4, 264, True),
+                                                 (9, 2048, 16, 1, 776, True), (70, 520, 24, 6, 72, True), (200, 264, 12, 2, 136, False)])
+def test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, same):
+    """Rows sorted by expert at sizes where experts have one row, a tile of 16, 32 or 64 rows, or (same: most rows choose alike) several tiles, the
+    shared expert one more group or a product of its own; widths that are no multiple of 64.  Against 64 bits: the activations are
+    rounded to bf16 once (2^-9 of each, 2e-3 in the norm), a chunk's slots once more."""
+    g = torch.Generator(device="cuda").manual_seed(M + E)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    up, down, sup, sdown = ((rand(*s) * s[-1] ** -0.5).to(BF16) for s in ((E, 2 * ff, D), (E, D, ff), (2 * ff, D), (D, ff)))
+    ldl = (E + 1 + 15) // 16 * 16
+    router = torch.zeros(ldl, D, dtype=BF16, device="cuda")
+    desc = pkg.hip.Moe(router.data_ptr(), up.data_ptr(), down.data_ptr(), sup.data_ptr() if shared else None, sdown.data_ptr() if shared else None, E, top, ff,
+                       ff if shared else 0, ldl)
+    h, logits, x = rand(M, D).to(BF16), rand(M, ldl), rand(M, D)
+    if same:
+        logits[M // 4:] = logits[:1]
+    s, index = torch.sigmoid(logits[:, :E].double()).topk(top, 1)
+    gated = lambda a, u, d: (torch.nn.functional.silu(a @ u[:ff].double().T) * (a @ u[ff:].double().T)) @ d.double().T
+    want = torch.sigmoid(logits[:, E:E + 1].double()) * gated(h.double(), sup, sdown) if shared else torch.zeros(M, D, device="cuda", dtype=torch.float64)
+    for e in range(E):
+        row, place = torch.where(index == e)
+        if len(row):
+            want[row] += gated(s[row, place, None] * h[row].double(), up[e], down[e])
+    outs = []
+    for _ in range(2):
+        stream = x.clone()
+        pkg.hip.moe(desc, h, logits, stream)
+        outs.append(stream)
+    assert torch.equal(*outs), "the order of an expert's rows must not show"
+    assert ((outs[0].double() - x.double() - want).norm() / want.norm()).item() < 5e-3
+
+
 @DT
 @pytest.mark.parametrize("M", [1, 20])
 def test_mixture_prefers_the_lower_index_among_equals(pkg, dtype, M):
