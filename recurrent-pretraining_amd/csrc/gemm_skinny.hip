@@ -1,13 +1,14 @@
 // Skinny GEMMs of the decode path: Y[M,N] = X[M,K] W[N,K]^T with M = a handful of token rows and
 // W a weight matrix that is streamed from HBM exactly once per call (per 32 rows of X).
 //
-// Two kernels:
+// Three kernels:
 //   gemv_kernel  (any T, up to 8 rows of X per pass)  -- X lives in LDS, every wave owns whole rows
 //                of W, reads them with 16-byte lane-contiguous loads and accumulates with
 //                v_dot2_f32_bf16 / fp32 FMA; a DPP wave reduction finishes each row.
 //   mfma_kernel  (bf16, up to 32 rows of X per pass)   -- 16-row tiles of W are the A operand of
 //                v_mfma_f32_16x16x32_bf16, X is the B operand; the four waves of a workgroup split
 //                K and reduce through LDS.
+//   rows_f32_kernel (float, 2 rows and more)          -- 16 rows of W against 16 to 64 rows of X on v_mfma_f64_16x16x4_f64.
 // Epilogues (all round the fp32 accumulator to T first, as an nn.Linear output would be stored):
 //   plain (+ residual add in T, + optional float store)   RMM:493, 509, 711, 534-535
 //   SwiGLU: T(T(silu(gate)) * up), gate row j, up row j+I  RMM:507-508
@@ -433,6 +434,102 @@ __global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// rows_f32_kernel: a workgroup owns 16 weight rows (SwiGLU: 16 gate rows and their up rows) and 16 MT token rows, its four waves split K
+// and add up through LDS.  A lane loads 16 bytes of row l % 16 at columns 16 c + 4 (l / 16) ..+3 straight from memory -- of W and of X
+// alike, so that product j of a chunk, which takes element j of every lane's load, multiplies the same columns on both sides.  Products
+// and sums are in 64 bits (exact products; the fp32 instruction's one long chain of sums per element was 1.7 times further from the
+// exact result than gemv_kernel's 64 short ones, and no faster here).
+// What bounds it is latency (small models) or the 64-byte row pieces (large matrices: about 3 TB/s), not the matrix cores; it
+// reads W once per 64 rows where gemv_kernel takes passes of 8, each a launch: a product of 17 rows, 256 x 704 to 1408 x 256, three
+// launches of 4.5 to 8 us, now one of 5; 200 rows 25 launches.
+// ------------------------------------------------------------------------------------------------
+template <int EPI, int MT>
+__global__ __launch_bounds__(256) void rows_f32_kernel(GemmArgs a) {
+    typedef __attribute__((ext_vector_type(4))) double f64x4;
+    constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, U = 4;
+    __shared__ __align__(16) f64x4 red[3][NT * MT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT, K = a.K;
+    const float* w[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) w[t] = static_cast<const float*>(a.w) + (int64_t)(min(n0 + r, a.N - 1) + t * a.N) * K;
+    int64_t row[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) row[j] = min(m0 + 16 * j + r, a.M - 1);
+    const int chunks = (K + 15) / 16, c0 = chunks * wave / 4, c1 = chunks * (wave + 1) / 4;
+
+    f64x4 acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[t][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    auto load_x = [&](int j, int k) __attribute__((always_inline)) {
+        const bool second = k >= a.k0;
+        const float* x = second ? static_cast<const float*>(a.x1) - a.k0 : static_cast<const float*>(a.x0);
+        return *reinterpret_cast<const f32x4*>(x + row[j] * (second ? a.k1 : a.k0) + k);
+    };
+    auto multiply = [&](const f32x4 (&wv)[NT], const f32x4 (&xv)[MT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) acc[t][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)wv[t][i], (double)xv[j][i], acc[t][j], 0, 0, 0);
+    };
+    int c = c0;
+    for (; c + U <= c1 && 16 * (c + U) <= K; c += U) {
+        f32x4 wv[U][NT], xv[U][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = 16 * (c + u) + 4 * q;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wv[u][t] = *reinterpret_cast<const f32x4*>(w[t] + k);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) xv[u][j] = load_x(j, k);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(wv[u], xv[u]);
+    }
+    for (; c < c1; ++c) {  // what is left, and a chunk that K ends inside
+        const int k = 16 * c + 4 * q, kc = min(k, K - 4);
+        f32x4 wv[NT], xv[MT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            wv[t] = *reinterpret_cast<const f32x4*>(w[t] + kc);
+            if (k >= K) wv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            xv[j] = load_x(j, kc);
+            if (k >= K) xv[j] = f32x4{0.f, 0.f, 0.f, 0.f};  // (0 times an infinity that lies elsewhere is no zero)
+        }
+        multiply(wv, xv);
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) red[wave - 1][t * MT + j][lane] = acc[t][j];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int m = m0 + 16 * j + r;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t][j] += (red[0][t * MT + j][lane] + red[1][t * MT + j][lane]) + red[2][t * MT + j][lane];
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {  // a lane holds weight rows 4 v + q of token row r
+            const int n = n0 + 4 * v + q;
+            if (n >= a.N) continue;
+            if constexpr (EPI == EPI_SWIGLU) static_cast<float*>(a.y)[(int64_t)m * a.N + n] = swiglu<float>((float)acc[0][j][v], (float)acc[NT - 1][j][v]);
+            else store_out<float, EPI>(a, m, n, (float)acc[0][j][v]);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // host dispatch
 // ------------------------------------------------------------------------------------------------
 static int n_cus() {
@@ -544,6 +641,20 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
     return raven_host::check_launch("mfma gemm");
 }
 
+// Float rows: all of them in one launch.  A few rows against a matrix that does not fit the caches stay with the vector kernel, whose
+// whole-row loads stream twice as fast (5.5 TB/s): up to 8 rows from 32 MB on.
+template <int EPI>
+static int launch_rows_f32(GemmArgs a, hipStream_t s) {
+    a.ldy = a.N;
+    const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
+    const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));
+    RAVEN_REQUIRE(grid.y <= 65535, "gemm: %d rows in one call", a.M);
+    if (mt == 1) rows_f32_kernel<EPI, 1><<<grid, dim3(256), 0, s>>>(a);
+    else if (mt == 2) rows_f32_kernel<EPI, 2><<<grid, dim3(256), 0, s>>>(a);
+    else rows_f32_kernel<EPI, 4><<<grid, dim3(256), 0, s>>>(a);
+    return raven_host::check_launch("gemm (fp32 rows)");
+}
+
 // Runs one GEMM over all M rows, in passes of at most 32 (MFMA) or 8 / 4 (vector) rows.
 template <int EPI>
 static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
@@ -551,6 +662,7 @@ static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
     const bool mfma_ok = dtype == RAVEN_BF16 && a.K % 32 == 0 && a.k0 % 32 == 0 && a.N % 16 == 0;
     const int M = a.M;
     const size_t out_es = a.out_f32 ? 4 : es;
+    if (dtype == RAVEN_F32 && M >= 2 && (M > 8 || (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20))) return launch_rows_f32<EPI>(a, s);
     for (int m0 = 0; m0 < M;) {
         const int left = M - m0;
         int pass;

@@ -192,6 +192,29 @@ def test_gemm_fp32_tiny_shapes(pkg, M):
         check(pkg.hip.gemm(x.cuda(), w.cuda()), lin(x, w), dt, f"fp32 gemm {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M", [2, 16, 17, 32, 33, 65, 130])
+@pytest.mark.parametrize("N,K0,K1", [(13, 4, 0), (40, 100, 0), (256, 256, 256), (70, 36, 20), (33, 1412, 0)])
+def test_fp32_rows_in_one_launch(pkg, M, N, K0, K1):
+    """Float products of 2 rows and more: tiles of 16 weight rows and 16 to 64 token rows that end early, K shares of the four waves that are
+    empty or end inside a chunk of 16, a boundary between two operands inside a chunk.  Products and sums are in 64 bits: one rounding
+    to float (2^-25 of the value at most, 3e-8 in the norm) for a plain product, a second one with a residual."""
+    x0, x1 = rnd((M, K0), torch.float32, 1).cuda(), (rnd((M, K1), torch.float32, 2).cuda() if K1 else None)
+    w, res = rnd((N, K0 + K1), torch.float32, 3).cuda(), rnd((M, N), torch.float32, 4).cuda()
+    want = (x0 if x1 is None else torch.cat([x0, x1], -1)).double() @ w.double().T
+    off = lambda got, ref: ((got.double() - ref).norm() / ref.norm()).item()
+    assert off(pkg.hip.linear(x0, w, x1=x1), want) < 6e-8
+    bias = rnd((N,), torch.float32, 5).cuda()
+    assert off(pkg.hip.linear_epilogue(x0, w, x1=x1, bias=bias, residual=res, scale=0.5), want * 0.5 + bias + res) < 2e-7
+    if not K1:
+        assert off(pkg.hip.linear(x0, w, residual=res), want + res) < 2e-7
+        if N % 2 == 0:
+            gate, up = want[:, :N // 2], want[:, N // 2:]
+            assert off(pkg.hip.linear(x0, w, swiglu=True), F.silu(gate) * up) < 1e-6
+    x0[0, 0], w[0, 0] = float("inf"), 1.0  # an infinity stays in its row
+    got = pkg.hip.linear(x0, w, x1=x1)
+    assert torch.isfinite(got[1:]).all() and not torch.isfinite(got[0]).any()
+
+
 @pytest.mark.parametrize("dt,M,h", [(torch.bfloat16, 1, 5280), (torch.bfloat16, 32, 5280), (torch.bfloat16, 6, 64),
                                     (torch.float32, 1, 256), (torch.float32, 12, 256)])
 def test_adapter_concat(pkg, dt, M, h):
