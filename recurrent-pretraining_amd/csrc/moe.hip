@@ -47,9 +47,34 @@ struct MoeArgs {
     const float* ys;        // [M, ld] or null
 };
 
-// one wave: the `top` experts of largest logit (lower index first among equals); lane k holds the k-th one and its score
+// a float as an integer of the same order; NaN below everything
+__device__ __forceinline__ int ordered_key(float v) {
+    const int b = __builtin_bit_cast(int, v + 0.0f);  // (the two zeros are equal)
+    return v != v ? (int)0x80000000 : b < 0 ? b ^ 0x7fffffff : b;
+}
+
+// one wave: the `top` experts of largest logit (lower index first among equals); lane k holds the k-th one and its score.
+// Up to 64 experts (a lane each) an expert's place is the number of experts before it, counted in one sweep over the others' logits
+// through the lane-to-lane broadcast: 64 steps without a dependence, where `top` maxima over the wave, twelve exchanges each, took 3 us
+// of every launch that picks (moe_up_kernel at one row 14.7 -> 12 us, routing of 20 rows 11.8 -> 8).
 __device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
     const int lane = threadIdx.x & 63;
+    if (experts <= 64) {
+        const float v = lane < experts ? logits[lane] : 0.f;
+        const int key = lane < experts ? ordered_key(v) : (int)0x80000000;
+        int before = 0;
+#pragma unroll
+        for (int j = 0; j < 64; ++j) {
+            const int other = __builtin_amdgcn_readlane(key, j);
+            before += other > key || (other == key && j < lane) ? 1 : 0;
+        }
+        // every lane has a place of its own (absent experts the last ones): lane l sends its number there
+        mine = __builtin_amdgcn_ds_permute(before * 4, lane);
+        const float s = __builtin_bit_cast(float, __builtin_amdgcn_ds_permute(before * 4, __builtin_bit_cast(int, v == v ? v : -INFINITY)));
+        mine = min(mine, experts - 1);
+        score = sigmoid_f32(s);
+        return;
+    }
     float v[kMaxExperts / 64];
 #pragma unroll
     for (int j = 0; j < kMaxExperts / 64; ++j) {

@@ -393,6 +393,32 @@ def test_mixture_prefers_the_lower_index_among_equals(pkg, dtype, M):
     assert (x.cpu() - want).abs().max() < (1e-5 if dtype == F32 else 2e-2)
 
 
+@pytest.mark.parametrize("E", [7, 64, 65, 200])
+@pytest.mark.parametrize("M", [1, 3])
+def test_mixture_picks_by_value_then_index(pkg, E, M):
+    """Zeros of either sign are equal, ties go to the lower index, minus infinity is a score of nothing; 64 experts and fewer are picked by
+    counting, more by repeated maxima.  Expert e multiplies by a power of its own, so that a sum names its experts."""
+    D, ff, top = 8, 8, 3
+    up = torch.zeros(E, 2 * ff, D, device="cuda")
+    up[:, 0, 0] = up[:, ff, 0] = 1.0
+    down = torch.zeros(E, D, ff, device="cuda")
+    down[:, torch.arange(1, D), 0] = torch.randn(E, D - 1, generator=torch.Generator().manual_seed(E)).cuda()
+    router = torch.zeros((E + 16) // 16 * 16, D, device="cuda")
+    desc = pkg.hip.Moe(router.data_ptr(), up.data_ptr(), down.data_ptr(), None, None, E, top, ff, 0, router.shape[0])
+    h = torch.zeros(M, D, device="cuda")
+    h[:, 0] = 1.0
+    for values, chosen in ((lambda l: l.fill_(0.0), [0, 1, 2]), (lambda l: (l.fill_(-0.0), l[:, 2:4].fill_(0.0)), [0, 1, 2]),
+                           (lambda l: (l.fill_(-1.0), l[:, E - 1].fill_(2.0), l[:, 1].fill_(0.0), l[:, 4].fill_(-0.0)), [E - 1, 1, 4]),
+                           (lambda l: (l.fill_(float("-inf")), l[:, 5].fill_(1.0)), [5])):
+        logits = torch.full((M, router.shape[0]), 1e9, device="cuda")
+        values(logits[:, :E])
+        x = torch.zeros(M, D, device="cuda")
+        pkg.hip.moe(desc, h, logits, x)
+        s = torch.sigmoid(logits[:, chosen])
+        want = sum((torch.nn.functional.silu(s[:, i]) * s[:, i])[:, None] * down[e, :, 0] for i, e in enumerate(chosen))
+        assert (x - want).abs().max() < 1e-5, (chosen, x, want)
+
+
 # ---- whole models ------------------------------------------------------------------------------------
 def feed(model, ids, cuts, cache=None, runner=None):
     """Portions of a prompt through forward(), single tokens through the decode runner; logits of every position."""
