@@ -57,6 +57,7 @@ struct Tuning {
     int gemv_wgs_per_cu = 4;
     int gemm_four_tiles = 1;
     int gemm_mfma_min_rows = 2;  // fewer rows go to the vector kernels (one row: the K-split GEMV)
+    int gemm_one_round = 1;      // 0 = never one workgroup of eight waves per CU
     int gemm_ragged = 1;         // 0 never, 1 = one workgroup per resident slot with partly empty last tiles where the shape divides so
 };
 static Tuning g_tuning;
@@ -68,6 +69,7 @@ int set_skinny_tuning(const char* key, int value) {
     else if (k == "gemv_nontemporal") g_tuning.gemv_nontemporal = value;
     else if (k == "gemv_wgs_per_cu") g_tuning.gemv_wgs_per_cu = value;
     else if (k == "gemm_four_tiles") g_tuning.gemm_four_tiles = value;
+    else if (k == "gemm_one_round") g_tuning.gemm_one_round = value;
     else if (k == "gemm_ragged") g_tuning.gemm_ragged = value;
     else if (k == "gemm_mfma_min_rows" && value >= 2) g_tuning.gemm_mfma_min_rows = value;
     else return -1;
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// mfma_kernel: bf16, 256 threads = 4 waves that split K; MT = ceil(M/16) batch tiles; NT weight
+// mfma_kernel: bf16, 4 waves (or 8) that split K; MT = ceil(M/16) batch tiles; NT weight
 // tiles of 16 rows per workgroup.  D = A * B with A = W tile [16 n x 32 k], B = X^T [32 k x 16 m]:
 // lane l supplies A[n = l%16][k = 8*(l/16) ..+8] and B[k = 8*(l/16) ..+8][m = l%16] and receives
 // D[n = 4*(l/16) + v][m = l%16], v = 0..3.
@@ -228,16 +230,18 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
 // 16 at a time and the last slot is partly empty (its missing rows are neither loaded nor stored).  This lets the host cut
 // a matrix into exactly as many workgroups as the chip holds at once (17920 gate rows = 512 x 35), where whole tiles
 // would leave a partly filled last round.
-template <int MT, int NT, int EPI, int KM = 128, bool RAG = false>
-__global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
+//
+// WAVES = 8 with D register sets in flight: the variants of launch_one_round, one workgroup per CU.
+template <int MT, int NT, int EPI, int KM = 128, bool RAG = false, int WAVES = 4, int D = 1>
+__global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
     constexpr int ROWS = 16 * (NT + MT);
     constexpr int kPitch = KM + 8;
     constexpr int LPR = KM / 8;        // lanes per row of a macro-step
     constexpr int RPI = 64 / LPR;      // rows per load instruction
     constexpr int IPT = 16 / RPI;      // load instructions per 16-row tile
     constexpr int NG = EPI == EPI_SWIGLU ? NT / 2 : NT;  // tiles side by side along N (SwiGLU: NG gate tiles + their NG up tiles)
-    __shared__ __align__(16) bf16 stage[4][ROWS][kPitch];
-    static_assert(sizeof(bf16) * 4 * ROWS * kPitch >= sizeof(float) * 3 * NT * MT * 64 * 4, "stage doubles as the reduction buffer");
+    __shared__ __align__(16) bf16 stage[WAVES][ROWS][kPitch];
+    static_assert(sizeof(bf16) * WAVES * ROWS * kPitch >= sizeof(float) * (WAVES - 1) * NT * MT * 64 * 4, "stage doubles as the reduction buffer");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ln = lane & 15, kq = lane >> 4;
     const int K = a.K;
@@ -302,8 +306,8 @@ __global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
             if (shift > seg_len) shift = 0;
         }
         const int n_macro = (seg_len - shift) / KM;
-        // the four waves take the macro-steps in turn, so that the workgroup as a whole walks its rows in pieces of
-        // 4 * KM contiguous elements (DRAM pages are then read in longer runs than one wave's 256 bytes)
+        // the waves take the macro-steps in turn, so that the workgroup as a whole walks its rows in pieces of
+        // WAVES * KM contiguous elements (DRAM pages are then read in longer runs than one wave's 256 bytes)
         const int mb = wave, me = n_macro;
 
         auto fetch = [&](int mac, Staged& st) {  // global -> registers, row-contiguous lanes
@@ -356,18 +360,48 @@ __global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         };
-        // one register set: its loads for macro-step s+1 are in flight while step s is multiplied out of LDS
-        Staged st{};
-        if (mb < me) fetch(mb, st);
-        for (int mac = mb; mac < me; mac += 4) {
-            park(st);
-            wave_sync();
-            if (mac + 4 < me) fetch(mac + 4, st);
-            multiply();
-            wave_sync();
+        if constexpr (D == 1) {
+            // one register set: its loads for macro-step s+1 are in flight while step s is multiplied out of LDS
+            Staged st{};
+            if (mb < me) fetch(mb, st);
+            for (int mac = mb; mac < me; mac += WAVES) {
+                park(st);
+                wave_sync();
+                if (mac + WAVES < me) fetch(mac + WAVES, st);
+                multiply();
+                wave_sync();
+            }
+        } else if (mb < me) {
+            // rounds of D steps, each requesting the next round's loads (none under a branch of its own, so that the waits count only the
+            // set being parked); what lies past the end loads the wave's first step again and is not multiplied
+            Staged st[D];
+            const int steps = (me - mb + WAVES - 1) / WAVES;
+            auto step_of = [&](int i) { return i < steps ? mb + i * WAVES : mb; };
+#pragma unroll
+            for (int d = 0; d < D; ++d) fetch(step_of(d), st[d]);
+            int done = 0;
+#pragma unroll 1
+            for (; done + D < steps; done += D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    park(st[d]);
+                    wave_sync();
+                    fetch(step_of(done + D + d), st[d]);
+                    multiply();
+                    wave_sync();
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (done + d >= steps) break;
+                park(st[d]);
+                wave_sync();
+                multiply();
+                wave_sync();
+            }
         }
         // 32-element steps in front of the first and behind the last macro-step: first and last wave, straight from global memory
-        if (wave == 0 || wave == 3) {
+        if (wave == 0 || wave == WAVES - 1) {
             const int kb = wave == 0 ? 0 : shift + n_macro * KM, ke = wave == 0 ? shift : seg_len;
             for (int k = kb; k < ke; k += 32) {
 #pragma unroll
@@ -403,8 +437,12 @@ __global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-                acc[t][mt][v] += red[0][t * MT + mt][lane][v] + red[1][t * MT + mt][lane][v] + red[2][t * MT + mt][lane][v];
+            for (int v = 0; v < 4; ++v) {
+                float others = red[0][t * MT + mt][lane][v];
+#pragma unroll
+                for (int r = 1; r < WAVES - 1; ++r) others += red[r][t * MT + mt][lane][v];
+                acc[t][mt][v] += others;
+            }
 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -584,6 +622,41 @@ static int dispatch_gemv(GemmArgs a, hipStream_t s) {
     return launch_gemv<T, 8, EPI>(a, s);
 }
 
+// A matrix of up to 1024 tiles of 16 rows (from 17 token rows on 768; SwiGLU: 256 pairs) in one round of the chip: the fewest tiles per workgroup that give every CU at
+// most one workgroup, of eight waves.  Four waves a tile leave a CU with one or two short workgroups, or a second round of them; with eight,
+// and the partial sums added through LDS, the K slices of gemm_splitk.hip and their second launch are not needed either, up to the
+// length of K where the workgroups become too long (splits_k there).  us per launch before / after: 2048 x 2048 at 8 rows 6.1 / 5.5, at 20 rows
+// 9.3 / 7.0; 8192 x 2048 9.9 / 9.5 and 15.3 / 10.9; 10304 x 2048 12.0 / 11.2 and 15.4 / 12.6; 15840 x 5280 at 16 rows 32.6 / 30.1.
+// More loads in flight than two sets of 64 columns per wave gain nothing: a CU's own rate of loads is the bound.
+template <int EPI, int MT>
+static bool launch_one_round(const GemmArgs& a, hipStream_t s) {
+    constexpr int side = EPI == EPI_SWIGLU ? 2 : 1;
+    const int rs = a.row_stride, n_tiles16 = a.N / 16;
+    auto groups = [&](int ng) { return (n_tiles16 + ng * rs - 1) / (ng * rs) * rs; };
+    if (!g_tuning.gemm_one_round || g_tuning.gemm_four_tiles == 2) return false;
+    if (groups(1) <= n_cus()) {
+        mfma_kernel<MT, side, EPI, 128, false, 8><<<dim3(groups(1)), dim3(512), 0, s>>>(a);
+        return true;
+    }
+    if constexpr (EPI != EPI_SWIGLU) {  // two gate tiles and their up tiles: no faster than the four-wave kernels (14.4 / 14.1 at 12288 x 2048)
+        if (groups(2) <= n_cus()) {
+            mfma_kernel<MT, 2, EPI, 64, false, 8, 2><<<dim3(groups(2)), dim3(512), 0, s>>>(a);
+            return true;
+        }
+        if (groups(3) <= n_cus()) {
+            mfma_kernel<MT, 3, EPI, 64, false, 8, 2><<<dim3(groups(3)), dim3(512), 0, s>>>(a);
+            return true;
+        }
+        if constexpr (MT == 1) {  // two token tiles against four weight tiles do not fit the registers
+            if (groups(4) <= n_cus()) {
+                mfma_kernel<1, 4, EPI, 64, false, 8><<<dim3(groups(4)), dim3(512), 0, s>>>(a);
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
 template <int EPI>
 static int dispatch_mfma(GemmArgs a, hipStream_t s) {
     const int n_tiles16 = a.N / 16;
@@ -593,6 +666,7 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
     a.row_stride = (pitch % 128 == 64 && a.N % 32 == 0) ? 2 : 1;
     a.line_aligned = (pitch * a.row_stride) % 128 == 0;
     const int rs = a.row_stride;
+    if (a.M <= 16 ? launch_one_round<EPI, 1>(a, s) : launch_one_round<EPI, 2>(a, s)) return raven_host::check_launch("mfma gemm");
     // Four tiles per workgroup (64-wide K steps) halve the X re-reads per weight byte: 5.0 -> 5.7 TB/s in steady state
     // at 32 rows.  Their workgroups are twice as long, so the gain only survives where the grid is balanced: at most
     // one workgroup per CU (Wqkv: 248), or so many that the last round does not matter.  Tuning key gemm_four_tiles:

@@ -310,6 +310,29 @@ def test_mfma_gemm_row_alignment_cases(pkg, tuned, M, four):
                   f"two operands {M}x{N}x({K0}+{K1})")
 
 
+@pytest.mark.parametrize("M", [2, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 32), (80, 96), (4096, 2048), (4112, 1184), (8192, 288), (8256, 160), (12304, 256), (16352, 416), (16400, 64)])
+def test_a_few_rows_in_one_round_of_the_chip(pkg, M, N, K):
+    """One to four tiles of 16 columns per workgroup, on both sides of each border at 256 compute units: K shares of the eight waves that are empty,
+    one step or several rounds of two, tiles of one row parity and whole ones, a last workgroup that is partly empty; every epilogue."""
+    dt = torch.bfloat16
+    x, w, res = rnd((M, K), dt, 240).cuda(), rnd((N, K), dt, 241, 0.05).cuda(), rnd((M, N), dt, 242).cuda()
+    ws = pkg.hip.linear_workspace(M, N, "cuda")
+    z = x.float() @ w.float().T
+    check(pkg.hip.linear(x, w, workspace=ws), z.to(dt), dt, "plain")
+    check(pkg.hip.linear(x, w, residual=res, workspace=ws), (z.to(dt).float() + res.float()).to(dt), dt, "+ residual", mag=z, ulps=ULPS_RESIDUAL)
+    bias, resf = torch.randn(N, device="cuda"), torch.randn(M, N, device="cuda")
+    got, want = pkg.hip.linear_epilogue(x, w, bias=bias, residual=resf, scale=0.5, workspace=ws), z * 0.5 + bias + resf
+    assert ((got - want).norm() / want.norm()).item() < 3e-6   # fp32 sums of at most 2048 products in another order
+    check(pkg.hip.linear_epilogue(x, w, bias=bias, act=pkg.hip.ACT_GELU, out_f32=False, workspace=ws), F.gelu(z + bias).to(dt), dt, "gelu")
+    check(pkg.hip.linear_epilogue(x, w, act=pkg.hip.ACT_TANH, out_f32=False, workspace=ws), torch.tanh(z).to(dt), dt, "tanh")
+    if N % 32 == 0:
+        u = z.to(dt).float()
+        check(pkg.hip.linear(x, w, swiglu=True, workspace=ws), (F.silu(u[:, :N // 2]).to(dt).float() * u[:, N // 2:]).to(dt), dt, "SwiGLU", ulps=ULPS_SWIGLU)
+    if K % 64 == 0:
+        check(pkg.hip.linear(x[:, :K // 2].contiguous(), w, x1=x[:, K // 2:].contiguous(), workspace=ws), z.to(dt), dt, "two operands")
+
+
 @pytest.mark.parametrize("M", [8, 32])
 def test_mfma_four_tile_variant_nebel_shapes(pkg, tuned, M):
     dt, h, I = torch.bfloat16, 5280, 17920
