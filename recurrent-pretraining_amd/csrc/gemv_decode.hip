@@ -12,7 +12,9 @@
 // 4-way LDS reduction finish the pair, and the epilogue is the same as in gemm_skinny.hip:
 // plain (+ residual, + float store) or SwiGLU (rows j and j + N).
 //
-// C = weight chunks per lane, per row: ceil(ceil(K / E / 4) / 64) rounded up to 3, 6 or 9.
+// C = weight chunks per lane, per row: ceil(ceil(K / E / 4) / 64), 5 rounded up to 6 and 7 and 8 to 9.  A kernel of more chunks than the row has
+// holds the registers of a full one, which costs the resident workgroups and with them the loads in flight: 8192 x 2048 in bf16 behind the norm
+// prologue takes 8.0 us with one chunk per lane and 10.4 with three, two of them empty.
 
 #include <string>
 
@@ -281,46 +283,51 @@ static int gemv1_cus() {
     return cus;
 }
 
+// The longest rows the one-row kernel takes (gemm_skinny.hip asks the same)
+static bool gemv1_fits(int K, int E) { return ((K / E + 3) / 4 + 1 + 63) / 64 <= 9; }
+
 template <typename T, int EPI>
 static int launch_gemv1(Gemv1Args a, hipStream_t s) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
     constexpr int E = Chunk<T>::N;
     const int n_chunks = a.K / E;
-    const int per_wave = (n_chunks + 3) / 4 + 1;  // a quarter, rounded up
-    const int c = (per_wave + 63) / 64;
+    const int c = ((n_chunks + 3) / 4 + 63) / 64;  // a wave's share is a quarter of the chunks, rounded up at most
     const int units = SWIGLU ? a.N : (a.N + 1) / 2;
     const bool norm = a.norm_a != nullptr;
     int ppw = norm ? g_gemv1_tuning.pairs_norm : g_gemv1_tuning.pairs_plain;
     // with a norm prologue: as many pairs as leave about ten workgroups per CU -- 4 for Wqkv (7920 pairs, 1980 workgroups),
     // 7 for mlp.fc (17920 gate / up pairs, 2560 workgroups: 57.6 us against 58.4 with 4, while Wqkv loses with more than 4)
-    if (norm && ppw <= 0) ppw = (units + 10 * gemv1_cus() - 1) / (10 * gemv1_cus());
+    // rows of one chunk per lane: about four workgroups per CU (8192 x 2048 behind the float norm 8.0 us against 8.4, 8192 x 1024 6.5 / 6.8)
+    const int per_cu = c <= 1 ? 4 : 10;
+    if (norm && ppw <= 0) ppw = (units + per_cu * gemv1_cus() - 1) / (per_cu * gemv1_cus());
     if (ppw < 1) ppw = 1;
     if (ppw > kMaxPairsPerWg) ppw = kMaxPairsPerWg;
     while (ppw > 1 && (units + ppw - 1) / ppw < 1024) --ppw;  // keep at least ~4 workgroups per CU
     if (c > 3) ppw = 1;  // the double-buffered variant exists for short rows only (registers)
     a.pairs_per_wg = ppw;
     const int wgs = (units + ppw - 1) / ppw;
-#define RAVEN_GEMV1(CC)                                                                            \
-    do {                                                                                           \
-        if (norm) gemv1_kernel<T, CC, EPI, PRO_NORM, false><<<dim3(wgs), dim3(256), 0, s>>>(a);     \
-        else gemv1_kernel<T, CC, EPI, PRO_NONE, false><<<dim3(wgs), dim3(256), 0, s>>>(a);         \
+    RAVEN_REQUIRE(gemv1_fits(a.K, E), "gemv_fused: K=%d is too long for the one-row kernel (max %d)", a.K, 9 * 64 * 4 * E - 4 * E);
+    RAVEN_REQUIRE(a.dim == 0 || c <= 3, "gemv: K=%d is too long for the float-row norm prologue", a.K);
+#define RAVEN_GEMV1(CC)                                                                                                \
+    do {                                                                                                               \
+        constexpr bool kMulti = CC <= 3;                                                                               \
+        if (a.dim > 0) {                                                                                               \
+            if constexpr (kMulti && (is_free(EPI) || SWIGLU)) {                                                        \
+                if (ppw > 1) gemv1_kernel<T, CC, EPI, PRO_STREAM, true><<<dim3(wgs), dim3(256), 0, s>>>(a);            \
+                else gemv1_kernel<T, CC, EPI, PRO_STREAM, false><<<dim3(wgs), dim3(256), 0, s>>>(a);                   \
+            }                                                                                                          \
+        } else if (kMulti && ppw > 1) {                                                                                \
+            if (norm) gemv1_kernel<T, CC, EPI, PRO_NORM, kMulti><<<dim3(wgs), dim3(256), 0, s>>>(a);                   \
+            else gemv1_kernel<T, CC, EPI, PRO_NONE, kMulti><<<dim3(wgs), dim3(256), 0, s>>>(a);                        \
+        } else if (norm) gemv1_kernel<T, CC, EPI, PRO_NORM, false><<<dim3(wgs), dim3(256), 0, s>>>(a);                 \
+        else gemv1_kernel<T, CC, EPI, PRO_NONE, false><<<dim3(wgs), dim3(256), 0, s>>>(a);                             \
     } while (0)
-    if (a.dim > 0) {  // PRO_STREAM
-        RAVEN_REQUIRE(c <= 3, "gemv: K=%d is too long for the float-row norm prologue", a.K);
-        if constexpr (is_free(EPI) || SWIGLU) {
-            if (ppw > 1) gemv1_kernel<T, 3, EPI, PRO_STREAM, true><<<dim3(wgs), dim3(256), 0, s>>>(a);
-            else gemv1_kernel<T, 3, EPI, PRO_STREAM, false><<<dim3(wgs), dim3(256), 0, s>>>(a);
-        }
-    } else if (c <= 3 && ppw > 1) {
-        if (norm) gemv1_kernel<T, 3, EPI, PRO_NORM, true><<<dim3(wgs), dim3(256), 0, s>>>(a);
-        else gemv1_kernel<T, 3, EPI, PRO_NONE, true><<<dim3(wgs), dim3(256), 0, s>>>(a);
-    } else if (c <= 3) RAVEN_GEMV1(3);
+    if (c <= 1) RAVEN_GEMV1(1);
+    else if (c <= 2) RAVEN_GEMV1(2);
+    else if (c <= 3) RAVEN_GEMV1(3);
+    else if (c <= 4) RAVEN_GEMV1(4);
     else if (c <= 6) RAVEN_GEMV1(6);
-    else if (c <= 9) RAVEN_GEMV1(9);
-    else {
-        raven_host::set_error("gemv_fused: K=%d is too long for the one-row kernel (max %d)", a.K, 9 * 64 * 4 * E - 4 * E);
-        return -1;
-    }
+    else RAVEN_GEMV1(9);
 #undef RAVEN_GEMV1
     return raven_host::check_launch("gemv_fused");
 }

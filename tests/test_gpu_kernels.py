@@ -347,6 +347,23 @@ def test_mfma_four_tile_variant_nebel_shapes(pkg, tuned, M):
     assert yf.dtype == torch.float32 and torch.equal(yf, pkg.hip.gemm(x.cuda(), wqkv.cuda()).float())
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("chunks", [1, 4, 255, 256, 257, 512, 513, 768, 769, 1024, 1025, 1536, 1537, 2300])
+def test_one_row_of_every_length_of_share(pkg, dt, chunks):
+    """One to nine 16-byte chunks per lane and the lengths around each border, an odd number of columns, with and without a norm in front
+    (of T, and of a float row where that is taken)."""
+    K, N = chunks * (8 if dt == torch.bfloat16 else 4), 77
+    x, w, nw = rnd((K,), dt, 250), rnd((N, K), dt, 251, 0.05), rnd((K,), dt, 252, 0.02, 1.0)
+    check(pkg.hip.linear(x[None].cuda(), w.cuda()), lin(x[None], w).to(dt), dt, "plain")
+    y, _ = pkg.hip.gemv_fused(x.cuda(), w.cuda(), norm_a=nw.cuda())
+    check(y[None], lin(O.rmsnorm(x[None], nw, 1e-6), w).to(dt), dt, "norm")
+    if pkg.hip.gemv_stream_fits(K, dt) and K % 8 == 0:
+        xf = x.float()
+        h = (xf / torch.sqrt((xf * xf).mean() + 1e-6) * nw.float()).to(dt)
+        got = pkg.hip.gemv_stream(xf.cuda(), nw.float().cuda(), K, 1e-6, w.cuda(), dt, out_f32=False)
+        check(got[None], lin(h[None], w).to(dt), dt, "float norm")
+
+
 @pytest.mark.parametrize("dt,h,I", [(torch.bfloat16, 5280, 17920), (torch.float32, 256, 704), (torch.bfloat16, 64, 176)])
 def test_gemv_fused_one_row(pkg, dt, h, I):
     """The one-row kernel with its norm prologues and epilogues, against the oracle's separate ops."""
