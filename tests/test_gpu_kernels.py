@@ -364,6 +364,15 @@ def test_one_row_of_every_length_of_share(pkg, dt, chunks):
         check(got[None], lin(h[None], w).to(dt), dt, "float norm")
 
 
+@pytest.mark.parametrize("vocab", [1, 63, 1024, 16383, 16384, 16385, 50001])
+def test_argmax_of_every_remainder(pkg, vocab):
+    """Rows that end inside a thread's 16 values, inside a stripe and on its border; the first of equal maxima, also the last value's."""
+    x = rnd((3, vocab), torch.float32, 260)
+    x[1, vocab // 2] = x[1, -1] = 50.0
+    x[2, -1] = 60.0
+    assert torch.equal(pkg.hip.argmax(x.cuda()).cpu(), x.argmax(-1))
+
+
 @pytest.mark.parametrize("dt,h,I", [(torch.bfloat16, 5280, 17920), (torch.float32, 256, 704), (torch.bfloat16, 64, 176)])
 def test_gemv_fused_one_row(pkg, dt, h, I):
     """The one-row kernel with its norm prologues and epilogues, against the oracle's separate ops."""
