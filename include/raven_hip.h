@@ -132,9 +132,8 @@ int raven_rmsnorm_residual(const void* x, const void* residual, const void* weig
                            void* sum_out, const void* weight2, void* y2,
                            int64_t rows, int32_t dim, float eps, int32_t dtype, void* stream);
 
-/* Y[M,N] = X[M,K] W[N,K]^T for skinny M (any M >= 1; the weight matrix is streamed once per 32
- * (bf16) or 8 (f32) rows).  Replaces the nn.Linear calls of attn.proj (RMM:493), mlp.proj (RMM:509)
- * and lm_head (RMM:711).  fp32 accumulate, result rounded to T; then, if residual != NULL,
+/* Y[M,N] = X[M,K] W[N,K]^T for skinny M (any M >= 1; up to 32 rows in bf16 and up to 8 in f32 read
+ * the weight matrix once).  Replaces the nn.Linear calls of attn.proj (RMM:493), mlp.proj (RMM:509) and lm_head (RMM:711).  fp32 accumulate, result rounded to T; then, if residual != NULL,
  * Y = T(Y + residual) (RMM:534-535); if out_f32 != 0 the rounded result is stored as float
  * (the `.float()` of RMM:711).  K * sizeof(T) % 16 == 0. */
 int raven_gemm(const void* x, const void* w, const void* residual, void* y,
@@ -153,11 +152,10 @@ int raven_gemm_swiglu(const void* x, const void* fc, void* out,
 
 /* The general form of the three calls above with an optional workspace:
  *     z = concat(x0, x1) W^T,  y = swiglu ? T(T(silu(T(z[:, :N]))) * T(z[:, N:])) : T(z) [+ residual] [as float]
- * With a workspace (raven_linear_workspace_bytes(M, widest output: 2N for SwiGLU)) and 5 or more bf16 rows,
- * K is split across workgroups and the X tile of a K step is shared by the workgroup's waves, which is
- * what batches of 8..32 rows need to approach HBM bandwidth; partial sums are added in a fixed order.  The same holds from 33
- * rows on for matrices with too few rows to give every compute unit a tile.
- * Without one (or for 1..4 rows, fp32) the call is forwarded to raven_gemm / _adapter_gemm_concat / _gemm_swiglu. */
+ * With a workspace (raven_linear_workspace_bytes(M, widest output: 2N for SwiGLU)) products of bf16 rows against matrices too
+ * narrow for their length to give every compute unit enough work are split over K across workgroups; partial sums are added in a
+ * fixed order.  The same holds from 33 rows on.
+ * Without one (or where no split pays, or fp32) the call is forwarded to raven_gemm / _adapter_gemm_concat / _gemm_swiglu. */
 size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max);
 int    raven_linear(const void* x0, const void* x1, const void* w, const void* residual, void* y,
                     int32_t M, int32_t N, int32_t K0, int32_t K1, int32_t swiglu, int32_t out_f32,

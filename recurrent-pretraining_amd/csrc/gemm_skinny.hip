@@ -6,8 +6,8 @@
 //                of W, reads them with 16-byte lane-contiguous loads and accumulates with
 //                v_dot2_f32_bf16 / fp32 FMA; a DPP wave reduction finishes each row.
 //   mfma_kernel  (bf16, up to 32 rows of X per pass)   -- 16-row tiles of W are the A operand of
-//                v_mfma_f32_16x16x32_bf16, X is the B operand; the four waves of a workgroup split
-//                K and reduce through LDS.
+//                v_mfma_f32_16x16x32_bf16, X is the B operand; the four or eight waves of a workgroup
+//                split K and reduce through LDS.
 //   rows_f32_kernel (float, 2 rows and more)          -- 16 rows of W against 16 to 64 rows of X on v_mfma_f64_16x16x4_f64.
 // Epilogues (all round the fp32 accumulator to T first, as an nn.Linear output would be stored):
 //   plain (+ residual add in T, + optional float store)   RMM:493, 509, 711, 534-535

@@ -1,4 +1,4 @@
-// Skinny bf16 GEMM for 5..32 token rows with a caller-provided workspace: Y[M,N] = X[M,K] W[N,K]^T.
+// Skinny bf16 GEMM for 2..32 token rows with a caller-provided workspace: Y[M,N] = X[M,K] W[N,K]^T, where K slices pay (splits_k).
 //
 // The four waves of a workgroup own four different 16-row weight tiles (a gate tile and an up tile each
 // for the SwiGLU epilogue) and walk the SAME K range, so the X tile of a macro-step (128 k-values) is
