@@ -11,6 +11,8 @@
 // are read once and not once per row that picked it: 20 rows over 64 experts of 768 channels at width 2048, 6 each, read
 // 55 experts instead of 120 (246 us before, 124 now).
 
+#include <algorithm>
+
 #include "gemm_common.h"
 #include "row_helpers.h"
 
@@ -397,12 +399,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
 // channels, 6 per row and a shared one), row kernels / grouped: 2 rows 31 / 34, 3: 45 / 42, 4: 59 / 55, 8: 105 / 78, 20: 246 / 124;
 // width 1024: 4 rows 22 / 26, 6: 29 / 27, 8: 38 / 31, 20: 80 / 40 -- the lines cross where rows would read 25 MB again.
 enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
+static bool few_rows_fit(const raven_moe* m, int M) {
+    return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs;
+}
 static MoePath moe_path(const raven_moe* m, int M, int ld, int dtype) {
     if (dtype != RAVEN_BF16) return kMoeRows;
     const double pairs = (double)M * m->top;
     if (M > 8 && (pairs >= 2.0 * m->experts || M > 128)) return kMoeChunk;
-    const bool fold = !m->shared_up || m->shared_ff == m->ff;
-    if (!fold || M < 2 || M > kRouteRows || pairs > kRoutePairs) return kMoeRows;
+    if (!few_rows_fit(m, M)) return kMoeRows;
     const double touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), again = pairs - touched + (m->shared_up ? M - 1 : 0);
     return again * 6.0 * ld * m->ff > kMoeBytesAgain ? kMoeFew : kMoeRows;
 }
@@ -415,7 +419,7 @@ struct MoeChunk {
     size_t lin_bytes;
     int n_tiles, tile_rows;
 };
-static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, char* base, MoeChunk* out) {
+static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, MoePath path, char* base, MoeChunk* out) {
     const size_t es = raven_host::elt_size(dtype), pairs = (size_t)M * m->top;
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -424,7 +428,6 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, char* base
         return p;
     };
     MoeChunk c{};
-    const MoePath path = moe_path(m, M, ld, dtype);
     if (path == kMoeRows) {
         c.act = take((size_t)M * (m->top * (size_t)m->ff + m->shared_ff) * es);
         c.pick = (int*)take(pairs * 4);
@@ -437,15 +440,17 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, char* base
         // tokens: 80 / 70 / 63 / 83, 1500: 144 / 109 / 94 / 96.  (128-row tiles of eight waves, as before: 230 at 500, 327 at 1500.)
         const size_t mean = pairs / m->experts;
         c.tile_rows = path == kMoeFew || mean <= 6 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows ? 64 : 256;
-        c.n_tiles = (int)(pairs / c.tile_rows) + m->experts + (fold ? (M + c.tile_rows - 1) / c.tile_rows : 0);
+        auto tiles = [&](int height) { return (int)(pairs / height) + m->experts + (fold ? (M + height - 1) / height : 0); };
+        c.n_tiles = tiles(c.tile_rows);
+        const size_t table = (size_t)tiles(16) * 4;  // room for the lowest tiles whatever the height, so that more rows never need less
         c.pick = (int*)take(pairs * 4);
         c.pick_scale = (float*)take(pairs * 4);
         c.slot_of = (int*)take(pairs * 4);
         c.slot_row = (int*)take(rows * 4);
         c.slot_scale = (float*)take(rows * 4);
-        c.group_of = (int*)take((size_t)c.n_tiles * 4);
-        c.group_row = (int*)take((size_t)c.n_tiles * 4);
-        c.group_end = (int*)take((size_t)c.n_tiles * 4);
+        c.group_of = (int*)take(table);
+        c.group_row = (int*)take(table);
+        c.group_end = (int*)take(table);
         c.used = (int*)take(4);
         c.block_count = (int*)take((size_t)((M + kPickRows - 1) / kPickRows) * m->experts * 4);
         c.act = take(rows * m->ff * es);
@@ -461,6 +466,17 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, char* base
     }
     if (out) *out = c;
     return off;
+}
+
+// Room for M rows and for any smaller number: a grouped call over few rows keeps float slots and can need more than row kernels or a
+// chunk over more rows do (64 experts, 8 per row, no shared one: 15 rows 1.17 MB, 16 rows 0.73)
+static size_t moe_workspace(const raven_moe* m, int M, int ld, int dtype) {
+    size_t need = carve_moe(m, M, ld, dtype, kMoeRows, nullptr, nullptr);
+    if (dtype != RAVEN_BF16) return need;
+    const int few = M < kRouteRows ? M : kRouteRows;
+    if (few_rows_fit(m, few)) need = std::max(need, carve_moe(m, few, ld, dtype, kMoeFew, nullptr, nullptr));
+    if (moe_path(m, M, ld, dtype) == kMoeChunk) need = std::max(need, carve_moe(m, M, ld, dtype, kMoeChunk, nullptr, nullptr));
+    return need;
 }
 
 static int check_moe(const char* who, const raven_moe* m, int M, int ld, int dtype) {
@@ -486,7 +502,7 @@ static int run_moe_rows(const MoeArgs& a, hipStream_t s) {
 
 extern "C" size_t raven_moe_workspace_bytes(const raven_moe* m, int32_t M, int32_t ld, int32_t dtype) {
     if (raven::check_moe("moe_workspace_bytes", m, M, ld, dtype) || M == 0) return 0;
-    return raven::carve_moe(m, M, ld, dtype, nullptr, nullptr);
+    return raven::moe_workspace(m, M, ld, dtype);
 }
 
 namespace raven {
@@ -496,15 +512,15 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
     if (const int rc = check_moe("moe", m, M, ld, dtype)) return rc;
     if (M == 0) return 0;
     RAVEN_REQUIRE(m->up && m->down && (h || (norm && M == 1)) && logits && x, "moe: null pointer");
-    RAVEN_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0 && carve_moe(m, M, ld, dtype, nullptr, nullptr) <= workspace_bytes,
+    const MoePath path = moe_path(m, M, ld, dtype);
+    RAVEN_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0 && carve_moe(m, M, ld, dtype, path, nullptr, nullptr) <= workspace_bytes,
                   "moe: workspace of %zu bytes is too small or unaligned", workspace_bytes);
     MoeChunk c;
-    carve_moe(m, M, ld, dtype, static_cast<char*>(workspace), &c);
+    carve_moe(m, M, ld, dtype, path, static_cast<char*>(workspace), &c);
     MoeArgs a{};
     a.h = h; a.up = m->up; a.down = m->down; a.shared_up = m->shared_up; a.shared_down = m->shared_down;
     a.logits = logits; a.x = x; a.act = c.act; a.norm = norm; a.dim = dim; a.eps = eps; a.pick = c.pick;
     a.M = M; a.ld = ld; a.ldl = m->logit_ld; a.experts = m->experts; a.top = m->top; a.ff = m->ff; a.sff = m->shared_ff;
-    const MoePath path = moe_path(m, M, ld, dtype);
     if (path == kMoeRows) {
         RAVEN_REQUIRE(M <= 65535, "moe: %d rows in one call", M);
         return dtype == RAVEN_BF16 ? run_moe_rows<bf16>(a, s) : run_moe_rows<float>(a, s);

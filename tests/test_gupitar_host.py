@@ -165,3 +165,15 @@ def test_oracle_mixture_scales_the_experts_input():
         assert torch.allclose(out[t], want, atol=1e-5)
     assert torch.allclose(O.gelu_tanh(h), torch.nn.functional.gelu(h, approximate="tanh"), atol=1e-6)
     assert torch.allclose(O.centred_norm(h, torch.zeros(D), 0.0).pow(2).mean(-1), torch.ones(7), atol=1e-5)
+
+
+@pytest.mark.parametrize("D,E,top,ff,shared", [(2048, 64, 8, 768, False), (1024, 300, 4, 264, True), (1024, 64, 1, 1024, True), (4096, 8, 2, 4096, False), (8, 1024, 1, 8, False),
+                                               (264, 12, 2, 136, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_mixture_workspace_for_more_rows_serves_fewer(pkg, D, E, top, ff, shared, dtype):
+    """A decode loop sizes its buffers for the most sequences and then runs with fewer: the size never shrinks with the rows, across the
+    borders between the row kernels, the grouped product of few rows (float slots) and chunks with tiles of every height."""
+    one = 1 if shared else None   # only whether there is a shared expert matters here
+    desc = pkg.hip.Moe(1, 1, 1, one, one, E, top, ff, ff if shared else 0, E + 16)
+    sizes = [pkg.hip.load().raven_moe_workspace_bytes(desc, M, D, pkg.hip.dtype_code(dtype)) for M in [*range(1, 700), 1000, 1500, 4096, 20000, 40000]]
+    assert sizes[0] > 0 and sizes == sorted(sizes)
