@@ -808,7 +808,7 @@ extern "C" int raven_qkv_bias_rope_cache_append(const void* qkv, const void* qk_
 
 namespace raven {
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
 int tiled_gemm_qkv_rope(const void* x, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out, void* k_cache,
                         void* v_cache, int64_t slot_off, int nh, int hd, int t_max, int M, int S, int K, int ldx, int pos0,
                         const int* pos_dev, void* workspace, size_t workspace_bytes, hipStream_t s);
@@ -821,7 +821,7 @@ int qkv_linear_rope_append(const void* x, int ldx, const void* wqkv, const void*
                            int head_dim, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* done) {
     *done = 0;
     const int M = B * S, h = n_heads * head_dim;
-    if (!g_fuse_qkv_rope || dtype != RAVEN_BF16 || M < g_tiled_min_rows || head_dim % 8 != 0 || !tiled_gemm_fits(M, 3 * h, h, 0, dtype, 0, workspace_bytes)) return 0;
+    if (!g_fuse_qkv_rope || dtype != RAVEN_BF16 || M < g_tiled_min_rows || head_dim % 8 != 0 || !tiled_gemm_fits(M, 3 * h, h, 0, dtype, 0, workspace_bytes, raven_host::aligned16(x, wqkv, qk_bias, freqs, q_out))) return 0;
     if (int rc = check_heads("qkv_append", n_heads, head_dim, dtype)) return rc;
     RAVEN_REQUIRE(x && wqkv && freqs && q_out, "qkv_append: null pointer");
     RAVEN_REQUIRE(B > 0 && S > 0 && pos0 >= 0, "qkv_append: bad B=%d S=%d pos0=%d", B, S, pos0);

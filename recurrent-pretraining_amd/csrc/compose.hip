@@ -39,7 +39,7 @@ int qkv_linear_rope_append(const void* x, int ldx, const void* wqkv, const void*
                            int head_dim, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* done);
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int rmsnorm_pitched(const void* x, const void* residual, const void* weight, void* y, int ldy, void* sum_out, const void* weight2,
@@ -155,12 +155,15 @@ static bool chunk_on_matrix_cores(const raven_dims* d, const raven_kv_cache* cac
 
 // Rows of n_embd bf16 values that are not whole cache lines (5280: 82.5 lines): norm_1's and norm_3's output and the
 // attention output, which the products over many rows read, are laid out with rows padded to whole lines (the pad
-// is never read: the products' K stays n_embd).  The row pitch of these; every block of a call decides this the same way.
-static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const raven_kv_cache* cache, int M, int S, bool paged) {
+// is never read: the products' K stays n_embd).  The row pitch of these, decided once for all blocks of a call.
+static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const raven_block_weights* blocks, int n_blocks, const void* x_in,
+                           const raven_kv_cache* cache, int M, int S, bool paged) {
     const int h = d->n_embd, dt = d->dtype;
-    const bool pad = g_pad_chunk_rows && chunk_on_matrix_cores(d, cache, S, paged) && s.ld_pad != h && M >= g_tiled_min_rows &&
-                     tiled_gemm_fits(M, 3 * h, h, 0, dt, 0, s.lin_ws_bytes) && tiled_gemm_fits(M, h, h, 0, dt, 0, s.lin_ws_bytes) &&
-                     tiled_gemm_fits(M, d->intermediate, h, 0, dt, 1, s.lin_ws_bytes);
+    if (!g_pad_chunk_rows || !chunk_on_matrix_cores(d, cache, S, paged) || s.ld_pad == h || M < g_tiled_min_rows) return h;
+    bool aligned = raven_host::aligned16(x_in);
+    for (int j = 0; j < n_blocks; ++j) aligned = aligned && raven_host::aligned16(blocks[j].wqkv, blocks[j].proj, blocks[j].fc);
+    const bool pad = tiled_gemm_fits(M, 3 * h, h, 0, dt, 0, s.lin_ws_bytes, aligned) && tiled_gemm_fits(M, h, h, 0, dt, 0, s.lin_ws_bytes, aligned) &&
+                     tiled_gemm_fits(M, d->intermediate, h, 0, dt, 1, s.lin_ws_bytes, aligned);
     return pad ? s.ld_pad : h;
 }
 
@@ -170,12 +173,12 @@ static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const rav
 static int run_block(const raven_dims* d, const raven_block_weights* w, const BlockScratch& s, bool n1_ready,
                      const void* x_in, void* y_out, const void* tail_w, void* tail_out, const float* freqs,
                      const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, void* stream,
-                     const raven_paged_kv* paged = nullptr, int layer = 0, int ld_decode = 0) {
+                     const raven_paged_kv* paged, int layer, int ld_decode, int ld_chunk) {
     const int M = B * S, h = d->n_embd, I = d->intermediate, dt = d->dtype;
     hipStream_t hs = static_cast<hipStream_t>(stream);
     int rc;
     const bool chunk = !paged && S > 1, mfma = chunk_on_matrix_cores(d, cache, S, paged != nullptr);
-    const bool pad = chunk_row_pitch(d, s, cache, M, S, paged != nullptr) != h;
+    const bool pad = ld_chunk != h;  // (chunk_row_pitch)
     // Decode steps of 17..32 rows: the MFMA kernels of Wqkv and mlp.fc stream 5 % faster over operands with rows of whole
     // lines (fc 67.9 -> 64.5 us, Wqkv 33.1 -> 31.6 at 32 rows; no gain at 8).  Where the caller has registered line-aligned
     // copies of both matrices, the two products run over the padded length: the copies' pad columns are zeros, and so are
@@ -290,9 +293,9 @@ extern "C" int raven_sandwich_block(const raven_dims* dims, const raven_block_we
         if (int rc = run_block_one_row(dims, w, s, x_in, nullptr, freqs, cache, slot, pos0, pos_dev, stream)) return rc;
         return close_one_row(dims, s, w->norm_4, ln_f, x_out, stream);
     }
-    const int ld_decode = decode_row_pitch(dims, s, w, 1, B * S, S, false);
-    if (ln_f) return run_block(dims, w, s, false, x_in, nullptr, ln_f, x_out, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode);
-    return run_block(dims, w, s, false, x_in, x_out, nullptr, nullptr, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode);
+    const int ld_decode = decode_row_pitch(dims, s, w, 1, B * S, S, false), ld_chunk = chunk_row_pitch(dims, s, w, 1, x_in, cache, B * S, S, false);
+    if (ln_f) return run_block(dims, w, s, false, x_in, nullptr, ln_f, x_out, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode, ld_chunk);
+    return run_block(dims, w, s, false, x_in, x_out, nullptr, nullptr, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode, ld_chunk);
 }
 
 namespace raven {
@@ -362,7 +365,8 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
         if ((rc = linear_column_block(embeds, static_cast<const char*>(adapter_w) + (size_t)h * 2, 2 * h, nullptr, s.e_sums, 1, M, h, h,
                                       s.lin_ws, s.lin_ws_bytes, hs))) return rc;
     const int ld_decode = decode_row_pitch(dims, s, blocks, n_blocks, M, S, paged != nullptr);
-    const int ld_n1 = ld_decode ? ld_decode : chunk_row_pitch(dims, s, cache, M, S, paged != nullptr);  // rows of norm_1's output as run_block reads them
+    const int ld_chunk = chunk_row_pitch(dims, s, blocks, n_blocks, state_in, cache, M, S, paged != nullptr);
+    const int ld_n1 = ld_decode ? ld_decode : ld_chunk;  // rows of norm_1's output as run_block reads them
     for (int it = 0; it < n_iterations; ++it) {
         const int32_t* sl = slots ? slots + (size_t)it * n_blocks : nullptr;
         const bool last_it = it == n_iterations - 1;
@@ -389,7 +393,7 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
             const void* tail_w = last ? lnw : blocks[j + 1].norm_1;
             void* tail_out = last ? (lnw ? state_out : nullptr) : s.n1;
             if ((rc = run_block(dims, &blocks[j], s, j > 0 || n1_ready, x_in, y_out, tail_w, tail_out, freqs, cache, sl ? sl[j] : 0, B, S, pos0,
-                                pos_dev, stream, paged, j, ld_decode))) return rc;
+                                pos_dev, stream, paged, j, ld_decode, ld_chunk))) return rc;
         }
     }
     return 0;

@@ -25,7 +25,7 @@ extern "C" int raven_gemv_fused(const void* x0, const void* x1, const void* norm
 namespace raven {
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 
@@ -834,7 +834,7 @@ extern "C" int raven_gemm(const void* x, const void* w, const void* residual, vo
     if (int rc = check_common("gemm", M, N, K, dtype)) return rc;
     if (M == 0) return 0;
     RAVEN_REQUIRE(x && w && y, "gemm: null pointer");
-    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K, 0, dtype, 0, 0))
+    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K, 0, dtype, 0, 0, raven_host::aligned16(x, w, residual, y)))
         return tiled_gemm(x, 0, nullptr, w, residual, y, M, N, K, 0, 0, out_f32, nullptr, 0, static_cast<hipStream_t>(stream), nullptr);
     GemmArgs a{};
     a.w = w; a.x0 = x; a.x1 = nullptr; a.residual = residual; a.y = y;
@@ -850,7 +850,7 @@ extern "C" int raven_adapter_gemm_concat(const void* x0, const void* x1, const v
     RAVEN_REQUIRE(x0 && x1 && w && y, "adapter: null pointer");
     const int elts = 16 / (int)raven_host::elt_size(dtype);
     RAVEN_REQUIRE(K0 > 0 && K1 > 0 && K0 % elts == 0 && K1 % elts == 0, "adapter: K0=%d, K1=%d must be positive multiples of %d", K0, K1, elts);
-    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, 0))
+    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, 0, raven_host::aligned16(x0, x1, w, y)))
         return tiled_gemm(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, 0, nullptr, 0, static_cast<hipStream_t>(stream), nullptr);
     GemmArgs a{};
     a.w = w; a.x0 = x0; a.x1 = x1; a.residual = nullptr; a.y = y;
@@ -864,7 +864,7 @@ extern "C" int raven_gemm_swiglu(const void* x, const void* fc, void* out, int32
     if (int rc = check_common("gemm_swiglu", M, I, K, dtype)) return rc;
     if (M == 0) return 0;
     RAVEN_REQUIRE(x && fc && out, "gemm_swiglu: null pointer");
-    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, I, K, 0, dtype, 1, 0))
+    if (M >= g_tiled_min_rows && tiled_gemm_fits(M, I, K, 0, dtype, 1, 0, raven_host::aligned16(x, fc, out)))
         return tiled_gemm(x, 0, nullptr, fc, nullptr, out, M, I, K, 0, 1, 0, nullptr, 0, static_cast<hipStream_t>(stream), nullptr);
     GemmArgs a{};
     a.w = fc; a.x0 = x; a.x1 = nullptr; a.residual = nullptr; a.y = out;

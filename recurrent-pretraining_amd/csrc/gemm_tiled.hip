@@ -842,13 +842,14 @@ static MidPlan mid_choice(int M, int N, int K0, int K1, int swiglu, size_t works
 // kernels, 32 rows per pass over the weights -- up to two passes at K = 5280, four at 10560 and five (160 rows) at 17920, where
 // the passes' split over K still beats one round of 128 x 128 tiles walking the whole of K (measured at 33 .. 160 rows: Wqkv
 // 98 / 130 us in three / four passes against 75 / 81 tiled, mlp.proj 172 against 199).
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes) {
+// aligned: whether all operands start on 16 bytes, which the kernels over many rows need; the passes take any address.
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned) {
     const bool ok = dtype == RAVEN_BF16 && M >= 1 && N % 8 == 0 && K0 % 8 == 0 && K0 > 0 && (K1 == 0 || K1 == K0) &&
                     (int64_t)M * (K0 > K1 ? K0 : K1) < (1ll << 31) && (int64_t)N * 2 * (K0 + K1) < (1ll << 31);
     if (!ok) return false;
     const int64_t small_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int passes = (K0 + K1 + 3499) / 3500;
-    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) return mid_choice(M, N, K0, K1, swiglu, workspace_bytes).nt != 0;
+    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) return aligned && mid_choice(M, N, K0, K1, swiglu, workspace_bytes).nt != 0;
     return true;
 }
 
@@ -884,7 +885,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
                            int K1, int swiglu, int out_f32, const RopeAppend* rope, void* workspace, size_t workspace_bytes, hipStream_t s,
                            const raven_epilogue* epi = nullptr, int* ks_left = nullptr) {
     if (ks_left) *ks_left = 0;
-    RAVEN_REQUIRE(tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
+    RAVEN_REQUIRE(tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32)), "gemm (tiled): the SwiGLU epilogue has no residual and stores bf16");
     RAVEN_REQUIRE(((uintptr_t)x0 & 15) == 0 && ((uintptr_t)x1 & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
                       ((uintptr_t)residual & 15) == 0, "gemm (tiled): operands must be 16-byte aligned");

@@ -195,6 +195,7 @@ void set_error(const char* fmt, ...);
 int  check_launch(const char* what);
 inline size_t elt_size(int dtype) { return dtype == RAVEN_BF16 ? 2 : 4; }
 inline size_t align_up(size_t x, size_t a = 256) { return (x + a - 1) / a * a; }
+template <typename... P> inline bool aligned16(const P*... p) { return (((uintptr_t)p | ...) & 15) == 0; }
 }  // namespace raven_host
 
 #define RAVEN_REQUIRE(cond, ...)                 \

@@ -175,6 +175,17 @@ def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, 
         assert torch.equal(pkg.hip.linear(x, w, workspace=ws), pkg.hip.linear(x, w, workspace=ws))
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 256, 4096), (100, 1024, 11008)])
+def test_a_residual_off_sixteen_bytes(pkg, M, N, K):
+    """The middle kernel loads whole 16-byte pieces; rows that the kernels of up to 32 rows can take in passes go there instead."""
+    dt = torch.bfloat16
+    x, w = _gpu_randn((M, K), 710), _gpu_randn((N, K), 711, 0.05)
+    res = _gpu_randn((M * N + 1,), 712)[1:].view(M, N)
+    z = x.float() @ w.float().T
+    for ws in (None, pkg.hip.linear_workspace(M, N, "cuda")):
+        check(pkg.hip.linear(x, w, residual=res, workspace=ws), (z.to(dt).float() + res.float()).to(dt), dt, "residual", mag=z, ulps=ULPS_RESIDUAL)
+
+
 @pytest.mark.parametrize("M", [40, 100])
 def test_slices_of_many_rows_folded_into_the_norm_change_no_bit(pkg, tuned, M):
     """A block over 33 and more rows at widths whose attn.proj and mlp.proj are cut into K slices: the norm launch adds them

@@ -46,6 +46,25 @@ def test_library_identity_and_argument_errors(pkg):
     assert 0 < n1 < n32 and n1 % 256 == 0
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where nothing can be launched")
+@pytest.mark.parametrize("shift", ["x", "w", "residual", "y"])
+@pytest.mark.parametrize("M,N,K", [(40, 256, 4096), (100, 1024, 11008), (160, 2048, 17920)])
+def test_operands_off_sixteen_bytes_are_refused_by_no_product(pkg, M, N, K, shift):
+    """Rows past 32 that the kernels of up to 32 rows take in passes accept operands at any address; those kernels must stay the ones that run.
+    Without a GPU a call that passes all checks ends with a runtime error (> 0), a refused one with a negative code."""
+    lib = pkg.hip.load()
+    at = {k: 0x100000 * (i + 1) + (2 if k == shift else 0) for i, k in enumerate(["x", "w", "residual", "y"])}
+    ws = 0x10000000
+    codes = [lib.raven_gemm(at["x"], at["w"], at["residual"], at["y"], M, N, K, 1, 0, None),
+             lib.raven_gemm_swiglu(at["x"], at["w"], at["y"], M, N // 2, K, 1, None),
+             lib.raven_adapter_gemm_concat(at["x"], 0x800000, at["w"], at["y"], M, N, K // 2, K // 2, 1, None)]
+    for room in (0, 1 << 30):
+        codes.append(lib.raven_linear(at["x"], None, at["w"], at["residual"], at["y"], M, N, K, 0, 0, 0, 1, ws, room, None))
+        epi = pkg.hip.Epilogue(None, None, 1.0, 0, 0)
+        codes.append(lib.raven_linear_epilogue(at["x"], None, at["w"], at["y"], M, N, K, 0, ctypes.byref(epi), 1, ws, room, None))
+    assert all(rc > 0 for rc in codes), (codes, lib.raven_last_error())
+
+
 def test_wrappers_refuse_cpu_tensors(pkg):
     x = torch.zeros(1, 16)
     with pytest.raises(pkg.hip.RavenHipError, match="GPU"):
