@@ -399,14 +399,18 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
 // channels, 6 per row and a shared one), row kernels / grouped: 2 rows 31 / 34, 3: 45 / 42, 4: 59 / 55, 8: 105 / 78, 20: 246 / 124;
 // width 1024: 4 rows 22 / 26, 6: 29 / 27, 8: 38 / 31, 20: 80 / 40 -- the lines cross where rows would read 25 MB again.
 enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
-static bool few_rows_fit(const raven_moe* m, int M) {
-    return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs;
+constexpr size_t kMoeRowLds = 64 * 1024 - 1024;  // what a row may take of the row kernels' LDS; longer ones are refused for few rows
+static bool few_rows_fit(const raven_moe* m, int M, int ld) {
+    return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs && ld * sizeof(bf16) <= kMoeRowLds &&
+           (int64_t)2 * m->ff * ld < (1ll << 31);
 }
-static MoePath moe_path(const raven_moe* m, int M, int ld, int dtype) {
-    if (dtype != RAVEN_BF16) return kMoeRows;
+// h: the rows, or null where only sizes are asked for.  The grouped kernels move whole 16-byte pieces into the LDS; operands that do not start
+// on one stay with the row kernels, which take any address.
+static MoePath moe_path(const raven_moe* m, const void* h, int M, int ld, int dtype) {
+    if (dtype != RAVEN_BF16 || !raven_host::aligned16(h, m->up, m->down, m->shared_up, m->shared_down)) return kMoeRows;
     const double pairs = (double)M * m->top;
     if (M > 8 && (pairs >= 2.0 * m->experts || M > 128)) return kMoeChunk;
-    if (!few_rows_fit(m, M)) return kMoeRows;
+    if (!few_rows_fit(m, M, ld)) return kMoeRows;
     const double touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), again = pairs - touched + (m->shared_up ? M - 1 : 0);
     return again * 6.0 * ld * m->ff > kMoeBytesAgain ? kMoeFew : kMoeRows;
 }
@@ -474,8 +478,8 @@ static size_t moe_workspace(const raven_moe* m, int M, int ld, int dtype) {
     size_t need = carve_moe(m, M, ld, dtype, kMoeRows, nullptr, nullptr);
     if (dtype != RAVEN_BF16) return need;
     const int few = M < kRouteRows ? M : kRouteRows;
-    if (few_rows_fit(m, few)) need = std::max(need, carve_moe(m, few, ld, dtype, kMoeFew, nullptr, nullptr));
-    if (moe_path(m, M, ld, dtype) == kMoeChunk) need = std::max(need, carve_moe(m, M, ld, dtype, kMoeChunk, nullptr, nullptr));
+    if (few_rows_fit(m, few, ld)) need = std::max(need, carve_moe(m, few, ld, dtype, kMoeFew, nullptr, nullptr));
+    if (moe_path(m, nullptr, M, ld, dtype) == kMoeChunk) need = std::max(need, carve_moe(m, M, ld, dtype, kMoeChunk, nullptr, nullptr));
     return need;
 }
 
@@ -491,7 +495,7 @@ static int check_moe(const char* who, const raven_moe* m, int M, int ld, int dty
 template <typename T>
 static int run_moe_rows(const MoeArgs& a, hipStream_t s) {
     const size_t lds = (size_t)a.ld * sizeof(T);
-    RAVEN_REQUIRE(lds <= 64 * 1024 - 1024, "moe: rows of %d channels do not fit the LDS", a.ld);
+    RAVEN_REQUIRE(lds <= kMoeRowLds, "moe: rows of %d channels do not fit the LDS", a.ld);
     const int total = a.top * a.ff + a.sff;
     moe_up_kernel<T><<<dim3((total + 3) / 4, a.M), dim3(256), lds, s>>>(a);
     moe_down_kernel<T><<<dim3((a.ld + 3) / 4, a.M), dim3(256), 0, s>>>(a);
@@ -512,7 +516,7 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
     if (const int rc = check_moe("moe", m, M, ld, dtype)) return rc;
     if (M == 0) return 0;
     RAVEN_REQUIRE(m->up && m->down && (h || (norm && M == 1)) && logits && x, "moe: null pointer");
-    const MoePath path = moe_path(m, M, ld, dtype);
+    const MoePath path = moe_path(m, h, M, ld, dtype);
     RAVEN_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0 && carve_moe(m, M, ld, dtype, path, nullptr, nullptr) <= workspace_bytes,
                   "moe: workspace of %zu bytes is too small or unaligned", workspace_bytes);
     MoeChunk c;

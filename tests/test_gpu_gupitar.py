@@ -375,6 +375,33 @@ def test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, same):
     assert ((outs[0].double() - x.double() - want).norm() / want.norm()).item() < 5e-3
 
 
+@pytest.mark.parametrize("M", [1, 3, 20, 200])
+@pytest.mark.parametrize("which", ["h", "up", "down", "shared"])
+def test_mixture_operands_off_sixteen_bytes(pkg, M, which):
+    """Operands at odd addresses, where the grouped kernels' whole pieces do not start, at row counts of every path."""
+    D, E, top, ff = 264, 16, 2, 136
+    g = torch.Generator(device="cuda").manual_seed(M)
+    def rand(off, *s):
+        n = math.prod(s)
+        return (torch.randn(n + 8, generator=g, device="cuda") * s[-1] ** -0.5).to(BF16)[off:off + n].view(s)
+    up, down = rand(which == "up", E, 2 * ff, D), rand(3 * (which == "down"), E, D, ff)
+    sup, sdown = rand(which == "shared", 2 * ff, D), rand(5 * (which == "shared"), D, ff)
+    h = rand(which == "h", M, D) * D ** 0.5 if which != "h" else rand(1, M, D)
+    ldl = 32
+    logits, x = torch.randn(M, ldl, generator=g, device="cuda"), torch.randn(M, D, generator=g, device="cuda")
+    desc = pkg.hip.Moe(up.data_ptr(), up.data_ptr(), down.data_ptr(), sup.data_ptr(), sdown.data_ptr(), E, top, ff, ff, ldl)
+    s, index = torch.sigmoid(logits[:, :E].double()).topk(top, 1)
+    gated = lambda a, u, d: (torch.nn.functional.silu(a @ u[:ff].double().T) * (a @ u[ff:].double().T)) @ d.double().T
+    want = torch.sigmoid(logits[:, E:E + 1].double()) * gated(h.double(), sup, sdown)
+    for e in range(E):
+        row, place = torch.where(index == e)
+        if len(row):
+            want[row] += gated(s[row, place, None] * h[row].double(), up[e], down[e])
+    stream = x.clone()
+    pkg.hip.moe(desc, h, logits, stream)
+    assert ((stream.double() - x.double() - want).norm() / want.norm()).item() < 5e-3   # activations rounded to bf16 once, as beside
+
+
 @DT
 @pytest.mark.parametrize("M", [1, 20])
 def test_mixture_prefers_the_lower_index_among_equals(pkg, dtype, M):
