@@ -715,18 +715,27 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
     return raven_host::check_launch("mfma gemm");
 }
 
-// Float rows: all of them in one launch.  A few rows against a matrix that does not fit the caches stay with the vector kernel, whose
-// whole-row loads stream twice as fast (5.5 TB/s): up to 8 rows from 32 MB on.
+// Float rows: all of them in one launch (per 4 194 240, what a grid holds).  A few rows against a matrix that does not fit the caches stay with
+// the vector kernel, whose whole-row loads stream twice as fast (5.5 TB/s): up to 8 rows from 32 MB on.
 template <int EPI>
 static int launch_rows_f32(GemmArgs a, hipStream_t s) {
     a.ldy = a.N;
-    const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
-    const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));
-    RAVEN_REQUIRE(grid.y <= 65535, "gemm: %d rows in one call", a.M);
-    if (mt == 1) rows_f32_kernel<EPI, 1><<<grid, dim3(256), 0, s>>>(a);
-    else if (mt == 2) rows_f32_kernel<EPI, 2><<<grid, dim3(256), 0, s>>>(a);
-    else rows_f32_kernel<EPI, 4><<<grid, dim3(256), 0, s>>>(a);
-    return raven_host::check_launch("gemm (fp32 rows)");
+    const int M = a.M, mt = M <= 16 ? 1 : M <= 32 ? 2 : 4, most = 65535 * 16 * mt;
+    for (int m0 = 0; m0 < M; m0 += most) {
+        a.M = M - m0 < most ? M - m0 : most;
+        const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));
+        if (mt == 1) rows_f32_kernel<EPI, 1><<<grid, dim3(256), 0, s>>>(a);
+        else if (mt == 2) rows_f32_kernel<EPI, 2><<<grid, dim3(256), 0, s>>>(a);
+        else rows_f32_kernel<EPI, 4><<<grid, dim3(256), 0, s>>>(a);
+        if (const int rc = raven_host::check_launch("gemm (fp32 rows)")) return rc;
+        a.x0 = static_cast<const float*>(a.x0) + (size_t)a.M * a.k0;
+        if (a.x1) a.x1 = static_cast<const float*>(a.x1) + (size_t)a.M * a.k1;
+        if (a.residual) a.residual = static_cast<const float*>(a.residual) + (size_t)a.M * a.N;
+        if (a.epi.residual) a.epi.residual += (size_t)a.M * a.N;
+        a.y = static_cast<float*>(a.y) + (size_t)a.M * a.N;
+        if (m0 > M - most) break;  // (the next start may not fit an int)
+    }
+    return 0;
 }
 
 // Runs one GEMM over all M rows, in passes of at most 32 (MFMA) or 8 / 4 (vector) rows.
@@ -736,6 +745,7 @@ static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
     const bool mfma_ok = dtype == RAVEN_BF16 && a.K % 32 == 0 && a.k0 % 32 == 0 && a.N % 16 == 0;
     const int M = a.M;
     const size_t out_es = a.out_f32 ? 4 : es;
+    RAVEN_REQUIRE(dtype != RAVEN_F32 || (size_t)a.K * es <= 160 * 1024, "gemm: one row of K=%d elements does not fit the 160 KB LDS", a.K);
     if (dtype == RAVEN_F32 && M >= 2 && (M > 8 || (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20))) return launch_rows_f32<EPI>(a, s);
     for (int m0 = 0; m0 < M;) {
         const int left = M - m0;

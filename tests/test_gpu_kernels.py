@@ -215,6 +215,18 @@ def test_fp32_rows_in_one_launch(pkg, M, N, K0, K1):
     assert torch.isfinite(got[1:]).all() and not torch.isfinite(got[0]).any()
 
 
+def test_more_fp32_rows_than_one_grid_holds(pkg):
+    M, N, K = 65535 * 64 + 17, 3, 4
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w, res = (torch.randn(*s, device="cuda", generator=g) for s in ((M, K), (N, K), (M, N)))
+    want = x.double() @ w.double().T
+    rel = lambda got, ref: ((got.double() - ref).norm(dim=0) / ref.norm(dim=0)).max().item()
+    tail = slice(M - 100, None)
+    for rows in (slice(None), tail):  # the second launch's rows on their own: they would not show in the whole norm
+        assert rel(pkg.hip.linear(x, w)[rows], want[rows]) < 6e-8
+        assert rel(pkg.hip.linear_epilogue(x, w, residual=res)[rows], (want + res)[rows]) < 2e-7
+
+
 @pytest.mark.parametrize("dt,M,h", [(torch.bfloat16, 1, 5280), (torch.bfloat16, 32, 5280), (torch.bfloat16, 6, 64),
                                     (torch.float32, 1, 256), (torch.float32, 12, 256)])
 def test_adapter_concat(pkg, dt, M, h):

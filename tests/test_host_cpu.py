@@ -65,6 +65,19 @@ def test_operands_off_sixteen_bytes_are_refused_by_no_product(pkg, M, N, K, shif
     assert all(rc > 0 for rc in codes), (codes, lib.raven_last_error())
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where nothing can be launched")
+@pytest.mark.parametrize("M", [1, 2, 9, 17, 100, 5_000_000])
+def test_float_products_take_rows_of_one_length_whatever_their_number(pkg, M):
+    """40960 values are the longest row of the vector kernel, and of every float product; the number of rows has no limit of its own."""
+    lib = pkg.hip.load()
+    epi = pkg.hip.Epilogue(None, None, 1.0, 0, 1)
+    for K, ok in ((4, True), (40960, True), (40964, False)):
+        codes = [lib.raven_gemm(0x1000, 0x2000, None, 0x3000, M, 16, K, 0, 0, None), lib.raven_gemm_swiglu(0x1000, 0x2000, 0x3000, M, 16, K, 0, None),
+                 lib.raven_linear(0x1000, None, 0x2000, None, 0x3000, M, 16, K, 0, 0, 0, 0, None, 0, None),
+                 lib.raven_linear_epilogue(0x1000, None, 0x2000, 0x3000, M, 16, K, 0, ctypes.byref(epi), 0, None, 0, None)]
+        assert all((rc > 0) == ok for rc in codes), (K, codes, lib.raven_last_error())
+
+
 def test_wrappers_refuse_cpu_tensors(pkg):
     x = torch.zeros(1, 16)
     with pytest.raises(pkg.hip.RavenHipError, match="GPU"):
