@@ -8,13 +8,14 @@
 //   mfma_kernel  (bf16, up to 32 rows of X per pass)   -- 16-row tiles of W are the A operand of
 //                v_mfma_f32_16x16x32_bf16, X is the B operand; the four or eight waves of a workgroup
 //                split K and reduce through LDS.
-//   rows_f32_kernel (float, 2 rows and more)          -- 16 rows of W against 16 to 64 rows of X on v_mfma_f64_16x16x4_f64.
+//   rows_f32_kernel (float, 5 rows and more, fewer where K is short) -- 16 rows of W against 16 to 64 rows of X on v_mfma_f64_16x16x4_f64.
 // Epilogues (all round the fp32 accumulator to T first, as an nn.Linear output would be stored):
 //   plain (+ residual add in T, + optional float store)   RMM:493, 509, 711, 534-535
 //   SwiGLU: T(T(silu(gate)) * up), gate row j, up row j+I  RMM:507-508
 // The adapter's concat (RMM:776) is folded in by giving X as two pointers that cover K0 and K1.
 
 #include <string>
+#include <type_traits>
 
 #include "raven_common.h"
 
@@ -107,10 +108,22 @@ __device__ __forceinline__ float swiglu(float gate_acc, float up_acc) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// gemv_kernel: 256 threads; dynamic LDS holds X as [MB][K] of T.
+// gemv_kernel: 256 threads; dynamic LDS holds X as [MB][K] of T.  WIDE (float): products and sums in 64 bits, as in rows_f32_kernel.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int MB, int EPI, bool NT>
+__device__ __forceinline__ double dot_chunk(const Chunk<float>& a, const Chunk<float>& b, double acc) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_fma((double)a.v[e], (double)b.v[e], acc);
+    return acc;
+}
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) v += __shfl_xor(v, d, 64);
+    return v;
+}
+
+template <typename T, int MB, int EPI, bool NT, bool WIDE = false>
 __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
+    typedef std::conditional_t<WIDE, double, float> Sum;
     constexpr int E = Chunk<T>::N;
     constexpr int U = 4;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -151,9 +164,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
         }
         const T* w0 = W + (int64_t)r0 * K;
         const T* w1 = W + (int64_t)r1 * K;
-        float acc0[MB], acc1[MB];
+        Sum acc0[MB], acc1[MB];
 #pragma unroll
-        for (int m = 0; m < MB; ++m) acc0[m] = acc1[m] = 0.f;
+        for (int m = 0; m < MB; ++m) acc0[m] = acc1[m] = 0;
 
         for (int c = lane; c < n_chunks; c += 64 * U) {
             Chunk<T> a0[U], a1[U];
@@ -189,10 +202,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
             for (int m = 0; m < MB; ++m) {
                 if (m < a.M) {
                     if (EPI == EPI_SWIGLU) {
-                        static_cast<T*>(a.y)[(int64_t)m * a.N + unit] = from_f32<T>(swiglu<T>(acc0[m], acc1[m]));
+                        static_cast<T*>(a.y)[(int64_t)m * a.N + unit] = from_f32<T>(swiglu<T>((float)acc0[m], (float)acc1[m]));
                     } else {
-                        store_out<T, EPI>(a, m, r0, acc0[m]);
-                        if (r1_ok) store_out<T, EPI>(a, m, r1, acc1[m]);
+                        store_out<T, EPI>(a, m, r0, (float)acc0[m]);
+                        if (r1_ok) store_out<T, EPI>(a, m, r1, (float)acc1[m]);
                     }
                 }
             }
@@ -472,20 +485,21 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// rows_f32_kernel: a workgroup owns 16 weight rows (SwiGLU: 16 gate rows and their up rows) and 16 MT token rows, its four waves split K
+// rows_f32_kernel: a workgroup owns 16 weight rows (SwiGLU: 16 gate rows and their up rows) and 16 MT token rows, its four or eight waves split K
 // and add up through LDS.  A lane loads 16 bytes of row l % 16 at columns 16 c + 4 (l / 16) ..+3 straight from memory -- of W and of X
 // alike, so that product j of a chunk, which takes element j of every lane's load, multiplies the same columns on both sides.  Products
 // and sums are in 64 bits (exact products; the fp32 instruction's one long chain of sums per element was 1.7 times further from the
 // exact result than gemv_kernel's 64 short ones, and no faster here).
-// What bounds it is latency (small models) or the 64-byte row pieces (large matrices: about 3 TB/s), not the matrix cores; it
-// reads W once per 64 rows where gemv_kernel takes passes of 8, each a launch: a product of 17 rows, 256 x 704 to 1408 x 256, three
-// launches of 4.5 to 8 us, now one of 5; 200 rows 25 launches.
+// What bounds it is a wave's walk over its share of K (small models) or the 64-byte row pieces (large matrices: about 3 TB/s), not the
+// matrix cores.  It reads W once per 64 rows where gemv_kernel takes passes of 8, each a launch: a product of 17 rows, 256 x 704 to 1408 x 256, three
+// launches of 4.5 to 8 us, now one of 5; 200 rows 25 launches.  With four waves the walk was longer than gemv_kernel's passes for few rows: us,
+// passes / four waves / eight, 2048 x 2048 at 8 rows 11.7 / 12.1 / 9.8, 512 x 4096 at 9 rows 21.4 / 19.7 / 15.8, SwiGLU of 512 x 2048 at 9, 17 and 33 rows 13.5 / 19.4 / 14.9, 23.0 / 24.6 / 21.9, 42.3 / 42.6 / 39.1.
 // ------------------------------------------------------------------------------------------------
-template <int EPI, int MT>
-__global__ __launch_bounds__(256) void rows_f32_kernel(GemmArgs a) {
+template <int EPI, int MT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(GemmArgs a) {
     typedef __attribute__((ext_vector_type(4))) double f64x4;
     constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, U = 4;
-    __shared__ __align__(16) f64x4 red[3][NT * MT][64];
+    __shared__ __align__(16) f64x4 red[WAVES - 1][NT * MT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
     const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT, K = a.K;
     const float* w[NT];
@@ -494,7 +508,7 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(GemmArgs a) {
     int64_t row[MT];
 #pragma unroll
     for (int j = 0; j < MT; ++j) row[j] = min(m0 + 16 * j + r, a.M - 1);
-    const int chunks = (K + 15) / 16, c0 = chunks * wave / 4, c1 = chunks * (wave + 1) / 4;
+    const int chunks = (K + 15) / 16, c0 = chunks * wave / WAVES, c1 = chunks * (wave + 1) / WAVES;
 
     f64x4 acc[NT][MT];
 #pragma unroll
@@ -555,7 +569,9 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(GemmArgs a) {
     for (int j = 0; j < MT; ++j) {
         const int m = m0 + 16 * j + r;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t][j] += (red[0][t * MT + j][lane] + red[1][t * MT + j][lane]) + red[2][t * MT + j][lane];
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int w = 0; w < WAVES - 1; ++w) acc[t][j] += red[w][t * MT + j][lane];
         if (m >= a.M) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {  // a lane holds weight rows 4 v + q of token row r
@@ -581,13 +597,13 @@ static int n_cus() {
     return cus;
 }
 
-template <typename T, int MB, int EPI, bool NT>
+template <typename T, int MB, int EPI, bool NT, bool WIDE = false>
 static int launch_gemv_nt(GemmArgs a, hipStream_t s) {
     const size_t lds = (size_t)MB * a.K * sizeof(T);
     RAVEN_REQUIRE(lds <= 160 * 1024, "gemm: %d rows x K=%d does not fit the 160 KB LDS", MB, a.K);
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemv_kernel<T, MB, EPI, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        hipError_t e = hipFuncSetAttribute((const void*)gemv_kernel<T, MB, EPI, NT, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) {
             raven_host::set_error("gemm: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
@@ -605,13 +621,30 @@ static int launch_gemv_nt(GemmArgs a, hipStream_t s) {
     a.units_per_wave = upw;
     a.interleave = g_tuning.gemv_interleave;
     const int wgs = (n_units + 4 * upw - 1) / (4 * upw);
-    gemv_kernel<T, MB, EPI, NT><<<dim3(wgs), dim3(256), lds, s>>>(a);
+    gemv_kernel<T, MB, EPI, NT, WIDE><<<dim3(wgs), dim3(256), lds, s>>>(a);
     return raven_host::check_launch("gemv");
 }
 
 template <typename T, int MB, int EPI>
 static int launch_gemv(GemmArgs a, hipStream_t s) {
     return g_tuning.gemv_nontemporal ? launch_gemv_nt<T, MB, EPI, true>(a, s) : launch_gemv_nt<T, MB, EPI, false>(a, s);
+}
+
+// Up to 8 float rows against a matrix that stays in the caches: once K is long, two rows of W per wave of the whole chip are read faster than 16 per
+// workgroup, also with 64-bit sums.  us, rows_f32_kernel / this: 2 rows, 512 x 256 3.7 / 3.9, 512 x 1024 5.5 / 4.5, 512 x 4096 15.4 / 9.8; 4 rows,
+// 512 x 1024 5.6 / 5.9, 512 x 4096 15.6 / 13.4; 8 rows, 512 x 4096 15.8 / 24.7.  SwiGLU: 2 rows, 512 x 128 4.0 / 3.8, 512 x 2048 15.2 / 6.8; 4 rows,
+// 512 x 256 4.8 / 4.8, 512 x 2048 15.2 / 8.8; 8 rows, 512 x 704 7.1 / 8.1, 512 x 2048 14.9 / 13.3.  (32-bit sums: 512 x 4096 at 2 rows 8.6.)
+// Of 8192 and more rows of W a wave takes several in turn: SwiGLU of 8192 x 512 at 2 and 4 rows 7.2 / 6.6 and 7.2 / 9.4, 16384 x 128 at 2 rows 5.5 / 9.0.
+static bool gemv_wide_pays(int M, int N, int K, bool swiglu) {
+    const int longest_rows = M <= 2 ? (swiglu ? 64 : 256) : M <= 4 ? (swiglu ? 256 : 1024) : swiglu ? 768 : 1 << 30;
+    return K > longest_rows && N * (swiglu ? 2 : 1) < 8192 && (size_t)(M <= 2 ? 2 : M <= 4 ? 4 : 8) * K * sizeof(float) <= 160 * 1024;
+}
+template <int EPI>
+static int dispatch_gemv_wide(GemmArgs a, hipStream_t s) {
+    a.ldy = a.N;
+    if (a.M <= 2) return launch_gemv_nt<float, 2, EPI, false, true>(a, s);
+    if (a.M <= 4) return launch_gemv_nt<float, 4, EPI, false, true>(a, s);
+    return launch_gemv_nt<float, 8, EPI, false, true>(a, s);
 }
 
 template <typename T, int EPI>
@@ -717,6 +750,13 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
 
 // Float rows: all of them in one launch (per 4 194 240, what a grid holds).  A few rows against a matrix that does not fit the caches stay with
 // the vector kernel, whose whole-row loads stream twice as fast (5.5 TB/s): up to 8 rows from 32 MB on.
+template <int EPI, int MT>
+static void launch_rows_f32_tiles(const GemmArgs& a, dim3 grid, hipStream_t s) {
+    // up to 256 columns a wave of four has one round of loads to wait for; where the grid is several rounds long, four waves leave more of it
+    // resident (8192 x 2048 at 16 rows 20.5 / 22.2 us; SwiGLU of 16384 x 704 at 200 rows 113 / 141)
+    if (a.K > 256 && grid.x * grid.y <= (unsigned)(MT > 1 ? 2 : 1) * n_cus()) rows_f32_kernel<EPI, MT, 8><<<grid, dim3(512), 0, s>>>(a);
+    else rows_f32_kernel<EPI, MT, 4><<<grid, dim3(256), 0, s>>>(a);
+}
 template <int EPI>
 static int launch_rows_f32(GemmArgs a, hipStream_t s) {
     a.ldy = a.N;
@@ -724,9 +764,9 @@ static int launch_rows_f32(GemmArgs a, hipStream_t s) {
     for (int m0 = 0; m0 < M; m0 += most) {
         a.M = M - m0 < most ? M - m0 : most;
         const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));
-        if (mt == 1) rows_f32_kernel<EPI, 1><<<grid, dim3(256), 0, s>>>(a);
-        else if (mt == 2) rows_f32_kernel<EPI, 2><<<grid, dim3(256), 0, s>>>(a);
-        else rows_f32_kernel<EPI, 4><<<grid, dim3(256), 0, s>>>(a);
+        if (mt == 1) launch_rows_f32_tiles<EPI, 1>(a, grid, s);
+        else if (mt == 2) launch_rows_f32_tiles<EPI, 2>(a, grid, s);
+        else launch_rows_f32_tiles<EPI, 4>(a, grid, s);
         if (const int rc = raven_host::check_launch("gemm (fp32 rows)")) return rc;
         a.x0 = static_cast<const float*>(a.x0) + (size_t)a.M * a.k0;
         if (a.x1) a.x1 = static_cast<const float*>(a.x1) + (size_t)a.M * a.k1;
@@ -746,7 +786,8 @@ static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
     const int M = a.M;
     const size_t out_es = a.out_f32 ? 4 : es;
     RAVEN_REQUIRE(dtype != RAVEN_F32 || (size_t)a.K * es <= 160 * 1024, "gemm: one row of K=%d elements does not fit the 160 KB LDS", a.K);
-    if (dtype == RAVEN_F32 && M >= 2 && (M > 8 || (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20))) return launch_rows_f32<EPI>(a, s);
+    if (dtype == RAVEN_F32 && M >= 2 && (M > 8 || (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20)))
+        return M <= 8 && gemv_wide_pays(M, a.N, a.K, EPI == EPI_SWIGLU) ? dispatch_gemv_wide<EPI>(a, s) : launch_rows_f32<EPI>(a, s);
     for (int m0 = 0; m0 < M;) {
         const int left = M - m0;
         int pass;

@@ -215,6 +215,13 @@ def test_fp32_rows_in_one_launch(pkg, M, N, K0, K1):
     assert torch.isfinite(got[1:]).all() and not torch.isfinite(got[0]).any()
 
 
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 8, 16, 17, 40])
+@pytest.mark.parametrize("N,K0,K1", [(14, 64, 0), (14, 256, 0), (14, 260, 0), (30, 268, 44), (15, 1028, 0), (16, 2052, 0), (4096, 320, 0), (4128, 320, 0)])
+def test_fp32_rows_by_every_kernel(pkg, M, N, K0, K1):
+    """Both sides of the borders in the length of K, in the rows, and in the number of workgroups (256 of 16 columns); shares of K that are of unequal length."""
+    test_fp32_rows_in_one_launch(pkg, M, N, K0, K1)
+
+
 def test_more_fp32_rows_than_one_grid_holds(pkg):
     M, N, K = 65535 * 64 + 17, 3, 4
     g = torch.Generator(device="cuda").manual_seed(1)
