@@ -58,10 +58,11 @@ __device__ __forceinline__ int ordered_key(float v) {
 // one wave: the `top` experts of largest logit (lower index first among equals); lane k holds the k-th one and its score.
 // Up to 64 experts (a lane each) an expert's place is the number of experts before it, counted in one sweep over the others' logits
 // through the lane-to-lane broadcast: 64 steps without a dependence, where `top` maxima over the wave, twelve exchanges each, took 3 us
-// of every launch that picks (moe_up_kernel at one row 14.7 -> 12 us, routing of 20 rows 11.8 -> 8).
+// of every launch that picks six (moe_up_kernel at one row 14.7 -> 12 us, routing of 20 rows 11.8 -> 8).  One or two are found sooner by
+// maxima (both launches of 8 rows of width 512, one of 8 experts of 512: 12.0 us, by counting 13.4).
 __device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
     const int lane = threadIdx.x & 63;
-    if (experts <= 64) {
+    if (experts <= 64 && top > 2) {
         const float v = lane < experts ? logits[lane] : 0.f;
         const int key = lane < experts ? ordered_key(v) : (int)0x80000000;
         int before = 0;

@@ -422,10 +422,10 @@ def test_mixture_prefers_the_lower_index_among_equals(pkg, dtype, M):
 
 @pytest.mark.parametrize("E", [7, 64, 65, 200])
 @pytest.mark.parametrize("M", [1, 3])
-def test_mixture_picks_by_value_then_index(pkg, E, M):
-    """Zeros of either sign are equal, ties go to the lower index, minus infinity is a score of nothing; 64 experts and fewer are picked by
-    counting, more by repeated maxima.  Expert e multiplies by a power of its own, so that a sum names its experts."""
-    D, ff, top = 8, 8, 3
+def test_mixture_picks_by_value_then_index(pkg, E, M, top=3):
+    """Zeros of either sign are equal, ties go to the lower index, minus infinity is a score of nothing; three and more of up to 64 experts are picked
+    by counting, others by repeated maxima.  Expert e multiplies by a power of its own, so that a sum names its experts."""
+    D, ff = 8, 8
     up = torch.zeros(E, 2 * ff, D, device="cuda")
     up[:, 0, 0] = up[:, ff, 0] = 1.0
     down = torch.zeros(E, D, ff, device="cuda")
@@ -441,9 +441,16 @@ def test_mixture_picks_by_value_then_index(pkg, E, M):
         values(logits[:, :E])
         x = torch.zeros(M, D, device="cuda")
         pkg.hip.moe(desc, h, logits, x)
+        chosen = chosen[:top]
         s = torch.sigmoid(logits[:, chosen])
         want = sum((torch.nn.functional.silu(s[:, i]) * s[:, i])[:, None] * down[e, :, 0] for i, e in enumerate(chosen))
         assert (x - want).abs().max() < 1e-5, (chosen, x, want)
+
+
+@pytest.mark.parametrize("E", [7, 64])
+@pytest.mark.parametrize("top", [1, 2])
+def test_mixture_picks_one_or_two(pkg, E, top):
+    test_mixture_picks_by_value_then_index(pkg, E, 3, top)
 
 
 # ---- whole models ------------------------------------------------------------------------------------
