@@ -23,7 +23,6 @@ int ring_grouped(const void* x, int x_rows, const void* w, void* y, int rows, in
 constexpr int kMaxExperts = 1024, kMaxTop = 32;
 constexpr int kBigTileRows = 110;  // rows per expert from which the grouped products take 256-row tiles
 constexpr int kPickRows = 32;  // tokens a workgroup of the two sorting kernels owns
-constexpr double kMoeBytesAgain = 25e6;
 constexpr int kRouteRows = 64, kRoutePairs = 2048;  // tokens and (token, expert) pairs up to which one workgroup picks and sorts
 
 struct MoeArgs {
@@ -396,14 +395,27 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
 
 // What runs the experts of M rows.  A chunk -- once its rows share weights (two per expert), or there are enough rows anyway -- keeps its slots in T
 // and runs the shared expert as a product of its own.  Fewer rows keep slots and sums in float, as the row kernels do, and take the
-// grouped product once reading each expert once saves more than its two further launches cost.  us at width 2048 (64 experts of 768
-// channels, 6 per row and a shared one), row kernels / grouped: 2 rows 31 / 34, 3: 45 / 42, 4: 59 / 55, 8: 105 / 78, 20: 246 / 124;
-// width 1024: 4 rows 22 / 26, 6: 29 / 27, 8: 38 / 31, 20: 80 / 40 -- the lines cross where rows would read 25 MB again.
+// grouped product once reading each expert once saves more than its two further launches cost.  us, row kernels / grouped, at width 2048 (64 experts of
+// 768 channels, 6 per row and a shared one): 2 rows 27 / 33, 3: 41 / 37, 4: 52 / 45, 8: 92 / 88, 20: 212 / 128; width 1024: 4 rows 33 / 36, 6: 45 / 39,
+// 8: 56 / 42; width 1024, one of 64 experts of 1024 and a shared one: 5 rows 16 / 28, 9: 22 / 30, 14: 32 / 34, 20: 47 / 42.
 enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
 constexpr size_t kMoeRowLds = 64 * 1024 - 1024;  // what a row may take of the row kernels' LDS; longer ones are refused for few rows
 static bool few_rows_fit(const raven_moe* m, int M, int ld) {
     return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs && ld * sizeof(bf16) <= kMoeRowLds &&
            (int64_t)2 * m->ff * ld < (1ll << 31);
+}
+// Estimates in us, within about 10 % of what 20 mixtures of 8 to 300 experts at widths 256 to 4096 took.  Row kernels: 5.4 TB/s whatever is read again, but
+// for the shared expert, which comes out of L2 from the second row on; past 64 experts the choice in every workgroup shows.  Grouped: four launches,
+// and per product a unit's walk over K (40 KB/us) or all weights once, at 5 TB/s, 3 where rows are so long that the last units' tail shows.
+// Nothing is grouped that would not read 25 MB again.
+static bool grouping_pays(const raven_moe* m, int M, int ld) {
+    const double pairs = (double)M * m->top, touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), shared = m->shared_up ? 1 : 0;
+    const double expert = 6e-6 * ld * m->ff;  // MB
+    if ((pairs - touched + shared * (M - 1)) * expert <= 25) return false;
+    const double rows = 8.2 + (pairs + shared) * expert / 5.4 + shared * (M - 1) * expert / 13 + (m->experts > 64 ? 0.55 * M : 0);
+    auto product = [&](int K, double bytes) { return std::max(6.4e-3 * K, bytes / (K > 3072 ? 3 : 5)); };
+    const double grouped = 14.4 + 0.25 * M + product(ld, (touched + shared) * expert * 2 / 3) + product(m->ff, (touched + shared) * expert / 3);
+    return grouped < 1.1 * rows;
 }
 // h: the rows, or null where only sizes are asked for.  The grouped kernels move whole 16-byte pieces into the LDS; operands that do not start
 // on one stay with the row kernels, which take any address.
@@ -412,8 +424,7 @@ static MoePath moe_path(const raven_moe* m, const void* h, int M, int ld, int dt
     const double pairs = (double)M * m->top;
     if (M > 8 && (pairs >= 2.0 * m->experts || M > 128)) return kMoeChunk;
     if (!few_rows_fit(m, M, ld)) return kMoeRows;
-    const double touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), again = pairs - touched + (m->shared_up ? M - 1 : 0);
-    return again * 6.0 * ld * m->ff > kMoeBytesAgain ? kMoeFew : kMoeRows;
+    return grouping_pays(m, M, ld) ? kMoeFew : kMoeRows;
 }
 
 struct MoeChunk {
