@@ -450,12 +450,16 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, MoePath pa
     } else {
         const bool fold = path == kMoeFew && m->shared_up;
         const size_t rows = pairs + (fold ? M : 0);
-        // The smallest tile that most experts' rows fit into; 256 (by the ring kernel, twice the speed per row) from an average of 110 on.
-        // us for all launches of a mixture, width 2048, tiles of 16 / 32 / 64 / 256 rows: 100 tokens 169 / 163 / 167 / 218, 500:
+        // The smallest tile that most experts' rows fit into; 256 (by the ring kernel, twice the speed per row) from an average of 110 on, if
+        // its units -- a tile by 128 channels of `up` or 256 of `down` -- fill the chip's 256 CUs over both products.  us for all launches of a mixture, width 2048, tiles of 16 / 32 / 64 / 256 rows: 100 tokens 169 / 163 / 167 / 218, 500:
         // 232 / 196 / 181 / 232, 1000: 344 / 255 / 218 / 249, 1500: 474 / 340 / 282 / 272, 4096: - / 695 / 518 / 394; width 1024, 500
         // tokens: 80 / 70 / 63 / 83, 1500: 144 / 109 / 94 / 96.  (128-row tiles of eight waves, as before: 230 at 500, 327 at 1500.)
+        // Few units, tiles of 64 / 256: 12 experts of 136 at width 256, 2 per row, 1000 tokens 29 / 47; 16 of 768 at 1024, 1000 tokens 73 / 93, 4000
+        // (400 units) 136 / 120; 8 of 2048 at 2048, 500 tokens (190) 105 / 116, 1000 (280) 134 / 122.
         const size_t mean = pairs / m->experts;
-        c.tile_rows = path == kMoeFew || mean <= 6 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows ? 64 : 256;
+        const size_t big_tiles = pairs / 256 + m->experts / 2;  // an expert's last tile is half full on average
+        const bool fills = big_tiles * ((m->ff + 127) / 128 + (ld + 255) / 256) > 256;
+        c.tile_rows = path == kMoeFew || mean <= 6 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows || !fills ? 64 : 256;
         auto tiles = [&](int height) { return (int)(pairs / height) + m->experts + (fold ? (M + height - 1) / height : 0); };
         c.n_tiles = tiles(c.tile_rows);
         const size_t table = (size_t)tiles(16) * 4;  // room for the lowest tiles whatever the height, so that more rows never need less

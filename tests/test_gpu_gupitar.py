@@ -342,6 +342,13 @@ def test_mixture_in_large_tiles(pkg, M, D, E, top, ff):
     assert (stream.cpu().double() - x - want).abs().max() < 2e-2 * max(1.0, want.abs().max().item())
 
 
+@pytest.mark.parametrize("M,D,E,top,ff,shared", [(2100, 1032, 8, 2, 1160, True), (2600, 264, 8, 3, 1928, False), (2100, 264, 8, 2, 136, False)])
+def test_mixture_tiles_of_256_rows_where_they_fill_the_chip(pkg, M, D, E, top, ff, shared):
+    """Averages past 110 rows per expert: units enough for 256-row tiles in the first two, 64-row tiles in the last; unequal shares of the rows."""
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, False)
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, True)
+
+
 @pytest.mark.parametrize("same", [False, True])
 @pytest.mark.parametrize("M,D,E,top,ff,shared", [(5, 1032, 64, 6, 392, True), (20, 1032, 64, 6, 392, True), (21, 1032, 64, 6, 392, False), (64, 520, 300, 4, 264, True),
                                                  (9, 2048, 16, 1, 776, True), (70, 520, 24, 6, 72, True), (200, 264, 12, 2, 136, False)])
