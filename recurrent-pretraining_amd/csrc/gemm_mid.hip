@@ -385,28 +385,30 @@ static constexpr int mid_stages(int nt, int mt) {
     return nt == 2 ? (mt == 1 ? 8 : mt == 2 ? 6 : 4) : nt == 4 ? (mt == 1 ? 6 : mt == 2 ? 5 : 3) : (mt == 1 ? 5 : mt == 2 ? 4 : 3);
 }
 
-// What a launch of a plan costs, in us, from what was measured on the products of the 3.5b shape and of models of width 1024 to 2304 at 33 to
-// 4096 rows (within 10 % there).  The memory pipe delivers first reads of the weights at 7 TB/s and what comes out of L2 -- the token
-// rows once per column of units, the weights again for further row tiles -- at 14; a K step takes the LDS the fragment reads of
-// eight waves (8 clocks per kilobyte) and the requests' writes, at 1.6 clocks per ns; outputs leave when a round ends.
+// What a launch of a plan costs, in us, fitted to 1847 products of 33 to 4100 rows, 64 to 36000 columns and K of 64 to 18000 (standard deviation 8 %).
+// The memory pipe delivers first reads of the weights at 9 TB/s and what comes out of L2 -- the token rows once per column of units, the
+// weights again for further row tiles -- at 18; a K step takes the LDS the fragment reads of eight waves (8 clocks per kilobyte) and the
+// requests' writes, at 2 clocks per ns; the largest units, with three or four stages in flight, fall short of that.  Every round of units fills its
+// ring and drains its outputs anew: 3514 x 592 x 64 in three rounds takes 12.4 us, where a round's own work is 0.3 (128 x 128 tiles, one round: 5.2).
 static double mid_estimate(const MidPlan& p, int M, int N, int K, int side, int cus) {
     const int64_t mn = (int64_t)p.tiles_n * p.tiles_m;
     const int nk = (K + 63) / 64, tiles_w = (p.cols * side + 15) / 16, wave_t = tiles_w < p.nt ? tiles_w : p.nt;
     const int rounds = (int)((mn * p.ks + cus - 1) / cus);
     const double weights = 2.0 * N * side * K, again = weights * (p.tiles_m - 1) + 2.0 * K * 64 * p.mt * mn;
-    const double mem = weights / 7e6 + again / 14e6;
-    const double lds = rounds * ((nk + p.ks - 1) / p.ks) * (128.0 * (wave_t + p.mt) + 16 * tiles_w + 64 * p.mt) / 1600.0;
-    double us = (mem > lds ? mem : lds) + 3.0 + 4.0 * M * N / 6e6 / rounds;
-    if (p.ks > 1) us += 5.0 + 8.0 * p.ks * M * N * side / 8e6;
+    const double mem = weights / 9e6 + again / 18e6;
+    const double lds = rounds * ((nk + p.ks - 1) / p.ks) * (128.0 * (wave_t + p.mt) + 16 * tiles_w + 64 * p.mt) / 2050.0;
+    double us = (mem > lds ? mem : lds) * (1.0 + (p.mt == 4 && p.ks == 1 ? 0.23 : 0) + (p.nt == 6 ? 0.11 : 0)) + 3.8 * rounds + 6.2 * M * N / 6e6 / rounds;
+    if (p.ks > 1) us += 1.2 + 15.0 * p.ks * M * N * side / 8e6;
     return us;
 }
 
-static MidPlan find_plan(int M, int N, int K, int swiglu) {
+static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room) {
     MidPlan best{};
     const int cus = mid_cus(), nk = (K + 63) / 64, side = swiglu ? 2 : 1;
-    // the 128 x 128 tiles of gemm_tiled.hip: a K step takes 0.68 us on a CU with one of them and 0.48 more with each further one
+    // the 128 x 128 tiles of gemm_tiled.hip: a K step takes 0.53 us on a CU with one of them and 0.34 more with each further one, and up to
+    // 0.15 more per round the fuller the chip is
     const int64_t small = (int64_t)((M + 127) / 128) * ((N * side + 127) / 128);
-    const double tiled = nk * (0.2 + 0.48 * (double)((small + cus - 1) / cus)) + 3.0 + 4.0 * M * N / 6e6;
+    const double tiled = nk * (0.19 + 0.34 * (double)((small + cus - 1) / cus) + 0.154 * (double)small / cus) + 3.8 + 2.6 * M * N / 6e6;
     const bool forced = g_mid_nt || g_mid_mt || g_mid_ks;
     for (int nt = 2; nt <= 6; nt += 2)
         for (int mt = 1; mt <= 4; mt *= 2) {
@@ -434,27 +436,30 @@ static MidPlan find_plan(int M, int N, int K, int swiglu) {
                 if (p.ks > 1 && (int64_t)p.tiles_n * p.tiles_m * p.ks > cus + cus / 32 && !g_mid_ks) break;
                 if (p.ks > 1 && nk / p.ks < (g_mid_ks ? 1 : 6)) break;
                 if (g_mid_ks && p.ks != g_mid_ks && p.ks < nk) continue;
+                if (mid_workspace_bytes(M, N, p, swiglu) > room) break;
                 p.us = (float)mid_estimate(p, M, N, K, side, cus);
                 if ((forced || p.us < tiled) && (best.nt == 0 || p.us < best.us)) best = p;
             }
         }
+    if (forced) best.us = 0.f;  // whatever else could run
     return best;
 }
 
-MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu) {
+MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room) {
     if (!g_mid) return MidPlan{};
     // a product is planned several times on its way (does it fit, which row pitch, which launch): the last few shapes of this thread
     struct Known {
         int M, N, K, swiglu, knobs;
+        size_t room;
         MidPlan plan;
     };
     static thread_local Known known[16];
     static thread_local int next = 0;
     const int K = K0 + K1, knobs = 1 + g_mid_nt + 10 * g_mid_mt + 100 * g_mid_ks;
     for (const Known& k : known)
-        if (k.M == M && k.N == N && k.K == K && k.swiglu == swiglu && k.knobs == knobs) return k.plan;
+        if (k.M == M && k.N == N && k.K == K && k.swiglu == swiglu && k.knobs == knobs && k.room == room) return k.plan;
     Known& k = known[next++ & 15];
-    k = Known{M, N, K, swiglu, knobs, find_plan(M, N, K, swiglu)};
+    k = Known{M, N, K, swiglu, knobs, room, find_plan(M, N, K, swiglu, room)};
     return k.plan;
 }
 

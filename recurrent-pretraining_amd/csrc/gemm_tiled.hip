@@ -826,22 +826,29 @@ static int launch_tiled(TiledArgs a, hipStream_t s) {
     return raven_host::check_launch("gemm (tiled MFMA)");
 }
 
-// The plan of gemm_mid.hip for a product, or one without tiles where the kernels of this file are the better choice: once 256 x 256 tiles
-// fill the chip (256 of them), and where the K slices of the plan would not fit the caller's workspace.
+// The best plan of gemm_mid.hip whose K slices fit the caller's workspace, or one without tiles where the kernels of this file are the better
+// choice: once 256 x 256 tiles fill the chip (256 of them), and where 128 x 128 tiles are estimated faster.
 static MidPlan mid_choice(int M, int N, int K0, int K1, int swiglu, size_t workspace_bytes) {
     MidPlan none{};
     const int bn_out = swiglu ? 128 : 256;
     if (g_tiled_variant != 0 || M < g_tiled_min_rows || (int64_t)((M + 255) / 256) * ((N + bn_out - 1) / bn_out) >= 256) return none;
-    const MidPlan p = mid_plan(M, N, K0, K1, swiglu);
-    return mid_workspace_bytes(M, N, p, swiglu) <= workspace_bytes ? p : none;
+    return mid_plan(M, N, K0, K1, swiglu, workspace_bytes);
+}
+
+// What passes of 32 rows by the skinny kernels take, in us: the walk of a workgroup's waves over K, or the weights at 5 TB/s (32 rows: 4096 columns
+// of 1024, 2048, 4096, 8192 4.9, 6.5, 10, 17; 8192 of 2048 and 4096 10 and 16.5; 15840 of 5280 34)
+static double passes_us(int M, int N, int K) {
+    const double walk = 2.8 + 0.0017 * K, stream = 2.5 + 2.0 * N * K / 5e6;
+    const double last = M % 32 ? 0.6 + 0.0125 * (M % 32) : 0;  // (a pass of few rows is shorter)
+    return (M / 32 + last) * (walk > stream ? walk : stream);
 }
 
 // Host entry for the other translation units: true when the shape is one the kernels over many rows take and they are the better
-// choice for.  Few token rows against a matrix with few rows give too few tiles to fill the chip: gemm_mid.hip then cuts K
-// into slices, which needs a workspace (workspace_bytes of raven_linear_workspace_bytes); without one those products go to the skinny
-// kernels, 32 rows per pass over the weights -- up to two passes at K = 5280, four at 10560 and five (160 rows) at 17920, where
-// the passes' split over K still beats one round of 128 x 128 tiles walking the whole of K (measured at 33 .. 160 rows: Wqkv
-// 98 / 130 us in three / four passes against 75 / 81 tiled, mlp.proj 172 against 199).
+// choice for.  Few token rows against a matrix with few rows give too few tiles to fill the chip: gemm_mid.hip then cuts it into units, and K
+// into slices where the caller's workspace holds them; where that is not estimated faster, those products go to the skinny kernels, 32 rows
+// per pass over the weights -- up to two passes at K = 5280, four at 10560 and five (160 rows) at 17920, where the passes still beat one round
+// of 128 x 128 tiles walking the whole of K (measured at 33 .. 160 rows: Wqkv 98 / 130 us in three / four passes against 75 / 81 tiled,
+// mlp.proj 172 against 199).
 // aligned: whether all operands start on 16 bytes, which the kernels over many rows need; the passes take any address.
 bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned) {
     const bool ok = dtype == RAVEN_BF16 && M >= 1 && N % 8 == 0 && K0 % 8 == 0 && K0 > 0 && (K1 == 0 || K1 == K0) &&
@@ -849,7 +856,10 @@ bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t
     if (!ok) return false;
     const int64_t small_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int passes = (K0 + K1 + 3499) / 3500;
-    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) return aligned && mid_choice(M, N, K0, K1, swiglu, workspace_bytes).nt != 0;
+    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) {
+        const MidPlan mid = aligned ? mid_choice(M, N, K0, K1, swiglu, workspace_bytes) : MidPlan{};
+        return mid.nt != 0 && mid.us < passes_us(M, swiglu ? 2 * N : N, K0 + K1);
+    }
     return true;
 }
 

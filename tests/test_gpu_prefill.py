@@ -175,6 +175,22 @@ def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, 
         assert torch.equal(pkg.hip.linear(x, w, workspace=ws), pkg.hip.linear(x, w, workspace=ws))
 
 
+@pytest.mark.parametrize("M,N,K", [(34, 96, 5184), (100, 1280, 1280), (150, 128, 1360), (260, 248, 1168), (400, 1024, 4096)])
+def test_products_with_any_room_for_slices(pkg, M, N, K):
+    """Shapes that are cut into K slices where the workspace holds them: with none, with room for two slices, with all of it; plain, + residual, float, SwiGLU,
+    two operands."""
+    dt = torch.bfloat16
+    x, w, res = _gpu_randn((M, K), 720), _gpu_randn((N, K), 721, 0.05), _gpu_randn((M, N), 722)
+    z = x.float() @ w.float().T
+    u = z.to(dt).float()
+    for ws in (None, torch.empty(2 * M * N * 4, dtype=torch.uint8, device="cuda"), pkg.hip.linear_workspace(M, N, "cuda")):
+        check(pkg.hip.linear(x, w, workspace=ws), u.to(dt), dt, "plain")
+        check(pkg.hip.linear(x, w, out_f32=True, workspace=ws), u, dt, "float")
+        check(pkg.hip.linear(x, w, residual=res, workspace=ws), (u + res.float()).to(dt), dt, "+ residual", mag=z, ulps=ULPS_RESIDUAL)
+        check(pkg.hip.linear(x, w, swiglu=True, workspace=ws), (F.silu(u[:, :N // 2]).to(dt).float() * u[:, N // 2:]).to(dt), dt, "SwiGLU", ulps=ULPS_SWIGLU)
+        check(pkg.hip.linear(x[:, :K // 2].contiguous(), w, x1=x[:, K // 2:].contiguous(), workspace=ws), u.to(dt), dt, "two operands")
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 256, 4096), (100, 1024, 11008)])
 def test_a_residual_off_sixteen_bytes(pkg, M, N, K):
     """The middle kernel loads whole 16-byte pieces; rows that the kernels of up to 32 rows can take in passes go there instead."""
