@@ -47,9 +47,11 @@ __global__ __launch_bounds__(256) void embed_kernel(const T* __restrict__ wte, c
 }
 
 // First index of the row maximum; one 1024-thread workgroup per row.  Its life is a chain of memory latencies, so U values per thread are
-// requested at once: 32768 values 4.8 us against 8.2 with one at a time, 24 rows of 65536 8.5 against 23.8.
+// requested at once: 32768 values 4.8 us against 8.2 with one at a time, 24 rows of 65536 8.5 against 23.8.  Values that a short row does not have
+// cost their requests all the same; us with 1 / 2 / 4 / 8 / 16: 2000 rows of 1024 10.2 / 10.5 / 10.8 / 11.5 / 19.8, of 4096 12.3 / 11.3 / 10.8 / 11.8 / 20.0, one of 4096
+// 3.15 / 2.91 / 2.89 / 3.14 / 3.69, one of 16384 5.0 / 4.0 / 3.7 / 3.7 / 3.7.  Many long rows keep the memory busy with 8: 600 of 65536 46.9 / 39.2 / 29.9 / 26.5 / 28.1.
+template <int U>
 __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int64_t vocab) {
-    constexpr int U = 16;
     __shared__ float sv[16];
     __shared__ long long si[16];
     const float* row = logits + (int64_t)blockIdx.x * vocab;
@@ -149,7 +151,12 @@ extern "C" int raven_argmax(const float* logits, int64_t* out, int32_t M, int64_
     RAVEN_REQUIRE(logits && out, "argmax: null pointer");
     RAVEN_REQUIRE(M >= 0 && vocab > 0, "argmax: bad shape M=%d vocab=%lld", M, (long long)vocab);
     if (M == 0) return 0;
-    argmax_kernel<<<dim3(M), dim3(1024), 0, static_cast<hipStream_t>(stream)>>>(logits, out, vocab);
+    const dim3 grid(M), block(1024);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (vocab <= 2048) argmax_kernel<2><<<grid, block, 0, s>>>(logits, out, vocab);
+    else if (vocab <= 16384) argmax_kernel<4><<<grid, block, 0, s>>>(logits, out, vocab);
+    else if (M > 256) argmax_kernel<8><<<grid, block, 0, s>>>(logits, out, vocab);
+    else argmax_kernel<16><<<grid, block, 0, s>>>(logits, out, vocab);
     return raven_host::check_launch("argmax");
 }
 

@@ -383,10 +383,10 @@ def test_one_row_of_every_length_of_share(pkg, dt, chunks):
         check(got[None], lin(h[None], w).to(dt), dt, "float norm")
 
 
-@pytest.mark.parametrize("vocab", [1, 63, 1024, 16383, 16384, 16385, 50001])
-def test_argmax_of_every_remainder(pkg, vocab):
-    """Rows that end inside a thread's 16 values, inside a stripe and on its border; the first of equal maxima, also the last value's."""
-    x = rnd((3, vocab), torch.float32, 260)
+@pytest.mark.parametrize("rows,vocab", [(3, 1), (3, 63), (3, 1024), (3, 2047), (3, 2048), (3, 2049), (3, 4097), (3, 16383), (3, 16384), (3, 16385), (3, 50001), (300, 1500), (300, 16385), (257, 50001)])
+def test_argmax_of_every_remainder(pkg, rows, vocab):
+    """Rows that end inside a thread's 2 to 16 values, inside a stripe and on its border; the first of equal maxima, also the last value's."""
+    x = rnd((rows, vocab), torch.float32, 260)
     x[1, vocab // 2] = x[1, -1] = 50.0
     x[2, -1] = 60.0
     assert torch.equal(pkg.hip.argmax(x.cuda()).cpu(), x.argmax(-1))
