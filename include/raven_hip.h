@@ -104,7 +104,7 @@ const char* raven_last_error(void);
  * shape and slice count, 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
- * gemm_one_round (1 = a 2..32-row product of up to about 16384 output columns runs as at most one workgroup of eight waves per compute unit, 0 = the
+ * gemm_one_round (1 = a 2..32-row product of up to about 16384 output columns runs as at most one workgroup of eight waves per compute unit where that is faster, 2 = wherever it is narrow enough, 0 = the
  * four-wave kernels),
  * gemm_ragged (1 = a 5..32-row product whose output columns divide into about two workgroups per compute unit runs as one
  * round of workgroups with a partly empty last tile, 0 = whole tiles only), norm_early (1 / 0 = the RMSNorm kernel requests

@@ -58,7 +58,7 @@ struct Tuning {
     int gemv_wgs_per_cu = 4;
     int gemm_four_tiles = 1;
     int gemm_mfma_min_rows = 2;  // fewer rows go to the vector kernels (one row: the K-split GEMV)
-    int gemm_one_round = 1;      // 0 = never one workgroup of eight waves per CU
+    int gemm_one_round = 1;      // one workgroup of eight waves per CU: 0 never, 1 by rule, 2 wherever the matrix is narrow enough
     int gemm_ragged = 1;         // 0 never, 1 = one workgroup per resident slot with partly empty last tiles where the shape divides so
 };
 static Tuning g_tuning;
@@ -655,39 +655,61 @@ static int dispatch_gemv(GemmArgs a, hipStream_t s) {
     return launch_gemv<T, 8, EPI>(a, s);
 }
 
-// A matrix of up to 1024 tiles of 16 rows (from 17 token rows on 768; SwiGLU: 256 pairs) in one round of the chip: the fewest tiles per workgroup that give every CU at
-// most one workgroup, of eight waves.  Four waves a tile leave a CU with one or two short workgroups, or a second round of them; with eight,
-// and the partial sums added through LDS, the K slices of gemm_splitk.hip and their second launch are not needed either, up to the
-// length of K where the workgroups become too long (splits_k there).  us per launch before / after: 2048 x 2048 at 8 rows 6.1 / 5.5, at 20 rows
-// 9.3 / 7.0; 8192 x 2048 9.9 / 9.5 and 15.3 / 10.9; 10304 x 2048 12.0 / 11.2 and 15.4 / 12.6; 15840 x 5280 at 16 rows 32.6 / 30.1.
-// More loads in flight than two sets of 64 columns per wave gain nothing: a CU's own rate of loads is the bound.
+// Whether a matrix of up to 1024 tiles of 16 rows (from 17 token rows on 768; SwiGLU: 256 pairs) goes in one round of the chip: the fewest tiles per
+// workgroup that give every CU at most one workgroup, of eight waves.  Four waves a tile leave a CU with one or two short workgroups, or a second
+// round of them; with eight, and the partial sums added through LDS, the K slices of gemm_splitk.hip and their second launch are not needed
+// either, up to the length of K where the workgroups become too long (splits_k there).  But eight waves of short rows do little else than
+// start and add up, and with few rows of X the shorter workgroups of four waves lose nothing.  Time of one round over that of four waves, from 2 x 3600 products:
+//   one tile    K of 256 1.03 - 1.07, 512 1.02 - 1.04, 640 0.92, 2048 0.85 - 0.98, 8192 0.68 - 0.97 (SwiGLU 512 1.03, 640 0.94, 4096 0.88 - 1.02)
+//   two tiles   up to 8 rows 0.95 - 1.18; 16 rows: K of 1536 1.05 - 1.08, 2048 0.92, 2560 1.02, 4096 0.95 - 1.03, 5120 0.92; 24 rows: 1536 1.05, 2048 0.90, 5120 0.87; with 257 tiles
+//               for 256 CUs, half of them without a workgroup, 1.0 - 1.27 up to 16 rows; from 509 tiles on (four tiles per four-wave workgroup past
+//               16 rows) 0.7 - 0.88 at 24 rows, whatever K
+//   three tiles 2 rows: 512 1.1 - 1.27, 1536 1.15, 2048 0.91 - 0.99, 2560 1.05 - 1.11, 3072 0.98 - 1.01, 5120 0.93 - 0.98, 8192 0.8; 24 rows 0.83 - 1.0
+//   four tiles  2 rows 1.0 - 1.17, but 0.91 at 4096; 16 rows: 512 1.09, 2048 1.05, 2560 1.0, 4096 0.9, 5120 0.97, 6144 1.1
+// Sets of two steps ahead (two and three tiles) throw away half of the last one when a wave's number of steps is odd, which a fifth step shows most;
+// rows of a power of two bytes from 8 KB on put all rows of a tile on the same channels, which more and shorter workgroups than here suffer from
+// with four tiles and less with two; tiles whose
+// rows alternate between whole and half lines (no pairs of tiles to sort them into) take 1.1 - 1.27 with two tiles and more.
+template <bool SWIGLU>
+static bool one_round_pays(const GemmArgs& a, int tiles) {
+    const int n = a.N / 16, cus = n_cus(), steps = (a.K / 64 + 7) / 8;  // steps: of 64 columns, per wave
+    if (tiles == 1) return a.K > 512;
+    if (SWIGLU) return false;  // two gate tiles and their up tiles: no faster than the four-wave kernels (14.4 / 14.1 at 12288 x 2048)
+    const int rs = a.row_stride;
+    if (a.M > 16 && (n + 4 * rs - 1) / (4 * rs) * rs >= cus / 2) return true;  // (else dispatch_mfma takes four tiles per four-wave workgroup)
+    if (!a.line_aligned || steps < 4) return false;
+    const int pitch = 2 * a.K;
+    const bool one_channel = pitch >= 8192 && (pitch & (pitch - 1)) == 0;
+    if (tiles == 2) {
+        if (a.M > 16) return n >= cus + cus / 8 || steps >= 6;
+        if (n < cus + cus / 8 || steps == 5 || one_channel) return false;
+        return a.M >= 16 || (n <= cus + cus / 2 && (a.M >= 12 || (rs == 2 && steps >= 6)));
+    }
+    if (tiles == 3) return a.M > 16 || steps == 4 || steps >= (a.M < 8 ? 8 : 6);
+    return one_channel || (a.M > 12 && steps >= 6 && pitch % 4096 != 0);
+}
+
+// us per launch before / after: 2048 x 2048 at 8 rows 6.1 / 5.5, at 20 rows 9.3 / 7.0; 8192 x 2048 at 20 rows 15.3 / 10.9; 10304 x 2048 12.0 / 11.2 and
+// 15.4 / 12.6; 15840 x 5280 at 16 rows 32.6 / 30.1.  More loads in flight than two sets of 64 columns per wave gain nothing: a CU's own rate of loads is
+// the bound.
 template <int EPI, int MT>
 static bool launch_one_round(const GemmArgs& a, hipStream_t s) {
     constexpr int side = EPI == EPI_SWIGLU ? 2 : 1;
     const int rs = a.row_stride, n_tiles16 = a.N / 16;
     auto groups = [&](int ng) { return (n_tiles16 + ng * rs - 1) / (ng * rs) * rs; };
     if (!g_tuning.gemm_one_round || g_tuning.gemm_four_tiles == 2) return false;
-    if (groups(1) <= n_cus()) {
+    int tiles = 1;
+    while (tiles < 5 && groups(tiles) > n_cus()) ++tiles;
+    // two token tiles against four weight tiles do not fit the registers
+    if (tiles > (EPI == EPI_SWIGLU ? 1 : MT == 1 ? 4 : 3) || (g_tuning.gemm_one_round == 1 && !one_round_pays<EPI == EPI_SWIGLU>(a, tiles))) return false;
+    if (tiles == 1) {
         mfma_kernel<MT, side, EPI, 128, false, 8><<<dim3(groups(1)), dim3(512), 0, s>>>(a);
-        return true;
+    } else if constexpr (EPI != EPI_SWIGLU) {
+        if (tiles == 2) mfma_kernel<MT, 2, EPI, 64, false, 8, 2><<<dim3(groups(2)), dim3(512), 0, s>>>(a);
+        else if (tiles == 3) mfma_kernel<MT, 3, EPI, 64, false, 8, 2><<<dim3(groups(3)), dim3(512), 0, s>>>(a);
+        else if constexpr (MT == 1) mfma_kernel<1, 4, EPI, 64, false, 8><<<dim3(groups(4)), dim3(512), 0, s>>>(a);
     }
-    if constexpr (EPI != EPI_SWIGLU) {  // two gate tiles and their up tiles: no faster than the four-wave kernels (14.4 / 14.1 at 12288 x 2048)
-        if (groups(2) <= n_cus()) {
-            mfma_kernel<MT, 2, EPI, 64, false, 8, 2><<<dim3(groups(2)), dim3(512), 0, s>>>(a);
-            return true;
-        }
-        if (groups(3) <= n_cus()) {
-            mfma_kernel<MT, 3, EPI, 64, false, 8, 2><<<dim3(groups(3)), dim3(512), 0, s>>>(a);
-            return true;
-        }
-        if constexpr (MT == 1) {  // two token tiles against four weight tiles do not fit the registers
-            if (groups(4) <= n_cus()) {
-                mfma_kernel<1, 4, EPI, 64, false, 8><<<dim3(groups(4)), dim3(512), 0, s>>>(a);
-                return true;
-            }
-        }
-    }
-    return false;
+    return true;
 }
 
 template <int EPI>

@@ -294,10 +294,11 @@ int g_linear_ks = 0;  // raven_set_tuning("linear_ks"): K slices per weight tile
 // is too narrow for one workgroup per CU to read it quickly and a workgroup's own range, all of K against all token rows, is long.  us,
 // slices / one round of the chip: 2048 x 2048 at 20 rows 9.3 / 7.0, 2048 x 4096 at 20 and 32 rows 11.6 / 9.5 and 12.4 / 10.7, 2048 x 8192 at
 // 16, 20, 32 rows 13.7 / 12.9, 14.5 / 15.0, 14.9 / 17.3; 5280 x 5280 at 16, 20, 32 rows 18.9 / 16.0, 18.4 / 17.9, 19.5 / 20.3; 5280 x 17920 at 16
-// rows 36.4 / 45.8.
-static bool splits_k(int n_tiles16, int M, int K) {
+// rows 36.4 / 45.8.  SwiGLU (two tiles a workgroup): 1024 x 8192 at 8 and 16 rows 13.5 / 14.3 and 14.3 / 15.7, 2048 x 8192 18.0 / 16.8 and 18.9 / 17.9.
+static bool splits_k(int n_tiles16, int M, int K, bool swiglu) {
     if (n_tiles16 >= 2 * ns_cus()) return false;
     if (M > 16) return K > 4096;
+    if (swiglu && M >= 8 && n_tiles16 <= ns_cus() / 2) return K >= 8192;
     return n_tiles16 <= ns_cus() ? K > 8192 : K >= 8192;
 }
 
@@ -424,7 +425,7 @@ extern "C" int raven_linear(const void* x0, const void* x1, const void* w, const
         return tiled_gemm(x0, 0, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, workspace, room, static_cast<hipStream_t>(stream), nullptr);
     bool fits = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                 ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1;
-    if (fits && g_linear_ks == 0) fits = splits_k((swiglu ? 2 * N : N) / 16, M, K0 + K1);
+    if (fits && g_linear_ks == 0) fits = splits_k((swiglu ? 2 * N : N) / 16, M, K0 + K1, swiglu != 0);
     if (!fits) {  // one to four rows, fp32, odd shapes, large N: the kernels without a workspace
         if (swiglu) return raven_gemm_swiglu(x0, w, y, M, N, K0, dtype, stream);
         if (K1) return raven_adapter_gemm_concat(x0, x1, w, y, M, N, K0, K1, dtype, stream);
@@ -479,7 +480,7 @@ extern "C" int raven_linear_epilogue(const void* x0, const void* x1, const void*
     // the same choice between the kernels with and without a K split as raven_linear
     const bool split = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                        ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1 &&
-                       (g_linear_ks != 0 || splits_k(N / 16, M, K0 + K1));
+                       (g_linear_ks != 0 || splits_k(N / 16, M, K0 + K1, false));
     if (!split) return gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, dtype, s);
     const size_t out_es = epi->out_f32 ? 4 : 2;
     for (int m0 = 0; m0 < M; m0 += 32) {

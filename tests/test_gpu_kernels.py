@@ -298,15 +298,15 @@ def test_linear_small_and_odd_shapes(pkg, tuned):
 
 
 @pytest.mark.parametrize("M", [6, 20])
-@pytest.mark.parametrize("four", [1, 2])
-def test_mfma_gemm_row_alignment_cases(pkg, tuned, M, four):
+@pytest.mark.parametrize("four,one_round", [(1, 2), (1, 0), (2, 1)])
+def test_mfma_gemm_row_alignment_cases(pkg, tuned, M, four, one_round):
     """Row pitches that are odd multiples of 64 bytes (tiles of one row parity, macro-steps shifted to the line
     boundary), with and without whole tile pairs, a second operand that starts mid-line, and a weight matrix
-    whose base address is not line-aligned; both MFMA kernels (with and without a workspace)."""
+    whose base address is not line-aligned; with a workspace the split-K kernel, without one workgroups of eight waves
+    (one_round) or of four, the latter with two tiles or four."""
     dt = torch.bfloat16
     ws = pkg.hip.linear_workspace(M, 4096, "cuda")
-    # four = 2: the four-tile, 64-wide-step variant wherever there is no workspace; with a workspace: the split-K kernel
-    tuned(gemm_four_tiles=four, linear_ks=2)
+    tuned(gemm_four_tiles=four, gemm_one_round=one_round, linear_ks=2)
     for N, K in ((32, 96), (64, 288), (64, 2336), (96, 416), (48, 416), (160, 1184), (64, 256)):
         x, w = rnd((M, K), dt, 180 + N), rnd((N, K), dt, 181 + K, 0.05)
         want = lin(x, w).to(dt)
@@ -330,11 +330,13 @@ def test_mfma_gemm_row_alignment_cases(pkg, tuned, M, four):
 
 
 @pytest.mark.parametrize("M", [2, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [(16, 32), (80, 96), (4096, 2048), (4112, 1184), (8192, 288), (8256, 160), (12304, 256), (16352, 416), (16400, 64)])
-def test_a_few_rows_in_one_round_of_the_chip(pkg, M, N, K):
+@pytest.mark.parametrize("N,K", [(16, 32), (80, 96), (4096, 2048), (4112, 1184), (8192, 288), (8256, 160), (12304, 256), (16352, 416), (16400, 64), (16400, 544), (16416, 544), (16416, 320)])
+def test_a_few_rows_in_one_round_of_the_chip(pkg, tuned, M, N, K):
     """One to four tiles of 16 columns per workgroup, on both sides of each border at 256 compute units: K shares of the eight waves that are empty,
-    one step or several rounds of two, tiles of one row parity and whole ones, a last workgroup that is partly empty; every epilogue."""
+    one step or several rounds of two, tiles of one row parity and whole ones, a last workgroup that is partly empty; every epilogue.  Past 1024 tiles
+    workgroups of four waves: a wave's share of several 128-wide steps, the 32 columns left over, shifted starts."""
     dt = torch.bfloat16
+    tuned(gemm_one_round=2)  # also where four waves are faster
     x, w, res = rnd((M, K), dt, 240).cuda(), rnd((N, K), dt, 241, 0.05).cuda(), rnd((M, N), dt, 242).cuda()
     ws = pkg.hip.linear_workspace(M, N, "cuda")
     z = x.float() @ w.float().T
