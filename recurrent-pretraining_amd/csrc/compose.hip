@@ -21,6 +21,7 @@ extern "C" int raven_gemv_fused(const void* x0, const void* x1, const void* norm
 
 namespace raven {
 
+bool gemv1_fits(int K, int dtype);
 int gemv1_column_block(const void* x, const void* norm_a, const void* w_block, int ldw, const float* acc_in, void* y, int raw_out,
                        int N, int K, float eps, int dtype, hipStream_t s);
 
@@ -126,9 +127,7 @@ static int check_block_weights(const char* who, const raven_block_weights* w) {
 
 // the one-row kernel keeps a quarter of K per wave in registers: 9 chunks of 16 bytes per lane at most
 static bool one_row_fits(const raven_dims* d) {
-    const int elts = 16 / (int)raven_host::elt_size(d->dtype);
-    const int longest = d->intermediate > 2 * d->n_embd ? d->intermediate : 2 * d->n_embd;
-    return ((longest / elts + 3) / 4 + 1 + 63) / 64 <= 9;
+    return gemv1_fits(d->intermediate > 2 * d->n_embd ? d->intermediate : 2 * d->n_embd, d->dtype);
 }
 
 // The padded row length that the decode steps of a call use for norm_1's / norm_3's output and for Wqkv / mlp.fc (see

@@ -30,6 +30,7 @@ bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 
+bool gemv1_fits(int K, int dtype);
 int gemv1_free(const void* x0, const void* x1, const void* w, void* y, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
                hipStream_t s);
 
@@ -813,8 +814,7 @@ static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
     for (int m0 = 0; m0 < M;) {
         const int left = M - m0;
         int pass;
-        const int elts = 16 / (int)es;
-        if (left == 1 && ((a.K / elts + 3) / 4 + 1 + 63) / 64 <= 9) {  // a single row: the K-split one-row kernel
+        if (left == 1 && gemv1_fits(a.K, dtype)) {  // a single row: the K-split one-row kernel
             const char* x0 = static_cast<const char*>(a.x0) + (size_t)m0 * a.k0 * es;
             const char* x1 = a.x1 ? static_cast<const char*>(a.x1) + (size_t)m0 * a.k1 * es : nullptr;
             const char* res = a.residual ? static_cast<const char*>(a.residual) + (size_t)m0 * a.N * es : nullptr;

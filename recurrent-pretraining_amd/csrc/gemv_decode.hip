@@ -283,8 +283,13 @@ static int gemv1_cus() {
     return cus;
 }
 
-// The longest rows the one-row kernel takes (gemm_skinny.hip asks the same)
-static bool gemv1_fits(int K, int E) { return ((K / E + 3) / 4 + 1 + 63) / 64 <= 9; }
+// The longest rows the one-row kernel takes: a quarter of the 16-byte chunks per wave and one to spare, in at most nine registers' worth per lane; three
+// behind the norm of a float row
+static bool gemv1_fits_in(int K, int dtype, int chunks_per_lane) {
+    return ((K / (16 / (int)raven_host::elt_size(dtype)) + 3) / 4 + 1 + 63) / 64 <= chunks_per_lane;
+}
+bool gemv1_fits(int K, int dtype) { return gemv1_fits_in(K, dtype, 9); }
+bool gemv1_stream_fits(int K, int dtype) { return gemv1_fits_in(K, dtype, 3); }
 
 template <typename T, int EPI>
 static int launch_gemv1(Gemv1Args a, hipStream_t s) {
@@ -306,8 +311,9 @@ static int launch_gemv1(Gemv1Args a, hipStream_t s) {
     if (c > 3) ppw = 1;  // the double-buffered variant exists for short rows only (registers)
     a.pairs_per_wg = ppw;
     const int wgs = (units + ppw - 1) / ppw;
-    RAVEN_REQUIRE(gemv1_fits(a.K, E), "gemv_fused: K=%d is too long for the one-row kernel (max %d)", a.K, 9 * 64 * 4 * E - 4 * E);
-    RAVEN_REQUIRE(a.dim == 0 || c <= 3, "gemv: K=%d is too long for the float-row norm prologue", a.K);
+    constexpr int dtype = sizeof(T) == 2 ? RAVEN_BF16 : RAVEN_F32;
+    RAVEN_REQUIRE(gemv1_fits(a.K, dtype), "gemv_fused: K=%d is too long for the one-row kernel (max %d)", a.K, 9 * 64 * 4 * E - 4 * E);
+    RAVEN_REQUIRE(a.dim == 0 || gemv1_stream_fits(a.K, dtype), "gemv: K=%d is too long for the float-row norm prologue", a.K);
 #define RAVEN_GEMV1(CC)                                                                                                \
     do {                                                                                                               \
         constexpr bool kMulti = CC <= 3;                                                                               \
@@ -368,11 +374,7 @@ int gemv1_free(const void* x0, const void* x1, const void* w, void* y, int N, in
     return gemv1_free_dispatch(a, dtype, s);
 }
 
-// The same behind an RMSNorm of a float row x [K] (weight float, mean over dim channels): true when K is short enough
-bool gemv1_stream_fits(int K, int dtype) {
-    const int n_chunks = K / (16 / (int)raven_host::elt_size(dtype));
-    return ((n_chunks + 3) / 4 + 1 + 63) / 64 <= 3;
-}
+// The same behind an RMSNorm of a float row x [K] (weight float, mean over dim channels), where gemv1_stream_fits
 int gemv1_stream(const float* x, const float* norm, int dim, float eps, const void* w, void* y, int N, int K, const raven_epilogue& epi, int dtype,
                  hipStream_t s) {
     Gemv1Args a{};
