@@ -175,6 +175,26 @@ def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, 
         assert torch.equal(pkg.hip.linear(x, w, workspace=ws), pkg.hip.linear(x, w, workspace=ws))
 
 
+@pytest.mark.parametrize("ks", [1, 3])
+@pytest.mark.parametrize("nt,mt", [(2, 1), (4, 2), (6, 4)])
+def test_infinities_stay_in_their_rows_and_columns(pkg, tuned, nt, mt, ks):
+    """Rows and columns past the end of a tile are repeats of the last ones, pieces past K are zeros, a tile that does not exist repeats another: an
+    infinity or NaN of the last row of x, the last row of w or the last column must reach the outputs it belongs to and no other."""
+    dt = torch.bfloat16
+    for M, N, K in ((33, 72, 72), (130, 328, 200), (70, 200, 1096)):
+        tuned(gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
+        ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+        x, w = _gpu_randn((M, K), 730 + M), _gpu_randn((2 * N, K), 731 + N, 0.05)
+        x[M - 1, K - 1], x[0, 3] = float("inf"), float("nan")
+        w[N - 1, 5] = w[2 * N - 1, 5] = float("inf")
+        bad = torch.zeros(M, 2 * N, dtype=torch.bool, device="cuda")
+        bad[0] = bad[M - 1] = bad[:, N - 1] = bad[:, 2 * N - 1] = True
+        got = pkg.hip.linear(x, w[:N].contiguous(), workspace=ws)
+        assert torch.equal(~got.isfinite(), bad[:, :N]), f"{M} x {N} x {K}"
+        got = pkg.hip.linear(x, w, swiglu=True, workspace=ws)  # (silu of minus infinity is a zero or NaN: that row and column may go either way)
+        assert got.isfinite()[~bad[:, :N]].all() and got[0].isnan().all(), f"{M} x {N} x {K}, SwiGLU"
+
+
 @pytest.mark.parametrize("M,N,K", [(34, 96, 5184), (100, 1280, 1280), (150, 128, 1360), (260, 248, 1168), (400, 1024, 4096)])
 def test_products_with_any_room_for_slices(pkg, M, N, K):
     """Shapes that are cut into K slices where the workspace holds them: with none, with room for two slices, with all of it; plain, + residual, float, SwiGLU,
