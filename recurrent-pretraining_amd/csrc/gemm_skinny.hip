@@ -661,7 +661,8 @@ static int dispatch_gemv(GemmArgs a, hipStream_t s) {
 // round of them; with eight, and the partial sums added through LDS, the K slices of gemm_splitk.hip and their second launch are not needed
 // either, up to the length of K where the workgroups become too long (splits_k there).  But eight waves of short rows do little else than
 // start and add up, and with few rows of X the shorter workgroups of four waves lose nothing.  Time of one round over that of four waves, from 2 x 3600 products:
-//   one tile    K of 256 1.03 - 1.07, 512 1.02 - 1.04, 640 0.92, 2048 0.85 - 0.98, 8192 0.68 - 0.97 (SwiGLU 512 1.03, 640 0.94, 4096 0.88 - 1.02)
+//   one tile    K of 256 1.03 - 1.07, 512 1.02 - 1.04, 640 0.92, 2048 0.85 - 0.98, 8192 0.68 - 0.97 (SwiGLU up to 16 rows 512 1.03, 640 0.94, 4096 0.88 - 0.96;
+//               17 rows 0.92 - 1.01, 32 rows 0.97 - 1.04, where rows alternate between whole and half lines 17 to 32 rows 1.01 - 1.07)
 //   two tiles   up to 8 rows 0.95 - 1.18; 16 rows: K of 1536 1.05 - 1.08, 2048 0.92, 2560 1.02, 4096 0.95 - 1.03, 5120 0.92; 24 rows: 1536 1.05, 2048 0.90, 5120 0.87; with 257 tiles
 //               for 256 CUs, half of them without a workgroup, 1.0 - 1.27 up to 16 rows; from 509 tiles on (four tiles per four-wave workgroup past
 //               16 rows) 0.7 - 0.88 at 24 rows, whatever K
@@ -674,7 +675,7 @@ static int dispatch_gemv(GemmArgs a, hipStream_t s) {
 template <bool SWIGLU>
 static bool one_round_pays(const GemmArgs& a, int tiles) {
     const int n = a.N / 16, cus = n_cus(), steps = (a.K / 64 + 7) / 8;  // steps: of 64 columns, per wave
-    if (tiles == 1) return a.K > 512;
+    if (tiles == 1) return a.K > 512 && (!SWIGLU || a.M <= 16 || (a.M <= 24 && a.line_aligned));
     if (SWIGLU) return false;  // two gate tiles and their up tiles: no faster than the four-wave kernels (14.4 / 14.1 at 12288 x 2048)
     const int rs = a.row_stride;
     if (a.M > 16 && (n + 4 * rs - 1) / (4 * rs) * rs >= cus / 2) return true;  // (else dispatch_mfma takes four tiles per four-wave workgroup)
