@@ -304,7 +304,13 @@ static int launch_gemv1(Gemv1Args a, hipStream_t s) {
     // 7 for mlp.fc (17920 gate / up pairs, 2560 workgroups: 57.6 us against 58.4 with 4, while Wqkv loses with more than 4)
     // rows of one chunk per lane: about four workgroups per CU (8192 x 2048 behind the float norm 8.0 us against 8.4, 8192 x 1024 6.5 / 6.8)
     const int per_cu = c <= 1 ? 4 : 10;
-    if (norm && ppw <= 0) ppw = (units + per_cu * gemv1_cus() - 1) / (per_cu * gemv1_cus());
+    if (norm && ppw <= 0) {
+        ppw = (units + per_cu * gemv1_cus() - 1) / (per_cu * gemv1_cus());
+        // ... but no more pairs of rows than 32 KB (two chunks per lane: 5 pairs), beyond which fewer and longer workgroups lose: 17920 x 2048 in bf16 behind
+        // the norm 13.4 us with 4 pairs, 14.2 with 9; 24000 x 2048 17.1 / 18.2; 65536 x 1536 floats behind the float norm 58.5 with 5, 62.7 with 13
+        const int most = c <= 1 ? 16384 / (a.K * (int)sizeof(T)) : c == 2 ? 5 : kMaxPairsPerWg;
+        if (ppw > most) ppw = most;
+    }
     if (ppw < 1) ppw = 1;
     if (ppw > kMaxPairsPerWg) ppw = kMaxPairsPerWg;
     while (ppw > 1 && (units + ppw - 1) / ppw < 1024) --ppw;  // keep at least ~4 workgroups per CU

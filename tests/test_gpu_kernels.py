@@ -385,6 +385,26 @@ def test_one_row_of_every_length_of_share(pkg, dt, chunks):
         check(got[None], lin(h[None], w).to(dt), dt, "float norm")
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,row_bytes", [(26001, 1024), (26001, 4096), (26001, 6144), (9001, 12288)])
+def test_one_row_in_many_pairs_per_workgroup(pkg, dt, N, row_bytes):
+    """Up to 13, 4, 5 and 2 pairs of rows in turn, the last workgroup and the last pair partly empty, behind both norms."""
+    K = row_bytes // dt.itemsize
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(dt)
+    xf, nw = torch.randn(K, generator=g, device="cuda"), 1 + 0.1 * torch.randn(K, generator=g, device="cuda")
+    h = xf * torch.rsqrt((xf * xf).mean() + 1e-6) * nw
+    if pkg.hip.gemv_stream_fits(K, dt):
+        got = pkg.hip.gemv_stream(xf, nw, K, 1e-6, w, dt)
+        want = w.double() @ h.to(dt).double()
+        assert ((got - want).norm() / want.norm()).item() < (2e-3 if dt == torch.bfloat16 else 1e-6)  # (a norm that rounds the other way here and there)
+    x, nt = xf.to(dt), nw.to(dt)
+    y = pkg.hip.gemv_fused(x, w, norm_a=nt)[0]
+    xd = x.double()
+    want = w.double() @ (xd * torch.rsqrt((xd * xd).mean() + 1e-6)).to(dt).mul(nt).double()
+    assert ((y.double() - want).norm() / want.norm()).item() < (6e-3 if dt == torch.bfloat16 else 1e-6)  # (outputs and norm in bf16: 2^-9 each)
+
+
 @pytest.mark.parametrize("rows,vocab", [(3, 1), (3, 63), (3, 1024), (3, 2047), (3, 2048), (3, 2049), (3, 4097), (3, 16383), (3, 16384), (3, 16385), (3, 50001), (300, 1500), (300, 16385), (257, 50001)])
 def test_argmax_of_every_remainder(pkg, rows, vocab):
     """Rows that end inside a thread's 2 to 16 values, inside a stripe and on its border; the first of equal maxima, also the last value's."""
