@@ -84,7 +84,7 @@ const char* raven_arch(void);
 const char* raven_last_error(void);
 
 /* Launch-shape overrides for experiments (grid sizing and load hints of the skinny-GEMM kernels);
- * results never depend on them.  Keys: gemv_units_per_wave, gemv_interleave, gemv_nontemporal,
+ * results depend on them only through the order of fp32 sums (keys that choose between kernels, K slices or ranges of cache positions).  Keys: gemv_units_per_wave, gemv_interleave, gemv_nontemporal,
  * gemv_wgs_per_cu, gemv1_pairs_norm (weight-row pairs per workgroup of the one-row kernel with a norm prologue; 0 = by shape,
  * about ten workgroups per compute unit), gemv1_pairs_plain, gemm_four_tiles (0 / 1 / 2 = never / by rule / always use
  * the four-tile MFMA variant), attn_split_target / attn_big_grid (workgroups a split decode-attention launch aims
@@ -132,8 +132,8 @@ int raven_rmsnorm_residual(const void* x, const void* residual, const void* weig
                            void* sum_out, const void* weight2, void* y2,
                            int64_t rows, int32_t dim, float eps, int32_t dtype, void* stream);
 
-/* Y[M,N] = X[M,K] W[N,K]^T for skinny M (any M >= 1; up to 32 rows in bf16 and up to 8 in f32 read
- * the weight matrix once).  Replaces the nn.Linear calls of attn.proj (RMM:493), mlp.proj (RMM:509) and lm_head (RMM:711).  fp32 accumulate, result rounded to T; then, if residual != NULL,
+/* Y[M,N] = X[M,K] W[N,K]^T for any M >= 1 (up to 32 rows in bf16 and up to 64 in f32 read
+ * the weight matrix once; f32 rows hold at most 40960 values).  Replaces the nn.Linear calls of attn.proj (RMM:493), mlp.proj (RMM:509) and lm_head (RMM:711).  fp32 accumulate, result rounded to T; then, if residual != NULL,
  * Y = T(Y + residual) (RMM:534-535); if out_f32 != 0 the rounded result is stored as float
  * (the `.float()` of RMM:711).  K * sizeof(T) % 16 == 0. */
 int raven_gemm(const void* x, const void* w, const void* residual, void* y,
@@ -506,7 +506,8 @@ int    raven_rglru_forward(const raven_rglru* l, const void* z, float* ring, flo
 /* Mixture of gated experts, added to the stream: x += sum over the `top` experts of largest score of E(s h) + sigmoid(g) E_shared(h), with
  * s = sigmoid(router logit) of the expert (not renormalised; it scales the expert's input) and E(h) = W_down (silu(W_gate h) * (W_up h)).
  * logits [M, logit_ld] float: one column per expert, then g (with a shared expert).  h [M, ld] of T, x [M, ld] float.
- * Equal scores: the lower index wins.  Chunks run the experts as one grouped product, few rows (and fp32) row by row. */
+ * Equal scores: the lower index wins.  Chunks, and from 2 rows on fewer wherever that is the faster way, run the experts as one grouped product; one row,
+ * fp32 and operands that do not start on 16 bytes run row by row. */
 typedef struct raven_moe {
     const void* router;      /* [logit_ld, ld]: a row per expert, the shared expert's gate, zeros */
     const void* up;          /* [experts, 2 * ff, ld]: gate rows, then up rows */

@@ -15,9 +15,10 @@
 // free of bank conflicts.  Unlike the tiles of gemm_tiled.hip a wave's partial sums over K slices are added after the fact, so results
 // differ from those in the order of fp32 sums.
 //
-// us per launch at 93 rows of the 3.5b shape, 128 x 128 tiles or passes of 32 rows before / this kernel (both launches where K is split):
-// Wqkv 67 / 47, attn.proj 63 / 23, mlp.fc 124 / 79, mlp.proj 113 / 54, adapter 77 / 35; at 195 rows 66 / 60, 61 / 35, 157 / 114, 192 / 85;
-// at 45 rows Wqkv 63 / 34, mlp.fc 108 / 68 (5.6 TB/s of weights), mlp.proj 72 / 43; 4096 x 2048 x 8192 with an fp32 residual 166 / 135.
+// us per launch at 93 rows of the 3.5b shape, weights from HBM (those of K = 5280 through their line-aligned copies), 128 x 128 tiles or passes of 32
+// rows before / this kernel (both launches where K is split): Wqkv 68 / 52, attn.proj 62 / 26, mlp.fc 125 / 91, mlp.proj 112 / 55, adapter 78 / 38; at
+// 195 rows 67 / 63, 59 / 35, 158 / 128, 188 / 83, 113 / 56; at 45 rows Wqkv 67 / 37, mlp.fc 110 / 74 (5.1 TB/s of weights), mlp.proj 72 / 43;
+// 4096 x 2048 x 8192 with an fp32 residual 163 / 133.
 
 #include "gemm_common.h"
 

@@ -63,7 +63,7 @@ struct TiledArgs {
     int out_f32;
     int tiles_m, tiles_n;
     raven_epilogue epi;    // EPI_FREE only (y and residual [M, ldy])
-    RowGroups groups;      // GROUPED only (grouped_gemm)
+    RowGroups groups;      // GROUPED only (ring_grouped)
     int rope_on;           // the epilogue below instead of y
     RopeAppend rope;       // (gemm_common.h)
 };
