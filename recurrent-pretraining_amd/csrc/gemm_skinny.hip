@@ -664,7 +664,7 @@ static int dispatch_gemv(GemmArgs a, hipStream_t s) {
 //   one tile    K of 256 1.03 - 1.07, 512 1.02 - 1.04, 640 0.92, 2048 0.85 - 0.98, 8192 0.68 - 0.97 (SwiGLU up to 16 rows 512 1.03, 640 0.94, 4096 0.88 - 0.96;
 //               17 rows 0.92 - 1.01, 32 rows 0.97 - 1.04, where rows alternate between whole and half lines 17 to 32 rows 1.01 - 1.07)
 //   two tiles   up to 8 rows 0.95 - 1.18; 16 rows: K of 1536 1.05 - 1.08, 2048 0.92, 2560 1.02, 4096 0.95 - 1.03, 5120 0.92; 24 rows: 1536 1.05, 2048 0.90, 5120 0.87; with 257 tiles
-//               for 256 CUs, half of them without a workgroup, 1.0 - 1.27 up to 16 rows; from 509 tiles on (four tiles per four-wave workgroup past
+//               for 256 CUs, half of them without a workgroup, 1.0 - 1.27 up to 16 rows, K of 2048 1.01, 0.98 and 0.95 at 17, 24 and 32, of 2560 1.10 - 1.05; from 509 tiles on (four tiles per four-wave workgroup past
 //               16 rows) 0.7 - 0.88 at 24 rows, whatever K
 //   three tiles 2 rows: 512 1.1 - 1.27, 1536 1.15, 2048 0.91 - 0.99, 2560 1.05 - 1.11, 3072 0.98 - 1.01, 5120 0.93 - 0.98, 8192 0.8; 24 rows 0.83 - 1.0
 //   four tiles  2 rows 1.0 - 1.17, but 0.91 at 4096; 16 rows: 512 1.09, 2048 1.05, 2560 1.0, 4096 0.9, 5120 0.97, 6144 1.1
@@ -683,7 +683,7 @@ static bool one_round_pays(const GemmArgs& a, int tiles) {
     const int pitch = 2 * a.K;
     const bool one_channel = pitch >= 8192 && (pitch & (pitch - 1)) == 0;
     if (tiles == 2) {
-        if (a.M > 16) return n >= cus + cus / 8 || steps >= 6;
+        if (a.M > 16) return n >= cus + cus / 8 || steps >= 6 || (steps == 4 && a.K >= 1792 && a.M > 24);
         if (n < cus + cus / 8 || steps == 5 || one_channel) return false;
         return a.M >= 16 || (n <= cus + cus / 2 && (a.M >= 12 || (rs == 2 && steps >= 6)));
     }
