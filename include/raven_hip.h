@@ -235,7 +235,10 @@ int raven_exit_latent_stats(const void* latents, const void* prev, void* rel_cha
  *   [T, n_heads * head_dim]; they are the LAST positions of its seq_lens[b] cached positions (already appended), so row
  *   r of the sequence attends to positions 0 .. seq_lens[b] - (rows of b) + r.  max_q_len >= every sequence's row count
  *   sizes the launch; a sequence with no rows, or more rows than positions, is left alone.  Same kernel as
- *   raven_prefill_attention with the key tiles gathered through the block table. */
+ *   raven_prefill_attention with the key tiles gathered through the block table; a sequence's only row goes through the cache on the
+ *   vector units instead.
+ * raven_paged_prefill_attention_rows: the same for a caller that knows T = q_start[B], the rows of all sequences together (-1: not known): the
+ *   launch then holds no workgroup for blocks of rows that the shorter sequences do not have. */
 enum { RAVEN_PAGED_NHD = 0, RAVEN_PAGED_HND = 1 };
 int raven_paged_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* slot_mapping,
                           int32_t T, int32_t n_heads, int32_t head_dim, int32_t block_size, int32_t kv_layout,
@@ -258,6 +261,10 @@ int raven_paged_prefill_attention(const void* q, void* y, const void* k_cache, c
                                   const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start,
                                   int32_t B, int32_t max_q_len, int32_t max_blocks, int32_t block_size,
                                   int32_t kv_layout, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
+int raven_paged_prefill_attention_rows(const void* q, void* y, const void* k_cache, const void* v_cache,
+                                       const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start,
+                                       int32_t B, int32_t T, int32_t max_q_len, int32_t max_blocks, int32_t block_size,
+                                       int32_t kv_layout, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
 
 /* A stack of SandwichBlocks over block-paged caches, one decode row per sequence (the flat layer list the plugin's
  * model runs, vllm/raven_vllm.py:365-432: every flat layer owns ONE paged cache, which the recurrences of a token

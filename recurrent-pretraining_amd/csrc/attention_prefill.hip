@@ -47,14 +47,135 @@ struct PrefillArgs {
     const int* block_table;  // [B, max_blocks]
     const int* seq_lens;     // [B]
     const int* q_start;      // [B + 1]
+    int B;
     int max_blocks, block_size, block_shift;  // block_shift = log2(block_size), or -1 when that is not a power of two
+    float per_block;                          // 1 / block_size
     int64_t page_stride, pos_stride, head_stride;  // elements between two pages / positions of a page / heads
 };
 
 constexpr int kPfTable = 1024;  // block-table entries of a sequence held in LDS (beyond that they are read from memory)
 
-template <int HD, int RG, bool PAGED = false, int NW = 4>
+// The only new row of a paged sequence: a decode row in a scheduler step that also carries a prompt chunk.  Four waves, 16 lanes to a cached position, 64
+// positions at a time with the next 64 requested before this tile's are used; float weights, the 16 groups' sums merged through LDS (`merge`, 16 * (HD + 2)
+// floats).  Bound by the cache's bytes and the two workgroups that a CU holds: 15 sequences of 420 positions, 55 heads of 96, 27 to 29 us = 4.6 to 4.9 TB/s
+// (the decode kernel over the same pages 28.5); as one of a tile's 16 query rows, three waves of four without a row and a wait for every staged tile,
+// 40.  off_of: element offset of a position's head row.
+template <int HD, typename OFF>
+__device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, const bf16* K, const bf16* V, int n_keys, float scale_log2, float* merge, OFF off_of) {
+    constexpr int U = 4, G = 16, NC = HD / 8;
+    const int lane = threadIdx.x & 63, ci = lane & 15, group = (threadIdx.x >> 6) * 4 + (lane >> 4);
+    const int at = min(ci, NC - 1) * 8;  // lanes past the row repeat its last chunk against a zero query
+    const Chunk<bf16> qc = ci < NC ? load_chunk(q + at) : zero_chunk<bf16>();
+    float m_run = -INFINITY, l_run = 0.f, o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+    Chunk<bf16> k[2][U], v[2][U];
+    auto request = [&](int base, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const int64_t off = off_of(min(base + G * j + group, n_keys - 1)) + at;
+            k[s][j] = load_chunk_stream(K + off);
+            v[s][j] = load_chunk_stream(V + off);
+        }
+    };
+    auto use = [&](int base, int s) __attribute__((always_inline)) {
+        float sc[U], top = m_run;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            sc[j] = row16_sum(dot_chunk(qc, k[s][j], 0.f)) * scale_log2;
+            if (base + G * j + group >= n_keys) sc[j] = -INFINITY;
+            top = fmaxf(top, sc[j]);
+        }
+        const float ref = top == -INFINITY ? 0.f : top;  // a group that has seen no position: all its weights are 0
+        const float corr = __builtin_amdgcn_exp2f(m_run - ref);
+        l_run *= corr;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] *= corr;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const float w = __builtin_amdgcn_exp2f(sc[j] - ref);
+            l_run += w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(w, to_f32(v[s][j].v[e]), o[e]);
+        }
+        m_run = top;
+    };
+    constexpr int T = G * U;
+    request(0, 0);
+    for (int base = 0; base < n_keys; base += 2 * T) {  // a request past the end repeats the last position
+        request(base + T, 1);
+        use(base, 0);
+        request(base + 2 * T, 0);
+        use(base + T, 1);
+    }
+    if (ci < NC) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) merge[group * HD + at + e] = o[e];
+    }
+    if (ci == 0) {
+        merge[G * HD + group] = m_run;
+        merge[G * HD + G + group] = l_run;
+    }
+    __syncthreads();
+    if (threadIdx.x < HD) {
+        float top = -INFINITY, L = 0.f, O = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) top = fmaxf(top, merge[G * HD + g]);  // finite: position 0 exists
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float w = __builtin_amdgcn_exp2f(merge[G * HD + g] - top);
+            L += merge[G * HD + G + g] * w;
+            O += merge[g * HD + threadIdx.x] * w;
+        }
+        y[threadIdx.x] = from_f32<bf16>(O / L);
+    }
+}
+
+// PAGES: 0 = a contiguous cache; 1 = block-paged, sequences of at most kPfTable pages and 2^20 positions, whose table entries all lie in LDS; 2 = block-paged,
+// longer tables: entries past kPfTable come from memory.  (That choice and the one between a shift and a division are branches around every position's loads,
+// which then are no longer in flight together: two rows each of 15 sequences of 420 positions and a chunk of 180 rows of 55 heads of 96 took 63 us with them,
+// 50 without.)
+// Which block of query rows a workgroup of a paged launch takes: the blocks of `rows` rows that the B sequences have, counted through their row starts and
+// handed out from the last one on -- schedulers put prompt chunks behind decode rows, and a sequence's last block has the most keys.  (A grid of the longest
+// sequence's blocks for every sequence starts workgroups without rows: 825 of them beside the 15 sequences and 180-row chunk above took 12 us.)
+__device__ __forceinline__ bool paged_block(const PrefillArgs& a, int rows, int* seq, int* block) {
+    const int lane = threadIdx.x & 63;
+    auto blocks_of = [&](int i) {
+        if (i >= a.B) return 0;
+        const int n = a.q_start[i + 1] - a.q_start[i];
+        return n > 0 && n <= a.seq_lens[i] ? (n + rows - 1) / rows : 0;
+    };
+    auto summed = [&](int n) {  // over the lanes up to this one
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int v = __shfl_up(n, d, 64);
+            if (lane >= d) n += v;
+        }
+        return n;
+    };
+    int mine = blocks_of(lane), upto = summed(mine), total = __shfl(upto, 63, 64);
+    for (int i0 = 64; i0 < a.B; i0 += 64) total += __shfl(summed(blocks_of(i0 + lane)), 63, 64);
+    int want = total - 1 - (int)blockIdx.x;
+    if (want < 0) return false;
+    for (int i0 = 0;; i0 += 64) {
+        if (i0 > 0) {
+            mine = blocks_of(i0 + lane);
+            upto = summed(mine);
+        }
+        const uint64_t past = __builtin_amdgcn_ballot_w64(upto > want);
+        if (past != 0) {
+            const int l = __builtin_ctzll(past);
+            *seq = i0 + l;
+            *block = want - __builtin_amdgcn_readlane(upto - mine, l);
+            return true;
+        }
+        want -= __shfl(upto, 63, 64);
+    }
+}
+
+template <int HD, int RG, int PAGES = 0, int NW = 4>
 __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_kernel(PrefillArgs a) {
+    constexpr bool PAGED = PAGES != 0;
     constexpr int NTH = NW * 64;     // threads; NW waves, each with its own query rows
     constexpr int KS = HD / 32;      // k-steps of the score MFMA
     constexpr int NT = HD / 16;      // 16-wide output tiles of O; tile NT holds the row sums
@@ -71,8 +192,12 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     // 32 lanes read transposed (8 banks each) hit 64 different banks
     bf16(*sv)[kPfKeys][kVPitch] = reinterpret_cast<bf16(*)[kPfKeys][kVPitch]>(smem_kv + SK_ELEMS);
 
-    const int qb = gridDim.x - 1 - blockIdx.x;  // the blocks with the most keys start first
-    const int head = blockIdx.y, b = blockIdx.z;
+    int qb = gridDim.x - 1 - blockIdx.x;  // the blocks with the most keys start first
+    int b = blockIdx.z;
+    if constexpr (PAGED) {
+        if (!paged_block(a, ROWS, &b, &qb)) return;
+    }
+    const int head = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qc = lane & 15, s4 = lane >> 4;
     const int h = a.nh * HD;
@@ -88,7 +213,6 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
         t_lim = a.seq_lens[b];
         pos0 = t_lim - n_rows;
         table_row = a.block_table + (int64_t)b * a.max_blocks;
-        if (n_rows <= 0 || pos0 < 0 || qb * ROWS >= n_rows) return;  // the grid is sized for the longest sequence
     } else {
         q_row0 = (int64_t)b * a.S;
         n_rows = a.S;
@@ -97,10 +221,32 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     }
 
     const int row0 = qb * ROWS + wave * WR;            // first query row (within the sequence) of this wave
+    const bool idle = PAGED && row0 >= n_rows;         // a wave without rows only helps staging
     const int64_t head_off = PAGED ? (int64_t)head * a.head_stride : a.slot_off + ((int64_t)b * a.nh + head) * a.t_max * HD;
     const bf16* Kb = a.k + head_off;
     const bf16* Vb = a.v + head_off;
 
+    // the page of position p: without a branch in a tile's loads.  (p + 1/2) / block_size in float is off by less than 2^-22 of itself, so that its whole
+    // part is right for positions below 2^20
+    auto page_of = [&](int p) {
+        if (PAGES == 1) return (int)(((float)p + 0.5f) * a.per_block);
+        return a.block_shift >= 0 ? p >> a.block_shift : p / a.block_size;
+    };
+    if constexpr (PAGED) {
+        if (n_rows == 1) {
+            const int n_pages = (t_lim + a.block_size - 1) / a.block_size;
+            for (int i = threadIdx.x; i < min(n_pages, kPfTable); i += NTH) tbl[i] = table_row[i];
+            __syncthreads();
+            static_assert(NW == 4 && (SK_ELEMS + SV_ELEMS) * sizeof(bf16) >= 16 * (HD + 2) * sizeof(float), "sixteen groups, room to merge them");
+            single_row_attention<HD>(a.q + q_row0 * h + head * HD, a.y + q_row0 * a.ldy + head * HD, Kb, Vb, t_lim, a.scale_log2, reinterpret_cast<float*>(smem_kv),
+                                     [&](int p) {
+                                         const int pg = page_of(p);
+                                         const int page = PAGES == 1 || pg < kPfTable ? tbl[pg] : table_row[pg];
+                                         return (int64_t)page * a.page_stride + (int64_t)((p - pg * a.block_size) * (int)a.pos_stride);
+                                     });
+            return;
+        }
+    }
     // Q fragments (B operand of S^T = K Q^T): lane supplies Q[q = l%16][d = 32*ks + 8*(l/16) ..+8] of each row group
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -154,18 +300,27 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     // (they are masked): only the pages up to it are in `tbl`, and only those are known to exist.
     auto paged_off = [&](int p) {
         p = min(p, n_keys - 1);
-        const int pg = a.block_shift >= 0 ? p >> a.block_shift : p / a.block_size;
-        const int page = pg < kPfTable ? tbl[pg] : table_row[pg];
+        const int pg = page_of(p);
+        const int page = PAGES == 1 || pg < kPfTable ? tbl[pg] : table_row[pg];
         return (int64_t)page * a.page_stride + (int64_t)(p - pg * a.block_size) * a.pos_stride;
     };
     auto fetch = [&](int kt) {
-        if constexpr (PAGED) {
+        if constexpr (PAGES == 1) {
+#pragma unroll
+            for (int i = 0; i < KCH; ++i) {
+                const int c = threadIdx.x + NTH * i;
+                const int key = c / CPR, dc = c - key * CPR;
+                const int64_t o = paged_off(kt + key);
+                kreg[i] = *reinterpret_cast<const u32x4*>(Kb + o + dc * 8);
+                vreg[i] = *reinterpret_cast<const u32x4*>(Vb + o + dc * 8);
+            }
+        } else if constexpr (PAGED) {
             if (a.block_shift >= 0 && kt + kPfKeys <= n_keys) {
                 // a whole tile of needed keys, pages of 2^n positions: shifts instead of divisions, no clamping
                 const int mask = a.block_size - 1;
                 auto off = [&](int p) {
                     const int pg = p >> a.block_shift;
-                    const int page = pg < kPfTable ? tbl[pg] : table_row[pg];
+                    const int page = PAGES == 1 || pg < kPfTable ? tbl[pg] : table_row[pg];
                     return (int64_t)page * a.page_stride + (int64_t)((p & mask) * (int)a.pos_stride);
                 };
 #pragma unroll
@@ -352,7 +507,8 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     __syncthreads();
     int buf = 0;
     for (int kt = 0; kt < n_keys; kt += kPfKeys, buf ^= 1) {
-        if (kt + kPfKeys - 1 <= pos0 + row0) tile(kt, buf, std::false_type{});
+        if (idle) {
+        } else if (kt + kPfKeys - 1 <= pos0 + row0) tile(kt, buf, std::false_type{});
         else if (kt <= wave_last) tile(kt, buf, std::true_type{});
         if (kt + kPfKeys < n_keys) {
             park(buf ^ 1);  // last read two tiles ago; every wave has passed the barrier since
@@ -435,7 +591,7 @@ int prefill_attention_pitched(const void* q, void* y, int ldy, const raven_kv_ca
 #define RAVEN_PREFILL(HD)                                                                  \
     if (rg == 2) attention_prefill_kernel<HD, 2><<<grid, dim3(256), 0, s>>>(a);            \
     else attention_prefill_kernel<HD, 1><<<grid, dim3(256), 0, s>>>(a)
-    if (six) attention_prefill_kernel<96, 2, false, 6><<<grid, dim3(384), 0, s>>>(a);
+    if (six) attention_prefill_kernel<96, 2, 0, 6><<<grid, dim3(384), 0, s>>>(a);
     else if (head_dim == 64) { RAVEN_PREFILL(64); }
     else if (head_dim == 96) { RAVEN_PREFILL(96); }
     else { RAVEN_PREFILL(128); }
@@ -454,6 +610,14 @@ extern "C" int raven_paged_prefill_attention(const void* q, void* y, const void*
                                              const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start, int32_t B,
                                              int32_t max_q_len, int32_t max_blocks, int32_t block_size, int32_t kv_layout,
                                              int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream) {
+    return raven_paged_prefill_attention_rows(q, y, k_cache, v_cache, block_table, seq_lens, q_start, B, -1, max_q_len, max_blocks, block_size, kv_layout,
+                                              n_heads, head_dim, dtype, stream);
+}
+
+extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const void* k_cache, const void* v_cache,
+                                                  const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start, int32_t B, int32_t T,
+                                                  int32_t max_q_len, int32_t max_blocks, int32_t block_size, int32_t kv_layout,
+                                                  int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream) {
     using namespace raven;
     RAVEN_REQUIRE(dtype == RAVEN_BF16, "paged_prefill_attention: bf16 only (dtype %d)", dtype);
     RAVEN_REQUIRE(head_dim == 64 || head_dim == 96 || head_dim == 128, "paged_prefill_attention: head_dim %d not in {64, 96, 128}", head_dim);
@@ -470,8 +634,10 @@ extern "C" int raven_paged_prefill_attention(const void* q, void* y, const void*
     a.v = static_cast<const bf16*>(v_cache);
     a.nh = n_heads; a.hd = head_dim;
     a.scale_log2 = (float)(1.0 / sqrt((double)head_dim) * 1.4426950408889634);
-    a.block_table = block_table; a.seq_lens = seq_lens; a.q_start = q_start;
+    a.block_table = block_table; a.seq_lens = seq_lens; a.q_start = q_start; a.B = B;
     a.max_blocks = max_blocks; a.block_size = block_size; a.block_shift = -1;
+    a.per_block = 1.0f / (float)block_size;
+    const bool short_tables = max_blocks <= kPfTable && (int64_t)max_blocks * block_size <= (1 << 20);
     for (int sh = 0; sh < 31; ++sh)
         if (block_size == (1 << sh)) a.block_shift = sh;
     RAVEN_REQUIRE((int64_t)block_size * n_heads * head_dim < (1ll << 31), "paged_prefill_attention: a page of %d positions is too large", block_size);
@@ -482,10 +648,17 @@ extern "C" int raven_paged_prefill_attention(const void* q, void* y, const void*
     const int64_t wgs128 = (int64_t)((max_q_len + 127) / 128) * n_heads * B;
     const int rg = wgs128 >= 512 ? 2 : 1;
     const int rows = 64 * rg;
-    const dim3 grid((max_q_len + rows - 1) / rows, n_heads, B);
+    // as many blocks as the sequences can have: those of the longest one each, or of T rows in all, each sequence's last one partly filled
+    int64_t blocks = (int64_t)((max_q_len + rows - 1) / rows) * B;
+    if (T >= 0 && T / rows + B < blocks) blocks = T / rows + B;
+    RAVEN_REQUIRE(blocks < (1ll << 31), "paged_prefill_attention: grid too large");
+    const dim3 grid((unsigned)blocks, n_heads);
 #define RAVEN_PREFILL(HD)                                                                        \
-    if (rg == 2) attention_prefill_kernel<HD, 2, true><<<grid, dim3(256), 0, s>>>(a);            \
-    else attention_prefill_kernel<HD, 1, true><<<grid, dim3(256), 0, s>>>(a)
+    if (short_tables) {                                                                          \
+        if (rg == 2) attention_prefill_kernel<HD, 2, 1><<<grid, dim3(256), 0, s>>>(a);           \
+        else attention_prefill_kernel<HD, 1, 1><<<grid, dim3(256), 0, s>>>(a);                   \
+    } else if (rg == 2) attention_prefill_kernel<HD, 2, 2><<<grid, dim3(256), 0, s>>>(a);        \
+    else attention_prefill_kernel<HD, 1, 2><<<grid, dim3(256), 0, s>>>(a)
     if (head_dim == 64) { RAVEN_PREFILL(64); }
     else if (head_dim == 96) { RAVEN_PREFILL(96); }
     else { RAVEN_PREFILL(128); }

@@ -160,6 +160,7 @@ SIGNATURES = {
                                         C.POINTER(KVCache), C.POINTER(C.c_int32), _I32, _I32, _I32, _I32, _VP, _VP, _SZ, _VP]),
     "raven_paged_qkv_rope_append": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _VP]),
     "raven_paged_prefill_attention": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _VP]),
+    "raven_paged_prefill_attention_rows": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _VP]),
     "raven_paged_decode_blocks": (C.c_int, [C.POINTER(Dims), _VP, C.POINTER(BlockWeights), _I32, _VP, _VP, _VP, _VP, _VP,
                                             C.POINTER(PagedKV), _I32, _I32, _VP, _SZ, _VP]),
     "raven_linear_epilogue": (C.c_int, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, C.POINTER(Epilogue), _I32, _VP, _SZ, _VP]),
@@ -399,11 +400,11 @@ def paged_prefill_attention(q, k_cache, v_cache, block_table, seq_lens, q_start,
         raise RavenHipError("paged_prefill_attention: block_table [B, max_blocks], seq_lens [B] and q_start [B + 1] do not fit together")
     block_size, nh, hd = _paged_dims(k_cache, layout)
     y = torch.empty_like(q)
-    rc = load().raven_paged_prefill_attention(
+    rc = load().raven_paged_prefill_attention_rows(
         _ptr(q, "q"), _ptr(y, "y"), _ptr(k_cache, "k_cache", q.dtype), _ptr(v_cache, "v_cache", q.dtype),
         _ptr(block_table, "block_table", torch.int32), _ptr(seq_lens, "seq_lens", torch.int32), _ptr(q_start, "q_start", torch.int32),
-        B, int(max_q_len), block_table.shape[1], block_size, layout, nh, hd, dtype_code(q.dtype), _stream())
-    _check(rc, "raven_paged_prefill_attention")
+        B, q.shape[0], int(max_q_len), block_table.shape[1], block_size, layout, nh, hd, dtype_code(q.dtype), _stream())
+    _check(rc, "raven_paged_prefill_attention_rows")
     return y
 
 

@@ -1032,3 +1032,48 @@ def test_paged_rope_append_and_prefill_attention_of_several_sequences(pkg, nh, h
         t0 += r
     with pytest.raises(pkg.hip.RavenHipError):
         pkg.hip.paged_prefill_attention(q[:T].float(), kc.float(), vc.float(), table.cuda(), lens.cuda(), q_start.cuda(), max_q, layout=lay)
+
+
+@pytest.mark.parametrize("layout", ["HND", "NHD"])
+@pytest.mark.parametrize("nh,hd,block_size", [(55, 96, 16), (3, 64, 12), (2, 128, 32)])
+def test_single_rows_beside_a_chunk_of_paged_attention(pkg, nh, hd, block_size, layout):
+    """raven_paged_prefill_attention: a sequence with one new row takes a path of its own (tiles of 64 positions, two in flight); lengths
+    around those tiles, one longer than the block-table entries held in LDS (other tables alone, without it), beside chunks whose last waves have no rows
+    and a sequence without rows, more sequences than a wave counts at once; against 64 bits.  Bound: one rounding of the output behind float sums;
+    for a chunk's rows, whose weights are rounded too, two."""
+    dt = torch.bfloat16
+    lens = [1, 2, 63, 64, 65, 128, 129, 191, 300, 700, 70, 40, 150]
+    rows = [1] * 10 + [35, 0, 130]
+    for extra in ([], [1024 * block_size + 5]) if nh < 10 else ([],):
+        _check_paged_rows(pkg, nh, hd, block_size, layout, dt, (lens + extra) * (6 if nh < 10 else 1), (rows + [1] * len(extra)) * (6 if nh < 10 else 1))
+
+
+def _check_paged_rows(pkg, nh, hd, block_size, layout, dt, lens, rows):
+    B, max_blocks = len(lens), (max(lens) + block_size - 1) // block_size
+    used = [(n + block_size - 1) // block_size for n in lens]
+    table = torch.zeros(B, max_blocks, dtype=torch.int32)
+    place = torch.randperm(sum(used), generator=torch.Generator().manual_seed(900 + hd)).to(torch.int32)
+    for b, n in enumerate(used):
+        table[b, :n], place = place[:n], place[n:]
+    shape = (sum(used), block_size, nh, hd) if layout == "NHD" else (sum(used), nh, block_size, hd)
+    k, v = rnd(shape, dt, 901).cuda(), rnd(shape, dt, 902).cuda()
+    q = rnd((sum(rows), nh * hd), dt, 903, 2.0).cuda()
+    q_start = torch.tensor([0] + rows).cumsum(0).to(torch.int32)
+    lay = pkg.hip.PAGED_NHD if layout == "NHD" else pkg.hip.PAGED_HND
+    dev = [t.cuda() for t in (table, torch.tensor(lens, dtype=torch.int32), q_start)]
+    y = pkg.hip.paged_prefill_attention(q, k, v, *dev, max(rows), layout=lay)
+    again = torch.zeros_like(y)  # a caller that does not say how many rows there are
+    assert pkg.hip.load().raven_paged_prefill_attention(q.data_ptr(), again.data_ptr(), k.data_ptr(), v.data_ptr(), *(t.data_ptr() for t in dev), B, max(rows),
+                                                        max_blocks, block_size, lay, nh, hd, pkg.hip.dtype_code(dt), pkg.hip._stream()) == 0
+    assert torch.equal(again, y)
+    by_pos = (lambda c: c) if layout == "NHD" else (lambda c: c.transpose(1, 2))
+    for b, (n, r) in enumerate(zip(lens, rows)):
+        if r == 0:
+            continue
+        pages = table[b, :used[b]].long().cuda()
+        keys, vals = (by_pos(c)[pages].reshape(-1, nh, hd)[:n].double().transpose(0, 1) for c in (k, v))
+        at = slice(int(q_start[b]), int(q_start[b + 1]))
+        s = q[at].view(r, nh, hd).double().transpose(0, 1) @ keys.transpose(1, 2) * hd ** -0.5
+        hidden = torch.arange(n)[None] > torch.arange(n - r, n)[:, None]
+        want = (torch.softmax(s.masked_fill(hidden.cuda(), -math.inf), -1) @ vals).transpose(0, 1).reshape(r, -1)
+        check(y[at], want.float().to(dt), dt, f"{r} rows of {n} positions", ulps=1 if r == 1 else 2)
