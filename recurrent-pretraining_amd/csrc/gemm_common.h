@@ -76,7 +76,7 @@ size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu);  // 0 wh
 // when the product was finished
 int mid_gemm(const ProductArgs& a, const MidPlan& p, void* workspace, hipStream_t s, int* ks_left);
 // y[r] = x[x_row[r]] W_g^T, W_g [N or 2N, K] the matrix of row r's group.  swiglu: y = T(silu(s gate) * (s up)) with s = x_scale[r]; else
-// y = the sums, as T or (out_f32) as they are.  tile_rows 16, 32 or 64; rows: rows of the product, x_rows: rows of x.
+// y = the sums, as T or (out_f32) as they are.  tile_rows 32 or 64; rows: rows of the product, x_rows: rows of x.
 int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, int out_f32, const RowGroups& g, hipStream_t s);
 
 }  // namespace raven

@@ -553,13 +553,12 @@ static int launch_grouped(const MidArgs& a, hipStream_t s) {
     return raven_host::check_launch("gemm (grouped)");
 }
 
-// Tiles of 16 and 32 rows: four waves side by side along the weight rows -- with few token rows the eight waves of the larger tiles would
-// read mostly rows that do not exist out of LDS --, four stages of 18 or 20 KB, two workgroups per CU, so that one streams while the
+// Tiles of 32 rows: four waves side by side along the weight rows -- with few token rows the eight waves of the larger tiles would
+// read mostly rows that do not exist out of LDS --, four stages of 20 KB, two workgroups per CU, so that one streams while the
 // other fills its ring or stores (a unit of an expert of 768 channels has 12 to 32 K steps).
 template <int EPI>
 static int launch_grouped_rows(const MidArgs& a, hipStream_t s) {
     switch (a.bm) {
-        case 16: return launch_grouped<EPI, 4, 1, 2, 1, 4>(a, s);
         case 32: return launch_grouped<EPI, 4, 1, 2, 2, 4>(a, s);
         case 64: return launch_grouped<EPI, 2, 4, 4, 1, 3>(a, s);
         default: RAVEN_REQUIRE(false, "gemm (grouped): tiles of %d rows", a.bm);

@@ -6,10 +6,10 @@
 // multiplies them by the down matrices and adds to the stream.  The first picks the row's experts itself from its logits -- a handful
 // of wave reductions -- so no routing launch stands in between; for a single row it also takes the norm of the stream as a prologue.
 // More bf16 rows: the rows are sorted by expert (moe_route_kernel, or moe_pick_kernel and moe_sort_kernel) and the experts run as one
-// grouped product on the matrix cores (gemm_mid.hip, gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of
+// grouped product on the matrix cores (expert_rows_kernel, gemm_mid.hip, gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of
 // its own, and moe_combine_kernel adds a token's slots and its shared expert to the stream in a fixed order.  So an expert's weights
 // are read once and not once per row that picked it: 20 rows over 64 experts of 768 channels at width 2048, 6 each, read
-// 55 experts instead of 120 (246 us before, 124 now).
+// 55 experts instead of 120 (246 us before, 105 now).
 
 #include <algorithm>
 
@@ -371,6 +371,157 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
         }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The grouped products of experts with at most 16 rows a tile: y[r] = x[x_row[r]] W_g^T.  One unit -- a tile's rows against 32 weight rows (up: 16 gate and 16 up
+// rows) -- per workgroup of four waves that take the K steps in turn and never wait for each other; a wave's weight rows come as
+// whole runs of 128 or 256 bytes into two sets of registers, go through its own LDS tile into operand layout and are multiplied on the
+// matrix cores (the scheme of mfma_kernel in gemm_skinny.hip).  Bound by first reads of the weights: three workgroups a CU keep 100 KB in flight, and
+// some 50 units an expert, started as others end, leave no round half empty -- the units of 128 weight rows of gemm_mid.hip, two to a CU, made 1.3 rounds.
+// The K loop asks for nothing past its end and has no load under a branch, so that a wait counts only the step being parked.  us for a whole mixture (four
+// launches, weights from HBM), 64 experts, 6 per row and a shared one, by gemm_mid.hip / now: width 2048, 4 rows 55 / 48, 8: 86 / 71, 20: 120 / 105,
+// 40: 149 / 125; width 1024, 20 rows 44 / 40.6; 128 experts of 512, 8 per row, 20 rows 146 / 113.  Two register sets in flight 110 at 20 rows (fewer
+// resident waves), three 133; 64 weight rows a unit 112.
+// ------------------------------------------------------------------------------------------------
+struct FewArgs {
+    const bf16 *x, *w;
+    void* y;               // [rows, N]
+    int N, K, tiles_n, out_f32;
+    RowGroups g;
+};
+
+template <bool UP, int KM, int NT>
+__global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
+    constexpr int NG = UP ? NT / 2 : NT, COLS = 16 * NG;  // output columns of a unit
+    constexpr int PITCH = KM + 8, LPR = KM / 8, RPI = 64 / LPR, IPT = 16 / RPI;   // lanes per row, rows per load, loads per tile
+    __shared__ __align__(16) bf16 stage[4][16 * (NT + 1)][PITCH];
+    static_assert(sizeof(stage) >= 3 * NT * 64 * 16, "the tiles double as the waves' sums");
+    const int tile = (int)blockIdx.x / a.tiles_n, n0 = ((int)blockIdx.x - tile * a.tiles_n) * COLS;
+    if (tile >= *a.g.used) return;
+    const int g = a.g.group_of[tile], row0 = a.g.group_row[tile], rows = a.g.group_end[tile] - row0;
+    const bf16* W = g == a.g.extra_group ? a.g.w_extra : a.w + g * a.g.w_stride;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ln = lane & 15, kq = lane >> 4;
+    const int lr = lane / LPR, lc = (lane % LPR) * 8, K = a.K;
+    bf16(*my)[PITCH] = stage[wave];
+    const int n_steps = (K + KM - 1) / KM, mine = (n_steps - wave + 3) / 4;
+
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // element offsets of this lane's rows: weight rows past N repeat the last one, token rows past the tile's likewise (neither is stored)
+    unsigned wo[NT][IPT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) wo[t][i] = (unsigned)(min(n0 + (t % NG) * 16 + RPI * i + lr, a.N - 1) + (UP && t >= NG ? a.N : 0)) * (unsigned)K;
+    // XI: load instructions that the tile's token rows need
+    auto run = [&](auto xi_tag) __attribute__((always_inline)) {
+        constexpr int XI = decltype(xi_tag)::value;
+        const bf16* xp[XI];
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int r = row0 + min(RPI * i + lr, rows - 1);
+            xp[i] = a.x + (int64_t)(a.g.x_row ? a.g.x_row[r] : r) * K;
+        }
+        struct Staged {
+            u32x4 w[NT][IPT], x[XI];
+        } st;
+        // step i of this wave
+        auto fetch = [&](int i, Staged& s) __attribute__((always_inline)) {
+            const int kc = min((wave + 4 * i) * KM + lc, K - 8);
+#pragma unroll
+            for (int t = 0; t < XI; ++t) s.x[t] = *reinterpret_cast<const u32x4*>(xp[t] + kc);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) s.w[t][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + wo[t][j] + kc));
+        };
+        auto park = [&](int i, Staged& s) __attribute__((always_inline)) {
+            const bool past = (wave + 4 * i) * KM + lc >= K;  // columns past K are zeros
+            const u32x4 z = {0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) *reinterpret_cast<u32x4*>(&my[t * 16 + RPI * j + lr][lc]) = past ? z : s.w[t][j];
+#pragma unroll
+            for (int t = 0; t < XI; ++t) *reinterpret_cast<u32x4*>(&my[NT * 16 + RPI * t + lr][lc]) = past ? z : s.x[t];
+        };
+        auto multiply = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < KM / 32; ++j) {
+                const bf16x8 xv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&my[NT * 16 + ln][32 * j + 8 * kq]));
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const bf16x8 wv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&my[t * 16 + ln][32 * j + 8 * kq]));
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv, acc[t], 0, 0, 0);
+                }
+            }
+        };
+        // lanes exchange data through the tile without a workgroup barrier: pin the order of the LDS accesses for the compiler
+        auto wave_sync = []() {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        if (mine <= 0) return;
+        fetch(0, st);
+#pragma unroll 1
+        for (int i = 1; i < mine; ++i) {
+            park(i - 1, st);
+            wave_sync();
+            fetch(i, st);
+            multiply();
+            wave_sync();
+        }
+        park(mine - 1, st);
+        wave_sync();
+        multiply();
+    };
+    if (rows <= RPI) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, IPT>{});
+
+    __syncthreads();
+    f32x4(*sums)[NT][64] = reinterpret_cast<f32x4(*)[NT][64]>(&stage[0][0][0]);
+    if (wave > 0) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) sums[wave - 1][t][lane] = acc[t];
+    }
+    __syncthreads();
+    if (wave != 0 || ln >= rows) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] += sums[0][t][lane] + sums[1][t][lane] + sums[2][t][lane];
+    // a lane holds columns 4 kq ..+3 of each tile for token row ln
+    const float xs = UP ? a.g.x_scale[row0 + ln] : 1.f;
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+        const int n = n0 + 16 * t + 4 * kq;
+        if (n >= a.N) continue;
+        const int64_t at = (int64_t)(row0 + ln) * a.N + n;
+        f32x4 v = acc[t];
+        if (UP) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = silu_f32(v[i] * xs) * (acc[UP ? NG + t : t][i] * xs);
+        }
+        if (a.out_f32) {
+            store4(static_cast<float*>(a.y) + at, v);
+        } else {
+            store4(static_cast<bf16*>(a.y) + at, v);
+        }
+    }
+}
+
+static int expert_rows(const void* x, const void* w, void* y, int N, int K, bool up, int out_f32, const RowGroups& g, hipStream_t s) {
+    RAVEN_REQUIRE(g.n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && (!up || g.x_scale), "moe: bad experts");
+    FewArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(w), y, N, K, 0, out_f32, g};
+    constexpr int kUp = 2, kDown = 2;
+    const int cols = up ? 8 * kUp : 16 * kDown;
+    a.tiles_n = (N + cols - 1) / cols;
+    const int64_t units = (int64_t)a.tiles_n * g.n_tiles;
+    RAVEN_REQUIRE(units < (1ll << 31), "moe: too many units");
+    if (up) expert_rows_kernel<true, 128, kUp><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
+    else expert_rows_kernel<false, 64, kDown><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
+    return raven_host::check_launch("moe (rows of an expert)");
+}
+
 template <typename Y>
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -452,14 +603,16 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, MoePath pa
         const size_t rows = pairs + (fold ? M : 0);
         // The smallest tile that most experts' rows fit into; 256 (by the ring kernel, twice the speed per row) from an average of 110 on, if
         // its units -- a tile by 128 channels of `up` or 256 of `down` -- fill the chip's 256 CUs over both products.  us for all launches of a mixture, width 2048, tiles of 16 / 32 / 64 / 256 rows: 100 tokens 169 / 163 / 167 / 218, 500:
-        // 232 / 196 / 181 / 232, 1000: 344 / 255 / 218 / 249, 1500: 474 / 340 / 282 / 272, 4096: - / 695 / 518 / 394; width 1024, 500
+        // 232 / 196 / 181 / 232 (16 rows as gemm_mid.hip took them), 1000: 344 / 255 / 218 / 249, 1500: 474 / 340 / 282 / 272, 4096: - / 695 / 518 / 394; width 1024, 500
         // tokens: 80 / 70 / 63 / 83, 1500: 144 / 109 / 94 / 96.  (128-row tiles of eight waves, as before: 230 at 500, 327 at 1500.)
         // Few units, tiles of 64 / 256: 12 experts of 136 at width 256, 2 per row, 1000 tokens 29 / 47; 16 of 768 at 1024, 1000 tokens 73 / 93, 4000
         // (400 units) 136 / 120; 8 of 2048 at 2048, 500 tokens (190) 105 / 116, 1000 (280) 134 / 122.
+        // 16 rows by expert_rows_kernel against 32: 64 experts, 6 per row, 100 tokens (9 per expert) at widths 1024 / 1536 / 2048 / 2304 61 / 65, 90 / 104,
+        // 136 / 157, 166 / 182; 150 (14) 65 / 66, 101 / 107, 154 / 161, 204 / 187; 200 (18) 72 / 67, 121 / 109, 178 / 168, 259 / 193.
         const size_t mean = pairs / m->experts;
         const size_t big_tiles = pairs / 256 + m->experts / 2;  // an expert's last tile is half full on average
         const bool fills = big_tiles * ((m->ff + 127) / 128 + (ld + 255) / 256) > 256;
-        c.tile_rows = path == kMoeFew || mean <= 6 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows || !fills ? 64 : 256;
+        c.tile_rows = path == kMoeFew || mean <= 10 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows || !fills ? 64 : 256;
         auto tiles = [&](int height) { return (int)(pairs / height) + m->experts + (fold ? (M + height - 1) / height : 0); };
         c.n_tiles = tiles(c.tile_rows);
         const size_t table = (size_t)tiles(16) * 4;  // room for the lowest tiles whatever the height, so that more rows never need less
@@ -563,12 +716,14 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
     const int64_t up_stride = (int64_t)2 * m->ff * ld, down_stride = (int64_t)ld * m->ff;
     RowGroups g{c.group_of, c.group_row, c.group_end, c.used, c.n_tiles, c.tile_rows, c.slot_row, c.slot_scale, up_stride,
                 fold ? static_cast<const bf16*>(m->shared_up) : nullptr, fold ? m->experts : -1};
-    const bool ring = c.tile_rows == 256;
-    int rc = ring ? ring_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, g, s) : mid_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, 0, g, s);
+    const bool ring = c.tile_rows == 256, low = c.tile_rows == 16;
+    int rc = ring ? ring_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, g, s)
+             : low ? expert_rows(h, m->up, c.act, m->ff, ld, true, 0, g, s) : mid_grouped(h, M, m->up, c.act, rows, m->ff, ld, 1, 0, g, s);
     if (rc) return rc;
     g.x_row = nullptr; g.x_scale = nullptr; g.w_stride = down_stride;
     g.w_extra = fold ? static_cast<const bf16*>(m->shared_down) : nullptr;
-    rc = ring ? ring_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, g, s) : mid_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, few, g, s);
+    rc = ring ? ring_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, g, s)
+         : low ? expert_rows(c.act, m->down, c.y, ld, m->ff, false, few, g, s) : mid_grouped(c.act, rows, m->down, c.y, rows, ld, m->ff, 0, few, g, s);
     if (rc) return rc;
     if (m->shared_up && !fold) {
         raven_epilogue e{};

@@ -382,6 +382,14 @@ def test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, same):
     assert ((outs[0].double() - x.double() - want).norm() / want.norm()).item() < 5e-3
 
 
+@pytest.mark.parametrize("M,D,E,top,ff,shared", [(130, 200, 160, 2, 40, False), (100, 2056, 64, 6, 760, True), (6, 1160, 64, 8, 520, True), (33, 1288, 40, 8, 1032, False)])
+def test_mixture_of_low_tiles(pkg, M, D, E, top, ff, shared):
+    """expert_rows_kernel: fewer columns than one K step, steps and 16-column tiles that end early, tiles with rows for one load and for more, as a chunk
+    (slots in bf16) and as few rows (slots in float); bound as beside."""
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, False)
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, True)
+
+
 @pytest.mark.parametrize("M", [1, 3, 20, 200])
 @pytest.mark.parametrize("which", ["h", "up", "down", "shared"])
 def test_mixture_operands_off_sixteen_bytes(pkg, M, which):
