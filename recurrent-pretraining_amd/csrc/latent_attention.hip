@@ -307,9 +307,8 @@ __global__ __launch_bounds__(256) void latent_rows_attention_kernel(LatentArgs a
 constexpr int kLsKeys = 64;
 
 template <int KS, int NTW, int RG>
-__global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
-    constexpr int PITCH = KS * 32 + 16, CPR = KS * 4, NKC = kLsKeys * CPR / 256, PP = kLsKeys + 8;
-    static_assert(kLsKeys * CPR % 256 == 0, "staging shape");
+__global__ __launch_bounds__(256, RG == 1 ? 2 : 1) void latent_step_kernel(LatentArgs a) {
+    constexpr int PITCH = KS * 32 + 16, CPR = KS * 4, CI = (CPR + 15) / 16, PP = kLsKeys + 8;
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
     typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -328,15 +327,43 @@ __global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
     const bf16* lat = static_cast<const bf16*>(a.latent) + (int64_t)b * a.t_max * a.kp;
     const bf16* rot = static_cast<const bf16*>(a.rotated) + (int64_t)b * a.t_max * a.rp;
 
-    u32x4 reg[NKC];
+    // staging: 16 lanes share a position, four positions a wave and load, 16 further per pass; a lane's pieces 16 apart.  Where a piece comes from -- latent
+    // or rotated part -- does not depend on the position: base and stride are set up once, and a load is one multiply-add.  (With the piece's
+    // row and column divided out of a running index per load the kernel was 3500 instructions long, which every workgroup ran through once out of a cold
+    // instruction cache: one row over 500 positions of 16 heads 10.7 us, now 6.9 with 2000; 20 rows over 75 10.3 / 7.2.)
+    const int srow = 4 * wave + q4;
+    const bf16* src[CI];
+    int step[CI];
+    const bool all_there = ld == KS * 32;
+#pragma unroll
+    for (int j = 0; j < CI; ++j) {
+        const int d = 8 * (l16 + 16 * j);
+        src[j] = d >= a.kp && d < ld ? rot + (d - a.kp) : lat + (d < a.kp ? d : 0);
+        step[j] = d >= a.kp && d < ld ? a.rp : a.kp;
+    }
+    u32x4 reg[4][CI];
     auto fetch = [&](int kt) {
 #pragma unroll
-        for (int i = 0; i < NKC; ++i) {
-            const int c = threadIdx.x + 256 * i, d = (c % CPR) * 8;
-            const int64_t p = min(kt + c / CPR, hi - 1);
-            const u32x4 v = *reinterpret_cast<const u32x4*>(d < a.kp ? lat + p * a.kp + d : d < ld ? rot + p * a.rp + (d - a.kp) : lat + p * a.kp);
-            reg[i] = d < ld ? v : u32x4{0, 0, 0, 0};
+        for (int i = 0; i < 4; ++i) {
+            const int p = min(kt + srow + 16 * i, hi - 1);
+#pragma unroll
+            for (int j = 0; j < CI; ++j) reg[i][j] = *reinterpret_cast<const u32x4*>(src[j] + (int64_t)p * step[j]);
         }
+    };
+    auto park = [&]() {
+        if (!all_there) {  // columns past the row are zeros
+#pragma unroll
+            for (int j = 0; j < CI; ++j)
+                if (8 * (l16 + 16 * j) >= ld) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) reg[i][j] = u32x4{0, 0, 0, 0};
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < CI; ++j)
+                if (16 * j + 15 < CPR || l16 + 16 * j < CPR) *reinterpret_cast<u32x4*>(&sk[srow + 16 * i][8 * (l16 + 16 * j)]) = reg[i][j];
     };
     if (lo < hi) fetch(lo);
     bf16x8 qf[RG][KS];
@@ -347,10 +374,11 @@ __global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
         my_pos[g] = pos0 + row / a.H;
         const bf16* qp = static_cast<const bf16*>(a.qa) + ((int64_t)b * n_rows + row) * ld;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int d = 32 * ks + 8 * q4;
-            const u32x4 v = *reinterpret_cast<const u32x4*>(qp + (d < ld ? d : 0));
-            qf[g][ks] = __builtin_bit_cast(bf16x8, d < ld ? v : u32x4{0, 0, 0, 0});
+        for (int ks = 0; ks < KS; ++ks) qf[g][ks] = *reinterpret_cast<const bf16x8*>(qp + min(32 * ks + 8 * q4, ld - 8));
+        if (!all_there) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                if (32 * ks + 8 * q4 >= ld) qf[g][ks] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
         }
     }
     f32x4 o[RG][NTW], osum[RG];
@@ -369,11 +397,7 @@ __global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
     const int n_tiles = (a.kp + 15) / 16;
 
     for (int kt = lo; kt < hi; kt += kLsKeys) {
-#pragma unroll
-        for (int i = 0; i < NKC; ++i) {
-            const int c = threadIdx.x + 256 * i;
-            *reinterpret_cast<u32x4*>(&sk[c / CPR][(c % CPR) * 8]) = reg[i];
-        }
+        park();
         __syncthreads();
         if (kt + kLsKeys < hi) fetch(kt + kLsKeys);
         f32x4 sc[RG];
@@ -411,6 +435,7 @@ __global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
             *reinterpret_cast<u32x2*>(&sp[r][16 * wave + 4 * q4]) = *reinterpret_cast<const u32x2*>(w);
             const float corr = __builtin_amdgcn_exp2f(ref[g] - m);  // 0 while nothing has been seen
             ref[g] = top;
+            if (kt == lo) continue;  // nothing to rescale
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const float cv = __shfl(corr, 4 * q4 + v, 64);
@@ -453,10 +478,13 @@ __global__ __launch_bounds__(256) void latent_step_kernel(LatentArgs a) {
             const float m = __shfl(ref[g], 4 * q4 + v, 64);
             if (row >= n_rows) continue;
             float* out = a.part + (((int64_t)b * n_rows + row) * a.splits + blockIdx.x) * (a.kp + 4);
+            if (a.kp == 64 * NTW) {
 #pragma unroll
-            for (int n = 0; n < NTW; ++n) {
-                const int col = 16 * (wave + 4 * n) + l16;
-                if (col < a.kp) out[col] = o[g][n][v];
+                for (int n = 0; n < NTW; ++n) out[16 * (wave + 4 * n) + l16] = o[g][n][v];
+            } else {
+#pragma unroll
+                for (int n = 0; n < NTW; ++n)
+                    if (16 * (wave + 4 * n) + l16 < a.kp) out[16 * (wave + 4 * n) + l16] = o[g][n][v];
             }
             if (wave == 0 && l16 == 0) {
                 out[a.kp] = m == -INFINITY ? m : m * 0.69314718055994531f;  // natural units
@@ -765,8 +793,8 @@ template <typename T, typename Z, int RB>
 static int run_absorbed(LatentArgs a, hipStream_t s) {
     // weight rows per workgroup: 16 for one or two token rows (latency), more for more
     a.per_wg = a.M <= 2 ? 1 : a.M <= 64 ? 2 : 4;
-    const int rows = 16 * a.per_wg, blocks = (a.M + RB - 1) / RB;
-    a.rows_out = (a.kp + rows - 1) / rows;
+    const int blocks = (a.M + RB - 1) / RB;
+    a.rows_out = (a.kp + 16 * a.per_wg - 1) / (16 * a.per_wg);
     absorb_kernel<T, Z, RB><<<dim3(a.H * a.rows_out + (a.append ? 1 : 0), blocks), dim3(256), (size_t)RB * a.np * sizeof(T), s>>>(a);
     if (const int rc = raven_host::check_launch("latent_attention (absorb)")) return rc;
     const int pieces = (a.kp / Chunk<T>::N + 63) / 64;
@@ -776,6 +804,8 @@ static int run_absorbed(LatentArgs a, hipStream_t s) {
     else if (pieces <= 2) rc = launch_rows_attention<T, 2>(a, s);
     else rc = launch_rows_attention<T, 4>(a, s);
     if (rc) return rc;
+    if (a.per_wg == 2) a.per_wg = 1;  // (its rows are four times as long: 20 rows 8.8 us with 32 weight rows, 8.0 with 16; the launch above 6.7 / 7.8)
+    const int rows = 16 * a.per_wg;
     a.rows_out = (a.vp + rows - 1) / rows;
     latent_out_kernel<T, Z, RB><<<dim3(a.H * a.rows_out, blocks), dim3(256), (size_t)RB * a.kp * sizeof(T), s>>>(a);
     return raven_host::check_launch("latent_attention (out)");
