@@ -334,6 +334,32 @@ def test_delta_rule_forms_its_decay_logits(pkg, dtype, rank):
                            decay_bias=w0.cuda())
 
 
+@DT
+@pytest.mark.parametrize("rank", [8, 64, 72, 256])
+@pytest.mark.parametrize("d", [24, 64, 88, 128, 192, 256])
+def test_delta_steps_with_a_state_off_sixteen_bytes(pkg, dtype, d, rank):
+    """The step kernel moves the state two or four values at a time where it starts on 16 bytes and one by one elsewhere, and the decay's weight rows 64 at a
+    time, the last ones cut short: same bits either way, over several steps from an empty, NaN-filled state; sequences side by side keep apart."""
+    B, H, eps = 2, 3, 1e-5
+    g = torch.Generator(device="cuda").manual_seed(d + rank)
+    n = H * d
+    wd, bias = (torch.randn(n, rank, generator=g, device="cuda") * 0.3).to(dtype), torch.randn(n, generator=g, device="cuda")
+    ab, nm = torch.randn(n, generator=g, device="cuda"), torch.rand(n, generator=g, device="cuda") + 0.5
+    zs = [torch.randn(B * s, 5 * n + rank, generator=g, device="cuda") for s in (1, 1, 3)]
+    outs = []
+    for off in (0, 1, 2):
+        flat = torch.full((B * H * d * d + 4,), float("nan"), device="cuda")
+        S = flat[off:off + B * H * d * d].view(B, H, d, d)
+        ys, pos = [], 0
+        for z in zs:
+            s = z.shape[0] // B
+            ys.append(pkg.hip.delta_rule(z, None, ab, nm, S, B, s, pos, d, eps, dtype, w_decay=wd, decay_bias=bias))
+            pos += s
+        assert flat[:off].isnan().all() and flat[off + B * H * d * d:].isnan().all()
+        outs.append(ys + [S.clone()])
+    assert outs[0][-1].isfinite().all() and all(torch.equal(a, b) for o in outs[1:] for a, b in zip(o, outs[0]))
+
+
 def test_delta_rule_long_sequences(pkg):
     """Far more tokens than a chunk: what the first tokens left must survive slow decays."""
     T, H, d, eps = 1500, 1, 64, 1e-5
