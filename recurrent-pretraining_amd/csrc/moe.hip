@@ -59,24 +59,28 @@ __device__ __forceinline__ int ordered_key(float v) {
 // through the lane-to-lane broadcast: 64 steps without a dependence, where `top` maxima over the wave, twelve exchanges each, took 3 us
 // of every launch that picks six (moe_up_kernel at one row 14.7 -> 12 us, routing of 20 rows 11.8 -> 8).  One or two are found sooner by
 // maxima (both launches of 8 rows of width 512, one of 8 experts of 512: 12.0 us, by counting 13.4).
+// (U steps unrolled.  In a workgroup alone on its CU all 64 are 2.5 KB of code run once out of a cold instruction cache: routing of 20 rows 9.7 us, with 16
+// 8.8; where thousands of workgroups run it, all: one row of 7 x 384 channels of width 1024, both launches 9.6, with 16 10.1.)
+__device__ __forceinline__ bool picks_by_place(int experts, int top) { return experts <= 64 && top > 2; }
+template <int U>
+__device__ __forceinline__ void pick_by_place(float v, int experts, int& mine, float& score) {  // v: expert `lane`'s logit
+    const int lane = threadIdx.x & 63;
+    const int key = lane < experts ? ordered_key(v) : (int)0x80000000;
+    int before = 0;
+#pragma unroll U
+    for (int j = 0; j < 64; ++j) {
+        const int other = __builtin_amdgcn_readlane(key, j);
+        before += other > key || (other == key && j < lane) ? 1 : 0;
+    }
+    // every lane has a place of its own (absent experts the last ones): lane l sends its number there
+    mine = __builtin_amdgcn_ds_permute(before * 4, lane);
+    const float s = __builtin_bit_cast(float, __builtin_amdgcn_ds_permute(before * 4, __builtin_bit_cast(int, v == v ? v : -INFINITY)));
+    mine = min(mine, experts - 1);
+    score = sigmoid_f32(s);
+}
 __device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
     const int lane = threadIdx.x & 63;
-    if (experts <= 64 && top > 2) {
-        const float v = lane < experts ? logits[lane] : 0.f;
-        const int key = lane < experts ? ordered_key(v) : (int)0x80000000;
-        int before = 0;
-#pragma unroll
-        for (int j = 0; j < 64; ++j) {
-            const int other = __builtin_amdgcn_readlane(key, j);
-            before += other > key || (other == key && j < lane) ? 1 : 0;
-        }
-        // every lane has a place of its own (absent experts the last ones): lane l sends its number there
-        mine = __builtin_amdgcn_ds_permute(before * 4, lane);
-        const float s = __builtin_bit_cast(float, __builtin_amdgcn_ds_permute(before * 4, __builtin_bit_cast(int, v == v ? v : -INFINITY)));
-        mine = min(mine, experts - 1);
-        score = sigmoid_f32(s);
-        return;
-    }
+    if (picks_by_place(experts, top)) return pick_by_place<64>(lane < experts ? logits[lane] : 0.f, experts, mine, score);
     float v[kMaxExperts / 64];
 #pragma unroll
     for (int j = 0; j < kMaxExperts / 64; ++j) {
@@ -309,14 +313,30 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, pairs = a.M * a.top;
     count[tid] = 0;
     __syncthreads();
-    for (int m = wave; m < a.M; m += 16) {
-        int e;
-        float s;
-        pick_experts(a.logits + (int64_t)m * a.ldl, a.experts, a.top, e, s);
+    auto keep = [&](int m, int e, float s) {
         if (lane < a.top) {
             pick[m * a.top + lane] = e;
             scale[m * a.top + lane] = s;
             atomicAdd(&count[e], 1);
+        }
+    };
+    if (picks_by_place(a.experts, a.top)) {  // a wave's next row is requested before the one at hand is sorted (20 rows 8.8 -> 8.2 us)
+        auto logit = [&](int m) { return a.logits[(int64_t)min(m, a.M - 1) * a.ldl + min(lane, a.experts - 1)]; };
+        float next = logit(wave);
+        for (int m = wave; m < a.M; m += 16) {
+            const float v = lane < a.experts ? next : 0.f;
+            next = logit(m + 16);
+            int e;
+            float s;
+            pick_by_place<16>(v, a.experts, e, s);
+            keep(m, e, s);
+        }
+    } else {
+        for (int m = wave; m < a.M; m += 16) {
+            int e;
+            float s;
+            pick_experts(a.logits + (int64_t)m * a.ldl, a.experts, a.top, e, s);
+            keep(m, e, s);
         }
     }
     __syncthreads();
