@@ -382,6 +382,28 @@ def test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, same):
     assert ((outs[0].double() - x.double() - want).norm() / want.norm()).item() < 5e-3
 
 
+@DT
+@pytest.mark.parametrize("W,blocks,taps", [(2048, 8, 4), (1032, 3, 4), (1320, 5, 3), (768, 1, 5)])
+def test_recurrent_step_of_several_sequences(pkg, dtype, W, blocks, taps):
+    """Steps of 3 and more sequences share a workgroup's weight rows four at a time, the last group cut short: the same bits as each sequence alone, from an
+    empty, NaN-filled state and ring on until the ring has wrapped."""
+    bl = W // blocks
+    g = torch.Generator(device="cuda").manual_seed(W + taps)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    conv, cb, gb, sp = rand(taps, W), rand(W), rand(2, W), rand(W).abs()
+    gates = (rand(blocks, 2, bl, bl) * bl ** -0.5).to(dtype)
+    desc = pkg.hip.Rglru(conv.data_ptr(), cb.data_ptr(), gates.data_ptr(), gb.data_ptr(), sp.data_ptr(), blocks, bl, taps, W)
+    for B in (3, 4, 9):
+        fresh = lambda n: (torch.full((n, taps, W), float("nan"), device="cuda"), torch.full((n, W), float("nan"), device="cuda"))
+        together, alone = fresh(B), [fresh(1) for _ in range(B)]
+        for pos in range(taps + 2):
+            z = rand(B, 2 * W).to(dtype)
+            y = pkg.hip.rglru(desc, z, *together, B, 1, pos)
+            for b, (ring, state) in enumerate(alone):
+                assert torch.equal(pkg.hip.rglru(desc, z[b:b + 1].contiguous(), ring, state, 1, 1, pos)[0], y[b]) and y[b].isfinite().all()
+                assert torch.equal(state[0], together[1][b])
+
+
 @pytest.mark.parametrize("M,D,E,top,ff,shared", [(130, 200, 160, 2, 40, False), (100, 2056, 64, 6, 760, True), (6, 1160, 64, 8, 520, True), (33, 1288, 40, 8, 1032, False)])
 def test_mixture_of_low_tiles(pkg, M, D, E, top, ff, shared):
     """expert_rows_kernel: fewer columns than one K step, steps and 16-column tiles that end early, tiles with rows for one load and for more, as a chunk
