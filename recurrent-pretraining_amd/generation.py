@@ -189,7 +189,8 @@ class MinimalGeneration:
 
 class GraphedStep:
     """A decode step whose launches are the same for every token (the position is read from `self.pos` on the device): eager the
-    first time, then captured once per `key` and replayed.  Subclasses implement _enqueue(hint)."""
+    first time, then captured once per `key` and replayed.  Subclasses implement _enqueue(hint), which only reads the position: launch()
+    writes it before every step (a kernel that advanced it as well cost 4 us of each step and was overwritten)."""
 
     def __init__(self, use_graph: bool, device):
         self.pos = torch.zeros(1, dtype=torch.int32, device=device)

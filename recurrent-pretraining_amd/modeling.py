@@ -932,7 +932,6 @@ class DecodeRunner(GraphedStep):
                                    cfg.padded_vocab_size, cfg.n_embd, hip.dtype_code(m.dtype), 1, hip._stream())
         hip._check(rc, "raven_gemm")
         hip.argmax(self.logits, out=self.next_ids)
-        hip.advance_pos(self.pos, 1)
 
     def step(self, ids: torch.Tensor, state: Optional[torch.Tensor], init_scale: float = 1.0):
         """Feeds one token per sequence; returns (logits [B,V] f32, next ids [B], latents [B,h]).

@@ -332,7 +332,6 @@ class MixerDecodeRunner(GraphedStep):
         x = m._stream(self.ids, self.buf, self.cache, self.B, 1, hint, pos_dev=self.pos)
         m._logits(x, self.h, self.logits, self.buf["ws"])
         hip.argmax(self.logits, out=self.next_ids)
-        hip.advance_pos(self.pos, 1)
 
     def _position_bound(self, pos0: int) -> int:
         """The by-value position that sizes a step's grids: the next power of two, so that a capture lasts until the sequence has
