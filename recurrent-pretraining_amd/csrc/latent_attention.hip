@@ -60,13 +60,14 @@ __device__ __forceinline__ void append_row(const LatentArgs& a, int m) {
     }
 }
 
-// a wave per row: the normed query latent and the cache entry
+// The rows' normed query latents and cache entries, a wave per row; with two blocks in y one wave for each of the two results, as a few rows are bound by the
+// latency of a wave's loads and sums
 template <typename T, typename Z>
 __global__ __launch_bounds__(256) void latent_rows_kernel(LatentArgs a) {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (m >= a.M) return;
-    if (a.cq) wave_norm<T, Z>(static_cast<const Z*>(a.z) + (int64_t)m * a.ldz, a.q_norm, static_cast<T*>(a.cq) + (int64_t)m * a.qp, a.qp, a.qd, a.eps);
-    if (a.append) append_row<T, Z>(a, m);
+    if (a.cq && blockIdx.y == 0) wave_norm<T, Z>(static_cast<const Z*>(a.z) + (int64_t)m * a.ldz, a.q_norm, static_cast<T*>(a.cq) + (int64_t)m * a.qp, a.qp, a.qd, a.eps);
+    if (a.append && blockIdx.y + 1 == gridDim.y) append_row<T, Z>(a, m);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -858,7 +859,8 @@ extern "C" int raven_latent_rows(const raven_latent* l, const void* z, int32_t l
     a.append = l->own_kv;
     if (!a.cq && !a.append) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid((a.M + 3) / 4);
+    // us, both results by one wave / by two, ranks 768 and 512, bf16: 1 row 3.4 / 2.6, 20: 3.9 / 2.9, 500: 4.2 / 3.2, 4096: 7.0 / 6.5, 16384 (bound by memory): 18.3 / 19.3
+    const dim3 grid((a.M + 3) / 4, a.cq && a.append && a.M <= 4096 ? 2 : 1);
     if (dtype == RAVEN_F32) latent_rows_kernel<float, float><<<grid, dim3(256), 0, s>>>(a);
     else if (z_f32) latent_rows_kernel<bf16, float><<<grid, dim3(256), 0, s>>>(a);
     else latent_rows_kernel<bf16, bf16><<<grid, dim3(256), 0, s>>>(a);

@@ -383,6 +383,27 @@ def test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, same):
 
 
 @DT
+@pytest.mark.parametrize("B,S", [(1, 1), (3, 3), (1, 4096), (1, 4097)])
+def test_latent_rows_give_both_results_as_each_alone(pkg, dtype, B, S):
+    """Up to 4096 rows a wave of its own takes each of a row's two results, beyond one wave takes both: the same bits as a call for one of them."""
+    qr, kr, rot, t_max = 136, 72, 16, S + 5
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    qn, kn, angles, z = rand(qr), rand(kr), rand(t_max, rot), rand(B * S, qr + kr + rot + 2 * 32).to(dtype)
+
+    def call(own, want_cq):
+        desc = pkg.hip.Latent(None, None, None, qn.data_ptr(), kn.data_ptr(), 0.1, 1e-6, 2, qr, qr, kr, kr, 32, rot, 32, 0, own)
+        latent, rotated = torch.zeros(B, t_max, kr, device="cuda", dtype=dtype), torch.zeros(B, t_max, rot, device="cuda", dtype=dtype)
+        cache = pkg.hip.LatentCache(latent.data_ptr(), rotated.data_ptr(), angles.data_ptr(), B, t_max)
+        return pkg.hip.latent_rows(desc, z, cache, B, S, 2, dtype, want_cq=want_cq), latent, rotated
+
+    cq, latent, rotated = call(1, True)
+    assert torch.equal(cq, call(0, True)[0])
+    _, l1, r1 = call(1, False)
+    assert torch.equal(latent, l1) and torch.equal(rotated, r1) and latent[:, 2:S + 2].float().abs().sum(-1).gt(0).all() and not latent[:, :2].any()
+
+
+@DT
 @pytest.mark.parametrize("W,blocks,taps", [(2048, 8, 4), (1032, 3, 4), (1320, 5, 3), (768, 1, 5)])
 def test_recurrent_step_of_several_sequences(pkg, dtype, W, blocks, taps):
     """Steps of 3 and more sequences share a workgroup's weight rows four at a time, the last group cut short: the same bits as each sequence alone, from an
