@@ -59,13 +59,14 @@ constexpr int kPfTable = 1024;  // block-table entries of a sequence held in LDS
 // positions at a time with the next 64 requested before this tile's are used; float weights, the 16 groups' sums merged through LDS (`merge`, 16 * (HD + 2)
 // floats).  Bound by the cache's bytes and the two workgroups that a CU holds: 15 sequences of 420 positions, 55 heads of 96, 27 to 29 us = 4.6 to 4.9 TB/s
 // (the decode kernel over the same pages 28.5); as one of a tile's 16 query rows, three waves of four without a row and a wait for every staged tile,
-// 40.  off_of: element offset of a position's head row.
+// 40.  off_of: element offset of a position's head row.  What is loaded without being part of the row or of the cache is selected away, not multiplied by
+// zero: infinities stay where they are.
 template <int HD, typename OFF>
 __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, const bf16* K, const bf16* V, int n_keys, float scale_log2, float* merge, OFF off_of) {
     constexpr int U = 4, G = 16, NC = HD / 8;
     const int lane = threadIdx.x & 63, ci = lane & 15, group = (threadIdx.x >> 6) * 4 + (lane >> 4);
-    const int at = min(ci, NC - 1) * 8;  // lanes past the row repeat its last chunk against a zero query
-    const Chunk<bf16> qc = ci < NC ? load_chunk(q + at) : zero_chunk<bf16>();
+    const int at = min(ci, NC - 1) * 8;  // lanes past the row repeat its last chunk
+    const Chunk<bf16> qc = load_chunk(q + at);
     float m_run = -INFINITY, l_run = 0.f, o[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = 0.f;
@@ -82,7 +83,9 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
         float sc[U], top = m_run;
 #pragma unroll
         for (int j = 0; j < U; ++j) {
-            sc[j] = row16_sum(dot_chunk(qc, k[s][j], 0.f)) * scale_log2;
+            float d = dot_chunk(qc, k[s][j], 0.f);
+            if (NC < 16 && ci >= NC) d = 0.f;
+            sc[j] = row16_sum(d) * scale_log2;
             if (base + G * j + group >= n_keys) sc[j] = -INFINITY;
             top = fmaxf(top, sc[j]);
         }
@@ -94,9 +97,10 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
 #pragma unroll
         for (int j = 0; j < U; ++j) {
             const float w = __builtin_amdgcn_exp2f(sc[j] - ref);
+            const Chunk<bf16> vc = base + G * j + group < n_keys ? v[s][j] : zero_chunk<bf16>();
             l_run += w;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(w, to_f32(v[s][j].v[e]), o[e]);
+            for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(w, to_f32(vc.v[e]), o[e]);
         }
         m_run = top;
     };

@@ -1077,3 +1077,27 @@ def _check_paged_rows(pkg, nh, hd, block_size, layout, dt, lens, rows):
         hidden = torch.arange(n)[None] > torch.arange(n - r, n)[:, None]
         want = (torch.softmax(s.masked_fill(hidden.cuda(), -math.inf), -1) @ vals).transpose(0, 1).reshape(r, -1)
         check(y[at], want.float().to(dt), dt, f"{r} rows of {n} positions", ulps=1 if r == 1 else 2)
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("n", [64, 100, 128, 200])
+def test_infinities_in_a_single_row_of_paged_attention(pkg, hd, n):
+    """A sequence's only row: a key whose last channels make its score -Inf drops out of the softmax, an infinity in the last position's values stays in its
+    own column; what the kernel loads beyond a row or the last position multiplies nothing.  Against 64 bits, elsewhere one rounding."""
+    dt, nh, bs = torch.bfloat16, 2, 16
+    k, v = rnd((n, nh, hd), dt, 920), rnd((n, nh, hd), dt, 921)
+    q = rnd((1, nh * hd), dt, 922, 2.0)
+    q.view(nh, hd)[:, -1] = 1.5
+    for p in (0, 40, n - 2):
+        k[p, :, -1] = -math.inf
+    v[n - 1, 0, 3] = math.inf
+    pages = (n + bs - 1) // bs
+    kc, vc = (torch.zeros(pages * bs, nh, hd, dtype=dt).index_copy_(0, torch.arange(n), t).view(pages, bs, nh, hd).cuda() for t in (k, v))
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32).cuda()
+    y = pkg.hip.paged_prefill_attention(q.cuda(), kc, vc, torch.arange(pages, dtype=torch.int32).view(1, -1).cuda(), i32(n), i32(0, 1), 1).cpu().view(nh, hd)
+    s = torch.einsum("hd,thd->ht", q.view(nh, hd).double(), k.double()) * hd ** -0.5
+    want = torch.einsum("ht,thd->hd", torch.softmax(s, -1), v.double())
+    want[0, 3] = math.inf
+    assert y[0, 3] == math.inf
+    y[0, 3] = want[0, 3] = 0.0
+    check(y, want.float().to(dt), dt, "single row beside infinities")
