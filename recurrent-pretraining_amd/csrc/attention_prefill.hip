@@ -53,7 +53,9 @@ struct PrefillArgs {
     int64_t page_stride, pos_stride, head_stride;  // elements between two pages / positions of a page / heads
 };
 
-constexpr int kPfTable = 1024;  // block-table entries of a sequence held in LDS (beyond that they are read from memory)
+constexpr int kPfTable = 1024;   // block-table entries of a sequence held in LDS (beyond that they are read from memory)
+constexpr int kRowTable = 8192;  // the same where a sequence has a single row, whose staging buffers are free
+constexpr int kFloatPages = 1 << 20;  // positions whose page a multiplication in float gives exactly
 
 // The only new row of a paged sequence: a decode row in a scheduler step that also carries a prompt chunk.  Four waves, 16 lanes to a cached position, 64
 // positions at a time with the next 64 requested before this tile's are used; float weights, the 16 groups' sums merged through LDS (`merge`, 16 * (HD + 2)
@@ -106,11 +108,19 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
     };
     constexpr int T = G * U;
     request(0, 0);
-    for (int base = 0; base < n_keys; base += 2 * T) {  // a request past the end repeats the last position
+    int base = 0;
+    for (; base + 2 * T < n_keys; base += 2 * T) {
         request(base + T, 1);
         use(base, 0);
         request(base + 2 * T, 0);
         use(base + T, 1);
+    }
+    if (base + T < n_keys) {  // one or two tiles are left; nothing is requested past them
+        request(base + T, 1);
+        use(base, 0);
+        use(base + T, 1);
+    } else {
+        use(base, 0);
     }
     if (ci < NC) {
 #pragma unroll
@@ -135,10 +145,6 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
     }
 }
 
-// PAGES: 0 = a contiguous cache; 1 = block-paged, sequences of at most kPfTable pages and 2^20 positions, whose table entries all lie in LDS; 2 = block-paged,
-// longer tables: entries past kPfTable come from memory.  (That choice and the one between a shift and a division are branches around every position's loads,
-// which then are no longer in flight together: two rows each of 15 sequences of 420 positions and a chunk of 180 rows of 55 heads of 96 took 63 us with them,
-// 50 without.)
 // Which block of query rows a workgroup of a paged launch takes: the blocks of `rows` rows that the B sequences have, counted through their row starts and
 // handed out from the last one on -- schedulers put prompt chunks behind decode rows, and a sequence's last block has the most keys.  (A grid of the longest
 // sequence's blocks for every sequence starts workgroups without rows: 825 of them beside the 15 sequences and 180-row chunk above took 12 us.)
@@ -177,6 +183,10 @@ __device__ __forceinline__ bool paged_block(const PrefillArgs& a, int rows, int*
     }
 }
 
+// PAGES: 0 = a contiguous cache; 1 = block-paged, sequences of at most kPfTable pages and 2^20 positions, whose table entries all lie in LDS; 2 = block-paged,
+// longer tables: entries past kPfTable come from memory.  (That choice and the one between a shift and a division are branches around every position's loads,
+// which then are no longer in flight together: two rows each of 15 sequences of 420 positions and a chunk of 180 rows of 55 heads of 96 took 63 us with them,
+// 50 without.)
 template <int HD, int RG, int PAGES = 0, int NW = 4>
 __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_kernel(PrefillArgs a) {
     constexpr bool PAGED = PAGES != 0;
@@ -230,24 +240,29 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     const bf16* Kb = a.k + head_off;
     const bf16* Vb = a.v + head_off;
 
-    // the page of position p: without a branch in a tile's loads.  (p + 1/2) / block_size in float is off by less than 2^-22 of itself, so that its whole
-    // part is right for positions below 2^20
+    // the page of position p without a branch in a tile's loads: (p + 1/2) / block_size in float is off by less than 2^-22 of itself, so that its whole
+    // part is right for positions below kFloatPages
+    auto float_page = [&](int p) { return (int)(((float)p + 0.5f) * a.per_block); };
     auto page_of = [&](int p) {
-        if (PAGES == 1) return (int)(((float)p + 0.5f) * a.per_block);
+        if (PAGES == 1) return float_page(p);
         return a.block_shift >= 0 ? p >> a.block_shift : p / a.block_size;
     };
     if constexpr (PAGED) {
-        if (n_rows == 1) {
-            const int n_pages = (t_lim + a.block_size - 1) / a.block_size;
-            for (int i = threadIdx.x; i < min(n_pages, kPfTable); i += NTH) tbl[i] = table_row[i];
+        // a single row has its whole table in LDS, however wide the table is.  us with the entries past kPfTable behind a branch in every position's loads / as
+        // rows of a tile / now: 30000 positions of 55 heads of 96 1000 / 482 / 292, 15 sequences of 420 in a table of 2000 entries, 12 heads of 64,
+        // 23 / 15 / 10
+        constexpr int kMerge = 16 * (HD + 2);
+        static_assert(NW == 4 && (SK_ELEMS + SV_ELEMS) * sizeof(bf16) >= (kMerge + kRowTable) * sizeof(float), "sixteen groups, room to merge them and the table");
+        const int n_pages = (t_lim + a.block_size - 1) / a.block_size;
+        if (n_rows == 1 && n_pages <= kRowTable && t_lim <= kFloatPages) {
+            float* merge = reinterpret_cast<float*>(smem_kv);
+            int* row_tbl = reinterpret_cast<int*>(merge + kMerge);
+            for (int i = threadIdx.x; i < n_pages; i += NTH) row_tbl[i] = table_row[i];
             __syncthreads();
-            static_assert(NW == 4 && (SK_ELEMS + SV_ELEMS) * sizeof(bf16) >= 16 * (HD + 2) * sizeof(float), "sixteen groups, room to merge them");
-            single_row_attention<HD>(a.q + q_row0 * h + head * HD, a.y + q_row0 * a.ldy + head * HD, Kb, Vb, t_lim, a.scale_log2, reinterpret_cast<float*>(smem_kv),
-                                     [&](int p) {
-                                         const int pg = page_of(p);
-                                         const int page = PAGES == 1 || pg < kPfTable ? tbl[pg] : table_row[pg];
-                                         return (int64_t)page * a.page_stride + (int64_t)((p - pg * a.block_size) * (int)a.pos_stride);
-                                     });
+            single_row_attention<HD>(a.q + q_row0 * h + head * HD, a.y + q_row0 * a.ldy + head * HD, Kb, Vb, t_lim, a.scale_log2, merge, [&](int p) {
+                const int pg = float_page(p);
+                return (int64_t)row_tbl[pg] * a.page_stride + (int64_t)((p - pg * a.block_size) * (int)a.pos_stride);
+            });
             return;
         }
     }
@@ -324,7 +339,7 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
                 const int mask = a.block_size - 1;
                 auto off = [&](int p) {
                     const int pg = p >> a.block_shift;
-                    const int page = PAGES == 1 || pg < kPfTable ? tbl[pg] : table_row[pg];
+                    const int page = pg < kPfTable ? tbl[pg] : table_row[pg];
                     return (int64_t)page * a.page_stride + (int64_t)((p & mask) * (int)a.pos_stride);
                 };
 #pragma unroll
@@ -641,7 +656,7 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
     a.block_table = block_table; a.seq_lens = seq_lens; a.q_start = q_start; a.B = B;
     a.max_blocks = max_blocks; a.block_size = block_size; a.block_shift = -1;
     a.per_block = 1.0f / (float)block_size;
-    const bool short_tables = max_blocks <= kPfTable && (int64_t)max_blocks * block_size <= (1 << 20);
+    const bool short_tables = max_blocks <= kPfTable && (int64_t)max_blocks * block_size <= kFloatPages;
     for (int sh = 0; sh < 31; ++sh)
         if (block_size == (1 << sh)) a.block_shift = sh;
     RAVEN_REQUIRE((int64_t)block_size * n_heads * head_dim < (1ll << 31), "paged_prefill_attention: a page of %d positions is too large", block_size);

@@ -1101,3 +1101,26 @@ def test_infinities_in_a_single_row_of_paged_attention(pkg, hd, n):
     assert y[0, 3] == math.inf
     y[0, 3] = want[0, 3] = 0.0
     check(y, want.float().to(dt), dt, "single row beside infinities")
+
+
+@pytest.mark.parametrize("block_size,n", [(1, 8192), (1, 8193), (129, 1 << 20), (256, (1 << 20) + 3), (12, 13000)])
+def test_a_single_row_of_a_long_paged_sequence(pkg, block_size, n):
+    """Up to 8192 pages and 2^20 positions a sequence's only row has its table in LDS and finds a position's page by a float product, beyond both it goes the
+    chunks' way: each query is aligned with one key far above the others, so that its output is that position's value to the bit."""
+    dt, nh, hd = torch.bfloat16, 1, 64
+    pages = (n + block_size - 1) // block_size
+    table = torch.randperm(pages, generator=torch.Generator().manual_seed(n)).to(torch.int32)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    k, v = (torch.randn(pages, block_size, nh, hd, device="cuda", generator=g).to(dt) for _ in "kv")
+    # the last positions of pages and the first ones, where a wrong page shows
+    spots = sorted({p for page in (0, 1, 2, pages // 2, 1023, 1024, pages - 1) for p in (page * block_size, min(page * block_size + block_size, n) - 1) if p < n})
+    B = len(spots)
+    q = torch.randn(B, hd, device="cuda", generator=g).to(dt)
+    places = [(int(table[p // block_size]), p % block_size) for p in spots]
+    for i, (pg, o) in enumerate(places):
+        q[i] = torch.sign(q[i].float()).to(dt) * 16
+        k[pg, o, 0] = torch.sign(q[i].float()).to(dt) * 16  # score 16 * 16 * 64 / 8; another's spot: no more than half of it
+    for layout, turn in ((pkg.hip.PAGED_NHD, lambda t: t), (pkg.hip.PAGED_HND, lambda t: t.transpose(1, 2).contiguous())):
+        y = pkg.hip.paged_prefill_attention(q, turn(k), turn(v), table.expand(B, -1).contiguous().cuda(), torch.full((B,), n, dtype=torch.int32).cuda(),
+                                            torch.arange(B + 1, dtype=torch.int32).cuda(), 1, layout=layout)
+        assert torch.equal(y, torch.stack([v[pg, o, 0] for pg, o in places]))
