@@ -24,6 +24,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "raven_common.h"
@@ -48,6 +49,8 @@ struct PrefillArgs {
     const int* seq_lens;     // [B]
     const int* q_start;      // [B + 1]
     int B;
+    int blocks, extra;       // blocks of query rows that have workgroups, the first `extra` of them behind the sequences' first ones; extra negative: blocks / B
+                             // for every sequence
     int max_blocks, block_size, block_shift;  // block_shift = log2(block_size), or -1 when that is not a power of two
     float per_block;                          // 1 / block_size
     int64_t page_stride, pos_stride, head_stride;  // elements between two pages / positions of a page / heads
@@ -145,42 +148,58 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
     }
 }
 
-// Which block of query rows a workgroup of a paged launch takes: the blocks of `rows` rows that the B sequences have, counted through their row starts and
-// handed out from the last one on -- schedulers put prompt chunks behind decode rows, and a sequence's last block has the most keys.  (A grid of the longest
-// sequence's blocks for every sequence starts workgroups without rows: 825 of them beside the 15 sequences and 180-row chunk above took 12 us.)
+// Which block of `rows` query rows a workgroup of a paged launch takes (its heads start side by side, x, so that long blocks start before short ones).  Every
+// sequence's first block has a workgroup of its own, found without a look at the other sequences: decode rows, most of what a scheduler step holds, have
+// no other.  Only the a.extra workgroups in front -- the blocks behind the first ones, at most T / rows of them, each with a whole block of rows
+// before it -- count through the sequences' row starts, 256 sequences a turn, from the last one on: schedulers put prompt chunks behind decode rows, and a
+// sequence's last block has the most keys.  False: none.  us with a count by every workgroup of all sequences, twice / now: single rows of 100 positions, 512
+// sequences of 8 heads of 128 89 / 44, 55 of 96 553 / 240, 1000 of 12 of 64 272 / 82; 15 of 420 positions beside a chunk of 1500 rows, 55 of 96, 88 / 74 --
+// 157 with the longest sequence's blocks for every sequence, in their order.
 __device__ __forceinline__ bool paged_block(const PrefillArgs& a, int rows, int* seq, int* block) {
-    const int lane = threadIdx.x & 63;
-    auto blocks_of = [&](int i) {
-        if (i >= a.B) return 0;
-        const int n = a.q_start[i + 1] - a.q_start[i];
-        return n > 0 && n <= a.seq_lens[i] ? (n + rows - 1) / rows : 0;
-    };
-    auto summed = [&](int n) {  // over the lanes up to this one
+    const int x = blockIdx.y + gridDim.y * blockIdx.z, lane = threadIdx.x & 63;
+    if (x >= a.blocks) return false;
+    if (a.extra < 0) {
+        *seq = x % a.B;
+        *block = a.blocks / a.B - 1 - x / a.B;
+        return true;
+    }
+    if (x >= a.extra) {
+        *seq = x - a.extra;
+        *block = 0;
+        return true;
+    }
+    int want = x;
+    for (int i0 = a.B - 1; i0 >= 0; i0 -= 256) {
+        int more[4], upto = 0;  // blocks behind the first of this lane's four sequences
 #pragma unroll
-        for (int d = 1; d < 64; d *= 2) {
-            const int v = __shfl_up(n, d, 64);
-            if (lane >= d) n += v;
+        for (int j = 0; j < 4; ++j) {
+            const int i = max(i0 - 4 * lane - j, 0), n = a.q_start[i + 1] - a.q_start[i];
+            more[j] = n > 0 && n <= a.seq_lens[i] && i0 >= 4 * lane + j ? (n - 1) / rows : 0;
+            upto += more[j];
         }
-        return n;
-    };
-    int mine = blocks_of(lane), upto = summed(mine), total = __shfl(upto, 63, 64);
-    for (int i0 = 64; i0 < a.B; i0 += 64) total += __shfl(summed(blocks_of(i0 + lane)), 63, 64);
-    int want = total - 1 - (int)blockIdx.x;
-    if (want < 0) return false;
-    for (int i0 = 0;; i0 += 64) {
-        if (i0 > 0) {
-            mine = blocks_of(i0 + lane);
-            upto = summed(mine);
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {  // summed over the lanes up to this one
+            const int v = __shfl_up(upto, d, 64);
+            if (lane >= d) upto += v;
         }
         const uint64_t past = __builtin_amdgcn_ballot_w64(upto > want);
         if (past != 0) {
             const int l = __builtin_ctzll(past);
-            *seq = i0 + l;
-            *block = want - __builtin_amdgcn_readlane(upto - mine, l);
-            return true;
+            want -= __builtin_amdgcn_readlane(upto - more[0] - more[1] - more[2] - more[3], l);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int n = __builtin_amdgcn_readlane(more[j], l);
+                if (want < n) {
+                    *seq = i0 - 4 * l - j;
+                    *block = n - want;
+                    return true;
+                }
+                want -= n;
+            }
         }
-        want -= __shfl(upto, 63, 64);
+        want -= __builtin_amdgcn_readlane(upto, 63);
     }
+    return false;
 }
 
 // PAGES: 0 = a contiguous cache; 1 = block-paged, sequences of at most kPfTable pages and 2^20 positions, whose table entries all lie in LDS; 2 = block-paged,
@@ -211,7 +230,7 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     if constexpr (PAGED) {
         if (!paged_block(a, ROWS, &b, &qb)) return;
     }
-    const int head = blockIdx.y;
+    const int head = PAGED ? blockIdx.x : blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qc = lane & 15, s4 = lane >> 4;
     const int h = a.nh * HD;
@@ -226,6 +245,7 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
         n_rows = a.q_start[b + 1] - (int)q_row0;
         t_lim = a.seq_lens[b];
         pos0 = t_lim - n_rows;
+        if (n_rows <= 0 || pos0 < 0 || qb * ROWS >= n_rows) return;
         table_row = a.block_table + (int64_t)b * a.max_blocks;
     } else {
         q_row0 = (int64_t)b * a.S;
@@ -664,14 +684,31 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
     a.pos_stride = kv_layout == RAVEN_PAGED_NHD ? (int64_t)n_heads * head_dim : head_dim;
     a.head_stride = kv_layout == RAVEN_PAGED_NHD ? head_dim : (int64_t)block_size * head_dim;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t wgs128 = (int64_t)((max_q_len + 127) / 128) * n_heads * B;
-    const int rg = wgs128 >= 512 ? 2 : 1;
+    // 64 query rows per workgroup while all such workgroups run at once, two on a CU (three with heads of 64), else 128, which share what is staged -- if any
+    // chunk has that many.  Single rows are short and not counted: what is left of T is rows behind the first of chunks of up to max_q_len.  us by 64 / 128:
+    // one chunk behind 140 positions, 55 heads of 96, 700 rows (605 workgroups of 64) 26 / 26, 180 (165) 10.2 / 12.3, 1500 (1320) 77 / 51; 8 heads of 128, 4000 (504)
+    // 95 / 108; 32 of 128, 1500 (768) 50 / 50, 4000 (2016) 240 / 169; 12 of 64, 4000 (756) 66 / 75; 64 chunks of 64, 55 of 96, 78 / 84
+    const int64_t behind = T < 0 ? (int64_t)(max_q_len - 1) * B : std::max(T - B, 0);
+    const int64_t chunks = behind > 0 ? (behind + max_q_len - 2) / (max_q_len - 1) : 0;
+    const int rg = max_q_len > 64 && chunks * ((max_q_len + 63) / 64) * n_heads > (head_dim == 64 ? 768 : 512) ? 2 : 1;
     const int rows = 64 * rg;
-    // as many blocks as the sequences can have: those of the longest one each, or of T rows in all, each sequence's last one partly filled
-    int64_t blocks = (int64_t)((max_q_len + rows - 1) / rows) * B;
-    if (T >= 0 && T / rows + B < blocks) blocks = T / rows + B;
+    // T rows in all fill less than T / rows blocks besides each sequence's last one.  Counting through the sequences costs more than starting fewer than 128
+    // workgroups that then leave: us with / without, a chunk of 180 rows, 8 heads of 128, alone 11.5 / 10.5, beside 4 decode rows (64 workgroups) 11.6 / 10.5;
+    // beside one, 55 heads of 96 (110), 11.2 / 11.2, beside 4 (440) 14.5 / 15.1
+    const int64_t most = (int64_t)((max_q_len + rows - 1) / rows) * B;
+    int64_t blocks = most;
+    a.extra = -1;
+    if (T >= 0) {
+        const int64_t extra = std::min<int64_t>(T > 0 ? (T - 1) / rows : 0, most - B);
+        if ((most - B - extra) * n_heads >= 128) {
+            a.extra = (int)extra;
+            blocks = B + extra;
+        }
+    }
     RAVEN_REQUIRE(blocks < (1ll << 31), "paged_prefill_attention: grid too large");
-    const dim3 grid((unsigned)blocks, n_heads);
+    a.blocks = (int)blocks;
+    const unsigned by = (unsigned)std::min<int64_t>(blocks, 32768);
+    const dim3 grid(n_heads, by, (a.blocks + by - 1) / by);
 #define RAVEN_PREFILL(HD)                                                                        \
     if (short_tables) {                                                                          \
         if (rg == 2) attention_prefill_kernel<HD, 2, 1><<<grid, dim3(256), 0, s>>>(a);           \

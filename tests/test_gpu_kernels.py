@@ -1124,3 +1124,23 @@ def test_a_single_row_of_a_long_paged_sequence(pkg, block_size, n):
         y = pkg.hip.paged_prefill_attention(q, turn(k), turn(v), table.expand(B, -1).contiguous().cuda(), torch.full((B,), n, dtype=torch.int32).cuda(),
                                             torch.arange(B + 1, dtype=torch.int32).cuda(), 1, layout=layout)
         assert torch.equal(y, torch.stack([v[pg, o, 0] for pg, o in places]))
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("chunks", [2, 40])
+@pytest.mark.parametrize("block_size", [2, 3])
+def test_chunks_of_paged_attention_behind_long_tables(pkg, hd, chunks, block_size):
+    """Chunks of several rows, two and forty of them (64 and 128 rows per workgroup), behind tables that fit the LDS and behind ones of more than 1024 entries,
+    past which lie their last tiles; pages of 2^n positions and of others."""
+    for n in (200, 1024 * block_size + 150):
+        rows = [130 if i % 2 == 0 else 65 + i for i in range(chunks)]
+        _check_paged_rows(pkg, 8, hd, block_size, "HND" if chunks == 2 else "NHD", torch.bfloat16, [n + i for i in range(chunks)], rows)
+
+
+def test_chunks_among_many_paged_sequences(pkg):
+    """Blocks behind a sequence's first one are found by counting 256 sequences a turn: chunks first, last and on both sides of the turns' bounds, sequences
+    without rows between."""
+    lens, rows = [20 + i % 50 for i in range(777)], [1 if i % 7 else 0 for i in range(777)]
+    for i in (0, 8, 264, 265, 520, 521, 700, 776):
+        lens[i], rows[i] = 400 + i, 200 + i % 100
+    _check_paged_rows(pkg, 2, 64, 16, "HND", torch.bfloat16, lens, rows)
