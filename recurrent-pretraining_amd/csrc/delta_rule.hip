@@ -60,13 +60,17 @@ constexpr int kMaxRank = 256;  // of the decay projection, where the kernel form
 __device__ __forceinline__ float delta_decay(float logit) { return expf(-0.60653065971263342f * sigmoid_f32(logit)); }
 
 // RPL rows per lane (16 * RPL >= hd), CP columns per lane group (32 * CP >= hd), moved V at a time (more than 1: the state starts on 16 bytes).
-// A decode step is one pass through memory latencies: every load of the state and of the decay's weight rows is unconditional (what lies outside is
-// selected away), so that all are in flight together.  One row, four
-// at a time and unconditional: 32 heads of 64 over rank 64, 1 sequence 5.3 -> 4.1 us, 20: 12.6 -> 8.5, 40: 20.2 -> 12.5; 16 heads of 128, 20: 40 -> 16.
+// A decode step is one pass through memory latencies: every load of the state and of eight pieces of the decay's weight rows is unconditional (what lies
+// outside is selected away), so that they are in flight together.  us value by value behind conditions, piece by piece / now: 32 heads of 64 over rank 64, bf16,
+// 1 sequence 5.3 / 4.1, 20: 12.6 / 8.5, 40: 20.2 / 12.5; 16 heads of 128, 20: 40 / 16.  Heads of up to 48 have little to load, and what counts is that
+// four workgroups fit a CU's registers: they keep the short way.  32 heads of 32 over rank 32, short way / all together: bf16, 1 sequence 3.6 / 3.65, 20:
+// 4.6 / 6.1, 20 of 4 tokens 5.8 / 7.7; fp32 3.7 / 4.0, 4.7 / 6.7, 6.4 / 9.9.
 template <typename T, int RPL, int CP, int V>
 __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
     constexpr int R = 16 * RPL;       // rows held, the last ones zero
     constexpr int KEEP = (R + 63) / 64;
+    constexpr bool kShort = RPL <= 3;
+    static_assert(!kShort || V == 1, "small heads take their state value by value");
     __shared__ __align__(16) float sw[kDeltaTile][R], su[kDeltaTile][R], sb[kDeltaTile][R], sk[kDeltaTile][R], sr[kDeltaTile][R];
     __shared__ __align__(16) float sv[kDeltaTile][32 * CP], so[kDeltaTile][32 * CP];
     __shared__ __align__(16) float slow[kDeltaTile][kMaxRank];
@@ -84,9 +88,13 @@ __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
 #pragma unroll
         for (int i = 0; i < RPL; i += V) {  // (hd is a multiple of 8: V rows exist together)
             const int col = col0 + 32 * c, r = l16 * RPL + i;
-            const fv s = *reinterpret_cast<const fv*>(state + min(col, hd - 1) * hd + min(r, hd - V));
+            if constexpr (kShort) {
+                S[c][i] = (pos0 > 0 && col < hd && r < hd) ? state[(int64_t)col * hd + r] : 0.f;  // a sequence starts from zero
+            } else {
+                const fv s = *reinterpret_cast<const fv*>(state + min(col, hd - 1) * hd + min(r, hd - V));
 #pragma unroll
-            for (int e = 0; e < V; ++e) S[c][i + e] = (pos0 > 0 && col < hd && r < hd) ? s[e] : 0.f;  // a sequence starts from zero
+                for (int e = 0; e < V; ++e) S[c][i + e] = (pos0 > 0 && col < hd && r < hd) ? s[e] : 0.f;
+            }
         }
 
     for (int t0 = 0; t0 < a.S; t0 += kDeltaTile) {
@@ -115,16 +123,25 @@ __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
 #pragma unroll
                 for (int i = 0; i < KEEP; ++i) {
                     const T* w = static_cast<const T*>(a.w_decay) + (int64_t)(h * hd + min(lane + 64 * i, hd - 1)) * a.rank;
-                    for (int c0 = 0; c0 < a.rank; c0 += 64) {
-                        Chunk<T> x[64 / E];
+                    if constexpr (kShort) {
+#pragma unroll(sizeof(T) == 2 ? 1 : 2)
+                        for (int c = 0; c < a.rank; c += E) {
+                            const Chunk<T> x = load_chunk(w + c);
 #pragma unroll
-                        for (int j = 0; j < 64 / E; ++j) x[j] = load_chunk(w + min(c0 + E * j, a.rank - E));
+                            for (int e = 0; e < E; ++e) dl[i] = __builtin_fmaf(to_f32(x.v[e]), slow[wave][c + e], dl[i]);
+                        }
+                    } else {
+                        for (int c0 = 0; c0 < a.rank; c0 += 8 * E) {
+                            Chunk<T> x[8];
 #pragma unroll
-                        for (int j = 0; j < 64 / E; ++j)
-                            if (c0 + E * j < a.rank) {
+                            for (int j = 0; j < 8; ++j) x[j] = load_chunk(w + min(c0 + E * j, a.rank - E));
 #pragma unroll
-                                for (int e = 0; e < E; ++e) dl[i] = __builtin_fmaf(to_f32(x[j].v[e]), slow[wave][c0 + E * j + e], dl[i]);
-                            }
+                            for (int j = 0; j < 8; ++j)
+                                if (c0 + E * j < a.rank) {
+#pragma unroll
+                                    for (int e = 0; e < E; ++e) dl[i] = __builtin_fmaf(to_f32(x[j].v[e]), slow[wave][c0 + E * j + e], dl[i]);
+                                }
+                        }
                     }
                 }
             }
@@ -599,7 +616,7 @@ static int launch_delta_steps(const DeltaArgs& a, int B, hipStream_t s) {
 #define RAVEN_DELTA_STEPS(RPL, CP, V)                                                 \
     if (wide) delta_steps_kernel<T, RPL, CP, V><<<grid, block, 0, s>>>(a);            \
     else delta_steps_kernel<T, RPL, CP, 1><<<grid, block, 0, s>>>(a)
-    if (a.hd <= 32) { RAVEN_DELTA_STEPS(2, 1, 2); }
+    if (a.hd <= 32) delta_steps_kernel<T, 2, 1, 1><<<grid, block, 0, s>>>(a);
     else if (a.hd <= 48) delta_steps_kernel<T, 3, 2, 1><<<grid, block, 0, s>>>(a);
     else if (a.hd <= 64) { RAVEN_DELTA_STEPS(4, 2, 4); }
     else if (a.hd <= 96) { RAVEN_DELTA_STEPS(6, 3, 2); }
