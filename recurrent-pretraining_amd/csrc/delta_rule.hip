@@ -70,6 +70,7 @@ __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
     constexpr int R = 16 * RPL;       // rows held, the last ones zero
     constexpr int KEEP = (R + 63) / 64;
     constexpr bool kShort = RPL <= 3;
+    constexpr int kUnroll = sizeof(T) == 2 ? 1 : 2;
     static_assert(!kShort || V == 1, "small heads take their state value by value");
     __shared__ __align__(16) float sw[kDeltaTile][R], su[kDeltaTile][R], sb[kDeltaTile][R], sk[kDeltaTile][R], sr[kDeltaTile][R];
     __shared__ __align__(16) float sv[kDeltaTile][32 * CP], so[kDeltaTile][32 * CP];
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
                 for (int i = 0; i < KEEP; ++i) {
                     const T* w = static_cast<const T*>(a.w_decay) + (int64_t)(h * hd + min(lane + 64 * i, hd - 1)) * a.rank;
                     if constexpr (kShort) {
-#pragma unroll(sizeof(T) == 2 ? 1 : 2)
+#pragma unroll kUnroll
                         for (int c = 0; c < a.rank; c += E) {
                             const Chunk<T> x = load_chunk(w + c);
 #pragma unroll
