@@ -394,13 +394,16 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
 // ------------------------------------------------------------------------------------------------
 // The grouped products of experts with at most 16 rows a tile: y[r] = x[x_row[r]] W_g^T.  One unit -- a tile's rows against 32 weight rows (up: 16 gate and 16 up
 // rows) -- per workgroup of four waves that take the K steps in turn and never wait for each other; a wave's weight rows come as
-// whole runs of 128 or 256 bytes into two sets of registers, go through its own LDS tile into operand layout and are multiplied on the
-// matrix cores (the scheme of mfma_kernel in gemm_skinny.hip).  Bound by first reads of the weights: three workgroups a CU keep 100 KB in flight, and
-// some 50 units an expert, started as others end, leave no round half empty -- the units of 128 weight rows of gemm_mid.hip, two to a CU, made 1.3 rounds.
-// The K loop asks for nothing past its end and has no load under a branch, so that a wait counts only the step being parked.  us for a whole mixture (four
-// launches, weights from HBM), 64 experts, 6 per row and a shared one, by gemm_mid.hip / now: width 2048, 4 rows 55 / 48, 8: 86 / 71, 20: 120 / 105,
-// 40: 149 / 125; width 1024, 20 rows 44 / 40.6; 128 experts of 512, 8 per row, 20 rows 146 / 113.  Two register sets in flight 110 at 20 rows (fewer
-// resident waves), three 133; 64 weight rows a unit 112.
+// whole runs of 128 (down) or 256 bytes (up) into registers, go through its own LDS tile into operand layout and are multiplied on the
+// matrix cores (the scheme of mfma_kernel in gemm_skinny.hip).  Bound by first reads of the weights: what the workgroups of a CU, three of up and five of down, keep
+// in flight is some 80 to 100 KB, and some 50 units an expert, started as others end, leave no round half empty -- the units of 128 weight rows of
+// gemm_mid.hip, two to a CU, made 1.3 rounds.  The K loop asks for nothing past its end and has no load under a branch, so that a wait counts only the step
+// being parked.  us for a whole mixture (four launches, weights from HBM), 64 experts, 6 per row and a shared one, by gemm_mid.hip / now: width 2048, 4 rows
+// 55 / 48, 8: 86 / 71, 20: 120 / 105, 40: 149 / 125; width 1024, 20 rows 44 / 40.6; 128 experts of 512, 8 per row, 20 rows 146 / 113.  Two register sets in
+// flight 110 at 20 rows (fewer resident waves), three 133; 64 weight rows a unit 112.
+// Weights that one tile alone reads are not kept in the caches.  An expert with several tiles keeps them, and its units of the same weight rows are numbered
+// alike modulo 8, which puts them on one XCD: where all rows pick the same experts -- equal sequences side by side -- 40 rows of 64 experts of 864 at
+// width 2304 took 76 us without either, 59 with both (61 by gemm_mid.hip).
 // ------------------------------------------------------------------------------------------------
 struct FewArgs {
     const bf16 *x, *w;
@@ -409,14 +412,17 @@ struct FewArgs {
     RowGroups g;
 };
 
-template <bool UP, int KM, int NT>
+constexpr int few_columns(bool up) { return up ? 16 : 32; }  // output columns of a unit
+
+template <bool UP>
 __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
-    constexpr int NG = UP ? NT / 2 : NT, COLS = 16 * NG;  // output columns of a unit
+    constexpr int KM = UP ? 128 : 64, NT = 2, COLS = few_columns(UP), NG = COLS / 16;  // a K step, tiles of 16 weight rows, of output columns
     constexpr int PITCH = KM + 8, LPR = KM / 8, RPI = 64 / LPR, IPT = 16 / RPI;   // lanes per row, rows per load, loads per tile
     __shared__ __align__(16) bf16 stage[4][16 * (NT + 1)][PITCH];
     static_assert(sizeof(stage) >= 3 * NT * 64 * 16, "the tiles double as the waves' sums");
-    const int tile = (int)blockIdx.x / a.tiles_n, n0 = ((int)blockIdx.x - tile * a.tiles_n) * COLS;
-    if (tile >= *a.g.used) return;
+    const int tile = (int)blockIdx.x / a.tiles_n, at = (int)blockIdx.x - tile * a.tiles_n, used = *a.g.used;
+    const int n0 = (at + (tile * a.tiles_n) % 8) % a.tiles_n * COLS;
+    if (tile >= used) return;
     const int g = a.g.group_of[tile], row0 = a.g.group_row[tile], rows = a.g.group_end[tile] - row0;
     const bf16* W = g == a.g.extra_group ? a.g.w_extra : a.w + g * a.g.w_stride;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ln = lane & 15, kq = lane >> 4;
@@ -433,9 +439,10 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < IPT; ++i) wo[t][i] = (unsigned)(min(n0 + (t % NG) * 16 + RPI * i + lr, a.N - 1) + (UP && t >= NG ? a.N : 0)) * (unsigned)K;
-    // XI: load instructions that the tile's token rows need
-    auto run = [&](auto xi_tag) __attribute__((always_inline)) {
+    // XI: load instructions that the tile's token rows need.  ONCE: no other tile reads these weights
+    auto run = [&](auto xi_tag, auto once_tag) __attribute__((always_inline)) {
         constexpr int XI = decltype(xi_tag)::value;
+        constexpr bool ONCE = decltype(once_tag)::value;
         const bf16* xp[XI];
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
@@ -453,7 +460,10 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int j = 0; j < IPT; ++j) s.w[t][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + wo[t][j] + kc));
+                for (int j = 0; j < IPT; ++j) {
+                    const u32x4* from = reinterpret_cast<const u32x4*>(W + wo[t][j] + kc);
+                    s.w[t][j] = ONCE ? __builtin_nontemporal_load(from) : *from;
+                }
         };
         auto park = [&](int i, Staged& s) __attribute__((always_inline)) {
             const bool past = (wave + 4 * i) * KM + lc >= K;  // columns past K are zeros
@@ -496,8 +506,11 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
         wave_sync();
         multiply();
     };
-    if (rows <= RPI) run(std::integral_constant<int, 1>{});
-    else run(std::integral_constant<int, IPT>{});
+    const int before = a.g.group_of[max(tile - 1, 0)], after = a.g.group_of[min(tile + 1, used - 1)];
+    const bool alone = (tile == 0 || before != g) && (tile + 1 == used || after != g);
+    if (!alone) run(std::integral_constant<int, IPT>{}, std::false_type{});
+    else if (rows <= RPI) run(std::integral_constant<int, 1>{}, std::true_type{});
+    else run(std::integral_constant<int, IPT>{}, std::true_type{});
 
     __syncthreads();
     f32x4(*sums)[NT][64] = reinterpret_cast<f32x4(*)[NT][64]>(&stage[0][0][0]);
@@ -519,7 +532,7 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
         f32x4 v = acc[t];
         if (UP) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = silu_f32(v[i] * xs) * (acc[UP ? NG + t : t][i] * xs);
+            for (int i = 0; i < 4; ++i) v[i] = silu_f32(v[i] * xs) * (acc[UP ? t + 1 : t][i] * xs);
         }
         if (a.out_f32) {
             store4(static_cast<float*>(a.y) + at, v);
@@ -532,13 +545,11 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
 static int expert_rows(const void* x, const void* w, void* y, int N, int K, bool up, int out_f32, const RowGroups& g, hipStream_t s) {
     RAVEN_REQUIRE(g.n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && (!up || g.x_scale), "moe: bad experts");
     FewArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(w), y, N, K, 0, out_f32, g};
-    constexpr int kUp = 2, kDown = 2;
-    const int cols = up ? 8 * kUp : 16 * kDown;
-    a.tiles_n = (N + cols - 1) / cols;
+    a.tiles_n = (N + few_columns(up) - 1) / few_columns(up);
     const int64_t units = (int64_t)a.tiles_n * g.n_tiles;
     RAVEN_REQUIRE(units < (1ll << 31), "moe: too many units");
-    if (up) expert_rows_kernel<true, 128, kUp><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
-    else expert_rows_kernel<false, 64, kDown><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
+    if (up) expert_rows_kernel<true><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
+    else expert_rows_kernel<false><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
     return raven_host::check_launch("moe (rows of an expert)");
 }
 
