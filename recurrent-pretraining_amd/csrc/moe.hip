@@ -9,7 +9,7 @@
 // grouped product on the matrix cores (expert_rows_kernel, gemm_mid.hip, gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of
 // its own, and moe_combine_kernel adds a token's slots and its shared expert to the stream in a fixed order.  So an expert's weights
 // are read once and not once per row that picked it: 20 rows over 64 experts of 768 channels at width 2048, 6 each, read
-// 55 experts instead of 120 (246 us before, 105 now).
+// 55 experts instead of 120 (215 us by row kernels, 97).
 
 #include <algorithm>
 
@@ -399,8 +399,8 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
 // in flight is some 80 to 100 KB, and some 50 units an expert, started as others end, leave no round half empty -- the units of 128 weight rows of
 // gemm_mid.hip, two to a CU, made 1.3 rounds.  The K loop asks for nothing past its end and has no load under a branch, so that a wait counts only the step
 // being parked.  us for a whole mixture (four launches, weights from HBM), 64 experts, 6 per row and a shared one, by gemm_mid.hip / now: width 2048, 4 rows
-// 55 / 48, 8: 86 / 71, 20: 120 / 105, 40: 149 / 125; width 1024, 20 rows 44 / 40.6; 128 experts of 512, 8 per row, 20 rows 146 / 113.  Two register sets in
-// flight 110 at 20 rows (fewer resident waves), three 133; 64 weight rows a unit 112.
+// 63 / 48, 8: 82 / 68, 20: 119 / 97, 40: 148 / 130; width 1024, 20 rows 44 / 38; 128 experts of 512, 8 per row, 20 rows 144 / 111.  Two register sets in
+// flight were 5 % slower at 20 rows (fewer resident waves), three 27 %; 64 weight rows a unit 7 %.
 // Weights that one tile alone reads are not kept in the caches.  An expert with several tiles keeps them, and its units of the same weight rows are numbered
 // alike modulo 8, which puts them on one XCD: where all rows pick the same experts -- equal sequences side by side -- 40 rows of 64 experts of 864 at
 // width 2304 took 76 us without either, 59 with both (61 by gemm_mid.hip).
@@ -577,27 +577,28 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
 
 // What runs the experts of M rows.  A chunk -- once its rows share weights (two per expert), or there are enough rows anyway -- keeps its slots in T
 // and runs the shared expert as a product of its own.  Fewer rows keep slots and sums in float, as the row kernels do, and take the
-// grouped product once reading each expert once saves more than its two further launches cost.  us, row kernels / grouped, at width 2048 (64 experts of
-// 768 channels, 6 per row and a shared one): 2 rows 27 / 33, 3: 41 / 37, 4: 52 / 45, 8: 92 / 88, 20: 212 / 128; width 1024: 4 rows 33 / 36, 6: 45 / 39,
-// 8: 56 / 42; width 1024, one of 64 experts of 1024 and a shared one: 5 rows 16 / 28, 9: 22 / 30, 14: 32 / 34, 20: 47 / 42.
+// grouped product once reading each expert once saves more than its two further launches cost.  us, row kernels / grouped (means of four draws of picks), at
+// width 2048 (64 experts of 768 channels, 6 per row and a shared one): 2 rows 29 / 36, 3: 40 / 44, 4: 52 / 48, 8: 93 / 68, 20: 215 / 97; width 1024
+// (64 of 384): 4 rows 18 / 23, 6: 24 / 26, 8: 31 / 30, 12: 43 / 35; width 1024, one of 64 experts of 1024 and a shared one: 4 rows 14 / 21, 8: 21 / 24,
+// 12: 27 / 27, 20: 43 / 32; width 4096, 2 of 8 experts of 4096: 2 rows 72 / 70, 4: 135 / 105, 8: 251 / 132.
 enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
 constexpr size_t kMoeRowLds = 64 * 1024 - 1024;  // what a row may take of the row kernels' LDS; longer ones are refused for few rows
 static bool few_rows_fit(const raven_moe* m, int M, int ld) {
     return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs && ld * sizeof(bf16) <= kMoeRowLds &&
            (int64_t)2 * m->ff * ld < (1ll << 31);
 }
-// Estimates in us, within about 10 % of what 20 mixtures of 8 to 300 experts at widths 256 to 4096 took.  Row kernels: 5.4 TB/s whatever is read again, but
-// for the shared expert, which comes out of L2 from the second row on; past 64 experts the choice in every workgroup shows.  Grouped: four launches,
-// and per product a unit's walk over K (40 KB/us) or all weights once, at 5 TB/s, 3 where rows are so long that the last units' tail shows.
-// Nothing is grouped that would not read 25 MB again.
+// Estimates in us, fitted to what 33 mixtures of 8 to 512 experts of 128 to 4096 channels at widths 256 to 7168 took with 2 to 32 rows (312 calls; standard
+// deviations 6 % for grouped, 8 % for rows).  Row kernels: weights by how often they are read, and a share for each pick, more where experts are
+// picked by maxima over more than 64.  Grouped: four launches, and once the weights of the experts that rows pick on average, with a share for each.  Of two that
+// are about the same, the row kernels.  Against the better of the two the choice costs 0.6 % on average, 24 % at most (128 experts of 512 at width 1024, one per
+// row, 32 rows: 38 / 31).
 static bool grouping_pays(const raven_moe* m, int M, int ld) {
     const double pairs = (double)M * m->top, touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), shared = m->shared_up ? 1 : 0;
     const double expert = 6e-6 * ld * m->ff;  // MB
-    if ((pairs - touched + shared * (M - 1)) * expert <= 25) return false;
-    const double rows = 8.2 + (pairs + shared) * expert / 5.4 + shared * (M - 1) * expert / 13 + (m->experts > 64 ? 0.55 * M : 0);
-    auto product = [&](int K, double bytes) { return std::max(6.4e-3 * K, bytes / (K > 3072 ? 3 : 5)); };
-    const double grouped = 14.4 + 0.25 * M + product(ld, (touched + shared) * expert * 2 / 3) + product(m->ff, (touched + shared) * expert / 3);
-    return grouped < 1.1 * rows;
+    const double rows = 7 + (touched + shared) * expert / 5.65 + (pairs - touched) * expert / 6.5 + shared * (M - 1) * expert / 11 +
+                        pairs * (m->experts > 64 ? 0.15 : 0.05);
+    const double grouped = 14.7 + (touched + shared) * (expert / 6.5 + 0.08);
+    return grouped < 0.94 * rows;
 }
 // h: the rows, or null where only sizes are asked for.  The grouped kernels move whole 16-byte pieces into the LDS; operands that do not start
 // on one stay with the row kernels, which take any address.

@@ -425,6 +425,13 @@ def test_recurrent_step_of_several_sequences(pkg, dtype, W, blocks, taps):
                 assert torch.equal(state[0], together[1][b])
 
 
+@pytest.mark.parametrize("M,D,E,top,ff,shared", [(3, 7176, 24, 8, 264, False), (3, 5128, 24, 2, 1032, True), (6, 2568, 16, 2, 1544, True), (20, 264, 300, 8, 136, False)])
+def test_mixture_of_a_handful_of_wide_or_of_many_small_experts(pkg, M, D, E, top, ff, shared):
+    """Two and more rows whose experts' weights alone pay for the grouped products' launches, and many small experts; bound as beside."""
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, False)
+    test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, True)
+
+
 @pytest.mark.parametrize("M,D,E,top,ff,shared", [(130, 200, 160, 2, 40, False), (100, 2056, 64, 6, 760, True), (6, 1160, 64, 8, 520, True), (33, 1288, 40, 8, 1032, False)])
 def test_mixture_of_low_tiles(pkg, M, D, E, top, ff, shared):
     """expert_rows_kernel: fewer columns than one K step, steps and 16-column tiles that end early, tiles with rows for one load and for more, as a chunk
