@@ -805,7 +805,13 @@ static int run_absorbed(LatentArgs a, hipStream_t s) {
     else if (pieces <= 2) rc = launch_rows_attention<T, 2>(a, s);
     else rc = launch_rows_attention<T, 4>(a, s);
     if (rc) return rc;
-    if (a.per_wg == 2) a.per_wg = 1;  // (its rows are four times as long: 20 rows 8.8 us with 32 weight rows, 8.0 with 16; the launch above 6.7 / 7.8)
+    // The output's weight rows per workgroup: every workgroup merges its token rows' ranges for itself, so that 16 pay while workgroups x ranges x kv_rank is
+    // small, then 32 until they fill the chip eight times.  us for all three launches with 16 / 32 / 64, kv_rank 512, values of 128, bf16: 16 heads, 20 rows
+    // behind 75 positions (640 workgroups of 16, 2 ranges) 21.1 / 21.8 / 24.6, 40 (1280) 28.5 / 27.5 / 29.1, 12 rows behind 500 (384, 8 ranges) 26.6 / 25.4 /
+    // 28.0; 32 heads, 20 rows (1280) 32.1 / 30.5 / 33.1, 64 behind 200 (4096, 4 ranges) 67 / 59 / 58, 100 (6400) 77 / 71 / 70; 4 heads, kv_rank 256, values of
+    // 64, 100 rows (400) 17.2 / 18.2 / 21.7; fp32, 32 heads, 40 rows 51 / 47 / 50
+    const int64_t wgs = (int64_t)a.H * ((a.vp + 15) / 16) * blocks;
+    a.per_wg = a.M <= 2 || wgs * a.splits * a.kp <= 1 << 20 ? 1 : wgs <= 4096 ? 2 : 4;
     const int rows = 16 * a.per_wg;
     a.rows_out = (a.vp + rows - 1) / rows;
     latent_out_kernel<T, Z, RB><<<dim3(a.H * a.rows_out, blocks), dim3(256), (size_t)RB * a.kp * sizeof(T), s>>>(a);
@@ -859,7 +865,9 @@ extern "C" int raven_latent_rows(const raven_latent* l, const void* z, int32_t l
     a.append = l->own_kv;
     if (!a.cq && !a.append) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // us, both results by one wave / by two, ranks 768 and 512, bf16: 1 row 3.4 / 2.6, 20: 3.9 / 2.9, 500: 4.2 / 3.2, 4096: 7.0 / 6.5, 16384 (bound by memory): 18.3 / 19.3
+    // us, both results by one wave / by two, ranks 768 and 512, bf16: 1 row 3.4 / 2.6, 20: 3.9 / 2.9, 500: 4.2 / 3.2, 4096: 7.0 / 6.5.  Beyond, memory bounds
+    // both: 8192 10.3 / 10.5, 16384 18.0 / 18.9; of float rows 14.1 / 14.1, 24.2 / 24.4; fp32 17.2 / 17.1, 31.5 / 31.2 (ranks 384 to 1728: -14 to +5 %,
+    // either way at every number of rows)
     const dim3 grid((a.M + 3) / 4, a.cq && a.append && a.M <= 4096 ? 2 : 1);
     if (dtype == RAVEN_F32) latent_rows_kernel<float, float><<<grid, dim3(256), 0, s>>>(a);
     else if (z_f32) latent_rows_kernel<bf16, float><<<grid, dim3(256), 0, s>>>(a);

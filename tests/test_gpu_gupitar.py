@@ -425,6 +425,21 @@ def test_recurrent_step_of_several_sequences(pkg, dtype, W, blocks, taps):
                 assert torch.equal(state[0], together[1][b])
 
 
+@DT
+@pytest.mark.parametrize("H,B", [(40, 4), (40, 24), (40, 48), (4, 70)])
+def test_attention_output_by_every_number_of_weight_rows(pkg, dtype, H, B):
+    """16, 32 and 64 weight rows a workgroup of the output's launch, by the number of heads and rows; 136 channels leave a remainder of each.  Bounds as above."""
+    T, dim, rot, vdim, kr = 6, 8, 8, 136, 512
+    ins = [inputs(T, H, dim, rot, vdim, kr, seed=b) for b in range(B)]
+    a = Latent(pkg, H, dim, rot, vdim, kr, T, dtype, t_max=T, batch=B)
+    rows = [a.rows(*i) for i in ins]
+    stack = lambda k, lo, n: torch.cat([r[k][lo:lo + n] for r in rows]).contiguous()
+    a.hip.latent_rows(a.desc, stack(0, 0, T), a.native, B, T, 0, dtype, want_cq=False)
+    got = a.hip.latent_attention(a.desc, stack(1, T - 1, 1), stack(0, T - 1, 1), a.native, B, 1, T - 1).float().cpu().view(B, H, a.desc.vdim)[..., :vdim]
+    for s in range(B):
+        assert G.rel(got[s], a.want(*ins[s])[T - 1]) < (2e-5 if dtype == F32 else 3e-2), s
+
+
 @pytest.mark.parametrize("M,D,E,top,ff,shared", [(3, 7176, 24, 8, 264, False), (3, 5128, 24, 2, 1032, True), (6, 2568, 16, 2, 1544, True), (20, 264, 300, 8, 136, False)])
 def test_mixture_of_a_handful_of_wide_or_of_many_small_experts(pkg, M, D, E, top, ff, shared):
     """Two and more rows whose experts' weights alone pay for the grouped products' launches, and many small experts; bound as beside."""
