@@ -379,8 +379,14 @@ static int run_rglru(RglruArgs a, int B, hipStream_t s) {
     const size_t lds = (size_t)a.bl * sizeof(T);
     if (a.S == 1) {
         a.parts = (a.bl + 15) / 16;
-        // four sequences share a workgroup's weight rows once one each would make more workgroups than CUs (96 channels, 5 sequences: 3.9 us by four, 3.7 alone)
-        const bool four = B >= 3 && (int64_t)a.blocks * a.parts * B > 256 && 4 * lds <= 32 * 1024;
+        // Four sequences share a workgroup's weight rows once one each would make more than two workgroups per CU and the fours are three quarters full (or the
+        // matrices are more than the caches hold).  They form four windows, in more turns the longer the block, one tap after the other where there are not four: then later.  us alone / by four, bf16: 2048
+        // channels in 8 blocks, 4 sequences (512 workgroups) 3.4 / 3.6, 7 (896) 4.1 / 3.6; 2304 in 9, 5 (720) 3.85 / 4.6; 512 in 1, 20 (640) 4.1 /
+        // 4.3, 40 (1280) 5.5 / 5.1; 4096 in 4, 4 (1024) 6.4 / 5.7; three taps, 1320 in 5, 5 (425) 4.3 / 5.0, 12 (1020) 5.3 / 5.1, 20 (1700) 6.5 / 5.7;
+        // fp32, 4096 in 4, 3 (768) 8.8 / 10.3, 5 (1280; 32 MB of matrices) 12.4 / 11.4, 7 (1792) 15.6 / 11.4
+        const int64_t alone = (int64_t)a.blocks * a.parts * B, turns = (a.bl + 255) / 256;
+        const bool full = B >= (B + 3) / 4 * 3 || 2 * (int64_t)a.W * a.bl * (int64_t)sizeof(T) >= 32 << 20;
+        const bool four = alone > (384 + 128 * turns) * (a.taps == 4 ? 1 : 2) && full && 4 * lds <= 32 * 1024;
         const dim3 grid(a.blocks * a.parts, four ? (B + 3) / 4 : B);
         if (four && a.taps == 4) rglru_step_kernel<T, 4, 4><<<grid, dim3(256), 4 * lds, s>>>(a);
         else if (four) rglru_step_kernel<T, 4, 0><<<grid, dim3(256), 4 * lds, s>>>(a);

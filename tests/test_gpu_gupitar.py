@@ -440,6 +440,36 @@ def test_attention_output_by_every_number_of_weight_rows(pkg, dtype, H, B):
         assert G.rel(got[s], a.want(*ins[s])[T - 1]) < (2e-5 if dtype == F32 else 3e-2), s
 
 
+@DT
+@pytest.mark.parametrize("W,blocks,taps,B", [(2048, 8, 4, 7), (1032, 3, 4, 11), (1320, 5, 3, 18), (96, 3, 3, 190), (768, 1, 5, 34), (768, 1, 5, 2)])
+def test_recurrent_step_by_fours_against_64_bits(pkg, dtype, W, blocks, taps, B):
+    """Enough sequences to share weight rows four at a time, the last group cut short, windows of four taps and of others (and two sequences, which do not
+    share): two steps after the ring has wrapped.  fp32: sums in another order.  bf16: one rounding of the output, 2^-9; the window is rounded as the gates
+    read it, and where float and 64 bits round it apart the state moves by 2^-9 of that channel."""
+    bl, pos = W // blocks, taps + 1
+    g = torch.Generator(device="cuda").manual_seed(W + B)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    conv, cb, gb, sp = rand(taps, W) * 0.5, rand(W) * 0.3, rand(2, W) * 0.5, rand(W).abs() * 0.2
+    gates = (rand(blocks, 2, bl, bl) * bl ** -0.5).to(dtype)
+    desc = pkg.hip.Rglru(conv.data_ptr(), cb.data_ptr(), gates.data_ptr(), gb.data_ptr(), sp.data_ptr(), blocks, bl, taps, W)
+    ring, state = rand(B, taps, W), rand(B, W)
+    past = torch.stack([ring[:, p % taps] for p in range(pos - taps + 1, pos)], 1).double()  # the window before the new row
+    S = state.double()
+    for step in range(2):
+        z = rand(B, 2 * W).to(dtype)
+        y = pkg.hip.rglru(desc, z, ring, state, B, 1, pos + step)
+        v, x = z.double().split(W, 1)
+        window = torch.cat([past, x[:, None]], 1)
+        u = (cb.double() + (window * conv.double()).sum(1)).to(dtype).double()
+        r, i = (torch.sigmoid(torch.matmul(gates[:, k].double(), u.view(B, blocks, bl, 1)).reshape(B, W) + gb[k].double()) for k in (0, 1))
+        la = -8 * r * sp.double()
+        S = la.exp() * S + torch.sqrt(-torch.expm1(2 * la)) * i * u
+        want = S * torch.nn.functional.gelu(v, approximate="tanh")
+        assert G.rel(y.cpu(), want.cpu()) < (1e-5 if dtype == F32 else 3e-3) and G.rel(state.cpu(), S.cpu()) < (1e-5 if dtype == F32 else 1e-3)
+        assert torch.equal(ring[:, (pos + step) % taps], x.float())
+        past = window[:, 1:]
+
+
 @pytest.mark.parametrize("M,D,E,top,ff,shared", [(3, 7176, 24, 8, 264, False), (3, 5128, 24, 2, 1032, True), (6, 2568, 16, 2, 1544, True), (20, 264, 300, 8, 136, False)])
 def test_mixture_of_a_handful_of_wide_or_of_many_small_experts(pkg, M, D, E, top, ff, shared):
     """Two and more rows whose experts' weights alone pay for the grouped products' launches, and many small experts; bound as beside."""
