@@ -641,10 +641,14 @@ static size_t carve_moe(const raven_moe* m, int M, int ld, int dtype, MoePath pa
         // (400 units) 136 / 120; 8 of 2048 at 2048, 500 tokens (190) 105 / 116, 1000 (280) 134 / 122.
         // 16 rows by expert_rows_kernel against 32: 64 experts, 6 per row, 100 tokens (9 per expert) at widths 1024 / 1536 / 2048 / 2304 61 / 65, 90 / 104,
         // 136 / 157, 166 / 182; 150 (14) 65 / 66, 101 / 107, 154 / 161, 204 / 187; 200 (18) 72 / 67, 121 / 109, 178 / 168, 259 / 193.
+        // Many experts so small that expert_rows_kernel's units are over before their loads overlap: 32 from three per expert on.  us by 16 / 32, 8 per row: 300 of 136
+        // at width 264, 130 tokens 49 / 47.5, 300: 52 / 50; 256 of 64 at 256, 200: 38 / 36; 128 of 128 at 512, 130: 51 / 48; 300 of 256 at 256, 300: 60.5 / 58;
+        // but 300 of 256 at 512, 300: 74 / 78; 200 of 384 at 384, 130: 64 / 67.5; 128 of 128 at 768, 130: 46.1 / 46.4; 64 of 128 at 256, 40: 25 / 27.
         const size_t mean = pairs / m->experts;
+        const bool small = (ld < 320 || (size_t)ld * m->ff <= 80 * 1024) && (size_t)m->experts * ((m->ff + 15) / 16 + (ld + 31) / 32) >= 2500;
         const size_t big_tiles = pairs / 256 + m->experts / 2;  // an expert's last tile is half full on average
         const bool fills = big_tiles * ((m->ff + 127) / 128 + (ld + 255) / 256) > 256;
-        c.tile_rows = path == kMoeFew || mean <= 10 ? 16 : mean <= 20 ? 32 : mean < kBigTileRows || !fills ? 64 : 256;
+        c.tile_rows = path == kMoeFew || mean <= (small ? 2 : 10) ? 16 : mean <= 20 ? 32 : mean < kBigTileRows || !fills ? 64 : 256;
         auto tiles = [&](int height) { return (int)(pairs / height) + m->experts + (fold ? (M + height - 1) / height : 0); };
         c.n_tiles = tiles(c.tile_rows);
         const size_t table = (size_t)tiles(16) * 4;  // room for the lowest tiles whatever the height, so that more rows never need less

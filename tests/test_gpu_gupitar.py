@@ -470,9 +470,10 @@ def test_recurrent_step_by_fours_against_64_bits(pkg, dtype, W, blocks, taps, B)
         past = window[:, 1:]
 
 
-@pytest.mark.parametrize("M,D,E,top,ff,shared", [(3, 7176, 24, 8, 264, False), (3, 5128, 24, 2, 1032, True), (6, 2568, 16, 2, 1544, True), (20, 264, 300, 8, 136, False)])
+@pytest.mark.parametrize("M,D,E,top,ff,shared", [(3, 7176, 24, 8, 264, False), (3, 5128, 24, 2, 1032, True), (6, 2568, 16, 2, 1544, True), (20, 264, 300, 8, 136, False), (140, 264, 300, 8, 136, True)])
 def test_mixture_of_a_handful_of_wide_or_of_many_small_experts(pkg, M, D, E, top, ff, shared):
-    """Two and more rows whose experts' weights alone pay for the grouped products' launches, and many small experts; bound as beside."""
+    """Two and more rows whose experts' weights alone pay for the grouped products' launches, and many small experts, as few rows and as a chunk in tiles of 32;
+    bound as beside."""
     test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, False)
     test_mixture_reads_each_expert_once(pkg, M, D, E, top, ff, shared, True)
 
