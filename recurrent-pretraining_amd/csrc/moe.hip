@@ -587,17 +587,16 @@ static bool few_rows_fit(const raven_moe* m, int M, int ld) {
     return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs && ld * sizeof(bf16) <= kMoeRowLds &&
            (int64_t)2 * m->ff * ld < (1ll << 31);
 }
-// Estimates in us, fitted to what 33 mixtures of 8 to 512 experts of 128 to 4096 channels at widths 256 to 7168 took with 2 to 32 rows (312 calls; standard
-// deviations 6 % for grouped, 8 % for rows).  Row kernels: weights by how often they are read, and a share for each pick, more where experts are
-// picked by maxima over more than 64.  Grouped: four launches, and once the weights of the experts that rows pick on average, with a share for each.  Of two that
-// are about the same, the row kernels.  Against the better of the two the choice costs 0.6 % on average, 24 % at most (128 experts of 512 at width 1024, one per
-// row, 32 rows: 38 / 31).
+// Estimates in us, fitted to what 42 mixtures of 8 to 512 experts of 32 to 4096 channels at widths 256 to 7168 took with 2 to 32 rows (412 calls; standard
+// deviations 8 % for grouped, 10 % for rows).  Row kernels: weights as often as they are read, the shared expert's faster from the second row on, a share for
+// each pick, and past 64 experts, where maxima pick, one for each workgroup that picks.  Grouped: four launches, and once the weights of the experts that rows
+// pick on average, with a share for each.  Of two that are about the same, the row kernels.  Against the better of the two the choice costs 0.5 % on average,
+// 24 % at most (300 experts of 136 at width 264, 8 per row, 12 rows: 28 / 23).
 static bool grouping_pays(const raven_moe* m, int M, int ld) {
     const double pairs = (double)M * m->top, touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), shared = m->shared_up ? 1 : 0;
     const double expert = 6e-6 * ld * m->ff;  // MB
-    const double rows = 7 + (touched + shared) * expert / 5.65 + (pairs - touched) * expert / 6.5 + shared * (M - 1) * expert / 11 +
-                        pairs * (m->experts > 64 ? 0.15 : 0.05);
-    const double grouped = 14.7 + (touched + shared) * (expert / 6.5 + 0.08);
+    const double rows = 7.4 + (pairs + shared) * expert / 6.1 + shared * (M - 1) * expert / 11 + pairs * (0.06 + (m->experts > 64 ? 0.57e-3 * m->ff : 0));
+    const double grouped = 14.7 + (touched + shared) * (expert / 6.45 + 0.08);
     return grouped < 0.94 * rows;
 }
 // h: the rows, or null where only sizes are asked for.  The grouped kernels move whole 16-byte pieces into the LDS; operands that do not start
