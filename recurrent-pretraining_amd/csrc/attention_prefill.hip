@@ -689,7 +689,7 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
     // one chunk behind 140 positions, 55 heads of 96, 700 rows (605 workgroups of 64) 26 / 26, 180 (165) 10.2 / 12.3, 1500 (1320) 77 / 51; 8 heads of 128, 4000 (504)
     // 95 / 108; 32 of 128, 1500 (768) 50 / 50, 4000 (2016) 240 / 169; 12 of 64, 4000 (756) 66 / 75; 64 chunks of 64, 55 of 96, 78 / 84
     const int64_t behind = T < 0 ? (int64_t)(max_q_len - 1) * B : std::max(T - B, 0);
-    const int64_t chunks = behind > 0 ? (behind + max_q_len - 2) / (max_q_len - 1) : 0;
+    const int64_t chunks = max_q_len > 1 ? (behind + max_q_len - 2) / (max_q_len - 1) : 0;
     const int rg = max_q_len > 64 && chunks * ((max_q_len + 63) / 64) * n_heads > (head_dim == 64 ? 768 : 512) ? 2 : 1;
     const int rows = 64 * rg;
     // T rows in all fill less than T / rows blocks besides each sequence's last one.  Counting through the sequences costs more than starting fewer than 128

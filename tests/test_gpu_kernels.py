@@ -1144,3 +1144,17 @@ def test_chunks_among_many_paged_sequences(pkg):
     for i in (0, 8, 264, 265, 520, 521, 700, 776):
         lens[i], rows[i] = 400 + i, 200 + i % 100
     _check_paged_rows(pkg, 2, 64, 16, "HND", torch.bfloat16, lens, rows)
+
+
+@pytest.mark.parametrize("rows", [[1] * 6, [1, 1, 90, 1, 0, 200]])
+def test_paged_attention_with_rows_that_no_sequence_owns(pkg, rows):
+    """A buffer of query rows padded past the sequences' last row: their results to the bit, whatever the launch makes of the number of rows."""
+    dt, nh, hd, bs, dev = torch.bfloat16, 3, 64, 16, "cuda"
+    lens = [n + 150 + 10 * i for i, n in enumerate(rows)]
+    B, pages = len(rows), (max(lens) + bs - 1) // bs
+    k, v = rnd((B * pages, bs, nh, hd), dt, 930).cuda(), rnd((B * pages, bs, nh, hd), dt, 931).cuda()
+    args = (torch.arange(B * pages, dtype=torch.int32).view(B, pages).cuda(), torch.tensor(lens, dtype=torch.int32).cuda(),
+            torch.tensor([0] + rows).cumsum(0).to(torch.int32).cuda(), max(rows))
+    q = rnd((sum(rows) + 300, nh * hd), dt, 932).cuda()
+    want = pkg.hip.paged_prefill_attention(q[:sum(rows)].contiguous(), k, v, *args)
+    assert torch.equal(pkg.hip.paged_prefill_attention(q, k, v, *args)[:sum(rows)], want)
