@@ -386,7 +386,7 @@ static int run_rglru(RglruArgs a, int B, hipStream_t s) {
         // fp32, 4096 in 4, 3 (768) 8.8 / 10.3, 5 (1280; 32 MB of matrices) 12.4 / 11.4, 7 (1792) 15.6 / 11.4
         const int64_t alone = (int64_t)a.blocks * a.parts * B, turns = (a.bl + 255) / 256;
         const bool full = B >= (B + 3) / 4 * 3 || 2 * (int64_t)a.W * a.bl * (int64_t)sizeof(T) >= 32 << 20;
-        const bool four = alone > (384 + 128 * turns) * (a.taps == 4 ? 1 : 2) && full && 4 * lds <= 32 * 1024;
+        const bool four = B >= 3 && alone > (384 + 128 * turns) * (a.taps == 4 ? 1 : 2) && full && 4 * lds <= 32 * 1024;
         const dim3 grid(a.blocks * a.parts, four ? (B + 3) / 4 : B);
         if (four && a.taps == 4) rglru_step_kernel<T, 4, 4><<<grid, dim3(256), 4 * lds, s>>>(a);
         else if (four) rglru_step_kernel<T, 4, 0><<<grid, dim3(256), 4 * lds, s>>>(a);
