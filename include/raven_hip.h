@@ -237,8 +237,8 @@ int raven_exit_latent_stats(const void* latents, const void* prev, void* rel_cha
  *   sizes the launch; a sequence with no rows, or more rows than positions, is left alone.  Same kernel as
  *   raven_prefill_attention with the key tiles gathered through the block table; a sequence's only row goes through the cache on the
  *   vector units instead.
- * raven_paged_prefill_attention_rows: the same for a caller that knows T = q_start[B], the rows of all sequences together (-1: not known): the
- *   launch then holds no workgroup for blocks of rows that the shorter sequences do not have. */
+ * raven_paged_prefill_attention_rows: the same for a caller that knows T = q_start[B], the rows of all sequences together or more (-1: not known):
+ *   the launch then holds few workgroups for blocks of rows that the shorter sequences do not have. */
 enum { RAVEN_PAGED_NHD = 0, RAVEN_PAGED_HND = 1 };
 int raven_paged_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* slot_mapping,
                           int32_t T, int32_t n_heads, int32_t head_dim, int32_t block_size, int32_t kv_layout,

@@ -5,7 +5,7 @@
 // S > 1: plain causal when the cache was empty, lower-right-aligned causal otherwise).  The new
 // keys/values are already in the cache (raven_qkv_bias_rope_cache_append ran before).
 //
-// Grid (query blocks of 64 or 128 rows, heads, sequences), the blocks with the most keys first; 4 waves, each owns
+// Grid (query blocks of 64 or 128 rows, heads, sequences), the blocks with the most keys first; over pages (heads, blocks of all sequences: paged_block); 4 waves, each owns
 // RG groups of 16 query rows (RG = 1 or 2) and walks all key tiles of 64 positions on its own (no cross-wave softmax
 // state).  Per key tile:
 //   * the workgroup stages K [64 x hd] and V [64 x hd] in one of two LDS buffers, through registers that
@@ -62,7 +62,7 @@ constexpr int kFloatPages = 1 << 20;  // positions whose page a multiplication i
 
 // The only new row of a paged sequence: a decode row in a scheduler step that also carries a prompt chunk.  Four waves, 16 lanes to a cached position, 64
 // positions at a time with the next 64 requested before this tile's are used; float weights, the 16 groups' sums merged through LDS (`merge`, 16 * (HD + 2)
-// floats).  Bound by the cache's bytes and the two workgroups that a CU holds: 15 sequences of 420 positions, 55 heads of 96, 27 to 29 us = 4.6 to 4.9 TB/s
+// floats).  Bound by the cache's bytes and the two workgroups that a CU holds: 15 sequences of 420 positions, 55 heads of 96, 26 us = 5.1 TB/s
 // (the decode kernel over the same pages 28.5); as one of a tile's 16 query rows, three waves of four without a row and a wait for every staged tile,
 // 40.  off_of: element offset of a position's head row.  What is loaded without being part of the row or of the cache is selected away, not multiplied by
 // zero: infinities stay where they are.
@@ -153,7 +153,7 @@ __device__ __forceinline__ void single_row_attention(const bf16* q, bf16* y, con
 // no other.  Only the a.extra workgroups in front -- the blocks behind the first ones, at most T / rows of them, each with a whole block of rows
 // before it -- count through the sequences' row starts, 256 sequences a turn, from the last one on: schedulers put prompt chunks behind decode rows, and a
 // sequence's last block has the most keys.  False: none.  us with a count by every workgroup of all sequences, twice / now: single rows of 100 positions, 512
-// sequences of 8 heads of 128 89 / 44, 55 of 96 553 / 240, 1000 of 12 of 64 272 / 82; 15 of 420 positions beside a chunk of 1500 rows, 55 of 96, 88 / 74 --
+// sequences of 8 heads of 128 89 / 40, 55 of 96 553 / 233, 1000 of 12 of 64 272 / 74; 15 of 420 positions beside a chunk of 1500 rows, 55 of 96, 88 / 74 --
 // 157 with the longest sequence's blocks for every sequence, in their order.
 __device__ __forceinline__ bool paged_block(const PrefillArgs& a, int rows, int* seq, int* block) {
     const int x = blockIdx.y + gridDim.y * blockIdx.z, lane = threadIdx.x & 63;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     };
     if constexpr (PAGED) {
         // a single row has its whole table in LDS, however wide the table is.  us with the entries past kPfTable behind a branch in every position's loads / as
-        // rows of a tile / now: 30000 positions of 55 heads of 96 1000 / 482 / 292, 15 sequences of 420 in a table of 2000 entries, 12 heads of 64,
+        // rows of a tile / now: 30000 positions of 55 heads of 96 1000 / 482 / 305, 15 sequences of 420 in a table of 2000 entries, 12 heads of 64,
         // 23 / 15 / 10
         constexpr int kMerge = 16 * (HD + 2);
         static_assert(NW == 4 && (SK_ELEMS + SV_ELEMS) * sizeof(bf16) >= (kMerge + kRowTable) * sizeof(float), "sixteen groups, room to merge them and the table");
