@@ -62,8 +62,8 @@ __device__ __forceinline__ float delta_decay(float logit) { return expf(-0.60653
 // RPL rows per lane (16 * RPL >= hd), CP columns per lane group (32 * CP >= hd), moved V at a time (more than 1: the state starts on 16 bytes).
 // A decode step is one pass through memory latencies: every load of the state and of eight pieces of the decay's weight rows is unconditional (what lies
 // outside is selected away), so that they are in flight together.  us value by value behind conditions, piece by piece / now: 32 heads of 64 over rank 64, bf16,
-// 1 sequence 5.3 / 4.1, 20: 12.6 / 8.5, 40: 20.2 / 12.5; 16 heads of 128, 20: 40 / 16.  Heads of up to 48 have little to load, and what counts is that
-// four workgroups fit a CU's registers: they keep the short way.  32 heads of 32 over rank 32, short way / all together: bf16, 1 sequence 3.6 / 3.65, 20:
+// 1 sequence 5.3 / 4.1, 20: 12.6 / 8.5, 40: 20.2 / 12.5; 16 heads of 128, 20: 40 / 16.  Heads of up to 48 have little to load, and up to 32 what counts is
+// that three workgroups fit a CU's registers (75 and 80 of them; two with all requests together): they keep the short way.  32 heads of 32 over rank 32, short way / all together: bf16, 1 sequence 3.6 / 3.65, 20:
 // 4.6 / 6.1, 20 of 4 tokens 5.8 / 7.7; fp32 3.7 / 4.0, 4.7 / 6.7, 6.4 / 9.9.
 template <typename T, int RPL, int CP, int V>
 __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
