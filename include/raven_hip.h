@@ -100,8 +100,8 @@ const char* raven_last_error(void);
  * no tile-count rule, 3 = 256 x 256 by the eight-wave kernel instead of the four-wave ring kernel), gemm_tiled_split_tail
  * (1 = the tile columns of a last round that fills at most half the chip go to
  * 128 x 128 tiles, 0 = never), gemm_mid (1 = products over 33 and more bf16 rows that do not fill the chip with 256 x 256 tiles may run as
- * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (its tile
- * shape and slice count, 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
+ * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (its largest
+ * weight tiles, 1 to 6, and token tiles, 1 to 4, of a wave and its slice count, 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
  * gemm_one_round (1 = a 2..32-row product of up to about 16384 output columns runs as at most one workgroup of eight waves per compute unit where that is faster, 2 = wherever it is narrow enough, 0 = the

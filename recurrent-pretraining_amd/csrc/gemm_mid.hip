@@ -2,23 +2,26 @@
 // accumulation, with the epilogues of gemm_tiled.hip -- prompts of ordinary length, decode batches past 32 sequences, a serving engine's
 // mixed steps, and long prompts against matrices too narrow to give every CU a 256 x 256 tile.
 //
-// What bounds these products is keeping weight bytes in flight (few rows) and the LDS (many), so
-//   * operands go global -> LDS directly through a ring of NS stages, NS - 1 K steps of 64 ahead: 60 to 120 KB in flight on every CU, where
-//     two stages behind staging registers left one step in flight (mlp.fc of the 3.5b shape at 93 rows: 3.2 TB/s);
-//   * a unit owns `cols` output columns -- not whole tiles: as many as leave the chip ONE nearly full round of units (17920 gate columns =
-//     249 x 72), the last 16-row tile partly filled; missing rows are clamped on the load side and not stored;
+// What bounds these products is how a CU's loads queue: it has about 32 KB of lines on their way at a time, answered in order, so that the token rows,
+// which hit the L2, wait as long as the weights from HBM in front of them (64 + 96 rows a step move at 53 bytes a ns on 30 CUs, 42 on all; the weights
+// alone 51 and 22.5, the chip's 5.8 TB/s; the token rows alone 110).  A ring deeper than about 64 KB gives nothing; what counts is how few lines a
+// unit asks for, and that products and LDS reads stay below that time.  So
+//   * operands go global -> LDS directly through a ring of NS stages, NS - 1 K steps of 64 ahead;
+//   * a unit owns `cols` output columns and `rows` token rows, not whole tiles: as many as leave the chip ONE nearly full round of units (17920 gate
+//     columns = 249 x 72); the ring holds the 16-row tiles that exist and no others;
 //   * where even the narrowest unit leaves CUs idle, K is cut into slices: fp32 sums in the workspace, added in slice order by a second
 //     launch or by the norm that follows (splitk_sums_then_norm);
-//   * 8 waves, two along the weight rows and four along the token rows, a wave NT x MT tiles of 16 x 16 (v_mfma_f32_16x16x32_bf16, W rows
-//     as the A operand): two waves per SIMD hide each other's LDS reads; one barrier per K step.
+//   * 8 waves, two along the weight rows and four along the token rows (v_mfma_f32_16x16x32_bf16, W rows as the A operand); the unit's tiles are dealt
+//     out evenly and a wave has a loop for each number of tiles it may get, NT or one less by MT or one less: with every wave multiplying NT x MT a
+//     unit of 9 x 13 tiles made 192 products for 117;
+//   * weight rows that one unit reads are loaded past the caches (`nt`): 5 to 9 % where HBM bounds the launch; those that two row tiles share are not (5 % slower).
 // LDS rows are 128 bytes, 16-byte piece c of row r at position c ^ ((r >> 1) & 7) (applied on the global side), so that fragment reads are
 // free of bank conflicts.  Unlike the tiles of gemm_tiled.hip a wave's partial sums over K slices are added after the fact, so results
 // differ from those in the order of fp32 sums.
 //
-// us per launch at 93 rows of the 3.5b shape, weights from HBM (those of K = 5280 through their line-aligned copies), 128 x 128 tiles or passes of 32
-// rows before / this kernel (both launches where K is split): Wqkv 68 / 52, attn.proj 62 / 26, mlp.fc 125 / 91, mlp.proj 112 / 55, adapter 78 / 38; at
-// 195 rows 67 / 63, 59 / 35, 158 / 128, 188 / 83, 113 / 56; at 45 rows Wqkv 67 / 37, mlp.fc 110 / 74 (5.1 TB/s of weights), mlp.proj 72 / 43;
-// 4096 x 2048 x 8192 with an fp32 residual 163 / 133.
+// us per launch, weights from HBM, rows of whole lines; whole 64 x 32-row tiles for every wave / these: 3.5b shape at 93 rows Wqkv 44.9 / 40, attn.proj 24.1 / 21.5,
+// mlp.fc 78 / 68 (5.6 TB/s of weights), mlp.proj 56 / 44.5; at 195 rows 54.7 / 53.8, 32.3 / 26, 118 / 93, 82 / 56; width 2048 at 500 rows up 24.4 / 24.3, down
+// 37 / 29.6; 1500 rows 63 / 59, 78 / 59; 4096 x 2048 x 8192 124 / 113; 260 x 3072 x 1536 10.5 / 9.5.
 
 #include "gemm_common.h"
 
@@ -30,8 +33,9 @@ struct MidArgs {
     float* partial;        // [ks, M, N or 2N] when ks > 1
     int M, N, K0, K1, ldw, ldx;
     int out_f32;
+    int kind;              // EPI_*
     int cols, bm;          // output columns / token rows of a unit
-    int wrows;             // LDS rows of a unit's weight tile (whole 16-row tiles)
+    int wtiles, xtiles;    // 16-row tiles of a unit's weight rows / token rows
     int tiles_m, tiles_n, ks;
     raven_epilogue epi;    // EPI_FREE only
     int rope_on;           // EPI_PLAIN: the rope epilogue instead of y
@@ -114,13 +118,11 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 
 }
 
 // GROUPED: row groups with a weight matrix each; a unit works on a copy of the arguments cut to its group's rows
-template <int EPI, int WN, int WM, int NT, int MT, int NS, bool GROUPED = false>
+// ONCE: every weight row is read by one unit
+template <int WN, int WM, int NT, int MT, int NS, bool ONCE, bool GROUPED = false>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
-    constexpr bool SWIGLU = EPI == EPI_SWIGLU;
-    constexpr int NW = WN * WM, XROWS = 16 * WM * MT, XP = XROWS / 8;
-    // kilobyte pieces (8 rows x 128 bytes) a wave requests per step; with fewer token pieces than waves some are requested twice
-    constexpr int WPW = 2 * NT / WM, XPW = XP >= NW ? XP / NW : 1, LPW = WPW + XPW;
-    static_assert(NT % 2 == 0 && (2 * NT) % WM == 0 && (XP % NW == 0 || NW % XP == 0) && (NS - 1) * LPW < 64, "whole pieces; the wait counter holds 63 requests");
+    constexpr int NW = WN * WM, WPW = (2 * WN * NT + NW - 1) / NW, XPW = (2 * WM * MT + NW - 1) / NW, LPW = WPW + XPW;  // requests of a wave per step
+    static_assert(NW % 2 == 0 && (NS - 1) * LPW < 64, "a wave's pieces have one parity; the wait counter holds 63 requests");
     extern __shared__ __align__(1024) unsigned char smem[];
 
     // which unit: K slices outermost, then bands of eight token tiles, so that the units of an XCD (ids congruent modulo 8) are neighbours
@@ -146,100 +148,88 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         tile_m = 0;
     }
 
+    const bool swiglu = a.kind == EPI_SWIGLU;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wn = wave % WN, wm = wave / WN;
     const int K = a.K0 + a.K1, nk = (K + 63) >> 6;
     const int k0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * slice / a.ks));
     const int n_steps = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * (slice + 1) / a.ks)) - k0;
-    const int n0 = tile_n * a.cols, ncols = min(a.cols, a.N - n0), m0 = tile_m * a.bm;
-    const int wbytes = a.wrows * 128, stage = wbytes + XROWS * 128;
+    const int n0 = tile_n * a.cols, ncols = min(a.cols, a.N - n0), m0 = tile_m * a.bm, rows = min(a.bm, a.M - m0);
+    // the wave's tiles, dealt out evenly; a SIMD's two waves (ids that differ by four) get a long and a short share of the token tiles
+    const int wn = wave / WM, wm = (wn & 1) ? WM - 1 - wave % WM : wave % WM;
+    const int tw = __builtin_amdgcn_readfirstlane(((swiglu ? 2 * ncols : ncols) + 15) >> 4), tx = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
+    const int nw = tw / WN + (wn < tw % WN), tw0 = wn * (tw / WN) + min(wn, tw % WN);
+    const int nx = tx / WM + (wm < tx % WM), tx0 = wm * (tx / WM) + min(wm, tx % WM);
+    const int wbytes = a.wtiles * 2048, stage = wbytes + a.xtiles * 2048, ring = NS * stage;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_byte*)smem;
 
-    // ---- global side: request i of a wave is piece NW i + wave, rows 8 (NW i + wave) ..+7 of the weight tile (i < WPW) or of the token
-    // rows; the lane that fills position s of row r fetches piece s ^ ((r >> 1) & 7) of the row's 128-byte step
+    // ---- global side: request i of a wave is piece NW i + wave, eight rows of the weight tile (i < WPW) or of the token rows; the lane that
+    // fills position s of row r fetches piece s ^ ((r >> 1) & 7) of the row's 128-byte step.  A SwiGLU tile is eight gate rows and their up
+    // rows.  Requests past the unit's last piece fetch one line, of the last row, to behind the ring: the count of requests stays.
     const int colp = ((lane & 7) ^ ((lane >> 4) | (4 * (wave & 1)))) * 8;
     unsigned goff[LPW];
-    unsigned dst[LPW];  // offset inside a stage; weight pieces past the tile land behind the ring
+    unsigned dst[LPW];  // offset inside a stage
+    bool spare[LPW];
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
         const bool is_w = i < WPW;
-        const int piece = is_w ? NW * i + wave : (NW * (i - WPW) + wave) % XP, r = piece * 8 + (lane >> 3);
+        const int piece = is_w ? NW * i + wave : NW * (i - WPW) + wave, r = piece * 8 + (lane >> 3);
+        spare[i] = (GROUPED || i == WPW - 1 || i == LPW - 1) && piece >= 2 * (is_w ? a.wtiles : a.xtiles);  // (of a plain unit only the last ones may be)
         if (is_w) {
-            int row;
-            if (SWIGLU) row = n0 + min((r >> 5) * 16 + (r & 15), ncols - 1) + ((r & 16) ? a.N : 0);
-            else row = n0 + min(r, ncols - 1);
-            goff[i] = (unsigned)row * (2u * a.ldw) + 2u * colp;
-            dst[i] = piece * 1024;
+            const int c = min(swiglu ? (r >> 4) * 8 + (r & 7) : r, ncols - 1);
+            goff[i] = (unsigned)(n0 + c + (swiglu && (r & 8) ? a.N : 0)) * (2u * a.ldw) + 2u * colp;
         } else {
-            int row = min(m0 + r, a.M - 1);
+            int row = m0 + min(r, rows - 1);
             if (GROUPED && x_row) row = x_row[row];
             goff[i] = (unsigned)row * (2u * a.ldx) + 2u * colp;
-            dst[i] = wbytes + piece * 1024;
         }
+        dst[i] = __builtin_amdgcn_readfirstlane(lds_base + (is_w ? 0 : wbytes) + piece * 1024);
     }
     const char* const zero = reinterpret_cast<const char*>(g_mid_zero);
     const char* const w0 = reinterpret_cast<const char*>(a.w);
     const char* const x0 = reinterpret_cast<const char*>(a.x0);
     const char* const x1 = reinterpret_cast<const char*>(a.x1) - 2 * (int64_t)a.K0;  // column c >= K0 of the token rows
-    // requests FIRST .. LAST - 1 of step kk (columns 64 kk ..+63; zeros past K) into the stage at offset o
-    auto issue = [&](int kk, int o, auto first_tag, auto last_tag) __attribute__((always_inline)) {
+    auto whole = [&](int kk) __attribute__((always_inline)) {  // the 64 columns of step kk lie in one segment and below K
         const int c0 = kk << 6;
-        const bool whole = c0 + 64 <= a.K0 || (c0 >= a.K0 && c0 + 64 <= K);  // the 64 columns lie in one segment and below K
+        return c0 + 64 <= a.K0 || (c0 >= a.K0 && c0 + 64 <= K);
+    };
+    // requests FIRST .. LAST - 1 of step kk (columns 64 kk ..+63; zeros past K) into the stage at offset o; whole_tag: 1 whole, 0 not, 2 either
+    auto issue = [&](int kk, int o, auto first_tag, auto last_tag, auto whole_tag) __attribute__((always_inline)) {
+        const int c0 = kk << 6;
+        if (decltype(whole_tag)::value == 1 || (decltype(whole_tag)::value == 2 && whole(kk))) {
+            const char *wb = w0 + 2 * c0, *xb = (c0 < a.K0 ? x0 : x1) + 2 * c0;
+#pragma unroll
+            for (int i = decltype(first_tag)::value; i < decltype(last_tag)::value; ++i) {
+                const unsigned to = __builtin_amdgcn_readfirstlane(spare[i] ? lds_base + ring : o + dst[i]);
+                if (ONCE && i < WPW) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(goff[i]), "s"(wb), "s"(to) : "memory");
+                else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(i < WPW ? wb : xb), "s"(to) : "memory");
+            }
+            return;
+        }
+        const int col = c0 + colp;
 #pragma unroll
         for (int i = decltype(first_tag)::value; i < decltype(last_tag)::value; ++i) {
-            const bool is_w = i < WPW;
-            const bool spare = is_w && (NW * i + wave) * 8 >= a.wrows;
-            const unsigned to = __builtin_amdgcn_readfirstlane(lds_base + (spare ? NS * stage : o + (int)dst[i]));
-            if (whole) {
-                const char* base = (is_w ? w0 : (c0 < a.K0 ? x0 : x1)) + 2 * c0;
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(goff[i]), "s"(base), "s"(to) : "memory");
-            } else {
-                const int col = c0 + colp;
-                const char* gp = col >= K ? zero : (is_w ? w0 : (col < a.K0 ? x0 : x1)) + 2 * c0 + goff[i];
-                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gp), "s"(to) : "memory");
-            }
+            const unsigned to = __builtin_amdgcn_readfirstlane(spare[i] ? lds_base + ring : o + dst[i]);
+            unsigned off = goff[i];
+            asm volatile("" : "+v"(off));  // (the address is not worth a register pair outside this step)
+            const char* gp = col >= K ? zero : (i < WPW ? w0 : (col < a.K0 ? x0 : x1)) + 2 * c0 + off;
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gp), "s"(to) : "memory");
         }
     };
 
-    // ---- LDS -> registers -> products
-    const int l16 = lane & 15, q4 = lane >> 4;
-    const unsigned pos0 = (q4 ^ ((l16 >> 1) & 7)) * 16;  // k-slice s of a step: pos0 ^ (64 s)
-    const unsigned a_row = lds_base + (wn * NT * 16 + l16) * 128, b_row = lds_base + wbytes + (wm * MT * 16 + l16) * 128;
-    const int used = min(max((a.wrows >> 4) - wn * NT, 0), NT);  // weight tiles of this wave that exist
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    u32x4 fa[2][NT], fb[2][MT];  // fragments of the two k-slices of a step
-    auto fetch = [&](int o, auto sl_tag, auto full_tag) __attribute__((always_inline)) {
-        constexpr bool FULL = decltype(full_tag)::value;
-        constexpr int sl = decltype(sl_tag)::value;
-        const unsigned ra = a_row + o + (pos0 ^ (64 * sl)), rb = b_row + o + (pos0 ^ (64 * sl));
-        if (!FULL && used == 0) return;
-#pragma unroll
-        for (int j = 0; j < MT; ++j) fb[sl][j] = *reinterpret_cast<const lds_u32x4*>(rb + j * 2048);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)  // (a tile that does not exist repeats the last one; its products are never stored)
-            fa[sl][t] = *reinterpret_cast<const lds_u32x4*>(ra + (FULL ? t : min(t, used - 1)) * 2048);
-    };
-    auto multiply = [&](auto sl_tag, auto full_tag) __attribute__((always_inline)) {
-        constexpr int sl = decltype(sl_tag)::value;
-        if (!decltype(full_tag)::value && used == 0) return;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-                acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[sl][t]), __builtin_bit_cast(bf16x8, fb[sl][j]), acc[t][j], 0, 0, 0);
-    };
 
     // ---- the ring: step i sits in stage i mod NS.  The barrier in the middle of step i says that every wave's requests of step i + 1 have
     // landed and that every wave has read out step i, whose stage step i + NS then takes.  The fragments of a slice are read under the
     // products of the slice before, the requests stand between the two slices' products: with reads, requests and products of all eight
     // waves one after the other behind the barrier a step took the sum of the three (Wqkv of the 3.5b shape at 93 rows 46 us).
-    const int ring = NS * stage;
+    const int l16 = lane & 15, q4 = lane >> 4;
     using ic0 = std::integral_constant<int, 0>;
     using ic1 = std::integral_constant<int, 1>;
+    using ic2 = std::integral_constant<int, 2>;
     using half = std::integral_constant<int, (LPW + 1) / 2>;
     using all = std::integral_constant<int, LPW>;
     auto arrive = [&](auto left_tag) __attribute__((always_inline)) {  // all but the requests of `left` steps have landed
@@ -249,61 +239,110 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
     };
+    auto arrive_left = [&](int left) __attribute__((always_inline)) {  // the same, NS - 2 at most
+        static_for<NS - 1>([&](auto n_tag) {
+            constexpr int n = decltype(n_tag)::value;
+            if (n < NS - 2 ? left == n : left >= n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n * LPW) : "memory");
+        });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    };
+    // NTW x MTW: tiles of this wave; a wave without any requests its share and multiplies nothing
+    auto run = [&](auto nt_tag, auto mt_tag) __attribute__((always_inline)) {
+        constexpr int NTW = decltype(nt_tag)::value, MTW = decltype(mt_tag)::value;
+        const unsigned pos0 = (q4 ^ ((l16 >> 1) & 7)) * 16;  // k-slice s of a step: pos0 ^ (64 s)
+        const unsigned a_row = lds_base + (tw0 * 16 + l16) * 128, b_row = lds_base + wbytes + (tx0 * 16 + l16) * 128;
+        u32x4 fa[2][NTW ? NTW : 1], fb[2][MTW ? MTW : 1];  // fragments of the two k-slices of a step
+        auto fetch = [&](int o, auto sl_tag) __attribute__((always_inline)) {
+            constexpr int sl = decltype(sl_tag)::value;
+            const unsigned ra = a_row + o + (pos0 ^ (64 * sl)), rb = b_row + o + (pos0 ^ (64 * sl));
+#pragma unroll
+            for (int j = 0; j < MTW; ++j) fb[sl][j] = *reinterpret_cast<const lds_u32x4*>(rb + j * 2048);
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) fa[sl][t] = *reinterpret_cast<const lds_u32x4*>(ra + t * 2048);
+        };
+        auto multiply = [&](auto sl_tag) __attribute__((always_inline)) {
+            constexpr int sl = decltype(sl_tag)::value;
+#pragma unroll
+            for (int t = 0; t < NTW; ++t)
+#pragma unroll
+                for (int j = 0; j < MTW; ++j)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[sl][t]), __builtin_bit_cast(bf16x8, fb[sl][j]), acc[t][j], 0, 0, 0);
+        };
+        int o = 0, i = 0;
+        arrive_left(n_steps - 1);
+        fetch(0, ic0{});
+        // Small tiles: a loop without a branch for the steps whose requests are whole, another for the few that are not (uq of 1536 to 3072 columns at
+        // 260 rows 10.7 -> 9.6 us).  Large ones: their products hide the branches, and registers are short.
+        auto steps = [&](int end, auto whole_tag) __attribute__((always_inline)) {  // whose requests are of whole steps, or none of them
+#pragma unroll 1
+            for (; i < end; ++i) {
+                const int free = o == 0 ? ring - stage : o - stage, next = o + stage == ring ? 0 : o + stage;
+                fetch(o, ic1{});
+                issue(k0 + i + NS - 1, free, ic0{}, half{}, whole_tag);
+                multiply(ic0{});
+                issue(k0 + i + NS - 1, free, half{}, all{}, whole_tag);
+                arrive(std::integral_constant<int, NS - 2>{});
+                fetch(next, ic0{});
+                multiply(ic1{});
+                o = next;
+            }
+        };
+        const int asked = n_steps - NS + 1;  // steps that still request
+#pragma unroll 1
+        while (i < asked) {
+            const int kk = k0 + i + NS - 1;
+            if constexpr (NT * MT > 6) steps(asked, ic2{});
+            else if (whole(kk)) steps(min(asked, ((a.K0 & 63) && kk < (a.K0 >> 6) ? a.K0 >> 6 : K >> 6) - (k0 + NS - 1)), ic1{});
+            else steps(i + 1, ic0{});
+        }
+        // nothing more to request: the last NS - 1 steps, or all of a shorter slice
+        static_for<NS - 1>([&](auto j_tag) {
+            constexpr int left = NS - 2 - decltype(j_tag)::value;  // steps behind this one
+            if (n_steps <= left) return;
+            const int next = o + stage == ring ? 0 : o + stage;
+            fetch(o, ic1{});
+            multiply(ic0{});
+            if constexpr (left > 0) {
+                arrive(std::integral_constant<int, (left > 0 ? left - 1 : 0)>{});
+                fetch(next, ic0{});
+            }
+            multiply(ic1{});
+            o = next;
+        });
+    };
+#pragma unroll 1
+    for (int i = 0; i < NS - 1 && i < n_steps; ++i) issue(k0 + i, i * stage, ic0{}, all{}, ic2{});
+    // (with fewer tiles than one less than the variant's the surplus fragments are whatever lies behind, and their products are not stored)
+    using nt0 = std::integral_constant<int, NT>;
+    using nt1 = std::integral_constant<int, NT - 1>;
+    using mt0 = std::integral_constant<int, MT>;
+    using mt1 = std::integral_constant<int, MT - 1>;
+    if (__builtin_expect(nw == NT && nx == MT, 1)) run(nt0{}, mt0{});
+    else if (nw == 0 || nx == 0) run(ic0{}, ic0{});
+    else if (nw == NT) { if constexpr (MT > 1) run(nt0{}, mt1{}); }
+    else if (nx == MT) { if constexpr (NT > 1) run(nt1{}, mt0{}); }
+    else { if constexpr (NT > 1 && MT > 1) run(nt1{}, mt1{}); }
+
+    // ---- out: a lane holds rows 4 q4 ..+3 of weight tile t for token row 16 j + l16.  A wave lays its sums down in LDS, rows of its columns,
+    // and a rolled loop takes them from there: whole runs of columns per store, and little code -- unrolled over the accumulators
+    // the epilogue ran once per unit out of a cold instruction cache (gelu outputs of 3000 x 4096 x 1024: 46 us, as a loop 36).
     // lanes of a wave exchange data through LDS without a workgroup barrier: pin the order of the accesses for the compiler
     auto wave_sync = []() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    auto run = [&](auto full_tag) __attribute__((always_inline)) {
-        int o = 0, i = 0;
-        arrive(std::integral_constant<int, NS - 2>{});
-        fetch(0, ic0{}, full_tag);
-#pragma unroll 1
-        for (; i + NS - 1 < n_steps; ++i) {
-            const int free = o == 0 ? ring - stage : o - stage, next = o + stage == ring ? 0 : o + stage;
-            fetch(o, ic1{}, full_tag);
-            issue(k0 + i + NS - 1, free, ic0{}, half{});
-            multiply(ic0{}, full_tag);
-            issue(k0 + i + NS - 1, free, half{}, all{});
-            arrive(std::integral_constant<int, NS - 2>{});
-            fetch(next, ic0{}, full_tag);
-            multiply(ic1{}, full_tag);
-            o = next;
-        }
-        static_for<NS - 1>([&](auto j_tag) {  // nothing more to request
-            constexpr int j = decltype(j_tag)::value;
-            if (i < n_steps) {
-                const int next = o + stage == ring ? 0 : o + stage;
-                fetch(o, ic1{}, full_tag);
-                multiply(ic0{}, full_tag);
-                if constexpr (j < NS - 2) {
-                    if (i + 1 < n_steps) {
-                        arrive(std::integral_constant<int, NS - 3 - j>{});
-                        fetch(next, ic0{}, full_tag);
-                    }
-                }
-                multiply(ic1{}, full_tag);
-                o = next;
-                ++i;
-            }
-        });
-    };
-#pragma unroll 1
-    for (int i = 0; i < NS - 1; ++i) issue(k0 + i, i * stage, ic0{}, all{});
-    if (used == NT) run(std::true_type{});
-    else run(std::false_type{});
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // requests past a short slice still write into the ring
-
-    // ---- out: a lane holds columns 16 t + 4 q4 ..+3 of token row 16 j + l16.  A wave lays its sums down in LDS, rows of its columns,
-    // and a rolled loop takes them from there: whole runs of columns per store, and little code -- unrolled over the accumulators
-    // the epilogue ran once per unit out of a cold instruction cache (gelu outputs of 3000 x 4096 x 1024: 46 us, as a loop 36).
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();  // every wave has left the ring
-    constexpr int JG = MT < 2 ? MT : 2, PITCH = NT * 64 + 16;   // row tiles at a time; bytes of an LDS row
-    constexpr int UPR = SWIGLU ? NT * 2 : NT * 4;               // runs of four output columns per row
+    constexpr int JG = MT % 2 ? 1 : 2, PITCH = NT * 64 + 16;    // row tiles at a time; bytes of an LDS row
     const unsigned mine = lds_base + wave * (JG * 16 * PITCH);
-    const int ntot = SWIGLU ? 2 * a.N : a.N;
-    const int col0 = wn * (SWIGLU ? NT * 8 : NT * 16);          // this wave's first output column inside the unit
+    const int ntot = swiglu ? 2 * a.N : a.N;
+    const int col0 = tw0 * (swiglu ? 8 : 16), col_end = min(ncols, col0 + nw * (swiglu ? 8 : 16));  // this wave's output columns inside the unit
+    const int row_end = min(rows, (tx0 + nx) * 16);
 #pragma unroll 1
     for (int pass = 0; pass < MT / JG; ++pass) {
         static_for<MT / JG>([&](auto p_tag) {
@@ -316,23 +355,33 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
                     *reinterpret_cast<__attribute__((address_space(3))) f32x4*>(mine + (j * 16 + l16) * PITCH + t * 64 + q4 * 16) = acc[t][ps * JG + j];
         });
         wave_sync();
+        const int first = (tx0 + pass * JG) * 16;
+        auto store = [&](auto kind_tag) __attribute__((always_inline)) {
+            constexpr int EPI = decltype(kind_tag)::value;
+            constexpr bool SWIGLU = EPI == EPI_SWIGLU;
+            constexpr int UPR = SWIGLU ? NT * 2 : NT * 4;  // runs of four output columns per row
 #pragma unroll 2
-        for (int it = 0; it < JG * 16 * UPR / 64; ++it) {
-            const int idx = it * 64 + lane, row = idx / UPR, u = idx - row * UPR;
-            const int col = col0 + 4 * u, mr = (wm * MT + pass * JG) * 16 + row, m = m0 + mr;
-            if (col >= ncols || mr >= a.bm || m >= a.M) continue;
-            const unsigned at = mine + row * PITCH + (SWIGLU ? (u >> 2) * 128 + (u & 3) * 16 : u * 16);
-            const f32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at);
-            const f32x4 up = SWIGLU ? *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at + 64) : f32x4{0.f, 0.f, 0.f, 0.f};
-            if (a.ks > 1) {
-                float* p = a.partial + ((int64_t)slice * a.M + m) * ntot + n0 + col;
-                *reinterpret_cast<f32x4*>(p) = v;
-                if (SWIGLU) *reinterpret_cast<f32x4*>(p + a.N) = up;
-            } else {
-                const float xs = GROUPED && SWIGLU ? a.groups.x_scale[m] : 1.f;
-                mid_store<EPI, GROUPED>(a, m, n0 + col, v, up, xs);
+            for (int idx = lane; idx < JG * 16 * UPR; idx += 64) {
+                const int row = idx / UPR, u = idx - row * UPR, col = col0 + 4 * u, mr = first + row, m = m0 + mr;
+                if (col >= col_end || mr >= row_end) continue;
+                const unsigned at = mine + row * PITCH + (SWIGLU ? (u >> 1) * 64 + (u & 1) * 16 : u * 16);
+                const f32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at);
+                const f32x4 up = SWIGLU ? *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at + 32) : f32x4{0.f, 0.f, 0.f, 0.f};
+                if (a.ks > 1) {
+                    float* p = a.partial + ((int64_t)slice * a.M + m) * ntot + n0 + col;
+                    *reinterpret_cast<f32x4*>(p) = v;
+                    if (SWIGLU) *reinterpret_cast<f32x4*>(p + a.N) = up;
+                } else {
+                    const float xs = GROUPED && SWIGLU ? a.groups.x_scale[m] : 1.f;
+                    mid_store<EPI, GROUPED>(a, m, n0 + col, v, up, xs);
+                }
             }
-        }
+        };
+        if (swiglu) store(std::integral_constant<int, EPI_SWIGLU>{});
+        else if (GROUPED || a.kind == EPI_FREE) store(std::integral_constant<int, EPI_FREE>{});
+        else if (a.kind == EPI_PLAIN || a.ks > 1) store(std::integral_constant<int, EPI_PLAIN>{});
+        else if (a.kind == EPI_FREE_GELU) store(std::integral_constant<int, EPI_FREE_GELU>{});
+        else store(std::integral_constant<int, EPI_FREE_TANH>{});
         wave_sync();
     }
 }
@@ -381,25 +430,31 @@ static int mid_cus() {
     return cus;
 }
 
-// stages of the ring of a variant (0: no such variant)
+// stages of the ring of a variant: as many as fit at its largest unit, 3 to 8 (nt 6, mt 4: three only up to 26 tiles in all)
 static constexpr int mid_stages(int nt, int mt) {
-    return nt == 2 ? (mt == 1 ? 8 : mt == 2 ? 6 : 4) : nt == 4 ? (mt == 1 ? 6 : mt == 2 ? 5 : 3) : (mt == 1 ? 5 : mt == 2 ? 4 : 3);
+    const int fit = (kLds - nt % 2 * 1024) / ((2 * nt + 4 * mt) * 2048);  // (odd nt: eight waves' requests are more than the unit's pieces)
+    return fit > 8 ? 8 : fit < 3 ? 3 : fit;
 }
 
-// What a launch of a plan costs, in us, fitted to 1847 products of 33 to 4100 rows, 64 to 36000 columns and K of 64 to 18000 (standard deviation 8 %).
-// The memory pipe delivers first reads of the weights at 9 TB/s and what comes out of L2 -- the token rows once per column of units, the
-// weights again for further row tiles -- at 18; a K step takes the LDS the fragment reads of eight waves (8 clocks per kilobyte) and the
-// requests' writes, at 2 clocks per ns; the largest units, with three or four stages in flight, fall short of that.  Every round of units fills its
-// ring and drains its outputs anew: 3514 x 592 x 64 in three rounds takes 12.4 us, where a round's own work is 0.3 (128 x 128 tiles, one round: 5.2).
+// LDS of a unit: the ring and the kilobyte behind it, where requests are left over, or the sums on their way out
+static size_t mid_lds_bytes(int waves, int nt, int mt, int ns, int wtiles, int xtiles) {
+    const size_t ring = (size_t)ns * (wtiles + xtiles) * 2048 + (2 * wtiles % waves || 2 * xtiles % waves ? 1024 : 0), sums = (size_t)waves * (mt % 2 ? 1 : 2) * 16 * (nt * 64 + 16);
+    return ring > sums ? ring : sums;
+}
+
+// What a launch of a plan costs, in us, fitted to 3634 products of 33 to 4096 rows, 768 to 36000 columns and K of 768 to 18000 (standard deviation 9 %;
+// the plans it picks for 317 shapes are 1.0 % slower than the best of each).  First reads of the weights come at 8.8 TB/s, what comes out of the caches --
+// the token rows once per column of units, the weights again for further row tiles -- at 60; a K step takes its fragment reads, products and
+// requests; of the two the shorter one is hidden to two fifths.  Every round of units fills its ring and drains its outputs anew.
 static double mid_estimate(const MidPlan& p, int M, int N, int K, int side, int cus) {
     const int64_t mn = (int64_t)p.tiles_n * p.tiles_m;
-    const int nk = (K + 63) / 64, tiles_w = (p.cols * side + 15) / 16, wave_t = tiles_w < p.nt ? tiles_w : p.nt;
+    const int nk = (K + 63) / 64, wtiles = (p.cols * side + 15) / 16;
     const int rounds = (int)((mn * p.ks + cus - 1) / cus);
-    const double weights = 2.0 * N * side * K, again = weights * (p.tiles_m - 1) + 2.0 * K * 64 * p.mt * mn;
-    const double mem = weights / 9e6 + again / 18e6;
-    const double lds = rounds * ((nk + p.ks - 1) / p.ks) * (128.0 * (wave_t + p.mt) + 16 * tiles_w + 64 * p.mt) / 2050.0;
-    double us = (mem > lds ? mem : lds) * (1.0 + (p.mt == 4 && p.ks == 1 ? 0.23 : 0) + (p.nt == 6 ? 0.11 : 0)) + 3.8 * rounds + 6.2 * M * N / 6e6 / rounds;
-    if (p.ks > 1) us += 1.2 + 15.0 * p.ks * M * N * side / 8e6;
+    const double weights = 2.0 * N * side * K, again = weights * (p.tiles_m - 1) + 2.0 * K * p.rows * mn;
+    const double mem = weights / 8.8e6 + again / 60e6;
+    const double step = rounds * ((nk + p.ks - 1) / p.ks) * (37.0 * p.nt + 123 * p.mt + 21.5 * wtiles + 34) / 2050.0;
+    double us = (mem > step ? mem + 0.6 * step : step + 0.6 * mem) + 2.1 * rounds + 6.7 * M * N / 6e6 / rounds + 1.3;
+    if (p.ks > 1) us += 2.4 + 14.0 * p.ks * M * N * side / 8e6;
     return us;
 }
 
@@ -411,37 +466,34 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room) {
     const int64_t small = (int64_t)((M + 127) / 128) * ((N * side + 127) / 128);
     const double tiled = nk * (0.19 + 0.34 * (double)((small + cus - 1) / cus) + 0.154 * (double)small / cus) + 3.8 + 2.6 * M * N / 6e6;
     const bool forced = g_mid_nt || g_mid_mt || g_mid_ks;
-    for (int nt = 2; nt <= 6; nt += 2)
-        for (int mt = 1; mt <= 4; mt *= 2) {
-            if ((g_mid_nt && nt != g_mid_nt) || (g_mid_mt && mt != g_mid_mt)) continue;
-            const int ns = mid_stages(nt, mt);
-            MidPlan p{};
-            p.nt = nt;
-            p.mt = mt;
-            int cap = 32 * nt / side;                      // output columns of the largest unit
-            // weight rows a stage has room for (the kilobyte behind the ring is needed where a tile has spare pieces)
-            const int max_rows = ((kLds - 1024) / ns / 128 - 64 * mt) / 16 * 16;
-            const bool whole_fits = ns * (32 * nt + 64 * mt) * 128 <= kLds;
-            if (!whole_fits) cap = max_rows / side / 16 * 16;
-            p.tiles_m = (M + 64 * mt - 1) / (64 * mt);
-            p.rows = ((M + p.tiles_m - 1) / p.tiles_m + 15) / 16 * 16;
-            // as few columns per unit as still run in the rounds that the largest unit needs
-            const int64_t whole = (int64_t)((N + cap - 1) / cap) * p.tiles_m;
-            int64_t tiles_n = (whole + cus - 1) / cus * cus / p.tiles_m;
-            p.cols = (int)((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
-            if (p.cols < 16 * nt / side) p.cols = 16 * nt / side;  // at least half of the variant's tiles
-            if (p.cols > cap) p.cols = cap;
-            if (whole_fits && (p.cols + 15) / 16 * 16 * side < 32 * nt && (p.cols + 15) / 16 * 16 * side > max_rows) p.cols = cap;
-            p.tiles_n = (N + p.cols - 1) / p.cols;
+    for (int mt = 1; mt <= 4; ++mt) {
+        if (g_mid_mt && mt != g_mid_mt) continue;
+        MidPlan p{};
+        p.tiles_m = (M + 64 * mt - 1) / (64 * mt);
+        p.rows = ((M + p.tiles_m - 1) / p.tiles_m + 15) / 16 * 16;
+        p.mt = (p.rows + 63) / 64;
+        for (int nt = 1; nt <= 6; ++nt) {
+            if (g_mid_nt && nt != g_mid_nt) continue;
             for (p.ks = 1; p.ks <= kMidMaxSlices; ++p.ks) {
+                if (g_mid_ks && p.ks != g_mid_ks && p.ks < nk) continue;
+                const int cap = 32 * nt / side;  // output columns of the largest unit
+                // as few columns per unit as still run in the rounds that the largest unit needs
+                const int64_t whole = (int64_t)((N + cap - 1) / cap) * p.tiles_m * p.ks;
+                const int64_t tiles_n = (whole + cus - 1) / cus * cus / (p.tiles_m * p.ks);
+                p.cols = (int)((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
+                if (p.cols > cap) p.cols = cap;
+                p.tiles_n = (N + p.cols - 1) / p.cols;
+                const int wtiles = (p.cols * side + 15) / 16;
+                p.nt = (wtiles + 1) / 2;
+                if (mid_lds_bytes(8, p.nt, p.mt, mid_stages(p.nt, p.mt), wtiles, p.rows / 16) > (size_t)kLds) continue;
                 if (p.ks > 1 && (int64_t)p.tiles_n * p.tiles_m * p.ks > cus + cus / 32 && !g_mid_ks) break;
                 if (p.ks > 1 && nk / p.ks < (g_mid_ks ? 1 : 6)) break;
-                if (g_mid_ks && p.ks != g_mid_ks && p.ks < nk) continue;
                 if (mid_workspace_bytes(M, N, p, swiglu) > room) break;
                 p.us = (float)mid_estimate(p, M, N, K, side, cus);
                 if ((forced || p.us < tiled) && (best.nt == 0 || p.us < best.us)) best = p;
             }
         }
+    }
     if (forced) best.us = 0.f;  // whatever else could run
     return best;
 }
@@ -468,41 +520,27 @@ size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu) {
     return p.ks > 1 ? (size_t)p.ks * M * N * (swiglu ? 2 : 1) * sizeof(float) : 0;
 }
 
-template <int EPI, int NT, int MT>
+template <int NT, int MT, bool ONCE>
 static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
     constexpr int NS = mid_stages(NT, MT);
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, 2, 4, NT, MT, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<2, 4, NT, MT, NS, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) {
             raven_host::set_error("gemm (mid): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
         }
         attr_set = true;
     }
-    const size_t lds = (size_t)NS * (a.wrows * 128 + MT * 8192) + (a.wrows < 32 * NT ? 1024 : 0);
-    RAVEN_REQUIRE(lds <= (size_t)kLds && a.wrows <= 32 * NT && a.bm <= 64 * MT, "gemm (mid): a unit of %d x %d does not fit", a.cols, a.bm);
+    const size_t lds = mid_lds_bytes(8, NT, MT, NS, a.wtiles, a.xtiles);
+    RAVEN_REQUIRE(lds <= (size_t)kLds && a.wtiles <= 2 * NT && a.wtiles > 2 * (NT - 1) && a.xtiles <= 4 * MT && a.xtiles > 4 * (MT - 1), "gemm (mid): a unit of %d x %d does not fit", a.cols, a.bm);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n * a.ks;
-    gemm_mid_kernel<EPI, 2, 4, NT, MT, NS><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
+    gemm_mid_kernel<2, 4, NT, MT, NS, ONCE><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
     return raven_host::check_launch("gemm (mid)");
 }
 
 template <int EPI>
-static int launch_mid(const MidArgs& a, const MidPlan& p, hipStream_t s, bool finish) {
-    int rc;
-    switch (p.nt * 10 + p.mt) {
-        case 21: rc = launch_mid_variant<EPI, 2, 1>(a, s); break;
-        case 22: rc = launch_mid_variant<EPI, 2, 2>(a, s); break;
-        case 24: rc = launch_mid_variant<EPI, 2, 4>(a, s); break;
-        case 41: rc = launch_mid_variant<EPI, 4, 1>(a, s); break;
-        case 42: rc = launch_mid_variant<EPI, 4, 2>(a, s); break;
-        case 44: rc = launch_mid_variant<EPI, 4, 4>(a, s); break;
-        case 61: rc = launch_mid_variant<EPI, 6, 1>(a, s); break;
-        case 62: rc = launch_mid_variant<EPI, 6, 2>(a, s); break;
-        case 64: rc = launch_mid_variant<EPI, 6, 4>(a, s); break;
-        default: RAVEN_REQUIRE(false, "gemm (mid): no variant of %d x %d tiles", p.nt, p.mt);
-    }
-    if (rc || !finish) return rc;
+static int finish_slices(const MidArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)(((int64_t)a.M * (a.N / 4) + 255) / 256));
 #define RAVEN_MID_FINISH(KS_) case KS_: gemm_mid_finish_kernel<EPI, KS_><<<grid, dim3(256), 0, s>>>(a); break;
     switch (a.ks) {
@@ -513,11 +551,32 @@ static int launch_mid(const MidArgs& a, const MidPlan& p, hipStream_t s, bool fi
     return raven_host::check_launch("gemm (mid, sums)");
 }
 
+static int launch_mid(const MidArgs& a, const MidPlan& p, hipStream_t s, bool finish) {
+    int rc;
+#define RAVEN_MID_CASE(NT_, MT_) case 10 * NT_ + MT_: rc = a.tiles_m == 1 ? launch_mid_variant<NT_, MT_, true>(a, s) : launch_mid_variant<NT_, MT_, false>(a, s); break;
+#define RAVEN_MID_ROW(NT_) RAVEN_MID_CASE(NT_, 1) RAVEN_MID_CASE(NT_, 2) RAVEN_MID_CASE(NT_, 3) RAVEN_MID_CASE(NT_, 4)
+    switch (p.nt * 10 + p.mt) {
+        RAVEN_MID_ROW(1) RAVEN_MID_ROW(2) RAVEN_MID_ROW(3) RAVEN_MID_ROW(4) RAVEN_MID_ROW(5) RAVEN_MID_ROW(6)
+        default: RAVEN_REQUIRE(false, "gemm (mid): no variant of %d x %d tiles", p.nt, p.mt);
+    }
+#undef RAVEN_MID_ROW
+#undef RAVEN_MID_CASE
+    if (rc || !finish) return rc;
+    switch (a.kind) {
+        case EPI_SWIGLU: return finish_slices<EPI_SWIGLU>(a, s);
+        case EPI_FREE: return finish_slices<EPI_FREE>(a, s);
+        case EPI_FREE_GELU: return finish_slices<EPI_FREE_GELU>(a, s);
+        case EPI_FREE_TANH: return finish_slices<EPI_FREE_TANH>(a, s);
+        default: return finish_slices<EPI_PLAIN>(a, s);
+    }
+}
+
 int mid_gemm(const ProductArgs& q, const MidPlan& p, void* workspace, hipStream_t s, int* ks_left) {
     MidArgs a{};
     a.w = q.w; a.x0 = q.x0; a.x1 = q.x1; a.residual = q.residual; a.y = q.y; a.partial = static_cast<float*>(workspace);
     a.M = q.M; a.N = q.N; a.K0 = q.K0; a.K1 = q.x1 ? q.K1 : 0; a.ldw = q.ldw; a.ldx = q.ldx; a.out_f32 = q.out_f32;
-    a.cols = p.cols; a.bm = p.rows; a.wrows = (p.cols + 15) / 16 * 16 * (q.swiglu ? 2 : 1);
+    a.kind = !q.epi ? (q.swiglu ? EPI_SWIGLU : EPI_PLAIN) : q.epi->act == RAVEN_ACT_GELU ? EPI_FREE_GELU : q.epi->act == RAVEN_ACT_TANH ? EPI_FREE_TANH : EPI_FREE;
+    a.cols = p.cols; a.bm = p.rows; a.wtiles = (p.cols * (q.swiglu ? 2 : 1) + 15) / 16; a.xtiles = p.rows / 16;
     a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.ks = p.ks;
     if (q.epi) a.epi = *q.epi;
     if (q.rope) {
@@ -527,40 +586,35 @@ int mid_gemm(const ProductArgs& q, const MidPlan& p, void* workspace, hipStream_
     RAVEN_REQUIRE(p.ks == 1 || (workspace && ((uintptr_t)workspace & 15) == 0), "gemm (mid): no workspace for the K slices");
     const bool finish = p.ks > 1 && !ks_left;
     if (ks_left) *ks_left = p.ks > 1 ? p.ks : 0;
-    if (q.epi && q.epi->act == RAVEN_ACT_GELU) return launch_mid<EPI_FREE_GELU>(a, p, s, finish);
-    if (q.epi && q.epi->act == RAVEN_ACT_TANH) return launch_mid<EPI_FREE_TANH>(a, p, s, finish);
-    if (q.epi) return launch_mid<EPI_FREE>(a, p, s, finish);
-    if (q.swiglu) return launch_mid<EPI_SWIGLU>(a, p, s, finish);
-    return launch_mid<EPI_PLAIN>(a, p, s, finish);
+    return launch_mid(a, p, s, finish);
 }
 
-template <int EPI, int WN, int WM, int NT, int MT, int NS>
+template <int WN, int WM, int NT, int MT, int NS>
 static int launch_grouped(const MidArgs& a, hipStream_t s) {
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, WN, WM, NT, MT, NS, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<WN, WM, NT, MT, NS, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) {
             raven_host::set_error("gemm (grouped): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
         }
         attr_set = true;
     }
-    const size_t lds = (size_t)NS * (a.wrows + 16 * WM * MT) * 128 + (a.wrows < 16 * WN * NT ? 1024 : 0);
-    RAVEN_REQUIRE(lds <= (size_t)kLds && a.wrows <= 16 * WN * NT, "gemm (grouped): a unit of %d columns does not fit", a.cols);
+    const size_t lds = mid_lds_bytes(WN * WM, NT, MT, NS, a.wtiles, a.xtiles);
+    RAVEN_REQUIRE(lds <= (size_t)kLds && a.wtiles <= WN * NT && a.wtiles >= WN * NT / 2 && a.xtiles == WM * MT, "gemm (grouped): a unit of %d columns does not fit", a.cols);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n;
     RAVEN_REQUIRE(units < (1 << 28), "gemm (grouped): too many units");
-    gemm_mid_kernel<EPI, WN, WM, NT, MT, NS, true><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(64 * WN * WM), lds, s>>>(a);
+    gemm_mid_kernel<WN, WM, NT, MT, NS, false, true><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(64 * WN * WM), lds, s>>>(a);
     return raven_host::check_launch("gemm (grouped)");
 }
 
 // Tiles of 32 rows: four waves side by side along the weight rows -- with few token rows the eight waves of the larger tiles would
 // read mostly rows that do not exist out of LDS --, four stages of 20 KB, two workgroups per CU, so that one streams while the
 // other fills its ring or stores (a unit of an expert of 768 channels has 12 to 32 K steps).
-template <int EPI>
 static int launch_grouped_rows(const MidArgs& a, hipStream_t s) {
     switch (a.bm) {
-        case 32: return launch_grouped<EPI, 4, 1, 2, 2, 4>(a, s);
-        case 64: return launch_grouped<EPI, 2, 4, 4, 1, 3>(a, s);
+        case 32: return launch_grouped<4, 1, 2, 2, 4>(a, s);
+        case 64: return launch_grouped<2, 4, 4, 1, 3>(a, s);
         default: RAVEN_REQUIRE(false, "gemm (grouped): tiles of %d rows", a.bm);
     }
 }
@@ -578,12 +632,13 @@ int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int
     const int tiles_n = (N + cap - 1) / cap;
     a.cols = ((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
     if (a.cols < cap / 2) a.cols = cap / 2;
-    a.wrows = (a.cols + 15) / 16 * 16 * side;
+    a.kind = swiglu ? EPI_SWIGLU : EPI_FREE;
+    a.wtiles = (a.cols * side + 15) / 16;
     a.tiles_n = (N + a.cols - 1) / a.cols;
-    a.bm = g.tile_rows; a.tiles_m = g.n_tiles; a.ks = 1;
+    a.bm = g.tile_rows; a.xtiles = (g.tile_rows + 15) / 16; a.tiles_m = g.n_tiles; a.ks = 1;
     a.epi.scale = 1.f;
     a.groups = g;
-    return swiglu ? launch_grouped_rows<EPI_SWIGLU>(a, s) : launch_grouped_rows<EPI_FREE>(a, s);
+    return launch_grouped_rows(a, s);
 }
 
 }  // namespace raven

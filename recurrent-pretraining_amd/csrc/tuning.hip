@@ -36,8 +36,8 @@ extern "C" int raven_set_tuning(const char* key, int32_t value) {
     else if (k == "gemm_tiled_variant" && value >= 0 && value <= 3) g_tiled_variant = value;
     else if (k == "gemm_tiled_split_tail" && (value == 0 || value == 1)) g_tiled_split_tail = value;
     else if (k == "gemm_mid" && (value == 0 || value == 1)) g_mid = value;
-    else if (k == "gemm_mid_nt" && (value == 0 || value == 2 || value == 4 || value == 6)) g_mid_nt = value;
-    else if (k == "gemm_mid_mt" && (value == 0 || value == 1 || value == 2 || value == 4)) g_mid_mt = value;
+    else if (k == "gemm_mid_nt" && value >= 0 && value <= 6) g_mid_nt = value;
+    else if (k == "gemm_mid_mt" && value >= 0 && value <= 4) g_mid_mt = value;
     else if (k == "gemm_mid_ks" && value >= 0 && value <= 8) g_mid_ks = value;
     else RAVEN_REQUIRE(set_gemv1_tuning(key, value) == 0 || set_skinny_tuning(key, value) == 0, "set_tuning: unknown key %s", key);
     return 0;

@@ -175,6 +175,24 @@ def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, 
         assert torch.equal(pkg.hip.linear(x, w, workspace=ws), pkg.hip.linear(x, w, workspace=ws))
 
 
+@pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("M", [35, 80, 143, 200, 300])
+def test_units_with_any_number_of_tiles(pkg, tuned, nt, M):
+    """gemm_mid.hip: units of every number of weight tiles and of 3 to 13 token tiles, so that waves get one tile more or less than others, or none;
+    weight rows read by one unit (up to 256 rows) and by two; K of 4 steps and of 11, the last one partly filled."""
+    dt = torch.bfloat16
+    for N in (32 * nt - 24, 32 * nt):
+        for K in (232, 680):
+            tuned(gemm_mid_nt=nt, gemm_mid_mt=min(4, (M + 63) // 64), gemm_mid_ks=1)
+            ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+            x, w = _gpu_randn((M, K), 760 + M), _gpu_randn((N, K), 761 + N, 0.05)
+            check(pkg.hip.linear(x, w, workspace=ws), (x.float() @ w.float().T).to(dt), dt, f"{M} x {N} x {K}")
+            half = max(8, N // 2 // 8 * 8)
+            fc = _gpu_randn((2 * half, K), 762, 0.05)
+            u = (x.float() @ fc.float().T).to(dt).float()
+            check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :half]).to(dt).float() * u[:, half:]).to(dt), dt, f"{M} x {half} x {K}, SwiGLU", ulps=ULPS_SWIGLU)
+
+
 @pytest.mark.parametrize("ks", [1, 3])
 @pytest.mark.parametrize("nt,mt", [(2, 1), (4, 2), (6, 4)])
 def test_infinities_stay_in_their_rows_and_columns(pkg, tuned, nt, mt, ks):
