@@ -287,6 +287,21 @@ int raven_paged_decode_blocks(const raven_dims* dims, const void* adapter_w, con
                               const float* freqs, const raven_paged_kv* kv, int32_t n_iterations, int32_t B,
                               void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same for the new rows of B sequences, prompt chunks and decode rows together (bf16, head_dim 64 / 96 / 128): x_in, embeds, x_out [T, h];
+ * positions and slot_mapping [T] and q_start [B + 1] in device memory, as raven_paged_qkv_rope_append and
+ * raven_paged_prefill_attention_rows take them; kv->block_table [B, max_blocks], kv->seq_lens [B] (new rows included).
+ * workspace: raven_block_workspace_bytes(dims, T). */
+typedef struct raven_paged_rows {
+    const int64_t* positions;
+    const int64_t* slot_mapping;
+    const int32_t* q_start;
+    int32_t T, B, max_q_len;
+} raven_paged_rows;
+int raven_paged_chunk_blocks(const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,
+                             int32_t n_blocks, const void* ln_f, const void* x_in, const void* embeds, void* x_out,
+                             const float* freqs, const raven_paged_kv* kv, const raven_paged_rows* rows, int32_t n_iterations,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
 /* Decode fast path for ONE token row, one launch:
  *     x  = norm_a ? T(rmsnorm(x0) * norm_a) : x0      -> stored to xa_out when non-NULL
  *     x  = norm_b ? T(rmsnorm(x)  * norm_b) : x

@@ -645,6 +645,12 @@ extern "C" int raven_prefill_attention(const void* q, void* y, const raven_kv_ca
     return raven::prefill_attention_pitched(q, y, n_heads * head_dim, cache, slot, B, S, pos0, pos_dev, n_heads, head_dim, dtype, stream);
 }
 
+namespace raven {
+int paged_prefill_attention_pitched(const void* q, void* y, int ldy, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                                    const int32_t* seq_lens, const int32_t* q_start, int32_t B, int32_t T, int32_t max_q_len, int32_t max_blocks,
+                                    int32_t block_size, int32_t kv_layout, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
+}
+
 extern "C" int raven_paged_prefill_attention(const void* q, void* y, const void* k_cache, const void* v_cache,
                                              const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start, int32_t B,
                                              int32_t max_q_len, int32_t max_blocks, int32_t block_size, int32_t kv_layout,
@@ -657,7 +663,16 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
                                                   const int32_t* block_table, const int32_t* seq_lens, const int32_t* q_start, int32_t B, int32_t T,
                                                   int32_t max_q_len, int32_t max_blocks, int32_t block_size, int32_t kv_layout,
                                                   int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream) {
-    using namespace raven;
+    return raven::paged_prefill_attention_pitched(q, y, n_heads * head_dim, k_cache, v_cache, block_table, seq_lens, q_start, B, T, max_q_len, max_blocks,
+                                                  block_size, kv_layout, n_heads, head_dim, dtype, stream);
+}
+
+namespace raven {
+// raven_paged_prefill_attention_rows with the rows of y ldy elements apart (>= n_heads * head_dim)
+int paged_prefill_attention_pitched(const void* q, void* y, int ldy, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                                    const int32_t* seq_lens, const int32_t* q_start, int32_t B, int32_t T, int32_t max_q_len, int32_t max_blocks,
+                                    int32_t block_size, int32_t kv_layout, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream) {
+    RAVEN_REQUIRE(ldy >= n_heads * head_dim && ldy % 8 == 0, "paged_prefill_attention: bad output row pitch %d", ldy);
     RAVEN_REQUIRE(dtype == RAVEN_BF16, "paged_prefill_attention: bf16 only (dtype %d)", dtype);
     RAVEN_REQUIRE(head_dim == 64 || head_dim == 96 || head_dim == 128, "paged_prefill_attention: head_dim %d not in {64, 96, 128}", head_dim);
     RAVEN_REQUIRE(kv_layout == RAVEN_PAGED_NHD || kv_layout == RAVEN_PAGED_HND, "paged_prefill_attention: unknown kv_layout %d", kv_layout);
@@ -668,7 +683,7 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
     PrefillArgs a{};
     a.q = static_cast<const bf16*>(q);
     a.y = static_cast<bf16*>(y);
-    a.ldy = n_heads * head_dim;
+    a.ldy = ldy;
     a.k = static_cast<const bf16*>(k_cache);
     a.v = static_cast<const bf16*>(v_cache);
     a.nh = n_heads; a.hd = head_dim;
@@ -721,3 +736,4 @@ extern "C" int raven_paged_prefill_attention_rows(const void* q, void* y, const 
 #undef RAVEN_PREFILL
     return raven_host::check_launch("paged_prefill_attention");
 }
+}  // namespace raven

@@ -47,6 +47,9 @@ int rmsnorm_pitched(const void* x, const void* residual, const void* weight, voi
                     void* y2, int ldy2, int64_t rows, int32_t dim, float eps, int32_t dtype, void* stream);
 int prefill_attention_pitched(const void* q, void* y, int ldy, const raven_kv_cache* cache, int32_t slot, int32_t B, int32_t S,
                               int32_t pos0, const int32_t* pos_dev, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
+int paged_prefill_attention_pitched(const void* q, void* y, int ldy, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                                    const int32_t* seq_lens, const int32_t* q_start, int32_t B, int32_t T, int32_t max_q_len, int32_t max_blocks,
+                                    int32_t block_size, int32_t kv_layout, int32_t n_heads, int32_t head_dim, int32_t dtype, void* stream);
 
 // y = round(round(x W^T) + residual), then RMSNorm(weight) -> out1 and RMSNorm(weight2) of that -> out2 (either may be
 // null): one launch fewer where the product is K-split (the norm launch adds the slices).  ldx: elements between two rows of x (chunks)
@@ -156,9 +159,9 @@ static bool chunk_on_matrix_cores(const raven_dims* d, const raven_kv_cache* cac
 // attention output, which the products over many rows read, are laid out with rows padded to whole lines (the pad
 // is never read: the products' K stays n_embd).  The row pitch of these, decided once for all blocks of a call.
 static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const raven_block_weights* blocks, int n_blocks, const void* x_in,
-                           const raven_kv_cache* cache, int M, int S, bool paged) {
+                           const raven_kv_cache* cache, int M, int S, bool paged, const raven_paged_rows* rows) {
     const int h = d->n_embd, dt = d->dtype;
-    if (!g_pad_chunk_rows || !chunk_on_matrix_cores(d, cache, S, paged) || s.ld_pad == h || M < g_tiled_min_rows) return h;
+    if (!g_pad_chunk_rows || !(rows || chunk_on_matrix_cores(d, cache, S, paged)) || s.ld_pad == h || M < g_tiled_min_rows) return h;
     bool aligned = raven_host::aligned16(x_in);
     for (int j = 0; j < n_blocks; ++j) aligned = aligned && raven_host::aligned16(blocks[j].wqkv, blocks[j].proj, blocks[j].fc);
     const bool pad = tiled_gemm_fits(M, 3 * h, h, 0, dt, 0, s.lin_ws_bytes, aligned) && tiled_gemm_fits(M, h, h, 0, dt, 0, s.lin_ws_bytes, aligned) &&
@@ -172,7 +175,7 @@ static int chunk_row_pitch(const raven_dims* d, const BlockScratch& s, const rav
 static int run_block(const raven_dims* d, const raven_block_weights* w, const BlockScratch& s, bool n1_ready,
                      const void* x_in, void* y_out, const void* tail_w, void* tail_out, const float* freqs,
                      const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, void* stream,
-                     const raven_paged_kv* paged, int layer, int ld_decode, int ld_chunk) {
+                     const raven_paged_kv* paged, const raven_paged_rows* rows, int layer, int ld_decode, int ld_chunk) {
     const int M = B * S, h = d->n_embd, I = d->intermediate, dt = d->dtype;
     hipStream_t hs = static_cast<hipStream_t>(stream);
     int rc;
@@ -205,7 +208,13 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
         else rc = raven_linear(s.n1, nullptr, w->wqkv, nullptr, s.qkv, M, 3 * h, h, 0, 0, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
         if (rc) return rc;
     }
-    if (paged) {   // decode over block-paged caches, every sequence at its own position
+    if (rows) {    // rows of any sequences over block-paged caches
+        if ((rc = raven_paged_qkv_rope_append(s.qkv, w->qk_bias, freqs, rows->positions, rows->slot_mapping, s.q, paged->k_caches[layer],
+                                              paged->v_caches[layer], M, d->n_heads, d->head_dim, paged->block_size, paged->kv_layout, dt, stream))) return rc;
+        if ((rc = paged_prefill_attention_pitched(s.q, s.ya, pad ? ld : h, paged->k_caches[layer], paged->v_caches[layer], paged->block_table, paged->seq_lens,
+                                                  rows->q_start, rows->B, M, rows->max_q_len, paged->max_blocks, paged->block_size, paged->kv_layout,
+                                                  d->n_heads, d->head_dim, dt, stream))) return rc;
+    } else if (paged) {  // decode over block-paged caches, every sequence at its own position
         if ((rc = raven_paged_qkv_attention_decode(s.qkv, w->qk_bias, freqs, s.ya, paged->k_caches[layer], paged->v_caches[layer],
                                                    paged->block_table, paged->seq_lens, B, paged->max_blocks, paged->block_size,
                                                    paged->kv_layout, paged->max_seq_len, d->n_heads, d->head_dim, dt, s.attn_ws, s.attn_ws_bytes, stream))) return rc;
@@ -292,20 +301,21 @@ extern "C" int raven_sandwich_block(const raven_dims* dims, const raven_block_we
         if (int rc = run_block_one_row(dims, w, s, x_in, nullptr, freqs, cache, slot, pos0, pos_dev, stream)) return rc;
         return close_one_row(dims, s, w->norm_4, ln_f, x_out, stream);
     }
-    const int ld_decode = decode_row_pitch(dims, s, w, 1, B * S, S, false), ld_chunk = chunk_row_pitch(dims, s, w, 1, x_in, cache, B * S, S, false);
-    if (ln_f) return run_block(dims, w, s, false, x_in, nullptr, ln_f, x_out, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode, ld_chunk);
-    return run_block(dims, w, s, false, x_in, x_out, nullptr, nullptr, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, 0, ld_decode, ld_chunk);
+    const int ld_decode = decode_row_pitch(dims, s, w, 1, B * S, S, false), ld_chunk = chunk_row_pitch(dims, s, w, 1, x_in, cache, B * S, S, false, nullptr);
+    if (ln_f) return run_block(dims, w, s, false, x_in, nullptr, ln_f, x_out, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, nullptr, 0, ld_decode, ld_chunk);
+    return run_block(dims, w, s, false, x_in, x_out, nullptr, nullptr, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, nullptr, 0, ld_decode, ld_chunk);
 }
 
 namespace raven {
 
 // n_iterations x ([adapter product] + n_blocks blocks), the closing norm(s) at the end.  The K/V of block j live either
 // in slot slots[it * n_blocks + j] of a contiguous cache (all sequences at position pos0 / *pos_dev) or, with `paged`,
-// in the j-th block-paged cache (every sequence at its own position, the same cache in every iteration).
+// in the j-th block-paged cache (every sequence at its own position, the same cache in every iteration); with `rows` the B * 1 rows belong
+// to the sequences that it describes.
 static int iterations_impl(const char* who, const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,
                            int32_t n_blocks, const void* ln_f, const void* state_in, const void* embeds, void* state_out,
                            const float* freqs, const raven_kv_cache* cache, const int32_t* slots, const raven_paged_kv* paged,
-                           int32_t n_iterations, int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace,
+                           const raven_paged_rows* rows, int32_t n_iterations, int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace,
                            size_t workspace_bytes, void* stream) {
     if (int rc = check_dims(who, dims)) return rc;
     RAVEN_REQUIRE(state_in && state_out && freqs && (slots || paged), "%s: null pointer", who);
@@ -326,7 +336,7 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
     hipStream_t hs = static_cast<hipStream_t>(stream);
 
     int rc;
-    if (M == 1 && one_row_fits(dims)) {
+    if (M == 1 && !rows && one_row_fits(dims)) {
         // One row: between two iterations the last block's closing norm_4 is the prologue of the next adapter product
         // (no launch of its own); only the last iteration closes with a norm launch (norm_4, then ln_f if asked for).
         // The embedding half of the adapter product is the same in every recurrence: with two or more of them its fp32
@@ -364,7 +374,7 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
         if ((rc = linear_column_block(embeds, static_cast<const char*>(adapter_w) + (size_t)h * 2, 2 * h, nullptr, s.e_sums, 1, M, h, h,
                                       s.lin_ws, s.lin_ws_bytes, hs))) return rc;
     const int ld_decode = decode_row_pitch(dims, s, blocks, n_blocks, M, S, paged != nullptr);
-    const int ld_chunk = chunk_row_pitch(dims, s, blocks, n_blocks, state_in, cache, M, S, paged != nullptr);
+    const int ld_chunk = chunk_row_pitch(dims, s, blocks, n_blocks, state_in, cache, M, S, paged != nullptr, rows);
     const int ld_n1 = ld_decode ? ld_decode : ld_chunk;  // rows of norm_1's output as run_block reads them
     for (int it = 0; it < n_iterations; ++it) {
         const int32_t* sl = slots ? slots + (size_t)it * n_blocks : nullptr;
@@ -392,7 +402,7 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
             const void* tail_w = last ? lnw : blocks[j + 1].norm_1;
             void* tail_out = last ? (lnw ? state_out : nullptr) : s.n1;
             if ((rc = run_block(dims, &blocks[j], s, j > 0 || n1_ready, x_in, y_out, tail_w, tail_out, freqs, cache, sl ? sl[j] : 0, B, S, pos0,
-                                pos_dev, stream, paged, j, ld_decode, ld_chunk))) return rc;
+                                pos_dev, stream, paged, rows, j, ld_decode, ld_chunk))) return rc;
         }
     }
     return 0;
@@ -407,7 +417,7 @@ extern "C" int raven_core_iterations(const raven_dims* dims, const void* adapter
                                      void* workspace, size_t workspace_bytes, void* stream) {
     RAVEN_REQUIRE(adapter_w && embeds && slots, "core_iterations: null pointer");
     return raven::iterations_impl("core_iterations", dims, adapter_w, blocks, n_blocks, ln_f, state_in, embeds, state_out, freqs, cache,
-                                  slots, nullptr, n_iterations, B, S, pos0, pos_dev, workspace, workspace_bytes, stream);
+                                  slots, nullptr, nullptr, n_iterations, B, S, pos0, pos_dev, workspace, workspace_bytes, stream);
 }
 
 extern "C" int raven_paged_decode_blocks(const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,
@@ -419,7 +429,21 @@ extern "C" int raven_paged_decode_blocks(const raven_dims* dims, const void* ada
     for (int j = 0; j < n_blocks; ++j)
         RAVEN_REQUIRE(kv->k_caches[j] && kv->v_caches[j], "paged_decode_blocks: null cache for block %d", j);
     return raven::iterations_impl("paged_decode_blocks", dims, adapter_w, blocks, n_blocks, ln_f, x_in, embeds, x_out, freqs, nullptr,
-                                  nullptr, kv, n_iterations, B, 1, 0, nullptr, workspace, workspace_bytes, stream);
+                                  nullptr, kv, nullptr, n_iterations, B, 1, 0, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int raven_paged_chunk_blocks(const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,
+                                        int32_t n_blocks, const void* ln_f, const void* x_in, const void* embeds, void* x_out,
+                                        const float* freqs, const raven_paged_kv* kv, const raven_paged_rows* rows, int32_t n_iterations,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+    RAVEN_REQUIRE(kv && kv->k_caches && kv->v_caches && kv->block_table && kv->seq_lens, "paged_chunk_blocks: null cache description");
+    RAVEN_REQUIRE(rows && rows->positions && rows->slot_mapping && rows->q_start && rows->T > 0 && rows->B > 0, "paged_chunk_blocks: null or empty row description");
+    RAVEN_REQUIRE(dims && dims->dtype == RAVEN_BF16, "paged_chunk_blocks: bf16 only");
+    RAVEN_REQUIRE(n_blocks >= 1 && blocks, "paged_chunk_blocks: needs at least one block (got %d)", n_blocks);
+    for (int j = 0; j < n_blocks; ++j)
+        RAVEN_REQUIRE(kv->k_caches[j] && kv->v_caches[j], "paged_chunk_blocks: null cache for block %d", j);
+    return raven::iterations_impl("paged_chunk_blocks", dims, adapter_w, blocks, n_blocks, ln_f, x_in, embeds, x_out, freqs, nullptr,
+                                  nullptr, kv, rows, n_iterations, rows->T, 1, 0, nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int raven_core_iteration(const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,

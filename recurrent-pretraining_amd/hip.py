@@ -46,6 +46,10 @@ class PagedKV(C.Structure):
                 ("kv_layout", C.c_int32)]
 
 
+class PagedRows(C.Structure):
+    _fields_ = [("positions", C.c_void_p), ("slot_mapping", C.c_void_p), ("q_start", C.c_void_p), ("T", C.c_int32), ("B", C.c_int32), ("max_q_len", C.c_int32)]
+
+
 class Epilogue(C.Structure):
     _fields_ = [("bias", C.c_void_p), ("residual", C.c_void_p), ("scale", C.c_float), ("act", C.c_int32), ("out_f32", C.c_int32)]
 
@@ -163,6 +167,8 @@ SIGNATURES = {
     "raven_paged_prefill_attention_rows": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _VP]),
     "raven_paged_decode_blocks": (C.c_int, [C.POINTER(Dims), _VP, C.POINTER(BlockWeights), _I32, _VP, _VP, _VP, _VP, _VP,
                                             C.POINTER(PagedKV), _I32, _I32, _VP, _SZ, _VP]),
+    "raven_paged_chunk_blocks": (C.c_int, [C.POINTER(Dims), _VP, C.POINTER(BlockWeights), _I32, _VP, _VP, _VP, _VP, _VP,
+                                           C.POINTER(PagedKV), C.POINTER(PagedRows), _I32, _VP, _SZ, _VP]),
     "raven_linear_epilogue": (C.c_int, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, C.POINTER(Epilogue), _I32, _VP, _SZ, _VP]),
     "raven_gemv_stream": (C.c_int, [_VP, _VP, _I32, _F, _VP, _VP, _I32, _I32, C.POINTER(Epilogue), _I32, _VP]),
     "raven_norm_conv": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _F, _I32, _VP, _I32, _VP]),
@@ -580,9 +586,9 @@ def advance_pos(pos_dev, delta=1):
     _check(load().raven_advance_pos(_ptr(pos_dev, "pos_dev", torch.int32), delta, _stream()), "raven_advance_pos")
 
 
-def block_workspace(dims: Dims, M: int, device) -> torch.Tensor:
+def block_workspace(dims: Dims, M: int, device, clear: bool = True) -> torch.Tensor:
     n = load().raven_block_workspace_bytes(C.byref(dims), M)
-    return torch.zeros(max(n, 256), dtype=torch.uint8, device=device)
+    return (torch.zeros if clear else torch.empty)(max(n, 256), dtype=torch.uint8, device=device)
 
 
 def sandwich_block(dims: Dims, w: BlockWeights, x_in, x_out, freqs, cache: KVCache, slot, B, S, pos0, workspace,
@@ -625,7 +631,7 @@ def core_iterations(dims: Dims, adapter_w, blocks, state_in, embeds, state_out, 
 
 def make_paged_kv(k_caches, v_caches, block_table, seq_lens, max_seq_len: int, layout: int = PAGED_NHD) -> PagedKV:
     """k_caches / v_caches: one paged cache tensor (as in paged_kv_append) per block of the stack; block_table [B, max_blocks] and
-    seq_lens [B] int32 on the GPU.  The returned structure holds pointers only: keep the tensors alive."""
+    seq_lens [B] int32 on the GPU.  The structure holds pointers, and this object the tensors behind them."""
     if len(k_caches) != len(v_caches) or not k_caches:
         raise RavenHipError("make_paged_kv: one key and one value cache per block")
     shape, dt = k_caches[0].shape, k_caches[0].dtype
@@ -638,7 +644,7 @@ def make_paged_kv(k_caches, v_caches, block_table, seq_lens, max_seq_len: int, l
         raise RavenHipError("make_paged_kv: block_table [B, max_blocks], seq_lens [B]")
     kv = PagedKV(C.cast(ka, C.POINTER(C.c_void_p)), C.cast(va, C.POINTER(C.c_void_p)), _ptr(block_table, "block_table", torch.int32),
                  _ptr(seq_lens, "seq_lens", torch.int32), block_table.shape[1], _paged_dims(k_caches[0], layout)[0], int(max_seq_len), layout)
-    kv._keep = (ka, va)  # the pointer arrays live in host memory owned by this object
+    kv._keep = (ka, va, list(k_caches), list(v_caches), block_table, seq_lens)
     return kv
 
 
@@ -650,6 +656,21 @@ def paged_decode_blocks(dims: Dims, blocks, x_in, x_out, freqs, kv: PagedKV, B, 
         _ptr(embeds, "embeds", x_in.dtype), _ptr(x_out, "x_out", x_in.dtype), _ptr(freqs, "freqs", torch.float32), C.byref(kv),
         int(n_iterations), B, _ptr(workspace, "workspace", torch.uint8), workspace.numel(), _stream())
     _check(rc, "raven_paged_decode_blocks")
+    return x_out
+
+
+def paged_chunk_blocks(dims: Dims, blocks, x_in, x_out, freqs, kv: PagedKV, positions, slot_mapping, q_start, max_q_len, workspace, adapter_w=None,
+                       embeds=None, n_iterations=1, ln_f=None):
+    """paged_decode_blocks for the new rows x_in [T, h] of several sequences, as paged_qkv_rope_append and paged_prefill_attention describe them."""
+    T, B = x_in.shape[0], q_start.shape[0] - 1
+    if positions.shape != (T,) or slot_mapping.shape != (T,) or x_out.shape != x_in.shape:
+        raise RavenHipError("paged_chunk_blocks: positions [T], slot_mapping [T] and x_out must match x_in [T, h]")
+    rows = PagedRows(_ptr(positions, "positions", torch.int64), _ptr(slot_mapping, "slot_mapping", torch.int64), _ptr(q_start, "q_start", torch.int32), T, B, int(max_q_len))
+    rc = load().raven_paged_chunk_blocks(
+        C.byref(dims), _ptr(adapter_w, "adapter_w", x_in.dtype), blocks, len(blocks), _ptr(ln_f, "ln_f", x_in.dtype), _ptr(x_in, "x_in"),
+        _ptr(embeds, "embeds", x_in.dtype), _ptr(x_out, "x_out", x_in.dtype), _ptr(freqs, "freqs", torch.float32), C.byref(kv), C.byref(rows),
+        int(n_iterations), _ptr(workspace, "workspace", torch.uint8), workspace.numel(), _stream())
+    _check(rc, "raven_paged_chunk_blocks")
     return x_out
 
 

@@ -11,8 +11,8 @@ across the batch, raven_modeling_minimal.py:660-665).
 
 The arithmetic of a step is the contiguous decode path's: the same SandwichBlock launches with the paged decode-attention
 kernel in place of the contiguous one (raven_paged_decode_blocks).  forward_tokens takes any mix of prompt chunks and decode
-rows of several sequences, flattened as a serving engine hands them over, through the paged chunk kernels
-(raven_paged_qkv_rope_append, raven_paged_prefill_attention)."""
+rows of several sequences, flattened as a serving engine hands them over, through the same launches with the paged chunk kernels
+(raven_paged_chunk_blocks)."""
 
 from __future__ import annotations
 
@@ -94,21 +94,6 @@ class PagedDecoder:
 
     # ------------------------------------------------------------------ rows of any sequences (prompt chunks, decode rows)
 
-    def _token_block(self, blk, f: int, x: torch.Tensor, meta, ws: torch.Tensor) -> torch.Tensor:
-        """One SandwichBlock (vllm/raven_vllm.py:289-294 around its attention layer, :184-203) on flat rows, flat layer f."""
-        eps = self.cfg.norm_eps
-        positions, slots, table, lens, q_start, max_q = meta
-        n1 = hip.rmsnorm_residual(x, blk.norm_1.weight, eps)[0]
-        qkv = hip.linear(n1, blk.attn.Wqkv.weight, workspace=ws)
-        bias = blk.attn.qk_bias if hasattr(blk.attn, "qk_bias") else None
-        q = hip.paged_qkv_rope_append(qkv, bias, self.model._natives()["freqs"], positions, slots, self.k[f], self.v[f], layout=self.layout)
-        ya = hip.paged_prefill_attention(q, self.k[f], self.v[f], table, lens, q_start, max_q, layout=self.layout)
-        # the residual adds (RMM:534-535) and the SwiGLU (RMM:507-508) ride in the epilogues of the products
-        x1 = hip.linear(ya, blk.attn.proj.weight, residual=x, workspace=ws)
-        x2, _, n3 = hip.rmsnorm_residual(x1, blk.norm_2.weight, eps, weight2=blk.norm_3.weight)
-        x3 = hip.linear(hip.linear(n3, blk.mlp.fc.weight, swiglu=True, workspace=ws), blk.mlp.proj.weight, residual=x2, workspace=ws)
-        return hip.rmsnorm_residual(x3, blk.norm_4.weight, eps)[0]
-
     @torch.no_grad()
     def forward_tokens(self, input_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor, block_table: torch.Tensor,
                        seq_lens: torch.Tensor, query_start_loc: torch.Tensor, max_query_len: int,
@@ -128,27 +113,36 @@ class PagedDecoder:
         if self._wants_check(check_bounds, block_table, seq_lens, positions, slot_mapping):
             self._check_pages(block_table, seq_lens, positions, slot_mapping)
         dev = m.device
-        meta = (positions.to(dev, torch.int64), slot_mapping.to(dev, torch.int64), block_table.to(dev, torch.int32).contiguous(),
-                seq_lens.to(dev, torch.int32), query_start_loc.to(dev, torch.int32), int(max_query_len))
+        positions, slots = positions.to(dev, torch.int64), slot_mapping.to(dev, torch.int64)
+        table, lens = block_table.to(dev, torch.int32).contiguous(), seq_lens.to(dev, torch.int32)
+        q_start, max_q = query_start_loc.to(dev, torch.int32), int(max_query_len)
         n_pre, n_core = cfg.n_layers_in_prelude, cfg.n_layers_in_recurrent_block
-        ws = hip.linear_workspace(T, max(3 * cfg.n_embd, 2 * cfg.intermediate_size), dev)  # K slices of the products
+        if T >= 17 and m.pack_chunk_weights:
+            m.pack_weights()  # the products read Wqkv, attn.proj and mlp.fc through their line-aligned copies
+        dims, freqs = m._natives()["dims"], m._natives()["freqs"]
+        ws = hip.block_workspace(dims, T, dev, clear=False)
         x = hip.embed(t.wte.weight, input_ids.reshape(-1).to(dev, torch.int64).contiguous(), m.emb_scale)
-        for i in range(n_pre):
-            x = self._token_block(t.prelude[i], i, x, meta, ws)
-        embeds = x
+
+        def blocks(stack, first, x, **core):  # a stack of SandwichBlocks (vllm/raven_vllm.py:289-294) on flat rows, flat layers from `first` on
+            if T == 0 or len(stack) == 0:
+                return x
+            last, weights = first + len(stack), (hip.BlockWeights * len(stack))(*[b.native() for b in stack])
+            kv = hip.make_paged_kv(self.k[first:last], self.v[first:last], table, lens, table.shape[1] * self.block_size, layout=self.layout)
+            return hip.paged_chunk_blocks(dims, weights, x, torch.empty_like(x), freqs, kv, positions, slots, q_start, max_q, ws, **core)
+
+        embeds = x = blocks(t.prelude, 0, x)
         if input_states is None:
             state = m.initialize_state(embeds, init_scale) if init_scale > 0 else torch.zeros_like(embeds)
         else:
             state = input_states.reshape(T, -1).to(dev, m.dtype)
-        for _ in range(self.r):
-            state = hip.linear(state, t.adapter.weight, x1=embeds, workspace=ws)  # the concat of RMM:776 as two K segments
-            for j in range(n_core):
-                state = self._token_block(t.core_block[j], n_pre + j, state, meta, ws)
-        latents = hip.rmsnorm_residual(state, t.ln_f.weight, cfg.norm_eps)[0]
-        x = latents
-        for i in range(cfg.n_layers_in_coda):
-            x = self._token_block(t.coda[i], n_pre + n_core + i, x, meta, ws)
-        x = hip.rmsnorm_residual(x, t.ln_f.weight, cfg.norm_eps)[0]
+        if self.r > 0 and T > 0:
+            latents = blocks(t.core_block, n_pre, state.contiguous(), adapter_w=t.adapter.weight, embeds=embeds, n_iterations=self.r, ln_f=t.ln_f.weight)
+        else:
+            latents = hip.rmsnorm_residual(state, t.ln_f.weight, cfg.norm_eps)[0]
+        if cfg.n_layers_in_coda > 0 and T > 0:
+            x = blocks(t.coda, n_pre + n_core, latents, ln_f=t.ln_f.weight)
+        else:
+            x = hip.rmsnorm_residual(latents, t.ln_f.weight, cfg.norm_eps)[0]
         logits = hip.gemm(x, m.lm_head.weight, out_f32=True)
         return logits, latents
 

@@ -1389,3 +1389,66 @@ def test_positions_and_pages_are_bounded_on_the_host(pkg, small242):
     cache._seen_tokens = model.config.block_size
     with pytest.raises(ValueError, match="RoPE table"):
         runner.step(torch.zeros(1, dtype=torch.int64, device="cuda"), None, 0.0)
+
+
+@pytest.mark.parametrize("chunk", [1, 14, 30, 90])
+def test_mixed_rows_on_pages_equal_the_launches_one_by_one(pkg, tuned, chunk):
+    """forward_tokens as one native call per stack (raven_paged_chunk_blocks) at an n_embd whose rows are not whole cache lines: padded rows and
+    line-aligned weight copies change no bit (17 to 32 rows: the order of sums), and each block is the sequence of single calls it stands for."""
+    hip, dt = pkg.hip, torch.bfloat16
+    cfg = pkg.RavenConfig(n_embd=288, n_heads=3, n_layers=5, n_layers_in_prelude=1, n_layers_in_recurrent_block=2, n_layers_in_coda=2,
+                          intermediate_size=480, vocab_size=512, mean_recurrence=2)
+    torch.manual_seed(17)
+    model = pkg.RavenForCausalLM(cfg, device="cuda", dtype=dt)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0.0, 0.05)
+    lens, news = (9, 40, 3), (1, 1, chunk)
+    T, bs = sum(news), 8
+    width = max((n + s + bs - 1) // bs for n, s in zip(lens, news))
+    table = torch.randperm(3 * width)[:3 * width].view(3, width).to(torch.int32)
+    pos = torch.cat([torch.arange(n, n + s) for n, s in zip(lens, news)])
+    owner = torch.cat([torch.full((s,), i) for i, s in enumerate(news)])
+    slots = table[owner, pos // bs].long() * bs + pos % bs
+    ids = torch.randint(0, 512, (T,)).cuda()
+    state = torch.randn(T, 288, device="cuda").to(dt)
+    starts = torch.tensor([0, 1, 2, 2 + chunk], dtype=torch.int32)
+    seq = torch.tensor([n + s for n, s in zip(lens, news)], dtype=torch.int32)
+
+    def run():
+        dec = pkg.PagedDecoder(model, num_blocks=3 * width, block_size=bs, num_steps=2)
+        for i, t in enumerate(dec.k + dec.v):
+            t.copy_(torch.randn(t.shape, generator=torch.Generator().manual_seed(i)).to(dt))
+        return dec, dec.forward_tokens(ids, pos, slots, table, seq, starts, max(news), input_states=state)
+
+    dec, (logits, latents) = run()
+    tuned(pad_chunk_rows=0, pad_decode_rows=0)
+    plain, (logits0, latents0) = run()
+    if 17 <= T <= 32:  # (these rows' products walk the padded K, whose slices are cut elsewhere)
+        check(logits, logits0, dt, f"logits of {T} rows", ulps=ULPS_COMPOSED)
+        check(latents, latents0, dt, f"latents of {T} rows", ulps=ULPS_COMPOSED)
+    else:
+        assert torch.equal(logits, logits0) and torch.equal(latents, latents0)
+        assert all(torch.equal(a, b) for a, b in zip(dec.k + dec.v, plain.k + plain.v))
+    # the first block, call by call
+    t, pos, slots, table, seq, starts = model.transformer, pos.cuda(), slots.cuda(), table.cuda(), seq.cuda(), starts.cuda()
+    blk, eps = t.prelude[0], cfg.norm_eps
+    one = pkg.PagedDecoder(model, num_blocks=3 * width, block_size=bs, num_steps=2)
+    for i, c in enumerate(one.k + one.v):
+        c.copy_(torch.randn(c.shape, generator=torch.Generator().manual_seed(i)).to(dt))
+    ws = hip.linear_workspace(T, 960, "cuda")
+    x = hip.embed(t.wte.weight, ids, model.emb_scale)
+    qkv = hip.linear(hip.rmsnorm_residual(x, blk.norm_1.weight, eps)[0], blk.attn.Wqkv.weight, workspace=ws)
+    bias = blk.attn.qk_bias if hasattr(blk.attn, "qk_bias") else None
+    q = hip.paged_qkv_rope_append(qkv, bias, model._natives()["freqs"], pos, slots, one.k[0], one.v[0], layout=one.layout)
+    ya = hip.paged_prefill_attention(q, one.k[0], one.v[0], table, seq, starts, max(news), layout=one.layout)
+    x2, _, n3 = hip.rmsnorm_residual(hip.linear(ya, blk.attn.proj.weight, residual=x, workspace=ws), blk.norm_2.weight, eps, weight2=blk.norm_3.weight)
+    x3 = hip.linear(hip.linear(n3, blk.mlp.fc.weight, swiglu=True, workspace=ws), blk.mlp.proj.weight, residual=x2, workspace=ws)
+    want = hip.rmsnorm_residual(x3, blk.norm_4.weight, eps)[0]
+    kv = hip.make_paged_kv(one.k[:1], one.v[:1], table, seq, width * bs, layout=one.layout)
+    dims = model._natives()["dims"]
+    got = hip.paged_chunk_blocks(dims, (hip.BlockWeights * 1)(blk.native()), x, torch.empty_like(x), model._natives()["freqs"], kv, pos, slots,
+                                 starts, max(news), hip.block_workspace(dims, T, "cuda"))
+    check(got, want, dt, f"block over {T} rows", ulps=ULPS_COMPOSED)
+    check(one.k[0], dec.k[0], dt, f"keys of {T} rows")
+    check(one.v[0], dec.v[0], dt, f"values of {T} rows")
