@@ -70,7 +70,7 @@ struct MidPlan {
     int tiles_m, tiles_n, ks;
     float us;              // the estimate it was chosen by
 };
-MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room);  // room: bytes of workspace for K slices
+MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room, int ks_from = 1);  // room: bytes of workspace for K slices, ks_from of them or more
 size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu);  // 0 when K is not split
 // ks_left (may be null): the K slices stay in the workspace ([slices, M, N] float) for the caller to add; receives their number, 0
 // when the product was finished

@@ -458,7 +458,7 @@ static double mid_estimate(const MidPlan& p, int M, int N, int K, int side, int 
     return us;
 }
 
-static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room) {
+static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room, int ks_from) {
     MidPlan best{};
     const int cus = mid_cus(), nk = (K + 63) / 64, side = swiglu ? 2 : 1;
     // the 128 x 128 tiles of gemm_tiled.hip: a K step takes 0.53 us on a CU with one of them and 0.34 more with each further one, and up to
@@ -474,7 +474,7 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room) {
         p.mt = (p.rows + 63) / 64;
         for (int nt = 1; nt <= 6; ++nt) {
             if (g_mid_nt && nt != g_mid_nt) continue;
-            for (p.ks = 1; p.ks <= kMidMaxSlices; ++p.ks) {
+            for (p.ks = ks_from; p.ks <= kMidMaxSlices; ++p.ks) {
                 if (g_mid_ks && p.ks != g_mid_ks && p.ks < nk) continue;
                 const int cap = 32 * nt / side;  // output columns of the largest unit
                 // as few columns per unit as still run in the rounds that the largest unit needs
@@ -498,7 +498,7 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room) {
     return best;
 }
 
-MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room) {
+MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room, int ks_from) {
     if (!g_mid) return MidPlan{};
     // a product is planned several times on its way (does it fit, which row pitch, which launch): the last few shapes of this thread
     struct Known {
@@ -508,11 +508,11 @@ MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room) {
     };
     static thread_local Known known[16];
     static thread_local int next = 0;
-    const int K = K0 + K1, knobs = 1 + g_mid_nt + 10 * g_mid_mt + 100 * g_mid_ks;
+    const int K = K0 + K1, knobs = 1 + g_mid_nt + 10 * g_mid_mt + 100 * g_mid_ks + 1000 * ks_from;
     for (const Known& k : known)
         if (k.M == M && k.N == N && k.K == K && k.swiglu == swiglu && k.knobs == knobs && k.room == room) return k.plan;
     Known& k = known[next++ & 15];
-    k = Known{M, N, K, swiglu, knobs, room, find_plan(M, N, K, swiglu, room)};
+    k = Known{M, N, K, swiglu, knobs, room, find_plan(M, N, K, swiglu, room, ks_from)};
     return k.plan;
 }
 

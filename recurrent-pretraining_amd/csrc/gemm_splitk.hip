@@ -28,6 +28,7 @@ namespace raven {
 
 extern int g_tiled_min_rows;
 bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
+bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_sums, const void* w, size_t workspace_bytes, bool aligned);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
@@ -376,7 +377,8 @@ int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, in
                       int N, int K0, int K1, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
     *ks_left = 0;
     const size_t room = usable(workspace, workspace_bytes);
-    if (!ldw && M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, raven_host::aligned16(x0, x1, w, residual, y)))
+    const bool aligned = raven_host::aligned16(x0, x1, w, residual, y);
+    if (!ldw && ((M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned)) || (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, 0, 0, w, room, aligned))))
         return tiled_gemm(x0, ldx, x1, w, residual, y, M, N, K0, K1, 0, 0, workspace, room, s, g_fuse_sums_norm && N <= 8192 ? ks_left : nullptr);
     RAVEN_REQUIRE(ldx == 0 || ldx == K0, "linear: rows of x0 %d elements apart", ldx);
     bool split = g_fuse_sums_norm && dtype == RAVEN_BF16 && M >= 2 && M <= 32 && N % 16 == 0 && N <= 8192 && K0 % 32 == 0 && K1 % 32 == 0 &&
@@ -420,8 +422,10 @@ extern "C" int raven_linear(const void* x0, const void* x1, const void* w, const
     RAVEN_REQUIRE((K1 == 0) == (x1 == nullptr), "linear: x1 and K1 must be given together");
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32 || K1)), "linear: the SwiGLU epilogue takes one operand, no residual, and stores T");
     RAVEN_REQUIRE(!(K1 && (residual || out_f32)), "linear: the two-operand form has a plain epilogue");
+    const bool aligned = raven_host::aligned16(x0, x1, w, residual, y);
     if (const size_t room = usable(workspace, workspace_bytes);  // many rows
-        M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, swiglu, room, raven_host::aligned16(x0, x1, w, residual, y)))
+        (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, swiglu, room, aligned)) ||
+        (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, swiglu, 0, w, room, aligned)))
         return tiled_gemm(x0, 0, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, workspace, room, static_cast<hipStream_t>(stream), nullptr);
     bool fits = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                 ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1;
@@ -475,7 +479,9 @@ extern "C" int raven_linear_epilogue(const void* x0, const void* x1, const void*
     RAVEN_REQUIRE(!epi->residual || epi->out_f32, "linear_epilogue: a residual needs a float output");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (K1 == 0 && gemm_narrow_fits(M, N, K0, dtype)) return gemm_narrow_free(x0, w, y, N, M, N, K0, *epi, s);
-    if (const size_t room = usable(workspace, workspace_bytes); M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, raven_host::aligned16(x0, x1, w, y)))
+    const bool aligned = raven_host::aligned16(x0, x1, w, y);
+    if (const size_t room = usable(workspace, workspace_bytes); (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned)) ||
+                                                               (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, 0, epi->out_f32, w, room, aligned)))
         return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, workspace, room, s);
     // the same choice between the kernels with and without a K split as raven_linear
     const bool split = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&

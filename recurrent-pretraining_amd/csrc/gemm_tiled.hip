@@ -891,11 +891,28 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const bf16* __restrict__
     }
 }
 
+// 17 to 32 rows, which else take the skinny kernels: gemm_mid.hip where K is long or the matrix large, and its rows (or their copies) are whole lines.
+// us, skinny kernels / these, at 20 rows, slices added by a launch of their own: 15840 x 5312 32.6 / 30.2, 2 x 17920 x 5312 64.2 / 60.8, 5280 x 17920 38.0 / 36.6,
+// 5280 x 5312 17.7 / 15.5, 2 x 5440 x 2048 12.6 / 11.3, 2048 x 5440 14.1 / 9.3, 2048 x 8192 14.1 / 11.0, 1280 x 5120 11.7 / 8.5; but 8192 x 2048 10.1 / 10.5,
+// 2048 x 2048 6.1 / 8.5, 3072 x 1536 5.6 / 7.4.  (16 rows: 1.04 to 1.08 where it is faster at all.)  f32_sums: the sums leave unrounded.  The skinny kernels add
+// each of them up in eight parts, so they are left alone unless these take eight slices: whole sums of 10304 x 2048 are 2.7e-7 from the exact ones, eight parts 1.0e-7.
+static int few_rows_slices(int f32_sums) { return f32_sums ? 8 : 1; }
+bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_sums, const void* w, size_t workspace_bytes, bool aligned) {
+    if (dtype != RAVEN_BF16 || !aligned || M < 17 || M > 32 || M >= g_tiled_min_rows || g_tiled_variant != 0 || K1 != 0 || K0 % 8 != 0 || N % 8 != 0) return false;
+    const int64_t rows = (int64_t)N * (swiglu ? 2 : 1);
+    if (N < 1024 || rows > 40000 || rows * K0 >= (1ll << 31) || !(K0 > 4096 || (rows * K0 >= 20000000 && !f32_sums))) return false;
+    int ld = 0;
+    if (K0 % 64 != 0 && !packed_weight_of(w, (int)rows, K0, &ld)) return false;
+    return mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)).nt != 0;
+}
+
 static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0,
                            int K1, int swiglu, int out_f32, const RopeAppend* rope, void* workspace, size_t workspace_bytes, hipStream_t s,
                            const raven_epilogue* epi = nullptr, int* ks_left = nullptr) {
     if (ks_left) *ks_left = 0;
-    RAVEN_REQUIRE(tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
+    const int f32_sums = epi && epi->out_f32;
+    const bool few = few_rows_fit(M, N, K0, K1, RAVEN_BF16, swiglu, f32_sums, w, workspace_bytes, true);
+    RAVEN_REQUIRE(few || tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32)), "gemm (tiled): the SwiGLU epilogue has no residual and stores bf16");
     RAVEN_REQUIRE(((uintptr_t)x0 & 15) == 0 && ((uintptr_t)x1 & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
                       ((uintptr_t)residual & 15) == 0, "gemm (tiled): operands must be 16-byte aligned");
@@ -919,7 +936,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
             a.ldw = it->second.ld;
         }
     }
-    const MidPlan mid = mid_choice(M, N, K0, a.K1, swiglu, workspace_bytes);
+    const MidPlan mid = few ? mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)) : mid_choice(M, N, K0, a.K1, swiglu, workspace_bytes);
     if (mid.nt) {
         const ProductArgs q{a.w, a.x0, a.x1, a.residual, y, M, N, K0, a.K1, a.ldw, a.ldx, swiglu, out_f32, epi, rope};
         return mid_gemm(q, mid, workspace, s, ks_left);

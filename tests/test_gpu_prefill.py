@@ -193,6 +193,26 @@ def test_units_with_any_number_of_tiles(pkg, tuned, nt, M):
             check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :half]).to(dt).float() * u[:, half:]).to(dt), dt, f"{M} x {half} x {K}, SwiGLU", ulps=ULPS_SWIGLU)
 
 
+@pytest.mark.parametrize("M", [16, 17, 20, 32, 33])
+def test_long_or_large_products_of_few_rows(pkg, M):
+    """17 to 32 rows against a matrix with a long K (1032 x 4160) or a large one (20000 x 1024, 2 x 10000 x 1024), and the row counts beside: rounded
+    results, SwiGLU, float sums added to a residual, slices left to the norm that follows."""
+    dt = torch.bfloat16
+    for N, K in ((1032, 4160), (20000, 1024)):
+        ws = pkg.hip.linear_workspace(M, N, "cuda")
+        x, w, res = _gpu_randn((M, K), 780 + M), _gpu_randn((N, K), 781, 0.05), _gpu_randn((M, N), 782)
+        z = x.float() @ w.float().T
+        check(pkg.hip.linear(x, w, residual=res, workspace=ws), (z.to(dt).float() + res.float()).to(dt), dt, f"{M} x {N} x {K} + residual", mag=z, ulps=ULPS_RESIDUAL)
+        resf = torch.randn(M, N, device="cuda")
+        exact = x.double() @ w.double().T * 0.5 + resf.double()
+        got = pkg.hip.linear_epilogue(x, w, residual=resf, scale=0.5, workspace=ws)
+        assert ((got.double() - exact).norm() / exact.norm()).item() < 4e-7, f"{M} x {N} x {K}, unrounded"  # 2^-24 sqrt(4160 / 32 / 8) and the residual's own rounding
+        assert torch.equal(got, pkg.hip.linear_epilogue(x, w, residual=resf, scale=0.5, workspace=ws))
+    fc = _gpu_randn((20000, 1024), 783, 0.05)
+    u = (x.float() @ fc.float().T).to(dt).float()
+    check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :10000]).to(dt).float() * u[:, 10000:]).to(dt), dt, f"{M} x 10000 x 1024, SwiGLU", ulps=ULPS_SWIGLU)
+
+
 @pytest.mark.parametrize("ks", [1, 3])
 @pytest.mark.parametrize("nt,mt", [(2, 1), (4, 2), (6, 4)])
 def test_infinities_stay_in_their_rows_and_columns(pkg, tuned, nt, mt, ks):
