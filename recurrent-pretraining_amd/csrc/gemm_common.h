@@ -41,9 +41,11 @@ struct ProductArgs {
     const bf16* w;         // [N or 2N, K0 + K1], rows ldw apart
     const bf16* x0;        // [M, K0], rows ldx apart
     const bf16* x1;        // [M, K1] or null, rows ldx apart
-    const bf16* residual;  // [M, N] or null
-    void* y;               // [M, N] bf16, or float when out_f32
+    const bf16* residual;  // [M, N] or null, rows ldy apart
+    void* y;               // [M, N] bf16, or float when out_f32, rows ldy apart
     int M, N, K0, K1, ldw, ldx;
+    int ldy;               // elements between two rows of y and of the residuals
+    int up_off;            // SwiGLU: weight rows from a gate row to its up row
     int swiglu, out_f32;
     const raven_epilogue* epi;   // free epilogue, or null
     const RopeAppend* rope;      // or null

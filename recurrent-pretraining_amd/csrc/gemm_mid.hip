@@ -32,6 +32,7 @@ struct MidArgs {
     void* y;
     float* partial;        // [ks, M, N or 2N] when ks > 1
     int M, N, K0, K1, ldw, ldx;
+    int ldy, up_off;       // elements between two rows of y and of the residuals; weight rows from a gate row to its up row
     int out_f32;
     int kind;              // EPI_*
     int cols, bm;          // output columns / token rows of a unit
@@ -48,7 +49,7 @@ __device__ __align__(16) unsigned int g_mid_zero[4];  // what a 16-byte piece pa
 // Four neighbouring output columns n .. n + 3 of token row m; xs: the factor of a grouped SwiGLU row
 template <int EPI, bool GROUPED = false>
 __device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 v, f32x4 up, float xs = 1.f) {
-    const int64_t at = (int64_t)m * a.N + n;
+    const int64_t at = (int64_t)m * a.ldy + n;
     if constexpr (EPI == EPI_SWIGLU) {
         bf16 o[4];
 #pragma unroll
@@ -84,8 +85,8 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 
         for (int i = 0; i < 4; ++i) o[i] = from_f32<bf16>(v[i]);
         if (a.rope_on) {
             const RopeAppend& r = a.rope;
-            const int h = r.nh * r.hd, sec = n >= 2 * h ? 2 : (n >= h ? 1 : 0);  // q, k or v columns; four of them lie in one head
-            const int col = n - sec * h, head = col / r.hd, d = col - head * r.hd;
+            const int h = r.nh * r.hd, nr = n + r.col0, sec = nr >= 2 * h ? 2 : (nr >= h ? 1 : 0);  // q, k or v columns; four of them lie in one head
+            const int col = nr - sec * h, head = col / r.hd, d = col - head * r.hd;
             const int b = m / r.S, sq = m - b * r.S, pos = (r.pos_dev ? *r.pos_dev : r.pos0) + sq;
             if (sec < 2) {
                 if (r.qk_bias) {
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         spare[i] = (GROUPED || i == WPW - 1 || i == LPW - 1) && piece >= 2 * (is_w ? a.wtiles : a.xtiles);  // (of a plain unit only the last ones may be)
         if (is_w) {
             const int c = min(swiglu ? (r >> 4) * 8 + (r & 7) : r, ncols - 1);
-            goff[i] = (unsigned)(n0 + c + (swiglu && (r & 8) ? a.N : 0)) * (2u * a.ldw) + 2u * colp;
+            goff[i] = (unsigned)(n0 + c + (swiglu && (r & 8) ? a.up_off : 0)) * (2u * a.ldw) + 2u * colp;
         } else {
             int row = m0 + min(r, rows - 1);
             if (GROUPED && x_row) row = x_row[row];
@@ -574,7 +575,7 @@ static int launch_mid(const MidArgs& a, const MidPlan& p, hipStream_t s, bool fi
 int mid_gemm(const ProductArgs& q, const MidPlan& p, void* workspace, hipStream_t s, int* ks_left) {
     MidArgs a{};
     a.w = q.w; a.x0 = q.x0; a.x1 = q.x1; a.residual = q.residual; a.y = q.y; a.partial = static_cast<float*>(workspace);
-    a.M = q.M; a.N = q.N; a.K0 = q.K0; a.K1 = q.x1 ? q.K1 : 0; a.ldw = q.ldw; a.ldx = q.ldx; a.out_f32 = q.out_f32;
+    a.M = q.M; a.N = q.N; a.K0 = q.K0; a.K1 = q.x1 ? q.K1 : 0; a.ldw = q.ldw; a.ldx = q.ldx; a.ldy = q.ldy; a.up_off = q.up_off; a.out_f32 = q.out_f32;
     a.kind = !q.epi ? (q.swiglu ? EPI_SWIGLU : EPI_PLAIN) : q.epi->act == RAVEN_ACT_GELU ? EPI_FREE_GELU : q.epi->act == RAVEN_ACT_TANH ? EPI_FREE_TANH : EPI_FREE;
     a.cols = p.cols; a.bm = p.rows; a.wtiles = (p.cols * (q.swiglu ? 2 : 1) + 15) / 16; a.xtiles = p.rows / 16;
     a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.ks = p.ks;
@@ -627,7 +628,7 @@ int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int
     a.w = static_cast<const bf16*>(w);
     a.x0 = static_cast<const bf16*>(x);
     a.y = y;
-    a.M = rows; a.N = N; a.K0 = K; a.ldw = K; a.ldx = K; a.out_f32 = out_f32;
+    a.M = rows; a.N = N; a.K0 = K; a.ldw = K; a.ldx = K; a.ldy = N; a.up_off = N; a.out_f32 = out_f32;
     const int side = swiglu ? 2 : 1, cap = 128 / side;
     const int tiles_n = (N + cap - 1) / cap;
     a.cols = ((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;

@@ -938,7 +938,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     }
     const MidPlan mid = few ? mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)) : mid_choice(M, N, K0, a.K1, swiglu, workspace_bytes);
     if (mid.nt) {
-        const ProductArgs q{a.w, a.x0, a.x1, a.residual, y, M, N, K0, a.K1, a.ldw, a.ldx, swiglu, out_f32, epi, rope};
+        const ProductArgs q{a.w, a.x0, a.x1, a.residual, y, M, N, K0, a.K1, a.ldw, a.ldx, N, N, swiglu, out_f32, epi, rope};
         return mid_gemm(q, mid, workspace, s, ks_left);
     }
     if (epi) a.epi = *epi;
@@ -965,6 +965,9 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     // columns are multiplied as 128 x 128 tiles instead -- four times as many workgroups, a quarter of the time each
     // (5.25 rounds of work then take about 5.4 rounds instead of 6: the N = 5280 products of the model at 16384 rows;
     // mlp.fc of a 512-token prompt: 280 tiles, 1.3 rounds instead of 2).
+    // Units of gemm_mid.hip, which are cut to fill one round whatever the columns' number, take them where that is estimated faster (without K slices: same
+    // bits).  us at 4000 rows, 1280 of 5280 columns, averaged over K of 5280, 10560 and 17920, small tiles / units: 191 / 120.  (Of a last round three quarters full,
+    // 2 x 3072 of 2 x 17920 columns, the big tiles run into the round before: 1039 in one launch, 995 + 122 with units.)
     const int64_t rest = big_tiles % 256;
     if (big && g_tiled_variant == 0 && g_tiled_split_tail && big_tiles > 256 && rest > 0 && rest <= 128 && rest % tiles_m == 0) {
         const int cols = (int)(rest / tiles_m);              // trailing tile columns
@@ -979,6 +982,12 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
         if (tail.epi.bias) tail.epi.bias += n_big;
         if (tail.epi.residual) tail.epi.residual += n_big;
         if (const int rc = launch(head, true)) return rc;
+        if (const MidPlan tail_plan = mid_plan(M, tail.N, K0, a.K1, swiglu, 0); tail_plan.nt) {
+            const raven_epilogue e = tail.epi;
+            const ProductArgs q{tail.w, tail.x0, tail.x1, tail.residual, tail.y, M, tail.N, K0, a.K1, a.ldw, a.ldx, a.ldy, a.up_off, swiglu, out_f32, epi ? &e : nullptr,
+                                rope ? &tail.rope : nullptr};
+            return mid_gemm(q, tail_plan, nullptr, s, nullptr);
+        }
         if (epi && a.K1 == 0 && a.ldx == K0 && a.ldw == K0 && gemm_narrow_fits(M, tail.N, K0, RAVEN_BF16))
             return gemm_narrow_free(tail.x0, tail.w, tail.y, tail.ldy, M, tail.N, K0, tail.epi, s);
         return launch(tail, false);
