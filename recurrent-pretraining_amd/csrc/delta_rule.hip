@@ -29,7 +29,11 @@
 //       16 x 16 piece of S in four registers per lane for the whole walk (the accumulator layout of the fp32 MFMA read as
 //       the B operand of the next product with the k slots permuted accordingly, so S and P never change layout).  The
 //       waves exchange their partial sums of P once per block, one barrier; partial sums of O ride along one block later.
-//       Operands are requested four blocks ahead.
+//       Operands are requested four blocks ahead.  The walk is bound by the lines a workgroup has to ask for against the 32 KB a CU
+//       keeps in flight, so every wave's rows of an operand are 1 KB in one piece and it asks for no 16 x 16 square but its own: 7 KB of
+//       lines a wave and block, 11 with rows of [16][R] and all three squares.  us with both kernels, before / now: 4096 tokens
+//       of 32 heads of 64 284 / 262, of 16 of 128 438 / 365; 64 tokens of 32 heads 17.6 / 16.5.  Six blocks ahead 273, two 365;
+//       V copied beside the operands 270 (half its lines, but written once more).
 //   delta_output_kernel  the output stage.
 //   All matrix products are fp32 MFMA (16 x 16 x 4).
 
@@ -237,13 +241,13 @@ __global__ __launch_bounds__(512) void delta_steps_kernel(DeltaArgs a) {
 constexpr int kBlk = 16;
 constexpr int kScanAhead = 4;        // blocks whose operands are in flight
 constexpr int kSegment = 256;        // most blocks per (block, scan) launch pair: bounds the workspace.  A pair costs about 13 us beside its
-                                     // blocks (4096 tokens, 32 heads of 64: 307 us in segments of 64 blocks, 281 of 128)
+                                     // blocks (4096 tokens, 32 heads of 64: 288 us in segments of 64 blocks, 262 of 128 and of 256)
 constexpr int kMinBlocked = 48;      // shorter chunks walk token by token
 constexpr int kMaxBlockedDim = 128;  // and so do wider heads (the scan's operands would not fit a wave's registers)
 
 // workspace of one (sequence, head, block), in floats; R = rows rounded up to 16
 __host__ __device__ constexpr int blk_floats(int R) { return 65 * R + 3 * kBlk * kBlk; }
-//   T U [16][R] | R [16][R] | -B^T G [R][16] | K^T G [R][16] | T M [16][16] | -tril(R B^T) | tril(R K^T) | G [R]
+//   T U [R/16][16][16] | R [R/16][16][16] | -B^T G [R][16] | K^T G [R][16] | T M [16][16] | -tril(R B^T) | tril(R K^T) | G [R]
 
 struct DeltaBlockArgs {
     DeltaArgs d;
@@ -349,7 +353,7 @@ __global__ __launch_bounds__(256, R <= 64 ? 4 : 2) void delta_block_kernel(Delta
             const float g = expf(log_g), rest = expf(total - log_g), back = expf(-log_g);
             const float rr = r[j][i] * g;
             Rt[t][c] = rr;
-            wR[t * R + c] = rr;
+            wR[(c & ~15) * 16 + t * 16 + (c & 15)] = rr;
             Bt[t][c] = bb[j][i] * back;
             Kt[t][c] = k[j][i] * back;
             bo[j] = -bb[j][i] * rest;
@@ -395,7 +399,7 @@ __global__ __launch_bounds__(256, R <= 64 ? 4 : 2) void delta_block_kernel(Delta
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             if (last) wTM[(4 * q + v) * 16 + l16] = x[v];
-            else wTU[(4 * q + v) * R + 16 * tile + l16] = x[v];
+            else wTU[(16 * tile + 4 * q + v) * 16 + l16] = x[v];
         }
     }
 }
@@ -420,15 +424,17 @@ __global__ __launch_bounds__(64 * NB) void delta_scan_kernel(DeltaBlockArgs p) {
     const char* vbase = reinterpret_cast<const char*>(a.z + (int64_t)b * a.S * a.ldz + 2 * inner + h * hd);
     // byte offsets below 2^32 (the host checks): uniform bases plus 32-bit lane offsets keep the address arithmetic off the loop
     const unsigned vcol = 4u * min(col, hd - 1), vrow = 4u * a.ldz, vlast = (a.S - 1) * vrow;
-    const unsigned at_row = 4u * (l16 * R + row), at_tok = 4u * ((16 * wave + l16) * 16 + 4 * q), at_sq = 4u * (l16 * 16 + 4 * q), at_g = 4u * row;
+    const unsigned at_wave = 4u * ((16 * wave + l16) * 16 + 4 * q), at_sq = 4u * (l16 * 16 + 4 * q), at_g = 4u * row;
     float* orow = p.o + (((int64_t)b * a.H + h) * p.o_rows) * R + 16 * tile + l16;
-    constexpr int wGV = 0, wRKV = NB - 1, wRBP = NB / 2;  // which wave adds the 16 x 16 products
+    // which wave adds which 16 x 16 product; each asks for its own square only, the others repeat T M's
+    constexpr int wGV = 0, wRKV = NB - 1, wRBP = NB / 2;
+    const int sq = 64 * R + (wave == wGV ? 0 : wave == wRBP ? 256 : wave == wRKV ? 512 : 0);
 
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
     if (!fresh && mine) S = *reinterpret_cast<const f32x4*>(state);
 
     struct Set {
-        f32x4 tu, r, bt, kt, g, tm, rb, rk;
+        f32x4 tu, r, bt, kt, g, sq, rk;  // rk apart only where one wave adds both products with R
         float v[4];
     };
     Set st[kScanAhead];
@@ -436,13 +442,12 @@ __global__ __launch_bounds__(64 * NB) void delta_scan_kernel(DeltaBlockArgs p) {
         const int cc = min(c, p.n_blocks - 1);
         const char* w = reinterpret_cast<const char*>(ws + (int64_t)cc * blk_floats(R));
         auto at = [&](int floats, unsigned off) { return *reinterpret_cast<const f32x4*>(w + 4 * floats + off); };
-        s.tu = at(0, at_row);
-        s.r = at(16 * R, at_row);
-        s.bt = at(32 * R, at_tok);
-        s.kt = at(48 * R, at_tok);
-        s.tm = at(64 * R, at_sq);
-        s.rb = at(64 * R + 256, at_sq);
-        s.rk = at(64 * R + 512, at_sq);
+        s.tu = at(0, at_wave);
+        s.r = at(16 * R, at_wave);
+        s.bt = at(32 * R, at_wave);
+        s.kt = at(48 * R, at_wave);
+        s.sq = at(sq, at_sq);
+        if constexpr (wRKV == wRBP) s.rk = at(64 * R + 512, at_sq);
         s.g = at(64 * R + 768, at_g);
         const unsigned first = (unsigned)((p.first + cc) * kBlk) * vrow;  // rows past the chunk repeat its last one: they meet zero factors
 #pragma unroll
@@ -475,7 +480,7 @@ __global__ __launch_bounds__(64 * NB) void delta_scan_kernel(DeltaBlockArgs p) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 O = zero, rb = zero;             // of the block before: its outputs so far, its -tril(R B^T) ...
     float pv[4] = {0.f, 0.f, 0.f, 0.f};    // ... and its removals
-    f32x4 P = wave == wGV ? mac4(st[0].tm, st[0].v, zero) : zero;
+    f32x4 P = wave == wGV ? mac4(st[0].sq, st[0].v, zero) : zero;
     for (int c0 = 0; c0 < p.n_blocks; c0 += kScanAhead) {
 #pragma unroll
         for (int d = 0; d < kScanAhead; ++d) {
@@ -492,11 +497,11 @@ __global__ __launch_bounds__(64 * NB) void delta_scan_kernel(DeltaBlockArgs p) {
             xp[buf][wave][lane] = P;
             if (wave == wRBP) O = mac4(rb, pv, O);
             __builtin_amdgcn_sched_barrier(0);
-            f32x4 O_next = wave == wRKV ? mac4(s.rk, s.v, zero) : zero;
+            f32x4 O_next = wave == wRKV ? mac4(wRKV == wRBP ? s.rk : s.sq, s.v, zero) : zero;
             O_next = mac4(s.r, sv, O_next);
             xo[buf][wave][lane] = O;
-            P = wave == wGV ? mac4(next.tm, next.v, zero) : zero;
-            rb = s.rb;
+            P = wave == wGV ? mac4(next.sq, next.v, zero) : zero;
+            rb = s.sq;
             __builtin_amdgcn_sched_barrier(0);
             __syncthreads();
             f32x4 sum = xp[buf][0][lane];
