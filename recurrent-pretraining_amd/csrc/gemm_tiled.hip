@@ -799,6 +799,7 @@ static int launch_ring(TiledArgs a, hipStream_t s) {
     return raven_host::check_launch("gemm (ring MFMA)");
 }
 
+extern int g_pad_decode_rows;  // compose.hip
 int g_tiled_min_rows = 33;  // raven_set_tuning("gemm_tiled_min_rows"): fewest rows that take this kernel
 int g_tiled_variant = 0;    // raven_set_tuning("gemm_tiled_variant"): 0 = by shape, 1 = 256 x 256 tiles, 2 = 128 x 128 tiles, 3 = 256 x 256 tiles by the eight-wave kernel
 int g_tiled_split_tail = 1; // raven_set_tuning("gemm_tiled_split_tail"): 0 = never hand the last round's tile columns to 128 x 128 tiles
@@ -902,7 +903,7 @@ bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_s
     const int64_t rows = (int64_t)N * (swiglu ? 2 : 1);
     if (N < 1024 || rows > 40000 || rows * K0 >= (1ll << 31) || !(K0 > 4096 || (rows * K0 >= 20000000 && !f32_sums))) return false;
     int ld = 0;
-    if (K0 % 64 != 0 && !packed_weight_of(w, (int)rows, K0, &ld)) return false;
+    if (K0 % 64 != 0 && !(g_pad_decode_rows && packed_weight_of(w, (int)rows, K0, &ld))) return false;
     return mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)).nt != 0;
 }
 
