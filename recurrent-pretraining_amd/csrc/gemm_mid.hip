@@ -1,6 +1,6 @@
-// Matrix-core products over a middling number of token rows (33 to a few thousand): Y[M,N] = concat(X0, X1)[M,K] W[N,K]^T in bf16 with fp32
+// Matrix-core products over a middling number of token rows (33 to a few thousand; from 17 against long or large matrices): Y[M,N] = concat(X0, X1)[M,K] W[N,K]^T in bf16 with fp32
 // accumulation, with the epilogues of gemm_tiled.hip -- prompts of ordinary length, decode batches past 32 sequences, a serving engine's
-// mixed steps, and long prompts against matrices too narrow to give every CU a 256 x 256 tile.
+// mixed steps, and long prompts against matrices too narrow to give every CU a 256 x 256 tile, or the last round of a product of such tiles.
 //
 // What bounds these products is how a CU's loads queue: it has about 32 KB of lines on their way at a time, answered in order, so that the token rows,
 // which hit the L2, wait as long as the weights from HBM in front of them (64 + 96 rows a step move at 53 bytes a ns on 30 CUs, 42 on all; the weights

@@ -1,4 +1,5 @@
-// Skinny bf16 GEMM for 2..32 token rows with a caller-provided workspace: Y[M,N] = X[M,K] W[N,K]^T, where K slices pay (splits_k).
+// Skinny bf16 GEMM for 2..32 token rows with a caller-provided workspace: Y[M,N] = X[M,K] W[N,K]^T, where K slices pay (splits_k) and
+// gemm_mid.hip does not (few_rows_fit: it takes long or large matrices from 17 rows).
 //
 // The four waves of a workgroup own four different 16-row weight tiles (a gate tile and an up tile each
 // for the SwiGLU epilogue) and walk the SAME K range, so the X tile of a macro-step (128 k-values) is
@@ -372,7 +373,7 @@ static size_t usable(const void* workspace, size_t bytes) { return workspace && 
 // takes the K-split kernel, its slices are left in the workspace un-added (*ks_left slices, to be handed to
 // splitk_sums_then_norm before anything else uses the workspace) and y is not written; otherwise the product is finished
 // into y and *ks_left is 0.
-// From 33 rows on the slices are those of gemm_mid.hip; ldx: elements between two rows of x0 there (0: K0).
+// From 33 rows on (few_rows_fit: 17) the slices are those of gemm_mid.hip; ldx: elements between two rows of x0 there (0: K0).
 int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
                       int N, int K0, int K1, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
     *ks_left = 0;

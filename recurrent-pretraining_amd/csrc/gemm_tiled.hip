@@ -802,7 +802,7 @@ static int launch_ring(TiledArgs a, hipStream_t s) {
 extern int g_pad_decode_rows;  // compose.hip
 int g_tiled_min_rows = 33;  // raven_set_tuning("gemm_tiled_min_rows"): fewest rows that take this kernel
 int g_tiled_variant = 0;    // raven_set_tuning("gemm_tiled_variant"): 0 = by shape, 1 = 256 x 256 tiles, 2 = 128 x 128 tiles, 3 = 256 x 256 tiles by the eight-wave kernel
-int g_tiled_split_tail = 1; // raven_set_tuning("gemm_tiled_split_tail"): 0 = never hand the last round's tile columns to 128 x 128 tiles
+int g_tiled_split_tail = 1; // raven_set_tuning("gemm_tiled_split_tail"): 0 = never hand the last round's tile columns to smaller tiles
 
 template <int EPI, int TM, int TN, int WM = 2, int WN = 4>
 static int launch_tiled(TiledArgs a, hipStream_t s) {
