@@ -40,7 +40,7 @@ int qkv_linear_rope_append(const void* x, int ldx, const void* wqkv, const void*
                            int head_dim, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* done);
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned, int f32_sums = 0);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int rmsnorm_pitched(const void* x, const void* residual, const void* weight, void* y, int ldy, void* sum_out, const void* weight2,

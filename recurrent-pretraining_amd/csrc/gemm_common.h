@@ -73,6 +73,11 @@ struct MidPlan {
     float us;              // the estimate it was chosen by
 };
 MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room, int ks_from = 1);  // room: bytes of workspace for K slices, ks_from of them or more
+struct MidParts {
+    int ks;                // 0: none
+    float us;
+};
+MidParts mid_float_parts(int M, int N, int K, size_t room);  // the fewest slices of 33 and more rows of sums that leave unrounded
 size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu);  // 0 when K is not split
 // ks_left (may be null): the K slices stay in the workspace ([slices, M, N] float) for the caller to add; receives their number, 0
 // when the product was finished

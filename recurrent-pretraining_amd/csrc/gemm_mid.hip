@@ -459,13 +459,17 @@ static double mid_estimate(const MidPlan& p, int M, int N, int K, int side, int 
     return us;
 }
 
+// What the 128 x 128 tiles of gemm_tiled.hip take, in us: a K step takes 0.53 us on a CU with one of them and 0.34 more with each further one,
+// and up to 0.15 more per round the fuller the chip is
+static double tiled_estimate(int M, int N, int K, int side, int cus) {
+    const int64_t small = (int64_t)((M + 127) / 128) * ((N * side + 127) / 128);
+    return (K + 63) / 64 * (0.19 + 0.34 * (double)((small + cus - 1) / cus) + 0.154 * (double)small / cus) + 3.8 + 2.6 * M * N / 6e6;
+}
+
 static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room, int ks_from) {
     MidPlan best{};
     const int cus = mid_cus(), nk = (K + 63) / 64, side = swiglu ? 2 : 1;
-    // the 128 x 128 tiles of gemm_tiled.hip: a K step takes 0.53 us on a CU with one of them and 0.34 more with each further one, and up to
-    // 0.15 more per round the fuller the chip is
-    const int64_t small = (int64_t)((M + 127) / 128) * ((N * side + 127) / 128);
-    const double tiled = nk * (0.19 + 0.34 * (double)((small + cus - 1) / cus) + 0.154 * (double)small / cus) + 3.8 + 2.6 * M * N / 6e6;
+    const double tiled = tiled_estimate(M, N, K, side, cus);
     const bool forced = g_mid_nt || g_mid_mt || g_mid_ks;
     for (int mt = 1; mt <= 4; ++mt) {
         if (g_mid_mt && mt != g_mid_mt) continue;
@@ -491,7 +495,7 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room, int ks_fr
                 if (p.ks > 1 && nk / p.ks < (g_mid_ks ? 1 : 6)) break;
                 if (mid_workspace_bytes(M, N, p, swiglu) > room) break;
                 p.us = (float)mid_estimate(p, M, N, K, side, cus);
-                if ((forced || p.us < tiled) && (best.nt == 0 || p.us < best.us)) best = p;
+                if ((forced || ks_from > 1 || p.us < tiled) && (best.nt == 0 || p.us < best.us)) best = p;
             }
         }
     }
@@ -515,6 +519,52 @@ MidPlan mid_plan(int M, int N, int K0, int K1, int swiglu, size_t room, int ks_f
     Known& k = known[next++ & 15];
     k = Known{M, N, K, swiglu, knobs, room, find_plan(M, N, K, swiglu, room, ks_from)};
     return k.plan;
+}
+
+// The parts in which the sums of a product are added up belong to their accuracy where they leave unrounded, so they don't follow the estimate
+// above, which drops slices as soon as a launch does without them: 2048 x 2048 at 33 to 165 rows in four slices 1.32e-7 from the
+// exact sums, in one 2.70e-7.  They are those that units of whole groups of 64 rows by 32 columns are best cut into, which these
+// sums have always had; a product takes that many or more.  0: 128 x 128 tiles.
+static MidParts find_parts(int M, int N, int K, size_t room) {
+    MidParts best{0, 0.f};
+    const int cus = mid_cus(), nk = (K + 63) / 64;
+    const double tiled = tiled_estimate(M, N, K, 1, cus);
+    for (int nt = 2; nt <= 6; nt += 2)
+        for (int mt = 1; mt <= 4; mt *= 2) {
+            const int cap = nt * mt == 24 ? 160 : 32 * nt;
+            const int64_t tiles_m = (M + 64 * mt - 1) / (64 * mt), whole = (N + cap - 1) / cap * tiles_m, across = (whole + cus - 1) / cus * cus / tiles_m;
+            int cols = (int)((N + across - 1) / across + 7) / 8 * 8;
+            cols = cols < 16 * nt ? 16 * nt : cols > cap ? cap : cols;
+            const int64_t units = (N + cols - 1) / cols * tiles_m;
+            const int tiles_w = (cols + 15) / 16, wave_t = tiles_w < nt ? tiles_w : nt;
+            const double weights = 2.0 * N * K, again = weights * (tiles_m - 1) + 2.0 * K * 64 * mt * units, mem = weights / 9e6 + again / 18e6;
+            for (int ks = 1; ks <= kMidMaxSlices; ++ks) {
+                if (ks > 1 && (units * ks > cus + cus / 32 || nk / ks < 6 || (size_t)ks * M * N * sizeof(float) > room)) break;
+                const int rounds = (int)((units * ks + cus - 1) / cus);
+                const double lds = rounds * ((nk + ks - 1) / ks) * (128.0 * (wave_t + mt) + 16 * tiles_w + 64 * mt) / 2050.0;
+                double us = (mem > lds ? mem : lds) * (1.0 + (mt == 4 && ks == 1 ? 0.23 : 0) + (nt == 6 ? 0.11 : 0)) + 3.8 * rounds + 6.2 * M * N / 6e6 / rounds;
+                if (ks > 1) us += 1.2 + 15.0 * ks * M * N / 8e6;
+                if ((float)us < tiled && (best.ks == 0 || (float)us < best.us)) best = MidParts{ks, (float)us};
+            }
+        }
+    return best;
+}
+
+MidParts mid_float_parts(int M, int N, int K, size_t room) {
+    if (!g_mid) return MidParts{0, 0.f};
+    if (g_mid_nt || g_mid_mt || g_mid_ks) return MidParts{1, 0.f};  // a plan of the caller's own
+    struct Known {
+        int M, N, K;
+        size_t room;
+        MidParts parts;
+    };
+    static thread_local Known known[16];  // as in mid_plan
+    static thread_local int next = 0;
+    for (const Known& k : known)
+        if (k.M == M && k.N == N && k.K == K && k.room == room) return k.parts;
+    Known& k = known[next++ & 15];
+    k = Known{M, N, K, room, find_parts(M, N, K, room)};
+    return k.parts;
 }
 
 size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu) {

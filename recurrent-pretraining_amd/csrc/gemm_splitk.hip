@@ -28,7 +28,7 @@ extern "C" int raven_gemm_swiglu(const void* x, const void* fc, void* out, int32
 namespace raven {
 
 extern int g_tiled_min_rows;
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned);
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned, int f32_sums = 0);
 bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_sums, const void* w, size_t workspace_bytes, bool aligned);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
@@ -481,7 +481,7 @@ extern "C" int raven_linear_epilogue(const void* x0, const void* x1, const void*
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (K1 == 0 && gemm_narrow_fits(M, N, K0, dtype)) return gemm_narrow_free(x0, w, y, N, M, N, K0, *epi, s);
     const bool aligned = raven_host::aligned16(x0, x1, w, y);
-    if (const size_t room = usable(workspace, workspace_bytes); (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned)) ||
+    if (const size_t room = usable(workspace, workspace_bytes); (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned, epi->out_f32)) ||
                                                                (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, 0, epi->out_f32, w, room, aligned)))
         return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, workspace, room, s);
     // the same choice between the kernels with and without a K split as raven_linear

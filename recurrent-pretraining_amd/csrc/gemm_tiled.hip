@@ -827,21 +827,33 @@ static int launch_tiled(TiledArgs a, hipStream_t s) {
     return raven_host::check_launch("gemm (tiled MFMA)");
 }
 
-// The best plan of gemm_mid.hip whose K slices fit the caller's workspace, or one without tiles where the kernels of this file are the better
-// choice: once 256 x 256 tiles fill the chip (256 of them), and where 128 x 128 tiles are estimated faster.
-static MidPlan mid_choice(int M, int N, int K0, int K1, int swiglu, size_t workspace_bytes) {
-    MidPlan none{};
-    const int bn_out = swiglu ? 128 : 256;
-    if (g_tiled_variant != 0 || M < g_tiled_min_rows || (int64_t)((M + 255) / 256) * ((N + bn_out - 1) / bn_out) >= 256) return none;
-    return mid_plan(M, N, K0, K1, swiglu, workspace_bytes);
-}
-
 // What passes of 32 rows by the skinny kernels take, in us: the walk of a workgroup's waves over K, or the weights at 5 TB/s (32 rows: 4096 columns
 // of 1024, 2048, 4096, 8192 4.9, 6.5, 10, 17; 8192 of 2048 and 4096 10 and 16.5; 15840 of 5280 34)
 static double passes_us(int M, int N, int K) {
     const double walk = 2.8 + 0.0017 * K, stream = 2.5 + 2.0 * N * K / 5e6;
     const double last = M % 32 ? 0.6 + 0.0125 * (M % 32) : 0;  // (a pass of few rows is shorter)
     return (M / 32 + last) * (walk > stream ? walk : stream);
+}
+
+// Few rows against few tiles, which passes of 32 rows may serve
+static bool passes_allowed(int M, int N, int K) {
+    return g_tiled_variant == 0 && (int64_t)((M + 127) / 128) * ((N + 127) / 128) < 128 && M <= 160 && M <= 32 * ((K + 3499) / 3500);
+}
+
+// The parts that the sums of a product are added up in at the least where they leave unrounded (mid_float_parts); the passes' waves add eight
+static int float_parts(int M, int N, int K, size_t room) {
+    const MidParts mid = mid_float_parts(M, N, K, room);
+    if (passes_allowed(M, N, K) && !(mid.ks && mid.us < passes_us(M, N, K))) return 8;
+    return mid.ks ? mid.ks : 1;
+}
+
+// The best plan of gemm_mid.hip whose K slices fit the caller's workspace, or one without tiles where the kernels of this file are the better
+// choice: once 256 x 256 tiles fill the chip (256 of them), and where 128 x 128 tiles are estimated faster.
+static MidPlan mid_choice(int M, int N, int K0, int K1, int swiglu, int f32_sums, size_t workspace_bytes) {
+    MidPlan none{};
+    const int bn_out = swiglu ? 128 : 256;
+    if (g_tiled_variant != 0 || M < g_tiled_min_rows || (int64_t)((M + 255) / 256) * ((N + bn_out - 1) / bn_out) >= 256) return none;
+    return mid_plan(M, N, K0, K1, swiglu, workspace_bytes, f32_sums ? float_parts(M, N, K0 + K1, workspace_bytes) : 1);
 }
 
 // Host entry for the other translation units: true when the shape is one the kernels over many rows take and they are the better
@@ -851,14 +863,12 @@ static double passes_us(int M, int N, int K) {
 // of 128 x 128 tiles walking the whole of K (measured at 33 .. 160 rows: Wqkv 98 / 130 us in three / four passes against 75 / 81 tiled,
 // mlp.proj 172 against 199).
 // aligned: whether all operands start on 16 bytes, which the kernels over many rows need; the passes take any address.
-bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned) {
+bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned, int f32_sums) {
     const bool ok = dtype == RAVEN_BF16 && M >= 1 && N % 8 == 0 && K0 % 8 == 0 && K0 > 0 && (K1 == 0 || K1 == K0) &&
                     (int64_t)M * (K0 > K1 ? K0 : K1) < (1ll << 31) && (int64_t)N * 2 * (K0 + K1) < (1ll << 31);
     if (!ok) return false;
-    const int64_t small_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-    const int passes = (K0 + K1 + 3499) / 3500;
-    if (g_tiled_variant == 0 && small_tiles < 128 && M <= 160 && M <= 32 * passes) {
-        const MidPlan mid = aligned ? mid_choice(M, N, K0, K1, swiglu, workspace_bytes) : MidPlan{};
+    if (passes_allowed(M, N, K0 + K1)) {
+        const MidPlan mid = aligned ? mid_choice(M, N, K0, K1, swiglu, f32_sums, workspace_bytes) : MidPlan{};
         return mid.nt != 0 && mid.us < passes_us(M, swiglu ? 2 * N : N, K0 + K1);
     }
     return true;
@@ -913,7 +923,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     if (ks_left) *ks_left = 0;
     const int f32_sums = epi && epi->out_f32;
     const bool few = few_rows_fit(M, N, K0, K1, RAVEN_BF16, swiglu, f32_sums, w, workspace_bytes, true);
-    RAVEN_REQUIRE(few || tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
+    RAVEN_REQUIRE(few || tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true, f32_sums), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32)), "gemm (tiled): the SwiGLU epilogue has no residual and stores bf16");
     RAVEN_REQUIRE(((uintptr_t)x0 & 15) == 0 && ((uintptr_t)x1 & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
                       ((uintptr_t)residual & 15) == 0, "gemm (tiled): operands must be 16-byte aligned");
@@ -937,7 +947,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
             a.ldw = it->second.ld;
         }
     }
-    const MidPlan mid = few ? mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)) : mid_choice(M, N, K0, a.K1, swiglu, workspace_bytes);
+    const MidPlan mid = few ? mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)) : mid_choice(M, N, K0, a.K1, swiglu, f32_sums, workspace_bytes);
     if (mid.nt) {
         const ProductArgs q{a.w, a.x0, a.x1, a.residual, y, M, N, K0, a.K1, a.ldw, a.ldx, N, N, swiglu, out_f32, epi, rope};
         return mid_gemm(q, mid, workspace, s, ks_left);

@@ -213,6 +213,20 @@ def test_long_or_large_products_of_few_rows(pkg, M):
     check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :10000]).to(dt).float() * u[:, 10000:]).to(dt), dt, f"{M} x 10000 x 1024, SwiGLU", ulps=ULPS_SWIGLU)
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(33, 1536, 1536, 4), (40, 2048, 2048, 4), (60, 1792, 7168, 8), (80, 2048, 5440, 8), (100, 2304, 2304, 3), (165, 2048, 2048, 4),
+                                         (165, 2048, 8192, 8), (230, 2048, 8192, 8), (300, 512, 2048, 3), (450, 1024, 4096, 4), (385, 1280, 5120, 6)])
+def test_float_sums_keep_the_parts_they_are_added_up_in(pkg, tuned, M, N, K, parts):
+    """Sums that leave unrounded are no further from the exact ones than sums cut into `parts` slices, the fewest these sizes take: a whole chain is
+    1.7 to 2.4 times as far.  (1.05: the same sums where the slices are as many; the error of M x N of them varies by less than a hundredth.)"""
+    x, w = _gpu_randn((M, K), 790 + M), _gpu_randn((N, K), 791, 0.05)
+    exact, ws = x.double() @ w.double().T, pkg.hip.linear_workspace(M, N, "cuda")
+    far = lambda: ((pkg.hip.linear_epilogue(x, w, workspace=ws).double() - exact).norm() / exact.norm()).item()
+    got = far()
+    tuned(gemm_mid_ks=parts)
+    bar = far()
+    assert got < 1.05 * bar, f"{M} x {N} x {K}: {got:.3g}, in {parts} slices {bar:.3g}"
+
+
 @pytest.mark.parametrize("ks", [1, 3])
 @pytest.mark.parametrize("nt,mt", [(2, 1), (4, 2), (6, 4)])
 def test_infinities_stay_in_their_rows_and_columns(pkg, tuned, nt, mt, ks):
