@@ -83,18 +83,18 @@ class SandwichBlock(torch.nn.Module):
 
 class _PackedWeights:
     """Line-aligned copies (hip.register_packed_weight) of the bf16 matrices whose rows are not whole 128-byte lines, read by
-    the tiled GEMM in place of the originals for products over 33 and more token rows.  A copy belongs to a weight tensor's
-    address and in-place version; `ensure` makes the copies again when either has changed (load_state_dict, .to()), `drop`
+    the tiled GEMM in place of the originals for products over 33 and more token rows (some of 17 to 32).  A copy belongs to a weight tensor's
+    address and in-place version; `ensure` makes the copies again when either has changed (load_state_dict, .to()) or when told to, `drop`
     unregisters them (also when the model is collected: the library's table is keyed by address)."""
 
     def __init__(self):
         self.key = None
         self.ptr_owner = []   # (weight tensor, packed buffer): both kept alive while registered
 
-    def ensure(self, mats) -> None:
+    def ensure(self, mats, force: bool = False) -> None:
         mats = [w for w in mats if w.is_cuda and w.dtype == torch.bfloat16 and (w.shape[1] * 2) % 128 != 0 and w.shape[1] % 8 == 0]
         key = tuple((w.data_ptr(), w._version) for w in mats)
-        if key == self.key:
+        if key == self.key and not force:
             return
         # matrices that only changed in place keep their copy's buffer (a captured graph may hold its address)
         old = {(w.data_ptr(), tuple(w.shape)): buf for w, buf in self.ptr_owner}
@@ -352,7 +352,7 @@ class RavenForCausalLM(MinimalGeneration, RavenPreTrainedModel, GenerationMixin)
         more (decode steps of 17..32 sequences read Wqkv and mlp.fc through them, chunks of 33 rows and more all three matrices)
         makes sure that the line-aligned weight copies are current."""
         if M >= 17 and self.dtype == torch.bfloat16 and self.pack_chunk_weights:
-            self.pack_weights()
+            self.pack_weights(force=False)
         ws = self._scratch.get(("ws", M))
         if ws is None:
             ws = hip.block_workspace(self._natives()["dims"], M, self.device)
@@ -559,10 +559,11 @@ class RavenForCausalLM(MinimalGeneration, RavenPreTrainedModel, GenerationMixin)
         finally:
             self._rope_override = None
 
-    def pack_weights(self) -> None:
+    def pack_weights(self, force: bool = True) -> None:
         """Makes (or refreshes) the line-aligned copies of Wqkv, attn.proj and mlp.fc that products over 33 and more token rows
-        read (bf16 models whose n_embd * 2 bytes is not a multiple of 128: n_embd = 5280).  Every block call over such a
-        chunk calls this; call it by hand after changing a weight through `.data`, which leaves no trace a check could see."""
+        read, and over 17 to 32 where few_rows_fit says so (bf16 models whose n_embd * 2 bytes is not a multiple of 128: n_embd = 5280).
+        Every block call over so many rows makes sure of them (force False: nothing to do while all version numbers are the copies'); call it by
+        hand after changing a weight through `.data`, which leaves no trace a check could see."""
         if not self._packed_finalizer.alive or self._packed_owner != id(self):
             # a copy of a model (copy.deepcopy) starts without registrations of its own
             self._packed = _PackedWeights()
@@ -570,7 +571,7 @@ class RavenForCausalLM(MinimalGeneration, RavenPreTrainedModel, GenerationMixin)
             self._packed_owner = id(self)
         t = self.transformer
         blocks = list(t.prelude) + list(t.core_block) + list(t.coda)
-        self._packed.ensure([w for b in blocks for w in (b.attn.Wqkv.weight, b.attn.proj.weight, b.mlp.fc.weight)])
+        self._packed.ensure([w for b in blocks for w in (b.attn.Wqkv.weight, b.attn.proj.weight, b.mlp.fc.weight)], force)
 
     def _forward_rows(self, input_ids, input_embeds, input_states, labels, output_details, init_scale, cache, private, pos0, B, S, r):
         cfg, t = self.config, self.transformer
@@ -863,7 +864,7 @@ class DecodeRunner(GraphedStep):
         self.logits = torch.empty(batch, cfg.padded_vocab_size, dtype=torch.float32, device=dev)
         self.next_ids = torch.zeros(batch, dtype=torch.int64, device=dev)
         if batch >= 17 and model.dtype == torch.bfloat16 and model.pack_chunk_weights:
-            model.pack_weights()  # decode steps of 17..32 rows read Wqkv and mlp.fc through their line-aligned copies
+            model.pack_weights(force=False)  # decode steps of 17..32 rows read Wqkv and mlp.fc through their line-aligned copies
         self.ws = hip.block_workspace(model._natives()["dims"], batch, dev)
 
     def _slots(self):
@@ -949,7 +950,7 @@ class DecodeRunner(GraphedStep):
             self.graph = None
         hint = self._position_bound(pos0)
         if self.B >= 17 and m.dtype == torch.bfloat16 and m.pack_chunk_weights:
-            m.pack_weights()  # no work unless a weight changed since the copies were made (in place: the copies keep their addresses)
+            m.pack_weights(force=False)  # no work unless a weight changed since the copies were made (in place: the copies keep their addresses)
         self.ids.copy_(ids.view(-1))
         if state is None:
             if init_scale > 0:

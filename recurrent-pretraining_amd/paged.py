@@ -118,7 +118,7 @@ class PagedDecoder:
         q_start, max_q = query_start_loc.to(dev, torch.int32), int(max_query_len)
         n_pre, n_core = cfg.n_layers_in_prelude, cfg.n_layers_in_recurrent_block
         if T >= 17 and m.pack_chunk_weights:
-            m.pack_weights()  # the products read Wqkv, attn.proj and mlp.fc through their line-aligned copies
+            m.pack_weights(force=False)  # the products read Wqkv, attn.proj and mlp.fc through their line-aligned copies
         dims, freqs = m._natives()["dims"], m._natives()["freqs"]
         ws = hip.block_workspace(dims, T, dev, clear=False)
         x = hip.embed(t.wte.weight, input_ids.reshape(-1).to(dev, torch.int64).contiguous(), m.emb_scale)
@@ -174,7 +174,7 @@ class PagedDecoder:
             dev, dt, h = m.device, m.dtype, cfg.n_embd
             nat = m._natives()
             if B >= 17 and dt == torch.bfloat16 and m.pack_chunk_weights:
-                m.pack_weights()  # decode steps of 17..32 rows read Wqkv and mlp.fc through their line-aligned copies
+                m.pack_weights(force=False)  # decode steps of 17..32 rows read Wqkv and mlp.fc through their line-aligned copies
             mk = lambda: torch.empty(B, h, dtype=dt, device=dev)
             self._ws[key] = {
                 "ids": torch.zeros(B, dtype=torch.int64, device=dev),

@@ -1452,3 +1452,31 @@ def test_mixed_rows_on_pages_equal_the_launches_one_by_one(pkg, tuned, chunk):
     check(got, want, dt, f"block over {T} rows", ulps=ULPS_COMPOSED)
     check(one.k[0], dec.k[0], dt, f"keys of {T} rows")
     check(one.v[0], dec.v[0], dt, f"values of {T} rows")
+
+
+def _half_line_model(pkg):
+    """n_embd = 288: rows of 576 bytes, whose matrices have line-aligned copies."""
+    cfg = pkg.RavenConfig(n_embd=288, n_heads=3, n_layers=5, n_layers_in_prelude=1, n_layers_in_recurrent_block=2, n_layers_in_coda=2,
+                          intermediate_size=480, vocab_size=512, mean_recurrence=2)
+    torch.manual_seed(18)
+    model = pkg.RavenForCausalLM(cfg, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0.0, 0.05)
+    return model
+
+
+def test_copies_made_by_hand_after_a_change_that_leaves_no_trace(pkg):
+    """pack_weights() called by the user copies again although no version number has moved (a change through `.data`), into the same buffers."""
+    model = _half_line_model(pkg)
+    ids, states = torch.randint(0, 512, (1, 40), device="cuda"), torch.randn(1, 40, 288, device="cuda")
+    before = model(input_ids=ids, input_states=states).logits
+    bufs = [buf.data_ptr() for _, buf in model._packed.ptr_owner]
+    assert bufs
+    model.transformer.core_block[0].mlp.fc.weight.data.mul_(1.5)
+    model.pack_weights()
+    fresh = pkg.RavenForCausalLM(model.config, device="cuda", dtype=torch.bfloat16)
+    fresh.load_state_dict(model.state_dict())
+    after = model(input_ids=ids, input_states=states).logits
+    assert not torch.equal(after, before) and torch.equal(after, fresh(input_ids=ids, input_states=states).logits)
+    assert [buf.data_ptr() for _, buf in model._packed.ptr_owner] == bufs
