@@ -559,6 +559,11 @@ class RavenForCausalLM(MinimalGeneration, RavenPreTrainedModel, GenerationMixin)
         finally:
             self._rope_override = None
 
+    @property
+    def holds_packed_weights(self) -> bool:
+        """Whether pack_weights() has made copies of this model's matrices."""
+        return self._packed_owner == id(self) and bool(self._packed.ptr_owner)
+
     def pack_weights(self, force: bool = True) -> None:
         """Makes (or refreshes) the line-aligned copies of Wqkv, attn.proj and mlp.fc that products over 33 and more token rows
         read, and over 17 to 32 where few_rows_fit says so (bf16 models whose n_embd * 2 bytes is not a multiple of 128: n_embd = 5280).

@@ -102,7 +102,9 @@ class PagedDecoder:
         the pages: input_ids [T] are the new rows of B sequences, flattened (prompt chunks of any length and decode rows
         together); positions [T] and slot_mapping [T] (int64) say where each row sits; sequence b owns rows
         query_start_loc[b] .. query_start_loc[b + 1] - 1 and holds seq_lens[b] positions once they are appended.
-        Returns (logits [T, V] float32, latents [T, h]).  bf16 models with head_dim 64 / 96 / 128."""
+        Returns (logits [T, V] float32, latents [T, h]).  bf16 models with head_dim 64 / 96 / 128.
+        The products read the weights themselves, so a change through `.data` counts at once, unless the model holds line-aligned
+        copies (of forward() over 17 rows and more, step() over as many sequences, or pack_weights(), which is to be called again then)."""
         m, cfg, t = self.model, self.cfg, self.model.transformer
         if m.dtype != torch.bfloat16:
             raise NotImplementedError("forward_tokens: the paged chunk attention kernel is bf16 only")
@@ -117,8 +119,8 @@ class PagedDecoder:
         table, lens = block_table.to(dev, torch.int32).contiguous(), seq_lens.to(dev, torch.int32)
         q_start, max_q = query_start_loc.to(dev, torch.int32), int(max_query_len)
         n_pre, n_core = cfg.n_layers_in_prelude, cfg.n_layers_in_recurrent_block
-        if T >= 17 and m.pack_chunk_weights:
-            m.pack_weights(force=False)  # the products read Wqkv, attn.proj and mlp.fc through their line-aligned copies
+        if T >= 17 and m.holds_packed_weights:
+            m.pack_weights(force=False)  # the products read the copies that the model holds: keep them current
         dims, freqs = m._natives()["dims"], m._natives()["freqs"]
         ws = hip.block_workspace(dims, T, dev, clear=False)
         x = hip.embed(t.wte.weight, input_ids.reshape(-1).to(dev, torch.int64).contiguous(), m.emb_scale)

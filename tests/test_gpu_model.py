@@ -1480,3 +1480,41 @@ def test_copies_made_by_hand_after_a_change_that_leaves_no_trace(pkg):
     after = model(input_ids=ids, input_states=states).logits
     assert not torch.equal(after, before) and torch.equal(after, fresh(input_ids=ids, input_states=states).logits)
     assert [buf.data_ptr() for _, buf in model._packed.ptr_owner] == bufs
+
+
+def _paged_step(pkg, model, chunk):
+    """One scheduler step of a fresh decoder: a decode row beside a chunk, the same pages and latent state each time."""
+    T, bs, width = 1 + chunk, 8, (chunk + 10 + 7) // 8
+    g = torch.Generator().manual_seed(chunk)
+    dec = pkg.PagedDecoder(model, num_blocks=2 * width, block_size=bs, num_steps=2)
+    for t in dec.k + dec.v:
+        t.copy_(torch.randn(t.shape, generator=g).to(t.dtype))
+    table = torch.arange(2 * width, dtype=torch.int32).view(2, width)
+    pos = torch.cat([torch.tensor([9]), torch.arange(chunk)])
+    slots = table[torch.tensor([0] + [1] * chunk), pos // bs].long() * bs + pos % bs
+    ids, state = torch.randint(0, 512, (T,), generator=g), torch.randn(T, model.config.n_embd, generator=g)
+    return dec.forward_tokens(ids, pos, slots, table, torch.tensor([10, chunk], dtype=torch.int32), torch.tensor([0, 1, T], dtype=torch.int32), chunk,
+                              input_states=state)[0]
+
+
+@pytest.mark.parametrize("chunk", [19, 80])
+def test_mixed_rows_see_weights_changed_without_a_trace(pkg, chunk):
+    """forward_tokens makes no copies: a weight changed through `.data` (as trainers hand new weights to an engine) counts from the next call on.
+    Copies that the model already holds follow the changes that a version number shows."""
+    model = _half_line_model(pkg)
+    before = _paged_step(pkg, model, chunk)
+    blk = model.transformer.core_block[0]
+    for w in (blk.attn.Wqkv.weight, blk.attn.proj.weight, blk.mlp.fc.weight):
+        w.data.mul_(1.5)
+    after = _paged_step(pkg, model, chunk)
+    fresh = pkg.RavenForCausalLM(model.config, device="cuda", dtype=torch.bfloat16)
+    fresh.load_state_dict(model.state_dict())
+    assert not torch.equal(before, after) and torch.equal(after, _paged_step(pkg, fresh, chunk))
+    assert not model.holds_packed_weights
+    model.pack_weights()
+    assert model.holds_packed_weights
+    with torch.no_grad():
+        blk.mlp.fc.weight.mul_(0.5)
+    fresh.load_state_dict(model.state_dict())
+    fresh.pack_weights()
+    assert torch.equal(_paged_step(pkg, model, chunk), _paged_step(pkg, fresh, chunk))
