@@ -175,8 +175,6 @@ class PagedDecoder:
             m, cfg = self.model, self.cfg
             dev, dt, h = m.device, m.dtype, cfg.n_embd
             nat = m._natives()
-            if B >= 17 and dt == torch.bfloat16 and m.pack_chunk_weights:
-                m.pack_weights(force=False)  # decode steps of 17..32 rows read Wqkv and mlp.fc through their line-aligned copies
             mk = lambda: torch.empty(B, h, dtype=dt, device=dev)
             self._ws[key] = {
                 "ids": torch.zeros(B, dtype=torch.int64, device=dev),
@@ -259,6 +257,8 @@ class PagedDecoder:
             raise ValueError("block_table [B, max_blocks] and seq_lens [B] must match ids [B]")
         if self._wants_check(check_bounds, block_table, seq_lens):
             self._check_pages(block_table, seq_lens)
+        if B >= 17 and m.dtype == torch.bfloat16 and m.pack_chunk_weights:
+            m.pack_weights(force=False)  # the products read line-aligned copies; no work unless a weight changed (in place: a captured step stays valid)
         buf = self._buffers(B, block_table.shape[1])
         buf["ids"].copy_(ids.view(-1))
         buf["table"].copy_(block_table)

@@ -1518,3 +1518,30 @@ def test_mixed_rows_see_weights_changed_without_a_trace(pkg, chunk):
     fresh.load_state_dict(model.state_dict())
     fresh.pack_weights()
     assert torch.equal(_paged_step(pkg, model, chunk), _paged_step(pkg, fresh, chunk))
+
+
+@pytest.mark.parametrize("B,use_graph", [(20, False), (20, True), (40, True)])
+def test_paged_steps_follow_weights_that_change_between_them(pkg, B, use_graph):
+    """Steps of 17 sequences and more read line-aligned copies (17 to 32 rows Wqkv, mlp.fc and long products, 33 and more attn.proj too): an in-place
+    change between two steps reaches the next one, launched or replayed."""
+    model = _half_line_model(pkg)
+    ids, state = torch.randint(0, 512, (B,), device="cuda"), torch.randn(B, 288, device="cuda").to(torch.bfloat16)
+    table, lens = torch.arange(B, dtype=torch.int32).view(B, 1), torch.full((B,), 3, dtype=torch.int32)
+
+    def step(dec):
+        return dec.step(ids, table, lens, input_states=state)[0].clone()
+
+    dec = pkg.PagedDecoder(model, num_blocks=B, block_size=16, num_steps=2, use_graph=use_graph)
+    first = [step(dec) for _ in range(3)]
+    assert torch.equal(first[0], first[2])
+    blk = model.transformer.core_block[0]
+    with torch.no_grad():
+        for w in (blk.attn.Wqkv.weight, blk.attn.proj.weight, blk.mlp.fc.weight):
+            w.mul_(1.5)
+    after = step(dec)
+    fresh = pkg.RavenForCausalLM(model.config, device="cuda", dtype=torch.bfloat16)
+    fresh.load_state_dict(model.state_dict())
+    other = pkg.PagedDecoder(fresh, num_blocks=B, block_size=16, num_steps=2)
+    for a, b in zip(other.k + other.v, dec.k + dec.v):
+        a.copy_(b)
+    assert not torch.equal(after, first[0]) and torch.equal(after, step(other))
