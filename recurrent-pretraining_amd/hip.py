@@ -662,9 +662,21 @@ def paged_decode_blocks(dims: Dims, blocks, x_in, x_out, freqs, kv: PagedKV, B, 
 def paged_chunk_blocks(dims: Dims, blocks, x_in, x_out, freqs, kv: PagedKV, positions, slot_mapping, q_start, max_q_len, workspace, adapter_w=None,
                        embeds=None, n_iterations=1, ln_f=None):
     """paged_decode_blocks for the new rows x_in [T, h] of several sequences, as paged_qkv_rope_append and paged_prefill_attention describe them."""
-    T, B = x_in.shape[0], q_start.shape[0] - 1
-    if positions.shape != (T,) or slot_mapping.shape != (T,) or x_out.shape != x_in.shape:
-        raise RavenHipError("paged_chunk_blocks: positions [T], slot_mapping [T] and x_out must match x_in [T, h]")
+    if x_in.dim() != 2 or x_in.shape[1] != dims.n_embd or x_out.shape != x_in.shape or dtype_code(x_in.dtype) != dims.dtype:
+        raise RavenHipError("paged_chunk_blocks: x_in and x_out [T, n_embd] of the model's type")
+    T = x_in.shape[0]
+    if positions.shape != (T,) or slot_mapping.shape != (T,):
+        raise RavenHipError("paged_chunk_blocks: positions [T] and slot_mapping [T] must match x_in [T, h]")
+    if (adapter_w is None) != (embeds is None) or (embeds is not None and (embeds.shape != x_in.shape or adapter_w.shape != (dims.n_embd, 2 * dims.n_embd))):
+        raise RavenHipError("paged_chunk_blocks: adapter_w [h, 2 h] and embeds [T, h] go together")
+    _, _, k_caches, _, table, lens = getattr(kv, "_keep", (None,) * 6)
+    if k_caches is None:
+        raise RavenHipError("paged_chunk_blocks: kv must come from make_paged_kv")
+    B = lens.shape[0]
+    if q_start.shape != (B + 1,) or table.shape[0] != B:
+        raise RavenHipError("paged_chunk_blocks: block_table [B, max_blocks], seq_lens [B] and q_start [B + 1] do not fit together")
+    if len(blocks) > len(k_caches) or _paged_dims(k_caches[0], kv.kv_layout)[1:] != (dims.n_heads, dims.head_dim) or k_caches[0].dtype != x_in.dtype:
+        raise RavenHipError(f"paged_chunk_blocks: {len(blocks)} blocks of {dims.n_heads} heads of {dims.head_dim} need as many caches of their shape and type")
     rows = PagedRows(_ptr(positions, "positions", torch.int64), _ptr(slot_mapping, "slot_mapping", torch.int64), _ptr(q_start, "q_start", torch.int32), T, B, int(max_q_len))
     rc = load().raven_paged_chunk_blocks(
         C.byref(dims), _ptr(adapter_w, "adapter_w", x_in.dtype), blocks, len(blocks), _ptr(ln_f, "ln_f", x_in.dtype), _ptr(x_in, "x_in"),

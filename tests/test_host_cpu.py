@@ -593,3 +593,40 @@ def test_generate_dispatch_follows_the_reference_keywords(pkg, monkeypatch):
     model.generate(ids, max_new_tokens=2)
     assert seen == ["generate_with_adaptive_compute", "generate_speculative", "generate_diffusion_style", "generate_minimal",
                     "generate_minimal", "generate_minimal", "transformers"]
+
+
+@pytest.mark.parametrize("wrong", ["q_start", "blocks", "heads", "head_dim", "layout", "width", "rows", "embeds", "no_adapter", "adapter", "kv_type", "type", "positions"])
+def test_paged_chunk_blocks_refuses_operands_that_do_not_fit_together(pkg, wrong):
+    """Block tables, caches and rows are read by these sizes on the device: every mismatch is refused on the host, before a pointer is taken (so also
+    without a GPU)."""
+    hip, dt = pkg.hip, torch.bfloat16
+    B, T, nh, hd, h = 3, 10, 2, 64, 128
+    cache = torch.zeros(5, nh, 8, hd, dtype=dt)
+    table, lens = torch.zeros(B, 4, dtype=torch.int32), torch.ones(B, dtype=torch.int32)
+    kv = hip.PagedKV(None, None, None, None, 4, 8, 32, hip.PAGED_HND)
+    kv._keep = (None, None, [cache] * 2, [cache] * 2, table, lens)
+    a = dict(dims=hip.make_dims(h, nh, 256, 1e-5, dt), blocks=(hip.BlockWeights * 2)(), x_in=torch.zeros(T, h, dtype=dt), x_out=torch.zeros(T, h, dtype=dt),
+             freqs=torch.zeros(32, hd // 2, 2), kv=kv, positions=torch.zeros(T, dtype=torch.int64), slot_mapping=torch.zeros(T, dtype=torch.int64),
+             q_start=torch.zeros(B + 1, dtype=torch.int32), max_q_len=4, workspace=torch.zeros(256, dtype=torch.uint8),
+             adapter_w=torch.zeros(h, 2 * h, dtype=dt), embeds=torch.zeros(T, h, dtype=dt))
+    with pytest.raises(hip.RavenHipError, match="must live on the GPU"):  # nothing to object to but the device
+        hip.paged_chunk_blocks(**a)
+    a.update({"q_start": {"q_start": torch.zeros(B + 2, dtype=torch.int32)},
+              "blocks": {"blocks": (hip.BlockWeights * 3)()},
+              "heads": {"dims": hip.make_dims(h, 1, 256, 1e-5, dt)},
+              "head_dim": {"dims": hip.make_dims(h, 4, 256, 1e-5, dt)},
+              "layout": {},
+              "width": {"x_in": torch.zeros(T, h + 8, dtype=dt), "x_out": torch.zeros(T, h + 8, dtype=dt)},
+              "rows": {"x_out": torch.zeros(T + 1, h, dtype=dt)},
+              "embeds": {"embeds": torch.zeros(T - 1, h, dtype=dt)},
+              "no_adapter": {"adapter_w": None},
+              "adapter": {"adapter_w": torch.zeros(h, h, dtype=dt)},
+              "kv_type": {},
+              "type": {"x_in": torch.zeros(T, h), "x_out": torch.zeros(T, h)},
+              "positions": {"positions": torch.zeros(T + 1, dtype=torch.int64)}}[wrong])
+    if wrong == "layout":
+        kv.kv_layout = hip.PAGED_NHD
+    if wrong == "kv_type":
+        kv._keep = (None, None, [cache.float()] * 2, [cache.float()] * 2, table, lens)
+    with pytest.raises(hip.RavenHipError, match="paged_chunk_blocks: "):
+        hip.paged_chunk_blocks(**a)
