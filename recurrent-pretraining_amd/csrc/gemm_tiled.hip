@@ -979,6 +979,10 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     // Units of gemm_mid.hip, which are cut to fill one round whatever the columns' number, take them where that is estimated faster (without K slices: same
     // bits).  us at 4000 rows, 1280 of 5280 columns, averaged over K of 5280, 10560 and 17920, small tiles / units: 191 / 120.  (Of a last round three quarters full,
     // 2 x 3072 of 2 x 17920 columns, the big tiles run into the round before: 1039 in one launch, 995 + 122 with units.)
+    // At most 128 columns whose sums leave unrounded belong to the narrow kernel: its waves add each of them up in parts, units here in one chain, twice as far
+    // from the exact sums (64 columns of K = 2048 behind 8128 x 10240: 1.32e-7 and 2.71e-7; of 2112 x 5280 at 8192 rows 2.2e-7 and 4.5e-7) for 2 to 23 % of the
+    // product's time (444 us and 433, 191 and 170).  Rounded ones take the units: nothing of that is left in them, and the same products take 281 us narrow and
+    // 274 with units, 167 and 153.
     const int64_t rest = big_tiles % 256;
     if (big && g_tiled_variant == 0 && g_tiled_split_tail && big_tiles > 256 && rest > 0 && rest <= 128 && rest % tiles_m == 0) {
         const int cols = (int)(rest / tiles_m);              // trailing tile columns
@@ -993,14 +997,14 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
         if (tail.epi.bias) tail.epi.bias += n_big;
         if (tail.epi.residual) tail.epi.residual += n_big;
         if (const int rc = launch(head, true)) return rc;
+        if (f32_sums && a.K1 == 0 && a.ldx == K0 && a.ldw == K0 && gemm_narrow_fits(M, tail.N, K0, RAVEN_BF16))
+            return gemm_narrow_free(tail.x0, tail.w, tail.y, tail.ldy, M, tail.N, K0, tail.epi, s);
         if (const MidPlan tail_plan = mid_plan(M, tail.N, K0, a.K1, swiglu, 0); tail_plan.nt) {
             const raven_epilogue e = tail.epi;
             const ProductArgs q{tail.w, tail.x0, tail.x1, tail.residual, tail.y, M, tail.N, K0, a.K1, a.ldw, a.ldx, a.ldy, a.up_off, swiglu, out_f32, epi ? &e : nullptr,
                                 rope ? &tail.rope : nullptr};
             return mid_gemm(q, tail_plan, nullptr, s, nullptr);
         }
-        if (epi && a.K1 == 0 && a.ldx == K0 && a.ldw == K0 && gemm_narrow_fits(M, tail.N, K0, RAVEN_BF16))
-            return gemm_narrow_free(tail.x0, tail.w, tail.y, tail.ldy, M, tail.N, K0, tail.epi, s);
         return launch(tail, false);
     }
     return launch(a, big);

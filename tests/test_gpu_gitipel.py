@@ -79,6 +79,19 @@ def test_linear_epilogue_narrow_rest_behind_large_tiles(pkg):
     assert ((got - ref).abs() <= ref.abs() * 2 ** -8 + 1e-4).all()
 
 
+@pytest.mark.parametrize("M,big,rest,K", [(4096, 4096, 64, 256), (3900, 4096, 16, 1056), (8192, 2048, 128, 2048), (2000, 8192, 112, 320)])
+def test_unrounded_rest_behind_large_tiles_adds_up_in_the_narrow_kernels_parts(pkg, M, big, rest, K):
+    """Float sums of up to 128 columns behind a whole round of 256 x 256 tiles are the narrow kernel's, to the bit: a chain over all of K is twice as far
+    from the exact ones."""
+    g = torch.Generator(device="cuda").manual_seed(rest)
+    N = big + rest
+    x, w = torch.randn(M, K, generator=g, device="cuda").to(BF16), (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(BF16)
+    bias, res = torch.randn(N, generator=g, device="cuda"), torch.randn(M, N, generator=g, device="cuda")
+    got = pkg.hip.linear_epilogue(x, w, bias=bias, residual=res, scale=0.5)
+    alone = pkg.hip.linear_epilogue(x, w[big:].contiguous(), bias=bias[big:].contiguous(), residual=res[:, big:].contiguous(), scale=0.5)
+    assert torch.equal(got[:, big:], alone)
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 2048, 96), (4200, 4096, 64), (16384, 1160, 128)])
 def test_linear_epilogue_large_tiles(pkg, M, N, K):
     """Shapes that take the 256 x 256 tiles, also with the last tile columns handed to small tiles."""
