@@ -905,16 +905,23 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const bf16* __restrict__
 // 17 to 32 rows, which else take the skinny kernels: gemm_mid.hip where K is long or the matrix large, and its rows (or their copies) are whole lines.
 // us, skinny kernels / these, at 20 rows, slices added by a launch of their own: 15840 x 5312 32.6 / 30.2, 2 x 17920 x 5312 64.2 / 60.8, 5280 x 17920 38.0 / 36.6,
 // 5280 x 5312 17.7 / 15.5, 2 x 5440 x 2048 12.6 / 11.3, 2048 x 5440 14.1 / 9.3, 2048 x 8192 14.1 / 11.0, 1280 x 5120 11.7 / 8.5; but 8192 x 2048 10.1 / 10.5,
-// 2048 x 2048 6.1 / 8.5, 3072 x 1536 5.6 / 7.4.  (16 rows: 1.04 to 1.08 where it is faster at all.)  f32_sums: the sums leave unrounded.  The skinny kernels add
+// 2048 x 2048 6.1 / 8.5, 3072 x 1536 5.6 / 7.4.  (16 rows: 1.04 to 1.08 where it is faster at all.)
+// Over 830 shapes of 1024 to 40000 weight rows and K of 512 to 18000 at 17, 24 and 32 rows the skinny kernels take 1.22 times as long (geometric mean; 0.88 at the
+// least, below 0.97 in 2 % of them), with two kinds of shapes left to them:
+// * K <= 4096 and at most 8192 weight rows, which are one round of their 32-row workgroups: 0.93 there (0.80 to 1.09; 7168 x 3072 11.6 / 13.3, 2 x 3584 x 4096 14.4 / 17.1);
+// * slices of whole 4 KB that units of eight weight tiles and more walk in step, so that all slices of a launch ask the same memory channels: 0.94
+//   (0.65 to 1.24; 4096 x 16384 in eight slices 33.1 / 51.2, 12288 x 8192 in four 35.9 / 49.7).
+// f32_sums: the sums leave unrounded.  The skinny kernels add
 // each of them up in eight parts, so they are left alone unless these take eight slices: whole sums of 10304 x 2048 are 2.7e-7 from the exact ones, eight parts 1.0e-7.
 static int few_rows_slices(int f32_sums) { return f32_sums ? 8 : 1; }
 bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_sums, const void* w, size_t workspace_bytes, bool aligned) {
     if (dtype != RAVEN_BF16 || !aligned || M < 17 || M > 32 || M >= g_tiled_min_rows || g_tiled_variant != 0 || K1 != 0 || K0 % 8 != 0 || N % 8 != 0) return false;
     const int64_t rows = (int64_t)N * (swiglu ? 2 : 1);
-    if (N < 1024 || rows > 40000 || rows * K0 >= (1ll << 31) || !(K0 > 4096 || (rows * K0 >= 20000000 && !f32_sums))) return false;
+    if (N < 1024 || rows > 40000 || rows * K0 >= (1ll << 31) || !(K0 > 4096 || (rows > 8192 && rows * K0 >= 20000000 && !f32_sums))) return false;
     int ld = 0;
     if (K0 % 64 != 0 && !(g_pad_decode_rows && packed_weight_of(w, (int)rows, K0, &ld))) return false;
-    return mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums)).nt != 0;
+    const MidPlan p = mid_plan(M, N, K0, 0, swiglu, workspace_bytes, few_rows_slices(f32_sums));
+    return p.nt != 0 && !(p.ks > 1 && K0 % (2048 * p.ks) == 0 && p.cols * (swiglu ? 2 : 1) > 7 * 16);
 }
 
 static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0,

@@ -213,6 +213,19 @@ def test_long_or_large_products_of_few_rows(pkg, M):
     check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :10000]).to(dt).float() * u[:, 10000:]).to(dt), dt, f"{M} x 10000 x 1024, SwiGLU", ulps=ULPS_SWIGLU)
 
 
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("N,K,swiglu,skinny", [(8192, 2560, 0, True), (8208, 2560, 0, False), (3584, 4096, 1, True), (4096, 16384, 0, True), (4096, 16448, 0, False),
+                                               (11008, 8192, 0, True), (11008, 8256, 0, False), (2560, 16384, 1, True)])
+def test_few_rows_stay_with_the_kernels_that_are_faster(pkg, tuned, M, N, K, swiglu, skinny):
+    """17 to 32 rows: matrices of up to 8192 rows and K <= 4096, and slices of whole 4 KB over wide units, are the skinny kernels' (their bits: the order of sums
+    differs); their neighbours are not."""
+    x, w = _gpu_randn((M, K), 800 + M), _gpu_randn((N * (1 + swiglu), K), 801, 0.02)
+    ws = pkg.hip.linear_workspace(M, N * (1 + swiglu), "cuda")
+    got = pkg.hip.linear(x, w, swiglu=bool(swiglu), workspace=ws)
+    tuned(gemm_mid=0)
+    assert torch.equal(got, pkg.hip.linear(x, w, swiglu=bool(swiglu), workspace=ws)) == skinny
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(33, 1536, 1536, 4), (40, 2048, 2048, 4), (60, 1792, 7168, 8), (80, 2048, 5440, 8), (100, 2304, 2304, 3), (165, 2048, 2048, 4),
                                          (165, 2048, 8192, 8), (230, 2048, 8192, 8), (300, 512, 2048, 3), (450, 1024, 4096, 4), (385, 1280, 5120, 6)])
 def test_float_sums_keep_the_parts_they_are_added_up_in(pkg, tuned, M, N, K, parts):
