@@ -100,8 +100,8 @@ const char* raven_last_error(void);
  * no tile-count rule, 3 = 256 x 256 by the eight-wave kernel instead of the four-wave ring kernel), gemm_tiled_split_tail
  * (1 = the tile columns of a last round that fills at most half the chip go to
  * 128 x 128 tiles, 0 = never), gemm_mid (1 = products over 33 and more bf16 rows that do not fill the chip with 256 x 256 tiles may run as
- * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (its largest
- * weight tiles, 1 to 6, and token tiles, 1 to 4, of a wave and its slice count, 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
+ * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (the
+ * weight tiles, 1 to 6, and token tiles, 1 to 4, of its waves, whether or not the product has so many, and its slice count; 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
  * gemm_one_round (1 = a 2..32-row product of up to about 16384 output columns runs as at most one workgroup of eight waves per compute unit where that is faster, 2 = wherever it is narrow enough, 0 = the
@@ -158,6 +158,9 @@ int raven_gemm_swiglu(const void* x, const void* fc, void* out,
  * fixed order.  The same holds from 33 rows on.
  * Without one (or where no split pays, or fp32) the call is forwarded to raven_gemm / _adapter_gemm_concat / _gemm_swiglu. */
 size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max);
+/* How the middle kernel would cut a bf16 product with room for workspace_bytes of slices, under the present knobs and without a launch:
+ * plan[6] = weight and token tiles of a wave at the most, columns and rows of a unit, K slices, units; all 0: it would not take it. */
+int    raven_middle_plan(int32_t M, int32_t N, int32_t K, int32_t swiglu, size_t workspace_bytes, int32_t* plan);
 int    raven_linear(const void* x0, const void* x1, const void* w, const void* residual, void* y,
                     int32_t M, int32_t N, int32_t K0, int32_t K1, int32_t swiglu, int32_t out_f32,
                     int32_t dtype, void* workspace, size_t workspace_bytes, void* stream);

@@ -476,16 +476,25 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room, int ks_fr
         MidPlan p{};
         p.tiles_m = (M + 64 * mt - 1) / (64 * mt);
         p.rows = ((M + p.tiles_m - 1) / p.tiles_m + 15) / 16 * 16;
+        if (g_mid_mt && p.rows < 64 * mt - 48) {  // the variant that was asked for, with tiles that have no rows
+            p.rows = 64 * mt - 48;
+            p.tiles_m = (M + p.rows - 1) / p.rows;
+        }
         p.mt = (p.rows + 63) / 64;
         for (int nt = 1; nt <= 6; ++nt) {
             if (g_mid_nt && nt != g_mid_nt) continue;
             for (p.ks = ks_from; p.ks <= kMidMaxSlices; ++p.ks) {
-                if (g_mid_ks && p.ks != g_mid_ks && p.ks < nk) continue;
+                if (g_mid_ks && p.ks != (g_mid_ks < nk ? g_mid_ks : nk)) continue;
                 const int cap = 32 * nt / side;  // output columns of the largest unit
                 // as few columns per unit as still run in the rounds that the largest unit needs
                 const int64_t whole = (int64_t)((N + cap - 1) / cap) * p.tiles_m * p.ks;
                 const int64_t tiles_n = (whole + cus - 1) / cus * cus / (p.tiles_m * p.ks);
                 p.cols = (int)((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
+                if (g_mid_nt) {  // as few units as hold the columns, with the variant's number of tiles
+                    const int fewest = (N + cap - 1) / cap, least = side == 2 ? 16 * nt - 8 : 32 * nt - 24;
+                    p.cols = ((N + fewest - 1) / fewest + 7) / 8 * 8;
+                    if (p.cols < least) p.cols = least;
+                }
                 if (p.cols > cap) p.cols = cap;
                 p.tiles_n = (N + p.cols - 1) / p.cols;
                 const int wtiles = (p.cols * side + 15) / 16;
@@ -693,3 +702,12 @@ int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int
 }
 
 }  // namespace raven
+
+extern "C" int raven_middle_plan(int32_t M, int32_t N, int32_t K, int32_t swiglu, size_t workspace_bytes, int32_t* plan) {
+    using namespace raven;
+    RAVEN_REQUIRE(plan && M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0, "middle_plan: bad arguments");
+    const MidPlan p = mid_plan(M, N, K, 0, swiglu, workspace_bytes);
+    const int32_t out[6] = {p.nt, p.mt, p.cols, p.rows, p.ks, p.tiles_m * p.tiles_n * p.ks};
+    for (int i = 0; i < 6; ++i) plan[i] = p.nt ? out[i] : 0;
+    return 0;
+}

@@ -131,6 +131,7 @@ SIGNATURES = {
     "raven_register_packed_weight": (C.c_int, [_VP, _I32, _I32, _VP, _VP]),
     "raven_unregister_packed_weight": (C.c_int, [_VP]),
     "raven_linear_workspace_bytes": (_SZ, [_I32, _I32]),
+    "raven_middle_plan": (C.c_int, [_I32, _I32, _I32, _I32, _SZ, C.POINTER(_I32)]),
     "raven_linear": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _VP, _SZ, _VP]),
     "raven_exit_logit_stats": (C.c_int, [_VP, _VP, _VP, _I32, _I32, _I32, _VP]),
     "raven_exit_latent_stats": (C.c_int, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _VP]),
@@ -355,6 +356,13 @@ def unregister_packed_weight(w: torch.Tensor) -> None:
 def linear_workspace(M, n_out_max, device):
     n = load().raven_linear_workspace_bytes(M, n_out_max)
     return torch.empty(max(n, 256), dtype=torch.uint8, device=device)
+
+
+def middle_plan(M, N, K, swiglu=False, workspace_bytes=0):
+    """(nt, mt, columns, rows, slices, units) by which gemm_mid.hip would cut the product, zeros where it would not take it; no launch."""
+    plan = (_I32 * 6)()
+    _check(load().raven_middle_plan(M, N, K, int(swiglu), workspace_bytes, plan), "raven_middle_plan")
+    return tuple(plan)
 
 
 def linear(x0, w, x1=None, residual=None, swiglu=False, out_f32=False, workspace=None):

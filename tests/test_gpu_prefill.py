@@ -144,9 +144,17 @@ def test_tiled_gemm_edges_against_oracle(pkg, tuned, variant, M, N, K):
         assert torch.equal(a, pkg.hip.linear(dev(x), dev(w))), (variant, other)
 
 
+def _assert_unit(pkg, M, N, K, nt, mt, ks, ws):
+    """The plain and the SwiGLU product run as units of 2 nt weight tiles or one less, 4 mt - 3 token tiles or more, in ks slices."""
+    for swiglu in (False, True):
+        n, m, cols, rows, slices, units = pkg.hip.middle_plan(M, N, K, swiglu, ws.numel())
+        wtiles = -(-cols * (2 if swiglu else 1) // 16)
+        assert (n, m, slices) == (nt, mt, ks) and wtiles in (2 * nt - 1, 2 * nt) and 4 * mt - 3 <= rows // 16 <= 4 * mt and units >= ks, (M, N, K, swiglu)
+
+
 @pytest.mark.parametrize("ks", [1, 3])
-@pytest.mark.parametrize("mt", [1, 2, 4])
-@pytest.mark.parametrize("nt", [2, 4, 6])
+@pytest.mark.parametrize("mt", [1, 2, 3, 4])
+@pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6])
 def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, ks):
     """gemm_mid.hip: every tile shape, whole and in K slices, at sizes where units, steps and tiles end early: columns that leave the last
     unit and its last tile partly filled, rows past the last tile, fewer K steps than the ring has stages, a K that is no
@@ -155,6 +163,7 @@ def test_products_of_a_middling_number_of_rows_in_every_cut(pkg, tuned, nt, mt, 
     for M, N, K in ((33, 72, 72), (130, 328, 200), (259, 1048, 456), (70, 200, 1096)):
         tuned(gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
         ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+        _assert_unit(pkg, M, N, K, nt, mt, min(ks, (K + 63) // 64), ws)
         x, w, res = _gpu_randn((M, K), 700 + M), _gpu_randn((N, K), 701 + N, 0.05), _gpu_randn((M, N), 702)
         z = x.float() @ w.float().T
         what = f"{M} x {N} x {K}"
@@ -185,6 +194,7 @@ def test_units_with_any_number_of_tiles(pkg, tuned, nt, M):
         for K in (232, 680):
             tuned(gemm_mid_nt=nt, gemm_mid_mt=min(4, (M + 63) // 64), gemm_mid_ks=1)
             ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+            _assert_unit(pkg, M, N, K, nt, min(4, (M + 63) // 64), 1, ws)
             x, w = _gpu_randn((M, K), 760 + M), _gpu_randn((N, K), 761 + N, 0.05)
             check(pkg.hip.linear(x, w, workspace=ws), (x.float() @ w.float().T).to(dt), dt, f"{M} x {N} x {K}")
             half = max(8, N // 2 // 8 * 8)
@@ -196,7 +206,7 @@ def test_units_with_any_number_of_tiles(pkg, tuned, nt, M):
 @pytest.mark.parametrize("M", [16, 17, 20, 32, 33])
 def test_long_or_large_products_of_few_rows(pkg, M):
     """17 to 32 rows against a matrix with a long K (1032 x 4160) or a large one (20000 x 1024, 2 x 10000 x 1024), and the row counts beside: rounded
-    results, SwiGLU, float sums added to a residual, slices left to the norm that follows."""
+    results, SwiGLU, float sums added to a residual."""
     dt = torch.bfloat16
     for N, K in ((1032, 4160), (20000, 1024)):
         ws = pkg.hip.linear_workspace(M, N, "cuda")
@@ -241,14 +251,16 @@ def test_float_sums_keep_the_parts_they_are_added_up_in(pkg, tuned, M, N, K, par
 
 
 @pytest.mark.parametrize("ks", [1, 3])
-@pytest.mark.parametrize("nt,mt", [(2, 1), (4, 2), (6, 4)])
+@pytest.mark.parametrize("nt,mt", [(1, 1), (2, 1), (3, 3), (4, 2), (5, 4), (6, 3), (6, 4)])
 def test_infinities_stay_in_their_rows_and_columns(pkg, tuned, nt, mt, ks):
-    """Rows and columns past the end of a tile are repeats of the last ones, pieces past K are zeros, a tile that does not exist repeats another: an
-    infinity or NaN of the last row of x, the last row of w or the last column must reach the outputs it belongs to and no other."""
+    """Rows and columns past the end of a tile are repeats of the last ones, pieces past K are zeros, waves with fewer tiles than their variant multiply
+    whatever lies behind them: an infinity or NaN of the last row of x, the last row of w or the last column must reach the outputs it belongs to and no
+    other.  (215 x 392: last units with fewer tiles a wave than the variant's less one.)"""
     dt = torch.bfloat16
-    for M, N, K in ((33, 72, 72), (130, 328, 200), (70, 200, 1096)):
+    for M, N, K in ((33, 72, 72), (130, 328, 200), (70, 200, 1096), (215, 392, 264)):
         tuned(gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
         ws = pkg.hip.linear_workspace(M, 2 * N, "cuda")
+        _assert_unit(pkg, M, N, K, nt, mt, min(ks, (K + 63) // 64), ws)
         x, w = _gpu_randn((M, K), 730 + M), _gpu_randn((2 * N, K), 731 + N, 0.05)
         x[M - 1, K - 1], x[0, 3] = float("inf"), float("nan")
         w[N - 1, 5] = w[2 * N - 1, 5] = float("inf")
@@ -315,18 +327,67 @@ def test_slices_of_many_rows_folded_into_the_norm_change_no_bit(pkg, tuned, M):
     check(pkg.hip.linear(a, w, workspace=tiny), (a.float() @ w.float().T).to(dt), dt, "without room for slices")
 
 
+@pytest.mark.parametrize("M", [17, 32])
+def test_slices_of_few_rows_folded_into_the_norm_change_no_bit(pkg, tuned, M):
+    """17 and 32 rows whose attn.proj and mlp.proj (K > 4096) the middle kernel cuts into K slices: added by the norm launches or by launches of their own, the
+    same bits; the skinny kernels' result within rounding."""
+    h, nh, inter, dt = 4224, 44, 4352, torch.bfloat16
+    mk = lambda seed, *s: _gpu_randn(s, seed, 0.02)
+    norms = [1 + mk(810 + i, h) for i in range(4)]
+    blk = pkg.hip.make_block_weights(*norms, *(keep := [mk(814, 3 * h, h), mk(815, 2, 1, nh, 96), mk(816, h, h), mk(817, 2 * inter, h), mk(818, h, inter)]))
+    dims = pkg.hip.make_dims(h, nh, inter, 1e-6, dt)
+    freqs = O.rope_table(96, M, 50000).to(dt).float().reshape(M, 48, 2).contiguous().cuda()
+    x, ws = _gpu_randn((M, h), 9), pkg.hip.block_workspace(dims, M, "cuda")
+    room = pkg.hip.linear_workspace(M, h, "cuda").numel()
+    assert pkg.hip.middle_plan(M, h, h, False, room)[4] > 1 and pkg.hip.middle_plan(M, h, inter, False, room)[4] > 1
+    outs = []
+    for fuse, mid in ((1, 1), (0, 1), (1, 0)):
+        tuned(fuse_sums_norm=fuse, gemm_mid=mid)
+        k, v = (torch.zeros(1, 1, nh, M, 96, dtype=dt, device="cuda") for _ in range(2))
+        out = pkg.hip.sandwich_block(dims, blk, x, torch.empty_like(x), freqs, pkg.hip.make_cache(k, v), 0, 1, M, 0, ws)
+        outs.append((out.clone(), k, v))
+    assert all(torch.equal(a, b) for a, b in zip(outs[0], outs[1]))
+    check(outs[0][0], outs[2][0].float(), dt, "the middle kernel against the skinny ones", ulps=ULPS_COMPOSED)
+    del keep
+
+
+def test_few_rows_read_a_copy_where_they_may(pkg, tuned):
+    """20 rows against 1032 x 4200, whose rows are not whole lines: with a registered copy the product is the middle kernel's and reads it; with
+    pad_decode_rows = 0, or without a copy, it reads the matrix."""
+    hip, dt, M, N, K = pkg.hip, torch.bfloat16, 20, 1032, 4200
+    x, w = _gpu_randn((M, K), 14), _gpu_randn((N, K), 15, 0.02)
+    ws, z = hip.linear_workspace(M, N, "cuda"), x.float() @ w.float().T
+    plain = hip.linear(x, w, workspace=ws)
+    packed = hip.register_packed_weight(w)
+    try:
+        w.mul_(2)  # (exact: the copy holds half of it)
+        copy = hip.linear(x, w, workspace=ws)
+        tuned(pad_decode_rows=0)
+        itself = hip.linear(x, w, workspace=ws)
+    finally:
+        hip.unregister_packed_weight(w)
+    check(plain, z.to(dt), dt, "without a copy")
+    check(copy, z.to(dt), dt, "the copy")
+    assert torch.equal(itself, plain * 2) and torch.equal(itself, hip.linear(x, w, workspace=ws))
+    del packed
+
+
 @pytest.mark.parametrize("N", [16640, 16544])
 def test_tiled_gemm_last_round_as_small_tiles_changes_no_bit(pkg, tuned, N):
     """4 x 65 tiles of 256 x 256 (4 x 130 under SwiGLU): the tiles of the last, nearly empty round (the last tile
-    columns, whole or partly filled) are multiplied as 128 x 128 tiles by a second launch over that column range.  Same
+    columns, whole or partly filled) are multiplied by a second launch over that column range, as units of the middle kernel here.  Same
     bits as one launch, for every epilogue, and right against the fp32 product on sampled columns of both ranges."""
     dt, M, K = torch.bfloat16, 1024, 192
     x, x1 = _gpu_randn((M, K), 600), _gpu_randn((M, K), 601)
     w, w2, res = _gpu_randn((N, K), 602, 0.05), _gpu_randn((N, 2 * K), 603, 0.05), _gpu_randn((M, N), 604)
-    fc = _gpu_randn((2 * N, K), 605, 0.05)
+    fc, bias = _gpu_randn((2 * N, K), 605, 0.05), _gpu_randn((N,), 606).float()
     calls = {"plain": lambda: pkg.hip.linear(x, w), "+ residual": lambda: pkg.hip.linear(x, w, residual=res),
              "float": lambda: pkg.hip.linear(x, w, out_f32=True), "two operands": lambda: pkg.hip.linear(x, w2, x1=x1),
-             "SwiGLU": lambda: pkg.hip.linear(x, fc, swiglu=True)}
+             "SwiGLU": lambda: pkg.hip.linear(x, fc, swiglu=True),
+             "gelu": lambda: pkg.hip.linear_epilogue(x, w, bias=bias, act=pkg.hip.ACT_GELU, out_f32=False),
+             "tanh": lambda: pkg.hip.linear_epilogue(x, w, bias=bias, act=pkg.hip.ACT_TANH, out_f32=False),
+             "unrounded": lambda: pkg.hip.linear_epilogue(x, w, bias=bias, residual=res.float(), scale=0.5)}
+    assert all(pkg.hip.middle_plan(M, N - 16384, k, swiglu)[0] for k, swiglu in ((K, False), (2 * K, False), (K, True)))
     for name, call in calls.items():
         tuned(gemm_tiled_split_tail=1)
         split = call()
