@@ -98,9 +98,10 @@ const char* raven_last_error(void);
  * non-zero also makes raven_linear use that kernel for every shape it accepts), gemm_tiled_min_rows (fewest rows, 33 or
  * more, that the tiled MFMA kernel takes), gemm_tiled_variant (0 = tile size by shape, 1 = 256 x 256, 2 = 128 x 128 and
  * no tile-count rule, 3 = 256 x 256 by the eight-wave kernel instead of the four-wave ring kernel), gemm_tiled_split_tail
- * (1 = the tile columns of a last round that fills at most half the chip go to
- * 128 x 128 tiles, 0 = never), gemm_mid (1 = products over 33 and more bf16 rows that do not fill the chip with 256 x 256 tiles may run as
- * units of the middle kernel, with K slices where a workspace allows; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (the
+ * (1 = the tile columns of a last round that fills at most half the chip go to smaller pieces: units of the middle kernel or 128 x 128 tiles,
+ * float sums of up to 128 columns to the narrow kernel; 0 = never), gemm_mid (1 = three kinds of bf16 products may run as units of the middle
+ * kernel, with K slices where a workspace allows: those over 33 and more rows that do not fill the chip with 256 x 256 tiles, those of 17 to 32 rows
+ * over K > 4096 or a large matrix, and last rounds; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (the
  * weight tiles, 1 to 6, and token tiles, 1 to 4, of its waves, whether or not the product has so many, and its slice count; 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
@@ -195,7 +196,7 @@ int raven_gemv_stream(const float* x, const float* norm, int32_t dim, float eps,
  * whose weight pointer is `w`, with this K and these rows, that runs on the tiled kernels reads the copy: same values in
  * the same order, same bits.  The caller registers again after changing w, and calls raven_unregister_packed_weight(w)
  * before it frees either buffer.  Products of fewer rows read w itself, but for 17..32 rows: decode steps of so many inside
- * raven_sandwich_block / raven_core_iteration(s) / raven_paged_decode_blocks take Wqkv and mlp.fc from the copies when both
+ * raven_sandwich_block / raven_core_iteration(s) / raven_paged_decode_blocks / raven_paged_chunk_blocks take Wqkv and mlp.fc from the copies when both
  * are registered for every block of the call, and a product over K > 4096 or a large matrix takes its copy where K is no
  * multiple of 64 (5 to 12 % faster, another summation order; see pad_decode_rows under raven_set_tuning). */
 int64_t raven_packed_weight_bytes(int32_t rows, int32_t K);

@@ -444,9 +444,10 @@ static size_t mid_lds_bytes(int waves, int nt, int mt, int ns, int wtiles, int x
 }
 
 // What a launch of a plan costs, in us, fitted to 3634 products of 33 to 4096 rows, 768 to 36000 columns and K of 768 to 18000 (standard deviation 9 %;
-// the plans it picks for 317 shapes are 1.0 % slower than the best of each).  First reads of the weights come at 8.8 TB/s, what comes out of the caches --
-// the token rows once per column of units, the weights again for further row tiles -- at 60; a K step takes its fragment reads, products and
-// requests; of the two the shorter one is hidden to two fifths.  Every round of units fills its ring and drains its outputs anew.
+// the plans it picks for 317 shapes are 1.0 % slower than the best of each).  The terms are fitted together, their divisors are no rates (a launch reads weights
+// at 5.8 TB/s at the most): bytes of weights by 8.8, bytes out of the caches -- the token rows once per column of units, the weights again for further
+// row tiles -- by 60; a K step takes its fragment reads, products and requests; of the two the shorter one is hidden to two fifths.  Every round of units
+// fills its ring and drains its outputs anew.
 static double mid_estimate(const MidPlan& p, int M, int N, int K, int side, int cus) {
     const int64_t mn = (int64_t)p.tiles_n * p.tiles_m;
     const int nk = (K + 63) / 64, wtiles = (p.cols * side + 15) / 16;

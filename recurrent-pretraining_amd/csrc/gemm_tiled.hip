@@ -980,7 +980,7 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
         return as_big ? launch_tiled<EPI_PLAIN, 4, 2>(t, s) : launch_tiled<EPI_PLAIN, 2, 1>(t, s);
     };
     // The last round of 256 x 256 tiles: when it would fill at most half of the 256 CUs and is whole tile columns, those
-    // columns are multiplied as 128 x 128 tiles instead -- four times as many workgroups, a quarter of the time each
+    // columns are multiplied in smaller pieces.  As 128 x 128 tiles, four times as many workgroups, a quarter of the time each
     // (5.25 rounds of work then take about 5.4 rounds instead of 6: the N = 5280 products of the model at 16384 rows;
     // mlp.fc of a 512-token prompt: 280 tiles, 1.3 rounds instead of 2).
     // Units of gemm_mid.hip, which are cut to fill one round whatever the columns' number, take them where that is estimated faster (without K slices: same
