@@ -137,9 +137,11 @@ class PagedDecoder:
             state = m.initialize_state(embeds, init_scale) if init_scale > 0 else torch.zeros_like(embeds)
         else:
             state = input_states.reshape(T, -1).to(dev, m.dtype)
-        if self.r > 0 and T > 0:
+        if self.r > 0 and T > 0 and n_core > 0:
             latents = blocks(t.core_block, n_pre, state.contiguous(), adapter_w=t.adapter.weight, embeds=embeds, n_iterations=self.r, ln_f=t.ln_f.weight)
         else:
+            for _ in range(self.r if T > 0 else 0):  # a core of no blocks: the adapter alone
+                state = hip.linear(state.contiguous(), t.adapter.weight, x1=embeds, workspace=hip.linear_workspace(T, cfg.n_embd, dev))
             latents = hip.rmsnorm_residual(state, t.ln_f.weight, cfg.norm_eps)[0]
         if cfg.n_layers_in_coda > 0 and T > 0:
             x = blocks(t.coda, n_pre + n_core, latents, ln_f=t.ln_f.weight)

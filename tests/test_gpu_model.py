@@ -1520,6 +1520,48 @@ def test_mixed_rows_see_weights_changed_without_a_trace(pkg, chunk):
     assert torch.equal(_paged_step(pkg, model, chunk), _paged_step(pkg, fresh, chunk))
 
 
+@pytest.mark.parametrize("n_pre,n_coda,T", [(1, 0, 5), (0, 1, 40), (1, 1, 20)])
+def test_mixed_rows_of_stacks_without_blocks(pkg, n_pre, n_coda, T):
+    """forward_tokens without blocks in the core: every recurrence is the adapter's product alone, the closing norm follows; likewise without prelude or coda."""
+    hip, dt, h = pkg.hip, torch.bfloat16, 192
+    cfg = pkg.RavenConfig(n_embd=h, n_heads=2, n_layers=n_pre + n_coda, n_layers_in_prelude=n_pre, n_layers_in_recurrent_block=0, n_layers_in_coda=n_coda,
+                          intermediate_size=256, vocab_size=512, mean_recurrence=2)
+    torch.manual_seed(19)
+    model = pkg.RavenForCausalLM(cfg, device="cuda", dtype=dt)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0.0, 0.05)
+    t, eps = model.transformer, cfg.norm_eps
+    ids, state, bs = torch.randint(0, 512, (T,), device="cuda"), torch.randn(T, h, device="cuda").to(dt), 8
+    table, pos = torch.arange((T + bs - 1) // bs, dtype=torch.int32)[None], torch.arange(T)
+
+    def decoder():
+        return pkg.PagedDecoder(model, num_blocks=table.numel(), block_size=bs, num_steps=2)
+
+    logits, latents = decoder().forward_tokens(ids, pos, pos, table, torch.tensor([T], dtype=torch.int32), torch.tensor([0, T], dtype=torch.int32), T, input_states=state)
+    dec = decoder()
+
+    def block(blk, f, x, **kw):
+        kv = hip.make_paged_kv(dec.k[f:f + 1], dec.v[f:f + 1], table.cuda(), torch.tensor([T], dtype=torch.int32, device="cuda"), table.numel() * bs, layout=dec.layout)
+        dims = model._natives()["dims"]
+        return hip.paged_chunk_blocks(dims, (hip.BlockWeights * 1)(blk.native()), x, torch.empty_like(x), model._natives()["freqs"], kv, pos.cuda(), pos.cuda(),
+                                      torch.tensor([0, T], dtype=torch.int32, device="cuda"), T, hip.block_workspace(dims, T, "cuda"), **kw)
+
+    embeds = hip.embed(t.wte.weight, ids, model.emb_scale)
+    if n_pre:
+        embeds = block(t.prelude[0], 0, embeds)
+    for _ in range(2):
+        state = torch.cat([state, embeds], 1).float() @ t.adapter.weight.float().T
+        state = state.to(dt)
+    want = hip.rmsnorm_residual(state, t.ln_f.weight, eps)[0]
+    check(latents, want, dt, "latents", ulps=ULPS_COMPOSED)
+    if n_coda:
+        x = block(t.coda[0], n_pre, latents, ln_f=t.ln_f.weight)
+    else:
+        x = hip.rmsnorm_residual(latents, t.ln_f.weight, eps)[0]
+    assert torch.equal(logits, hip.gemm(x, model.lm_head.weight, out_f32=True))
+
+
 @pytest.mark.parametrize("B,use_graph", [(20, False), (20, True), (40, True)])
 def test_paged_steps_follow_weights_that_change_between_them(pkg, B, use_graph):
     """Steps of 17 sequences and more read line-aligned copies (17 to 32 rows Wqkv, mlp.fc and long products, 33 and more attn.proj too): an in-place
