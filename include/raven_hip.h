@@ -162,6 +162,8 @@ size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max);
 /* How the middle kernel would cut a bf16 product with room for workspace_bytes of slices, under the present knobs and without a launch:
  * plan[6] = weight and token tiles of a wave at the most, columns and rows of a unit, K slices, units; all 0: it would not take it. */
 int    raven_middle_plan(int32_t M, int32_t N, int32_t K, int32_t swiglu, size_t workspace_bytes, int32_t* plan);
+/* The same for the grouped products of mixtures in tiles of 32 or 64 rows: unit[3] = columns, 16-row weight tiles and bytes of LDS of a unit. */
+int    raven_grouped_unit(int32_t N, int32_t swiglu, int32_t tile_rows, int32_t* unit);
 int    raven_linear(const void* x0, const void* x1, const void* w, const void* residual, void* y,
                     int32_t M, int32_t N, int32_t K0, int32_t K1, int32_t swiglu, int32_t out_f32,
                     int32_t dtype, void* workspace, size_t workspace_bytes, void* stream);

@@ -118,11 +118,14 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, int m, int n, f32x4 
     }
 }
 
+// kilobyte pieces, two a tile, that a workgroup of so many waves asks for per step where its variant has room for so many tiles
+__host__ __device__ constexpr int mid_requests(int tiles, int waves) { return (2 * tiles + waves - 1) / waves * waves; }
+
 // GROUPED: row groups with a weight matrix each; a unit works on a copy of the arguments cut to its group's rows
 // ONCE: every weight row is read by one unit
 template <int WN, int WM, int NT, int MT, int NS, bool ONCE, bool GROUPED = false>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
-    constexpr int NW = WN * WM, WPW = (2 * WN * NT + NW - 1) / NW, XPW = (2 * WM * MT + NW - 1) / NW, LPW = WPW + XPW;  // requests of a wave per step
+    constexpr int NW = WN * WM, WPW = mid_requests(WN * NT, NW) / NW, XPW = mid_requests(WM * MT, NW) / NW, LPW = WPW + XPW;  // requests of a wave per step
     static_assert(NW % 2 == 0 && (NS - 1) * LPW < 64, "a wave's pieces have one parity; the wait counter holds 63 requests");
     extern __shared__ __align__(1024) unsigned char smem[];
 
@@ -437,9 +440,11 @@ static constexpr int mid_stages(int nt, int mt) {
     return fit > 8 ? 8 : fit < 3 ? 3 : fit;
 }
 
-// LDS of a unit: the ring and the kilobyte behind it, where requests are left over, or the sums on their way out
-static size_t mid_lds_bytes(int waves, int nt, int mt, int ns, int wtiles, int xtiles) {
-    const size_t ring = (size_t)ns * (wtiles + xtiles) * 2048 + (2 * wtiles % waves || 2 * xtiles % waves ? 1024 : 0), sums = (size_t)waves * (mt % 2 ? 1 : 2) * 16 * (nt * 64 + 16);
+// LDS of a unit of WN x WM waves: the ring and the kilobyte behind it, where more is asked for than the unit has pieces, or the sums on their way out
+static size_t mid_lds_bytes(int wn, int wm, int nt, int mt, int ns, int wtiles, int xtiles) {
+    const int waves = wn * wm;
+    const bool spare = mid_requests(wn * nt, waves) > 2 * wtiles || mid_requests(wm * mt, waves) > 2 * xtiles;
+    const size_t ring = (size_t)ns * (wtiles + xtiles) * 2048 + (spare ? 1024 : 0), sums = (size_t)waves * (mt % 2 ? 1 : 2) * 16 * (nt * 64 + 16);
     return ring > sums ? ring : sums;
 }
 
@@ -500,7 +505,7 @@ static MidPlan find_plan(int M, int N, int K, int swiglu, size_t room, int ks_fr
                 p.tiles_n = (N + p.cols - 1) / p.cols;
                 const int wtiles = (p.cols * side + 15) / 16;
                 p.nt = (wtiles + 1) / 2;
-                if (mid_lds_bytes(8, p.nt, p.mt, mid_stages(p.nt, p.mt), wtiles, p.rows / 16) > (size_t)kLds) continue;
+                if (mid_lds_bytes(2, 4, p.nt, p.mt, mid_stages(p.nt, p.mt), wtiles, p.rows / 16) > (size_t)kLds) continue;
                 if (p.ks > 1 && (int64_t)p.tiles_n * p.tiles_m * p.ks > cus + cus / 32 && !g_mid_ks) break;
                 if (p.ks > 1 && nk / p.ks < (g_mid_ks ? 1 : 6)) break;
                 if (mid_workspace_bytes(M, N, p, swiglu) > room) break;
@@ -593,7 +598,7 @@ static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
         }
         attr_set = true;
     }
-    const size_t lds = mid_lds_bytes(8, NT, MT, NS, a.wtiles, a.xtiles);
+    const size_t lds = mid_lds_bytes(2, 4, NT, MT, NS, a.wtiles, a.xtiles);
     RAVEN_REQUIRE(lds <= (size_t)kLds && a.wtiles <= 2 * NT && a.wtiles > 2 * (NT - 1) && a.xtiles <= 4 * MT && a.xtiles > 4 * (MT - 1), "gemm (mid): a unit of %d x %d does not fit", a.cols, a.bm);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n * a.ks;
     gemm_mid_kernel<2, 4, NT, MT, NS, ONCE><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
@@ -650,6 +655,11 @@ int mid_gemm(const ProductArgs& q, const MidPlan& p, void* workspace, hipStream_
     return launch_mid(a, p, s, finish);
 }
 
+// LDS of a unit of row groups
+static size_t grouped_lds_bytes(int tile_rows, int wtiles, int xtiles) {
+    return tile_rows == 32 ? mid_lds_bytes(4, 1, 2, 2, 4, wtiles, xtiles) : mid_lds_bytes(2, 4, 4, 1, 3, wtiles, xtiles);
+}
+
 template <int WN, int WM, int NT, int MT, int NS>
 static int launch_grouped(const MidArgs& a, hipStream_t s) {
     static bool attr_set = false;
@@ -661,7 +671,7 @@ static int launch_grouped(const MidArgs& a, hipStream_t s) {
         }
         attr_set = true;
     }
-    const size_t lds = mid_lds_bytes(WN * WM, NT, MT, NS, a.wtiles, a.xtiles);
+    const size_t lds = grouped_lds_bytes(a.bm, a.wtiles, a.xtiles);
     RAVEN_REQUIRE(lds <= (size_t)kLds && a.wtiles <= WN * NT && a.wtiles >= WN * NT / 2 && a.xtiles == WM * MT, "gemm (grouped): a unit of %d columns does not fit", a.cols);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n;
     RAVEN_REQUIRE(units < (1 << 28), "gemm (grouped): too many units");
@@ -680,6 +690,12 @@ static int launch_grouped_rows(const MidArgs& a, hipStream_t s) {
     }
 }
 
+// output columns of a unit, at least half of the variant's tiles
+static int grouped_cols(int N, int swiglu) {
+    const int cap = 128 / (swiglu ? 2 : 1), tiles_n = (N + cap - 1) / cap, cols = ((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
+    return cols < cap / 2 ? cap / 2 : cols;
+}
+
 int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int N, int K, int swiglu, int out_f32, const RowGroups& g, hipStream_t s) {
     RAVEN_REQUIRE(x && w && y && g.group_of && g.group_row && g.group_end && g.used && g.n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 &&
                       (!swiglu || (g.x_scale && !out_f32)) && (g.extra_group < 0 || g.w_extra), "gemm (grouped): bad arguments");
@@ -689,12 +705,9 @@ int mid_grouped(const void* x, int x_rows, const void* w, void* y, int rows, int
     a.x0 = static_cast<const bf16*>(x);
     a.y = y;
     a.M = rows; a.N = N; a.K0 = K; a.ldw = K; a.ldx = K; a.ldy = N; a.up_off = N; a.out_f32 = out_f32;
-    const int side = swiglu ? 2 : 1, cap = 128 / side;
-    const int tiles_n = (N + cap - 1) / cap;
-    a.cols = ((N + tiles_n - 1) / tiles_n + 7) / 8 * 8;
-    if (a.cols < cap / 2) a.cols = cap / 2;
+    a.cols = grouped_cols(N, swiglu);
     a.kind = swiglu ? EPI_SWIGLU : EPI_FREE;
-    a.wtiles = (a.cols * side + 15) / 16;
+    a.wtiles = (a.cols * (swiglu ? 2 : 1) + 15) / 16;
     a.tiles_n = (N + a.cols - 1) / a.cols;
     a.bm = g.tile_rows; a.xtiles = (g.tile_rows + 15) / 16; a.tiles_m = g.n_tiles; a.ks = 1;
     a.epi.scale = 1.f;
@@ -710,5 +723,15 @@ extern "C" int raven_middle_plan(int32_t M, int32_t N, int32_t K, int32_t swiglu
     const MidPlan p = mid_plan(M, N, K, 0, swiglu, workspace_bytes);
     const int32_t out[6] = {p.nt, p.mt, p.cols, p.rows, p.ks, p.tiles_m * p.tiles_n * p.ks};
     for (int i = 0; i < 6; ++i) plan[i] = p.nt ? out[i] : 0;
+    return 0;
+}
+
+extern "C" int raven_grouped_unit(int32_t N, int32_t swiglu, int32_t tile_rows, int32_t* unit) {
+    using namespace raven;
+    RAVEN_REQUIRE(unit && N > 0 && N % 8 == 0 && (tile_rows == 32 || tile_rows == 64), "grouped_unit: bad arguments");
+    const int cols = grouped_cols(N, swiglu), wtiles = (cols * (swiglu ? 2 : 1) + 15) / 16;
+    unit[0] = cols;
+    unit[1] = wtiles;
+    unit[2] = (int32_t)grouped_lds_bytes(tile_rows, wtiles, tile_rows / 16);
     return 0;
 }

@@ -132,6 +132,7 @@ SIGNATURES = {
     "raven_unregister_packed_weight": (C.c_int, [_VP]),
     "raven_linear_workspace_bytes": (_SZ, [_I32, _I32]),
     "raven_middle_plan": (C.c_int, [_I32, _I32, _I32, _I32, _SZ, C.POINTER(_I32)]),
+    "raven_grouped_unit": (C.c_int, [_I32, _I32, _I32, C.POINTER(_I32)]),
     "raven_linear": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _VP, _SZ, _VP]),
     "raven_exit_logit_stats": (C.c_int, [_VP, _VP, _VP, _I32, _I32, _I32, _VP]),
     "raven_exit_latent_stats": (C.c_int, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _VP]),
@@ -363,6 +364,13 @@ def middle_plan(M, N, K, swiglu=False, workspace_bytes=0):
     plan = (_I32 * 6)()
     _check(load().raven_middle_plan(M, N, K, int(swiglu), workspace_bytes, plan), "raven_middle_plan")
     return tuple(plan)
+
+
+def grouped_unit(N, swiglu, tile_rows):
+    """(columns, 16-row weight tiles, bytes of LDS) of a unit of gemm_mid.hip's grouped products; no launch."""
+    unit = (_I32 * 3)()
+    _check(load().raven_grouped_unit(N, int(swiglu), tile_rows, unit), "raven_grouped_unit")
+    return tuple(unit)
 
 
 def linear(x0, w, x1=None, residual=None, swiglu=False, out_f32=False, workspace=None):

@@ -630,3 +630,16 @@ def test_paged_chunk_blocks_refuses_operands_that_do_not_fit_together(pkg, wrong
         kv._keep = (None, None, [cache.float()] * 2, [cache.float()] * 2, table, lens)
     with pytest.raises(hip.RavenHipError, match="paged_chunk_blocks: "):
         hip.paged_chunk_blocks(**a)
+
+
+@pytest.mark.parametrize("tile_rows,waves,stages", [(32, 4, 4), (64, 8, 3)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_grouped_units_have_room_for_every_request(pkg, tile_rows, waves, stages, swiglu):
+    """The waves of a grouped product ask for 16 kilobyte pieces of weights a step, whatever the unit has: those past its last tile land in a kilobyte behind
+    the ring, which has to belong to the launch.  Two units of 32 rows fit a CU."""
+    for N in range(8, 4097, 8):
+        cols, wtiles, lds = pkg.hip.grouped_unit(N, swiglu, tile_rows)
+        assert 4 <= wtiles <= 8 and cols * (2 if swiglu else 1) <= 16 * wtiles, N
+        ring = stages * (wtiles + tile_rows // 16) * 2048
+        assert lds >= ring + (1024 if 2 * wtiles < 16 else 0), (N, wtiles, lds, ring)
+        assert lds <= 160 * 1024 // (2 if tile_rows == 32 else 1), N
