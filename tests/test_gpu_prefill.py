@@ -223,6 +223,19 @@ def test_long_or_large_products_of_few_rows(pkg, M):
     check(pkg.hip.linear(x, fc, swiglu=True, workspace=ws), (F.silu(u[:, :10000]).to(dt).float() * u[:, 10000:]).to(dt), dt, f"{M} x 10000 x 1024, SwiGLU", ulps=ULPS_SWIGLU)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 1024, 4160), (24, 2048, 5440), (32, 2048, 8192), (20, 1280, 17920), (29, 5280, 5312), (32, 10304, 2048)])
+def test_float_sums_of_few_rows_are_as_near_as_the_skinny_kernels(pkg, tuned, M, N, K):
+    """Sums that leave unrounded, 17 to 32 rows: no further from the exact ones than those of the skinny kernels, which add each up in eight parts; one chain
+    is twice as far.  (1.05: the error of M x N sums varies by less than a hundredth.)"""
+    x, w = _gpu_randn((M, K), 795 + M), _gpu_randn((N, K), 796, 0.05)
+    exact, ws = x.double() @ w.double().T, pkg.hip.linear_workspace(M, N, "cuda")
+    far = lambda: ((pkg.hip.linear_epilogue(x, w, workspace=ws).double() - exact).norm() / exact.norm()).item()
+    got = far()
+    tuned(gemm_mid=0)
+    bar = far()
+    assert got < 1.05 * bar, f"{M} x {N} x {K}: {got:.3g}, skinny kernels {bar:.3g}"
+
+
 @pytest.mark.parametrize("M", [17, 32])
 @pytest.mark.parametrize("N,K,swiglu,skinny", [(8192, 2560, 0, True), (8208, 2560, 0, False), (3584, 4096, 1, True), (4096, 16384, 0, True), (4096, 16448, 0, False),
                                                (11008, 8192, 0, True), (11008, 8256, 0, False), (2560, 16384, 1, True)])
