@@ -364,6 +364,28 @@ def test_slices_of_few_rows_folded_into_the_norm_change_no_bit(pkg, tuned, M):
     del keep
 
 
+@pytest.mark.parametrize("h, nh, ks", [(64, 1, 1), (2048, 32, 8), (2080, 26, 5), (8192, 64, 2)])
+def test_rows_formed_from_slices_have_the_norm_of_stored_rows(pkg, tuned, h, nh, ks):
+    """Rows of fewer than 256 pieces of eight columns, exactly as many, a few more (in padded rows) and the most there may be: the launch that adds the slices of
+    attn.proj and mlp.proj and norms the sums gives the bits of the launches that do one after the other."""
+    M, inter, dt = 33, 1536, torch.bfloat16
+    mk = lambda seed, *s: _gpu_randn(s, seed, 0.02)
+    norms = [1 + mk(910 + i, h) for i in range(4)]
+    blk = pkg.hip.make_block_weights(*norms, *(keep := [mk(914, 3 * h, h), mk(915, 2, 1, nh, h // nh), mk(916, h, h), mk(917, 2 * inter, h), mk(918, h, inter)]))
+    dims = pkg.hip.make_dims(h, nh, inter, 1e-6, dt)
+    hd = h // nh
+    freqs = O.rope_table(hd, M, 50000).to(dt).float().reshape(M, hd // 2, 2).contiguous().cuda()
+    x, ws = _gpu_randn((M, h), 9), pkg.hip.block_workspace(dims, M, "cuda")
+    outs = []
+    for fuse in (1, 0):
+        tuned(fuse_sums_norm=fuse, gemm_mid_ks=ks)
+        k, v = (torch.zeros(1, 1, nh, M, hd, dtype=dt, device="cuda") for _ in range(2))
+        out = pkg.hip.sandwich_block(dims, blk, x, torch.empty_like(x), freqs, pkg.hip.make_cache(k, v), 0, 1, M, 0, ws)
+        outs.append((out.clone(), k, v))
+    assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
+    del keep
+
+
 def test_few_rows_read_a_copy_where_they_may(pkg, tuned):
     """20 rows against 1032 x 4200, whose rows are not whole lines: with a registered copy the product is the middle kernel's and reads it; with
     pad_decode_rows = 0, or without a copy, it reads the matrix."""
