@@ -10,7 +10,7 @@
 //     the attention kernel; one closing norm_4 (+ ln_f) launch per call.
 //   several rows: the residual adds still ride in the GEMM epilogues, norm_2 + norm_3 are one launch, and
 //     inside an iteration norm_4 of one block and norm_1 of the next are one launch.  From 33 rows on the five
-//     products are tiles on the matrix cores (SwiGLU and the residual adds in their epilogues, the adapter's two
+//     products are tiles on the matrix cores (SwiGLU and the residual adds in their epilogues, a single recurrence's adapter
 //     operands as two K segments), and chunks of 16 or more rows per sequence attend through the MFMA kernel.
 
 #include "raven_common.h"
@@ -28,6 +28,7 @@ int gemv1_column_block(const void* x, const void* norm_a, const void* w_block, i
 int linear_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K,
                         void* workspace, size_t workspace_bytes, hipStream_t s);
 
+bool column_block_fits(int M, int N, int K, int ldw, size_t workspace_bytes, bool aligned);
 int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, int ldw, const float* extra, const void* residual, void* y, int M,
                       int N, int K0, int K1, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 
@@ -70,7 +71,7 @@ int g_pad_decode_rows = 1; // raven_set_tuning("pad_decode_rows"): 0 = decode st
 struct BlockScratch {
     char *n1, *qkv, *q, *ya, *x1, *x2, *n3, *g, *x3, *xa, *xr;
     int ld_pad;     // n1, ya and n3 have room for rows this many elements apart (n_embd, or the next multiple of 64 for chunks)
-    float* e_sums;  // up to 32 rows: fp32 sums of the adapter's embedding half, computed once for all recurrences
+    float* e_sums;  // fp32 sums of the adapter's embedding half, computed once for all recurrences (bf16; up to 32 rows of floats for the one-row kernels)
     void* attn_ws;
     size_t attn_ws_bytes;
     void* lin_ws;
@@ -104,7 +105,7 @@ static size_t carve(const raven_dims* d, int M, char* base, BlockScratch* out) {
     s.x3 = take(row);
     s.xa = take(row);
     s.xr = take(row);
-    s.e_sums = reinterpret_cast<float*>(take(M <= 32 ? (size_t)M * d->n_embd * sizeof(float) : 0));
+    s.e_sums = reinterpret_cast<float*>(take(M <= 32 || d->dtype == RAVEN_BF16 ? (size_t)M * d->n_embd * sizeof(float) : 0));
     s.attn_ws_bytes = raven_decode_attention_workspace_bytes(M, d->n_heads, d->head_dim);
     s.attn_ws = s.attn_ws_bytes ? take(s.attn_ws_bytes) : nullptr;
     const int widest = 3 * d->n_embd > 2 * d->intermediate ? 3 * d->n_embd : 2 * d->intermediate;
@@ -367,9 +368,13 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
         }
         return close_one_row(dims, s, last_blk.norm_4, ln_f, state_out, stream);
     }
-    // 2..32 rows in bf16: the adapter is split by columns as for one row (embedding half summed once, in fp32)
-    const bool split = adapter_w && n_iterations >= 2 && dims->dtype == RAVEN_BF16 && M >= 2 && M <= 32 && h % 32 == 0 && h >= 256 &&
-                       s.lin_ws;
+    // bf16: the adapter is split by columns as for one row (embedding half summed once, in fp32).  From 33 rows on that is one launch more for half of
+    // every other one, which a few recurrences of a small adapter don't repay: from 32 MB of weights that are not read again on.  us per recurrence at 5280 columns, whole / split: 93
+    // rows 38.5 / 21, 195 rows 41 / 26; eight recurrences of 4000 rows take 1.3 ms of 101 less.
+    const bool split = adapter_w && n_iterations >= 2 && dims->dtype == RAVEN_BF16 && s.lin_ws &&
+                       (M <= 32 ? h % 32 == 0 && h >= 256
+                                : (int64_t)(n_iterations - 1) * h * h * 2 >= (32 << 20) &&
+                                      column_block_fits(M, h, h, 2 * h, s.lin_ws_bytes, raven_host::aligned16(adapter_w, static_cast<const char*>(adapter_w) + (size_t)h * 2, state_in, embeds, state_out)));
     if (split)
         if ((rc = linear_column_block(embeds, static_cast<const char*>(adapter_w) + (size_t)h * 2, 2 * h, nullptr, s.e_sums, 1, M, h, h,
                                       s.lin_ws, s.lin_ws_bytes, hs))) return rc;

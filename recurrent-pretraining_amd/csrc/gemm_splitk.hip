@@ -34,6 +34,8 @@ int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const voi
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
                     void* workspace, size_t workspace_bytes, hipStream_t s);
+int tiled_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K, void* workspace,
+                       size_t workspace_bytes, hipStream_t s, int* ks_left);
 int gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
               hipStream_t s);
 
@@ -346,12 +348,17 @@ static int launch_ns(NsArgs a, void* workspace, size_t workspace_bytes, hipStrea
     return raven_host::check_launch("linear (split-K MFMA)");
 }
 
-// Column block [c0, c0 + K) of a wider bf16 weight matrix with row pitch ldw, for 2..32 rows:
+// Column block [c0, c0 + K) of a wider bf16 weight matrix with row pitch ldw, for 2..32 rows and those that column_block_fits names:
 // y = round(x W[:, c0 : c0 + K]^T + extra), or the unrounded fp32 sums (raw_out) that a later call takes as `extra`.
 // The adapter product over [state, embedding] (recpre/raven_modeling_minimal.py:776) is split with it when the
 // embedding half stays the same over many calls; the product keeps its single rounding.
+bool column_block_fits(int M, int N, int K, int ldw, size_t workspace_bytes, bool aligned) {
+    return M >= g_tiled_min_rows && M > 32 && ldw % 8 == 0 && (int64_t)N * 2 * ldw < (1ll << 31) && aligned && tiled_gemm_fits(M, N, K, 0, RAVEN_BF16, 0, workspace_bytes, true, 0) &&
+           tiled_gemm_fits(M, N, K, 0, RAVEN_BF16, 0, workspace_bytes, true, 1);
+}
 int linear_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K,
                         void* workspace, size_t workspace_bytes, hipStream_t s) {
+    if (M > 32) return tiled_column_block(x, w_block, ldw, extra, y, raw_out, M, N, K, workspace, workspace_bytes, s, nullptr);
     if (M < 2 || M > 32 || N % 16 || K % 32 || K < 256 || !workspace || ((uintptr_t)workspace & 255)) {
         raven_host::set_error("linear_column_block: unsupported shape M=%d N=%d K=%d", M, N, K);
         return -1;
@@ -381,6 +388,7 @@ int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, in
     const bool aligned = raven_host::aligned16(x0, x1, w, residual, y);
     if (!ldw && ((M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned)) || (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, 0, 0, w, room, aligned))))
         return tiled_gemm(x0, ldx, x1, w, residual, y, M, N, K0, K1, 0, 0, workspace, room, s, g_fuse_sums_norm && N <= 8192 ? ks_left : nullptr);
+    if (ldw && M > 32) return tiled_column_block(x0, w, ldw, extra, y, 0, M, N, K0, workspace, room, s, g_fuse_sums_norm && N <= 8192 ? ks_left : nullptr);
     RAVEN_REQUIRE(ldx == 0 || ldx == K0, "linear: rows of x0 %d elements apart", ldx);
     bool split = g_fuse_sums_norm && dtype == RAVEN_BF16 && M >= 2 && M <= 32 && N % 16 == 0 && N <= 8192 && K0 % 32 == 0 && K1 % 32 == 0 &&
                  workspace != nullptr && ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 8 && M > g_linear_min_rows;

@@ -93,7 +93,7 @@ __device__ __forceinline__ void store_tiles(const TiledArgs& a, const f32x4 (&ac
                     o[i] = from_f32<bf16>(round_to<bf16>(silu_f32(g)) * u);
                 }
                 *reinterpret_cast<u32x2*>(static_cast<bf16*>(a.y) + (int64_t)m * a.ldy + n) = *reinterpret_cast<const u32x2*>(o);
-            } else if (is_free(EPI)) {  // float outputs; N is a multiple of 8, so the four columns exist together
+            } else if (is_free(EPI)) {  // float outputs, or bf16 ones with a residual; N is a multiple of 8, so the four columns exist together
                 const int64_t at = (int64_t)m * a.ldy + n;
                 f32x4 v = acc[t][tb] * a.epi.scale;
                 if (a.epi.bias) v += *reinterpret_cast<const f32x4*>(a.epi.bias + n);
@@ -103,7 +103,14 @@ __device__ __forceinline__ void store_tiles(const TiledArgs& a, const f32x4 (&ac
                     if (EPI == EPI_FREE_TANH) v[i] = tanhf(v[i]);
                 }
                 if (a.epi.residual) v += *reinterpret_cast<const f32x4*>(a.epi.residual + at);
-                *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
+                if (a.out_f32) {
+                    *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
+                } else {
+                    bf16 o[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[i] = from_f32<bf16>(v[i]);
+                    *reinterpret_cast<u32x2*>(static_cast<bf16*>(a.y) + at) = *reinterpret_cast<const u32x2*>(o);
+                }
             } else {
                 float r[4];
 #pragma unroll
@@ -556,7 +563,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(TiledArgs a) {
             return;
         }
     }
-    if (a.out_f32) store_tiles<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wm, wn, l16, q4);
+    if (a.out_f32 || (is_free(EPI) && a.epi.residual)) store_tiles<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wm, wn, l16, q4);
     else store_tiles_lds<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wave, lane, lds_base);
 }
 
@@ -772,7 +779,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(TiledArgs a) {
             return;
         }
     }
-    if (a.out_f32) store_tiles<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wm, wn, l16, q4);
+    if (a.out_f32 || (is_free(EPI) && a.epi.residual)) store_tiles<EPI, TM, TN, WM, WN>(a, acc, tile_m, tile_n, wm, wn, l16, q4);
     else store_tiles_lds<EPI, TM, TN, WM, WN, GROUPED>(a, acc, tile_m, tile_n, wave, lane, lds_base);
 }
 
@@ -926,10 +933,10 @@ bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_s
 
 static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0,
                            int K1, int swiglu, int out_f32, const RopeAppend* rope, void* workspace, size_t workspace_bytes, hipStream_t s,
-                           const raven_epilogue* epi = nullptr, int* ks_left = nullptr) {
+                           const raven_epilogue* epi = nullptr, int* ks_left = nullptr, int ldw = 0) {
     if (ks_left) *ks_left = 0;
     const int f32_sums = epi && epi->out_f32;
-    const bool few = few_rows_fit(M, N, K0, K1, RAVEN_BF16, swiglu, f32_sums, w, workspace_bytes, true);
+    const bool few = !ldw && few_rows_fit(M, N, K0, K1, RAVEN_BF16, swiglu, f32_sums, w, workspace_bytes, true);
     RAVEN_REQUIRE(few || tiled_gemm_fits(M, N, K0, K1, RAVEN_BF16, swiglu, workspace_bytes, true, f32_sums), "gemm (tiled): unsupported shape M=%d N=%d K0=%d K1=%d", M, N, K0, K1);
     RAVEN_REQUIRE(!(swiglu && (residual || out_f32)), "gemm (tiled): the SwiGLU epilogue has no residual and stores bf16");
     RAVEN_REQUIRE(((uintptr_t)x0 & 15) == 0 && ((uintptr_t)x1 & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
@@ -943,10 +950,11 @@ static int tiled_gemm_impl(const void* x0, int ldx, const void* x1, const void* 
     a.M = M; a.N = N; a.K0 = K0; a.K1 = x1 ? K1 : 0; a.out_f32 = out_f32;
     a.ldy = N;
     a.up_off = N;
-    a.ldw = K0 + a.K1;
+    a.ldw = ldw ? ldw : K0 + a.K1;
     a.ldx = ldx > 0 ? ldx : K0;
     RAVEN_REQUIRE(a.ldx >= K0 && a.ldx % 8 == 0 && (a.ldx == K0 || a.K1 == 0) && (int64_t)M * a.ldx < (1ll << 31), "gemm (tiled): bad row pitch %d of x", ldx);
-    {
+    RAVEN_REQUIRE(a.ldw >= K0 + a.K1 && a.ldw % 8 == 0 && (int64_t)N * 2 * a.ldw < (1ll << 31), "gemm (tiled): bad row pitch %d of w", ldw);
+    if (!ldw) {
         std::lock_guard<std::mutex> lock(g_packed_mutex);
         const auto it = g_packed.find(w);
         if (it != g_packed.end() && it->second.K == a.ldw && it->second.rows == (swiglu ? 2 * N : N) && (int64_t)it->second.rows * it->second.ld < (1ll << 31)) {
@@ -1028,6 +1036,15 @@ int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const voi
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
                     void* workspace, size_t workspace_bytes, hipStream_t s) {
     return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, workspace, workspace_bytes, s, &epi);
+}
+
+// Columns 0 .. K - 1 of a wider matrix with rows ldw apart, for rows that tiled_gemm_fits takes: y = round(x W^T + extra), or with raw_out the float sums themselves that
+// a later call takes as `extra`.  ks_left: as in tiled_gemm (the caller then adds `extra` as well).
+int tiled_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K, void* workspace,
+                       size_t workspace_bytes, hipStream_t s, int* ks_left) {
+    raven_epilogue e{};
+    e.scale = 1.f; e.act = RAVEN_ACT_NONE; e.out_f32 = raw_out; e.residual = extra;
+    return tiled_gemm_impl(x, 0, nullptr, w_block, nullptr, y, M, N, K, 0, 0, raw_out, nullptr, workspace, workspace_bytes, s, &e, ks_left, ldw);
 }
 
 // mid_grouped (gemm_common.h) in tiles of 256 rows by the ring kernel

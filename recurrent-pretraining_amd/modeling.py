@@ -624,6 +624,13 @@ class RavenForCausalLM(MinimalGeneration, RavenPreTrainedModel, GenerationMixin)
         """The r-loop of iterate_forward plus its closing ln_f (RMM:751-762)."""
         n_core = len(self.transformer.core_block)
         x = state
+        steps = [block_idx + 1 + i for i in range(r * n_core)]
+        if r > 1 and n_core > 0 and B * S > 1 and self.config.test_time_noise <= 0 and (private or not any(cache.has_gap(s_, pos0) for s_ in steps)):
+            # every position is cached at every step and nothing happens between two recurrences: one call for all of them
+            nat, t = self._natives(), self.transformer
+            slots = [0 if private else cache.note_append(s_, S, pos0) for s_ in steps]
+            return hip.core_iterations(nat["dims"], t.adapter.weight, nat["core"], x, embeds, torch.empty_like(x), self._freqs(), cache.native(),
+                                       [slots[i:i + n_core] for i in range(0, len(slots), n_core)], B, S, pos0, self._workspace(B * S), ln_f=t.ln_f.weight)
         for it in range(r):
             x = self._run_core(x, embeds, block_idx + 1 + it * n_core, cache, private, B, S, pos0, ln_f=(it == r - 1), current_step=it)
         if r == 0:

@@ -386,6 +386,34 @@ def test_rows_formed_from_slices_have_the_norm_of_stored_rows(pkg, tuned, h, nh,
     del keep
 
 
+@pytest.mark.parametrize("M, h, nh", [(33, 4096, 64), (300, 4096, 64), (4096, 5280, 55)])
+def test_embedding_half_of_the_adapter_summed_once(pkg, tuned, M, h, nh):
+    """Two recurrences over 33 and more rows, whose adapter is split by columns: in K slices that the norm adds, or a launch of their own, and in 256 x 256 tiles with a last
+    round of smaller pieces.  The block's output matrices are zero, so that a recurrence is the adapter behind norms."""
+    hip, dt, hd, inter = pkg.hip, torch.bfloat16, h // nh, 64
+    one, zero = torch.ones(h, dtype=dt, device="cuda"), lambda *s: torch.zeros(*s, dtype=dt, device="cuda")
+    keep = [one, _gpu_randn((3 * h, h), 931, 0.02), zero(2, 1, nh, hd), zero(h, h), _gpu_randn((2 * inter, h), 932, 0.02), zero(h, inter)]
+    blocks = (hip.BlockWeights * 1)(hip.make_block_weights(one, one, one, one, *keep[1:]))
+    dims = hip.make_dims(h, nh, inter, 1e-6, dt)
+    ws = hip.block_workspace(dims, M, "cuda")
+    freqs = O.rope_table(hd, M, 50000).to(dt).float().reshape(M, hd // 2, 2).contiguous().cuda()
+    adapter, state, embeds = _gpu_randn((h, 2 * h), 933, h ** -0.5), _gpu_randn((M, h), 934), _gpu_randn((M, h), 935)
+
+    def norm(x):
+        return (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6)).to(dt).float()
+
+    want = state.float()
+    for _ in range(2):
+        z = (want @ adapter[:, :h].float().T + embeds.float() @ adapter[:, h:].float().T).to(dt).float()
+        want = norm(norm(z))
+    for fuse in (1, 0):
+        tuned(fuse_sums_norm=fuse)
+        k, v = zero(2, 1, nh, M, hd), zero(2, 1, nh, M, hd)
+        got = hip.core_iterations(dims, adapter, blocks, state, embeds, torch.empty_like(state), freqs, hip.make_cache(k, v), [[0], [1]], 1, M, 0, ws)
+        check(got, want.to(dt), dt, f"two recurrences, fuse_sums_norm={fuse}", ulps=ULPS_COMPOSED)
+    del keep
+
+
 def test_few_rows_read_a_copy_where_they_may(pkg, tuned):
     """20 rows against 1032 x 4200, whose rows are not whole lines: with a registered copy the product is the middle kernel's and reads it; with
     pad_decode_rows = 0, or without a copy, it reads the matrix."""
