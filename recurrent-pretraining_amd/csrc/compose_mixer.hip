@@ -26,8 +26,13 @@ namespace raven {
 RAVEN_WEAK int latent_attention(const raven_latent* l, const void* q, const void* z, int ldz, int z_f32, const raven_latent_cache* cache, void* y, int B,
                                 int S, int pos0, const int* pos_dev, int append, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s);
 
-RAVEN_WEAK int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, float eps, const float* logits, float* x, int M, int ld, int dtype,
-                           void* workspace, size_t workspace_bytes, hipStream_t s);
+RAVEN_WEAK int moe_forward(const raven_moe* m, const void* h, const float* factors, const float* norm, int dim, float eps, const float* logits, float* x, int M, int ld,
+                           int dtype, void* workspace, size_t workspace_bytes, hipStream_t s);
+RAVEN_WEAK bool moe_takes_factors(const raven_moe* m, const void* h, int M, int ld, int dtype);
+
+bool epilogue_in_one_launch(const void* x, const void* w, const void* y, int M, int N, int K, int out_f32, const void* workspace, size_t workspace_bytes);
+int gemm_free_normed(const void* x, const void* w, void* y, int M, int N, int K, const raven_epilogue& epi, const NormAhead* ahead, const NormBehind* behind,
+                     hipStream_t s);
 
 bool gemv1_stream_fits(int K, int dtype);
 int gemv1_stream(const float* x, const float* norm, int dim, float eps, const void* w, void* y, int N, int K, const raven_epilogue& epi, int dtype,
@@ -38,6 +43,7 @@ struct MixerScratch {
     char *h, *z, *low, *y, *ff;  // low: the decay's low-rank rows / the normed query latents
     char* q;
     float *decay, *logits;
+    float *squares, *factors;  // 2 to 32 rows of bf16: a norm shared out between two products (NormAhead)
     char *mix_ws, *ff_ws, *lin_ws;
     size_t mix_ws_bytes, ff_ws_bytes, lin_ws_bytes;
 };
@@ -74,6 +80,9 @@ static size_t carve_mixer(const raven_stream_dims* d, const raven_mixer_layer* l
     s.y = take(M * inner * es);
     s.ff = take(ff ? M * l->ff * es : 0);
     s.logits = reinterpret_cast<float*>(take(moe ? M * l->moe->logit_ld * sizeof(float) : 0));
+    const bool shared_norm = d->dtype == RAVEN_BF16 && M >= 2 && M <= 32;
+    s.squares = reinterpret_cast<float*>(take(shared_norm ? M * norm_pitch(d->ld / 16) * sizeof(float) : 0));
+    s.factors = reinterpret_cast<float*>(take(shared_norm ? M * sizeof(float) : 0));
     switch (l->mixer) {
         case RAVEN_MIXER_ATTENTION: s.mix_ws_bytes = raven_capped_attention_workspace_bytes((int)M, l->heads, l->kv_heads, l->head_dim); break;
         case RAVEN_MIXER_GENERAL_DELTA: s.mix_ws_bytes = raven_delta_rule_workspace_bytes(B, S, l->heads, l->head_dim); break;
@@ -204,12 +213,34 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
         if (int rc = normed_product(l.norm1, l.w_in, w.z, 2 * inner, RAVEN_ACT_NONE, l.in_bias, 0)) return rc;
         if (int rc = raven_rglru_forward(l.rglru, w.z, state->ring, state->state, w.y, B, S, pos0, pos_dev, dt, w.mix_ws, w.mix_ws_bytes, stream)) return rc;
     }
+    // A few rows: the norm in front of the feed-forward is shared out between the output product and the first product behind it, where both are single launches
+    const void* second = l.ff_kind == RAVEN_FF_MOE ? l.moe->router : l.ff_kind == RAVEN_FF_GELU ? l.up : nullptr;
+    const int second_n = l.ff_kind == RAVEN_FF_MOE ? l.moe->logit_ld : l.ff;
+    void* const second_y = l.ff_kind == RAVEN_FF_MOE ? static_cast<void*>(w.logits) : static_cast<void*>(w.ff);
+    if (second && !one_row && dt == RAVEN_BF16 && M <= 32 && ld <= 16 * kNormParts && epilogue_in_one_launch(w.y, l.w_out, x, M, ld, inner, 1, w.lin_ws, w.lin_ws_bytes) &&
+        epilogue_in_one_launch(w.h, second, second_y, M, second_n, ld, l.ff_kind == RAVEN_FF_MOE, w.lin_ws, w.lin_ws_bytes) &&
+        (l.ff_kind != RAVEN_FF_MOE || moe_takes_factors(l.moe, w.h, M, ld, dt))) {
+        raven_epilogue out{}, in{};
+        out.scale = in.scale = 1.f;
+        out.out_f32 = 1; out.residual = x; out.act = in.act = RAVEN_ACT_NONE;
+        const NormAhead ahead{l.norm2, reinterpret_cast<bf16*>(w.h), w.squares};
+        const NormBehind behind{w.squares, l.ff_kind == RAVEN_FF_MOE ? w.factors : nullptr, ld / 16, dims->width, dims->eps};
+        if (int rc = gemm_free_normed(w.y, l.w_out, x, M, ld, inner, out, &ahead, nullptr, s)) return rc;
+        if (l.ff_kind == RAVEN_FF_MOE) {
+            in.out_f32 = 1;
+            if (int rc = gemm_free_normed(w.h, second, second_y, M, second_n, ld, in, nullptr, &behind, s)) return rc;
+            return moe_forward(l.moe, w.h, w.factors, nullptr, 0, 0.f, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s);
+        }
+        in.act = RAVEN_ACT_GELU;
+        if (int rc = gemm_free_normed(w.h, second, second_y, M, second_n, ld, in, nullptr, &behind, s)) return rc;
+        return product(w.ff, l.down, x, ld, l.ff, RAVEN_ACT_NONE, nullptr, x, 1);
+    }
     if (int rc = product(w.y, l.w_out, x, ld, inner, RAVEN_ACT_NONE, nullptr, x, 1)) return rc;
 
     if (l.ff_kind == RAVEN_FF_MOE) {
         // (one row: the norm rides in the router's product and again in the experts' first one; else it lies in w.h)
         if (int rc = normed_product(l.norm2, l.moe->router, w.logits, l.moe->logit_ld, RAVEN_ACT_NONE, nullptr, 1)) return rc;
-        return moe_forward(l.moe, one_row ? nullptr : w.h, l.norm2, dims->width, dims->eps, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s);
+        return moe_forward(l.moe, one_row ? nullptr : w.h, nullptr, l.norm2, dims->width, dims->eps, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s);
     }
     if (!l.up) return 0;
     if (l.ff_kind == RAVEN_FF_SWIGLU) {

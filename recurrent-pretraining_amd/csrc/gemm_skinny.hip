@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "raven_common.h"
+#include "row_helpers.h"
 
 extern "C" int raven_gemv_fused(const void* x0, const void* x1, const void* norm_a, const void* norm_b, void* xa_out,
                                 const void* w, const void* residual, void* y, int32_t N, int32_t K0, int32_t K1, float eps,
@@ -34,6 +35,8 @@ bool gemv1_fits(int K, int dtype);
 int gemv1_free(const void* x0, const void* x1, const void* w, void* y, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
                hipStream_t s);
 
+constexpr int kNormNone = 0, kNormAhead = 1, kNormBehind = 2;
+
 struct GemmArgs {
     const void* w;         // [N_total, K]
     const void* x0;        // [M, k0]
@@ -49,6 +52,9 @@ struct GemmArgs {
     raven_epilogue epi;    // EPI_FREE only (residual and y already offset to the pass)
     int ldy;               // EPI_FREE only: elements between two rows of y and residual
     int rows_per_unit;     // mfma, ragged variants: weight rows (per side for SwiGLU) a workgroup owns; its last tile is partly empty
+    int early;             // mfma, EPI_FREE: a residual whose pieces and those of y start on 16 bytes, requested in front of the weights
+    NormAhead ahead;       // mfma, EPI_FREE only
+    NormBehind behind;     // mfma, free epilogues only
 };
 
 // Launch-shape knobs (raven_set_tuning); 0 = automatic.
@@ -246,7 +252,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemmArgs a) {
 // would leave a partly filled last round.
 //
 // WAVES = 8 with D register sets in flight: the variants of launch_one_round, one workgroup per CU.
-template <int MT, int NT, int EPI, int KM = 128, bool RAG = false, int WAVES = 4, int D = 1>
+// NORM: half of a norm that is shared out between two products (NormAhead, NormBehind); instantiations of their own, for with both behind run-time branches
+// every launch of a free epilogue was 0.3 to 0.5 us longer.
+template <int MT, int NT, int EPI, int KM = 128, bool RAG = false, int WAVES = 4, int D = 1, int NORM = kNormNone>
 __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
     constexpr int ROWS = 16 * (NT + MT);
     constexpr int kPitch = KM + 8;
@@ -256,6 +264,7 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
     constexpr int NG = EPI == EPI_SWIGLU ? NT / 2 : NT;  // tiles side by side along N (SwiGLU: NG gate tiles + their NG up tiles)
     __shared__ __align__(16) bf16 stage[WAVES][ROWS][kPitch];
     static_assert(sizeof(bf16) * WAVES * ROWS * kPitch >= sizeof(float) * (WAVES - 1) * NT * MT * 64 * 4, "stage doubles as the reduction buffer");
+    __shared__ float row_inv[NORM == kNormBehind ? 16 * MT : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ln = lane & 15, kq = lane >> 4;
     const int K = a.K;
@@ -300,6 +309,53 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
     };
     bf16(*my)[kPitch] = stage[wave];
     const int lr = lane / LPR, lc = (lane % LPR) * 8;  // loader role: row within a group of RPI, first element of the chunk
+
+    // What the ends of a shared norm read is requested in front of the weights, so that nothing waits for it: the sums of squares (16 lanes to a row, the
+    // rows shared out over the waves), and the residuals and weights of wave 0, which stores.
+    constexpr int RP = NORM == kNormBehind ? (16 * MT + 4 * WAVES - 1) / (4 * WAVES) : 1, SP = kNormParts / 64;
+    f32x4 squares[RP][SP];
+    const int pitch = norm_pitch(a.behind.parts);
+    if constexpr (NORM == kNormBehind) {
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+#pragma unroll
+            for (int i = 0; i < SP; ++i)
+                squares[j][i] = *reinterpret_cast<const f32x4*>(a.behind.squares + min(4 * (wave + WAVES * j) + kq, a.M - 1) * pitch + min(4 * (ln + 16 * i), pitch - 4));
+    }
+    constexpr bool EARLY = EPI == EPI_FREE && !RAG;  // (a residual requested behind the products: 2048 x 2048 at 20 rows 8.2 us, so 6.7)
+    f32x4 res[EARLY ? NT : 1][MT], norm_w[NORM == kNormAhead ? NT : 1];
+    if constexpr (EARLY) {
+        auto four_of = [&](const float* p) { return rs == 1 ? *reinterpret_cast<const f32x4*>(p) : f32x4{p[0], p[2], p[4], p[6]}; };
+        if (wave == 0 && a.early) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int n = tile_out0[t] + kq * 4 * rs;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) res[t][mt] = four_of(a.epi.residual + (int64_t)min(mt * 16 + ln, a.M - 1) * a.ldy + n);
+                if constexpr (NORM == kNormAhead) norm_w[t] = four_of(a.ahead.weight + n);
+            }
+        }
+    }
+    // the rows' factors, formed while the first weights are on their way
+    auto row_factors = [&]() __attribute__((always_inline)) {
+        if constexpr (NORM == kNormBehind) {
+            const NormBehind& b = a.behind;
+#pragma unroll
+            for (int j = 0; j < RP; ++j) {
+                float sum = 0.f;
+#pragma unroll
+                for (int i = 0; i < SP; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum += 4 * (ln + 16 * i) + e < b.parts ? squares[j][i][e] : 0.f;
+                const float inv = 1.0f / sqrtf(row16_sum(sum) / (float)b.dim + b.eps);
+                const int m = 4 * (wave + WAVES * j) + kq;
+                if (ln == 0 && m < a.M) {
+                    row_inv[m] = inv;
+                    if (b.factors && blockIdx.x == 0) b.factors[m] = inv;
+                }
+            }
+        }
+    };
 
     // X is given as up to two K segments (the adapter's concat); each is walked on its own
 #pragma unroll 1
@@ -378,6 +434,7 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
             // one register set: its loads for macro-step s+1 are in flight while step s is multiplied out of LDS
             Staged st{};
             if (mb < me) fetch(mb, st);
+            if (seg == 0) row_factors();
             for (int mac = mb; mac < me; mac += WAVES) {
                 park(st);
                 wave_sync();
@@ -385,7 +442,9 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
                 multiply();
                 wave_sync();
             }
-        } else if (mb < me) {
+        } else if (mb >= me) {
+            if (seg == 0) row_factors();
+        } else {
             // rounds of D steps, each requesting the next round's loads (none under a branch of its own, so that the waits count only the
             // set being parked); what lies past the end loads the wave's first step again and is not multiplied
             Staged st[D];
@@ -393,6 +452,7 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
             auto step_of = [&](int i) { return i < steps ? mb + i * WAVES : mb; };
 #pragma unroll
             for (int d = 0; d < D; ++d) fetch(step_of(d), st[d]);
+            if (seg == 0) row_factors();
             int done = 0;
 #pragma unroll 1
             for (; done + D < steps; done += D) {
@@ -458,6 +518,52 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
                 acc[t][mt][v] += others;
             }
 
+    if constexpr (NORM == kNormBehind) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const float inv = row_inv[min(mt * 16 + ln, a.M - 1)];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t][mt] *= inv;
+        }
+    }
+    if (EARLY && a.early) {  // (float outputs)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int m = mt * 16 + ln;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                if (!tile_ok[t]) continue;
+                const int n = tile_out0[t] + kq * 4 * rs;
+                const int64_t at = (int64_t)m * a.ldy + n;
+                f32x4 f = acc[t][mt] * a.epi.scale;
+                if (NORM == kNormNone && a.epi.bias) f += rs == 1 ? load4(a.epi.bias + n) : f32x4{a.epi.bias[n], a.epi.bias[n + 2], a.epi.bias[n + 4], a.epi.bias[n + 6]};
+                f += res[t][mt];
+                f32x4 g{};
+                if constexpr (NORM == kNormAhead) g = f * norm_w[t];
+                if (m < a.M) {
+                    float* y = static_cast<float*>(a.y) + at;
+                    if (rs == 1) {
+                        store4(y, f);
+                        if constexpr (NORM == kNormAhead) store4(a.ahead.xw + at, g);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            y[2 * v] = f[v];
+                            if constexpr (NORM == kNormAhead) a.ahead.xw[at + 2 * v] = from_f32<bf16>(g[v]);
+                        }
+                    }
+                }
+                if constexpr (NORM == kNormAhead) {
+                    float sq = f[0] * f[0] + f[1] * f[1] + f[2] * f[2] + f[3] * f[3];
+                    sq += __shfl_xor(sq, 16, 64);
+                    sq += __shfl_xor(sq, 32, 64);
+                    // tiles in the order of their first columns; with rs = 2 the even and the odd columns of 32 are a tile each
+                    if (kq == 0 && m < a.M) a.ahead.squares[m * norm_pitch(a.N / 16) + (tile_out0[t] - parity) / 16 + parity] = sq;
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = mt * 16 + ln;
@@ -694,7 +800,7 @@ static bool one_round_pays(const GemmArgs& a, int tiles) {
 // us per launch before / after: 2048 x 2048 at 8 rows 6.1 / 5.5, at 20 rows 9.3 / 7.0; 8192 x 2048 at 20 rows 15.3 / 10.9; 10304 x 2048 12.0 / 11.2 and
 // 15.4 / 12.6; 15840 x 5280 at 16 rows 32.6 / 30.1.  More loads in flight than two sets of 64 columns per wave gain nothing: a CU's own rate of loads is
 // the bound.
-template <int EPI, int MT>
+template <int EPI, int MT, int NORM>
 static bool launch_one_round(const GemmArgs& a, hipStream_t s) {
     constexpr int side = EPI == EPI_SWIGLU ? 2 : 1;
     const int rs = a.row_stride, n_tiles16 = a.N / 16;
@@ -705,25 +811,31 @@ static bool launch_one_round(const GemmArgs& a, hipStream_t s) {
     // two token tiles against four weight tiles do not fit the registers
     if (tiles > (EPI == EPI_SWIGLU ? 1 : MT == 1 ? 4 : 3) || (g_tuning.gemm_one_round == 1 && !one_round_pays<EPI == EPI_SWIGLU>(a, tiles))) return false;
     if (tiles == 1) {
-        mfma_kernel<MT, side, EPI, 128, false, 8><<<dim3(groups(1)), dim3(512), 0, s>>>(a);
+        mfma_kernel<MT, side, EPI, 128, false, 8, 1, NORM><<<dim3(groups(1)), dim3(512), 0, s>>>(a);
     } else if constexpr (EPI != EPI_SWIGLU) {
-        if (tiles == 2) mfma_kernel<MT, 2, EPI, 64, false, 8, 2><<<dim3(groups(2)), dim3(512), 0, s>>>(a);
-        else if (tiles == 3) mfma_kernel<MT, 3, EPI, 64, false, 8, 2><<<dim3(groups(3)), dim3(512), 0, s>>>(a);
-        else if constexpr (MT == 1) mfma_kernel<1, 4, EPI, 64, false, 8><<<dim3(groups(4)), dim3(512), 0, s>>>(a);
+        if (tiles == 2) mfma_kernel<MT, 2, EPI, 64, false, 8, 2, NORM><<<dim3(groups(2)), dim3(512), 0, s>>>(a);
+        else if (tiles == 3) mfma_kernel<MT, 3, EPI, 64, false, 8, 2, NORM><<<dim3(groups(3)), dim3(512), 0, s>>>(a);
+        else if constexpr (MT == 1) mfma_kernel<1, 4, EPI, 64, false, 8, 1, NORM><<<dim3(groups(4)), dim3(512), 0, s>>>(a);
     }
     return true;
 }
 
 template <int EPI>
+static int reads_residual_early(const GemmArgs& a) {
+    return EPI == EPI_FREE && a.epi.residual && a.epi.out_f32 && a.ldy % 4 == 0 && raven_host::aligned16(a.y, a.epi.residual, a.epi.bias);
+}
+
+template <int EPI, int NORM = kNormNone>
 static int dispatch_mfma(GemmArgs a, hipStream_t s) {
     const int n_tiles16 = a.N / 16;
+    a.early = reads_residual_early<EPI>(a);
     // rows alternate between line-aligned and 64 bytes off when the row pitch is an odd multiple of 64 bytes:
     // tiles of equal parity then (needs whole pairs of tiles); any multiple of 128 bytes needs nothing special
     const int pitch = a.K * 2;
     a.row_stride = (pitch % 128 == 64 && a.N % 32 == 0) ? 2 : 1;
     a.line_aligned = (pitch * a.row_stride) % 128 == 0;
     const int rs = a.row_stride;
-    if (a.M <= 16 ? launch_one_round<EPI, 1>(a, s) : launch_one_round<EPI, 2>(a, s)) return raven_host::check_launch("mfma gemm");
+    if (a.M <= 16 ? launch_one_round<EPI, 1, NORM>(a, s) : launch_one_round<EPI, 2, NORM>(a, s)) return raven_host::check_launch("mfma gemm");
     // Four tiles per workgroup (64-wide K steps) halve the X re-reads per weight byte: 5.0 -> 5.7 TB/s in steady state
     // at 32 rows.  Their workgroups are twice as long, so the gain only survives where the grid is balanced: at most
     // one workgroup per CU (Wqkv: 248), or so many that the last round does not matter.  Tuning key gemm_four_tiles:
@@ -754,19 +866,19 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
         else
             mfma_kernel<2, 2, EPI><<<dim3(n_tiles16), dim3(256), 0, s>>>(a);
     } else if (four) {
-        if (a.M <= 16) mfma_kernel<1, 4, EPI, 64><<<dim3(groups4), dim3(256), 0, s>>>(a);
-        else           mfma_kernel<2, 4, EPI, 64><<<dim3(groups4), dim3(256), 0, s>>>(a);
+        if (a.M <= 16) mfma_kernel<1, 4, EPI, 64, false, 4, 1, NORM><<<dim3(groups4), dim3(256), 0, s>>>(a);
+        else           mfma_kernel<2, 4, EPI, 64, false, 4, 1, NORM><<<dim3(groups4), dim3(256), 0, s>>>(a);
     } else {
         // two tiles per workgroup (X is then re-read from L2 once per two tiles) while that still leaves every
         // CU more than one workgroup; L2 -> L1 traffic, not HBM, is what limits this kernel
         const bool two = n_tiles16 / 2 >= n_cus() + n_cus() / 2;
         const int units = two ? groups2 : n_tiles16;
         if (a.M <= 16) {
-            if (two) mfma_kernel<1, 2, EPI><<<dim3(units), dim3(256), 0, s>>>(a);
-            else     mfma_kernel<1, 1, EPI><<<dim3(units), dim3(256), 0, s>>>(a);
+            if (two) mfma_kernel<1, 2, EPI, 128, false, 4, 1, NORM><<<dim3(units), dim3(256), 0, s>>>(a);
+            else     mfma_kernel<1, 1, EPI, 128, false, 4, 1, NORM><<<dim3(units), dim3(256), 0, s>>>(a);
         } else {
-            if (two) mfma_kernel<2, 2, EPI><<<dim3(units), dim3(256), 0, s>>>(a);
-            else     mfma_kernel<2, 1, EPI><<<dim3(units), dim3(256), 0, s>>>(a);
+            if (two) mfma_kernel<2, 2, EPI, 128, false, 4, 1, NORM><<<dim3(units), dim3(256), 0, s>>>(a);
+            else     mfma_kernel<2, 1, EPI, 128, false, 4, 1, NORM><<<dim3(units), dim3(256), 0, s>>>(a);
         }
     }
     return raven_host::check_launch("mfma gemm");
@@ -867,6 +979,25 @@ int gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int
     }
 }
 
+bool gemm_free_normed_fits(int M, int N, int K) { return M >= g_tuning.gemm_mfma_min_rows && M <= 32 && N % 16 == 0 && K % 32 == 0; }
+// One of two products of 2 to 32 rows with an RMSNorm between them, both of which gemm_free takes in one launch (epilogue_in_one_launch): y = x W^T + residual in float and
+// what the norm needs of it, or a product of such rows
+int gemm_free_normed(const void* x, const void* w, void* y, int M, int N, int K, const raven_epilogue& epi, const NormAhead* ahead, const NormBehind* behind,
+                     hipStream_t s) {
+    RAVEN_REQUIRE(gemm_free_normed_fits(M, N, K) && (ahead != nullptr) != (behind != nullptr) && epi.act != RAVEN_ACT_TANH &&
+                      !(ahead && (epi.act != RAVEN_ACT_NONE || !epi.out_f32 || !epi.residual || epi.bias || !raven_host::aligned16(y, epi.residual, ahead->weight, ahead->xw))) && !(behind && behind->parts > kNormParts),
+                  "gemm (norm between): unsupported shape M=%d N=%d K=%d", M, N, K);
+    GemmArgs a{};
+    a.w = w; a.x0 = x; a.y = y;
+    a.M = M; a.N = N; a.K = K; a.k0 = K; a.out_f32 = epi.out_f32; a.epi = epi; a.ldy = N;
+    if (ahead) {
+        a.ahead = *ahead;
+        return dispatch_mfma<EPI_FREE, kNormAhead>(a, s);
+    }
+    a.behind = *behind;
+    return epi.act == RAVEN_ACT_GELU ? dispatch_mfma<EPI_FREE_GELU, kNormBehind>(a, s) : dispatch_mfma<EPI_FREE, kNormBehind>(a, s);
+}
+
 // Many rows against a matrix of at most 128 rows, where 128 x 128 tiles would leave most of the chip idle: 32 x 32 pieces of the output,
 // K split over a workgroup's waves.  ldy: row pitch of y and the residual.
 bool gemm_narrow_fits(int M, int N, int K, int dtype) {
@@ -874,6 +1005,7 @@ bool gemm_narrow_fits(int M, int N, int K, int dtype) {
 }
 template <int EPI>
 static int launch_narrow(GemmArgs a, hipStream_t s) {
+    a.early = reads_residual_early<EPI>(a);
     const int pitch = a.K * 2, n_tiles16 = a.N / 16;
     a.row_stride = (pitch % 128 == 64 && a.N % 32 == 0) ? 2 : 1;
     a.line_aligned = (pitch * a.row_stride) % 128 == 0;

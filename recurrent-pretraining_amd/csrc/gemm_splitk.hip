@@ -39,6 +39,7 @@ int tiled_column_block(const void* x, const void* w_block, int ldw, const float*
 int gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
               hipStream_t s);
 
+bool gemm_free_normed_fits(int M, int N, int K);
 bool gemm_narrow_fits(int M, int N, int K, int dtype);
 int gemm_narrow_free(const void* x, const void* w, void* y, int ldy, int M, int N, int K, const raven_epilogue& epi, hipStream_t s);
 
@@ -405,6 +406,14 @@ int linear_leave_sums(const void* x0, int ldx, const void* x1, const void* w, in
     a.y = y;
     a.M = M; a.N = N; a.K = K0 + K1; a.k0 = K0; a.k1 = K1; a.ldw = ldw; a.extra = extra;
     return launch_ns<EPI_PLAIN>(a, workspace, workspace_bytes, s, ks_left);
+}
+
+// Whether a product with a free epilogue is one launch of the matrix-core kernel of gemm_skinny.hip: the choice of raven_linear_epilogue, so that a norm may be
+// shared out between such products (gemm_free_normed)
+bool epilogue_in_one_launch(const void* x, const void* w, const void* y, int M, int N, int K, int out_f32, const void* workspace, size_t workspace_bytes) {
+    const bool aligned = raven_host::aligned16(x, w, y);
+    return gemm_free_normed_fits(M, N, K) && M < g_tiled_min_rows && M > g_linear_min_rows && g_linear_ks == 0 &&
+           !few_rows_fit(M, N, K, 0, RAVEN_BF16, 0, out_f32, w, usable(workspace, workspace_bytes), aligned) && !splits_k(N / 16, M, K, false);
 }
 
 }  // namespace raven

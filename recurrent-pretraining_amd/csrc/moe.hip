@@ -29,6 +29,7 @@ struct MoeArgs {
     const void *h, *up, *down, *shared_up, *shared_down;
     const float* logits;
     float* x;
+    const float* factors;   // few rows: factors of the rows of h that are still to be applied (NormBehind), or null
     const float* norm;      // h null (one row): the norm of x that gives it, with its true width and eps
     int dim;
     float eps;
@@ -382,12 +383,12 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
         const int slot = atomicAdd(&start[pick[i]], 1);
         a.slot_of[i] = slot;
         a.slot_row[slot] = i / a.top;
-        a.slot_scale[slot] = scale[i];
+        a.slot_scale[slot] = a.factors ? scale[i] * a.factors[i / a.top] : scale[i];
     }
     if (a.fold)
         for (int m = tid; m < a.M; m += 1024) {
             a.slot_row[pairs + m] = m;
-            a.slot_scale[pairs + m] = 1.f;
+            a.slot_scale[pairs + m] = a.factors ? a.factors[m] : 1.f;
         }
 }
 
@@ -714,13 +715,18 @@ extern "C" size_t raven_moe_workspace_bytes(const raven_moe* m, int32_t M, int32
 }
 
 namespace raven {
-// h null (one row): moe_up_kernel norms the row of x itself
-int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, float eps, const float* logits, float* x, int M, int ld, int dtype,
+// Whether moe_forward applies rows' factors of its own for so many rows
+bool moe_takes_factors(const raven_moe* m, const void* h, int M, int ld, int dtype) {
+    return moe_path(m, h, M, ld, dtype) == kMoeFew && (!m->shared_up || m->shared_ff == m->ff);
+}
+// h null (one row): moe_up_kernel norms the row of x itself.  factors: the rows of the experts' inputs are these times h (moe_takes_factors)
+int moe_forward(const raven_moe* m, const void* h, const float* factors, const float* norm, int dim, float eps, const float* logits, float* x, int M, int ld, int dtype,
                 void* workspace, size_t workspace_bytes, hipStream_t s) {
     if (const int rc = check_moe("moe", m, M, ld, dtype)) return rc;
     if (M == 0) return 0;
     RAVEN_REQUIRE(m->up && m->down && (h || (norm && M == 1)) && logits && x, "moe: null pointer");
     const MoePath path = moe_path(m, h, M, ld, dtype);
+    RAVEN_REQUIRE(!factors || path == kMoeFew, "moe: factors of %d rows", M);
     RAVEN_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0 && carve_moe(m, M, ld, dtype, path, nullptr, nullptr) <= workspace_bytes,
                   "moe: workspace of %zu bytes is too small or unaligned", workspace_bytes);
     MoeChunk c;
@@ -738,7 +744,7 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
     const int rows = pairs + (fold ? M : 0);
     a.pick_scale = c.pick_scale; a.slot_of = c.slot_of; a.slot_row = c.slot_row; a.slot_scale = c.slot_scale;
     a.group_of = c.group_of; a.group_row = c.group_row; a.group_end = c.group_end; a.used = c.used; a.tile_rows = c.tile_rows; a.block_count = c.block_count;
-    a.y = c.y; a.ys = c.ys; a.fold = fold;
+    a.y = c.y; a.ys = c.ys; a.fold = fold; a.factors = factors;
     // one workgroup picks for 16 rows at a time: from 33 rows on two launches of several are sooner done (64 rows, 2 of 12 experts of 136 at
     // width 256, the whole mixture 27.5 / 25.3 us; 4 of 32 of 96 43 / 39)
     if (few || (M <= kPickRows && pairs <= kRoutePairs)) {
@@ -776,5 +782,5 @@ int moe_forward(const raven_moe* m, const void* h, const float* norm, int dim, f
 extern "C" int raven_moe_forward(const raven_moe* m, const void* h, const float* logits, float* x, int32_t M, int32_t ld, int32_t dtype,
                                  void* workspace, size_t workspace_bytes, void* stream) {
     RAVEN_REQUIRE(h || M == 0, "moe: null pointer");
-    return raven::moe_forward(m, h, nullptr, 0, 0.f, logits, x, M, ld, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    return raven::moe_forward(m, h, nullptr, nullptr, 0, 0.f, logits, x, M, ld, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }

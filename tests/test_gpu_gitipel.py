@@ -463,6 +463,25 @@ def test_batch_of_equal_lengths_against_each_alone(pkg):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-5
 
 
+@pytest.mark.parametrize("M", [2, 16, 17, 32])
+@pytest.mark.parametrize("width", [512, 540, 2304])
+def test_norm_between_two_products_of_a_few_rows(pkg, width, M):
+    """Batches whose output product and up product share the norm between them: rows of whole lines, rows that alternate between whole and half lines behind a width that
+    is padded (34 sums of squares a row), and wide ones; against the oracle, each row by itself."""
+    cfg = G.config(width, 96, [G.attn(4, 2, 64, 2 * pad8(width)), G.attn(2, 2, 96, pad8(width))], taps=3)
+    w = O.random_weights(cfg, 8, 3)
+    model = pkg.GitipelForCausalLM(pkg.GitipelConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    ids = torch.stack([G.tokens(cfg, 3, seed=s) for s in range(M)])
+    cache = model.new_cache()
+    got = [model.forward(ids[:, :1], past_key_values=cache).logits]
+    runner = model.decode_runner(cache, M)
+    got += [runner.step(ids[:, t].cuda())[0].clone()[:, None] for t in (1, 2)]
+    got = torch.cat(got, 1)
+    for b in range(M):
+        assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
+
+
 def test_interleaved_requests_of_unequal_length(pkg):
     """Requests that live at the same time, end, and hand their caches on."""
     from recurrent_pretraining_amd.trace import TraceReplay

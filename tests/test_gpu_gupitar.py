@@ -631,6 +631,26 @@ def test_batch_of_equal_lengths_against_each_alone(pkg, name):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 5e-5
 
 
+@pytest.mark.parametrize("shared", [264, None])
+@pytest.mark.parametrize("M", [2, 4, 8])
+@pytest.mark.parametrize("width", [512, 540])
+def test_norm_between_the_output_product_and_a_mixture(pkg, width, M, shared):
+    """Batches whose output product and router share the norm between them and whose experts take the rows' factors (every expert is picked, so that no close call
+    decides): against the oracle, each row by itself."""
+    cfg = G.config(width, 96, [G.rglru(width, 4, 3, G.moe(16, 16, 264, shared))])
+    w = O.random_weights(cfg, 3)
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    ids = torch.stack([G.tokens(cfg, 3, seed=s) for s in range(M)])
+    cache = model.new_cache()
+    got = [model.forward(ids[:, :1], past_key_values=cache).logits]
+    runner = model.decode_runner(cache, M)
+    got += [runner.step(ids[:, t].cuda())[0].clone()[:, None] for t in (1, 2)]
+    got = torch.cat(got, 1)
+    for b in range(M):
+        assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
+
+
 def test_interleaved_requests_of_unequal_length(pkg):
     """Requests that live at the same time, end, and hand their caches on."""
     from recurrent_pretraining_amd.trace import TraceReplay
