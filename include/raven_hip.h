@@ -597,6 +597,11 @@ size_t raven_mixer_layer_workspace_bytes(const raven_stream_dims* dims, const ra
 int    raven_mixer_layer_forward(const raven_stream_dims* dims, const raven_mixer_layer* layer, const raven_mixer_state* state, float* x,
                                  int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace, size_t workspace_bytes,
                                  void* stream);
+/* n layers one after the other on the same rows, as n calls of raven_mixer_layer_forward with a workspace for the largest of them; between two of
+ * them the last launch of the first and the first launch of the second may be one. */
+int    raven_mixer_layers_forward(const raven_stream_dims* dims, const raven_mixer_layer* const* layers, const raven_mixer_state* const* states,
+                                  int32_t n, float* x, int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace,
+                                  size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1,7 +1,8 @@
 // One pre-norm layer of a decoder with an fp32 residual stream and a choice of mixers and feed-forwards, as a sequence of this
 // library's kernels on one stream: norm (+ convolution) -> fused input projection -> mixer -> output projection added to the
 // stream -> norm -> feed-forward added to the stream.  Residual adds and activations ride in the products' epilogues, norms of a
-// single row in their prologues.
+// single row in their prologues; of a few rows the second norm is shared out between the products around it.  Between two layers of one call the slices of the
+// last product are added by the norm of the next layer, and a mixture's sums are normed for it.
 //
 // The mixers' entry points are referenced weakly: a build of one model family's kernels links without the others', and a layer
 // that needs a missing one is refused.
@@ -27,9 +28,14 @@ RAVEN_WEAK int latent_attention(const raven_latent* l, const void* q, const void
                                 int S, int pos0, const int* pos_dev, int append, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s);
 
 RAVEN_WEAK int moe_forward(const raven_moe* m, const void* h, const float* factors, const float* norm, int dim, float eps, const float* logits, float* x, int M, int ld,
-                           int dtype, void* workspace, size_t workspace_bytes, hipStream_t s);
+                           int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, const float* next_norm, void* next_h);
+RAVEN_WEAK bool moe_norms_behind(const raven_moe* m, const void* h, int M, int ld, int dtype);
 RAVEN_WEAK bool moe_takes_factors(const raven_moe* m, const void* h, int M, int ld, int dtype);
 
+int add_product_leave_sums(const void* x, const void* w, float* y, int M, int N, int K, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
+bool norm_conv_adds_slices(const float* conv, int taps, int ld, int dtype);
+int norm_conv_step_over_slices(float* x, const float* slices, int ks, const float* weight, const float* conv, float* ring, void* y, int B, int dim, int ld, int taps,
+                               float eps, int pos0, const int* pos_dev, int dtype, hipStream_t s);
 bool epilogue_in_one_launch(const void* x, const void* w, const void* y, int M, int N, int K, int out_f32, const void* workspace, size_t workspace_bytes);
 int gemm_free_normed(const void* x, const void* w, void* y, int M, int N, int K, const raven_epilogue& epi, const NormAhead* ahead, const NormBehind* behind,
                      hipStream_t s);
@@ -143,18 +149,22 @@ extern "C" size_t raven_mixer_layer_workspace_bytes(const raven_stream_dims* dim
     return raven::carve_mixer(dims, layer, B, S, pos0, nullptr, nullptr);
 }
 
-extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const raven_mixer_layer* layer, const raven_mixer_state* state, float* x,
-                                         int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace,
-                                         size_t workspace_bytes, void* stream) {
-    using namespace raven;
-    if (const int rc = check_mixer_layer("mixer_layer", dims, layer)) return rc;
-    RAVEN_REQUIRE(B >= 0 && S >= 0 && (int64_t)B * S < (1 << 30), "mixer_layer: bad B=%d S=%d", B, S);
-    if (B == 0 || S == 0) return 0;
-    RAVEN_REQUIRE(state && x && workspace && ((uintptr_t)workspace & 255) == 0, "mixer_layer: null pointer or unaligned workspace");
-    RAVEN_REQUIRE(carve_mixer(dims, layer, B, S, pos0, nullptr, nullptr) <= workspace_bytes, "mixer_layer: workspace of %zu bytes is too small",
-                  workspace_bytes);
+namespace raven {
+
+// What a layer leaves for the next one of the same call to do with its first launch
+struct LeftOver {
+    int ks = 0;                     // slices of the last product, to be added to the stream
+    const float* slices = nullptr;
+    bool normed = false;            // the next layer's first norm lies in its h already
+};
+
+// One layer; next: the layer behind it, or null.  left: what the layer before left, and what this one leaves
+static int run_mixer_layer(const raven_stream_dims* dims, const raven_mixer_layer* layer, const raven_mixer_state* state, const raven_mixer_layer* next, LeftOver* left,
+                           float* x, int B, int S, int pos0, const int32_t* pos_dev, void* workspace, void* stream) {
     MixerScratch w;
     carve_mixer(dims, layer, B, S, pos0, static_cast<char*>(workspace), &w);
+    const LeftOver before = *left;
+    *left = LeftOver{};
     const raven_mixer_layer& l = *layer;
     const int M = B * S, dt = dims->dtype, ld = dims->ld, inner = l.heads * l.head_dim;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -166,7 +176,8 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
     };
     const bool one_row = M == 1 && gemv1_stream_fits(ld, dt);
     // a product behind an RMSNorm of the stream: one row takes the norm as its prologue, more go through w.h
-    auto normed_product = [&](const float* norm, const void* wt, void* y, int N, int act, const float* bias, int out_f32) {
+    auto normed_product = [&](const float* norm, const void* wt, void* y, int N, int act, const float* bias, int out_f32, bool normed = false) {
+        if (normed) return product(w.h, wt, y, N, ld, act, bias, nullptr, out_f32);
         if (one_row) {
             raven_epilogue e{};
             e.bias = bias; e.scale = 1.f; e.act = act; e.out_f32 = out_f32;
@@ -176,12 +187,28 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
         return product(w.h, wt, y, N, ld, act, bias, nullptr, out_f32);
     };
 
+    auto first_norm = [&]() {
+        if (before.ks) return norm_conv_step_over_slices(x, before.slices, before.ks, l.norm1, l.conv, state->ring, w.h, B, dims->width, ld, l.taps, dims->eps, pos0, pos_dev, dt, s);
+        return raven_norm_conv(x, l.norm1, l.conv, state->ring, w.h, B, S, dims->width, ld, l.taps, dims->eps, pos0, pos_dev, dt, stream);
+    };
+    const bool next_convolves = next && (next->mixer == RAVEN_MIXER_ATTENTION || next->mixer == RAVEN_MIXER_GENERAL_DELTA);
+    // the feed-forward's last product: one token per sequence may leave its slices to the norm of the next layer
+    auto last_product = [&]() {
+        if (!(next_convolves && S == 1 && norm_conv_adds_slices(next->conv, next->taps, ld, dt))) return product(w.ff, l.down, x, ld, l.ff, RAVEN_ACT_NONE, nullptr, x, 1);
+        left->slices = reinterpret_cast<const float*>(w.lin_ws);
+        return add_product_leave_sums(w.ff, l.down, x, M, ld, l.ff, dt, w.lin_ws, w.lin_ws_bytes, s, &left->ks);
+    };
+    // a mixture may end with the norm that the next layer begins with
+    const bool norm_behind = l.ff_kind == RAVEN_FF_MOE && next && !next_convolves && !one_row && moe_norms_behind(l.moe, w.h, M, ld, dt);
+    left->normed = norm_behind;
+    const float* next_norm = norm_behind ? next->norm1 : nullptr;
+
     if (l.mixer == RAVEN_MIXER_ATTENTION) {
-        if (int rc = raven_norm_conv(x, l.norm1, l.conv, state->ring, w.h, B, S, dims->width, ld, l.taps, dims->eps, pos0, pos_dev, dt, stream)) return rc;
+        if (int rc = first_norm()) return rc;
         if (int rc = product(w.h, l.w_in, w.z, (l.heads + l.kv_heads) * l.head_dim, ld, RAVEN_ACT_NONE, nullptr, nullptr, 0)) return rc;
         if (int rc = raven_capped_attention(w.z, w.y, &state->keys, &l.score, B, S, pos0, pos_dev, l.heads, dt, w.mix_ws, w.mix_ws_bytes, stream)) return rc;
     } else if (l.mixer == RAVEN_MIXER_GENERAL_DELTA) {
-        if (int rc = raven_norm_conv(x, l.norm1, l.conv, state->ring, w.h, B, S, dims->width, ld, l.taps, dims->eps, pos0, pos_dev, dt, stream)) return rc;
+        if (int rc = first_norm()) return rc;
         // a few tokens: the low-rank rows ride in the fused projection and the recurrence's kernel forms the decay logits;
         // more: two small products of their own
         const bool few = S <= 8 && l.rank <= 256;
@@ -198,7 +225,7 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
     } else if (l.mixer == RAVEN_MIXER_LATENT) {
         const raven_latent& a = *l.latent;
         const int ldz = input_columns(layer), q_cols = a.heads * (a.nope + a.rot), z_f32 = M == 1 || dt == RAVEN_F32;
-        if (int rc = normed_product(l.norm1, l.w_in, w.z, ldz, RAVEN_ACT_NONE, nullptr, z_f32)) return rc;
+        if (int rc = normed_product(l.norm1, l.w_in, w.z, ldz, RAVEN_ACT_NONE, nullptr, z_f32, before.normed)) return rc;
         const bool fold = M == 1 && gemv1_stream_fits(a.q_rank, dt);  // the query latent's norm rides in W_uq, the cache entry in the attention
         if (fold) {
             raven_epilogue e{};
@@ -210,7 +237,7 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
         }
         if (int rc = latent_attention(&a, w.q, w.z, ldz, z_f32, &state->latent, w.y, B, S, pos0, pos_dev, fold, dt, w.mix_ws, w.mix_ws_bytes, s)) return rc;
     } else {
-        if (int rc = normed_product(l.norm1, l.w_in, w.z, 2 * inner, RAVEN_ACT_NONE, l.in_bias, 0)) return rc;
+        if (int rc = normed_product(l.norm1, l.w_in, w.z, 2 * inner, RAVEN_ACT_NONE, l.in_bias, 0, before.normed)) return rc;
         if (int rc = raven_rglru_forward(l.rglru, w.z, state->ring, state->state, w.y, B, S, pos0, pos_dev, dt, w.mix_ws, w.mix_ws_bytes, stream)) return rc;
     }
     // A few rows: the norm in front of the feed-forward is shared out between the output product and the first product behind it, where both are single launches
@@ -229,18 +256,18 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
         if (l.ff_kind == RAVEN_FF_MOE) {
             in.out_f32 = 1;
             if (int rc = gemm_free_normed(w.h, second, second_y, M, second_n, ld, in, nullptr, &behind, s)) return rc;
-            return moe_forward(l.moe, w.h, w.factors, nullptr, 0, 0.f, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s);
+            return moe_forward(l.moe, w.h, w.factors, nullptr, dims->width, dims->eps, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s, next_norm, w.h);
         }
         in.act = RAVEN_ACT_GELU;
         if (int rc = gemm_free_normed(w.h, second, second_y, M, second_n, ld, in, nullptr, &behind, s)) return rc;
-        return product(w.ff, l.down, x, ld, l.ff, RAVEN_ACT_NONE, nullptr, x, 1);
+        return last_product();
     }
     if (int rc = product(w.y, l.w_out, x, ld, inner, RAVEN_ACT_NONE, nullptr, x, 1)) return rc;
 
     if (l.ff_kind == RAVEN_FF_MOE) {
         // (one row: the norm rides in the router's product and again in the experts' first one; else it lies in w.h)
         if (int rc = normed_product(l.norm2, l.moe->router, w.logits, l.moe->logit_ld, RAVEN_ACT_NONE, nullptr, 1)) return rc;
-        return moe_forward(l.moe, one_row ? nullptr : w.h, nullptr, l.norm2, dims->width, dims->eps, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s);
+        return moe_forward(l.moe, one_row ? nullptr : w.h, nullptr, l.norm2, dims->width, dims->eps, w.logits, x, M, ld, dt, w.ff_ws, w.ff_ws_bytes, s, next_norm, w.h);
     }
     if (!l.up) return 0;
     if (l.ff_kind == RAVEN_FF_SWIGLU) {
@@ -253,5 +280,37 @@ extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const ra
     } else {
         if (int rc = normed_product(l.norm2, l.up, w.ff, l.ff, RAVEN_ACT_GELU, nullptr, 0)) return rc;
     }
-    return product(w.ff, l.down, x, ld, l.ff, RAVEN_ACT_NONE, nullptr, x, 1);
+    return last_product();
+}
+
+static int run_mixer_layers(const char* who, const raven_stream_dims* dims, const raven_mixer_layer* const* layers, const raven_mixer_state* const* states, int n,
+                            float* x, int B, int S, int pos0, const int32_t* pos_dev, void* workspace, size_t workspace_bytes, void* stream) {
+    RAVEN_REQUIRE(n >= 0 && (n == 0 || (layers && states)), "%s: null pointer", who);
+    for (int i = 0; i < n; ++i)
+        if (const int rc = check_mixer_layer(who, dims, layers[i])) return rc;
+    RAVEN_REQUIRE(B >= 0 && S >= 0 && (int64_t)B * S < (1 << 30), "%s: bad B=%d S=%d", who, B, S);
+    if (B == 0 || S == 0 || n == 0) return 0;
+    RAVEN_REQUIRE(x && workspace && ((uintptr_t)workspace & 255) == 0, "%s: null pointer or unaligned workspace", who);
+    for (int i = 0; i < n; ++i) {
+        RAVEN_REQUIRE(states[i], "%s: null pointer", who);
+        RAVEN_REQUIRE(carve_mixer(dims, layers[i], B, S, pos0, nullptr, nullptr) <= workspace_bytes, "%s: workspace of %zu bytes is too small", who, workspace_bytes);
+    }
+    LeftOver left;
+    for (int i = 0; i < n; ++i)
+        if (const int rc = run_mixer_layer(dims, layers[i], states[i], i + 1 < n ? layers[i + 1] : nullptr, &left, x, B, S, pos0, pos_dev, workspace, stream)) return rc;
+    return 0;
+}
+
+}  // namespace raven
+
+extern "C" int raven_mixer_layer_forward(const raven_stream_dims* dims, const raven_mixer_layer* layer, const raven_mixer_state* state, float* x,
+                                         int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+    return raven::run_mixer_layers("mixer_layer", dims, &layer, &state, 1, x, B, S, pos0, pos_dev, workspace, workspace_bytes, stream);
+}
+
+extern "C" int raven_mixer_layers_forward(const raven_stream_dims* dims, const raven_mixer_layer* const* layers, const raven_mixer_state* const* states, int32_t n,
+                                          float* x, int32_t B, int32_t S, int32_t pos0, const int32_t* pos_dev, void* workspace, size_t workspace_bytes,
+                                          void* stream) {
+    return raven::run_mixer_layers("mixer_layers", dims, layers, states, n, x, B, S, pos0, pos_dev, workspace, workspace_bytes, stream);
 }

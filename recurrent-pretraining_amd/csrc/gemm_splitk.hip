@@ -33,7 +33,7 @@ bool few_rows_fit(int M, int N, int K0, int K1, int dtype, int swiglu, int f32_s
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
                int out_f32, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
-                    void* workspace, size_t workspace_bytes, hipStream_t s);
+                    void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 int tiled_column_block(const void* x, const void* w_block, int ldw, const float* extra, void* y, int raw_out, int M, int N, int K, void* workspace,
                        size_t workspace_bytes, hipStream_t s, int* ks_left);
 int gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi, int dtype,
@@ -416,6 +416,20 @@ bool epilogue_in_one_launch(const void* x, const void* w, const void* y, int M, 
            !few_rows_fit(M, N, K, 0, RAVEN_BF16, 0, out_f32, w, usable(workspace, workspace_bytes), aligned) && !splits_k(N / 16, M, K, false);
 }
 
+// y += x W^T in float, or, where raven_linear_epilogue would cut K into slices of gemm_mid.hip, the slices alone: *ks_left of them in the workspace ([slices, M, N]), to
+// be added to y in their order by the caller
+int add_product_leave_sums(const void* x, const void* w, float* y, int M, int N, int K, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
+    *ks_left = 0;
+    raven_epilogue e{};
+    e.scale = 1.f; e.act = RAVEN_ACT_NONE; e.out_f32 = 1; e.residual = y;
+    const size_t room = usable(workspace, workspace_bytes);
+    const bool aligned = raven_host::aligned16(x, w, y);
+    if (g_fuse_sums_norm && !gemm_narrow_fits(M, N, K, dtype) &&
+        ((M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K, 0, dtype, 0, room, aligned, 1)) || (g_linear_ks == 0 && few_rows_fit(M, N, K, 0, dtype, 0, 1, w, room, aligned))))
+        return tiled_gemm_free(x, nullptr, w, y, M, N, K, 0, e, workspace, room, s, ks_left);
+    return raven_linear_epilogue(x, nullptr, w, y, M, N, K, 0, &e, dtype, workspace, workspace_bytes, s);
+}
+
 }  // namespace raven
 
 extern "C" size_t raven_linear_workspace_bytes(int32_t M, int32_t n_out_max) {
@@ -500,7 +514,7 @@ extern "C" int raven_linear_epilogue(const void* x0, const void* x1, const void*
     const bool aligned = raven_host::aligned16(x0, x1, w, y);
     if (const size_t room = usable(workspace, workspace_bytes); (M >= g_tiled_min_rows && tiled_gemm_fits(M, N, K0, K1, dtype, 0, room, aligned, epi->out_f32)) ||
                                                                (g_linear_ks == 0 && few_rows_fit(M, N, K0, K1, dtype, 0, epi->out_f32, w, room, aligned)))
-        return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, workspace, room, s);
+        return tiled_gemm_free(x0, x1, w, y, M, N, K0, K1, *epi, workspace, room, s, nullptr);
     // the same choice between the kernels with and without a K split as raven_linear
     const bool split = dtype == RAVEN_BF16 && M > g_linear_min_rows && N % 16 == 0 && K0 % 32 == 0 && K1 % 32 == 0 && workspace != nullptr &&
                        ((uintptr_t)workspace & 255) == 0 && K0 / 128 + K1 / 128 >= 1 &&

@@ -1032,10 +1032,10 @@ int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const voi
     return tiled_gemm_impl(x0, ldx, x1, w, residual, y, M, N, K0, K1, swiglu, out_f32, nullptr, workspace, workspace_bytes, s, nullptr, ks_left);
 }
 
-// The product with the free epilogue: y = act(scale * z + bias) + residual, float or bf16
+// The product with the free epilogue: y = act(scale * z + bias) + residual, float or bf16.  ks_left: as in tiled_gemm (the epilogue is then the caller's)
 int tiled_gemm_free(const void* x0, const void* x1, const void* w, void* y, int M, int N, int K0, int K1, const raven_epilogue& epi,
-                    void* workspace, size_t workspace_bytes, hipStream_t s) {
-    return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, workspace, workspace_bytes, s, &epi);
+                    void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left) {
+    return tiled_gemm_impl(x0, 0, x1, w, nullptr, y, M, N, K0, K1, 0, epi.out_f32, nullptr, workspace, workspace_bytes, s, &epi, ks_left);
 }
 
 // Columns 0 .. K - 1 of a wider matrix with rows ldw apart, for rows that tiled_gemm_fits takes: y = round(x W^T + extra), or with raw_out the float sums themselves that

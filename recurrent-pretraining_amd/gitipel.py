@@ -108,10 +108,12 @@ class GitipelForCausalLM(StreamDecoderForCausalLM):
     def layer_runs(self) -> list:
         return self.config.runs()
 
-    def enter_run(self, layer: int, turn: Optional[int], buf: dict) -> None:
-        if turn is not None and layer == self.config.loop["start"]:  # a pass begins: x <- W [x; embedding] + the pass's vector
-            hip.round_rows(buf["x"], buf["xr"])
-            hip.linear_epilogue(buf["xr"], self.loop_in, x1=buf["x0"], bias=self.loop_step[turn], out=buf["x"], workspace=buf["ws"])
+    def enters_run(self, layer: int, turn: Optional[int]) -> bool:
+        return turn is not None and layer == self.config.loop["start"]
+
+    def enter_run(self, layer: int, turn: Optional[int], buf: dict) -> None:  # a pass begins: x <- W [x; embedding] + the pass's vector
+        hip.round_rows(buf["x"], buf["xr"])
+        hip.linear_epilogue(buf["xr"], self.loop_in, x1=buf["x0"], bias=self.loop_step[turn], out=buf["x"], workspace=buf["ws"])
 
     def initial_mean(self, name: str) -> float:
         return 1.0 if name.rsplit(".", 1)[-1] in ("norm", "norm1", "norm2", "r1", "r2") else 0.0

@@ -191,6 +191,8 @@ SIGNATURES = {
     "raven_mixer_layer_workspace_bytes": (_SZ, [C.POINTER(StreamDims), C.POINTER(MixerLayer), _I32, _I32, _I32]),
     "raven_mixer_layer_forward": (C.c_int, [C.POINTER(StreamDims), C.POINTER(MixerLayer), C.POINTER(MixerState), _VP, _I32, _I32, _I32, _VP,
                                             _VP, _SZ, _VP]),
+    "raven_mixer_layers_forward": (C.c_int, [C.POINTER(StreamDims), C.POINTER(C.POINTER(MixerLayer)), C.POINTER(C.POINTER(MixerState)), _I32, _VP, _I32, _I32,
+                                             _I32, _VP, _VP, _SZ, _VP]),
 }
 
 _lib: Optional[C.CDLL] = None
@@ -877,3 +879,12 @@ def mixer_layer(dims: StreamDims, layer: MixerLayer, state: MixerState, x, B, S,
                                           _ptr(pos_dev, "pos_dev", torch.int32), _ptr(workspace, "workspace", torch.uint8),
                                           workspace.numel(), _stream())
     _check(rc, "raven_mixer_layer_forward")
+
+
+def mixer_layers(dims: StreamDims, layers, states, x, B, S, pos0, workspace, pos_dev=None):
+    """Layers (MixerLayer structures) one after the other on the same rows, with a state each: one native call."""
+    n = len(layers)
+    rc = load().raven_mixer_layers_forward(C.byref(dims), (C.POINTER(MixerLayer) * n)(*[C.pointer(v) for v in layers]),
+                                           (C.POINTER(MixerState) * n)(*[C.pointer(v) for v in states]), n, _ptr(x, "x", torch.float32), B, S, int(pos0),
+                                           _ptr(pos_dev, "pos_dev", torch.int32), _ptr(workspace, "workspace", torch.uint8), workspace.numel(), _stream())
+    _check(rc, "raven_mixer_layers_forward")

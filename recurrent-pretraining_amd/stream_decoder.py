@@ -114,8 +114,12 @@ class StreamDecoderForCausalLM(MinimalGeneration, PreTrainedModel, GenerationMix
         """(layer, pass) in the order they run; pass is None outside a loop."""
         return [(i, None) for i in range(len(self.layers))]
 
+    def enters_run(self, layer: int, turn: Optional[int]) -> bool:
+        """Whether enter_run() is called before a layer runs in pass `turn`: wherever a family that has one does not say."""
+        return type(self).enter_run is not StreamDecoderForCausalLM.enter_run
+
     def enter_run(self, layer: int, turn: Optional[int], buf: dict) -> None:
-        """Called before a layer runs in pass `turn`."""
+        """What happens to the stream before a layer runs in pass `turn`, where enters_run() says so."""
 
     def initial_mean(self, name: str) -> float:
         """Mean of the synthetic values of a checkpoint tensor (init_weights)."""
@@ -214,11 +218,18 @@ class StreamDecoderForCausalLM(MinimalGeneration, PreTrainedModel, GenerationMix
         """Embedding and every layer run for rows ids [B*S]; leaves the stream in buf["x"]."""
         x = buf["x"]
         hip.embed_stream(self.embed, ids, self.embed_scale, x, buf["x0"])
-        for run, (i, t) in enumerate(self.runs):
-            self.enter_run(i, t, buf)
-            hip.mixer_layer(self.dims, self.layers[i].native, cache.native(run), x, B, S, pos0, buf["ws"], pos_dev=pos_dev)
+        at = 0
+        while at < len(self.runs):  # runs with nothing in between are one native call
+            if self.enters_run(*self.runs[at]):
+                self.enter_run(*self.runs[at], buf)
+            end = at + 1
+            while trail is None and end < len(self.runs) and not self.enters_run(*self.runs[end]):
+                end += 1
+            hip.mixer_layers(self.dims, [self.layers[i].native for i, _ in self.runs[at:end]], [cache.native(run) for run in range(at, end)], x, B, S, pos0,
+                             buf["ws"], pos_dev=pos_dev)
             if trail is not None:
                 trail.append(x[:, :self.config.width].clone())
+            at = end
         return x
 
     def _logits(self, x: torch.Tensor, h: torch.Tensor, out: torch.Tensor, ws) -> torch.Tensor:

@@ -482,6 +482,25 @@ def test_norm_between_two_products_of_a_few_rows(pkg, width, M):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
 
 
+@pytest.mark.parametrize("M", [17, 32, 40])
+@pytest.mark.parametrize("width,ff", [(1024, 4608), (2048, 8192), (2504, 5120)])
+def test_slices_of_a_layer_added_by_the_norm_of_the_next(pkg, width, ff, M):
+    """Single tokens of 17 sequences and more, whose last product is cut into slices: layers in one call, whose next norm adds them, give the bits of layers called one by
+    one (as output_hidden_states has them); widths of one, two and three pieces a thread."""
+    cfg = G.config(width, 96, [G.attn(4, 2, 64, ff), G.delta(2, 64, ff), G.attn(2, 2, 96, ff)], taps=3)
+    w = O.random_weights(cfg, 8, 3)
+    raw = {**cfg, "layers": [{**x, "mixer": {**x["mixer"], **({"rank": 8} if x["type"] == "general_delta" else {})}} for x in cfg["layers"]]}
+    model = pkg.GitipelForCausalLM(pkg.GitipelConfig(**raw), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    assert pkg.hip.middle_plan(M, pad8(width), ff, False, pkg.hip.linear_workspace(M, width, "cuda").numel())[4] > 1
+    ids = torch.stack([G.tokens(cfg, 3, seed=s) for s in range(M)])
+    caches = [model.new_cache(), model.new_cache()]
+    for t in range(3):
+        got, want = (model.forward(ids[:, t:t + 1], past_key_values=c, output_hidden_states=apart).logits for c, apart in zip(caches, (False, True)))
+        assert torch.equal(got, want) and got.isfinite().all(), t
+    assert all(torch.equal(a, b) for a, b in zip(*(c.rings for c in caches)))
+
+
 def test_interleaved_requests_of_unequal_length(pkg):
     """Requests that live at the same time, end, and hand their caches on."""
     from recurrent_pretraining_amd.trace import TraceReplay

@@ -651,6 +651,22 @@ def test_norm_between_the_output_product_and_a_mixture(pkg, width, M, shared):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
 
 
+@pytest.mark.parametrize("B,S", [(4, 1), (40, 1), (3, 70)])
+@pytest.mark.parametrize("width", [512, 2056, 4104])
+def test_mixture_ends_with_the_norm_of_the_next_layer(pkg, width, B, S):
+    """Layers in one call against layers called one by one (as output_hidden_states has them): only the order of a norm's squares differs.  One, two and three pieces a
+    thread; few rows and chunks."""
+    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(12, 12, 136, 136)), G.latent(2, 64, 16, 64, 64, 64, 9, G.moe(12, 12, 136)), G.rglru(256, 4, 3, G.dense(136))])
+    w = O.random_weights(cfg, 3)
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    ids = torch.stack([G.tokens(cfg, 2 * S, seed=s) for s in range(B)])
+    caches = [model.new_cache(), model.new_cache()]
+    for lo in (0, S):
+        got, want = (model.forward(ids[:, lo:lo + S], past_key_values=c, output_hidden_states=apart).logits for c, apart in zip(caches, (False, True)))
+        assert got.isfinite().all() and G.rel(got, want) < 1e-2, lo
+
+
 def test_interleaved_requests_of_unequal_length(pkg):
     """Requests that live at the same time, end, and hand their caches on."""
     from recurrent_pretraining_amd.trace import TraceReplay
