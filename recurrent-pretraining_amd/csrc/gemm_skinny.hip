@@ -888,15 +888,40 @@ static int dispatch_mfma(GemmArgs a, hipStream_t s) {
 // the vector kernel, whose whole-row loads stream twice as fast (5.5 TB/s): up to 8 rows from 32 MB on.
 template <int EPI, int MT>
 static void launch_rows_f32_tiles(const GemmArgs& a, dim3 grid, hipStream_t s) {
-    // up to 256 columns a wave of four has one round of loads to wait for; where the grid is several rounds long, four waves leave more of it
-    // resident (8192 x 2048 at 16 rows 20.5 / 22.2 us; SwiGLU of 16384 x 704 at 200 rows 113 / 141)
-    if (a.K > 256 && grid.x * grid.y <= (unsigned)(MT > 1 ? 2 : 1) * n_cus()) rows_f32_kernel<EPI, MT, 8><<<grid, dim3(512), 0, s>>>(a);
+    // Up to 256 columns a wave of four has one round of loads to wait for (SwiGLU: two matrices' worth, eight waves are faster from there on).  Where the grid is several
+    // rounds long, four waves leave more of it resident (16384 x 704 at 200 rows, SwiGLU, 113 / 141 us), but long rows of X are read sooner by eight:
+    // us by four / eight, 16 token rows a workgroup, SwiGLU of 1408 x 512 at 50 rows 9.9 / 8.1, of 2816 x 1024 at 200 58.7 / 52.7; 32, 1536 x 512 at 400 18.7 / 16.9;
+    // 64, 8192 x 2048 at 100 87 / 80, 1408 x 5632 at 500 173 / 158, but 1536 x 512 at 400 20.1 / 21.2.
+    const int64_t units = (int64_t)grid.x * grid.y, cus = n_cus();
+    const bool eight = EPI == EPI_SWIGLU ? (MT == 1 ? a.K >= 256 : a.K > 256 && units <= 2 * cus)
+                                         : a.K > 256 && (MT == 1 ? units <= cus : MT == 2 || units <= 2 * cus || a.K >= 1024);
+    if (eight) rows_f32_kernel<EPI, MT, 8><<<grid, dim3(512), 0, s>>>(a);
     else rows_f32_kernel<EPI, MT, 4><<<grid, dim3(256), 0, s>>>(a);
+}
+// Token rows of a workgroup, in tiles of 16: the fewest that take the fewest rounds of work.  The 64-bit matrix instruction is the slow part (64 cycles for 16 x 16 x 4), so a small
+// model's product over 16 to 90 workgroups of 64 token rows leaves the chip idle.  us, 64 / 16 rows a workgroup: 256 x 704 at 17 rows (32 then) 6.7 / 4.8, at 100 11.6 / 5.0;
+// 768 x 256 at 50 6.1 / 3.2; 512 x 1408 at 100 18.3 / 7.6.  Past one round 16 rows cost a quarter more for the same work (weights and token rows are
+// read, and widened, for fewer products): 1536 x 512 at 400 20.1 / 20.4, with 32 rows 16.9; 2048 x 2048 at 500 88 / 115.  Matrices past 32 MB, which the caches between the XCDs
+// and memory would hand out once per row tile, keep as many rows as there are (8192 x 2048 at 40 rows 40 / 43).
+static int rows_f32_tiles(int M, int N, int K, bool swiglu) {
+    const int most = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    if ((int64_t)N * K * (swiglu ? 8 : 4) > (32 << 20)) return most;
+    int best = most;
+    double least = 0;
+    for (int mt = most; mt >= 1; mt /= 2) {
+        const int64_t units = (int64_t)((N + 15) / 16) * ((M + 16 * mt - 1) / (16 * mt)), rounds = (units + n_cus() - 1) / n_cus();
+        const double work = (double)rounds * mt * (mt == 1 && rounds > 1 ? 1.25 : 1.0);
+        if (mt == most || work < least) {
+            best = mt;
+            least = work;
+        }
+    }
+    return best;
 }
 template <int EPI>
 static int launch_rows_f32(GemmArgs a, hipStream_t s) {
     a.ldy = a.N;
-    const int M = a.M, mt = M <= 16 ? 1 : M <= 32 ? 2 : 4, most = 65535 * 16 * mt;
+    const int M = a.M, mt = rows_f32_tiles(M, a.N, a.K, EPI == EPI_SWIGLU), most = 65535 * 16 * mt;
     for (int m0 = 0; m0 < M; m0 += most) {
         a.M = M - m0 < most ? M - m0 : most;
         const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));

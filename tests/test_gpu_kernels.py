@@ -1158,3 +1158,17 @@ def test_paged_attention_with_rows_that_no_sequence_owns(pkg, rows):
     q = rnd((sum(rows) + 300, nh * hd), dt, 932).cuda()
     want = pkg.hip.paged_prefill_attention(q[:sum(rows)].contiguous(), k, v, *args)
     assert torch.equal(pkg.hip.paged_prefill_attention(q, k, v, *args)[:sum(rows)], want)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 48, 64), (17, 256, 704), (33, 40, 260), (65, 768, 256), (129, 1024, 1024), (200, 1536, 512), (400, 1536, 512), (500, 1024, 4096), (600, 2056, 1036)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_float_rows_by_every_number_of_tiles(pkg, M, N, K, swiglu):
+    """Workgroups of 16, 32 and 64 token rows and of four and eight waves, last tiles that are partly empty: plain sums are the exact ones rounded (added up in 64 bits, half
+    a step; a whole one allows for sums next to a tie), gated ones within float's rounding of their functions."""
+    x, w = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).cuda(), torch.randn(N * (1 + swiglu), K, generator=torch.Generator().manual_seed(N)).cuda()
+    got, z = pkg.hip.linear(x, w, swiglu=swiglu).double(), x.double() @ w.double().T
+    if swiglu:
+        gate, up = z.chunk(2, -1)
+        assert close(got, torch.nn.functional.silu(gate) * up, "gated")[1] < 1e-6
+    else:
+        assert ((got - z).abs() <= z.abs() * 2.0 ** -23 + 1e-30).all()
