@@ -812,6 +812,22 @@ bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t
 int tiled_gemm_qkv_rope(const void* x, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out, void* k_cache,
                         void* v_cache, int64_t slot_off, int nh, int hd, int t_max, int M, int S, int K, int ldx, int pos0,
                         const int* pos_dev, void* workspace, size_t workspace_bytes, hipStream_t s);
+int rows_f32_fused(const void* x0, const void* x1, const void* norm_a, const void* norm_b, void* xa_out, const void* w, void* y, int M, int N, int K0, int K1, float eps,
+                   int swiglu, const RopeRows* rope, hipStream_t s);
+// A chunk of a few float rows: one or two norms, Wqkv and raven_qkv_bias_rope_cache_append in one launch
+int rows_f32_qkv(const void* x, const void* norm_a, const void* norm_b, void* xa_out, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out,
+                 const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, int n_heads, int head_dim, float eps, hipStream_t s) {
+    if (int rc = check_heads("qkv_append", n_heads, head_dim, RAVEN_F32)) return rc;
+    RAVEN_REQUIRE(x && wqkv && freqs && q_out, "qkv_append: null pointer");
+    RAVEN_REQUIRE(B > 0 && S > 0 && pos0 >= 0, "qkv_append: bad B=%d S=%d pos0=%d", B, S, pos0);
+    CacheView cv;
+    if (int rc = make_view("qkv_append", cache, slot, B, n_heads, head_dim, &cv)) return rc;
+    RAVEN_REQUIRE(pos0 + S <= cv.t_max, "qkv_append: positions %d..%d exceed the cache length %d", pos0, pos0 + S - 1, cv.t_max);
+    const RopeRows rope{freqs, static_cast<const float*>(qk_bias), static_cast<float*>(q_out), static_cast<float*>(cv.k) + cv.slot_off,
+                        static_cast<float*>(cv.v) + cv.slot_off, pos_dev, n_heads, head_dim, cv.t_max, S, pos0};
+    const int h = n_heads * head_dim;
+    return rows_f32_fused(x, nullptr, norm_a, norm_b, xa_out, wqkv, nullptr, B * S, 3 * h, h, 0, eps, 0, &rope, s);
+}
 int g_fuse_qkv_rope = 1;  // raven_set_tuning("fuse_qkv_rope"): 0 = a chunk's q | k | v product is stored and rotated by a launch of its own
 
 // A chunk's Wqkv product with raven_qkv_bias_rope_cache_append as its epilogue (bf16 shapes that take the tiled GEMM):

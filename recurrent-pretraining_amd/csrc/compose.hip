@@ -40,6 +40,12 @@ int qkv_linear_rope_append(const void* x, int ldx, const void* wqkv, const void*
                            const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, int n_heads,
                            int head_dim, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* done);
 
+bool rows_f32_fused_fits(int M, int N, int K0, int K1, bool swiglu);
+int rows_f32_fused(const void* x0, const void* x1, const void* norm_a, const void* norm_b, void* xa_out, const void* w, void* y, int M, int N, int K0, int K1, float eps,
+                   int swiglu, const RopeRows* rope, hipStream_t s);
+int rows_f32_qkv(const void* x, const void* norm_a, const void* norm_b, void* xa_out, const void* wqkv, const void* qk_bias, const float* freqs, void* q_out,
+                 const raven_kv_cache* cache, int slot, int B, int S, int pos0, const int32_t* pos_dev, int n_heads, int head_dim, float eps, hipStream_t s);
+
 extern int g_tiled_min_rows;
 bool tiled_gemm_fits(int M, int N, int K0, int K1, int dtype, int swiglu, size_t workspace_bytes, bool aligned, int f32_sums = 0);
 int tiled_gemm(const void* x0, int ldx, const void* x1, const void* w, const void* residual, void* y, int M, int N, int K0, int K1, int swiglu,
@@ -243,38 +249,60 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
     return linear_then_norm(s.g, 0, w->mlp_proj, s.x2, s.x3, w->norm_4, y_out, tail_w, tail_out, M, h, I, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, tail_ld);
 }
 
-// One row.  x_raw is the block input before `pre_norm` (the previous block's norm_4, or null when x_raw is
+// Whether a few float rows take the schedule of one row: every norm in front of a product is that product's own
+static bool few_float_rows(const raven_dims* d, const raven_block_weights* blocks, int n_blocks, const void* adapter_w, int M, bool paged) {
+    const int h = d->n_embd;
+    if (d->dtype != RAVEN_F32 || paged || !rows_f32_fused_fits(M, 3 * h, h, 0, false) || !rows_f32_fused_fits(M, d->intermediate, h, 0, true) ||
+        (adapter_w && !rows_f32_fused_fits(M, h, h, h, false)) || !raven_host::aligned16(adapter_w)) return false;
+    for (int j = 0; j < n_blocks; ++j) {
+        const raven_block_weights& w = blocks[j];
+        if (!raven_host::aligned16(w.wqkv, w.fc, w.norm_1, w.norm_2, w.norm_3, w.norm_4)) return false;
+    }
+    return true;
+}
+
+// A product of that schedule: raven_gemv_fused, or its like for a few float rows
+static int fused_rows(int M, const void* x0, const void* x1, const void* norm_a, const void* norm_b, void* xa_out, const void* w, const void* residual, void* y, int N,
+                      int K0, int K1, float eps, int swiglu, int dt, const BlockScratch& s, void* stream) {
+    if (M == 1) return raven_gemv_fused(x0, x1, norm_a, norm_b, xa_out, w, residual, y, N, K0, K1, eps, swiglu, 0, dt, stream);
+    if (norm_a) return rows_f32_fused(x0, x1, norm_a, norm_b, xa_out, w, y, M, N, K0, K1, eps, swiglu, nullptr, static_cast<hipStream_t>(stream));
+    return raven_linear(x0, x1, w, residual, y, M, N, K0, K1, swiglu, 0, dt, s.lin_ws, s.lin_ws_bytes, stream);
+}
+
+// One row, or a few float rows (few_float_rows).  x_raw is the block input before `pre_norm` (the previous block's norm_4, or null when x_raw is
 // the input itself).  Leaves the block output BEFORE its norm_4 in scratch.x3.
 static int run_block_one_row(const raven_dims* d, const raven_block_weights* w, const BlockScratch& s, const void* x_raw,
-                             const void* pre_norm, const float* freqs, const raven_kv_cache* cache, int slot, int pos0,
+                             const void* pre_norm, const float* freqs, const raven_kv_cache* cache, int slot, int B, int S, int pos0,
                              const int32_t* pos_dev, void* stream, const raven_paged_kv* paged = nullptr, int layer = 0) {
-    const int h = d->n_embd, I = d->intermediate, dt = d->dtype;
+    const int M = B * S, h = d->n_embd, I = d->intermediate, dt = d->dtype;
     const float eps = d->eps;
     int rc;
-    const void* x_res = x_raw;  // the residual the attention output is added to (RMM:534)
-    if (pre_norm) {
-        if ((rc = raven_gemv_fused(x_raw, nullptr, pre_norm, w->norm_1, s.xr, w->wqkv, nullptr, s.qkv, 3 * h, h, 0, eps, 0, 0, dt, stream))) return rc;
-        x_res = s.xr;
+    const void* x_res = pre_norm ? s.xr : x_raw;  // the residual the attention output is added to (RMM:534)
+    const void *norm_a = pre_norm ? pre_norm : w->norm_1, *norm_b = pre_norm ? w->norm_1 : nullptr;
+    if (S > 1) {  // a chunk: every row's keys must be in the cache before any row attends
+        if ((rc = rows_f32_qkv(x_raw, norm_a, norm_b, s.xr, w->wqkv, w->qk_bias, freqs, s.q, cache, slot, B, S, pos0, pos_dev, d->n_heads, d->head_dim, eps,
+                               static_cast<hipStream_t>(stream)))) return rc;
+        rc = raven_decode_attention(s.q, s.ya, cache, slot, B, S, pos0, pos_dev, d->n_heads, d->head_dim, dt, s.attn_ws, s.attn_ws_bytes, stream);
     } else {
-        if ((rc = raven_gemv_fused(x_raw, nullptr, w->norm_1, nullptr, nullptr, w->wqkv, nullptr, s.qkv, 3 * h, h, 0, eps, 0, 0, dt, stream))) return rc;
+        if ((rc = fused_rows(M, x_raw, nullptr, norm_a, norm_b, pre_norm ? s.xr : nullptr, w->wqkv, nullptr, s.qkv, 3 * h, h, 0, eps, 0, dt, s, stream))) return rc;
+        if (paged)
+            rc = raven_paged_qkv_attention_decode(s.qkv, w->qk_bias, freqs, s.ya, paged->k_caches[layer], paged->v_caches[layer],
+                                                  paged->block_table, paged->seq_lens, 1, paged->max_blocks, paged->block_size,
+                                                  paged->kv_layout, paged->max_seq_len, d->n_heads, d->head_dim, dt, s.attn_ws, s.attn_ws_bytes, stream);
+        else
+            rc = raven_qkv_attention_decode(s.qkv, w->qk_bias, freqs, s.ya, cache, slot, B, pos0, pos_dev, d->n_heads, d->head_dim, dt,
+                                            s.attn_ws, s.attn_ws_bytes, stream);
     }
-    if (paged)
-        rc = raven_paged_qkv_attention_decode(s.qkv, w->qk_bias, freqs, s.ya, paged->k_caches[layer], paged->v_caches[layer],
-                                              paged->block_table, paged->seq_lens, 1, paged->max_blocks, paged->block_size,
-                                              paged->kv_layout, paged->max_seq_len, d->n_heads, d->head_dim, dt, s.attn_ws, s.attn_ws_bytes, stream);
-    else
-        rc = raven_qkv_attention_decode(s.qkv, w->qk_bias, freqs, s.ya, cache, slot, 1, pos0, pos_dev, d->n_heads, d->head_dim, dt,
-                                        s.attn_ws, s.attn_ws_bytes, stream);
     if (rc) return rc;
-    if ((rc = raven_gemv_fused(s.ya, nullptr, nullptr, nullptr, nullptr, w->proj, x_res, s.x1, h, h, 0, eps, 0, 0, dt, stream))) return rc;
-    if ((rc = raven_gemv_fused(s.x1, nullptr, w->norm_2, w->norm_3, s.x2, w->fc, nullptr, s.g, I, h, 0, eps, 1, 0, dt, stream))) return rc;
-    return raven_gemv_fused(s.g, nullptr, nullptr, nullptr, nullptr, w->mlp_proj, s.x2, s.x3, h, I, 0, eps, 0, 0, dt, stream);
+    if ((rc = fused_rows(M, s.ya, nullptr, nullptr, nullptr, nullptr, w->proj, x_res, s.x1, h, h, 0, eps, 0, dt, s, stream))) return rc;
+    if ((rc = fused_rows(M, s.x1, nullptr, w->norm_2, w->norm_3, s.x2, w->fc, nullptr, s.g, I, h, 0, eps, 1, dt, s, stream))) return rc;
+    return fused_rows(M, s.g, nullptr, nullptr, nullptr, nullptr, w->mlp_proj, s.x2, s.x3, h, I, 0, eps, 0, dt, s, stream);
 }
 
 // closing norm_4 (+ ln_f) of the one-row schedule
-static int close_one_row(const raven_dims* d, const BlockScratch& s, const void* norm_4, const void* ln_f, void* out, void* stream) {
-    if (ln_f) return raven_rmsnorm_residual(s.x3, nullptr, norm_4, nullptr, nullptr, ln_f, out, 1, d->n_embd, d->eps, d->dtype, stream);
-    return raven_rmsnorm_residual(s.x3, nullptr, norm_4, out, nullptr, nullptr, nullptr, 1, d->n_embd, d->eps, d->dtype, stream);
+static int close_one_row(const raven_dims* d, const BlockScratch& s, const void* norm_4, const void* ln_f, void* out, int M, void* stream) {
+    if (ln_f) return raven_rmsnorm_residual(s.x3, nullptr, norm_4, nullptr, nullptr, ln_f, out, M, d->n_embd, d->eps, d->dtype, stream);
+    return raven_rmsnorm_residual(s.x3, nullptr, norm_4, out, nullptr, nullptr, nullptr, M, d->n_embd, d->eps, d->dtype, stream);
 }
 
 }  // namespace raven
@@ -298,9 +326,9 @@ extern "C" int raven_sandwich_block(const raven_dims* dims, const raven_block_we
     RAVEN_REQUIRE(((uintptr_t)workspace & 255) == 0, "sandwich_block: workspace must be 256-byte aligned");
     BlockScratch s;
     carve(dims, B * S, static_cast<char*>(workspace), &s);
-    if (B * S == 1 && one_row_fits(dims)) {
-        if (int rc = run_block_one_row(dims, w, s, x_in, nullptr, freqs, cache, slot, pos0, pos_dev, stream)) return rc;
-        return close_one_row(dims, s, w->norm_4, ln_f, x_out, stream);
+    if ((B * S == 1 && one_row_fits(dims)) || (raven_host::aligned16(x_in) && few_float_rows(dims, w, 1, nullptr, B * S, false))) {
+        if (int rc = run_block_one_row(dims, w, s, x_in, nullptr, freqs, cache, slot, B, S, pos0, pos_dev, stream)) return rc;
+        return close_one_row(dims, s, w->norm_4, ln_f, x_out, B * S, stream);
     }
     const int ld_decode = decode_row_pitch(dims, s, w, 1, B * S, S, false), ld_chunk = chunk_row_pitch(dims, s, w, 1, x_in, cache, B * S, S, false, nullptr);
     if (ln_f) return run_block(dims, w, s, false, x_in, nullptr, ln_f, x_out, freqs, cache, slot, B, S, pos0, pos_dev, stream, nullptr, nullptr, 0, ld_decode, ld_chunk);
@@ -337,12 +365,12 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
     hipStream_t hs = static_cast<hipStream_t>(stream);
 
     int rc;
-    if (M == 1 && !rows && one_row_fits(dims)) {
-        // One row: between two iterations the last block's closing norm_4 is the prologue of the next adapter product
+    if (!rows && ((M == 1 && one_row_fits(dims)) || (raven_host::aligned16(state_in, embeds) && few_float_rows(dims, blocks, n_blocks, adapter_w, M, paged != nullptr)))) {
+        // One row, or a few float ones: between two iterations the last block's closing norm_4 is the prologue of the next adapter product
         // (no launch of its own); only the last iteration closes with a norm launch (norm_4, then ln_f if asked for).
         // The embedding half of the adapter product is the same in every recurrence: with two or more of them its fp32
         // sums are formed once, and each recurrence streams the state half of the weight only.
-        const bool split = n_iterations >= 2;
+        const bool split = M == 1 && n_iterations >= 2;
         const size_t es = raven_host::elt_size(dims->dtype);
         if (split)
             if ((rc = gemv1_column_block(embeds, nullptr, static_cast<const char*>(adapter_w) + (size_t)h * es, 2 * h, nullptr, s.e_sums,
@@ -355,18 +383,17 @@ static int iterations_impl(const char* who, const raven_dims* dims, const void* 
                 if (split)
                     rc = gemv1_column_block(x_in, pre_norm, adapter_w, 2 * h, s.e_sums, s.xa, 0, h, h, dims->eps, dims->dtype, hs);
                 else
-                    rc = raven_gemv_fused(x_in, embeds, pre_norm, nullptr, nullptr, adapter_w, nullptr, s.xa, h, h, h, dims->eps, 0, 0,
-                                          dims->dtype, stream);
+                    rc = fused_rows(M, x_in, embeds, pre_norm, nullptr, nullptr, adapter_w, nullptr, s.xa, h, h, h, dims->eps, 0, dims->dtype, s, stream);
                 if (rc) return rc;
             }
             for (int j = 0; j < n_blocks; ++j) {
                 const void* x_raw = j == 0 ? (adapter_w ? (const void*)s.xa : state_in) : (const void*)s.x3;
                 const void* pre = j == 0 ? nullptr : blocks[j - 1].norm_4;
-                if ((rc = run_block_one_row(dims, &blocks[j], s, x_raw, pre, freqs, cache, sl ? sl[j] : 0, pos0, pos_dev, stream, paged, j)))
+                if ((rc = run_block_one_row(dims, &blocks[j], s, x_raw, pre, freqs, cache, sl ? sl[j] : 0, B, S, pos0, pos_dev, stream, paged, j)))
                     return rc;
             }
         }
-        return close_one_row(dims, s, last_blk.norm_4, ln_f, state_out, stream);
+        return close_one_row(dims, s, last_blk.norm_4, ln_f, state_out, M, stream);
     }
     // bf16: the adapter is split by columns as for one row (embedding half summed once, in fp32).  From 33 rows on that is one launch more for half of
     // every other one, which a few recurrences of a small adapter don't repay: from 32 MB of weights that are not read again on.  us per recurrence at 5280 columns, whole / split: 93

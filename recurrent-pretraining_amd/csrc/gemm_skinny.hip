@@ -14,6 +14,7 @@
 //   SwiGLU: T(T(silu(gate)) * up), gate row j, up row j+I  RMM:507-508
 // The adapter's concat (RMM:776) is folded in by giving X as two pointers that cover K0 and K1.
 
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -69,6 +70,7 @@ struct Tuning {
     int gemm_ragged = 1;         // 0 never, 1 = one workgroup per resident slot with partly empty last tiles where the shape divides so
 };
 static Tuning g_tuning;
+extern int g_f32_norm_rows;
 
 int set_skinny_tuning(const char* key, int value) {
     const std::string k(key);
@@ -79,6 +81,7 @@ int set_skinny_tuning(const char* key, int value) {
     else if (k == "gemm_four_tiles") g_tuning.gemm_four_tiles = value;
     else if (k == "gemm_one_round") g_tuning.gemm_one_round = value;
     else if (k == "gemm_ragged") g_tuning.gemm_ragged = value;
+    else if (k == "f32_norm_rows") g_f32_norm_rows = value;
     else if (k == "gemm_mfma_min_rows" && value >= 2) g_tuning.gemm_mfma_min_rows = value;
     else return -1;
     return 0;
@@ -602,8 +605,21 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_kernel(GemmArgs a) {
 // launches of 4.5 to 8 us, now one of 5; 200 rows 25 launches.  With four waves the walk was longer than gemv_kernel's passes for few rows: us,
 // passes / four waves / eight, 2048 x 2048 at 8 rows 11.7 / 12.1 / 9.8, 512 x 4096 at 9 rows 21.4 / 19.7 / 15.8, SwiGLU of 512 x 2048 at 9, 17 and 33 rows 13.5 / 19.4 / 14.9, 23.0 / 24.6 / 21.9, 42.3 / 42.6 / 39.1.
 // ------------------------------------------------------------------------------------------------
-template <int EPI, int MT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(GemmArgs a) {
+// NORMED: the rows of x0 go through one or two RMSNorms first.  A workgroup norms its token rows itself, a wave per row in turn, and multiplies them out of
+// the LDS: a small model's launch of its own for a norm takes 3.2 us, and 2.8 to enqueue, more than the repeated work of 16 to 90 workgroups.  Squares are added
+// as rmsnorm_kernel adds them, rows of up to 1024 columns: the same bits.  Rotation and cache append of a chunk's q | k | v rows may ride in the epilogue.
+struct NormedRows : GemmArgs {
+    const float *norm_a, *norm_b;  // x0 <- norm_b(norm_a(x0)); norm_a may be null
+    float* xa_out;                 // norm_a(x0), or null
+    float eps;
+    int rope_on;                   // EPI_PLAIN: the rows leave as RopeRows says instead of to y
+    RopeRows rope;
+};
+constexpr int kNormedColumns = 1024;
+__host__ __device__ constexpr int normed_pitch(int k0) { return k0 + 20; }  // floats: 16 rows' pieces of 16 bytes on all 64 banks
+
+template <int EPI, int MT, int WAVES, bool NORMED = false>
+__global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(std::conditional_t<NORMED, NormedRows, GemmArgs> a) {
     typedef __attribute__((ext_vector_type(4))) double f64x4;
     constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, U = 4;
     __shared__ __align__(16) f64x4 red[WAVES - 1][NT * MT][64];
@@ -617,6 +633,54 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(GemmArgs a) {
     for (int j = 0; j < MT; ++j) row[j] = min(m0 + 16 * j + r, a.M - 1);
     const int chunks = (K + 15) / 16, c0 = chunks * wave / WAVES, c1 = chunks * (wave + 1) / WAVES;
 
+    extern __shared__ __align__(16) float normed[];  // NORMED: [16 MT][normed_pitch(k0)]
+    if constexpr (NORMED) {
+        constexpr int RPW = 16 * MT / WAVES, NI = kNormedColumns / 256;
+        const int pieces = a.k0 / 4, pitch = normed_pitch(a.k0);
+        f32x4 v[RPW][NI];
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int n = 0; n < NI; ++n)
+                if (256 * n < a.k0) v[i][n] = load4(static_cast<const float*>(a.x0) + (int64_t)min(m0 + wave + WAVES * i, a.M - 1) * a.k0 + 4 * min(lane + 64 * n, pieces - 1));
+        auto norm = [&](f32x4 (&x)[NI], const float* weight) __attribute__((always_inline)) {
+            float sums[NI];
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+                sums[n] = 0.f;
+                if (256 * n >= a.k0) continue;
+                float ss = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(x[n][e], x[n][e], ss);
+                sums[n] = raven::wave_sum(lane + 64 * n < pieces ? ss : 0.f);
+            }
+            const float inv = rsqrtf((sums[0] + sums[1] + sums[2] + sums[3]) / (float)a.k0 + a.eps);
+#pragma unroll
+            for (int n = 0; n < NI; ++n)
+                if (256 * n < a.k0) {
+                    const f32x4 w = load4(weight + 4 * min(lane + 64 * n, pieces - 1));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[n][e] = x[n][e] * inv * w[e];
+                }
+        };
+        static_assert(NI == 4, "the sum above");
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            const int at = wave + WAVES * i;
+            if (a.norm_a) {
+                norm(v[i], a.norm_a);
+#pragma unroll
+                for (int n = 0; n < NI; ++n)
+                    if (a.xa_out && blockIdx.x == 0 && m0 + at < a.M && lane + 64 * n < pieces) store4(a.xa_out + (int64_t)(m0 + at) * a.k0 + 4 * (lane + 64 * n), v[i][n]);
+            }
+            norm(v[i], a.norm_b);
+#pragma unroll
+            for (int n = 0; n < NI; ++n)
+                if (lane + 64 * n < pieces) store4(normed + at * pitch + 4 * (lane + 64 * n), v[i][n]);
+        }
+        __syncthreads();
+    }
+
     f64x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -624,6 +688,9 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(GemmArgs a) {
         for (int j = 0; j < MT; ++j) acc[t][j] = f64x4{0.0, 0.0, 0.0, 0.0};
     auto load_x = [&](int j, int k) __attribute__((always_inline)) {
         const bool second = k >= a.k0;
+        if constexpr (NORMED) {
+            if (!second) return load4(normed + (16 * j + r) * normed_pitch(a.k0) + k);
+        }
         const float* x = second ? static_cast<const float*>(a.x1) - a.k0 : static_cast<const float*>(a.x0);
         return *reinterpret_cast<const f32x4*>(x + row[j] * (second ? a.k1 : a.k0) + k);
     };
@@ -679,6 +746,29 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(GemmArgs a) {
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int w = 0; w < WAVES - 1; ++w) acc[t][j] += red[w][t * MT + j][lane];
+        if constexpr (NORMED && EPI == EPI_PLAIN) {
+            if (a.rope_on) {  // as qkv_rope_append_tiled_kernel; a pair's halves lie in lanes 16 apart
+                const RopeRows& p = a.rope;
+                const int h = p.nh * p.hd, b = min(m, a.M - 1) / p.S, sq = min(m, a.M - 1) - b * p.S, pos = (p.pos_dev ? *p.pos_dev : p.pos0) + sq;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int n = min(n0 + 4 * v + q, a.N - 1), sec = n >= 2 * h ? 2 : n >= h ? 1 : 0, col = n - sec * h, head = col / p.hd, d = col - head * p.hd;
+                    float x = (float)acc[0][j][v];
+                    if (sec < 2 && p.qk_bias) x += p.qk_bias[n];
+                    const float other = __shfl_xor(x, 16, 64);
+                    if (sec < 2) {
+                        const float* f = p.freqs + ((int64_t)pos * (p.hd / 2) + d / 2) * 2;
+                        float first = q & 1 ? other : x, second = q & 1 ? x : other;
+                        rope_pair<float>(first, second, f[0], f[1]);
+                        x = q & 1 ? second : first;
+                    }
+                    if (m >= a.M || n0 + 4 * v + q >= a.N) continue;
+                    if (sec == 0) p.q_out[(int64_t)m * h + col] = x;
+                    else if (pos < p.t_max) (sec == 1 ? p.k : p.v)[(((int64_t)b * p.nh + head) * p.t_max + pos) * p.hd + d] = x;
+                }
+                continue;
+            }
+        }
         if (m >= a.M) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {  // a lane holds weight rows 4 v + q of token row r
@@ -939,6 +1029,55 @@ static int launch_rows_f32(GemmArgs a, hipStream_t s) {
     return 0;
 }
 
+// ---- float rows behind norms ----
+// What rows_f32_fused takes: rows of up to 1024 columns that go to rows_f32_kernel, few enough that norming them in every workgroup is cheaper than a launch.  us of a whole
+// prompt (four recurrences of two blocks; passes queued one after the other), launches of their own / this: width 256, 5 to 64 tokens 392 to 425 / 306 to 331, 100: 391 / 389, 400: 628 / 785;
+// width 384, 33: 424 / 375, 64: 442 / 461; width 512, 17: 423 / 407, 33: 447 / 505.
+static bool rows_f32_takes(int M, int N, int K, bool swiglu) {
+    return M >= 2 && (M > 8 || (size_t)N * K * (swiglu ? 8 : 4) < (32u << 20)) && !(M <= 8 && gemv_wide_pays(M, N, K, swiglu));
+}
+constexpr int kNormedValues = 16384;
+int g_f32_norm_rows = 64;  // raven_set_tuning("f32_norm_rows"): up to so many rows
+static size_t rows_f32_fused_lds(int mt, int K0) { return (size_t)16 * mt * normed_pitch(K0) * sizeof(float); }
+static int rows_f32_fused_tiles(int M, int N, int K, bool swiglu) { return std::min(rows_f32_tiles(M, N, K, swiglu), 2); }
+bool rows_f32_fused_fits(int M, int N, int K0, int K1, bool swiglu) {
+    if (M < 2 || M > g_f32_norm_rows || (int64_t)M * K0 > kNormedValues || K0 > kNormedColumns || K0 % 4 != 0 || K1 % 4 != 0 || !rows_f32_takes(M, N, K0 + K1, swiglu)) return false;
+    return rows_f32_fused_lds(rows_f32_fused_tiles(M, N, K0 + K1, swiglu), K0) <= 80 * 1024;  // (the waves' sums take up to 57 KB more)
+}
+template <int EPI, int MT, int WAVES>
+static int launch_rows_f32_fused(const NormedRows& a, hipStream_t s) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        const hipError_t e = hipFuncSetAttribute((const void*)rows_f32_kernel<EPI, MT, WAVES, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+        if (e != hipSuccess) {
+            raven_host::set_error("gemm (fp32 rows): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+            return (int)e;
+        }
+        attr_set = true;
+    }
+    rows_f32_kernel<EPI, MT, WAVES, true><<<dim3((a.N + 15) / 16, (a.M + 16 * MT - 1) / (16 * MT)), dim3(64 * WAVES), rows_f32_fused_lds(MT, a.k0), s>>>(a);
+    return raven_host::check_launch("gemm (fp32 rows, norms)");
+}
+// raven_gemv_fused for 2 and more float rows that rows_f32_fused_fits takes: y = concat(norm_b(norm_a(x0)), x1) W^T, or the gated half of it; xa_out = norm_a(x0).  With one
+// norm it is norm_a that is given, as there.  rope (may be null): see RopeRows; y is then not written.
+int rows_f32_fused(const void* x0, const void* x1, const void* norm_a, const void* norm_b, void* xa_out, const void* w, void* y, int M, int N, int K0, int K1, float eps,
+                   int swiglu, const RopeRows* rope, hipStream_t s) {
+    RAVEN_REQUIRE(rows_f32_fused_fits(M, N, K0, K1, swiglu != 0) && norm_a && raven_host::aligned16(x0, x1, norm_a, norm_b, xa_out, w), "gemm (fp32 rows, norms): unsupported shape or operands");
+    NormedRows a{};
+    a.w = w; a.x0 = x0; a.x1 = x1; a.y = y;
+    a.M = M; a.N = N; a.K = K0 + K1; a.k0 = K0; a.k1 = K1; a.ldy = N; a.eps = eps;
+    a.norm_a = norm_b ? static_cast<const float*>(norm_a) : nullptr;
+    a.norm_b = static_cast<const float*>(norm_b ? norm_b : norm_a);
+    a.xa_out = norm_b ? static_cast<float*>(xa_out) : nullptr;
+    if (rope) {
+        a.rope = *rope;
+        a.rope_on = 1;
+    }
+    const bool one = rows_f32_fused_tiles(M, N, a.K, swiglu != 0) == 1;
+    if (swiglu) return one ? launch_rows_f32_fused<EPI_SWIGLU, 1, 8>(a, s) : launch_rows_f32_fused<EPI_SWIGLU, 2, 8>(a, s);
+    return one ? launch_rows_f32_fused<EPI_PLAIN, 1, 8>(a, s) : launch_rows_f32_fused<EPI_PLAIN, 2, 8>(a, s);
+}
+
 // Runs one GEMM over all M rows, in passes of at most 32 (MFMA) or 8 / 4 (vector) rows.
 template <int EPI>
 static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
@@ -947,8 +1086,8 @@ static int run_gemm(GemmArgs a, int dtype, hipStream_t s) {
     const int M = a.M;
     const size_t out_es = a.out_f32 ? 4 : es;
     RAVEN_REQUIRE(dtype != RAVEN_F32 || (size_t)a.K * es <= 160 * 1024, "gemm: one row of K=%d elements does not fit the 160 KB LDS", a.K);
-    if (dtype == RAVEN_F32 && M >= 2 && (M > 8 || (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20)))
-        return M <= 8 && gemv_wide_pays(M, a.N, a.K, EPI == EPI_SWIGLU) ? dispatch_gemv_wide<EPI>(a, s) : launch_rows_f32<EPI>(a, s);
+    if (dtype == RAVEN_F32 && rows_f32_takes(M, a.N, a.K, EPI == EPI_SWIGLU)) return launch_rows_f32<EPI>(a, s);
+    if (dtype == RAVEN_F32 && M >= 2 && M <= 8 && (size_t)a.N * a.K * (EPI == EPI_SWIGLU ? 8 : 4) < (32u << 20)) return dispatch_gemv_wide<EPI>(a, s);
     for (int m0 = 0; m0 < M;) {
         const int left = M - m0;
         int pass;

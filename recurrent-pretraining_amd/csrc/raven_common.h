@@ -206,6 +206,14 @@ __device__ __forceinline__ void rope_pair(T& a, T& b, float cs, float sn) {
     b = from_f32<T>(r1);
 }
 
+// Where a chunk's float q | k | v rows go (rows_f32_fused): bias, rotation, q to q_out and k, v to their cache rows
+struct RopeRows {
+    const float *freqs, *qk_bias;  // qk_bias [2, nh * hd] or null
+    float *q_out, *k, *v;          // k, v: the slot's first element
+    const int* pos_dev;            // position of a sequence's first row, on the device (or null: pos0)
+    int nh, hd, t_max, S, pos0;
+};
+
 }  // namespace raven
 
 // ---- host side ------------------------------------------------------------------------------

@@ -984,6 +984,31 @@ def test_core_iterations_equal_single_iterations(pkg, tiny32, tiny16, dt, B):
         pkg.hip.core_iterations(nat["dims"], t.adapter.weight, nat["core"], state, emb, many, nat["freqs"], caches[0][2], [[0]], B, 1, T, ws)
 
 
+@pytest.mark.parametrize("B,S", [(2, 1), (17, 1), (1, 17), (3, 5), (1, 16), (2, 29)])
+@pytest.mark.parametrize("h,nh", [(64, 1), (264, 3), (256, 4), (512, 8), (1000, 25)])
+def test_norms_inside_the_products_of_a_few_float_rows_change_no_bit(pkg, tuned, h, nh, B, S):
+    """Float rows whose norms, rotation and cache append ride in the products (f32_norm_rows): recurrences and a single block, chunks and single tokens behind cached
+    positions, give the bits of launches of their own, in the result and in the cache; rows of one to four pieces a lane, whole and partial tiles."""
+    hip, dt, hd, inter, T, r = pkg.hip, torch.float32, h // nh, 176, 6, 2
+    g = torch.Generator().manual_seed(h + S)
+    mk = lambda *s: (torch.randn(*s, generator=g) * 0.05).cuda()
+    keep = [[1 + mk(h) for _ in range(4)] + [mk(3 * h, h), mk(2, 1, nh, hd), mk(h, h), mk(2 * inter, h), mk(h, inter)] for _ in range(2)]
+    blocks = (hip.BlockWeights * 2)(*[hip.make_block_weights(*k) for k in keep])
+    dims, M = hip.make_dims(h, nh, inter, 1e-6, dt), B * S
+    freqs = O.rope_table(hd, 64, 50000).float().reshape(64, hd // 2, 2).contiguous().cuda()
+    adapter, ln_f, x, e, k0, v0 = mk(h, 2 * h), 1 + mk(h), mk(M, h) * 20, mk(M, h) * 20, mk(2 * r, B, nh, T + S, hd), mk(2 * r, B, nh, T + S, hd)
+    ws, outs = hip.block_workspace(dims, M, "cuda"), []
+    for rows in (64, 0):
+        tuned(f32_norm_rows=rows)
+        k, v = k0.clone(), v0.clone()
+        cache = hip.make_cache(k, v)
+        many = hip.core_iterations(dims, adapter, blocks, x, e, torch.empty_like(x), freqs, cache, [[0, 1], [2, 3]], B, S, T, ws, ln_f=ln_f)
+        one = hip.sandwich_block(dims, blocks[0], x, torch.empty_like(x), freqs, cache, 0, B, S, T, ws)
+        outs.append((many, one, k, v))
+    assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
+    del keep
+
+
 def test_from_pretrained_directory_gives_the_same_model(pkg, tiny32, tmp_path):
     """A checkpoint directory written by save_pretrained (the layout of the reference's published checkpoints) loads
     onto the GPU into a model with the same bits in every output."""
