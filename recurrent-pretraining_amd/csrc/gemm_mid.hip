@@ -123,7 +123,12 @@ __host__ __device__ constexpr int mid_requests(int tiles, int waves) { return (2
 
 // GROUPED: row groups with a weight matrix each; a unit works on a copy of the arguments cut to its group's rows
 // ONCE: every weight row is read by one unit
-template <int WN, int WM, int NT, int MT, int NS, bool ONCE, bool GROUPED = false>
+// HALF: rows of K = 64 n + 32 elements on a matrix that starts on a line (5280: 82.5 lines), so that odd rows start in the middle of one, and a step of 64 columns of such a
+// row would be two half lines.  The unit's even rows are the first wave row's tiles and its odd rows the second's; odd rows are requested line by line too, 32 columns in
+// front of the even ones, and their waves multiply each of the lines' halves with the token fragments of the half before: the same products in the same order, without
+// slices; with slices the odd rows' begin and end 32 columns earlier.  us per launch at 195 rows, weights from HBM, half lines / so: mlp.fc 110 / 99 (copies
+// with padded rows 93), Wqkv 61 / 57, attn.proj 25.4 / 24.5; at 93 rows 90 / 74, 51 / 45, 24 / 22.6 (there with token rows of half lines as well).
+template <int WN, int WM, int NT, int MT, int NS, bool ONCE, bool GROUPED = false, bool HALF = false>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     constexpr int NW = WN * WM, WPW = mid_requests(WN * NT, NW) / NW, XPW = mid_requests(WM * MT, NW) / NW, LPW = WPW + XPW;  // requests of a wave per step
     static_assert(NW % 2 == 0 && (NS - 1) * LPW < 64, "a wave's pieces have one parity; the wait counter holds 63 requests");
@@ -160,8 +165,9 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     const int n0 = tile_n * a.cols, ncols = min(a.cols, a.N - n0), m0 = tile_m * a.bm, rows = min(a.bm, a.M - m0);
     // the wave's tiles, dealt out evenly; a SIMD's two waves (ids that differ by four) get a long and a short share of the token tiles
     const int wn = wave / WM, wm = (wn & 1) ? WM - 1 - wave % WM : wave % WM;
-    const int tw = __builtin_amdgcn_readfirstlane(((swiglu ? 2 * ncols : ncols) + 15) >> 4), tx = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
-    const int nw = tw / WN + (wn < tw % WN), tw0 = wn * (tw / WN) + min(wn, tw % WN);
+    static_assert(!HALF || (WN == 2 && !GROUPED), "a wave row for each parity");
+    const int tw = __builtin_amdgcn_readfirstlane(((HALF == swiglu ? ncols : HALF ? ncols / 2 : 2 * ncols) + 15) >> 4), tx = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
+    const int nw = HALF ? tw : tw / WN + (wn < tw % WN), tw0 = HALF ? wn * NT : wn * (tw / WN) + min(wn, tw % WN);
     const int nx = tx / WM + (wm < tx % WM), tx0 = wm * (tx / WM) + min(wm, tx % WM);
     const int wbytes = a.wtiles * 2048, stage = wbytes + a.xtiles * 2048, ring = NS * stage;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_byte*)smem;
@@ -179,8 +185,9 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         const int piece = is_w ? NW * i + wave : NW * (i - WPW) + wave, r = piece * 8 + (lane >> 3);
         spare[i] = (GROUPED || i == WPW - 1 || i == LPW - 1) && piece >= 2 * (is_w ? a.wtiles : a.xtiles);  // (of a plain unit only the last ones may be)
         if (is_w) {
-            const int c = min(swiglu ? (r >> 4) * 8 + (r & 7) : r, ncols - 1);
-            goff[i] = (unsigned)(n0 + c + (swiglu && (r & 8) ? a.up_off : 0)) * (2u * a.ldw) + 2u * colp;
+            const int odd = HALF && r >= 16 * NT, rr = r - odd * 16 * NT, k = swiglu ? (rr >> 4) * 8 + (rr & 7) : rr;
+            const int c = HALF ? (2 * k + odd < ncols ? 2 * k + odd : ncols - 2 + odd) : min(k, ncols - 1);
+            goff[i] = (unsigned)(n0 + c + (swiglu && (rr & 8) ? a.up_off : 0)) * (2u * a.ldw) + 2u * colp - 64u * odd;
         } else {
             int row = m0 + min(r, rows - 1);
             if (GROUPED && x_row) row = x_row[row];
@@ -215,7 +222,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
             const unsigned to = __builtin_amdgcn_readfirstlane(spare[i] ? lds_base + ring : o + dst[i]);
             unsigned off = goff[i];
             asm volatile("" : "+v"(off));  // (the address is not worth a register pair outside this step)
-            const char* gp = col >= K ? zero : (i < WPW ? w0 : (col < a.K0 ? x0 : x1)) + 2 * c0 + off;
+            const bool past = HALF && i < WPW && (NW * i + wave) * 8 >= 16 * NT ? false : col >= K;  // (odd rows: 32 columns less)
+            const char* gp = past ? zero : (i < WPW ? w0 : (col < a.K0 ? x0 : x1)) + 2 * c0 + off;
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gp), "s"(to) : "memory");
         }
     };
@@ -255,7 +263,9 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         asm volatile("" ::: "memory");
     };
     // NTW x MTW: tiles of this wave; a wave without any requests its share and multiplies nothing
-    auto run = [&](auto nt_tag, auto mt_tag) __attribute__((always_inline)) {
+    // LATE: the odd rows' waves of HALF, half a step behind
+    auto run = [&](auto nt_tag, auto mt_tag, auto late_tag) __attribute__((always_inline)) {
+        constexpr bool LATE = decltype(late_tag)::value;
         constexpr int NTW = decltype(nt_tag)::value, MTW = decltype(mt_tag)::value;
         const unsigned pos0 = (q4 ^ ((l16 >> 1) & 7)) * 16;  // k-slice s of a step: pos0 ^ (64 s)
         const unsigned a_row = lds_base + (tw0 * 16 + l16) * 128, b_row = lds_base + wbytes + (tx0 * 16 + l16) * 128;
@@ -276,21 +286,67 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
                 for (int j = 0; j < MTW; ++j)
                     acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[sl][t]), __builtin_bit_cast(bf16x8, fb[sl][j]), acc[t][j], 0, 0, 0);
         };
+        // LATE: fragments of weight slice SL of the stage at o, of token slice SL into set DST; the products of set 0, whose fragments are followed by the next ones
+        auto fetch_w = [&](int o, auto sl_tag) __attribute__((always_inline)) {
+            constexpr int sl = decltype(sl_tag)::value;
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) fa[sl][t] = *reinterpret_cast<const lds_u32x4*>(a_row + o + (pos0 ^ (64 * sl)) + t * 2048);
+        };
+        auto fetch_x = [&](int o, auto sl_tag, auto dst_tag) __attribute__((always_inline)) {
+            constexpr int sl = decltype(sl_tag)::value, dst = decltype(dst_tag)::value;
+#pragma unroll
+            for (int j = 0; j < MTW; ++j) fb[dst][j] = *reinterpret_cast<const lds_u32x4*>(b_row + o + (pos0 ^ (64 * sl)) + j * 2048);
+        };
+        auto multiply_late = [&](int o) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < MTW; ++j) {
+#pragma unroll
+                for (int t = 0; t < NTW; ++t)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[0][t]), __builtin_bit_cast(bf16x8, fb[0][j]), acc[t][j], 0, 0, 0);
+                fb[0][j] = *reinterpret_cast<const lds_u32x4*>(b_row + o + (pos0 ^ 64) + j * 2048);
+            }
+        };
         int o = 0, i = 0;
         arrive_left(n_steps - 1);
-        fetch(0, ic0{});
+        if constexpr (LATE) {
+            fetch_w(0, ic0{});
+            if (k0 > 0) {
+                fetch_x(ring - stage, ic1{}, ic0{});
+            } else {  // the first line of an odd row begins with the end of the row before
+#pragma unroll
+                for (int t = 0; t < NTW; ++t) fa[0][t] = u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int j = 0; j < MTW; ++j) fb[0][j] = u32x4{0, 0, 0, 0};
+            }
+        } else {
+            fetch(0, ic0{});
+        }
+        if (HALF && k0 > 0) {  // the last stage held the token rows of the step before; it is free once they are read
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+        }
         // Small tiles: a loop without a branch for the steps whose requests are whole, another for the few that are not (uq of 1536 to 3072 columns at
         // 260 rows 10.7 -> 9.6 us).  Large ones: their products hide the branches, and registers are short.
         auto steps = [&](int end, auto whole_tag) __attribute__((always_inline)) {  // whose requests are of whole steps, or none of them
 #pragma unroll 1
             for (; i < end; ++i) {
                 const int free = o == 0 ? ring - stage : o - stage, next = o + stage == ring ? 0 : o + stage;
-                fetch(o, ic1{});
+                if constexpr (LATE) {
+                    fetch_w(o, ic1{});
+                    fetch_x(o, ic0{}, ic1{});
+                } else {
+                    fetch(o, ic1{});
+                }
                 issue(k0 + i + NS - 1, free, ic0{}, half{}, whole_tag);
-                multiply(ic0{});
+                if constexpr (LATE) multiply_late(o);
+                else multiply(ic0{});
                 issue(k0 + i + NS - 1, free, half{}, all{}, whole_tag);
                 arrive(std::integral_constant<int, NS - 2>{});
-                fetch(next, ic0{});
+                if constexpr (LATE) fetch_w(next, ic0{});
+                else fetch(next, ic0{});
                 multiply(ic1{});
                 o = next;
             }
@@ -308,16 +364,24 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
             constexpr int left = NS - 2 - decltype(j_tag)::value;  // steps behind this one
             if (n_steps <= left) return;
             const int next = o + stage == ring ? 0 : o + stage;
-            fetch(o, ic1{});
-            multiply(ic0{});
+            if constexpr (LATE) {
+                fetch_w(o, ic1{});
+                fetch_x(o, ic0{}, ic1{});
+                multiply_late(o);
+            } else {
+                fetch(o, ic1{});
+                multiply(ic0{});
+            }
             if constexpr (left > 0) {
                 arrive(std::integral_constant<int, (left > 0 ? left - 1 : 0)>{});
-                fetch(next, ic0{});
+                if constexpr (LATE) fetch_w(next, ic0{});
+                else fetch(next, ic0{});
             }
             multiply(ic1{});
             o = next;
         });
     };
+    if (HALF && k0 > 0) issue(k0 - 1, ring - stage, std::integral_constant<int, WPW>{}, all{}, ic1{});  // (a step in front of others is whole)
 #pragma unroll 1
     for (int i = 0; i < NS - 1 && i < n_steps; ++i) issue(k0 + i, i * stage, ic0{}, all{}, ic2{});
     // (with fewer tiles than one less than the variant's the surplus fragments are whatever lies behind, and their products are not stored)
@@ -325,11 +389,19 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     using nt1 = std::integral_constant<int, NT - 1>;
     using mt0 = std::integral_constant<int, MT>;
     using mt1 = std::integral_constant<int, MT - 1>;
-    if (__builtin_expect(nw == NT && nx == MT, 1)) run(nt0{}, mt0{});
-    else if (nw == 0 || nx == 0) run(ic0{}, ic0{});
-    else if (nw == NT) { if constexpr (MT > 1) run(nt0{}, mt1{}); }
-    else if (nx == MT) { if constexpr (NT > 1) run(nt1{}, mt0{}); }
-    else { if constexpr (NT > 1 && MT > 1) run(nt1{}, mt1{}); }
+    auto run_tiles = [&](auto late_tag) __attribute__((always_inline)) {
+        if (__builtin_expect(nw == NT && nx == MT, 1)) run(nt0{}, mt0{}, late_tag);
+        else if (nw == 0 || nx == 0) run(ic0{}, ic0{}, std::false_type{});
+        else if (nw == NT) { if constexpr (MT > 1) run(nt0{}, mt1{}, late_tag); }
+        else if (nx == MT) { if constexpr (NT > 1) run(nt1{}, mt0{}, late_tag); }
+        else { if constexpr (NT > 1 && MT > 1) run(nt1{}, mt1{}, late_tag); }
+    };
+    if constexpr (HALF) {
+        if (wn == 1) run_tiles(std::true_type{});
+        else run_tiles(std::false_type{});
+    } else {
+        run_tiles(std::false_type{});
+    }
 
     // ---- out: a lane holds rows 4 q4 ..+3 of weight tile t for token row 16 j + l16.  A wave lays its sums down in LDS, rows of its columns,
     // and a rolled loop takes them from there: whole runs of columns per store, and little code -- unrolled over the accumulators
@@ -342,10 +414,20 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     };
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();  // every wave has left the ring
-    constexpr int JG = MT % 2 ? 1 : 2, PITCH = NT * 64 + 16;    // row tiles at a time; bytes of an LDS row
-    const unsigned mine = lds_base + wave * (JG * 16 * PITCH);
+    // HALF: the two waves of the same token rows lay their columns down side by side, and each stores every other run of them.
+    constexpr int JG = MT % 2 ? 1 : 2, PITCH = (HALF ? 2 : 1) * NT * 64 + 16;    // row tiles at a time; bytes of an LDS row
+    const unsigned mine = lds_base + (HALF ? wm : wave) * (JG * 16 * PITCH);
     const int ntot = swiglu ? 2 * a.N : a.N;
-    const int col0 = tw0 * (swiglu ? 8 : 16), col_end = min(ncols, col0 + nw * (swiglu ? 8 : 16));  // this wave's output columns inside the unit
+    const int col0 = HALF ? 0 : tw0 * (swiglu ? 8 : 16), col_end = HALF ? ncols : min(ncols, col0 + nw * (swiglu ? 8 : 16));  // this wave's output columns inside the unit
+    auto out_sync = [&]() __attribute__((always_inline)) {
+        if constexpr (HALF) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        } else {
+            wave_sync();
+        }
+    };
     const int row_end = min(rows, (tx0 + nx) * 16);
 #pragma unroll 1
     for (int pass = 0; pass < MT / JG; ++pass) {
@@ -355,22 +437,30 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
 #pragma unroll
             for (int j = 0; j < JG; ++j)
 #pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    *reinterpret_cast<__attribute__((address_space(3))) f32x4*>(mine + (j * 16 + l16) * PITCH + t * 64 + q4 * 16) = acc[t][ps * JG + j];
+                for (int t = 0; t < NT; ++t) {
+                    const unsigned row = mine + (j * 16 + l16) * PITCH;
+                    if constexpr (HALF) {  // column 2 k + wn, k = 16 t + 4 q4 + v; SwiGLU: gates, k = 8 t + 4 q4 + v, and behind them all the ups
+                        const unsigned at = row + wn * 4 + (swiglu ? (q4 & 1) * 32 + t * 64 + (q4 >> 1) * (NT * 64) : t * 128 + q4 * 32);
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) *reinterpret_cast<__attribute__((address_space(3))) float*>(at + 8 * v) = acc[t][ps * JG + j][v];
+                    } else {
+                        *reinterpret_cast<__attribute__((address_space(3))) f32x4*>(row + t * 64 + q4 * 16) = acc[t][ps * JG + j];
+                    }
+                }
         });
-        wave_sync();
+        out_sync();
         const int first = (tx0 + pass * JG) * 16;
         auto store = [&](auto kind_tag) __attribute__((always_inline)) {
             constexpr int EPI = decltype(kind_tag)::value;
             constexpr bool SWIGLU = EPI == EPI_SWIGLU;
-            constexpr int UPR = SWIGLU ? NT * 2 : NT * 4;  // runs of four output columns per row
+            constexpr int UPR = (HALF ? 2 : 1) * (SWIGLU ? NT * 2 : NT * 4);  // runs of four output columns per row
 #pragma unroll 2
-            for (int idx = lane; idx < JG * 16 * UPR; idx += 64) {
+            for (int idx = HALF ? 64 * wn + lane : lane; idx < JG * 16 * UPR; idx += HALF ? 128 : 64) {
                 const int row = idx / UPR, u = idx - row * UPR, col = col0 + 4 * u, mr = first + row, m = m0 + mr;
                 if (col >= col_end || mr >= row_end) continue;
-                const unsigned at = mine + row * PITCH + (SWIGLU ? (u >> 1) * 64 + (u & 1) * 16 : u * 16);
+                const unsigned at = mine + row * PITCH + (SWIGLU && !HALF ? (u >> 1) * 64 + (u & 1) * 16 : u * 16);
                 const f32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at);
-                const f32x4 up = SWIGLU ? *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at + 32) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 up = SWIGLU ? *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(at + (HALF ? NT * 64 : 32)) : f32x4{0.f, 0.f, 0.f, 0.f};
                 if (a.ks > 1) {
                     float* p = a.partial + ((int64_t)slice * a.M + m) * ntot + n0 + col;
                     *reinterpret_cast<f32x4*>(p) = v;
@@ -386,7 +476,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         else if (a.kind == EPI_PLAIN || a.ks > 1) store(std::integral_constant<int, EPI_PLAIN>{});
         else if (a.kind == EPI_FREE_GELU) store(std::integral_constant<int, EPI_FREE_GELU>{});
         else store(std::integral_constant<int, EPI_FREE_TANH>{});
-        wave_sync();
+        out_sync();
     }
 }
 
@@ -418,6 +508,7 @@ __global__ __launch_bounds__(256) void gemm_mid_finish_kernel(MidArgs a) {
 // host
 // ------------------------------------------------------------------------------------------------
 int g_mid = 1;                              // raven_set_tuning("gemm_mid"): 0 = never
+int g_mid_half = 1;                         // raven_set_tuning("gemm_mid_half"): 0 = rows that are no whole lines are read as they lie
 int g_mid_nt = 0, g_mid_mt = 0, g_mid_ks = 0;  // raven_set_tuning("gemm_mid_nt" / "_mt" / "_ks"): 0 = by shape
 
 constexpr int kMidMaxSlices = 8;
@@ -586,12 +677,12 @@ size_t mid_workspace_bytes(int M, int N, const MidPlan& p, int swiglu) {
     return p.ks > 1 ? (size_t)p.ks * M * N * (swiglu ? 2 : 1) * sizeof(float) : 0;
 }
 
-template <int NT, int MT, bool ONCE>
+template <int NT, int MT, bool ONCE, bool HALF>
 static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
     constexpr int NS = mid_stages(NT, MT);
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<2, 4, NT, MT, NS, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_mid_kernel<2, 4, NT, MT, NS, ONCE, false, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) {
             raven_host::set_error("gemm (mid): hipFuncSetAttribute failed: %s", hipGetErrorString(e));
             return (int)e;
@@ -601,7 +692,7 @@ static int launch_mid_variant(const MidArgs& a, hipStream_t s) {
     const size_t lds = mid_lds_bytes(2, 4, NT, MT, NS, a.wtiles, a.xtiles);
     RAVEN_REQUIRE(lds <= (size_t)kLds && a.wtiles <= 2 * NT && a.wtiles > 2 * (NT - 1) && a.xtiles <= 4 * MT && a.xtiles > 4 * (MT - 1), "gemm (mid): a unit of %d x %d does not fit", a.cols, a.bm);
     const int64_t units = (int64_t)a.tiles_m * a.tiles_n * a.ks;
-    gemm_mid_kernel<2, 4, NT, MT, NS, ONCE><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
+    gemm_mid_kernel<2, 4, NT, MT, NS, ONCE, false, HALF><<<dim3((unsigned)((units + 7) / 8 * 8)), dim3(512), lds, s>>>(a);
     return raven_host::check_launch("gemm (mid)");
 }
 
@@ -617,9 +708,21 @@ static int finish_slices(const MidArgs& a, hipStream_t s) {
     return raven_host::check_launch("gemm (mid, sums)");
 }
 
-static int launch_mid(const MidArgs& a, const MidPlan& p, hipStream_t s, bool finish) {
+// Rows that start on lines and in their middles by turns, in units whose tiles may be one more (HALF)
+static bool half_lines(const MidArgs& a, const MidPlan& p) {
+    return g_mid_half && a.K1 == 0 && a.ldw == a.K0 && a.K0 % 64 == 32 && a.K0 > 64 && ((uintptr_t)a.w & 127) == 0 && a.up_off % 2 == 0 &&
+           mid_lds_bytes(2, 4, p.nt, p.mt, mid_stages(p.nt, p.mt), 2 * p.nt, a.xtiles) <= (size_t)kLds;
+}
+
+static int launch_mid(MidArgs a, const MidPlan& p, hipStream_t s, bool finish) {
     int rc;
-#define RAVEN_MID_CASE(NT_, MT_) case 10 * NT_ + MT_: rc = a.tiles_m == 1 ? launch_mid_variant<NT_, MT_, true>(a, s) : launch_mid_variant<NT_, MT_, false>(a, s); break;
+    const bool half = half_lines(a, p);
+    if (half) a.wtiles = 2 * p.nt;
+#define RAVEN_MID_CASE(NT_, MT_)                                                                                                                    \
+    case 10 * NT_ + MT_:                                                                                                                            \
+        rc = a.tiles_m == 1 ? (half ? launch_mid_variant<NT_, MT_, true, true>(a, s) : launch_mid_variant<NT_, MT_, true, false>(a, s))             \
+                            : (half ? launch_mid_variant<NT_, MT_, false, true>(a, s) : launch_mid_variant<NT_, MT_, false, false>(a, s));          \
+        break;
 #define RAVEN_MID_ROW(NT_) RAVEN_MID_CASE(NT_, 1) RAVEN_MID_CASE(NT_, 2) RAVEN_MID_CASE(NT_, 3) RAVEN_MID_CASE(NT_, 4)
     switch (p.nt * 10 + p.mt) {
         RAVEN_MID_ROW(1) RAVEN_MID_ROW(2) RAVEN_MID_ROW(3) RAVEN_MID_ROW(4) RAVEN_MID_ROW(5) RAVEN_MID_ROW(6)

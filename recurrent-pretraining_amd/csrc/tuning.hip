@@ -8,7 +8,7 @@ namespace raven {
 int set_gemv1_tuning(const char* key, int value);
 int set_skinny_tuning(const char* key, int value);
 extern int g_linear_ks;
-extern int g_mid, g_mid_nt, g_mid_mt, g_mid_ks;
+extern int g_mid, g_mid_half, g_mid_nt, g_mid_mt, g_mid_ks;
 extern int g_tiled_min_rows, g_tiled_variant, g_tiled_split_tail;
 extern int g_attn_split_target, g_attn_big_grid, g_attn_wide, g_linear_min_rows, g_attn_nosplit_pairs, g_attn_nosplit_len, g_rope_tiled_rows, g_prefill_waves, g_norm_early, g_fuse_sums_norm, g_attn_prefetch, g_fuse_qkv_rope, g_pad_chunk_rows, g_pad_decode_rows;
 }  // namespace raven
@@ -36,6 +36,7 @@ extern "C" int raven_set_tuning(const char* key, int32_t value) {
     else if (k == "gemm_tiled_variant" && value >= 0 && value <= 3) g_tiled_variant = value;
     else if (k == "gemm_tiled_split_tail" && (value == 0 || value == 1)) g_tiled_split_tail = value;
     else if (k == "gemm_mid" && (value == 0 || value == 1)) g_mid = value;
+    else if (k == "gemm_mid_half") g_mid_half = value;
     else if (k == "gemm_mid_nt" && value >= 0 && value <= 6) g_mid_nt = value;
     else if (k == "gemm_mid_mt" && value >= 0 && value <= 4) g_mid_mt = value;
     else if (k == "gemm_mid_ks" && value >= 0 && value <= 8) g_mid_ks = value;

@@ -414,6 +414,30 @@ def test_embedding_half_of_the_adapter_summed_once(pkg, tuned, M, h, nh):
     del keep
 
 
+@pytest.mark.parametrize("mt", [1, 2, 3, 4])
+@pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6])
+def test_rows_of_half_lines_by_parity(pkg, tuned, nt, mt):
+    """Weight rows that start on lines and in their middles by turns, every variant of units: read line by line (gemm_mid_half) they give the bits of rows read as they lie
+    where K is whole, and with slices, which odd rows begin 32 columns earlier, sums in another order; short and long K, a last unit of few columns, SwiGLU, a residual."""
+    hip, dt = pkg.hip, torch.bfloat16
+    for K, N, swiglu in ((160, 264, False), (672, 1048, False), (672, 520, True), (2080, 136, True)):
+        x, w = _gpu_randn((64 * mt - 20, K), 21), _gpu_randn((N * (1 + swiglu), K), 22, K ** -0.5)
+        res = None if swiglu else _gpu_randn((x.shape[0], N), 23)
+        for ks in (1, 3):
+            ws = hip.linear_workspace(x.shape[0], w.shape[0], "cuda")
+            outs = []
+            for half in (1, 0):
+                tuned(gemm_mid_half=half, gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
+                outs.append(hip.linear(x, w, residual=res, swiglu=swiglu, workspace=ws))
+            if ks == 1:
+                assert torch.equal(*outs), (K, N, swiglu)
+            else:
+                check(outs[0], outs[1].float(), dt, f"slices of {K} x {N}", ulps=ULPS_SWIGLU if swiglu else ULPS_RESIDUAL)
+            z = x.float() @ w.float().T
+            want = F.silu(z[:, :N]) * z[:, N:] if swiglu else z + res.float()
+            assert close(outs[0], want, "against float")[1] < 1e-2
+
+
 def test_few_rows_read_a_copy_where_they_may(pkg, tuned):
     """20 rows against 1032 x 4200, whose rows are not whole lines: with a registered copy the product is the middle kernel's and reads it; with
     pad_decode_rows = 0, or without a copy, it reads the matrix."""
