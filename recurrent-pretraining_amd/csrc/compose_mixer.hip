@@ -31,6 +31,9 @@ RAVEN_WEAK int moe_forward(const raven_moe* m, const void* h, const float* facto
                            int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, const float* next_norm, void* next_h);
 RAVEN_WEAK bool moe_norms_behind(const raven_moe* m, const void* h, int M, int ld, int dtype);
 RAVEN_WEAK bool moe_takes_factors(const raven_moe* m, const void* h, int M, int ld, int dtype);
+RAVEN_WEAK bool moe_picks_itself(const raven_moe* m, const void* h, int M, int ld, int dtype);
+RAVEN_WEAK int moe_forward_picked(const raven_moe* m, const void* xw, const NormBehind& behind, float* factors, float* logits, float* x, int M, int ld, float eps, int dim,
+                                  void* workspace, size_t workspace_bytes, hipStream_t s, const float* next_norm, void* next_h);
 
 int add_product_leave_sums(const void* x, const void* w, float* y, int M, int N, int K, int dtype, void* workspace, size_t workspace_bytes, hipStream_t s, int* ks_left);
 bool norm_conv_adds_slices(const float* conv, int taps, int ld, int dtype);
@@ -253,6 +256,8 @@ static int run_mixer_layer(const raven_stream_dims* dims, const raven_mixer_laye
         const NormAhead ahead{l.norm2, reinterpret_cast<bf16*>(w.h), w.squares};
         const NormBehind behind{w.squares, l.ff_kind == RAVEN_FF_MOE ? w.factors : nullptr, ld / 16, dims->width, dims->eps};
         if (int rc = gemm_free_normed(w.y, l.w_out, x, M, ld, inner, out, &ahead, nullptr, s)) return rc;
+        if (l.ff_kind == RAVEN_FF_MOE && moe_picks_itself(l.moe, w.h, M, ld, dt))
+            return moe_forward_picked(l.moe, w.h, behind, w.factors, w.logits, x, M, ld, dims->eps, dims->width, w.ff_ws, w.ff_ws_bytes, s, next_norm, w.h);
         if (l.ff_kind == RAVEN_FF_MOE) {
             in.out_f32 = 1;
             if (int rc = gemm_free_normed(w.h, second, second_y, M, second_n, ld, in, nullptr, &behind, s)) return rc;

@@ -30,6 +30,7 @@ struct MoeArgs {
     const float* logits;
     float* x;
     const float* factors;   // few rows: factors of the rows of h that are still to be applied (NormBehind), or null
+    int picked;             // rows by pick_rows_kernel: a pair's row of the products is its number, slot_of is not used
     const float* norm;      // h null (one row): the norm of x that gives it, with its true width and eps
     int dim;
     float eps;
@@ -392,6 +393,63 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(MoeArgs a) {
         }
 }
 
+// ---- few rows, no sorting ----------------------------------------------------------------------------------
+// Up to 32 rows over up to 64 experts, behind a norm that is shared out between two products (NormBehind): logits and picks of a row in one launch, a workgroup per
+// row and its waves the experts in turn.  A pair's row of the grouped products is its own number, and their units find the rows of their expert in the list of
+// picks themselves (expert_rows_kernel, PICKED), so that nothing is sorted.  Bound by a workgroup's own read of the router (330 KB out of the L2 at width 2048); us at 20
+// rows of width 2048, router product and sorting / this: 6.4 + 8.6 / 9.0; finding their rows costs the products 0.6 to 0.9 (59.0 -> 59.6, 28.1 -> 29.0).
+template <int NC>
+__global__ __launch_bounds__(1024) void pick_rows_kernel(MoeArgs a, const bf16* __restrict__ router, NormBehind b, float* __restrict__ logits, float* __restrict__ factors) {
+    __shared__ float logit[80];
+    const int m = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, pieces = a.ld / 8, rows = a.experts + (a.shared_up ? 1 : 0);
+    float squares[kNormParts / 64];
+#pragma unroll
+    for (int i = 0; i < kNormParts / 64; ++i) squares[i] = b.squares[m * norm_pitch(b.parts) + min(lane + 64 * i, b.parts - 1)];
+    Chunk<bf16> x[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) x[c] = lane + 64 * c < pieces ? load_chunk(static_cast<const bf16*>(a.h) + (int64_t)m * a.ld + 8 * (lane + 64 * c)) : zero_chunk<bf16>();
+    constexpr int R = 3;  // expert rows requested together
+    float inv = 0.f;
+#pragma unroll
+    for (int e0 = 0; e0 < 5; e0 += R) {
+        Chunk<bf16> w[R][NC];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                w[r][c] = load_chunk(router + (int64_t)min(wave + 16 * (e0 + r), rows - 1) * a.ld + 8 * min(lane + 64 * c, pieces - 1));
+        if (e0 == 0) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < kNormParts / 64; ++i) sum += lane + 64 * i < b.parts ? squares[i] : 0.f;
+            inv = 1.0f / sqrtf(wave_sum(sum) / (float)b.dim + b.eps);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int e = wave + 16 * (e0 + r);
+            if (e >= rows) continue;
+            float s = 0.f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) s = dot_chunk(w[r][c], x[c], s);
+            s = wave_sum(s) * inv;
+            if (lane == 0) {
+                logit[e] = s;
+                logits[(int64_t)m * a.ldl + e] = s;
+            }
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    int e;
+    float s;
+    pick_experts(logit, a.experts, a.top, e, s);
+    if (lane < a.top) {
+        a.pick[m * a.top + lane] = e;
+        a.pick_scale[m * a.top + lane] = s * inv;
+    }
+    if (lane == 0) factors[m] = inv;
+}
+
 // ------------------------------------------------------------------------------------------------
 // The grouped products of experts with at most 16 rows a tile: y[r] = x[x_row[r]] W_g^T.  One unit -- a tile's rows against 32 weight rows (up: 16 gate and 16 up
 // rows) -- per workgroup of four waves that take the K steps in turn and never wait for each other; a wave's weight rows come as
@@ -411,20 +469,101 @@ struct FewArgs {
     void* y;               // [rows, N]
     int N, K, tiles_n, out_f32;
     RowGroups g;
+    // PICKED: rows by their picks
+    const int* pick;       // [M * top]
+    const float* factors;  // UP: of the shared expert's rows
+    int M, top, experts;
 };
+constexpr int kPickedRows = 32;  // tokens
+
+// or of all lanes, by moves inside a row of 16 and four scalar reads (an exchange through the LDS costs 0.05 us a step)
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+    auto row = [](unsigned x, auto ctrl) { return x | (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
+    v = row(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+    v = row(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    v = row(v, std::integral_constant<int, 0x124>{});  // row_ror 4
+    v = row(v, std::integral_constant<int, 0x128>{});  // row_ror 8
+    return (unsigned)(__builtin_amdgcn_readlane((int)v, 0) | __builtin_amdgcn_readlane((int)v, 16) | __builtin_amdgcn_readlane((int)v, 32) | __builtin_amdgcn_readlane((int)v, 48));
+}
+
+// PICKED: the rows of unit group `which`, in LDS: row of x, row of the product and factor of each; the experts that rows pick come first, in their order, then tiles of
+// 16 rows of the shared expert.  Returns their number, 0 behind the last group; *group: the expert, `experts` for the shared one
+constexpr int kHeldPicks = 4;  // pieces of 64 picks that a lane keeps
+template <bool UP>
+__device__ __forceinline__ int picked_rows(const FewArgs& a, int which, int* group, int* x_row, int* y_row, float* scale) {
+    const int lane = threadIdx.x & 63, pairs = a.M * a.top;
+    unsigned low = 0, high = 0;
+    int held[kHeldPicks];
+    for (int p0 = 0; p0 < pairs; p0 += 64 * kHeldPicks) {
+        int e[kHeldPicks];
+#pragma unroll
+        for (int c = 0; c < kHeldPicks; ++c) e[c] = a.pick[min(p0 + 64 * c + lane, pairs - 1)];
+#pragma unroll
+        for (int c = 0; c < kHeldPicks; ++c) {
+            const unsigned bit = 1u << (e[c] & 31);
+            if (e[c] < 32) low |= bit;
+            else high |= bit;
+            if (p0 == 0) held[c] = e[c];
+        }
+    }
+    const unsigned long long mask = ((unsigned long long)wave_or(high) << 32) | wave_or(low);
+    const int touched = __popcll(mask);
+    if (which >= touched) {
+        const int first = (which - touched) * 16, n = a.g.extra_group < 0 ? 0 : min(a.M - first, 16);
+        *group = a.experts;
+        if (n > 0 && threadIdx.x < (unsigned)n) {
+            x_row[threadIdx.x] = UP ? first + (int)threadIdx.x : pairs + first + (int)threadIdx.x;
+            y_row[threadIdx.x] = pairs + first + threadIdx.x;
+            if (UP) scale[threadIdx.x] = a.factors[first + threadIdx.x];
+        }
+        return max(n, 0);
+    }
+    const bool is_it = (mask >> lane) & 1 && __popcll(mask & ((1ull << lane) - 1)) == which;
+    const int g = __builtin_ctzll(__ballot(is_it));
+    *group = g;
+    int n = 0;
+    auto take = [&](int p0, int e) {
+        const int p = p0 + lane;
+        const bool own = p < pairs && e == g;
+        const unsigned long long found = __ballot(own);
+        if (own && threadIdx.x < 64) {
+            const int at = n + __popcll(found & ((1ull << lane) - 1));
+            x_row[at] = UP ? p / a.top : p;
+            y_row[at] = p;
+            if (UP) scale[at] = a.g.x_scale[p];
+        }
+        n += __popcll(found);
+    };
+#pragma unroll
+    for (int c = 0; c < kHeldPicks; ++c)
+        if (64 * c < pairs) take(64 * c, held[c]);
+    for (int p0 = 64 * kHeldPicks; p0 < pairs; p0 += 64) take(p0, a.pick[min(p0 + lane, pairs - 1)]);
+    return n;
+}
 
 constexpr int few_columns(bool up) { return up ? 16 : 32; }  // output columns of a unit
 
-template <bool UP>
+// PICKED: see picked_rows
+template <bool UP, bool PICKED = false>
 __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
     constexpr int KM = UP ? 128 : 64, NT = 2, COLS = few_columns(UP), NG = COLS / 16;  // a K step, tiles of 16 weight rows, of output columns
     constexpr int PITCH = KM + 8, LPR = KM / 8, RPI = 64 / LPR, IPT = 16 / RPI;   // lanes per row, rows per load, loads per tile
     __shared__ __align__(16) bf16 stage[4][16 * (NT + 1)][PITCH];
     static_assert(sizeof(stage) >= 3 * NT * 64 * 16, "the tiles double as the waves' sums");
-    const int tile = (int)blockIdx.x / a.tiles_n, at = (int)blockIdx.x - tile * a.tiles_n, used = *a.g.used;
+    __shared__ int x_rows[PICKED ? kPickedRows : 1], y_rows[PICKED ? kPickedRows : 1];
+    __shared__ float scales[PICKED && UP ? kPickedRows : 1];
+    const int tile = (int)blockIdx.x / a.tiles_n, at = (int)blockIdx.x - tile * a.tiles_n;
     const int n0 = (at + (tile * a.tiles_n) % 8) % a.tiles_n * COLS;
-    if (tile >= used) return;
-    const int g = a.g.group_of[tile], row0 = a.g.group_row[tile], rows = a.g.group_end[tile] - row0;
+    int g, row0 = 0, all, used = 0;
+    if constexpr (PICKED) {
+        all = picked_rows<UP>(a, tile, &g, x_rows, y_rows, scales);
+        if (all == 0) return;
+        __syncthreads();
+    } else {
+        used = *a.g.used;
+        if (tile >= used) return;
+        g = a.g.group_of[tile], row0 = a.g.group_row[tile], all = a.g.group_end[tile] - row0;
+    }
     const bf16* W = g == a.g.extra_group ? a.g.w_extra : a.w + g * a.g.w_stride;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ln = lane & 15, kq = lane >> 4;
     const int lr = lane / LPR, lc = (lane % LPR) * 8, K = a.K;
@@ -432,23 +571,21 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
     const int n_steps = (K + KM - 1) / KM, mine = (n_steps - wave + 3) / 4;
 
     f32x4 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     // element offsets of this lane's rows: weight rows past N repeat the last one, token rows past the tile's likewise (neither is stored)
     unsigned wo[NT][IPT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < IPT; ++i) wo[t][i] = (unsigned)(min(n0 + (t % NG) * 16 + RPI * i + lr, a.N - 1) + (UP && t >= NG ? a.N : 0)) * (unsigned)K;
-    // XI: load instructions that the tile's token rows need.  ONCE: no other tile reads these weights
-    auto run = [&](auto xi_tag, auto once_tag) __attribute__((always_inline)) {
+    // XI: load instructions that the token rows from `first` on need.  ONCE: no other tile reads these weights
+    auto run = [&](int first, int rows, auto xi_tag, auto once_tag) __attribute__((always_inline)) {
         constexpr int XI = decltype(xi_tag)::value;
         constexpr bool ONCE = decltype(once_tag)::value;
         const bf16* xp[XI];
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
-            const int r = row0 + min(RPI * i + lr, rows - 1);
-            xp[i] = a.x + (int64_t)(a.g.x_row ? a.g.x_row[r] : r) * K;
+            const int r = row0 + first + min(RPI * i + lr, rows - 1);
+            xp[i] = a.x + (int64_t)(PICKED ? x_rows[r] : a.g.x_row ? a.g.x_row[r] : r) * K;
         }
         struct Staged {
             u32x4 w[NT][IPT], x[XI];
@@ -507,51 +644,80 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(FewArgs a) {
         wave_sync();
         multiply();
     };
-    const int before = a.g.group_of[max(tile - 1, 0)], after = a.g.group_of[min(tile + 1, used - 1)];
-    const bool alone = (tile == 0 || before != g) && (tile + 1 == used || after != g);
-    if (!alone) run(std::integral_constant<int, IPT>{}, std::false_type{});
-    else if (rows <= RPI) run(std::integral_constant<int, 1>{}, std::true_type{});
-    else run(std::integral_constant<int, IPT>{}, std::true_type{});
-
-    __syncthreads();
-    f32x4(*sums)[NT][64] = reinterpret_cast<f32x4(*)[NT][64]>(&stage[0][0][0]);
-    if (wave > 0) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) sums[wave - 1][t][lane] = acc[t];
+    bool alone;
+    if constexpr (PICKED) {
+        alone = all <= 16 && (g != a.experts || a.M <= 16);
+    } else {
+        const int before = a.g.group_of[max(tile - 1, 0)], after = a.g.group_of[min(tile + 1, used - 1)];
+        alone = (tile == 0 || before != g) && (tile + 1 == used || after != g);
     }
-    __syncthreads();
-    if (wave != 0 || ln >= rows) return;
+    for (int first = 0; first < all; first += 16) {  // (a second round only of a picked expert with more than 16 rows)
+        const int rows = min(16, all - first);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] += sums[0][t][lane] + sums[1][t][lane] + sums[2][t][lane];
-    // a lane holds columns 4 kq ..+3 of each tile for token row ln
-    const float xs = UP ? a.g.x_scale[row0 + ln] : 1.f;
+        for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!alone) run(first, rows, std::integral_constant<int, IPT>{}, std::false_type{});
+        else if (rows <= RPI) run(first, rows, std::integral_constant<int, 1>{}, std::true_type{});
+        else run(first, rows, std::integral_constant<int, IPT>{}, std::true_type{});
+
+        __syncthreads();
+        f32x4(*sums)[NT][64] = reinterpret_cast<f32x4(*)[NT][64]>(&stage[0][0][0]);
+        if (wave > 0) {
 #pragma unroll
-    for (int t = 0; t < NG; ++t) {
-        const int n = n0 + 16 * t + 4 * kq;
-        if (n >= a.N) continue;
-        const int64_t at = (int64_t)(row0 + ln) * a.N + n;
-        f32x4 v = acc[t];
-        if (UP) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = silu_f32(v[i] * xs) * (acc[UP ? t + 1 : t][i] * xs);
+            for (int t = 0; t < NT; ++t) sums[wave - 1][t][lane] = acc[t];
         }
-        if (a.out_f32) {
-            store4(static_cast<float*>(a.y) + at, v);
-        } else {
-            store4(static_cast<bf16*>(a.y) + at, v);
+        __syncthreads();
+        if (wave == 0 && ln < rows) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t] += sums[0][t][lane] + sums[1][t][lane] + sums[2][t][lane];
+            // a lane holds columns 4 kq ..+3 of each tile for token row ln
+            const int r = row0 + first + ln;
+            const float xs = UP ? (PICKED ? scales[r] : a.g.x_scale[r]) : 1.f;
+#pragma unroll
+            for (int t = 0; t < NG; ++t) {
+                const int n = n0 + 16 * t + 4 * kq;
+                if (n >= a.N) continue;
+                const int64_t to = (int64_t)(PICKED ? y_rows[r] : r) * a.N + n;
+                f32x4 v = acc[t];
+                if (UP) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = silu_f32(v[i] * xs) * (acc[UP ? t + 1 : t][i] * xs);
+                }
+                if (a.out_f32) {
+                    store4(static_cast<float*>(a.y) + to, v);
+                } else {
+                    store4(static_cast<bf16*>(a.y) + to, v);
+                }
+            }
         }
+        if (!PICKED || first + 16 >= all) return;
+        __syncthreads();  // the sums have been read
     }
 }
 
 static int expert_rows(const void* x, const void* w, void* y, int N, int K, bool up, int out_f32, const RowGroups& g, hipStream_t s) {
     RAVEN_REQUIRE(g.n_tiles > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && (!up || g.x_scale), "moe: bad experts");
-    FewArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(w), y, N, K, 0, out_f32, g};
+    FewArgs a{};
+    a.x = static_cast<const bf16*>(x); a.w = static_cast<const bf16*>(w); a.y = y; a.N = N; a.K = K; a.out_f32 = out_f32; a.g = g;
     a.tiles_n = (N + few_columns(up) - 1) / few_columns(up);
     const int64_t units = (int64_t)a.tiles_n * g.n_tiles;
     RAVEN_REQUIRE(units < (1ll << 31), "moe: too many units");
     if (up) expert_rows_kernel<true><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
     else expert_rows_kernel<false><<<dim3((unsigned)units), dim3(256), 0, s>>>(a);
     return raven_host::check_launch("moe (rows of an expert)");
+}
+
+// The same over picks: g gives the matrices and, up, the factors of the pairs
+static int picked_expert_rows(const void* x, const void* w, void* y, int N, int K, bool up, const RowGroups& g, const MoeArgs& m, hipStream_t s) {
+    RAVEN_REQUIRE(m.M > 0 && m.M <= kPickedRows && m.experts <= 64 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && m.pick && m.factors &&
+                      (!up || g.x_scale) && (g.extra_group < 0 || (g.extra_group == m.experts && g.w_extra)), "moe: bad picked experts");
+    FewArgs a{};
+    a.x = static_cast<const bf16*>(x); a.w = static_cast<const bf16*>(w); a.y = y; a.N = N; a.K = K; a.out_f32 = up ? 0 : 1; a.g = g;
+    a.pick = m.pick; a.factors = m.factors; a.M = m.M; a.top = m.top; a.experts = m.experts;
+    a.tiles_n = (N + few_columns(up) - 1) / few_columns(up);
+    const int64_t groups = std::min(m.experts, m.M * m.top) + (g.extra_group >= 0 ? (m.M + 15) / 16 : 0);
+    if (up) expert_rows_kernel<true, true><<<dim3((unsigned)(groups * a.tiles_n)), dim3(256), 0, s>>>(a);
+    else expert_rows_kernel<false, true><<<dim3((unsigned)(groups * a.tiles_n)), dim3(256), 0, s>>>(a);
+    return raven_host::check_launch("moe (rows of a picked expert)");
 }
 
 template <typename Y>
@@ -567,7 +733,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     for (int k0 = 0; k0 < a.top; k0 += 8) {
         f32x4 v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)a.slot_of[m * a.top + min(k0 + k, a.top - 1)] * a.ld + c);
+        for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)(a.picked ? m * a.top + min(k0 + k, a.top - 1) : a.slot_of[m * a.top + min(k0 + k, a.top - 1)]) * a.ld + c);
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (k0 + k < a.top) x += v[k];
@@ -603,7 +769,7 @@ __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeAr
         for (int k0 = 0; k0 < a.top; k0 += 8) {
             f32x4 v[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)a.slot_of[m * a.top + min(k0 + k, a.top - 1)] * a.ld + c);
+            for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)(a.picked ? m * a.top + min(k0 + k, a.top - 1) : a.slot_of[m * a.top + min(k0 + k, a.top - 1)]) * a.ld + c);
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 if (k0 + k < a.top) x[j] += v[k];
@@ -773,6 +939,46 @@ extern "C" size_t raven_moe_workspace_bytes(const raven_moe* m, int32_t M, int32
 }
 
 namespace raven {
+// Rows behind a norm that is shared out between two products, which route themselves (moe_forward_picked)
+bool moe_picks_itself(const raven_moe* m, const void* h, int M, int ld, int dtype) {
+    return moe_path(m, h, M, ld, dtype) == kMoeFew && M <= kPickedRows && m->experts <= 64 && ld <= 16 * kNormParts && ld % 16 == 0 && raven_host::aligned16(m->router);
+}
+// Router, experts and sums of M rows: xw and behind as NormAhead left them; logits and factors are written.  next_norm, next_h: as for moe_forward
+int moe_forward_picked(const raven_moe* m, const void* xw, const NormBehind& behind, float* factors, float* logits, float* x, int M, int ld, float eps, int dim, void* workspace,
+                       size_t workspace_bytes, hipStream_t s, const float* next_norm, void* next_h) {
+    if (const int rc = check_moe("moe", m, M, ld, RAVEN_BF16)) return rc;
+    RAVEN_REQUIRE(m->up && m->down && m->router && xw && behind.squares && behind.parts > 0 && behind.parts <= kNormParts && factors && logits && x &&
+                      moe_picks_itself(m, xw, M, ld, RAVEN_BF16), "moe: %d rows don't pick for themselves", M);
+    RAVEN_REQUIRE(!next_norm || (next_h && dim > 0 && ld <= 16 * kCombineThreads), "moe: no norm behind %d rows", M);
+    RAVEN_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0 && carve_moe(m, M, ld, RAVEN_BF16, kMoeFew, nullptr, nullptr) <= workspace_bytes,
+                  "moe: workspace of %zu bytes is too small or unaligned", workspace_bytes);
+    MoeChunk c;
+    carve_moe(m, M, ld, RAVEN_BF16, kMoeFew, static_cast<char*>(workspace), &c);
+    const bool fold = m->shared_up != nullptr;
+    MoeArgs a{};
+    a.h = xw; a.up = m->up; a.down = m->down; a.shared_up = m->shared_up; a.shared_down = m->shared_down;
+    a.logits = logits; a.x = x; a.factors = factors; a.pick = c.pick; a.pick_scale = c.pick_scale; a.picked = 1;
+    a.M = M; a.ld = ld; a.ldl = m->logit_ld; a.experts = m->experts; a.top = m->top; a.ff = m->ff; a.sff = m->shared_ff;
+    a.y = c.y; a.ys = c.ys; a.fold = fold;
+    const bf16* router = static_cast<const bf16*>(m->router);
+    switch ((ld / 8 + 63) / 64) {
+        case 1: pick_rows_kernel<1><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+        case 2: pick_rows_kernel<2><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+        case 3: pick_rows_kernel<3><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+        case 4: pick_rows_kernel<4><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+        case 5: pick_rows_kernel<5><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+        default: pick_rows_kernel<6><<<dim3(M), dim3(1024), 0, s>>>(a, router, behind, logits, factors); break;
+    }
+    if (const int rc = raven_host::check_launch("moe (router, picks)")) return rc;
+    RowGroups g{};
+    g.x_scale = c.pick_scale; g.w_stride = (int64_t)2 * m->ff * ld; g.w_extra = static_cast<const bf16*>(m->shared_up); g.extra_group = fold ? m->experts : -1;
+    if (const int rc = picked_expert_rows(xw, m->up, c.act, m->ff, ld, true, g, a, s)) return rc;
+    g.w_stride = (int64_t)ld * m->ff; g.w_extra = static_cast<const bf16*>(m->shared_down);
+    if (const int rc = picked_expert_rows(c.act, m->down, c.y, ld, m->ff, false, g, a, s)) return rc;
+    if (next_norm) return launch_combine_norm<float>(a, NextNorm{next_norm, next_h, dim, eps}, s);
+    moe_combine_kernel<float><<<dim3((unsigned)(((int64_t)M * (ld / 4) + 255) / 256)), dim3(256), 0, s>>>(a);
+    return raven_host::check_launch("moe (combine)");
+}
 // Whether moe_forward applies rows' factors of its own for so many rows
 bool moe_norms_behind(const raven_moe* m, const void* h, int M, int ld, int dtype) {  // ... and whether it can end with the norm that the next layer begins with
     return moe_path(m, h, M, ld, dtype) != kMoeRows && ld <= 16 * kCombineThreads;

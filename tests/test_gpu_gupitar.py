@@ -651,6 +651,30 @@ def test_norm_between_the_output_product_and_a_mixture(pkg, width, M, shared):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
 
 
+@pytest.mark.parametrize("shared", [264, None])
+@pytest.mark.parametrize("M", [3, 16, 17, 32])
+@pytest.mark.parametrize("width,E,top", [(512, 64, 6), (992, 40, 2), (1536, 64, 1)])
+def test_rows_that_route_themselves(pkg, width, E, top, M, shared):
+    """Batches whose picks no launch sorts: equal sequences, of which every expert picked gets all rows (more than a tile of 16 of them as well), give equal rows, and those of
+    one sequence by itself; different ones the oracle's but for close calls."""
+    if M > 8 and M * top >= 2 * E:
+        pytest.skip("a chunk")
+    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(E, top, 264, shared))])
+    w = O.random_weights(cfg, 3)
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    for same in (True, False):
+        ids = torch.stack([G.tokens(cfg, 2, seed=1 if same else s) for s in range(M)])
+        cache = model.new_cache()
+        got = torch.cat([model.forward(ids[:, t:t + 1], past_key_values=cache).logits for t in range(2)], 1)
+        want = [O.forward(cfg, w, ids[b])[0] for b in range(1 if same else M)]
+        err = torch.stack([G.rows(got[b], want[min(b, len(want) - 1)]) for b in range(M)])
+        if same:
+            assert all(torch.equal(got[b], got[0]) for b in range(M)) and err.max() < 6e-2
+        else:
+            assert err.median() < 2e-2 and err.quantile(0.8) < 6e-2
+
+
 @pytest.mark.parametrize("B,S", [(4, 1), (40, 1), (3, 70)])
 @pytest.mark.parametrize("width", [512, 2056, 4104])
 def test_mixture_ends_with_the_norm_of_the_next_layer(pkg, width, B, S):
