@@ -30,7 +30,6 @@ struct MoeArgs {
     const float* logits;
     float* x;
     const float* factors;   // few rows: factors of the rows of h that are still to be applied (NormBehind), or null
-    int picked;             // rows by pick_rows_kernel: a pair's row of the products is its number, slot_of is not used
     const float* norm;      // h null (one row): the norm of x that gives it, with its true width and eps
     int dim;
     float eps;
@@ -720,7 +719,13 @@ static int picked_expert_rows(const void* x, const void* w, void* y, int N, int 
     return raven_host::check_launch("moe (rows of a picked expert)");
 }
 
-template <typename Y>
+// Row of the products that a token's k-th pair has.  (Known at compile time which: decided per load, the loads of a token waited for each other, 32 of them 5.3 -> 11.9 us.)
+template <bool PICKED>
+__device__ __forceinline__ int64_t pair_row(const MoeArgs& a, int m, int k) {
+    const int i = m * a.top + min(k, a.top - 1);
+    return PICKED ? i : a.slot_of[i];
+}
+template <typename Y, bool PICKED>
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int per = a.ld / 4;
@@ -733,7 +738,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     for (int k0 = 0; k0 < a.top; k0 += 8) {
         f32x4 v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)(a.picked ? m * a.top + min(k0 + k, a.top - 1) : a.slot_of[m * a.top + min(k0 + k, a.top - 1)]) * a.ld + c);
+        for (int k = 0; k < 8; ++k) v[k] = load4(y + pair_row<PICKED>(a, m, k0 + k) * a.ld + c);
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (k0 + k < a.top) x += v[k];
@@ -751,7 +756,7 @@ struct NextNorm {
     int dim;
     float eps;
 };
-template <typename Y, int P>
+template <typename Y, int P, bool PICKED>
 __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeArgs a, NextNorm next) {
     __shared__ float red[kCombineThreads / 64];
     const int m = blockIdx.x, tid = threadIdx.x, per = a.ld / 4;
@@ -769,7 +774,7 @@ __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeAr
         for (int k0 = 0; k0 < a.top; k0 += 8) {
             f32x4 v[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = load4(y + (int64_t)(a.picked ? m * a.top + min(k0 + k, a.top - 1) : a.slot_of[m * a.top + min(k0 + k, a.top - 1)]) * a.ld + c);
+            for (int k = 0; k < 8; ++k) v[k] = load4(y + pair_row<PICKED>(a, m, k0 + k) * a.ld + c);
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 if (k0 + k < a.top) x[j] += v[k];
@@ -791,12 +796,12 @@ __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeAr
     for (int j = 0; j < P; ++j)
         if (tid + kCombineThreads * j < per) store4(static_cast<bf16*>(next.h) + (int64_t)m * a.ld + 4 * (tid + kCombineThreads * j), x[j] * inv * w[j]);
 }
-template <typename Y>
+template <typename Y, bool PICKED>
 static int launch_combine_norm(const MoeArgs& a, const NextNorm& next, hipStream_t s) {
     const int p = (a.ld / 4 + kCombineThreads - 1) / kCombineThreads;
-    if (p <= 1) moe_combine_norm_kernel<Y, 1><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
-    else if (p <= 2) moe_combine_norm_kernel<Y, 2><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
-    else moe_combine_norm_kernel<Y, 4><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
+    if (p <= 1) moe_combine_norm_kernel<Y, 1, PICKED><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
+    else if (p <= 2) moe_combine_norm_kernel<Y, 2, PICKED><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
+    else moe_combine_norm_kernel<Y, 4, PICKED><<<dim3(a.M), dim3(kCombineThreads), 0, s>>>(a, next);
     return raven_host::check_launch("moe (combine, norm)");
 }
 
@@ -957,7 +962,7 @@ int moe_forward_picked(const raven_moe* m, const void* xw, const NormBehind& beh
     const bool fold = m->shared_up != nullptr;
     MoeArgs a{};
     a.h = xw; a.up = m->up; a.down = m->down; a.shared_up = m->shared_up; a.shared_down = m->shared_down;
-    a.logits = logits; a.x = x; a.factors = factors; a.pick = c.pick; a.pick_scale = c.pick_scale; a.picked = 1;
+    a.logits = logits; a.x = x; a.factors = factors; a.pick = c.pick; a.pick_scale = c.pick_scale;
     a.M = M; a.ld = ld; a.ldl = m->logit_ld; a.experts = m->experts; a.top = m->top; a.ff = m->ff; a.sff = m->shared_ff;
     a.y = c.y; a.ys = c.ys; a.fold = fold;
     const bf16* router = static_cast<const bf16*>(m->router);
@@ -975,8 +980,8 @@ int moe_forward_picked(const raven_moe* m, const void* xw, const NormBehind& beh
     if (const int rc = picked_expert_rows(xw, m->up, c.act, m->ff, ld, true, g, a, s)) return rc;
     g.w_stride = (int64_t)ld * m->ff; g.w_extra = static_cast<const bf16*>(m->shared_down);
     if (const int rc = picked_expert_rows(c.act, m->down, c.y, ld, m->ff, false, g, a, s)) return rc;
-    if (next_norm) return launch_combine_norm<float>(a, NextNorm{next_norm, next_h, dim, eps}, s);
-    moe_combine_kernel<float><<<dim3((unsigned)(((int64_t)M * (ld / 4) + 255) / 256)), dim3(256), 0, s>>>(a);
+    if (next_norm) return launch_combine_norm<float, true>(a, NextNorm{next_norm, next_h, dim, eps}, s);
+    moe_combine_kernel<float, true><<<dim3((unsigned)(((int64_t)M * (ld / 4) + 255) / 256)), dim3(256), 0, s>>>(a);
     return raven_host::check_launch("moe (combine)");
 }
 // Whether moe_forward applies rows' factors of its own for so many rows
@@ -1043,11 +1048,11 @@ int moe_forward(const raven_moe* m, const void* h, const float* factors, const f
     }
     if (next_norm) {
         const NextNorm next{next_norm, next_h, dim, eps};
-        return few ? launch_combine_norm<float>(a, next, s) : launch_combine_norm<bf16>(a, next, s);
+        return few ? launch_combine_norm<float, false>(a, next, s) : launch_combine_norm<bf16, false>(a, next, s);
     }
     const dim3 grid((unsigned)(((int64_t)M * (ld / 4) + 255) / 256));
-    if (few) moe_combine_kernel<float><<<grid, dim3(256), 0, s>>>(a);
-    else moe_combine_kernel<bf16><<<grid, dim3(256), 0, s>>>(a);
+    if (few) moe_combine_kernel<float, false><<<grid, dim3(256), 0, s>>>(a);
+    else moe_combine_kernel<bf16, false><<<grid, dim3(256), 0, s>>>(a);
     return raven_host::check_launch("moe (combine)");
 }
 }  // namespace raven
