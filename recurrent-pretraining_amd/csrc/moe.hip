@@ -62,7 +62,7 @@ __device__ __forceinline__ int ordered_key(float v) {
 // maxima (both launches of 8 rows of width 512, one of 8 experts of 512: 12.0 us, by counting 13.4).
 // (U steps unrolled.  In a workgroup alone on its CU all 64 are 2.5 KB of code run once out of a cold instruction cache: routing of 20 rows 9.7 us, with 16
 // 8.8; where thousands of workgroups run it, all: one row of 7 x 384 channels of width 1024, both launches 9.6, with 16 10.1.)
-__device__ __forceinline__ bool picks_by_place(int experts, int top) { return experts <= 64 && top > 2; }
+__host__ __device__ __forceinline__ bool picks_by_place(int experts, int top) { return experts <= 64 && top > 2; }
 template <int U>
 __device__ __forceinline__ void pick_by_place(float v, int experts, int& mine, float& score) {  // v: expert `lane`'s logit
     const int lane = threadIdx.x & 63;
@@ -79,9 +79,8 @@ __device__ __forceinline__ void pick_by_place(float v, int experts, int& mine, f
     mine = min(mine, experts - 1);
     score = sigmoid_f32(s);
 }
-__device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
+__device__ __forceinline__ void pick_by_maxima(const float* logits, int experts, int top, int& mine, float& score) {
     const int lane = threadIdx.x & 63;
-    if (picks_by_place(experts, top)) return pick_by_place<64>(lane < experts ? logits[lane] : 0.f, experts, mine, score);
     float v[kMaxExperts / 64];
 #pragma unroll
     for (int j = 0; j < kMaxExperts / 64; ++j) {
@@ -114,6 +113,11 @@ __device__ __forceinline__ void pick_experts(const float* logits, int experts, i
     }
     score = sigmoid_f32(logit);
 }
+__device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
+    const int lane = threadIdx.x & 63;
+    if (picks_by_place(experts, top)) pick_by_place<64>(lane < experts ? logits[lane] : 0.f, experts, mine, score);
+    else pick_by_maxima(logits, experts, top, mine, score);
+}
 
 // ---- few rows --------------------------------------------------------------------------------------------
 // A wave per (gate, up) row pair, over the concatenation of the row's experts and the shared one
@@ -131,7 +135,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(MoeArgs a) {
     if (wave == 0) {
         int e;
         float s;
-        pick_experts(a.logits + (int64_t)m * a.ldl, a.experts, a.top, e, s);
+        pick_by_maxima(a.logits + (int64_t)m * a.ldl, a.experts, a.top, e, s);
         if (lane < a.top) {
             idx[lane] = e;
             score[lane] = s;
@@ -185,32 +189,124 @@ __global__ __launch_bounds__(256) void moe_up_kernel(MoeArgs a) {
     static_cast<T*>(a.act)[(int64_t)m * total + p] = from_f32<T>(v);
 }
 
-// a wave per output channel: its row of every chosen down matrix and of the shared one, as one long row
+// The same where experts are picked by place, with nothing waited for twice: logits, row and norm weights are requested together, each wave counts a quarter of every
+// expert's place (one wave counting all of it held up its SIMD, where the first waves of a CU's five workgroups meet), and a wave knows its own expert right behind the first
+// barrier, so that its weights are on their way before the row is normed.  Bound by latencies in front of the weights: 44 MB (one row, 7 x 768 channels of width 2048)
+// 13.4 -> 10.9 us, 6.9 of them at the rate of HBM.
 template <typename T>
+__global__ __launch_bounds__(256) void moe_up_place_kernel(MoeArgs a) {
+    constexpr int E = Chunk<T>::N, U = 4, H = 2;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);  // [ld]
+    __shared__ int place[4][64];
+    __shared__ float red[4];
+    const int m = blockIdx.y, nc = a.ld / E, total = a.top * a.ff + a.sff, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float* logits = a.logits + (int64_t)m * a.ldl;
+    const float* x = a.x + (int64_t)m * a.ld;
+    const float logit = logits[min(lane, a.experts - 1)];
+    f32x4 xv[H], nv[H];
+    if (a.h) {
+        for (int i = tid; i < nc; i += 256) store_chunk(xs + i * E, load_chunk(static_cast<const T*>(a.h) + (int64_t)m * a.ld + i * E));
+    } else {
+#pragma unroll
+        for (int j = 0; j < H; ++j) xv[j] = load4(x + min(4 * tid + 1024 * j, a.ld - 4));
+#pragma unroll
+        for (int j = 0; j < H; ++j) nv[j] = load4(a.norm + min(4 * tid + 1024 * j, a.ld - 4));
+    }
+    const int key = lane < a.experts ? ordered_key(logit) : (int)0x80000000;
+    int before = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int at = 16 * wave + j, other = __builtin_amdgcn_readlane(key, at);
+        before += other > key || (other == key && at < lane) ? 1 : 0;
+    }
+    place[wave][lane] = before;
+    if (!a.h) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < H; ++j)
+            if (4 * tid + 1024 * j < a.ld) ss += xv[j][0] * xv[j][0] + xv[j][1] * xv[j][1] + xv[j][2] * xv[j][2] + xv[j][3] * xv[j][3];
+        for (int i = 4 * tid + 1024 * H; i < a.ld; i += 1024) {
+            const f32x4 v = load4(x + i);
+            ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+    }
+    __syncthreads();
+    before = place[0][lane] + place[1][lane] + place[2][lane] + place[3][lane];
+    if (blockIdx.x == 0 && wave == 0 && before < a.top) a.pick[(int64_t)m * a.top + before] = lane;
+    const int own = blockIdx.x * 4 + wave, p = min(own, total - 1);
+    const bool shared = p >= a.top * a.ff;
+    const int slot = shared ? 0 : p / a.ff, r = shared ? p - a.top * a.ff : p - slot * a.ff;
+    const int expert = __builtin_ctzll(__ballot(before == slot));  // (every lane has a place of its own)
+    const T* g = shared ? static_cast<const T*>(a.shared_up) + (int64_t)r * a.ld : static_cast<const T*>(a.up) + ((int64_t)expert * 2 * a.ff + r) * a.ld;
+    const T* u = g + (int64_t)(shared ? a.sff : a.ff) * a.ld;
+    Chunk<T> vg[U], vu[U];
+    auto request = [&](int c0) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const int c = min(c0 + 64 * j, nc - 1);
+            vg[j] = load_chunk_stream(g + c * E);
+            vu[j] = load_chunk_stream(u + c * E);
+        }
+    };
+    request(lane);
+    const float gate = shared ? logits[a.experts] : __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, logit), expert));
+    if (!a.h) {
+        const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)a.dim + a.eps);
+#pragma unroll
+        for (int j = 0; j < H; ++j)
+            if (4 * tid + 1024 * j < a.ld) store4(xs + 4 * tid + 1024 * j, xv[j] * inv * nv[j]);
+        for (int i = 4 * tid + 1024 * H; i < a.ld; i += 1024) store4(xs + i, load4(x + i) * inv * load4(a.norm + i));
+        __syncthreads();
+    }
+    float sg = 0.f, su = 0.f;
+    for (int c0 = lane;;) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            if (c0 + 64 * j >= nc) break;
+            const Chunk<T> v = load_chunk(xs + (c0 + 64 * j) * E);
+            sg = dot_chunk(vg[j], v, sg);
+            su = dot_chunk(vu[j], v, su);
+        }
+        c0 += 64 * U;
+        if (c0 - lane >= nc) break;
+        request(c0);
+    }
+    sg = wave_sum(sg);
+    su = wave_sum(su);
+    if (lane != 0 || own >= total) return;
+    const float s = shared ? 1.f : sigmoid_f32(gate == gate ? gate : -INFINITY);
+    float v = silu_f32(s * sg) * (s * su);
+    if (shared) v *= sigmoid_f32(gate);
+    static_cast<T*>(a.act)[(int64_t)m * total + p] = from_f32<T>(v);
+}
+
+// a wave per output channel: its row of every chosen down matrix and of the shared one, as one long row, U pieces of 64 chunks at a time (up to 12: all at once).
+// The picks are requested first and handed out by lane exchange, so that the weights wait for one round trip: 22 MB 7.4 -> 6.7 us (with six pieces at a time and a
+// load of the pick in front of each).
+template <typename T, int U>
 __global__ __launch_bounds__(256) void moe_down_kernel(MoeArgs a) {
-    constexpr int E = Chunk<T>::N, U = 6;
+    constexpr int E = Chunk<T>::N;
     const int m = blockIdx.y, n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (n >= a.ld) return;
-    const int* pick = a.pick + (int64_t)m * a.top;
+    const int pick = a.pick[(int64_t)m * a.top + min(lane, a.top - 1)];
     const float x = a.x[(int64_t)m * a.ld + n];
-    const int nf = a.ff / E, nr = a.top * nf, nc = nr + a.sff / E;
+    const unsigned nf = a.ff / E, nr = a.top * nf, nc = nr + a.sff / E;
     const T* act = static_cast<const T*>(a.act) + (int64_t)m * nc * E;
     const T* down = static_cast<const T*>(a.down);
     const T* sdown = static_cast<const T*>(a.shared_down);
     float sum = 0.f;
-    for (int c0 = lane; c0 < nc; c0 += 64 * U) {
+    for (unsigned c0 = lane; c0 - lane < nc; c0 += 64 * U) {
         Chunk<T> w[U], v[U];
-        int e[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) v[j] = load_chunk(act + min(c0 + 64 * j, nc - 1) * E);
 #pragma unroll
         for (int j = 0; j < U; ++j) {
-            const int c = min(c0 + 64 * j, nc - 1);
-            v[j] = load_chunk(act + c * E);
-            e[j] = c < nr ? pick[c / nf] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            const int c = min(c0 + 64 * j, nc - 1);
-            w[j] = load_chunk_stream(c < nr ? down + ((int64_t)e[j] * a.ld + n) * a.ff + (c % nf) * E : sdown + (int64_t)n * a.sff + (c - nr) * E);
+            const unsigned c = min(c0 + 64 * j, nc - 1), slot = c / nf;
+            const int e = __shfl(pick, slot, 64);
+            w[j] = load_chunk_stream(c < nr ? down + ((int64_t)e * a.ld + n) * a.ff + (c - slot * nf) * E : sdown + (int64_t)n * a.sff + (c - nr) * E);
         }
 #pragma unroll
         for (int j = 0; j < U; ++j)
@@ -931,8 +1027,19 @@ static int run_moe_rows(const MoeArgs& a, hipStream_t s) {
     const size_t lds = (size_t)a.ld * sizeof(T);
     RAVEN_REQUIRE(lds <= kMoeRowLds, "moe: rows of %d channels do not fit the LDS", a.ld);
     const int total = a.top * a.ff + a.sff;
-    moe_up_kernel<T><<<dim3((total + 3) / 4, a.M), dim3(256), lds, s>>>(a);
-    moe_down_kernel<T><<<dim3((a.ld + 3) / 4, a.M), dim3(256), 0, s>>>(a);
+    const dim3 up((total + 3) / 4, a.M), down((a.ld + 3) / 4, a.M);
+    if (picks_by_place(a.experts, a.top)) moe_up_place_kernel<T><<<up, dim3(256), lds, s>>>(a);
+    else moe_up_kernel<T><<<up, dim3(256), lds, s>>>(a);
+    // the fewest rounds of at most 12 pieces, of equal length
+    const int pieces = (total / Chunk<T>::N + 63) / 64, rounds = (pieces + 11) / 12;
+    switch (((pieces + rounds - 1) / rounds + 1) / 2) {
+        case 1: moe_down_kernel<T, 2><<<down, dim3(256), 0, s>>>(a); break;
+        case 2: moe_down_kernel<T, 4><<<down, dim3(256), 0, s>>>(a); break;
+        case 3: moe_down_kernel<T, 6><<<down, dim3(256), 0, s>>>(a); break;
+        case 4: moe_down_kernel<T, 8><<<down, dim3(256), 0, s>>>(a); break;
+        case 5: moe_down_kernel<T, 10><<<down, dim3(256), 0, s>>>(a); break;
+        default: moe_down_kernel<T, 12><<<down, dim3(256), 0, s>>>(a); break;
+    }
     return raven_host::check_launch("moe (rows)");
 }
 

@@ -321,6 +321,27 @@ def test_mixture(pkg, dtype, M, D, E, top, ff, shared):
     assert Dp == D or stream[:, D:].abs().max() == 0
 
 
+@DT
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("D,E,top,ff,shared", [(264, 5, 3, 328, 40), (264, 64, 4, 512, None), (520, 40, 5, 520, 40), (264, 64, 6, 600, 200), (264, 9, 8, 616, None),
+                                               (4104, 16, 8, 696, 264), (264, 12, 9, 688, 16)])
+def test_mixture_of_a_few_rows_by_every_number_of_pieces(pkg, dtype, M, D, E, top, ff, shared):
+    test_mixture(pkg, dtype, M, D, E, top, ff, shared)
+
+
+@DT
+@pytest.mark.parametrize("width", [512, 2056, 4104])
+def test_one_row_norms_itself_in_front_of_a_mixture(pkg, dtype, width):
+    """A token at a time through a mixture whose experts are all picked (no close call decides), against the oracle: one, two and more pieces of the row a thread."""
+    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(7, 7, 136, 136))])
+    w = O.random_weights(cfg, 3)
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=dtype)
+    model.load_state_dict(w)
+    ids = G.tokens(cfg, 4)
+    got, _ = feed(model, ids, [1] * 4)
+    assert G.rel(got, O.forward(cfg, w, ids)[0]) < (5e-5 if dtype == F32 else 3e-2)
+
+
 @pytest.mark.parametrize("M,D,E,top,ff", [(900, 96, 2, 1, 136), (700, 64, 3, 3, 264), (1100, 264, 1, 1, 72)])
 def test_mixture_in_large_tiles(pkg, M, D, E, top, ff):
     """Enough rows per expert for the 256-row tiles, a last tile cut short, experts of unequal share; every row against a dense sum."""
