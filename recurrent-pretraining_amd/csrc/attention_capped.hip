@@ -31,6 +31,7 @@ struct CappedArgs {
     int H, G, hd, t_max, S, pos0;
     const int* pos_dev;
     float scale, cap;
+    int last_block;  // chunks: the last block of query rows of this launch
     const float* r1;
     const float* r2;
     int append;       // S == 1: the row's own key comes from qk and goes to the cache
@@ -325,8 +326,8 @@ __global__ __launch_bounds__(256, 2) void capped_attention_prefill_kernel(Capped
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-    const int qb = gridDim.x - 1 - blockIdx.x;  // the blocks with the most keys start first
-    const int head = blockIdx.y, b = blockIdx.z, g = head / (a.H / a.G);
+    const int qb = a.last_block - blockIdx.z;  // the blocks with the most keys start first
+    const int head = blockIdx.x, b = blockIdx.y, g = head / (a.H / a.G);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qc = lane & 15, s4 = lane >> 4;
     const int pos0 = a.pos_dev ? *a.pos_dev : a.pos0;
@@ -538,18 +539,20 @@ __global__ __launch_bounds__(256, 2) void capped_attention_prefill_kernel(Capped
 }
 
 template <int HD>
-static int launch_capped_prefill(const CappedArgs& a, int B, hipStream_t s) {
+static int launch_capped_prefill(CappedArgs a, int B, hipStream_t s) {
     const int rg = (int64_t)((a.S + 127) / 128) * a.H * B >= 512 ? 2 : 1;
-    const dim3 grid((a.S + 64 * rg - 1) / (64 * rg), a.H, B);
     const bool fixed = fixed_reference(a.cap);
-    if (rg == 2) {
-        if (fixed) capped_attention_prefill_kernel<HD, 2, true><<<grid, dim3(256), 0, s>>>(a);
-        else capped_attention_prefill_kernel<HD, 2, false><<<grid, dim3(256), 0, s>>>(a);
-    } else {
-        if (fixed) capped_attention_prefill_kernel<HD, 1, true><<<grid, dim3(256), 0, s>>>(a);
-        else capped_attention_prefill_kernel<HD, 1, false><<<grid, dim3(256), 0, s>>>(a);
-    }
-    return raven_host::check_launch("capped_attention (prefill)");
+    return raven_host::causal_blocks((a.S + 64 * rg - 1) / (64 * rg), a.H, B, [&](dim3 grid, int last) {
+        a.last_block = last;
+        if (rg == 2) {
+            if (fixed) capped_attention_prefill_kernel<HD, 2, true><<<grid, dim3(256), 0, s>>>(a);
+            else capped_attention_prefill_kernel<HD, 2, false><<<grid, dim3(256), 0, s>>>(a);
+        } else {
+            if (fixed) capped_attention_prefill_kernel<HD, 1, true><<<grid, dim3(256), 0, s>>>(a);
+            else capped_attention_prefill_kernel<HD, 1, false><<<grid, dim3(256), 0, s>>>(a);
+        }
+        return raven_host::check_launch("capped_attention (prefill)");
+    });
 }
 
 constexpr int kCpMinRows = 16;  // fewer new rows per sequence go to the row kernel

@@ -34,6 +34,7 @@ namespace raven {
 constexpr int kPfKeys = 64;     // keys per tile
 
 struct PrefillArgs {
+    int last_block;  // contiguous caches: the last block of query rows of this launch
     const bf16* q;   // [B*S, h]
     bf16* y;         // [B*S, h], rows ldy elements apart
     int ldy;
@@ -225,12 +226,12 @@ __global__ __launch_bounds__(NW * 64, NW == 6 ? 3 : 2) void attention_prefill_ke
     // 32 lanes read transposed (8 banks each) hit 64 different banks
     bf16(*sv)[kPfKeys][kVPitch] = reinterpret_cast<bf16(*)[kPfKeys][kVPitch]>(smem_kv + SK_ELEMS);
 
-    int qb = gridDim.x - 1 - blockIdx.x;  // the blocks with the most keys start first
-    int b = blockIdx.z;
+    int qb = a.last_block - (int)blockIdx.z;  // the blocks with the most keys start first
+    int b = blockIdx.y;
     if constexpr (PAGED) {
         if (!paged_block(a, ROWS, &b, &qb)) return;
     }
-    const int head = PAGED ? blockIdx.x : blockIdx.y;
+    const int head = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qc = lane & 15, s4 = lane >> 4;
     const int h = a.nh * HD;
@@ -626,16 +627,18 @@ int prefill_attention_pitched(const void* q, void* y, int ldy, const raven_kv_ca
     const bool six = head_dim == 96 && rg == 2 && g_prefill_waves != 4 &&
                      (g_prefill_waves == 6 || (int64_t)((S + 191) / 192) * n_heads * B >= 512);
     const int rows = six ? 192 : 64 * rg;
-    const dim3 grid((S + rows - 1) / rows, n_heads, B);
+    return raven_host::causal_blocks((S + rows - 1) / rows, n_heads, B, [&](dim3 grid, int last) {
+        a.last_block = last;
 #define RAVEN_PREFILL(HD)                                                                  \
-    if (rg == 2) attention_prefill_kernel<HD, 2><<<grid, dim3(256), 0, s>>>(a);            \
-    else attention_prefill_kernel<HD, 1><<<grid, dim3(256), 0, s>>>(a)
-    if (six) attention_prefill_kernel<96, 2, 0, 6><<<grid, dim3(384), 0, s>>>(a);
-    else if (head_dim == 64) { RAVEN_PREFILL(64); }
-    else if (head_dim == 96) { RAVEN_PREFILL(96); }
-    else { RAVEN_PREFILL(128); }
+        if (rg == 2) attention_prefill_kernel<HD, 2><<<grid, dim3(256), 0, s>>>(a);        \
+        else attention_prefill_kernel<HD, 1><<<grid, dim3(256), 0, s>>>(a)
+        if (six) attention_prefill_kernel<96, 2, 0, 6><<<grid, dim3(384), 0, s>>>(a);
+        else if (head_dim == 64) { RAVEN_PREFILL(64); }
+        else if (head_dim == 96) { RAVEN_PREFILL(96); }
+        else { RAVEN_PREFILL(128); }
 #undef RAVEN_PREFILL
-    return raven_host::check_launch("prefill_attention");
+        return raven_host::check_launch("prefill_attention");
+    });
 }
 }  // namespace raven
 

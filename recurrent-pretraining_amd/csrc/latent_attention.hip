@@ -17,6 +17,7 @@
 namespace raven {
 
 struct LatentArgs {
+    int last_block;  // chunks: the last block of query rows of this launch
     const void* q;        // [M, H * (np + rp)] of T, not rotated
     const void* z;        // [M, ldz] of Z
     void* latent;         // [batch, t_max, kp] of T
@@ -542,8 +543,8 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(LatentArgs a) {
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-    const int qb = gridDim.x - 1 - blockIdx.x;
-    const int head = blockIdx.y, b = blockIdx.z;
+    const int qb = a.last_block - blockIdx.z;
+    const int head = blockIdx.x, b = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qc = lane & 15, s4 = lane >> 4;
     const int pos0 = a.pos0, row0 = qb * ROWS + wave * WR;
@@ -738,12 +739,14 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(LatentArgs a) {
 }
 
 template <int HDQ, int HDV>
-static int launch_latent_prefill(const LatentArgs& a, int B, hipStream_t s) {
-    if ((int64_t)((a.S + 127) / 128) * a.H * B >= 512)
-        latent_prefill_kernel<HDQ, HDV, 2><<<dim3((a.S + 127) / 128, a.H, B), dim3(256), 0, s>>>(a);
-    else
-        latent_prefill_kernel<HDQ, HDV, 1><<<dim3((a.S + 63) / 64, a.H, B), dim3(256), 0, s>>>(a);
-    return raven_host::check_launch("latent_attention (chunk)");
+static int launch_latent_prefill(LatentArgs a, int B, hipStream_t s) {
+    const int rg = (int64_t)((a.S + 127) / 128) * a.H * B >= 512 ? 2 : 1;
+    return raven_host::causal_blocks((a.S + 64 * rg - 1) / (64 * rg), a.H, B, [&](dim3 grid, int last) {
+        a.last_block = last;
+        if (rg == 2) latent_prefill_kernel<HDQ, HDV, 2><<<grid, dim3(256), 0, s>>>(a);
+        else latent_prefill_kernel<HDQ, HDV, 1><<<grid, dim3(256), 0, s>>>(a);
+        return raven_host::check_launch("latent_attention (chunk)");
+    });
 }
 
 constexpr int kLpMinRows = 16;  // fewer new rows per sequence take the absorbed route
