@@ -596,33 +596,37 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(LatentArgs a) {
     const int t0 = a.k0 + (first - a.k0) / kLpKeys * kLpKeys;
     const int wave_first = pos0 + row0 - window + 1, wave_last = pos0 + row0 + WR - 1;
     u32x4 rk[NKC], rv[NVC];
+    // A key's channels lie in two buffers; which one a piece comes from is a selection and no branch, and its address is formed anew for every tile: ten
+    // pointers kept over the walk were spilled, and a load from scratch waits for the rows requested before it, six memory latencies in a row (4096 rows of 16
+    // heads of 192 / 128 in a window of 1024: 145 us a launch, now 96)
+    const bf16* vbase = vn - (int64_t)a.k0 * ldkv;
     auto fetch = [&](int kt) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
 #pragma unroll
         for (int i = 0; i < NKC; ++i) {
-            const int c = threadIdx.x + 256 * i, d = (c % CQ) * 8;
-            const int64_t key = min(kt + c / CQ, n_keys - 1);
-            const bf16* p = d < a.np ? kn + (key - a.k0) * ldkv + d : kr + key * a.rp + (d < hd ? d - a.np : 0);
-            const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-            rk[i] = d < hd ? v : u32x4{0, 0, 0, 0};
+            const int c = tid + 256 * i, d = (c % CQ) * 8, key = min(kt + c / CQ, n_keys - 1);
+            const bool nope = d < a.np;
+            const bf16* base = nope ? kn : kr;
+            const int64_t at = (int64_t)(nope ? key - a.k0 : key) * (nope ? ldkv : a.rp) + (nope ? d : d < hd ? d - a.np : 0);
+            rk[i] = *reinterpret_cast<const u32x4*>(base + at);
         }
 #pragma unroll
         for (int i = 0; i < NVC; ++i) {
-            const int c = threadIdx.x + 256 * i, d = (c % CV) * 8;
-            const int64_t key = min(kt + c / CV, n_keys - 1);
-            const u32x4 v = *reinterpret_cast<const u32x4*>(vn + (key - a.k0) * ldkv + (d < a.vp ? d : 0));
-            rv[i] = d < a.vp ? v : u32x4{0, 0, 0, 0};
+            const int c = tid + 256 * i, d = (c % CV) * 8, key = min(kt + c / CV, n_keys - 1);
+            rv[i] = *reinterpret_cast<const u32x4*>(vbase + (int64_t)key * ldkv + (d < a.vp ? d : 0));
         }
     };
     auto park = [&]() {
 #pragma unroll
         for (int i = 0; i < NKC; ++i) {
-            const int c = threadIdx.x + 256 * i;
-            *reinterpret_cast<u32x4*>(&sk[c / CQ][(c % CQ) * 8]) = rk[i];
+            const int c = threadIdx.x + 256 * i, d = (c % CQ) * 8;
+            *reinterpret_cast<u32x4*>(&sk[c / CQ][d]) = d < hd ? rk[i] : u32x4{0, 0, 0, 0};
         }
 #pragma unroll
         for (int i = 0; i < NVC; ++i) {
-            const int c = threadIdx.x + 256 * i;
-            *reinterpret_cast<u32x4*>(&sv[c / CV][(c % CV) * 8]) = rv[i];
+            const int c = threadIdx.x + 256 * i, d = (c % CV) * 8;
+            *reinterpret_cast<u32x4*>(&sv[c / CV][d]) = d < a.vp ? rv[i] : u32x4{0, 0, 0, 0};
         }
     };
     auto tile = [&](int kt, bool masked) {

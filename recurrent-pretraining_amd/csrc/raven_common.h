@@ -226,7 +226,7 @@ template <typename... P> inline bool aligned16(const P*... p) { return (((uintpt
 // Causal attention over `blocks` blocks of query rows: grid (head, sequence, block), launch(grid, last) with the kernel's block last - blockIdx.z, so that workgroups
 // start with the longest blocks of ALL heads and sequences.  With the block as the fastest coordinate, an XCD (every eighth workgroup) and a CU got blocks of
 // the same few lengths head after head wherever their number is a multiple of eight.  us, before and now: 32 heads of 64 with capped scores over 4096 rows 257 / 166
-// (32 blocks), 55 heads of 96 over 2 x 2000 rows 214 / 175, 16 windowed heads over 4096 rows 144 / 145.  (Every second 256 workgroups in reverse: 161, 169.)
+// (32 blocks), 55 heads of 96 over 2 x 2000 rows 214 / 175.  (Every second 256 workgroups in reverse: 161, 169.)
 template <typename F>
 inline int causal_blocks(int blocks, int heads, int sequences, F&& launch) {
     for (int first = 0; first < blocks; first += 65535) {  // (what a grid's last coordinate holds)
