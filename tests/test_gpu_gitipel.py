@@ -157,6 +157,22 @@ def test_norm_conv_in_portions(pkg, dtype, D, taps):
     assert ((plain - want).abs() <= (2e-5 if dtype == F32 else 2 ** -8 * want.abs() + 1e-4)).all()
 
 
+@DT
+@pytest.mark.parametrize("B,T,D,taps", [(1, 2053, 264, 4), (2, 1030, 1032, 3), (1, 16390, 72, 2), (1, 33, 2056, 4), (3, 5, 4096, 4)])
+def test_norm_conv_walks_over_tiles_of_every_height(pkg, dtype, B, T, D, taps):
+    """Tiles of 4, 8 and 16 rows of one, two and four pieces a thread, and one more token behind them, which reads the ring that they left."""
+    g = torch.Generator().manual_seed(D)
+    x, w, c = torch.randn(B, T + 1, D, generator=g) * 5, torch.rand(D, generator=g) + 0.5, torch.randn(D, taps, generator=g)
+    want = torch.stack([(lambda h: h + O.causal_conv(h, c))(O.rms_norm(x[b], w, 1e-3)) for b in range(B)])
+    ring = torch.full((B, taps, D), float("nan"), device="cuda")
+    conv, weight, got = c.t().cuda().contiguous(), w.cuda(), []
+    for pos, n in ((0, T), (T, 1)):
+        rows = x[:, pos:pos + n].reshape(B * n, D).cuda()
+        got.append(pkg.hip.norm_conv(rows, weight, D, 1e-3, B, n, dtype, conv=conv, ring=ring, pos0=pos).view(B, n, D))
+    got = torch.cat(got, 1).float().cpu()
+    assert ((got - want).abs() <= (2e-5 if dtype == F32 else 2 ** -8 * want.abs() + 1e-4)).all()
+
+
 # ---- attention ---------------------------------------------------------------------------------------
 def run_attention(pkg, q, k, score, cuts, dtype, t_max=None, dp=None):
     """q [T, H, d], k [T, G, d] in portions; returns [T, H, d] float."""
