@@ -58,10 +58,10 @@ __device__ __forceinline__ int ordered_key(float v) {
 // one wave: the `top` experts of largest logit (lower index first among equals); lane k holds the k-th one and its score.
 // Up to 64 experts (a lane each) an expert's place is the number of experts before it, counted in one sweep over the others' logits
 // through the lane-to-lane broadcast: 64 steps without a dependence, where `top` maxima over the wave, twelve exchanges each, took 3 us
-// of every launch that picks six (moe_up_kernel at one row 14.7 -> 12 us, routing of 20 rows 11.8 -> 8).  One or two are found sooner by
+// of every launch that picks six (routing of 20 rows 11.8 -> 8 us; a single row's products share the counting out over four waves).  One or two are found sooner by
 // maxima (both launches of 8 rows of width 512, one of 8 experts of 512: 12.0 us, by counting 13.4).
 // (U steps unrolled.  In a workgroup alone on its CU all 64 are 2.5 KB of code run once out of a cold instruction cache: routing of 20 rows 9.7 us, with 16
-// 8.8; where thousands of workgroups run it, all: one row of 7 x 384 channels of width 1024, both launches 9.6, with 16 10.1.)
+// 8.8.)
 __host__ __device__ __forceinline__ bool picks_by_place(int experts, int top) { return experts <= 64 && top > 2; }
 template <int U>
 __device__ __forceinline__ void pick_by_place(float v, int experts, int& mine, float& score) {  // v: expert `lane`'s logit
@@ -918,6 +918,7 @@ static bool few_rows_fit(const raven_moe* m, int M, int ld) {
 // each pick, and past 64 experts, where maxima pick, one for each workgroup that picks.  Grouped: four launches, and once the weights of the experts that rows
 // pick on average, with a share for each.  Of two that are about the same, the row kernels.  Against the better of the two the choice costs 0.5 % on average,
 // 24 % at most (300 experts of 136 at width 264, 8 per row, 12 rows: 28 / 23).
+// (Fitted to row kernels that took longer than now: width 2048, 2 rows 25 us, 3: 34, 4: 43; where the two ways are about the same, either may be ahead by a tenth.)
 static bool grouping_pays(const raven_moe* m, int M, int ld) {
     const double pairs = (double)M * m->top, touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), shared = m->shared_up ? 1 : 0;
     const double expert = 6e-6 * ld * m->ff;  // MB
