@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void moe_up_place_kernel(MoeArgs a) {
     constexpr int E = Chunk<T>::N, U = 4, H = 2;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* xs = reinterpret_cast<T*>(smem_raw);  // [ld]
-    __shared__ int place[4][64];
+    __shared__ unsigned char place[4][64];  // (in bytes: beside the longest row, kMoeRowLds, there is 1 KB)
     __shared__ float red[4];
     const int m = blockIdx.y, nc = a.ld / E, total = a.top * a.ff + a.sff, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const float* logits = a.logits + (int64_t)m * a.ldl;
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void moe_up_place_kernel(MoeArgs a) {
         const int at = 16 * wave + j, other = __builtin_amdgcn_readlane(key, at);
         before += other > key || (other == key && at < lane) ? 1 : 0;
     }
-    place[wave][lane] = before;
+    place[wave][lane] = (unsigned char)before;
     if (!a.h) {
         float ss = 0.f;
 #pragma unroll

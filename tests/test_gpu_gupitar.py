@@ -330,6 +330,15 @@ def test_mixture_of_a_few_rows_by_every_number_of_pieces(pkg, dtype, M, D, E, to
 
 
 @DT
+def test_mixture_of_the_longest_rows(pkg, dtype):
+    """What the row kernels' LDS holds: the longest row is taken, a longer one refused."""
+    D = 63 * 1024 // (4 if dtype == F32 else 2)
+    test_mixture(pkg, dtype, 1, D, 5, 3, 8, 8)
+    with pytest.raises(pkg.hip.RavenHipError):
+        test_mixture(pkg, dtype, 1, D + 8, 5, 3, 8, 8)
+
+
+@DT
 @pytest.mark.parametrize("width", [512, 2056, 4104])
 def test_one_row_norms_itself_in_front_of_a_mixture(pkg, dtype, width):
     """A token at a time through a mixture whose experts are all picked (no close call decides), against the oracle: one, two and more pieces of the row a thread."""
