@@ -547,6 +547,9 @@ typedef struct raven_moe {
     int32_t     experts, top, ff, shared_ff, logit_ld;
 } raven_moe;
 size_t raven_moe_workspace_bytes(const raven_moe* m, int32_t M, int32_t ld, int32_t dtype);
+/* What runs M rows (aligned ones): plan[0] = 0 the row kernels, 1 grouped products of few rows, 2 of a chunk; plan[1] = 1: behind a norm that is shared out between
+ * two products the rows route themselves.  No launch. */
+int    raven_moe_plan(const raven_moe* m, int32_t M, int32_t ld, int32_t dtype, int32_t* plan);
 int    raven_moe_forward(const raven_moe* m, const void* h, const float* logits, float* x, int32_t M, int32_t ld, int32_t dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* One pre-norm layer on the stream x [B*S, ld] (in place):

@@ -79,6 +79,8 @@ __device__ __forceinline__ void pick_by_place(float v, int experts, int& mine, f
     mine = min(mine, experts - 1);
     score = sigmoid_f32(s);
 }
+// The picks of a row are different experts whatever its logits are, as by place: where only minus infinity and NaN are left, the lowest numbers that have not been
+// taken (the lists of picked_rows have room for one row of a token per expert).
 __device__ __forceinline__ void pick_by_maxima(const float* logits, int experts, int top, int& mine, float& score) {
     const int lane = threadIdx.x & 63;
     float v[kMaxExperts / 64];
@@ -102,7 +104,6 @@ __device__ __forceinline__ void pick_by_maxima(const float* logits, int experts,
         int who = best == m ? at : 0x7fffffff;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) who = min(who, __shfl_xor(who, d, 64));
-        who = min(who, experts - 1);  // all logits NaN: still an expert
         if (lane == k) {
             mine = who;
             logit = m;
@@ -111,6 +112,12 @@ __device__ __forceinline__ void pick_by_maxima(const float* logits, int experts,
         for (int j = 0; j < kMaxExperts / 64; ++j)
             if (lane + 64 * j == who) v[j] = -INFINITY;
     }
+    if (const unsigned long long none = __ballot(lane < top && logit == -INFINITY))
+        for (int k = __builtin_ctzll(none), e = 0; k < top; ++e) {  // (top <= experts)
+            if (__any(lane < k && mine == e)) continue;
+            if (lane == k) mine = e;
+            ++k;
+        }
     score = sigmoid_f32(logit);
 }
 __device__ __forceinline__ void pick_experts(const float* logits, int experts, int top, int& mine, float& score) {
@@ -621,8 +628,8 @@ __device__ __forceinline__ int picked_rows(const FewArgs& a, int which, int* gro
         const int p = p0 + lane;
         const bool own = p < pairs && e == g;
         const unsigned long long found = __ballot(own);
-        if (own && threadIdx.x < 64) {
-            const int at = n + __popcll(found & ((1ull << lane) - 1));
+        const int at = n + __popcll(found & ((1ull << lane) - 1));
+        if (own && threadIdx.x < 64 && at < kPickedRows) {  // (a token picks an expert once, so that there are no more)
             x_row[at] = UP ? p / a.top : p;
             y_row[at] = p;
             if (UP) scale[at] = a.g.x_scale[p];
@@ -633,7 +640,7 @@ __device__ __forceinline__ int picked_rows(const FewArgs& a, int which, int* gro
     for (int c = 0; c < kHeldPicks; ++c)
         if (64 * c < pairs) take(64 * c, held[c]);
     for (int p0 = 64 * kHeldPicks; p0 < pairs; p0 += 64) take(p0, a.pick[min(p0 + lane, pairs - 1)]);
-    return n;
+    return min(n, kPickedRows);
 }
 
 constexpr int few_columns(bool up) { return up ? 16 : 32; }  // output columns of a unit
@@ -1164,6 +1171,16 @@ int moe_forward(const raven_moe* m, const void* h, const float* factors, const f
     return raven_host::check_launch("moe (combine)");
 }
 }  // namespace raven
+
+extern "C" int raven_moe_plan(const raven_moe* m, int32_t M, int32_t ld, int32_t dtype, int32_t* plan) {
+    RAVEN_REQUIRE(plan, "moe_plan: null pointer");
+    plan[0] = plan[1] = 0;
+    if (const int rc = raven::check_moe("moe_plan", m, M, ld, dtype)) return rc;
+    if (M == 0) return 0;
+    plan[0] = raven::moe_path(m, nullptr, M, ld, dtype);
+    plan[1] = raven::moe_picks_itself(m, nullptr, M, ld, dtype);
+    return 0;
+}
 
 extern "C" int raven_moe_forward(const raven_moe* m, const void* h, const float* logits, float* x, int32_t M, int32_t ld, int32_t dtype,
                                  void* workspace, size_t workspace_bytes, void* stream) {

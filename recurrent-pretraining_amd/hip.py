@@ -187,6 +187,7 @@ SIGNATURES = {
     "raven_rglru_workspace_bytes": (_SZ, [C.POINTER(Rglru), _I32, _I32, _I32]),
     "raven_rglru_forward": (C.c_int, [C.POINTER(Rglru), _VP, _VP, _VP, _VP, _I32, _I32, _I32, _VP, _I32, _VP, _SZ, _VP]),
     "raven_moe_workspace_bytes": (_SZ, [C.POINTER(Moe), _I32, _I32, _I32]),
+    "raven_moe_plan": (C.c_int, [C.POINTER(Moe), _I32, _I32, _I32, C.POINTER(_I32)]),
     "raven_moe_forward": (C.c_int, [C.POINTER(Moe), _VP, _VP, _VP, _I32, _I32, _I32, _VP, _SZ, _VP]),
     "raven_mixer_layer_workspace_bytes": (_SZ, [C.POINTER(StreamDims), C.POINTER(MixerLayer), _I32, _I32, _I32]),
     "raven_mixer_layer_forward": (C.c_int, [C.POINTER(StreamDims), C.POINTER(MixerLayer), C.POINTER(MixerState), _VP, _I32, _I32, _I32, _VP,
@@ -855,6 +856,13 @@ def rglru(desc: Rglru, z, ring, state, B, S, pos0, pos_dev=None):
                                     int(pos0), _ptr(pos_dev, "pos_dev", torch.int32), code, _ptr(ws, "ws"), 0 if ws is None else ws.numel(), _stream())
     _check(rc, "raven_rglru_forward")
     return y
+
+
+def moe_plan(desc: Moe, M: int, ld: int, dtype):
+    """(0 row kernels, 1 grouped products of few rows, 2 of a chunk; whether rows behind a shared norm route themselves); no launch."""
+    plan = (_I32 * 2)()
+    _check(load().raven_moe_plan(C.byref(desc), M, ld, dtype_code(dtype), plan), "raven_moe_plan")
+    return plan[0], bool(plan[1])
 
 
 def moe(desc: Moe, h, logits, x):

@@ -338,6 +338,59 @@ def test_mixture_of_the_longest_rows(pkg, dtype):
         test_mixture(pkg, dtype, 1, D + 8, 5, 3, 8, 8)
 
 
+@pytest.mark.parametrize("M", [7, 300])
+@pytest.mark.parametrize("E,top", [(5, 1), (5, 2), (64, 2), (40, 6), (70, 8), (300, 2)])
+def test_picks_are_different_experts_whatever_the_logits(pkg, E, top, M):
+    """Rows of numbers, of equal ones, of minus infinity and NaN, alone and mixed: the experts in falling order of their logits, NaN last or beside minus infinity, lower
+    numbers first among equals, and none of them twice.  Read where the kernels keep them, at the workspace's start or behind a row's activations."""
+    D, ff = 64, 16
+    cfg = G.config(D, 8, [G.rglru(8, 1, 1, G.moe(E, top, ff))])
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(O.random_weights(cfg, E))
+    desc, hip = model.layers[0].moe, pkg.hip
+    g = torch.Generator().manual_seed(M)
+    logits = torch.randn(M, E, generator=g)
+    odd = torch.rand(M, E, generator=g)
+    kinds = [lambda r: r, lambda r: r * 0, lambda r: r * 0 + math.nan, lambda r: r * 0 - math.inf, lambda r: r.masked_fill(torch.arange(E) != E // 2, math.nan),
+             lambda r: r.masked_fill(torch.arange(E) != E - 1, -math.inf), None]
+    for m in range(M):
+        kind = kinds[m % len(kinds)]
+        logits[m] = kind(logits[m]) if kind else logits[m].masked_fill(odd[m] < 0.5, -math.inf).masked_fill(odd[m] > 0.6, math.nan)
+    rows = torch.full((M, desc.logit_ld), 1e9)
+    rows[:, :E] = logits
+    rows, h, x = rows.cuda(), torch.randn(M, D, generator=g).to(BF16).cuda(), torch.zeros(M, D, device="cuda")
+    n = hip.load().raven_moe_workspace_bytes(hip.C.byref(desc), M, D, hip.dtype_code(BF16))
+    ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    assert hip.load().raven_moe_forward(hip.C.byref(desc), h.data_ptr(), rows.data_ptr(), x.data_ptr(), M, D, hip.dtype_code(BF16), ws.data_ptr(), n, hip._stream()) == 0
+    at = (M * top * ff * 2 + 255) // 256 * 256 if hip.moe_plan(desc, M, D, BF16)[0] == 0 else 0
+    picks = ws[at:at + M * top * 4].view(torch.int32).view(M, top).cpu()
+    order = logits.nan_to_num(nan=-math.inf, posinf=math.inf, neginf=-math.inf)
+    if E <= 64 and top > 2:  # by place: NaN behind minus infinity
+        order = torch.where(logits.isnan(), order, order.clamp(min=-1e30))
+    assert torch.equal(picks.long(), order.sort(dim=-1, descending=True, stable=True).indices[:, :top])
+    assert x.isfinite().all()
+
+
+@pytest.mark.parametrize("M,E", [(20, 40), (20, 64), (32, 40), (32, 64)])
+def test_sequences_of_nan_leave_the_others_of_a_batch_alone(pkg, M, E):
+    """Rows that route themselves, two picks each, most of the sequences all NaN: the others keep the bits that they have beside ordinary ones."""
+    width = 1536
+    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(E, 2, 520, 520))])
+    w = O.random_weights(cfg, 3)
+    w["embed"][95] = math.nan
+    model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(w)
+    assert pkg.hip.moe_plan(model.layers[0].moe, M, width, BF16) == (1, True)
+    ids = torch.stack([G.tokens(cfg, 2, seed=s) % 95 for s in range(M)])
+    spoilt = ids.clone()
+    spoilt[3:] = 95
+    got = []
+    for i in (ids, spoilt):
+        cache = model.new_cache()
+        got.append(torch.cat([model.forward(i[:, t:t + 1], past_key_values=cache).logits for t in range(2)], 1))
+    assert got[0].isfinite().all() and torch.equal(got[0][:3], got[1][:3]) and got[1][3:].isnan().all()
+
+
 @DT
 @pytest.mark.parametrize("width", [512, 2056, 4104])
 def test_one_row_norms_itself_in_front_of_a_mixture(pkg, dtype, width):
