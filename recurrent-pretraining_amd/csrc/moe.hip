@@ -850,7 +850,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
     store4(a.x + (int64_t)m * a.ld + c, x);
 }
 
-// The same with the norm that the next layer begins with, h = T(x / rms(x) * w): a workgroup per row, whose pieces stay in registers.  us at 20 rows of
+// The same with the norm that the next layer begins with, h = T(x / rms(x) * w): a workgroup per row, whose pieces stay in registers.  The squares are added as
+// norm_conv_kernel adds them, so that a layer gives the same bits whether it is called with the next one or by itself.  us at 20 rows of
 // width 2048, sums and norm / this: 4.7 + 4.6 / 4.9; at 4096 rows 32 + 9.8 / 34.
 constexpr int kCombineThreads = 512;
 struct NextNorm {
@@ -861,12 +862,11 @@ struct NextNorm {
 };
 template <typename Y, int P, bool PICKED>
 __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeArgs a, NextNorm next) {
-    __shared__ float red[kCombineThreads / 64];
+    __shared__ float squares[kCombineThreads * P], red[4];
     const int m = blockIdx.x, tid = threadIdx.x, per = a.ld / 4;
     const Y* y = static_cast<const Y*>(a.y);
     const float gate = a.ys ? sigmoid_f32(a.logits[(int64_t)m * a.ldl + a.experts]) : 0.f;
     f32x4 x[P], w[P];
-    float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < P; ++j) {
         const int c = 4 * min(tid + kCombineThreads * j, per - 1);
@@ -883,18 +883,20 @@ __global__ __launch_bounds__(kCombineThreads) void moe_combine_norm_kernel(MoeAr
                 if (k0 + k < a.top) x[j] += v[k];
         }
         if (a.ys) x[j] += shared * gate;
-        if (tid + kCombineThreads * j < per) {
-            store4(a.x + (int64_t)m * a.ld + c, x[j]);
-            ss += x[j][0] * x[j][0] + x[j][1] * x[j][1] + x[j][2] * x[j][2] + x[j][3] * x[j][3];
-        }
+        const bool own = tid + kCombineThreads * j < per;
+        if (own) store4(a.x + (int64_t)m * a.ld + c, x[j]);
+        squares[tid + kCombineThreads * j] = own ? x[j][0] * x[j][0] + x[j][1] * x[j][1] + x[j][2] * x[j][2] + x[j][3] * x[j][3] : 0.f;
     }
-    ss = wave_sum(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
-    ss = 0.f;
+    if (tid < 256) {
+        float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < kCombineThreads / 64; ++i) ss += red[i];
-    const float inv = 1.0f / sqrtf(ss / (float)next.dim + next.eps);
+        for (int i = 0; i < kCombineThreads / 256 * P; ++i) ss += squares[tid + 256 * i];
+        ss = wave_sum(ss);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+    }
+    __syncthreads();
+    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)next.dim + next.eps);
 #pragma unroll
     for (int j = 0; j < P; ++j)
         if (tid + kCombineThreads * j < per) store4(static_cast<bf16*>(next.h) + (int64_t)m * a.ld + 4 * (tid + kCombineThreads * j), x[j] * inv * w[j]);
