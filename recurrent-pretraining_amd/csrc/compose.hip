@@ -77,7 +77,7 @@ int g_pad_decode_rows = 1; // raven_set_tuning("pad_decode_rows"): 0 = decode st
 struct BlockScratch {
     char *n1, *qkv, *q, *ya, *x1, *x2, *n3, *g, *x3, *xa, *xr;
     int ld_pad;     // n1, ya and n3 have room for rows this many elements apart (n_embd, or the next multiple of 64 for chunks)
-    float* e_sums;  // fp32 sums of the adapter's embedding half, computed once for all recurrences (bf16; up to 32 rows of floats for the one-row kernels)
+    float* e_sums;  // fp32 sums of the adapter's embedding half, computed once for all recurrences (up to 32 rows; bf16 ones past that lie in x3 and xr)
     void* attn_ws;
     size_t attn_ws_bytes;
     void* lin_ws;
@@ -108,10 +108,11 @@ static size_t carve(const raven_dims* d, int M, char* base, BlockScratch* out) {
     s.x2 = take(row);
     s.n3 = take(row_pad);
     s.g = take((size_t)M * d->intermediate * es);
-    s.x3 = take(row);
     s.xa = take(row);
+    s.x3 = take(row);  // x3 and xr: the schedule of one row (and of a few float ones) alone
     s.xr = take(row);
-    s.e_sums = reinterpret_cast<float*>(take(M <= 32 || d->dtype == RAVEN_BF16 ? (size_t)M * d->n_embd * sizeof(float) : 0));
+    s.e_sums = reinterpret_cast<float*>(take(M <= 32 ? (size_t)M * d->n_embd * sizeof(float) : 0));
+    if (M > 32 && d->dtype == RAVEN_BF16) s.e_sums = reinterpret_cast<float*>(s.x3);
     s.attn_ws_bytes = raven_decode_attention_workspace_bytes(M, d->n_heads, d->head_dim);
     s.attn_ws = s.attn_ws_bytes ? take(s.attn_ws_bytes) : nullptr;
     const int widest = 3 * d->n_embd > 2 * d->intermediate ? 3 * d->n_embd : 2 * d->intermediate;
@@ -246,7 +247,7 @@ static int run_block(const raven_dims* d, const raven_block_weights* w, const Bl
     }
     // the tail norm's output is the next block's norm_1 input when it goes to scratch.n1: rows as that block will read them
     const int tail_ld = tail_out == static_cast<void*>(s.n1) ? ld : h;
-    return linear_then_norm(s.g, 0, w->mlp_proj, s.x2, s.x3, w->norm_4, y_out, tail_w, tail_out, M, h, I, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, tail_ld);
+    return linear_then_norm(s.g, 0, w->mlp_proj, s.x2, s.x1, w->norm_4, y_out, tail_w, tail_out, M, h, I, d->eps, dt, s.lin_ws, s.lin_ws_bytes, hs, tail_ld);
 }
 
 // Whether a few float rows take the schedule of one row: every norm in front of a product is that product's own

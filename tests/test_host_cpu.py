@@ -46,6 +46,18 @@ def test_library_identity_and_argument_errors(pkg):
     assert 0 < n1 < n32 and n1 % 256 == 0
 
 
+@pytest.mark.parametrize("h,heads,inter", [(5280, 55, 17920), (256, 4, 704), (1000, 25, 136)])
+@pytest.mark.parametrize("M", [33, 93, 4096, 16384])
+def test_block_workspace_of_many_rows_holds_their_activations_alone(pkg, h, heads, inter, M):
+    """Six rows of n_embd, q | k | v, three rows that may be padded to whole lines, the gated row, and what attention and products ask for: nothing more past 32 rows, whatever
+    calls keep between recurrences."""
+    lib, up = pkg.hip.load(), lambda n: (n + 255) // 256 * 256
+    dims = pkg.hip.make_dims(h, heads, inter, 1e-6, torch.bfloat16)
+    parts = [3 * up(2 * M * h)] + [up(2 * M * h)] * 6 + [up(2 * M * ((h + 63) // 64 * 64))] * 3 + [up(2 * M * inter)]
+    parts += [up(lib.raven_decode_attention_workspace_bytes(M, heads, h // heads)), up(lib.raven_linear_workspace_bytes(M, max(3 * h, 2 * inter)))]
+    assert lib.raven_block_workspace_bytes(ctypes.byref(dims), M) == sum(parts)
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where nothing can be launched")
 @pytest.mark.parametrize("shift", ["x", "w", "residual", "y"])
 @pytest.mark.parametrize("M,N,K", [(40, 256, 4096), (100, 1024, 11008), (160, 2048, 17920)])
