@@ -52,7 +52,7 @@ struct MixerScratch {
     char *h, *z, *low, *y, *ff;  // low: the decay's low-rank rows / the normed query latents
     char* q;
     float *decay, *logits;
-    float *squares, *factors;  // 2 to 32 rows of bf16: a norm shared out between two products (NormAhead)
+    float *squares, *factors;  // a norm shared out between two products (NormAhead): in lin_ws, or null
     char *mix_ws, *ff_ws, *lin_ws;
     size_t mix_ws_bytes, ff_ws_bytes, lin_ws_bytes;
 };
@@ -89,9 +89,6 @@ static size_t carve_mixer(const raven_stream_dims* d, const raven_mixer_layer* l
     s.y = take(M * inner * es);
     s.ff = take(ff ? M * l->ff * es : 0);
     s.logits = reinterpret_cast<float*>(take(moe ? M * l->moe->logit_ld * sizeof(float) : 0));
-    const bool shared_norm = d->dtype == RAVEN_BF16 && M >= 2 && M <= 32;
-    s.squares = reinterpret_cast<float*>(take(shared_norm ? M * norm_pitch(d->ld / 16) * sizeof(float) : 0));
-    s.factors = reinterpret_cast<float*>(take(shared_norm ? M * sizeof(float) : 0));
     switch (l->mixer) {
         case RAVEN_MIXER_ATTENTION: s.mix_ws_bytes = raven_capped_attention_workspace_bytes((int)M, l->heads, l->kv_heads, l->head_dim); break;
         case RAVEN_MIXER_GENERAL_DELTA: s.mix_ws_bytes = raven_delta_rule_workspace_bytes(B, S, l->heads, l->head_dim); break;
@@ -107,6 +104,11 @@ static size_t carve_mixer(const raven_stream_dims* d, const raven_mixer_layer* l
     if (moe && (size_t)l->moe->logit_ld > widest) widest = l->moe->logit_ld;
     s.lin_ws_bytes = M > 1 ? raven_linear_workspace_bytes((int)M, (int)widest) : 0;
     s.lin_ws = take(s.lin_ws_bytes);
+    // (the products around a shared norm are single launches without slices, and what a mixture needs it has in ff_ws)
+    if (const size_t squares = raven_host::align_up(M * norm_pitch(d->ld / 16) * sizeof(float)); base && squares + M * sizeof(float) <= s.lin_ws_bytes) {
+        s.squares = reinterpret_cast<float*>(s.lin_ws);
+        s.factors = reinterpret_cast<float*>(s.lin_ws + squares);
+    }
     if (out) *out = s;
     return off;
 }
@@ -247,7 +249,7 @@ static int run_mixer_layer(const raven_stream_dims* dims, const raven_mixer_laye
     const void* second = l.ff_kind == RAVEN_FF_MOE ? l.moe->router : l.ff_kind == RAVEN_FF_GELU ? l.up : nullptr;
     const int second_n = l.ff_kind == RAVEN_FF_MOE ? l.moe->logit_ld : l.ff;
     void* const second_y = l.ff_kind == RAVEN_FF_MOE ? static_cast<void*>(w.logits) : static_cast<void*>(w.ff);
-    if (second && !one_row && dt == RAVEN_BF16 && M <= 32 && ld <= 16 * kNormParts && epilogue_in_one_launch(w.y, l.w_out, x, M, ld, inner, 1, w.lin_ws, w.lin_ws_bytes) &&
+    if (second && !one_row && dt == RAVEN_BF16 && M <= 32 && w.squares && ld <= 16 * kNormParts && epilogue_in_one_launch(w.y, l.w_out, x, M, ld, inner, 1, w.lin_ws, w.lin_ws_bytes) &&
         epilogue_in_one_launch(w.h, second, second_y, M, second_n, ld, l.ff_kind == RAVEN_FF_MOE, w.lin_ws, w.lin_ws_bytes) &&
         (l.ff_kind != RAVEN_FF_MOE || moe_takes_factors(l.moe, w.h, M, ld, dt))) {
         raven_epilogue out{}, in{};

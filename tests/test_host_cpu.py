@@ -58,6 +58,21 @@ def test_block_workspace_of_many_rows_holds_their_activations_alone(pkg, h, head
     assert lib.raven_block_workspace_bytes(ctypes.byref(dims), M) == sum(parts)
 
 
+@pytest.mark.parametrize("width,heads,ff", [(72, 2, 40), (512, 8, 2048), (2048, 32, 8192)])
+@pytest.mark.parametrize("M", [2, 20, 32, 33])
+def test_layer_workspace_holds_its_activations_alone(pkg, width, heads, ff, M):
+    """An attention layer with a GELU feed-forward: the normed row, the projections, heads, the hidden row, and what attention and products ask for."""
+    hip, lib, up = pkg.hip, pkg.hip.load(), lambda n: (n + 255) // 256 * 256
+    some = 4096  # (only sizes are asked for)
+    dims = hip.StreamDims(width, width, 1e-5, hip.dtype_code(torch.bfloat16))
+    layer = hip.MixerLayer(mixer=hip.MIXER_ATTENTION, norm1=some, w_in=some, w_out=some, norm2=some, up=some, down=some, ff=ff, heads=heads, kv_heads=1, dim=64, head_dim=64,
+                           ff_kind=hip.FF_GELU)
+    z, inner = (heads + 1) * 64, heads * 64
+    parts = [2 * M * n for n in (width, z, inner, ff)]
+    parts += [lib.raven_capped_attention_workspace_bytes(M, heads, 1, 64), lib.raven_linear_workspace_bytes(M, max(z, width, 2 * ff))]
+    assert hip.mixer_layer_workspace_bytes(dims, layer, M, 1) == sum(map(up, parts))
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: only where nothing can be launched")
 @pytest.mark.parametrize("shift", ["x", "w", "residual", "y"])
 @pytest.mark.parametrize("M,N,K", [(40, 256, 4096), (100, 1024, 11008), (160, 2048, 17920)])
