@@ -249,7 +249,7 @@ static int run_mixer_layer(const raven_stream_dims* dims, const raven_mixer_laye
     const void* second = l.ff_kind == RAVEN_FF_MOE ? l.moe->router : l.ff_kind == RAVEN_FF_GELU ? l.up : nullptr;
     const int second_n = l.ff_kind == RAVEN_FF_MOE ? l.moe->logit_ld : l.ff;
     void* const second_y = l.ff_kind == RAVEN_FF_MOE ? static_cast<void*>(w.logits) : static_cast<void*>(w.ff);
-    if (second && !one_row && dt == RAVEN_BF16 && M <= 32 && w.squares && ld <= 16 * kNormParts && epilogue_in_one_launch(w.y, l.w_out, x, M, ld, inner, 1, w.lin_ws, w.lin_ws_bytes) &&
+    if (second && !one_row && dt == RAVEN_BF16 && M <= 32 && w.squares && ld <= 16 * kNormParts && raven_host::aligned16(l.norm2) && epilogue_in_one_launch(w.y, l.w_out, x, M, ld, inner, 1, w.lin_ws, w.lin_ws_bytes) &&
         epilogue_in_one_launch(w.h, second, second_y, M, second_n, ld, l.ff_kind == RAVEN_FF_MOE, w.lin_ws, w.lin_ws_bytes) &&
         (l.ff_kind != RAVEN_FF_MOE || moe_takes_factors(l.moe, w.h, M, ld, dt))) {
         raven_epilogue out{}, in{};

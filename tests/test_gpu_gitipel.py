@@ -498,6 +498,29 @@ def test_norm_between_two_products_of_a_few_rows(pkg, width, M):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
 
 
+@pytest.mark.parametrize("M", [1, 4, 20, 40])
+def test_norm_weights_off_sixteen_bytes(pkg, M):
+    """A norm takes weights that start on any float, behind an output product as well."""
+    width = 512
+    cfg = G.config(width, 96, [G.attn(4, 2, 64, 1024)], taps=3)
+    model = pkg.GitipelForCausalLM(pkg.GitipelConfig(**cfg), device="cuda", dtype=BF16)
+    model.load_state_dict(O.random_weights(cfg, 8, 3))
+    layer, rows = model.layers[0], torch.randn(M, width, generator=torch.Generator().manual_seed(M)).cuda()
+    ws = torch.empty(pkg.hip.mixer_layer_workspace_bytes(model.dims, layer.native, M, 1), dtype=torch.uint8, device="cuda")
+    off = torch.empty(width + 1, device="cuda")
+    off[1:] = layer.norm2
+    got = []
+    for norm2 in (layer.norm2, off[1:]):
+        cache = model.new_cache(16)
+        cache.ensure(M, 1, BF16, "cuda")
+        x = rows.clone()
+        layer.native.norm2 = norm2.data_ptr()
+        pkg.hip.mixer_layer(model.dims, layer.native, cache.native(0), x, M, 1, 0, ws)
+        got.append(x.cpu())
+    layer.native.norm2 = layer.norm2.data_ptr()
+    assert not torch.equal(got[0], rows.cpu()) and G.rel(got[1], got[0]) < 1e-2
+
+
 @pytest.mark.parametrize("M", [17, 32, 40])
 @pytest.mark.parametrize("width,ff", [(1024, 4608), (2048, 8192), (2504, 5120)])
 def test_slices_of_a_layer_added_by_the_norm_of_the_next(pkg, width, ff, M):
