@@ -718,12 +718,13 @@ def test_batch_of_equal_lengths_against_each_alone(pkg, name):
 @pytest.mark.parametrize("M", [2, 4, 8])
 @pytest.mark.parametrize("width", [512, 540])
 def test_norm_between_the_output_product_and_a_mixture(pkg, width, M, shared):
-    """Batches whose output product and router share the norm between them and whose experts take the rows' factors (every expert is picked, so that no close call
-    decides): against the oracle, each row by itself."""
+    """Batches whose output product and router share the norm between them, rows that route themselves, and two rows, which have a norm of their own (every expert is picked,
+    so that no close call decides): against the oracle, each row by itself."""
     cfg = G.config(width, 96, [G.rglru(width, 4, 3, G.moe(16, 16, 264, shared))])
     w = O.random_weights(cfg, 3)
     model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
     model.load_state_dict(w)
+    assert pkg.hip.moe_plan(model.layers[0].moe, M, model.dims.ld, BF16) == ((0, False) if M == 2 else (1, True))
     ids = torch.stack([G.tokens(cfg, 3, seed=s) for s in range(M)])
     cache = model.new_cache()
     got = [model.forward(ids[:, :1], past_key_values=cache).logits]
@@ -734,18 +735,14 @@ def test_norm_between_the_output_product_and_a_mixture(pkg, width, M, shared):
         assert G.rel(got[b], O.forward(cfg, w, ids[b])[0]) < 3e-2, b
 
 
-@pytest.mark.parametrize("shared", [264, None])
-@pytest.mark.parametrize("M", [3, 16, 17, 32])
-@pytest.mark.parametrize("width,E,top", [(512, 64, 6), (992, 40, 2), (1536, 64, 1)])
-def test_rows_that_route_themselves(pkg, width, E, top, M, shared):
-    """Batches whose picks no launch sorts: equal sequences, of which every expert picked gets all rows (more than a tile of 16 of them as well), give equal rows, and those of
-    one sequence by itself; different ones the oracle's but for close calls."""
-    if M > 8 and M * top >= 2 * E:
-        pytest.skip("a chunk")
-    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(E, top, 264, shared))])
+def batch_through_a_mixture(pkg, width, E, top, ff, shared, M, plan):
+    """A batch of single tokens by the kernels named: equal sequences, of which every expert picked gets all rows (more than a tile of 16 of them as well), give equal rows, and
+    those of one sequence by itself; different ones the oracle's but for close calls."""
+    cfg = G.config(width, 96, [G.rglru(256, 4, 3, G.moe(E, top, ff, ff if shared else None))])
     w = O.random_weights(cfg, 3)
     model = pkg.GupitarForCausalLM(pkg.GupitarConfig(**cfg), device="cuda", dtype=BF16)
     model.load_state_dict(w)
+    assert pkg.hip.moe_plan(model.layers[0].moe, M, model.dims.ld, BF16) == plan
     for same in (True, False):
         ids = torch.stack([G.tokens(cfg, 2, seed=1 if same else s) for s in range(M)])
         cache = model.new_cache()
@@ -756,6 +753,27 @@ def test_rows_that_route_themselves(pkg, width, E, top, M, shared):
             assert all(torch.equal(got[b], got[0]) for b in range(M)) and err.max() < 6e-2
         else:
             assert err.median() < 2e-2 and err.quantile(0.8) < 6e-2
+
+
+@pytest.mark.parametrize("width,E,top,ff,shared,M", [(512, 64, 6, 264, True, 16), (512, 64, 6, 264, True, 17), (512, 64, 6, 264, False, 17), (992, 40, 2, 264, True, 32),
+                                                     (992, 40, 2, 264, False, 32), (1536, 64, 1, 264, True, 32), (2048, 40, 3, 520, True, 8), (2048, 40, 3, 264, False, 16),
+                                                     (2304, 40, 2, 136, True, 32), (2304, 40, 2, 136, False, 32), (3072, 40, 3, 136, True, 17), (3072, 24, 1, 264, False, 32)])
+def test_rows_that_route_themselves(pkg, width, E, top, ff, shared, M):
+    """Batches whose picks no launch sorts: one to six pieces of a row a lane, 8 to 32 rows, one to six picks."""
+    batch_through_a_mixture(pkg, width, E, top, ff, shared, M, (1, True))
+
+
+@pytest.mark.parametrize("width,E,top,ff,shared,M", [(512, 72, 3, 520, True, 8), (512, 128, 6, 264, True, 20), (544, 128, 6, 264, False, 32), (540, 128, 6, 264, True, 20),
+                                                     (1024, 128, 6, 264, False, 8), (2304, 72, 2, 136, True, 32)])
+def test_factors_of_rows_in_sorted_experts(pkg, width, E, top, ff, shared, M):
+    """Batches over more than 64 experts, whose router is the product behind the shared norm and whose rows are sorted with their factors."""
+    batch_through_a_mixture(pkg, width, E, top, ff, shared, M, (1, False))
+
+
+@pytest.mark.parametrize("width,E,top,ff,shared,M", [(512, 64, 6, 264, True, 3), (512, 64, 6, 264, False, 16), (992, 40, 2, 264, True, 17), (1536, 64, 1, 264, False, 32)])
+def test_rows_that_share_too_little_for_groups(pkg, width, E, top, ff, shared, M):
+    """Batches that the row kernels take."""
+    batch_through_a_mixture(pkg, width, E, top, ff, shared, M, (0, False))
 
 
 @pytest.mark.parametrize("width,E,top,ff,B,S,plan", [(2056, 12, 12, 136, 4, 1, (1, False)), (4104, 12, 12, 136, 4, 1, (1, False)), (512, 64, 6, 264, 20, 1, (1, True)),

@@ -414,20 +414,24 @@ def test_embedding_half_of_the_adapter_summed_once(pkg, tuned, M, h, nh):
     del keep
 
 
+@pytest.mark.parametrize("rows_of_units", [1, 3])
 @pytest.mark.parametrize("mt", [1, 2, 3, 4])
 @pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6])
-def test_rows_of_half_lines_by_parity(pkg, tuned, nt, mt):
-    """Weight rows that start on lines and in their middles by turns, every variant of units: read line by line (gemm_mid_half) they give the bits of rows read as they lie
+def test_rows_of_half_lines_by_parity(pkg, tuned, nt, mt, rows_of_units):
+    """Weight rows that start on lines and in their middles by turns, every variant of units, with weights that one unit reads or several: read line by line (gemm_mid_half) they give the bits of rows read as they lie
     where K is whole, and with slices, which odd rows begin 32 columns earlier, sums in another order; short and long K, a last unit of few columns, SwiGLU, a residual."""
     hip, dt = pkg.hip, torch.bfloat16
     for K, N, swiglu in ((160, 264, False), (672, 1048, False), (672, 520, True), (2080, 136, True)):
-        x, w = _gpu_randn((64 * mt - 20, K), 21), _gpu_randn((N * (1 + swiglu), K), 22, K ** -0.5)
+        M = 64 * mt - 20 if rows_of_units == 1 else 128 * mt + 5
+        x, w = _gpu_randn((M, K), 21), _gpu_randn((N * (1 + swiglu), K), 22, K ** -0.5)
         res = None if swiglu else _gpu_randn((x.shape[0], N), 23)
         for ks in (1, 3):
             ws = hip.linear_workspace(x.shape[0], w.shape[0], "cuda")
             outs = []
             for half in (1, 0):
                 tuned(gemm_mid_half=half, gemm_mid_nt=nt, gemm_mid_mt=mt, gemm_mid_ks=ks)
+                plan = hip.middle_plan(M, N, K, swiglu, ws.numel())
+                assert plan[:2] == (nt, mt) and plan[4] == ks and -(-M // plan[3]) == rows_of_units
                 outs.append(hip.linear(x, w, residual=res, swiglu=swiglu, workspace=ws))
             if ks == 1:
                 assert torch.equal(*outs), (K, N, swiglu)
