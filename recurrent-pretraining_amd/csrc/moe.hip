@@ -590,23 +590,20 @@ __device__ __forceinline__ unsigned wave_or(unsigned v) {
 
 // PICKED: the rows of unit group `which`, in LDS: row of x, row of the product and factor of each; the experts that rows pick come first, in their order, then tiles of
 // 16 rows of the shared expert.  Returns their number, 0 behind the last group; *group: the expert, `experts` for the shared one
-constexpr int kHeldPicks = 4;  // pieces of 64 picks that a lane keeps
+constexpr int kHeldPicks = 4;  // pieces of 64 picks that a lane keeps: all there are (moe_path: more than 8 rows go here with less than two picks per expert)
+static_assert(64 * kHeldPicks >= 8 * kMaxTop && 64 * kHeldPicks >= 2 * 64, "every pick is held");
 template <bool UP>
 __device__ __forceinline__ int picked_rows(const FewArgs& a, int which, int* group, int* x_row, int* y_row, float* scale) {
     const int lane = threadIdx.x & 63, pairs = a.M * a.top;
     unsigned low = 0, high = 0;
     int held[kHeldPicks];
-    for (int p0 = 0; p0 < pairs; p0 += 64 * kHeldPicks) {
-        int e[kHeldPicks];
 #pragma unroll
-        for (int c = 0; c < kHeldPicks; ++c) e[c] = a.pick[min(p0 + 64 * c + lane, pairs - 1)];
+    for (int c = 0; c < kHeldPicks; ++c) held[c] = a.pick[min(64 * c + lane, pairs - 1)];
 #pragma unroll
-        for (int c = 0; c < kHeldPicks; ++c) {
-            const unsigned bit = 1u << (e[c] & 31);
-            if (e[c] < 32) low |= bit;
-            else high |= bit;
-            if (p0 == 0) held[c] = e[c];
-        }
+    for (int c = 0; c < kHeldPicks; ++c) {
+        const unsigned bit = 1u << (held[c] & 31);
+        if (held[c] < 32) low |= bit;
+        else high |= bit;
     }
     const unsigned long long mask = ((unsigned long long)wave_or(high) << 32) | wave_or(low);
     const int touched = __popcll(mask);
@@ -639,7 +636,6 @@ __device__ __forceinline__ int picked_rows(const FewArgs& a, int which, int* gro
 #pragma unroll
     for (int c = 0; c < kHeldPicks; ++c)
         if (64 * c < pairs) take(64 * c, held[c]);
-    for (int p0 = 64 * kHeldPicks; p0 < pairs; p0 += 64) take(p0, a.pick[min(p0 + lane, pairs - 1)]);
     return min(n, kPickedRows);
 }
 
@@ -810,7 +806,7 @@ static int expert_rows(const void* x, const void* w, void* y, int N, int K, bool
 
 // The same over picks: g gives the matrices and, up, the factors of the pairs
 static int picked_expert_rows(const void* x, const void* w, void* y, int N, int K, bool up, const RowGroups& g, const MoeArgs& m, hipStream_t s) {
-    RAVEN_REQUIRE(m.M > 0 && m.M <= kPickedRows && m.experts <= 64 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && m.pick && m.factors &&
+    RAVEN_REQUIRE(m.M > 0 && m.M <= kPickedRows && m.M * m.top <= 64 * kHeldPicks && m.experts <= 64 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && (int64_t)2 * N * K < (1ll << 31) && m.pick && m.factors &&
                       (!up || g.x_scale) && (g.extra_group < 0 || (g.extra_group == m.experts && g.w_extra)), "moe: bad picked experts");
     FewArgs a{};
     a.x = static_cast<const bf16*>(x); a.w = static_cast<const bf16*>(w); a.y = y; a.N = N; a.K = K; a.out_f32 = up ? 0 : 1; a.g = g;
