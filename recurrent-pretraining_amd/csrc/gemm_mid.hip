@@ -125,9 +125,9 @@ __host__ __device__ constexpr int mid_requests(int tiles, int waves) { return (2
 // ONCE: every weight row is read by one unit
 // HALF: rows of K = 64 n + 32 elements on a matrix that starts on a line (5280: 82.5 lines), so that odd rows start in the middle of one, and a step of 64 columns of such a
 // row would be two half lines.  The unit's even rows are the first wave row's tiles and its odd rows the second's; odd rows are requested line by line too, 32 columns in
-// front of the even ones, and their waves multiply each of the lines' halves with the token fragments of the half before: the same products in the same order, without
-// slices; with slices the odd rows' begin and end 32 columns earlier.  us per launch at 195 rows, weights from HBM, half lines / so: mlp.fc 110 / 99 (copies
-// with padded rows 93), Wqkv 61 / 57, attn.proj 25.4 / 24.5; at 93 rows 90 / 74, 51 / 45, 24 / 22.6 (there with token rows of half lines as well).
+// front of the even ones, and their waves multiply each of the lines' halves with the token fragments of the half before: the same products in the same order.  Whole sums
+// only: the odd rows' slices would begin and end 32 columns earlier, and a matrix give other bits than its copy with padded rows.  us per launch at 195 rows, weights from HBM,
+// half lines / so: mlp.fc 110 / 99 (copies with padded rows 93), Wqkv 61 / 57; at 93 rows 90 / 74, 51 / 45 (there with token rows of half lines as well).
 template <int WN, int WM, int NT, int MT, int NS, bool ONCE, bool GROUPED = false, bool HALF = false>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     constexpr int NW = WN * WM, WPW = mid_requests(WN * NT, NW) / NW, XPW = mid_requests(WM * MT, NW) / NW, LPW = WPW + XPW;  // requests of a wave per step
@@ -160,8 +160,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
     const bool swiglu = a.kind == EPI_SWIGLU;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int K = a.K0 + a.K1, nk = (K + 63) >> 6;
-    const int k0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * slice / a.ks));
-    const int n_steps = __builtin_amdgcn_readfirstlane((int)((int64_t)nk * (slice + 1) / a.ks)) - k0;
+    const int k0 = HALF ? 0 : __builtin_amdgcn_readfirstlane((int)((int64_t)nk * slice / a.ks));
+    const int n_steps = HALF ? nk : __builtin_amdgcn_readfirstlane((int)((int64_t)nk * (slice + 1) / a.ks)) - k0;
     const int n0 = tile_n * a.cols, ncols = min(a.cols, a.N - n0), m0 = tile_m * a.bm, rows = min(a.bm, a.M - m0);
     // the wave's tiles, dealt out evenly; a SIMD's two waves (ids that differ by four) get a long and a short share of the token tiles
     const int wn = wave / WM, wm = (wn & 1) ? WM - 1 - wave % WM : wave % WM;
@@ -309,24 +309,13 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
         int o = 0, i = 0;
         arrive_left(n_steps - 1);
         if constexpr (LATE) {
-            fetch_w(0, ic0{});
-            if (k0 > 0) {
-                fetch_x(ring - stage, ic1{}, ic0{});
-            } else {  // the first line of an odd row begins with the end of the row before
+            // the first line of an odd row begins with the end of the row before
 #pragma unroll
-                for (int t = 0; t < NTW; ++t) fa[0][t] = u32x4{0, 0, 0, 0};
+            for (int t = 0; t < NTW; ++t) fa[0][t] = u32x4{0, 0, 0, 0};
 #pragma unroll
-                for (int j = 0; j < MTW; ++j) fb[0][j] = u32x4{0, 0, 0, 0};
-            }
+            for (int j = 0; j < MTW; ++j) fb[0][j] = u32x4{0, 0, 0, 0};
         } else {
             fetch(0, ic0{});
-        }
-        if (HALF && k0 > 0) {  // the last stage held the token rows of the step before; it is free once they are read
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("" ::: "memory");
         }
         // Small tiles: a loop without a branch for the steps whose requests are whole, another for the few that are not (uq of 1536 to 3072 columns at
         // 260 rows 10.7 -> 9.6 us).  Large ones: their products hide the branches, and registers are short.
@@ -381,7 +370,6 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_mid_kernel(MidArgs a) {
             o = next;
         });
     };
-    if (HALF && k0 > 0) issue(k0 - 1, ring - stage, std::integral_constant<int, WPW>{}, all{}, ic1{});  // (a step in front of others is whole)
 #pragma unroll 1
     for (int i = 0; i < NS - 1 && i < n_steps; ++i) issue(k0 + i, i * stage, ic0{}, all{}, ic2{});
     // (with fewer tiles than one less than the variant's the surplus fragments are whatever lies behind, and their products are not stored)
@@ -708,9 +696,10 @@ static int finish_slices(const MidArgs& a, hipStream_t s) {
     return raven_host::check_launch("gemm (mid, sums)");
 }
 
-// Rows that start on lines and in their middles by turns, in units whose tiles may be one more (HALF)
+// Rows that start on lines and in their middles by turns, in units whose tiles may be one more (HALF).  Not in slices: attn.proj at 195 rows takes 25.4 us
+// where slices that begin 32 columns earlier took 24.5
 static bool half_lines(const MidArgs& a, const MidPlan& p) {
-    return g_mid_half && a.K1 == 0 && a.ldw == a.K0 && a.K0 % 64 == 32 && a.K0 > 64 && ((uintptr_t)a.w & 127) == 0 && a.up_off % 2 == 0 &&
+    return g_mid_half && a.ks == 1 && a.K1 == 0 && a.ldw == a.K0 && a.K0 % 64 == 32 && a.K0 > 64 && ((uintptr_t)a.w & 127) == 0 && a.up_off % 2 == 0 &&
            mid_lds_bytes(2, 4, p.nt, p.mt, mid_stages(p.nt, p.mt), 2 * p.nt, a.xtiles) <= (size_t)kLds;
 }
 

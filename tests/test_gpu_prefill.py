@@ -418,8 +418,8 @@ def test_embedding_half_of_the_adapter_summed_once(pkg, tuned, M, h, nh):
 @pytest.mark.parametrize("mt", [1, 2, 3, 4])
 @pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6])
 def test_rows_of_half_lines_by_parity(pkg, tuned, nt, mt, rows_of_units):
-    """Weight rows that start on lines and in their middles by turns, every variant of units, with weights that one unit reads or several: read line by line (gemm_mid_half) they give the bits of rows read as they lie
-    where K is whole, and with slices, which odd rows begin 32 columns earlier, sums in another order; short and long K, a last unit of few columns, SwiGLU, a residual."""
+    """Weight rows that start on lines and in their middles by turns, every variant of units, with weights that one unit reads or several: read line by line (gemm_mid_half) they
+    give the bits of rows read as they lie, as slices do, which always are; short and long K, a last unit of few columns, SwiGLU, a residual."""
     hip, dt = pkg.hip, torch.bfloat16
     for K, N, swiglu in ((160, 264, False), (672, 1048, False), (672, 520, True), (2080, 136, True)):
         M = 64 * mt - 20 if rows_of_units == 1 else 128 * mt + 5
@@ -433,10 +433,7 @@ def test_rows_of_half_lines_by_parity(pkg, tuned, nt, mt, rows_of_units):
                 plan = hip.middle_plan(M, N, K, swiglu, ws.numel())
                 assert plan[:2] == (nt, mt) and plan[4] == ks and -(-M // plan[3]) == rows_of_units
                 outs.append(hip.linear(x, w, residual=res, swiglu=swiglu, workspace=ws))
-            if ks == 1:
-                assert torch.equal(*outs), (K, N, swiglu)
-            else:
-                check(outs[0], outs[1].float(), dt, f"slices of {K} x {N}", ulps=ULPS_SWIGLU if swiglu else ULPS_RESIDUAL)
+            assert torch.equal(*outs), (K, N, swiglu, ks)
             z = x.float() @ w.float().T
             want = F.silu(z[:, :N]) * z[:, N:] if swiglu else z + res.float()
             assert close(outs[0], want, "against float")[1] < 1e-2
@@ -657,31 +654,33 @@ def test_chunk_qkv_epilogue_writes_the_bits_of_the_two_launch_path(pkg, tuned, n
 
 
 @pytest.mark.parametrize("M,N,K,swiglu", [(300, 5280, 5280, False), (700, 1032, 136, False), (2048, 8448, 2816, False), (1100, 4096, 5280, True),
-                                          (40, 64, 72, False)])
+                                          (40, 64, 72, False), (93, 5280, 5280, False), (195, 5280, 5280, False)])
 def test_packed_weight_copies_change_no_bit(pkg, M, N, K, swiglu):
     """raven_register_packed_weight: a product over 33 and more rows reads the line-aligned copy and writes the bits it
     writes from the matrix itself (both tile sizes, the last tile columns as small tiles, SwiGLU's gate / up rows, a
-    K with a partial last step); a matrix that changes must be registered again; after unregistering the matrix is read."""
+    K with a partial last step, K in slices); a matrix that changes must be registered again; after unregistering the matrix is read."""
     hip = pkg.hip
     x = _gpu_randn((M, K), 11)
     w = _gpu_randn((2 * N if swiglu else N, K), 12, std=0.02)
     res = None if swiglu else _gpu_randn((M, N), 13)
-    plain = hip.linear(x, w, residual=res, swiglu=swiglu).clone()
+    ws = hip.linear_workspace(M, w.shape[0], "cuda") if M < 200 else None
+    run = lambda: hip.linear(x, w, residual=res, swiglu=swiglu, workspace=ws)
+    plain = run().clone()
     packed = hip.register_packed_weight(w)
     try:
         ld = (K + 63) // 64 * 64
         assert packed.numel() == w.shape[0] * ld * 2
         view = packed.view(torch.bfloat16).view(w.shape[0], ld)
         assert torch.equal(view[:, :K], w) and not view[:, K:].any()
-        assert torch.equal(hip.linear(x, w, residual=res, swiglu=swiglu), plain)
+        assert torch.equal(run(), plain)
         w.mul_(2)                                          # exact in bf16; the copy still holds the old values ...
-        assert torch.equal(hip.linear(x, w, residual=res, swiglu=swiglu), plain), "the product did not read the registered copy"
+        assert torch.equal(run(), plain), "the product did not read the registered copy"
         few = hip.linear(x[:8], w, residual=None if res is None else res[:8], swiglu=swiglu).clone()   # ... which 8 rows never read
         packed2 = hip.register_packed_weight(w)            # ... until the matrix is registered again
-        again = hip.linear(x, w, residual=res, swiglu=swiglu).clone()
+        again = run().clone()
     finally:
         hip.unregister_packed_weight(w)
-    want = hip.linear(x, w, residual=res, swiglu=swiglu)   # the matrix itself
+    want = run()                                           # the matrix itself
     assert torch.equal(again, want) and not torch.equal(again, plain)
     check(few, want[:8].float(), torch.bfloat16, "8 rows against the first rows of the large product", ulps=ULPS_SWIGLU if swiglu else ULPS_RESIDUAL)
     del packed, packed2
