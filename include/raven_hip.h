@@ -103,6 +103,8 @@ const char* raven_last_error(void);
  * kernel, with K slices where a workspace allows: those over 33 and more rows that do not fill the chip with 256 x 256 tiles, those of 17 to 32 rows
  * over K > 4096 or a large matrix, and last rounds; 0 = never), gemm_mid_nt / gemm_mid_mt / gemm_mid_ks (the
  * weight tiles, 1 to 6, and token tiles, 1 to 4, of its waves, whether or not the product has so many, and its slice count; 0 = by shape), prefill_waves (waves per workgroup of the chunk attention at head_dim 96: 0 = by shape, 4 or 6),
+ * gemm_mid_half (1 = whole sums over weight rows that are half lines longer than whole ones read odd rows by lines too; 0 = as they lie; same bits), f32_norm_rows (up to how
+ * many float rows the norms, rotation and cache append of a small model's block ride in its products; 0 = never; same bits),
  * attn_prefetch (1 = an unsplit decode-attention launch of fewer than 256 or of 1024 and more (head, row) pairs requests a
  * tile before it uses the one before, 2 = every launch does, 0 = never),
  * gemm_one_round (1 = a 2..32-row product of up to about 16384 output columns runs as at most one workgroup of eight waves per compute unit where that is faster, 2 = wherever it is narrow enough, 0 = the
@@ -420,7 +422,9 @@ int raven_core_iteration(const raven_dims* dims, const void* adapter_w,
 
 /* n_iterations recurrences in a row (the loop of iterate_forward, RMM:751-761): iteration i reads and appends to the
  * cache slots slots[i * n_blocks + j], j = 0 .. n_blocks - 1 (a host array, read before the call returns).  The same
- * results as n_iterations calls of raven_core_iteration with ln_f on the last one; for one token row the closing
+ * results as n_iterations calls of raven_core_iteration with ln_f on the last one, up to the order of the adapter's sums: the
+ * half of them that belongs to embeds may be formed once for all iterations, in float, and is added before the product's one rounding
+ * (one row; bf16 rows where that is faster).  For one token row the closing
  * norm_4 of an iteration runs as the prologue of the next adapter product instead of a launch of its own.
  * state_out may not alias state_in or embeds. */
 int raven_core_iterations(const raven_dims* dims, const void* adapter_w, const raven_block_weights* blocks,

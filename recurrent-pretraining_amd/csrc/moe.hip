@@ -5,11 +5,11 @@
 // One to a handful of rows (and fp32): moe_up_kernel forms the gated activations of a row's experts and of the shared one side by side, moe_down_kernel
 // multiplies them by the down matrices and adds to the stream.  The first picks the row's experts itself from its logits -- a handful
 // of wave reductions -- so no routing launch stands in between; for a single row it also takes the norm of the stream as a prologue.
-// More bf16 rows: the rows are sorted by expert (moe_route_kernel, or moe_pick_kernel and moe_sort_kernel) and the experts run as one
+// More bf16 rows: the rows are sorted by expert (moe_route_kernel, or moe_pick_kernel and moe_sort_kernel), or a few of them route themselves (pick_rows_kernel), and the experts run as one
 // grouped product on the matrix cores (expert_rows_kernel, gemm_mid.hip, gemm_tiled.hip), rows gathered through the sorted list; every (token, expert) pair has a slot of
 // its own, and moe_combine_kernel adds a token's slots and its shared expert to the stream in a fixed order.  So an expert's weights
 // are read once and not once per row that picked it: 20 rows over 64 experts of 768 channels at width 2048, 6 each, read
-// 55 experts instead of 120 (215 us by row kernels, 97).
+// 55 experts instead of 120 (a layer of 16 rows: 168 us by row kernels, 109).
 
 #include <algorithm>
 
@@ -908,22 +908,21 @@ static int launch_combine_norm(const MoeArgs& a, const NextNorm& next, hipStream
 
 // What runs the experts of M rows.  A chunk -- once its rows share weights (two per expert), or there are enough rows anyway -- keeps its slots in T
 // and runs the shared expert as a product of its own.  Fewer rows keep slots and sums in float, as the row kernels do, and take the
-// grouped product once reading each expert once saves more than its two further launches cost.  us, row kernels / grouped (means of four draws of picks), at
-// width 2048 (64 experts of 768 channels, 6 per row and a shared one): 2 rows 29 / 36, 3: 40 / 44, 4: 52 / 48, 8: 93 / 68, 20: 215 / 97; width 1024
-// (64 of 384): 4 rows 18 / 23, 6: 24 / 26, 8: 31 / 30, 12: 43 / 35; width 1024, one of 64 experts of 1024 and a shared one: 4 rows 14 / 21, 8: 21 / 24,
-// 12: 27 / 27, 20: 43 / 32; width 4096, 2 of 8 experts of 4096: 2 rows 72 / 70, 4: 135 / 105, 8: 251 / 132.
+// grouped products once reading each expert once saves more than their further launches cost.  us of a whole layer (a small recurrent unit in front), row kernels / grouped, means
+// of four draws of picks: width 2048 (64 experts of 768 channels, 6 per row and a shared one) 2 rows 45 / 51, 3: 54 / 59, 4: 63 / 65, 6: 81 / 77, 8: 98 / 85, 16: 168 / 109; width
+// 1024 (64 of 384) 4 rows 33 / 36, 6: 38 / 38, 8: 43 / 42, 12: 51 / 47; width 1024, one of 64 experts of 1024 and a shared one, 4 rows 31 / 34, 8: 38.5 / 37, 12: 45 / 41,
+// 24: 68 / 51; width 4096, 2 of 8 experts of 4096, 2 rows 92 / 96, 3: 120 / 111, 8: 269 / 154.
 enum MoePath { kMoeRows, kMoeFew, kMoeChunk };
 constexpr size_t kMoeRowLds = 64 * 1024 - 1024;  // what a row may take of the row kernels' LDS; longer ones are refused for few rows
 static bool few_rows_fit(const raven_moe* m, int M, int ld) {
     return (!m->shared_up || m->shared_ff == m->ff) && M >= 2 && M <= kRouteRows && M * m->top <= kRoutePairs && ld * sizeof(bf16) <= kMoeRowLds &&
            (int64_t)2 * m->ff * ld < (1ll << 31);
 }
-// Estimates in us, fitted to what 42 mixtures of 8 to 512 experts of 32 to 4096 channels at widths 256 to 7168 took with 2 to 32 rows (412 calls; standard
-// deviations 8 % for grouped, 10 % for rows).  Row kernels: weights as often as they are read, the shared expert's faster from the second row on, a share for
+// Estimates in us, fitted to what 42 mixtures of 8 to 512 experts of 32 to 4096 channels at widths 256 to 7168 took with 2 to 32 rows, when the row kernels took 4 to 25 %
+// longer and every batch was sorted.  Row kernels: weights as often as they are read, the shared expert's faster from the second row on, a share for
 // each pick, and past 64 experts, where maxima pick, one for each workgroup that picks.  Grouped: four launches, and once the weights of the experts that rows
-// pick on average, with a share for each.  Of two that are about the same, the row kernels.  Against the better of the two the choice costs 0.5 % on average,
-// 24 % at most (300 experts of 136 at width 264, 8 per row, 12 rows: 28 / 23).
-// (Fitted to row kernels that took longer than now: width 2048, 2 rows 25 us, 3: 34, 4: 43; where the two ways are about the same, either may be ahead by a tenth.)
+// pick on average, with a share for each.  Of two that are about the same, the row kernels.  With the present kernels the choice is 0.6 % slower than the better of the two on
+// average, 13 % at most (layers of 16 mixtures of 8 to 300 experts at widths 256 to 4096, 111 calls; 40 experts of 384 at width 768, 4 per row, 12 rows: 39 / 34).
 static bool grouping_pays(const raven_moe* m, int M, int ld) {
     const double pairs = (double)M * m->top, touched = m->experts * (1.0 - pow(1.0 - (double)m->top / m->experts, M)), shared = m->shared_up ? 1 : 0;
     const double expert = 6e-6 * ld * m->ff;  // MB
